@@ -360,6 +360,29 @@ def test_delayed_scaling_update_matches_the_torch_rule(dev, history_len, slots, 
         gpu.amax_history[0] += bump.to(dev)
 
 
+@pytest.mark.parametrize("history_len", [2, 63, 65, 1023, 1025, 2049])
+@pytest.mark.parametrize("slots", [15, 17, 40])
+def test_delayed_scaling_update_at_the_edges_of_its_pieces(dev, history_len, slots):
+    """A workgroup moves 16 columns by 1024 rows at once, 64 rows side by side: histories and slot counts around those
+    numbers, the row that carries the maximum walking through all of them, bit for bit against the torch rule."""
+    from fp8_gmm_amd import fp8
+
+    g = gen(7 * history_len + slots)
+    hist = torch.rand(history_len, slots, generator=g)
+    for j in range(slots):
+        hist[(j * history_len) // slots, j] = 2.0 + j
+    hist[history_len - 1, 3], hist[history_len // 2, 5] = float("nan"), float("inf")
+    recipe = fp8.DelayedScaling(amax_history_len=history_len)
+    cpu, gpu = (fp8.Fp8MetaTensors(slots, history_len, d) for d in (torch.device("cpu"), dev))
+    cpu.amax_history.copy_(hist), gpu.amax_history.copy_(hist)
+    for step in range(2):
+        for meta in (cpu, gpu):
+            fp8.amax_and_scale_update(meta, 448.0, recipe)
+        for name in ("scale", "scale_inv", "amax_history"):
+            a, b = getattr(gpu, name).cpu(), getattr(cpu, name)
+            assert torch.equal(a.view(torch.int32), b.view(torch.int32)), f"{name} differs at step {step}"
+
+
 def test_several_scaling_updates_in_one_launch_equal_one_launch_each(dev):
     """fp8gmm_delayed_scaling_updates: up to four directions in one kernel launch (a module's forward and backward
     state go together) must leave every tensor exactly as one launch per direction does: different history
