@@ -174,6 +174,10 @@ class PassPlan(ctypes.Structure):
 
 PASS_CAST = 1
 PASS_GEMM = 2
+LINEAR_FORWARD, LINEAR_BACKWARD, MLP_FORWARD, MLP_BACKWARD = range(4)
+PASS_MAX_EXPERTS = 448
+PASS_MAX_GRID = 512
+PassTables = ctypes.c_uint64 * (4032 // 8)   # FP8GMM_PASS_TABLES_BYTES, opaque
 
 EXPORTS = (
     "fp8gmm_version",
@@ -190,6 +194,8 @@ EXPORTS = (
     "fp8gmm_plan_mlp_forward",
     "fp8gmm_plan_mlp_backward",
     "fp8gmm_sizeof_mlp_pass",
+    "fp8gmm_lay_out_pass",
+    "fp8gmm_build_pass",
     "fp8gmm_run_planned",
     "fp8gmm_host_alloc",
     "fp8gmm_host_free",
@@ -301,6 +307,10 @@ def load():
         fn.argtypes = [ctypes.POINTER(MlpPass), vp, ctypes.c_size_t, ctypes.POINTER(PassPlan)]
     L.fp8gmm_sizeof_mlp_pass.restype = ctypes.c_size_t
     L.fp8gmm_sizeof_mlp_pass.argtypes = []
+    L.fp8gmm_lay_out_pass.restype = ci
+    L.fp8gmm_lay_out_pass.argtypes = [ci, vp, ctypes.POINTER(PassPlan), vp]
+    L.fp8gmm_build_pass.restype = ci
+    L.fp8gmm_build_pass.argtypes = [vp, vp, vp, vp, ci, vp]
     L.fp8gmm_run_planned.restype = ci
     L.fp8gmm_run_planned.argtypes = [vp, ctypes.POINTER(PassLaunch), vp, ctypes.c_size_t, vp]
     L.fp8gmm_sizeof_linear_pass.restype = ctypes.c_size_t

@@ -951,10 +951,11 @@ def warm_up(device=None):
 # ------------------------------------------------------------------------------------------------
 # a whole pass of a grouped linear layer, planned by one library call
 # ------------------------------------------------------------------------------------------------
-def _run_pass(device, desc, fields, plan_fn, bound_fn):
-    """Fill the pass description `desc` from `fields`, plan it with `plan_fn` straight into staging memory (of
-    `bound_fn(desc, grid)` bytes at first; the planner says how much it needs when that is too little), upload the
-    tables and enqueue the launches."""
+def _run_pass(device, which, desc, fields, snapshot, host_planned):
+    """Fill the pass description `desc` from `fields`, have its tables built and enqueue its launches.  The tables are
+    written by a kernel of the library from a description of the pass (fp8gmm_build_pass), which also takes the
+    `snapshot` (source, destination) of fp32 values; a pass of more experts than fit a kernel argument is planned on
+    the host (`host_planned`: planning function, bound on its bytes) and uploaded."""
     L = _lib.load()
     flush_uploads()   # launches queued before this pass come first
     keep = []
@@ -971,19 +972,20 @@ def _run_pass(device, desc, fields, plan_fn, bound_fn):
     desc.grid = grid
     desc.stream_k = int(bool(options.stream_k))
     desc.tile_policy = {"auto": 0, "256": 256, "128": 128, "dual": _lib.GEMM_TILE_DUAL}[options.tile]
-    bound = bound_fn(desc, grid)
     plan = _lib.PassPlan()
-    while True:
-        def fill(address, _):
-            fill.rc = plan_fn(ctypes.byref(desc), address, bound, ctypes.byref(plan))
-            return int(plan.blob_bytes) if fill.rc == 0 else 0
-
-        blob = _to_device(device, bound, fill)
-        if fill.rc == -8 and plan.blob_bytes > bound:   # FP8GMM_ERR_BUFFER_TOO_SMALL
-            bound = int(plan.blob_bytes)
-            continue
-        _lib.check(fill.rc)
-        break
+    if desc.experts <= _lib.PASS_MAX_EXPERTS and 2 * grid <= _lib.PASS_MAX_GRID:
+        tables = _lib.PassTables()
+        _lib.check(L.fp8gmm_lay_out_pass(which, ctypes.byref(desc), ctypes.byref(plan), tables))
+        with _on_device(device):
+            blob = torch.empty(plan.blob_bytes, dtype=torch.uint8, device=device)
+            src, dst = snapshot if snapshot is not None else (None, None)
+            n = src.numel() if src is not None else 0
+            _lib.check(L.fp8gmm_build_pass(tables, blob.data_ptr(), src.data_ptr() if n else None,
+                                           dst.data_ptr() if n else None, n, _stream(device)))
+    else:
+        blob = _plan_on_host(device, desc, plan, *host_planned, grid)
+        if snapshot is not None:
+            snapshot[1].copy_(snapshot[0])
     if blob is None:
         return plan
     with _on_device(device):
@@ -1002,6 +1004,23 @@ def _run_pass(device, desc, fields, plan_fn, bound_fn):
     return plan
 
 
+def _plan_on_host(device, desc, plan, plan_fn, bound_fn, grid):
+    """The tables of a pass planned straight into staging memory (of ``bound_fn(desc, grid)`` bytes at first; the
+    planner says how much it needs when that is too little) and uploaded."""
+    bound = bound_fn(desc, grid)
+    while True:
+        def fill(address, _):
+            fill.rc = plan_fn(ctypes.byref(desc), address, bound, ctypes.byref(plan))
+            return int(plan.blob_bytes) if fill.rc == 0 else 0
+
+        blob = _to_device(device, bound, fill)
+        if fill.rc == -8 and plan.blob_bytes > bound:   # FP8GMM_ERR_BUFFER_TOO_SMALL
+            bound = int(plan.blob_bytes)
+            continue
+        _lib.check(fill.rc)
+        return blob
+
+
 def _pass_room(experts, tokens, shapes, casts, grid):
     """Bytes that surely hold the tables of a pass with GEMMs over ``shapes`` (pairs of feature counts; every GEMM
     is token-sliced in one dimension or per expert in both) and ``casts`` cast descriptors: per GEMM a problem table
@@ -1015,25 +1034,27 @@ def _pass_room(experts, tokens, shapes, casts, grid):
     return room
 
 
-def linear_pass(device, backward=False, **fields):
-    """Plans one pass of a grouped linear layer with ONE library call (fp8gmm_plan_linear_forward / _backward),
-    uploads its tables with one copy and enqueues its launches.  ``fields`` are the members of
-    ``fp8gmm_linear_pass`` (include/fp8gmm.h): tensors are given as tensors (their addresses are taken here),
-    ``group_sizes`` as an int64 numpy array.  The tables are the ones the per-launch entry points of this module
-    build for the same tensors; what this call saves is the host time of building them in Python."""
+def linear_pass(device, backward=False, snapshot=None, **fields):
+    """Runs one pass of a grouped linear layer: one library call describes it, one kernel writes its tables, its
+    launches follow.  ``fields`` are the members of ``fp8gmm_linear_pass`` (include/fp8gmm.h): tensors are given as
+    tensors (their addresses are taken here), ``group_sizes`` as an int64 numpy array.  The tables are the ones the
+    per-launch entry points of this module build for the same tensors.  ``snapshot=(source, destination)``: fp32
+    tensors, the first of which is copied to the second in front of the pass."""
     L = _lib.load()
     return _run_pass(
-        device, _lib.LinearPass(), fields, L.fp8gmm_plan_linear_backward if backward else L.fp8gmm_plan_linear_forward,
-        lambda d, grid: _pass_room(d.experts, d.tokens, [(d.in_features, d.out_features)] * 3, 2 * d.experts, grid))
+        device, _lib.LINEAR_BACKWARD if backward else _lib.LINEAR_FORWARD, _lib.LinearPass(), fields, snapshot,
+        (L.fp8gmm_plan_linear_backward if backward else L.fp8gmm_plan_linear_forward,
+         lambda d, grid: _pass_room(d.experts, d.tokens, [(d.in_features, d.out_features)] * 3, 2 * d.experts, grid)))
 
 
-def mlp_pass(device, backward=False, **fields):
-    """The same for one pass of a grouped MLP in its default data flow (fp8gmm_plan_mlp_forward / _backward, members
-    of ``fp8gmm_mlp_pass``): three launches forward, up to six backward, from one library call and one upload."""
+def mlp_pass(device, backward=False, snapshot=None, **fields):
+    """The same for one pass of a grouped MLP in its default data flow (members of ``fp8gmm_mlp_pass``): three launches
+    forward, up to six backward."""
     L = _lib.load()
     return _run_pass(
-        device, _lib.MlpPass(), fields, L.fp8gmm_plan_mlp_backward if backward else L.fp8gmm_plan_mlp_forward,
-        lambda d, grid: _pass_room(d.experts, d.tokens, [(d.hidden, d.ffn)] * 4, 3 * d.experts, grid))
+        device, _lib.MLP_BACKWARD if backward else _lib.MLP_FORWARD, _lib.MlpPass(), fields, snapshot,
+        (L.fp8gmm_plan_mlp_backward if backward else L.fp8gmm_plan_mlp_forward,
+         lambda d, grid: _pass_room(d.experts, d.tokens, [(d.hidden, d.ffn)] * 4, 3 * d.experts, grid)))
 
 
 def delayed_scaling_update(amax_history, scale, scale_inv, fp8_max, margin=0, most_recent=False, keep_scale_inv=None):

@@ -20,4 +20,16 @@ int launch_gemm_merging(const fp8gmm_gemm_problem* probs_dev, int n, const fp8gm
                         int out_kind, int epilogue, void* workspace, size_t workspace_bytes,
                         const fp8gmm_tensor_desc* merge_descs, int merge_n, void* stream);
 
+struct GemmRanges;
+struct PassTables;
+
+// fp8gmm_plan_grouped_gemm_launch without the records: the sizes of the launch and, per XCD, the ranges that the records
+// follow from (pass_spec.h).  The same decisions from the same code.
+int plan_gemm_ranges(fp8gmm_gemm_problem* probs, int n, int layout, int grid, int stream_k, fp8gmm_gemm_plan* plan,
+                     GemmRanges* out);
+
+// Writes the tables of a pass into device memory (pass_tables.hip), and copies `copy_n` floats on the side.
+int launch_pass_tables(const PassTables& tables, void* blob_dev, const float* copy_src, float* copy_dst, int copy_n,
+                       void* stream);
+
 }  // namespace fp8gmm

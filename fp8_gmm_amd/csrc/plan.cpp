@@ -12,6 +12,8 @@
 
 #include "../../include/fp8gmm.h"
 #include "gemm_schedule.h"
+#include "internal.h"
+#include "pass_spec.h"
 #include "tiling.h"
 
 extern "C" {
@@ -187,17 +189,23 @@ int fp8gmm_plan_grouped_gemm_layout(fp8gmm_gemm_problem* probs, int n, int layou
 // The same launch cut into 128 x 128 tiles (FP8GMM_GEMM_TILE_128) or into 128 x 256 tiles for the kernel with two
 // sets of accumulators (FP8GMM_GEMM_TILE_DUAL): whole tiles only, the tile list in 8 contiguous ranges of equal
 // work, the workgroups of an XCD striding through their range.
+constexpr int kSmallTileOverhead = 3, kDualTileOverhead = 2;
 // kOverhead: what a tile costs besides its steps, in K = 128 steps: epilogue and switch of a small tile on a
 // workgroup that shares its compute unit; with two sets of accumulators, the slower steps that carry the result.
-static int plan_whole_tiles(const int TM, const int TN, const int kOverhead, fp8gmm_gemm_problem* probs, int n, int layout,
-                            int grid, fp8gmm_gemm_item* items, int max_items, fp8gmm_gemm_plan* plan) {
+struct WholeTileCuts {
+  std::vector<int64_t> tile_begin;        // per problem
+  int cut[fp8gmm::kNumXcd + 1];           // XCD x takes the tiles [cut[x], cut[x + 1])
+};
+static int cut_whole_tiles(const int TM, const int TN, const int kOverhead, fp8gmm_gemm_problem* probs, int n, int layout,
+                           int grid, WholeTileCuts* out, fp8gmm_gemm_plan* plan) {
   using namespace fp8gmm;
   int unused = 0;
   const int rc = fp8gmm_plan_grouped_gemm_layout(probs, n, layout, &unused);
   if (rc != FP8GMM_OK) return rc;
-  const bool a_kmajor = (layout & FP8GMM_GEMM_A_KMAJOR) != 0, b_kmajor = (layout & FP8GMM_GEMM_B_KMAJOR) != 0;
   // tiles and work per problem
-  std::vector<int64_t> tile_begin((size_t)n + 1, 0), work_begin((size_t)n + 1, 0);
+  std::vector<int64_t>& tile_begin = out->tile_begin;
+  std::vector<int64_t> work_begin((size_t)n + 1, 0);
+  tile_begin.assign((size_t)n + 1, 0);
   for (int p = 0; p < n; ++p) {
     const int64_t tiles = (int64_t)((probs[p].m + TM - 1) / TM) * ((probs[p].n + TN - 1) / TN);
     const int64_t steps = (probs[p].k + 127) / 128;
@@ -214,36 +222,43 @@ static int plan_whole_tiles(const int TM, const int TN, const int kOverhead, fp8
     const int needed = ((total_tiles + kNumXcd - 1) / kNumXcd) * kNumXcd;
     if (grid > needed) grid = needed;
   }
-  const int wgs = grid / kNumXcd;
-  // XCD x takes the tiles [cut[x], cut[x + 1]): the first tile at or past x / 8 of the work
-  int cut[kNumXcd + 1];
+  plan->grid = grid;
+  // the first tile of XCD x: the first one at or past x / 8 of the work
+  int* cut = out->cut;
   cut[0] = 0;
   cut[kNumXcd] = total_tiles;
-  {
-    int p = 0;
-    for (int x = 1; x < kNumXcd; ++x) {
-      const int64_t target = (work_begin[n] * x + kNumXcd - 1) / kNumXcd;
-      while (p < n && work_begin[p + 1] <= target) ++p;
-      if (p >= n) {
-        cut[x] = total_tiles;
-        continue;
-      }
-      const int64_t per_tile = (work_begin[p + 1] - work_begin[p]) / (tile_begin[p + 1] - tile_begin[p]);
-      cut[x] = (int)(tile_begin[p] + (target - work_begin[p] + per_tile - 1) / per_tile);
+  int p = 0;
+  for (int x = 1; x < kNumXcd; ++x) {
+    const int64_t target = (work_begin[n] * x + kNumXcd - 1) / kNumXcd;
+    while (p < n && work_begin[p + 1] <= target) ++p;
+    if (p >= n) {
+      cut[x] = total_tiles;
+      continue;
     }
+    const int64_t per_tile = (work_begin[p + 1] - work_begin[p]) / (tile_begin[p + 1] - tile_begin[p]);
+    cut[x] = (int)(tile_begin[p] + (target - work_begin[p] + per_tile - 1) / per_tile);
   }
+  const int wgs = grid / kNumXcd;
   int rounds = 0;
   for (int x = 0; x < kNumXcd; ++x) rounds = std::max(rounds, (cut[x + 1] - cut[x] + wgs - 1) / wgs);
-  rounds += 1;  // every list ends with a record whose prob is -1
-  plan->grid = grid;
-  plan->rounds = rounds;
-  if ((int64_t)rounds * grid > INT32_MAX / 64) return FP8GMM_ERR_BAD_SHAPE;
+  plan->rounds = rounds + 1;  // every list ends with a record whose prob is -1
+  return (int64_t)plan->rounds * grid > INT32_MAX / 64 ? FP8GMM_ERR_BAD_SHAPE : FP8GMM_OK;
+}
+
+static int plan_whole_tiles(const int TM, const int TN, const int kOverhead, fp8gmm_gemm_problem* probs, int n, int layout,
+                            int grid, fp8gmm_gemm_item* items, int max_items, fp8gmm_gemm_plan* plan) {
+  using namespace fp8gmm;
+  WholeTileCuts cuts;
+  const int rc = cut_whole_tiles(TM, TN, kOverhead, probs, n, layout, grid, &cuts, plan);
+  if (rc != FP8GMM_OK || plan->total_tiles == 0) return rc;
+  const bool a_kmajor = (layout & FP8GMM_GEMM_A_KMAJOR) != 0, b_kmajor = (layout & FP8GMM_GEMM_B_KMAJOR) != 0;
+  const std::vector<int64_t>& tile_begin = cuts.tile_begin;
+  const int* cut = cuts.cut;
+  const int rounds = plan->rounds, wgs = plan->grid / kNumXcd;
+  grid = plan->grid;
   if ((int64_t)rounds * grid > max_items) return FP8GMM_ERR_BUFFER_TOO_SMALL;
   if (items == nullptr) return FP8GMM_ERR_NULL_POINTER;
-  fp8gmm_gemm_item end_record{};
-  end_record.prob = -1;
-  end_record.slot = -1;
-  for (int i = 0; i < rounds * grid; ++i) items[i] = end_record;
+  for (int i = 0; i < rounds * grid; ++i) items[i] = gemm_end_item();
   for (int x = 0; x < kNumXcd; ++x) {
     int p = 0;
     for (int t = cut[x]; t < cut[x + 1]; ++t) {
@@ -251,40 +266,23 @@ static int plan_whole_tiles(const int TM, const int TN, const int kOverhead, fp8
       const fp8gmm_gemm_problem& pr = probs[p];
       const int local = t - cut[x];
       const int r = local / wgs, j = (local + kRoundRotation * r) % wgs;   // position in the round rotates
-      fp8gmm_gemm_item& o = items[(size_t)r * grid + (size_t)j * kNumXcd + x];
-      o = fp8gmm_gemm_item{};
       int m0 = 0, n0 = 0;
       tile_origin(pr.m, pr.n, (int)(t - tile_begin[p]), TM, TN, &m0, &n0);
-      const int64_t rows = pr.m - m0 < TM ? pr.m - m0 : TM;
-      const int64_t cols = pr.n - n0 < TN ? pr.n - n0 : TN;
-      if (pr.k > 0) {
-        if (!a_kmajor) {
-          o.a = (uint64_t)reinterpret_cast<uintptr_t>(pr.a) + (uint64_t)m0 * (uint64_t)pr.lda;
-          o.a_bytes = (uint32_t)((rows - 1) * pr.lda + ((pr.k + 15) & ~15));
-        } else {
-          o.a = (uint64_t)reinterpret_cast<uintptr_t>(pr.a) + (uint64_t)m0;
-          o.a_bytes = (uint32_t)((int64_t)(pr.k - 1) * pr.lda + (pr.m - m0));
-        }
-        if (!b_kmajor) {
-          o.b = (uint64_t)reinterpret_cast<uintptr_t>(pr.b) + (uint64_t)n0 * (uint64_t)pr.ldb;
-          o.b_bytes = (uint32_t)((cols - 1) * pr.ldb + pr.k);
-        } else {
-          o.b = (uint64_t)reinterpret_cast<uintptr_t>(pr.b) + (uint64_t)n0;
-          o.b_bytes = (uint32_t)((int64_t)(pr.k - 1) * pr.ldb + (pr.n - n0));
-        }
-      }
-      o.lda = pr.lda;
-      o.ldb = pr.ldb;
-      o.k = pr.k;
-      o.k_begin = 0;
-      o.nk = (pr.k + 127) / 128;
-      o.m0 = m0;
-      o.n0 = n0;
-      o.prob = p;
-      o.slot = -1;
+      items[(size_t)r * grid + (size_t)j * kNumXcd + x] =
+          gemm_item(pr, p, m0, n0, TM, TN, a_kmajor, b_kmajor, 0, (pr.k + 127) / 128, -1);
     }
   }
   return FP8GMM_OK;
+}
+
+// Tail balancing can only pay when the launch has few rounds; it needs the whole grid even for few tiles.  Without it
+// the grid shrinks to the tiles there are.
+static bool share_tail(int stream_k, int total_tiles, int* grid) {
+  using namespace fp8gmm;
+  if (stream_k != 0 && (int64_t)total_tiles <= (int64_t)kSkMaxRounds * *grid && *grid > kNumXcd) return true;
+  const int needed = ((total_tiles + kNumXcd - 1) / kNumXcd) * kNumXcd;
+  if (*grid > needed) *grid = needed;
+  return false;
 }
 
 int fp8gmm_plan_grouped_gemm_launch(fp8gmm_gemm_problem* probs, int n, int layout, int grid, int stream_k,
@@ -299,9 +297,10 @@ int fp8gmm_plan_grouped_gemm_launch(fp8gmm_gemm_problem* probs, int n, int layou
     if ((layout & FP8GMM_GEMM_TILE_128) && (layout & FP8GMM_GEMM_TILE_DUAL)) return FP8GMM_ERR_BAD_ARGUMENT;
     const int operands = layout & ~(FP8GMM_GEMM_TILE_128 | FP8GMM_GEMM_TILE_DUAL);
     if (layout & FP8GMM_GEMM_TILE_128)
-      return plan_whole_tiles(FP8GMM_GEMM_SMALL_TILE, FP8GMM_GEMM_SMALL_TILE, 3, probs, n, operands, grid, items,
+      return plan_whole_tiles(FP8GMM_GEMM_SMALL_TILE, FP8GMM_GEMM_SMALL_TILE, kSmallTileOverhead, probs, n, operands, grid, items,
                               max_items, plan);
-    return plan_whole_tiles(FP8GMM_GEMM_DUAL_TILE_M, kGemmTileN, 2, probs, n, operands, grid, items, max_items, plan);
+    return plan_whole_tiles(FP8GMM_GEMM_DUAL_TILE_M, kGemmTileN, kDualTileOverhead, probs, n, operands, grid, items, max_items,
+                            plan);
   }
   plan->tile = kGemmTileM;
   const int layout_given = layout, grid_given = grid;
@@ -313,12 +312,7 @@ int fp8gmm_plan_grouped_gemm_launch(fp8gmm_gemm_problem* probs, int n, int layou
   if (rc != FP8GMM_OK) return rc;
   plan->total_tiles = total_tiles;
   if (total_tiles == 0) return FP8GMM_OK;
-  // tail balancing can only pay when the launch has few rounds; it needs the whole grid even for few tiles
-  const bool sk = stream_k != 0 && (int64_t)total_tiles <= (int64_t)kSkMaxRounds * grid && grid > kNumXcd;
-  if (!sk) {
-    const int needed = ((total_tiles + kNumXcd - 1) / kNumXcd) * kNumXcd;
-    if (grid > needed) grid = needed;
-  }
+  const bool sk = share_tail(stream_k, total_tiles, &grid);
   const int wgs = grid / kNumXcd;
   const bool a_kmajor = (layout & FP8GMM_GEMM_A_KMAJOR) != 0, b_kmajor = (layout & FP8GMM_GEMM_B_KMAJOR) != 0;
 
@@ -360,42 +354,12 @@ int fp8gmm_plan_grouped_gemm_launch(fp8gmm_gemm_problem* probs, int n, int layou
   bool dangling_piece = false;
   auto write_record = [&](const Item& it, size_t index) {
     const fp8gmm_gemm_problem& p = probs[it.prob];
-    fp8gmm_gemm_item o{};   // assembled in registers and stored once: stores into the list could alias anything
-    const int64_t rows = p.m - it.m0 < BM ? p.m - it.m0 : BM;
-    const int64_t cols = p.n - it.n0 < BN ? p.n - it.n0 : BN;
-    if (p.k > 0) {
-      // extents: up to the last byte of the tile's last row (row-major) / of the operand's last contraction row.
-      // A row-major a whose k is not a multiple of 16 (allowed next to a contraction-major b) ends inside a
-      // 16-byte piece; the bound includes the whole piece, which lies inside the row's pitch: the hardware
-      // checks the range per dword, and a dword that straddled the bound would lose its valid bytes too.
-      if (!a_kmajor) {
-        o.a = (uint64_t)reinterpret_cast<uintptr_t>(p.a) + (uint64_t)it.m0 * (uint64_t)p.lda;
-        o.a_bytes = (uint32_t)((rows - 1) * p.lda + ((p.k + 15) & ~15));
-      } else {
-        o.a = (uint64_t)reinterpret_cast<uintptr_t>(p.a) + (uint64_t)it.m0;
-        o.a_bytes = (uint32_t)((int64_t)(p.k - 1) * p.lda + (p.m - it.m0));
-      }
-      if (!b_kmajor) {
-        o.b = (uint64_t)reinterpret_cast<uintptr_t>(p.b) + (uint64_t)it.n0 * (uint64_t)p.ldb;
-        o.b_bytes = (uint32_t)((cols - 1) * p.ldb + p.k);
-      } else {
-        o.b = (uint64_t)reinterpret_cast<uintptr_t>(p.b) + (uint64_t)it.n0;
-        o.b_bytes = (uint32_t)((int64_t)(p.k - 1) * p.ldb + (p.n - it.n0));
-      }
-    }
-    o.lda = p.lda;
-    o.ldb = p.ldb;
-    o.k = p.k;
-    o.k_begin = it.k_begin;
-    o.nk = it.nk;
-    o.m0 = it.m0;
-    o.n0 = it.n0;
-    o.prob = it.prob;
-    o.slot = -1;
+    // assembled in registers and stored once: stores into the list could alias anything
+    fp8gmm_gemm_item o = gemm_item(p, it.prob, it.m0, it.n0, BM, BN, a_kmajor, b_kmajor, it.k_begin, it.nk, -1);
     if (it.slot >= 0) {
       o.slot = slot_map[it.slot];
       if (o.slot < 0) dangling_piece = true;  // a partial item that no fix-up record completes
-    } else if (rows <= BM / 2) {
+    } else if (p.m - it.m0 <= BM / 2) {
       o.flags = FP8GMM_ITEM_HALF_HEIGHT;      // a whole tile with at most 128 valid rows
     }
     items[index] = o;
@@ -496,13 +460,82 @@ int fp8gmm_plan_grouped_gemm_launch(fp8gmm_gemm_problem* probs, int n, int layou
   if (items == nullptr || (n_fixups > 0 && fixups == nullptr)) return FP8GMM_ERR_NULL_POINTER;
   if (dangling_piece) return FP8GMM_ERR_BAD_ARGUMENT;
   for (int f = 0; f < n_fixups; ++f) fixups[f] = fix[f];
-  fp8gmm_gemm_item end_record{};
-  end_record.prob = -1;
-  end_record.slot = -1;
   for (int r = 0; r < rounds; ++r)
     for (int wg = 0; wg < grid; ++wg)
-      if (r >= count[wg]) items[(size_t)r * grid + wg] = end_record;
+      if (r >= count[wg]) items[(size_t)r * grid + wg] = gemm_end_item();
   return FP8GMM_OK;
 }
 
 }  // extern "C"
+
+namespace fp8gmm {
+
+int plan_gemm_ranges(fp8gmm_gemm_problem* probs, int n, int layout, int grid, int stream_k, fp8gmm_gemm_plan* plan,
+                     GemmRanges* out) {
+  *plan = fp8gmm_gemm_plan{};
+  *out = GemmRanges{};
+  if (grid <= 0 || (grid % kNumXcd) != 0) return FP8GMM_ERR_BAD_ARGUMENT;
+  if (layout & (FP8GMM_GEMM_TILE_128 | FP8GMM_GEMM_TILE_DUAL)) {
+    const bool small = (layout & FP8GMM_GEMM_TILE_128) != 0;
+    WholeTileCuts cuts;
+    const int rc = cut_whole_tiles(small ? FP8GMM_GEMM_SMALL_TILE : FP8GMM_GEMM_DUAL_TILE_M, small ? FP8GMM_GEMM_SMALL_TILE : kGemmTileN,
+                                   small ? kSmallTileOverhead : kDualTileOverhead, probs, n,
+                                   layout & (FP8GMM_GEMM_A_KMAJOR | FP8GMM_GEMM_B_KMAJOR), grid, &cuts, plan);
+    if (rc != FP8GMM_OK || plan->total_tiles == 0) return rc;
+    for (int x = 0; x < kNumXcd; ++x) {
+      out->xcd[x].begin = cuts.cut[x];
+      out->xcd[x].end = cuts.cut[x + 1];
+    }
+  } else {
+    const bool gelu = (layout & (FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU)) != 0;
+    plan->tile = kGemmTileM;
+    int total_tiles = 0;
+    const int rc = fp8gmm_plan_grouped_gemm_layout(probs, n, layout & ~(FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU), &total_tiles);
+    if (rc != FP8GMM_OK) return rc;
+    plan->total_tiles = total_tiles;
+    if (total_tiles == 0) return FP8GMM_OK;
+    const bool sk = share_tail(stream_k, total_tiles, &grid);
+    const int wgs = grid / kNumXcd;
+    plan->grid = grid;
+    for (int x = 0; x < kNumXcd; ++x) {
+      Sched s;
+      sched_init(s, probs, n, total_tiles, x, wgs, sk, gelu ? 3 : 1);
+      GemmRanges::Xcd& o = out->xcd[x];
+      o.begin = s.range_begin;
+      o.end = s.range_end;
+      o.dp_rounds = s.dp_rounds;
+      o.sk_begin = s.sk_begin;
+      o.sk_wgs = s.sk_wgs;
+      o.sk_c0 = (int32_t)s.sk_c0;
+      o.sk_cost = (int32_t)s.sk_cost;
+      out->total_cost = (int32_t)s.total_cost;
+      int rounds = s.dp_rounds;
+      for (int j = 0; j < s.sk_wgs; ++j) {
+        // with a shared remainder every strided round is full: the pieces of workgroup j follow its dp_rounds tiles
+        Cursor c;
+        cursor_init(s, j, c);
+        int count = s.dp_rounds;
+        c.dp_i = s.dp_rounds;
+        for (; cursor_valid(s, j, c); cursor_advance(s, j, c)) ++count;
+        rounds = std::max(rounds, count);
+        int nf = 0;
+        if (fixup_tile(s, j, &nf) >= 0) {
+          plan->n_fixups += 1;
+          plan->n_slots += nf + 1;
+        }
+      }
+      plan->rounds = std::max(plan->rounds, rounds);
+    }
+    if (sk && stream_k > 1 && plan->n_slots > stream_k)   // a fixed amount of workspace: whole tiles then
+      return plan_gemm_ranges(probs, n, layout, grid, 0, plan, out);
+    plan->rounds += 1;
+    if ((int64_t)plan->rounds * grid > INT32_MAX / 64) return FP8GMM_ERR_BAD_SHAPE;
+  }
+  out->grid = plan->grid;
+  out->rounds = plan->rounds;
+  out->total_tiles = plan->total_tiles;
+  out->n_fixups = plan->n_fixups;
+  return FP8GMM_OK;
+}
+
+}  // namespace fp8gmm

@@ -149,7 +149,8 @@ class _GroupedLinear(torch.autograd.Function):
                     weight_cache.require(False)
             out = torch.empty(input.size(0), weight.size(1), dtype=torch.bfloat16, device=dev)
             fwd = fp8_meta["scaling_fwd"]
-            linear_pass(dev, False, experts=num_groups, in_features=weight.size(2), out_features=weight.size(1),
+            linear_pass(dev, False, snapshot=meta.forward_scale_inv_snapshot() if is_grad_enabled else None,
+                        experts=num_groups, in_features=weight.size(2), out_features=weight.size(1),
                         fwd_fmt=_lib.E4M3 if fp8_dtype == torch.float8_e4m3fn else _lib.E5M2, cast_weights=cast_weights,
                         tokens=input.size(0), group_sizes=sizes, x=input, x_fp8=input_fp8, w=weight, w_fp8=weight_fp8,
                         y=out, fwd_scale=fwd.scale, fwd_scale_inv=fwd.scale_inv, fwd_amax=fwd.amax_history)
@@ -159,7 +160,6 @@ class _GroupedLinear(torch.autograd.Function):
                 ctx.planned = True
                 ctx.sizes = sizes
                 ctx.group_sizes = group_sizes
-                meta.set_forward_scale_inv_cloned()
                 ctx.meta = meta
                 ctx.num_groups = num_groups
                 ctx.padded = padded

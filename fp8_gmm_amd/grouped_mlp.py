@@ -110,7 +110,8 @@ class _GroupedMlp(torch.autograd.Function):
             gelu_out_fp8 = torch.empty(tokens, ffn, dtype=fp8_dtype, device=dev)
             out = torch.empty(tokens, input.size(1), dtype=torch.bfloat16, device=dev)
             fwd = fp8_meta["scaling_fwd"]
-            mlp_pass(dev, False, experts=num_groups, hidden=input.size(1), ffn=ffn,
+            mlp_pass(dev, False, snapshot=meta.forward_scale_inv_snapshot() if is_grad_enabled else None,
+                     experts=num_groups, hidden=input.size(1), ffn=ffn,
                      fwd_fmt=_lib.E4M3 if fp8_dtype == torch.float8_e4m3fn else _lib.E5M2, cast_weights=cast_weights,
                      tokens=tokens, group_sizes=sizes, x=input, x_fp8=input_fp8, w1=fc1_weight, w1_fp8=fc1_weight_fp8,
                      w2=fc2_weight, w2_fp8=fc2_weight_fp8, pre=pre_gelu_out, act_fp8=gelu_out_fp8, y=out,
@@ -201,6 +202,7 @@ class _GroupedMlp(torch.autograd.Function):
                 w2_dgrad = fc2_weight_fp8 if dgrad_needed else None
             ctx.save_for_backward(x_wgrad, w1_dgrad, w2_dgrad, pre_gelu_out, gelu_out_fp8)
             ctx.planned = False
+            meta.set_forward_scale_inv_cloned()
             _GroupedMlp._remember(ctx, reference_layout, group_sizes, meta, num_groups, padded, cumsums, padded_cumsums,
                                   fp8_meta, fc1_weight, fc2_weight, input_requires_grad, weight_requires_grad, has_tp,
                                   tp_group)
@@ -212,7 +214,6 @@ class _GroupedMlp(torch.autograd.Function):
         """What the backward pass needs besides the saved tensors."""
         ctx.reference_layout = reference_layout
         ctx.group_sizes = group_sizes
-        meta.set_forward_scale_inv_cloned()
         ctx.meta = meta
         ctx.num_groups = num_groups
         ctx.padded = padded

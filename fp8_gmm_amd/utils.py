@@ -113,6 +113,12 @@ class Fp8MetaWrapper:
     def set_forward_scale_inv_cloned(self):
         self._forward_scale_inv_cloned = self._fp8_meta["scaling_fwd"].scale_inv.clone()
 
+    def forward_scale_inv_snapshot(self):
+        """``(source, destination)`` of the same copy for a caller that has it made by a kernel of its own."""
+        src = self._fp8_meta["scaling_fwd"].scale_inv
+        self._forward_scale_inv_cloned = torch.empty_like(src)
+        return src, self._forward_scale_inv_cloned
+
     def _select(self, fp8_tensor_type, meta_tensor_type):
         """(flat tensor, first index, stride) of the E slots of this tensor type."""
         rule = _SLOT_RULES.get(int(fp8_tensor_type))

@@ -839,3 +839,55 @@ def test_fused_dgelu_backward_against_the_oracle(dev):
         assert_gemm_close(module.fc1_weight.grad[i], o["grad_w1"][0].float(), 1e-2, f"expert {i} grad_fc1")
         assert_gemm_close(module.fc2_weight.grad[i], o["grad_w2"][0].float(), 1e-2, f"expert {i} grad_fc2")
     assert not module.fc1_weight.grad[1].any() and not module.fc2_weight.grad[1].any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes,h,f,policy", [
+    ([700, 0, 33, 1291, 5, 256], 512, 768, 0), ([300], 4096, 7168, 256), ([0, 513, 90, 0], 4112, 2064, 256),
+    ([1, 0, 2] * 149 + [3], 64, 48, 0), ([128, 129, 0, 256, 257, 1], 272, 1408, 512), ([64] * 9 + [0], 256, 128, 128),
+    ([0, 0], 64, 64, 0)])
+def test_tables_built_on_the_device_are_those_of_the_host_planner(dev, sizes, h, f, policy):
+    """fp8gmm_build_pass writes a pass's tables into device memory from a kernel argument: descriptors, problem tables,
+    work lists and shared-tile records must be the host planner's, byte for byte, at the same offsets, and nothing else
+    may be written (all tile forms, tiles shared along K, experts without rows, as many experts as an argument holds)."""
+    import ctypes
+
+    import numpy as np
+
+    from fp8_gmm_amd import _lib
+
+    L = _lib.load()
+    e, gs = len(sizes), np.asarray(sizes, dtype=np.int64)
+    address = iter(range(1 << 40, 1 << 45, 1 << 38))    # never followed: tables hold addresses only
+    common = dict(experts=e, fwd_fmt=_lib.E4M3, bwd_fmt=_lib.E5M2, cast_weights=1, dgrad=1, wgrad=1, stream_k=1,
+                  grid=_lib.gemm_grid(_lib.init(torch.cuda.current_device())), tile_policy=policy, tokens=sum(sizes),
+                  group_sizes=gs.ctypes.data)
+    linear = _lib.LinearPass(in_features=h, out_features=f, **common,
+                             **{n: next(address) for n, _ in _lib.LinearPass._fields_[14:]})
+    mlp = _lib.MlpPass(hidden=h, ffn=f, **common, **{n: next(address) for n, _ in _lib.MlpPass._fields_[14:]})
+    src = torch.arange(5, dtype=torch.float32, device=dev)
+    for which, desc, host in ((_lib.LINEAR_FORWARD, linear, L.fp8gmm_plan_linear_forward),
+                              (_lib.LINEAR_BACKWARD, linear, L.fp8gmm_plan_linear_backward),
+                              (_lib.MLP_FORWARD, mlp, L.fp8gmm_plan_mlp_forward),
+                              (_lib.MLP_BACKWARD, mlp, L.fp8gmm_plan_mlp_backward)):
+        blob, want, plan = np.zeros(1 << 25, dtype=np.uint8), _lib.PassPlan(), _lib.PassPlan()
+        _lib.check(host(ctypes.byref(desc), blob.ctypes.data, blob.nbytes, ctypes.byref(want)))
+        tables = _lib.PassTables()
+        _lib.check(L.fp8gmm_lay_out_pass(which, ctypes.byref(desc), ctypes.byref(plan), tables))
+        assert bytes(plan) == bytes(want)
+        dst = torch.zeros(6, device=dev)
+        out = torch.full((plan.blob_bytes + 4096,), 0xAB, dtype=torch.uint8, device=dev)
+        _lib.check(L.fp8gmm_build_pass(tables, out.data_ptr(), src.data_ptr(), dst.data_ptr(), 5,
+                                       torch.cuda.current_stream(dev).cuda_stream))
+        got = out.cpu().numpy()
+        used = np.zeros(got.size, dtype=bool)
+        for i in range(plan.n_launches):
+            rec = plan.launch[i]
+            parts = [(rec.table_offset, rec.n * (96 if rec.plan.tile else 128))]
+            if rec.plan.tile:
+                parts += [(rec.items_offset, rec.plan.rounds * rec.plan.grid * 64), (rec.fixups_offset, rec.plan.n_fixups * 32)]
+            for off, nbytes in parts:
+                assert np.array_equal(got[off: off + nbytes], blob[off: off + nbytes]), f"pass {which} launch {i}"
+                used[off: off + nbytes] = True
+        assert np.all(got[~used] == 0xAB)
+        assert dst.tolist() == [0.0, 1.0, 2.0, 3.0, 4.0, 0.0]
