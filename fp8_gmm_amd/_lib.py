@@ -175,7 +175,7 @@ class PassPlan(ctypes.Structure):
 PASS_CAST = 1
 PASS_GEMM = 2
 LINEAR_FORWARD, LINEAR_BACKWARD, MLP_FORWARD, MLP_BACKWARD = range(4)
-PASS_MAX_EXPERTS = 448
+PASS_MAX_EXPERTS = 384
 PASS_MAX_GRID = 512
 PassTables = ctypes.c_uint64 * (4032 // 8)   # FP8GMM_PASS_TABLES_BYTES, opaque
 
@@ -310,7 +310,7 @@ def load():
     L.fp8gmm_lay_out_pass.restype = ci
     L.fp8gmm_lay_out_pass.argtypes = [ci, vp, ctypes.POINTER(PassPlan), vp]
     L.fp8gmm_build_pass.restype = ci
-    L.fp8gmm_build_pass.argtypes = [vp, vp, vp, vp, ci, vp]
+    L.fp8gmm_build_pass.argtypes = [vp, vp, ctypes.POINTER(ScalingUpdate), ci, vp, vp, ci, vp]
     L.fp8gmm_run_planned.restype = ci
     L.fp8gmm_run_planned.argtypes = [vp, ctypes.POINTER(PassLaunch), vp, ctypes.c_size_t, vp]
     L.fp8gmm_sizeof_linear_pass.restype = ctypes.c_size_t
@@ -442,6 +442,17 @@ def init(device_index):
 
 def gemm_grid(num_cu):
     return load().fp8gmm_gemm_grid(num_cu)
+
+
+_grids = {}
+
+
+def device_grid(device_index):
+    """Workgroups of a grouped-GEMM launch on a device (looked up once per device)."""
+    grid = _grids.get(device_index)
+    if grid is None:
+        grid = _grids[device_index] = gemm_grid(init(device_index))
+    return grid
 
 
 def gemm_schedule(table, total_tiles, grid, stream_k, wg, max_items=4096):

@@ -854,6 +854,7 @@ class GemmOptions:
 
 
 options = GemmOptions()
+TILE_POLICIES = {"auto": 0, "256": 256, "128": 128, "dual": _lib.GEMM_TILE_DUAL}
 
 
 @contextlib.contextmanager
@@ -971,7 +972,7 @@ def _run_pass(device, which, desc, fields, snapshot, host_planned):
     grid = _lib.gemm_grid(_lib.init(index))
     desc.grid = grid
     desc.stream_k = int(bool(options.stream_k))
-    desc.tile_policy = {"auto": 0, "256": 256, "128": 128, "dual": _lib.GEMM_TILE_DUAL}[options.tile]
+    desc.tile_policy = TILE_POLICIES[options.tile]
     plan = _lib.PassPlan()
     if desc.experts <= _lib.PASS_MAX_EXPERTS and 2 * grid <= _lib.PASS_MAX_GRID:
         tables = _lib.PassTables()
@@ -980,7 +981,7 @@ def _run_pass(device, which, desc, fields, snapshot, host_planned):
             blob = torch.empty(plan.blob_bytes, dtype=torch.uint8, device=device)
             src, dst = snapshot if snapshot is not None else (None, None)
             n = src.numel() if src is not None else 0
-            _lib.check(L.fp8gmm_build_pass(tables, blob.data_ptr(), src.data_ptr() if n else None,
+            _lib.check(L.fp8gmm_build_pass(tables, blob.data_ptr(), None, 0, src.data_ptr() if n else None,
                                            dst.data_ptr() if n else None, n, _stream(device)))
     else:
         blob = _plan_on_host(device, desc, plan, *host_planned, grid)

@@ -1,0 +1,378 @@
+// The host path of the modules in native code: one call from Python per forward pass, none per backward pass.
+//
+// A pass of a small layer is bound by its host: its kernels take 50 us, and the Python that allocated its tensors, filled
+// the C structures and walked through two autograd functions took 250 - 350 (the backward half of it in the autograd
+// engine's thread, where the interpreter's data is cold).  Here a pass is: allocate the results, describe the pass
+// (fp8gmm_lay_out_pass), enqueue the kernel that builds its tables, enqueue its launches; the backward pass is a node of
+// the autograd graph that does the same without entering the interpreter.
+//
+// What a pass computes is stated in fp8gmm.h and grouped_linear.py / grouped_mlp.py (reference fp8_gmm/grouped_linear.py:11-183,
+// fp8_gmm/grouped_mlp.py:18-325); the Python functions there launch the same kernels with the same tables and serve
+// the layouts and options that this file leaves to them.
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/utils/pybind.h>
+
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+
+#include "fp8gmm.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::Node;
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+
+void check(int status) { TORCH_CHECK(status == FP8GMM_OK, "fp8gmm error ", status, ": ", fp8gmm_status_string(status)); }
+
+void* current_stream(const at::Device& device) {
+  return c10::hip::getCurrentHIPStream(device.index()).stream();
+}
+
+template <class T>
+T* ptr(const Tensor& t) {
+  return t.defined() ? static_cast<T*>(t.data_ptr()) : nullptr;
+}
+
+// Rows per expert, from a CPU tensor or a sequence.
+std::vector<int64_t> sizes_of(const py::object& group_sizes) {
+  if (THPVariable_Check(group_sizes.ptr())) {
+    const Tensor t = THPVariable_Unpack(group_sizes.ptr()).to(at::kCPU, at::kLong).contiguous();
+    TORCH_CHECK(t.dim() == 1, "fp8_gmm_amd: group_sizes must be 1-D");
+    const int64_t* p = t.const_data_ptr<int64_t>();
+    return std::vector<int64_t>(p, p + t.numel());
+  }
+  return py::cast<std::vector<int64_t>>(group_sizes);
+}
+
+// How the launches of a module are planned, and its scaling state of both directions.
+struct Setup {
+  int fwd_fmt = 0, bwd_fmt = 0;
+  int grid = 0, stream_k = 0, tile_policy = 0;
+  Tensor fwd_scale, fwd_scale_inv, fwd_amax, bwd_scale, bwd_scale_inv, bwd_amax;
+  at::ScalarType fwd_type() const { return fwd_fmt == FP8GMM_E4M3 ? at::kFloat8_e4m3fn : at::kFloat8_e5m2; }
+  at::ScalarType bwd_type() const { return bwd_fmt == FP8GMM_E4M3 ? at::kFloat8_e4m3fn : at::kFloat8_e5m2; }
+};
+
+// The scaling update that is due in front of a pass.
+struct Due {
+  bool due = false;
+  double fwd_max = 0, bwd_max = 0;
+  int margin = 0;
+  bool most_recent = false, keep_weights = false;
+};
+
+// Builds the tables of a pass and enqueues its launches on the current stream.
+void run_pass(int which, const void* desc, const at::Device& device, const Setup* update, const Due* due, const Tensor& snapshot_of,
+              const Tensor& snapshot) {
+  fp8gmm_pass_plan plan;
+  alignas(16) unsigned char tables[FP8GMM_PASS_TABLES_BYTES];
+  check(fp8gmm_lay_out_pass(which, desc, &plan, tables));
+  const auto bytes = at::TensorOptions().dtype(at::kByte).device(device);
+  const Tensor blob = at::empty({plan.blob_bytes}, bytes);
+  void* const stream = current_stream(device);
+  fp8gmm_scaling_update updates[2] = {};
+  int n = 0;
+  if (due != nullptr && due->due) {
+    const Tensor* state[2][3] = {{&update->fwd_amax, &update->fwd_scale, &update->fwd_scale_inv},
+                                 {&update->bwd_amax, &update->bwd_scale, &update->bwd_scale_inv}};
+    for (n = 0; n < 2; ++n) {
+      fp8gmm_scaling_update& u = updates[n];
+      u.amax_history = ptr<float>(*state[n][0]);
+      u.scale = ptr<float>(*state[n][1]);
+      u.scale_inv = ptr<float>(*state[n][2]);
+      u.history_len = (int32_t)state[n][0]->size(0);
+      u.slots = (int32_t)state[n][0]->size(1);
+      u.fp8_max = (float)(n == 0 ? due->fwd_max : due->bwd_max);
+      u.margin = due->margin;
+      u.most_recent = due->most_recent;
+      if (n == 0 && due->keep_weights) {   // forward slots: input, weight, output
+        u.keep_period = 3;
+        u.keep_phase = 1;
+      }
+    }
+  }
+  check(fp8gmm_build_pass(tables, blob.data_ptr(), updates, n, ptr<const float>(snapshot_of), ptr<float>(snapshot),
+                          snapshot.defined() ? (int)snapshot.numel() : 0, stream));
+  int slots = 0;
+  for (int i = 0; i < plan.n_launches; ++i) slots = std::max(slots, plan.launch[i].plan.n_slots);
+  // partial sums of tiles shared along K: from the caching allocator, which hands memory out again in stream order
+  Tensor workspace;
+  if (slots > 0) workspace = at::empty({(int64_t)slots * FP8GMM_GEMM_SLOT_BYTES}, bytes);
+  for (int i = 0; i < plan.n_launches; ++i)
+    check(fp8gmm_run_planned(blob.data_ptr(), &plan.launch[i], ptr<void>(workspace),
+                             (size_t)slots * FP8GMM_GEMM_SLOT_BYTES, stream));
+}
+
+void check_rows(const std::vector<int64_t>& sizes, const Tensor& x) {
+  int64_t rows = 0;
+  for (const int64_t s : sizes) rows += s;
+  TORCH_CHECK(rows == x.size(0), "group_sizes must sum to the number of input rows");
+}
+
+// ---- GroupedLinear ------------------------------------------------------------------------------------------------
+fp8gmm_linear_pass linear_desc(const Setup& s, const std::vector<int64_t>& sizes, int64_t tokens, int64_t in, int64_t out) {
+  fp8gmm_linear_pass d{};
+  d.experts = (int32_t)sizes.size();
+  d.in_features = (int32_t)in;
+  d.out_features = (int32_t)out;
+  d.fwd_fmt = s.fwd_fmt;
+  d.bwd_fmt = s.bwd_fmt;
+  d.grid = s.grid;
+  d.stream_k = s.stream_k;
+  d.tile_policy = s.tile_policy;
+  d.tokens = tokens;
+  d.group_sizes = sizes.data();
+  return d;
+}
+
+struct GroupedLinearBackward : public Node {
+  Setup setup;
+  std::vector<int64_t> sizes;
+  int64_t in = 0, out = 0;
+  SavedVariable x_fp8, w_fp8;
+  Tensor scale_inv;   // the forward factors as they were
+
+  std::string name() const override { return "GroupedLinearBackward"; }
+  void release_variables() override {
+    x_fp8.reset_data();
+    w_fp8.reset_data();
+  }
+  variable_list apply(variable_list&& grads) override {
+    at::AutoGradMode no_grad(false);
+    variable_list result(2);
+    const bool dgrad = task_should_compute_output(0), wgrad = task_should_compute_output(1);
+    if (!grads[0].defined() || !(dgrad || wgrad)) return result;
+    const Tensor dy = grads[0].contiguous();
+    const c10::OptionalDeviceGuard guard(dy.device());
+    const Tensor x = wgrad ? x_fp8.unpack() : Tensor(), w = dgrad ? w_fp8.unpack() : Tensor();
+    const Tensor dy_fp8 = at::empty(dy.sizes(), dy.options().dtype(setup.bwd_type()));
+    if (dgrad) result[0] = at::empty({dy.size(0), in}, dy.options());
+    if (wgrad) result[1] = at::empty({(int64_t)sizes.size(), out, in}, dy.options());
+    fp8gmm_linear_pass d = linear_desc(setup, sizes, dy.size(0), in, out);
+    d.dgrad = dgrad;
+    d.wgrad = wgrad;
+    d.dy = ptr<void>(dy);
+    d.dy_fp8 = ptr<void>(dy_fp8);
+    d.x_fp8 = ptr<void>(x);
+    d.w_fp8 = ptr<void>(w);
+    d.dx = ptr<void>(result[0]);
+    d.dw = ptr<void>(result[1]);
+    d.fwd_scale_inv = ptr<float>(scale_inv);
+    d.bwd_scale = ptr<float>(setup.bwd_scale);
+    d.bwd_scale_inv = ptr<float>(setup.bwd_scale_inv);
+    d.bwd_amax = ptr<float>(setup.bwd_amax);
+    run_pass(FP8GMM_LINEAR_BACKWARD, &d, dy.device(), nullptr, nullptr, Tensor(), Tensor());
+    return result;
+  }
+};
+
+Tensor linear_step(const Tensor& x, const Tensor& w, const py::object& group_sizes, const std::optional<Tensor>& cached,
+                   bool cast_weights, const Setup& setup, const Due& due) {
+  std::vector<int64_t> sizes = sizes_of(group_sizes);
+  py::gil_scoped_release no_gil;
+  check_rows(sizes, x);
+  const c10::OptionalDeviceGuard guard(x.device());
+  const bool grad = at::GradMode::is_enabled();
+  const bool dgrad = grad && x.requires_grad(), wgrad = grad && w.requires_grad();
+  Tensor y, x_fp8, w_fp8, scale_inv;
+  {
+    at::AutoGradMode no_grad(false);
+    const auto fp8 = x.options().dtype(setup.fwd_type());
+    x_fp8 = at::empty(x.sizes(), fp8);
+    w_fp8 = cached.has_value() ? *cached : at::empty(w.sizes(), fp8);
+    y = at::empty({x.size(0), w.size(1)}, x.options());
+    if (dgrad || wgrad) scale_inv = at::empty_like(setup.fwd_scale_inv);
+    fp8gmm_linear_pass d = linear_desc(setup, sizes, x.size(0), w.size(2), w.size(1));
+    d.cast_weights = cast_weights;
+    d.x = ptr<void>(x);
+    d.x_fp8 = ptr<void>(x_fp8);
+    d.w = ptr<void>(w);
+    d.w_fp8 = ptr<void>(w_fp8);
+    d.y = ptr<void>(y);
+    d.fwd_scale = ptr<float>(setup.fwd_scale);
+    d.fwd_scale_inv = ptr<float>(setup.fwd_scale_inv);
+    d.fwd_amax = ptr<float>(setup.fwd_amax);
+    run_pass(FP8GMM_LINEAR_FORWARD, &d, x.device(), &setup, &due, scale_inv.defined() ? setup.fwd_scale_inv : Tensor(),
+             scale_inv);
+  }
+  if (dgrad || wgrad) {
+    auto node = std::shared_ptr<GroupedLinearBackward>(new GroupedLinearBackward(), torch::autograd::deleteNode);
+    node->set_next_edges(torch::autograd::collect_next_edges(x, w));
+    node->setup = setup;
+    node->sizes = std::move(sizes);
+    node->in = w.size(2);
+    node->out = w.size(1);
+    if (wgrad) node->x_fp8 = SavedVariable(x_fp8, false);
+    if (dgrad) node->w_fp8 = SavedVariable(w_fp8, false);
+    node->scale_inv = scale_inv;
+    torch::autograd::set_history(y, node);
+  }
+  return y;
+}
+
+// ---- GroupedMlp ---------------------------------------------------------------------------------------------------
+fp8gmm_mlp_pass mlp_desc(const Setup& s, const std::vector<int64_t>& sizes, int64_t tokens, int64_t hidden, int64_t ffn) {
+  fp8gmm_mlp_pass d{};
+  d.experts = (int32_t)sizes.size();
+  d.hidden = (int32_t)hidden;
+  d.ffn = (int32_t)ffn;
+  d.fwd_fmt = s.fwd_fmt;
+  d.bwd_fmt = s.bwd_fmt;
+  d.grid = s.grid;
+  d.stream_k = s.stream_k;
+  d.tile_policy = s.tile_policy;
+  d.tokens = tokens;
+  d.group_sizes = sizes.data();
+  return d;
+}
+
+struct GroupedMlpBackward : public Node {
+  Setup setup;
+  std::vector<int64_t> sizes;
+  bool dgrad = false, wgrad = false;
+  int64_t hidden = 0, ffn = 0;
+  SavedVariable x_fp8, w1_fp8, w2_fp8, pre, act_fp8;
+  Tensor scale_inv;
+
+  std::string name() const override { return "GroupedMlpBackward"; }
+  void release_variables() override {
+    for (SavedVariable* v : {&x_fp8, &w1_fp8, &w2_fp8, &pre, &act_fp8}) v->reset_data();
+  }
+  variable_list apply(variable_list&& grads) override {
+    at::AutoGradMode no_grad(false);
+    variable_list result(3);
+    const bool want_x = dgrad && task_should_compute_output(0);
+    const bool want_w = wgrad && (task_should_compute_output(1) || task_should_compute_output(2));
+    if (!grads[0].defined() || !(want_x || want_w)) return result;
+    const Tensor dy = grads[0].contiguous();
+    const c10::OptionalDeviceGuard guard(dy.device());
+    const int64_t tokens = dy.size(0), e = (int64_t)sizes.size();
+    const auto bf16 = dy.options(), fp8 = dy.options().dtype(setup.bwd_type());
+    const Tensor p = pre.unpack(), w2 = w2_fp8.unpack(), w1 = want_x ? w1_fp8.unpack() : Tensor();
+    const Tensor x = want_w ? x_fp8.unpack() : Tensor(), act = want_w ? act_fp8.unpack() : Tensor();
+    const Tensor dy_fp8 = at::empty(dy.sizes(), fp8), dact = at::empty({tokens, ffn}, bf16), dpre = at::empty({tokens, ffn}, fp8);
+    if (want_x) result[0] = at::empty(dy.sizes(), bf16);
+    if (want_w) {
+      result[1] = at::empty({e, ffn, hidden}, bf16);
+      result[2] = at::empty({e, hidden, ffn}, bf16);
+    }
+    fp8gmm_mlp_pass d = mlp_desc(setup, sizes, tokens, hidden, ffn);
+    d.dgrad = want_x;
+    d.wgrad = want_w;
+    d.x_fp8 = ptr<void>(x);
+    d.w1_fp8 = ptr<void>(w1);
+    d.w2_fp8 = ptr<void>(w2);
+    d.pre = ptr<void>(p);
+    d.act_fp8 = ptr<void>(act);
+    d.dy = ptr<void>(dy);
+    d.dy_fp8 = ptr<void>(dy_fp8);
+    d.dact = ptr<void>(dact);
+    d.dpre_fp8 = ptr<void>(dpre);
+    d.dx = ptr<void>(result[0]);
+    d.dw1 = ptr<void>(result[1]);
+    d.dw2 = ptr<void>(result[2]);
+    d.fwd_scale_inv = ptr<float>(scale_inv);
+    d.bwd_scale = ptr<float>(setup.bwd_scale);
+    d.bwd_scale_inv = ptr<float>(setup.bwd_scale_inv);
+    d.bwd_amax = ptr<float>(setup.bwd_amax);
+    run_pass(FP8GMM_MLP_BACKWARD, &d, dy.device(), nullptr, nullptr, Tensor(), Tensor());
+    return result;
+  }
+};
+
+Tensor mlp_step(const Tensor& x, const Tensor& w1, const Tensor& w2, const py::object& group_sizes,
+                const std::optional<Tensor>& cached1, const std::optional<Tensor>& cached2, bool cast_weights,
+                const Setup& setup, const Due& due) {
+  std::vector<int64_t> sizes = sizes_of(group_sizes);
+  py::gil_scoped_release no_gil;
+  check_rows(sizes, x);
+  const c10::OptionalDeviceGuard guard(x.device());
+  const bool grad = at::GradMode::is_enabled();
+  const bool dgrad = grad && x.requires_grad(), wgrad = grad && w1.requires_grad();
+  const int64_t tokens = x.size(0), hidden = x.size(1), ffn = w1.size(1);
+  Tensor y, x_fp8, w1_fp8, w2_fp8, pre, act_fp8, scale_inv;
+  {
+    at::AutoGradMode no_grad(false);
+    const auto fp8 = x.options().dtype(setup.fwd_type());
+    x_fp8 = at::empty(x.sizes(), fp8);
+    w1_fp8 = cached1.has_value() ? *cached1 : at::empty(w1.sizes(), fp8);
+    w2_fp8 = cached2.has_value() ? *cached2 : at::empty(w2.sizes(), fp8);
+    pre = at::empty({tokens, ffn}, x.options());
+    act_fp8 = at::empty({tokens, ffn}, fp8);
+    y = at::empty(x.sizes(), x.options());
+    if (dgrad || wgrad) scale_inv = at::empty_like(setup.fwd_scale_inv);
+    fp8gmm_mlp_pass d = mlp_desc(setup, sizes, tokens, hidden, ffn);
+    d.cast_weights = cast_weights;
+    d.x = ptr<void>(x);
+    d.x_fp8 = ptr<void>(x_fp8);
+    d.w1 = ptr<void>(w1);
+    d.w1_fp8 = ptr<void>(w1_fp8);
+    d.w2 = ptr<void>(w2);
+    d.w2_fp8 = ptr<void>(w2_fp8);
+    d.pre = ptr<void>(pre);
+    d.act_fp8 = ptr<void>(act_fp8);
+    d.y = ptr<void>(y);
+    d.fwd_scale = ptr<float>(setup.fwd_scale);
+    d.fwd_scale_inv = ptr<float>(setup.fwd_scale_inv);
+    d.fwd_amax = ptr<float>(setup.fwd_amax);
+    run_pass(FP8GMM_MLP_FORWARD, &d, x.device(), &setup, &due, scale_inv.defined() ? setup.fwd_scale_inv : Tensor(),
+             scale_inv);
+  }
+  if (dgrad || wgrad) {
+    auto node = std::shared_ptr<GroupedMlpBackward>(new GroupedMlpBackward(), torch::autograd::deleteNode);
+    node->set_next_edges(torch::autograd::collect_next_edges(x, w1, w2));
+    node->setup = setup;
+    node->sizes = std::move(sizes);
+    node->dgrad = dgrad;
+    node->wgrad = wgrad;
+    node->hidden = hidden;
+    node->ffn = ffn;
+    node->pre = SavedVariable(pre, false);
+    node->w2_fp8 = SavedVariable(w2_fp8, false);
+    if (dgrad) node->w1_fp8 = SavedVariable(w1_fp8, false);
+    if (wgrad) {
+      node->x_fp8 = SavedVariable(x_fp8, false);
+      node->act_fp8 = SavedVariable(act_fp8, false);
+    }
+    node->scale_inv = scale_inv;
+    torch::autograd::set_history(y, node);
+  }
+  return y;
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_host, m) {
+  m.doc() = "Host path of the grouped modules in native code (see host_passes.cpp).";
+  py::class_<Setup>(m, "Setup")
+      .def(py::init([](int fwd_fmt, int bwd_fmt, int grid, const Tensor& fs, const Tensor& fsi, const Tensor& fa,
+                       const Tensor& bs, const Tensor& bsi, const Tensor& ba) {
+        Setup s;
+        s.fwd_fmt = fwd_fmt;
+        s.bwd_fmt = bwd_fmt;
+        s.grid = grid;
+        s.fwd_scale = fs;
+        s.fwd_scale_inv = fsi;
+        s.fwd_amax = fa;
+        s.bwd_scale = bs;
+        s.bwd_scale_inv = bsi;
+        s.bwd_amax = ba;
+        return s;
+      }))
+      .def_readonly("fwd_fmt", &Setup::fwd_fmt)
+      .def_readwrite("stream_k", &Setup::stream_k)
+      .def_readwrite("tile_policy", &Setup::tile_policy);
+  py::class_<Due>(m, "Due")
+      .def(py::init<>())
+      .def(py::init([](double fwd_max, double bwd_max, int margin, bool most_recent, bool keep_weights) {
+        return Due{true, fwd_max, bwd_max, margin, most_recent, keep_weights};
+      }));
+  m.def("linear_step", &linear_step);
+  m.def("mlp_step", &mlp_step);
+}

@@ -28,8 +28,9 @@ struct PassTables;
 int plan_gemm_ranges(fp8gmm_gemm_problem* probs, int n, int layout, int grid, int stream_k, fp8gmm_gemm_plan* plan,
                      GemmRanges* out);
 
-// Writes the tables of a pass into device memory (pass_tables.hip), and copies `copy_n` floats on the side.
-int launch_pass_tables(const PassTables& tables, void* blob_dev, const float* copy_src, float* copy_dst, int copy_n,
-                       void* stream);
+// Writes the tables of a pass into device memory, runs up to two scaling updates and copies `copy_n` floats on the
+// side, in one launch (pass_tables.hip).
+int launch_pass_tables(const PassTables& tables, void* blob_dev, const fp8gmm_scaling_update* updates, int n_updates,
+                       const float* copy_src, float* copy_dst, int copy_n, void* stream);
 
 }  // namespace fp8gmm

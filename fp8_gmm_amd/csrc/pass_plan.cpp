@@ -545,12 +545,13 @@ int fp8gmm_lay_out_pass(int which, const void* desc, fp8gmm_pass_plan* out, void
   return lay_out_pass(pass, out, static_cast<PassTables*>(tables));
 }
 
-int fp8gmm_build_pass(const void* tables, void* blob_dev, const float* copy_src, float* copy_dst, int copy_n, void* stream) {
+int fp8gmm_build_pass(const void* tables, void* blob_dev, const fp8gmm_scaling_update* updates, int n_updates,
+                      const float* copy_src, float* copy_dst, int copy_n, void* stream) {
   if (tables == nullptr || copy_n < 0 || (copy_n > 0 && (copy_src == nullptr || copy_dst == nullptr)))
     return FP8GMM_ERR_NULL_POINTER;
   const PassTables* t = static_cast<const PassTables*>(tables);
   if (t->blocks > 0 && blob_dev == nullptr) return FP8GMM_ERR_NULL_POINTER;
-  return fp8gmm::launch_pass_tables(*t, blob_dev, copy_src, copy_dst, copy_n, stream);
+  return fp8gmm::launch_pass_tables(*t, blob_dev, updates, n_updates, copy_src, copy_dst, copy_n, stream);
 }
 
 int fp8gmm_run_planned(const void* blob_dev, const fp8gmm_pass_launch* rec, void* workspace, size_t workspace_bytes,

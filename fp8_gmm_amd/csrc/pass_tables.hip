@@ -17,6 +17,7 @@
 #include "device_utils.h"
 #include "internal.h"
 #include "pass_spec.h"
+#include "scaling_update.h"
 
 namespace fp8gmm {
 namespace {
@@ -243,9 +244,19 @@ __device__ void write_gemm(const PassTables& t, int g, int block, uint8_t* blob,
   reinterpret_cast<fp8gmm_gemm_item*>(blob + spec.items_offset)[index] = o;
 }
 
+constexpr int kUpdates = 2;   // a module's two directions
+static_assert(sizeof(PassTables) + sizeof(ScalingUpdatesOf<kUpdates>) + 64 <= 4096, "kernel arguments");
+static_assert(kScalingThreads == kThreads, "one launch");
+
+// Workgroups: the tables', one for the copy on the side if there is one, then the scaling updates'.
 __global__ __launch_bounds__(kThreads) void pass_tables_kernel(const PassTables argument, uint8_t* __restrict__ blob,
                                                                const float* __restrict__ copy_src,
-                                                               float* __restrict__ copy_dst, int copy_n) {
+                                                               float* __restrict__ copy_dst, int copy_n,
+                                                               const ScalingUpdatesOf<kUpdates> updates, int update_block) {
+  if ((int)blockIdx.x >= update_block) {
+    run_scaling_update(updates, (int)blockIdx.x - update_block);
+    return;
+  }
   __shared__ fp8gmm_gemm_problem probs[kExperts];
   __shared__ int row_begin[kExperts + 1], begin[kExperts + 1], cost[kExperts + 1];
   __shared__ int slots[FP8GMM_PASS_MAX_GRID + 1];
@@ -284,12 +295,23 @@ __global__ __launch_bounds__(kThreads) void pass_tables_kernel(const PassTables 
 
 }  // namespace
 
-int launch_pass_tables(const PassTables& tables, void* blob_dev, const float* copy_src, float* copy_dst, int copy_n,
-                       void* stream) {
-  const int blocks = tables.blocks + (copy_n > 0 ? 1 : 0);
+int launch_pass_tables(const PassTables& tables, void* blob_dev, const fp8gmm_scaling_update* updates, int n_updates,
+                       const float* copy_src, float* copy_dst, int copy_n, void* stream) {
+  ScalingUpdatesOf<kUpdates> all;
+  const int rc = collect_scaling_updates(updates, n_updates, &all);
+  if (rc != FP8GMM_OK) return rc;
+  // a copy of what an update is about to write is made by that update
+  for (int i = 0; i < all.n && copy_n > 0; ++i)
+    if (all.u[i].scale_inv == copy_src) {
+      if (copy_n != all.u[i].slots) return FP8GMM_ERR_BAD_ARGUMENT;
+      all.snapshot[i] = copy_dst;
+      copy_n = 0;
+    }
+  const int update_block = tables.blocks + (copy_n > 0 ? 1 : 0);
+  const int blocks = update_block + all.first_block[all.n];
   if (blocks == 0) return FP8GMM_OK;
   hipLaunchKernelGGL(pass_tables_kernel, dim3(blocks), dim3(kThreads), 0, static_cast<hipStream_t>(stream), tables,
-                     static_cast<uint8_t*>(blob_dev), copy_src, copy_dst, copy_n);
+                     static_cast<uint8_t*>(blob_dev), copy_src, copy_dst, copy_n, all, update_block);
   return hipGetLastError() == hipSuccess ? FP8GMM_OK : FP8GMM_ERR_LAUNCH;
 }
 

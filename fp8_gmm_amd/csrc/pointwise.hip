@@ -9,6 +9,7 @@
 // workgroup issues a single integer atomic max.
 #include "device_utils.h"
 #include "internal.h"
+#include "scaling_update.h"
 #include "tiling.h"
 
 namespace fp8gmm {
@@ -151,95 +152,16 @@ __global__ __launch_bounds__(kPwThreads) void multi_scale_mul_kernel(const fp8gm
   }
 }
 
-// Delayed-scaling update of one direction.  Columns of the [history, slots] amax matrix are independent:
-//   amax      = max over the history column (or its row 0)
-//   scale     = (1 / amax) * fp8_max * 2^-margin   where amax is finite and > 0, else unchanged
-//   scale_inv = 1 / scale, except in slots with slot % keep_period == keep_phase (keep_period > 0): those
-//               keep their value, for tensors whose fp8 copy from an earlier pass is still in use
-//   history   : row i <- row i + 1, last row <- old row 0, then row 0 <- 0 (a history of one row is just cleared)
-// The factor is formed as reciprocal times fp8_max, which is what `fp8_max / amax` on a torch tensor
-// evaluates to; the two differ in the last bit for some inputs.
-//
-// Bound: latency.  The default recipe keeps 1024 rows; a module of 128 expert MLPs then has 1280 columns, 5 MB to
-// read and to write, a few microseconds of memory traffic.  With one lane per column the rows are a chain of dependent
-// round trips (61 us for 20 columns, 111 us for 1280 with the rows read eight at a time).  Here a workgroup owns
-// kScalingCols neighbouring columns (one 64-byte piece of every row) and moves kScalingRows rows at once: every lane
-// has its sixteen rows in flight together, all of them are read before the barrier and written one place up behind it, so the
-// shift can be done in place; longer histories take the next rows in turn.  A workgroup per column piece and not per
-// row range: the row that one range writes is the row its neighbour still has to read.
-constexpr int kScalingCols = 16;
-constexpr int kScalingThreads = 1024;
-constexpr int kScalingLanes = kScalingThreads / kScalingCols;   // rows side by side: 64
-constexpr int kScalingPerLane = 16;
-constexpr int kScalingRows = kScalingLanes * kScalingPerLane;   // 1024
-
-// torch.max semantics: a NaN anywhere in the column wins
-__device__ __forceinline__ float history_max(float a, float b) { return (b > a || b != b) ? b : a; }
-
-__device__ __forceinline__ void delayed_scaling_update_columns(float* __restrict__ history, float* __restrict__ scale,
-                                                                float* __restrict__ scale_inv, int history_len, int slots,
-                                                                float fp8_max, float margin_factor, int most_recent,
-                                                                int keep_period, int keep_phase, int c0) {
-  __shared__ float stage[kScalingThreads / kWaveSize][kScalingCols];
-  const int lane_col = threadIdx.x % kScalingCols, lane_row = threadIdx.x / kScalingCols;
-  const int c = c0 + lane_col;
-  const bool live = c < slots;
-  float* col = history + c;
-  const float first = live ? col[0] : 0.f;
-  float amax = first;
-  for (int base = 0; base < history_len; base += kScalingRows) {
-    float v[kScalingPerLane];
-#pragma unroll
-    for (int j = 0; j < kScalingPerLane; ++j) {
-      const int r = base + j * kScalingLanes + lane_row;
-      v[j] = live && r < history_len ? col[(size_t)r * slots] : 0.f;   // 0 never raises a maximum of magnitudes
-    }
-#pragma unroll
-    for (int j = 0; j < kScalingPerLane; ++j) amax = history_max(amax, v[j]);
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < kScalingPerLane; ++j) {
-      const int r = base + j * kScalingLanes + lane_row;
-      if (live && r >= 2 && r < history_len) col[(size_t)(r - 1) * slots] = v[j];
-    }
-  }
-  // lanes 16 apart hold the same column
-  for (int off = kScalingCols; off < kWaveSize; off <<= 1) amax = history_max(amax, __shfl_xor(amax, off));
-  if (threadIdx.x % kWaveSize < kScalingCols) stage[threadIdx.x / kWaveSize][lane_col] = amax;
-  __syncthreads();   // (the last rows have been read by now, too: the row written below is one of them)
-  if (threadIdx.x >= kScalingCols || !live) return;
-  for (int w = 1; w < kScalingThreads / kWaveSize; ++w) amax = history_max(amax, stage[w][lane_col]);
-  if (most_recent) amax = first;
-  float sc = scale[c];
-  if (amax > 0.f && amax <= 3.4028234663852886e38f) sc = ((1.0f / amax) * fp8_max) * margin_factor;
-  scale[c] = sc;
-  if (!(keep_period > 0 && c % keep_period == keep_phase)) scale_inv[c] = 1.0f / sc;
-  if (history_len > 1) col[(size_t)(history_len - 1) * slots] = first;
-  col[0] = 0.f;
-}
-
 __global__ __launch_bounds__(kScalingThreads) void delayed_scaling_update_kernel(
     float* __restrict__ history, float* __restrict__ scale, float* __restrict__ scale_inv, int history_len, int slots,
     float fp8_max, float margin_factor, int most_recent, int keep_period, int keep_phase) {
   delayed_scaling_update_columns(history, scale, scale_inv, history_len, slots, fp8_max, margin_factor, most_recent,
-                                 keep_period, keep_phase, (int)blockIdx.x * kScalingCols);
+                                 keep_period, keep_phase, nullptr, (int)blockIdx.x * kScalingCols);
 }
 
-// Several directions (a module's forward and backward scaling state) in one launch: the workgroups of update u
-// follow those of update u - 1.  The updates travel as a kernel argument.
-struct ScalingUpdates {
-  fp8gmm_scaling_update u[FP8GMM_MAX_SCALING_UPDATES];
-  float margin_factor[FP8GMM_MAX_SCALING_UPDATES];
-  int first_block[FP8GMM_MAX_SCALING_UPDATES + 1];
-  int n;
-};
+// Several directions in one launch
 __global__ __launch_bounds__(kScalingThreads) void delayed_scaling_updates_kernel(const ScalingUpdates all) {
-  int i = 0;
-  while (i + 1 < all.n && (int)blockIdx.x >= all.first_block[i + 1]) ++i;
-  const fp8gmm_scaling_update& u = all.u[i];
-  delayed_scaling_update_columns(u.amax_history, u.scale, u.scale_inv, u.history_len, u.slots, u.fp8_max,
-                                 all.margin_factor[i], u.most_recent, u.keep_period, u.keep_phase,
-                                 ((int)blockIdx.x - all.first_block[i]) * kScalingCols);
+  run_scaling_update(all, (int)blockIdx.x);
 }
 
 }  // namespace
@@ -288,7 +210,7 @@ extern "C" {
 int fp8gmm_delayed_scaling_update(float* amax_history, float* scale, float* scale_inv, int history_len, int slots,
                                   float fp8_max, int margin, int most_recent, int keep_period, int keep_phase,
                                   void* stream) {
-  if (history_len < 1 || slots < 0 || margin < -126 || margin > 126) return FP8GMM_ERR_BAD_ARGUMENT;
+  if (history_len < 1 || slots < 0 || slots > (1 << 20) - 1 || margin < -126 || margin > 126) return FP8GMM_ERR_BAD_ARGUMENT;
   if (keep_period < 0 || (keep_period > 0 && (keep_phase < 0 || keep_phase >= keep_period)))
     return FP8GMM_ERR_BAD_ARGUMENT;
   if (slots == 0) return FP8GMM_OK;
@@ -301,27 +223,10 @@ int fp8gmm_delayed_scaling_update(float* amax_history, float* scale, float* scal
 }
 
 int fp8gmm_delayed_scaling_updates(const fp8gmm_scaling_update* updates, int n, void* stream) {
-  if (n < 0 || n > FP8GMM_MAX_SCALING_UPDATES) return FP8GMM_ERR_BAD_ARGUMENT;
-  if (n == 0) return FP8GMM_OK;
-  if (updates == nullptr) return FP8GMM_ERR_NULL_POINTER;
-  fp8gmm::ScalingUpdates all{};
-  int blocks = 0;
-  for (int i = 0; i < n; ++i) {
-    const fp8gmm_scaling_update& u = updates[i];
-    if (u.history_len < 1 || u.slots < 0 || u.margin < -126 || u.margin > 126) return FP8GMM_ERR_BAD_ARGUMENT;
-    if (u.keep_period < 0 || (u.keep_period > 0 && (u.keep_phase < 0 || u.keep_phase >= u.keep_period)))
-      return FP8GMM_ERR_BAD_ARGUMENT;
-    if (u.slots > 0 && (u.amax_history == nullptr || u.scale == nullptr || u.scale_inv == nullptr))
-      return FP8GMM_ERR_NULL_POINTER;
-    all.u[i] = u;
-    all.margin_factor[i] = __builtin_ldexpf(1.0f, -u.margin);
-    all.first_block[i] = blocks;
-    blocks += (u.slots + fp8gmm::kScalingCols - 1) / fp8gmm::kScalingCols;
-  }
-  all.first_block[n] = blocks;
-  all.n = n;
-  if (blocks == 0) return FP8GMM_OK;
-  hipLaunchKernelGGL(fp8gmm::delayed_scaling_updates_kernel, dim3(blocks), dim3(fp8gmm::kScalingThreads), 0,
+  fp8gmm::ScalingUpdates all;
+  const int rc = fp8gmm::collect_scaling_updates(updates, n, &all);
+  if (rc != FP8GMM_OK || all.first_block[all.n] == 0) return rc;
+  hipLaunchKernelGGL(fp8gmm::delayed_scaling_updates_kernel, dim3(all.first_block[all.n]), dim3(fp8gmm::kScalingThreads), 0,
                      static_cast<hipStream_t>(stream), all);
   return hipGetLastError() == hipSuccess ? FP8GMM_OK : FP8GMM_ERR_LAUNCH;
 }

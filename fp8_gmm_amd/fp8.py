@@ -89,16 +89,20 @@ class _State(threading.local):
 _STATE = _State()
 
 
-@contextlib.contextmanager
-def fp8_autocast(enabled=True, fp8_recipe=None):
+class fp8_autocast(contextlib.ContextDecorator):  # noqa: N801 - TransformerEngine's spelling
     """Selects the recipe used by modules called inside the block."""
-    prev = (_STATE.enabled, _STATE.recipe)
-    _STATE.enabled = enabled
-    _STATE.recipe = (fp8_recipe or DelayedScaling()) if enabled else None
-    try:
-        yield
-    finally:
-        _STATE.enabled, _STATE.recipe = prev
+
+    def __init__(self, enabled=True, fp8_recipe=None):
+        self.enabled, self.recipe = enabled, (fp8_recipe or DelayedScaling()) if enabled else None
+        self.outer = []
+
+    def __enter__(self):
+        self.outer.append((_STATE.enabled, _STATE.recipe))
+        _STATE.enabled, _STATE.recipe = self.enabled, self.recipe
+
+    def __exit__(self, *exc):
+        _STATE.enabled, _STATE.recipe = self.outer.pop()
+        return False
 
 
 def current_recipe():
@@ -172,6 +176,15 @@ class Fp8WeightCache:
             self.valid_t = False
         return self.fp8, self.fp8_t
 
+    def take(self, weight, setup, refresh):
+        """The row-major buffer for a pass that casts into it (``refresh``) or reuses it."""
+        fp8, _ = self.buffers(weight, torch.float8_e4m3fn if setup.fwd_fmt == 0 else torch.float8_e5m2, False)
+        if refresh:
+            self.valid, self.valid_t = True, False
+        else:
+            self.require(False)
+        return fp8
+
     def require(self, transposed):
         if not self.valid or (transposed and not self.valid_t):
             raise RuntimeError(
@@ -225,28 +238,82 @@ class Fp8GroupedModuleBase(torch.nn.Module):
         update of both directions, every ``recipe.interval`` passes.  ``is_first_microbatch=False``
         (cached fp8 weights are reused) keeps the weights' ``scale_inv`` out of that update.
         """
-        update_weights = is_first_microbatch is None or bool(is_first_microbatch)
+        self._run_update(self._prepare(inp.device, is_first_microbatch, num_gemms))
+        yield
+
+    def _prepare(self, device, is_first_microbatch, num_gemms):
+        """``prepare_forward`` without the scaling update, of which it returns whether one is due, and whether the
+        weights' ``scale_inv`` stays out of it: None or ``(keep_weights,)``."""
         fp8_recipe = current_recipe() or self.fp8_meta.get("recipe") or DelayedScaling()
-        self._init_fp8_meta(fp8_recipe, num_gemms, inp.device)
+        self._init_fp8_meta(fp8_recipe, num_gemms, device)
         self._apply_pending_state()
+        due = None
         if self.training and torch.is_grad_enabled():
             if self._fp8_steps > 0 and self._fp8_steps % fp8_recipe.interval == 0:
-                fwd, bwd = self.fp8_meta["scaling_fwd"], self.fp8_meta["scaling_bwd"]
-                keep = None if update_weights else (self.FWD_SLOTS_PER_GEMM, self.WEIGHT_SLOT)
-                with torch.no_grad():
-                    if fwd.amax_history.is_cuda and float(fp8_recipe.margin) == int(fp8_recipe.margin):
-                        # both directions in one kernel launch (the rule is amax_and_scale_update's)
-                        from . import backend
-
-                        margin, recent = int(fp8_recipe.margin), fp8_recipe.amax_compute_algo != "max"
-                        backend.delayed_scaling_updates([
-                            (fwd.amax_history, fwd.scale, fwd.scale_inv, self.fp8_meta["fp8_max_fwd"], margin, recent, keep),
-                            (bwd.amax_history, bwd.scale, bwd.scale_inv, self.fp8_meta["fp8_max_bwd"], margin, recent)])
-                    else:
-                        amax_and_scale_update(fwd, self.fp8_meta["fp8_max_fwd"], fp8_recipe, keep)
-                        amax_and_scale_update(bwd, self.fp8_meta["fp8_max_bwd"], fp8_recipe)
+                due = (is_first_microbatch is not None and not is_first_microbatch,)
             self._fp8_steps += 1
-        yield
+        return due
+
+    def _run_update(self, due):
+        """The scaling update of both directions that ``_prepare`` found due."""
+        if due is None:
+            return
+        fp8_recipe = self.fp8_meta["recipe"]
+        fwd, bwd = self.fp8_meta["scaling_fwd"], self.fp8_meta["scaling_bwd"]
+        keep = (self.FWD_SLOTS_PER_GEMM, self.WEIGHT_SLOT) if due[0] else None
+        with torch.no_grad():
+            if fwd.amax_history.is_cuda and float(fp8_recipe.margin) == int(fp8_recipe.margin):
+                # both directions in one kernel launch (the rule is amax_and_scale_update's)
+                from . import backend
+
+                margin, recent = int(fp8_recipe.margin), fp8_recipe.amax_compute_algo != "max"
+                backend.delayed_scaling_updates([
+                    (fwd.amax_history, fwd.scale, fwd.scale_inv, self.fp8_meta["fp8_max_fwd"], margin, recent, keep),
+                    (bwd.amax_history, bwd.scale, bwd.scale_inv, self.fp8_meta["fp8_max_bwd"], margin, recent)])
+            else:
+                amax_and_scale_update(fwd, self.fp8_meta["fp8_max_fwd"], fp8_recipe, keep)
+                amax_and_scale_update(bwd, self.fp8_meta["fp8_max_bwd"], fp8_recipe)
+
+    def _native(self, input, *weights):
+        """Whether a pass on these tensors can take the native host path: the default layout and options, planned
+        passes, nothing that looks at the launches one by one."""
+        from . import _lib, backend
+
+        meta = self.fp8_meta
+        if not (meta["planned_passes"] and not meta["reference_layout"] and backend.kernel_timing._active is None
+                and backend.options.wgrad == "in_place" and self.num_groups <= _lib.PASS_MAX_EXPERTS
+                and getattr(backend._pending, "items", None) is None):
+            return False
+        if not (input.is_cuda and input.dtype == torch.bfloat16 and input.dim() == 2 and input.is_contiguous()):
+            return False
+        for w in weights:
+            if not (w.dtype == torch.bfloat16 and w.is_contiguous() and w.device == input.device
+                    and w.size(1) % 16 == 0 and w.size(2) % 16 == 0):
+                return False
+        return float(meta["recipe"].margin) == int(meta["recipe"].margin)
+
+    def _native_setup(self, device):
+        """The module's scaling state and the launch policy in force, as the native host path takes them."""
+        from . import _lib, backend
+        from .native import Setup
+
+        meta = self.fp8_meta
+        fwd, bwd, r = meta["scaling_fwd"], meta["scaling_bwd"], meta["recipe"]
+        setup = Setup(0 if get_fp8_te_dtype(r, True) == DType.kFloat8E4M3 else 1,
+                      0 if get_fp8_te_dtype(r, False) == DType.kFloat8E4M3 else 1, _lib.device_grid(device.index),
+                      fwd.scale, fwd.scale_inv, fwd.amax_history, bwd.scale, bwd.scale_inv, bwd.amax_history)
+        setup.stream_k = int(bool(backend.options.stream_k))
+        setup.tile_policy = backend.TILE_POLICIES[backend.options.tile]
+        return setup
+
+    def _native_due(self, due):
+        from .native import Due
+
+        if due is None:
+            return Due()
+        meta = self.fp8_meta
+        r = meta["recipe"]
+        return Due(meta["fp8_max_fwd"], meta["fp8_max_bwd"], int(r.margin), r.amax_compute_algo != "max", due[0])
 
     def _cast_ahead(self, weights_and_groups):
         """The part of a forward pass that needs no group sizes, run now: the delayed-scaling update and the cast of

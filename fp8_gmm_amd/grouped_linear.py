@@ -19,7 +19,6 @@ gradient is zero), wgrad is a single launch instead of a per-expert loop, and th
 grouped GEMM is the same HIP kernel whatever ``cutlass`` says (``cutlass=True`` keeps
 the two-rounding data flow of the reference's CUTLASS path, see ``backend.fp8_gmm``).
 """
-import contextlib
 import math
 
 import numpy as np
@@ -29,6 +28,7 @@ from . import _lib
 from .backend import (TensorBatch, batched_uploads, fp8_gmm, grouped_gemm, linear_pass, multi_cast_transpose,
                       multi_quantize, wgrad_wants_transposed_gradient)
 from .fp8 import Fp8GroupedModuleBase, Fp8WeightCache, get_fp8_te_dtype
+from .native import linear_step
 from .utils import PAD_MULTIPLE, Fp8MetaWrapper, Fp8TensorType, MetaTensorType, cumsum_group_sizes, to_torch_dtype
 
 
@@ -364,14 +364,25 @@ class GroupedLinear(Fp8GroupedModuleBase):
 
     def forward(self, input, group_sizes, is_first_microbatch=None):
         ahead = self._take_ahead(is_first_microbatch)
-        with (contextlib.nullcontext() if ahead is not None else
-              self.prepare_forward(input, is_first_microbatch, self.num_groups)):
-            grad = torch.is_grad_enabled()
-            args = (input, self.weight_tensor, group_sizes, self.fp8_meta, grad, self.cutlass)
-            if ahead is not None:
-                args += (ahead[0], False)
-            elif is_first_microbatch is not None:
-                args += (self._weight_cache, bool(is_first_microbatch))
-            if grad:
-                return _GroupedLinear.apply(*args)
-            return _GroupedLinear.forward(None, *args)
+        due = None
+        if ahead is None:
+            due = self._prepare(input.device, is_first_microbatch, self.num_groups)
+        # the fp8 weights: temporaries of the pass, or the buffers of a cache that the pass refreshes or reuses
+        cache, refresh = None, True
+        if ahead is not None:
+            cache, refresh = ahead[0], False
+        elif is_first_microbatch is not None:
+            cache, refresh = self._weight_cache, bool(is_first_microbatch)
+        weight = self.weight_tensor
+        if not self.cutlass and self._native(input, weight):
+            setup = self._native_setup(input.device)
+            held = cache.take(weight, setup, refresh) if cache is not None else None
+            return linear_step(input, weight, group_sizes, held, refresh, setup, self._native_due(due))
+        self._run_update(due)
+        grad = torch.is_grad_enabled()
+        args = (input, weight, group_sizes, self.fp8_meta, grad, self.cutlass)
+        if cache is not None:
+            args += (cache, refresh)
+        if grad:
+            return _GroupedLinear.apply(*args)
+        return _GroupedLinear.forward(None, *args)

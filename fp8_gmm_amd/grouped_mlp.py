@@ -21,7 +21,6 @@ Experts with zero tokens are allowed; each wgrad is one grouped launch.  In the 
 planned by one library call (``backend.mlp_pass``); the launch-by-launch code below it builds the same tables and
 serves the other layouts and options.
 """
-import contextlib
 import math
 
 import numpy as np
@@ -44,6 +43,7 @@ from .backend import (
 )
 from .fp8 import Fp8GroupedModuleBase, Fp8WeightCache, get_fp8_te_dtype
 from .grouped_linear import MODULE_PAD_MULTIPLE, alloc_transposed, row_slices, stage_weight_cast, transposed_views
+from .native import mlp_step
 from .utils import PAD_MULTIPLE, Fp8MetaWrapper, Fp8TensorType, MetaTensorType, cumsum_group_sizes, to_torch_dtype
 
 _T = Fp8TensorType
@@ -449,14 +449,26 @@ class GroupedMlp(Fp8GroupedModuleBase):
 
     def forward(self, input, group_sizes, has_tp=False, tp_group=None, is_first_microbatch=None):
         ahead = self._take_ahead(is_first_microbatch)
-        with (contextlib.nullcontext() if ahead is not None else
-              self.prepare_forward(input, is_first_microbatch, self.num_groups * 2)):
-            grad = torch.is_grad_enabled()
-            args = (input, self.fc1_weight, self.fc2_weight, group_sizes, self.fp8_meta, grad, has_tp, tp_group)
-            if ahead is not None:
-                args += (ahead, False)
-            elif is_first_microbatch is not None:
-                args += (tuple(self._weight_caches), bool(is_first_microbatch))
-            if grad:
-                return _GroupedMlp.apply(*args)
-            return _GroupedMlp.forward(None, *args)
+        due = None
+        if ahead is None:
+            due = self._prepare(input.device, is_first_microbatch, self.num_groups * 2)
+        # the fp8 weights: temporaries of the pass, or the buffers of caches that the pass refreshes or reuses
+        caches, refresh = None, True
+        if ahead is not None:
+            caches, refresh = ahead, False
+        elif is_first_microbatch is not None:
+            caches, refresh = tuple(self._weight_caches), bool(is_first_microbatch)
+        w1, w2 = self.fc1_weight, self.fc2_weight
+        if not has_tp and not self.fp8_meta["fused_dgelu"] and "capture" not in self.fp8_meta and self._native(input, w1, w2):
+            setup = self._native_setup(input.device)
+            held1, held2 = (c.take(w, setup, refresh) for c, w in zip(caches, (w1, w2))) if caches is not None \
+                else (None, None)
+            return mlp_step(input, w1, w2, group_sizes, held1, held2, refresh, setup, self._native_due(due))
+        self._run_update(due)
+        grad = torch.is_grad_enabled()
+        args = (input, w1, w2, group_sizes, self.fp8_meta, grad, has_tp, tp_group)
+        if caches is not None:
+            args += (caches, refresh)
+        if grad:
+            return _GroupedMlp.apply(*args)
+        return _GroupedMlp.forward(None, *args)

@@ -470,30 +470,6 @@ int fp8gmm_plan_mlp_forward(const fp8gmm_mlp_pass* pass, void* blob, size_t blob
 int fp8gmm_plan_mlp_backward(const fp8gmm_mlp_pass* pass, void* blob, size_t blob_bytes, fp8gmm_pass_plan* out);
 
 /*
- * The same passes with their tables written by the device: fp8gmm_lay_out_pass describes the launches (the offsets of
- * out->launch and out->blob_bytes, as the planning calls above report them) and what the tables hold, and
- * fp8gmm_build_pass enqueues the kernel that writes them into blob_dev (device memory, 128-byte aligned,
- * out->blob_bytes bytes) - the same bytes the planning calls write into host memory.  fp8gmm_run_planned runs the
- * launches as before.  Nothing is uploaded: the description travels as a kernel argument, so a captured pass replays
- * with the same group sizes without host memory that has to stay.
- *   which  : FP8GMM_LINEAR_* with a fp8gmm_linear_pass, FP8GMM_MLP_* with a fp8gmm_mlp_pass
- *   tables : FP8GMM_PASS_TABLES_BYTES of host memory, 8-byte aligned, opaque; filled by the first call, read by the second
- *   copy_* : copy_n floats (0: none) that the same kernel copies on the side, e.g. the snapshot of the forward
- *            scale_inv that the backward pass wants
- * More than FP8GMM_PASS_MAX_EXPERTS experts do not fit a kernel argument (FP8GMM_ERR_BAD_ARGUMENT): plan those passes on
- * the host.
- */
-#define FP8GMM_LINEAR_FORWARD 0
-#define FP8GMM_LINEAR_BACKWARD 1
-#define FP8GMM_MLP_FORWARD 2
-#define FP8GMM_MLP_BACKWARD 3
-#define FP8GMM_PASS_MAX_EXPERTS 448
-#define FP8GMM_PASS_MAX_GRID 512
-#define FP8GMM_PASS_TABLES_BYTES 4032
-int fp8gmm_lay_out_pass(int which, const void* pass, fp8gmm_pass_plan* out, void* tables);
-int fp8gmm_build_pass(const void* tables, void* blob_dev, const float* copy_src, float* copy_dst, int copy_n, void* stream);
-
-/*
  * Delayed-scaling update of one direction, in place, for `slots` scaling factors:
  *   amax = max over the `history_len` rows of amax_history[history_len, slots] (most_recent != 0: row 0)
  *   scale = (1 / amax) * fp8_max * 2^-margin where amax is finite and > 0, else unchanged;  scale_inv = 1 / scale
@@ -520,6 +496,33 @@ typedef struct fp8gmm_scaling_update {
   int32_t margin, most_recent, keep_period, keep_phase, reserved;
 } fp8gmm_scaling_update;   /* 56 bytes */
 int fp8gmm_delayed_scaling_updates(const fp8gmm_scaling_update* updates, int n, void* stream);
+
+/*
+ * The same passes with their tables written by the device: fp8gmm_lay_out_pass describes the launches (the offsets of
+ * out->launch and out->blob_bytes, as the planning calls above report them) and what the tables hold, and
+ * fp8gmm_build_pass enqueues the kernel that writes them into blob_dev (device memory, 128-byte aligned,
+ * out->blob_bytes bytes) - the same bytes the planning calls write into host memory.  fp8gmm_run_planned runs the
+ * launches as before.  Nothing is uploaded: the description travels as a kernel argument, so a captured pass replays
+ * with the same group sizes without host memory that has to stay.
+ *   which  : FP8GMM_LINEAR_* with a fp8gmm_linear_pass, FP8GMM_MLP_* with a fp8gmm_mlp_pass
+ *   tables : FP8GMM_PASS_TABLES_BYTES of host memory, 8-byte aligned, opaque; filled by the first call, read by the second
+ *   updates: up to two scaling updates that the same launch runs, ahead of everything else in the pass (the launches
+ *            read the new scales), as fp8gmm_delayed_scaling_updates would
+ *   copy_* : copy_n floats (0: none) that the same launch copies on the side, e.g. the snapshot of the forward
+ *            scale_inv that the backward pass wants; a copy of an updated scale_inv (all of it) holds the new values
+ * More than FP8GMM_PASS_MAX_EXPERTS experts do not fit a kernel argument (FP8GMM_ERR_BAD_ARGUMENT): plan those passes on
+ * the host.
+ */
+#define FP8GMM_LINEAR_FORWARD 0
+#define FP8GMM_LINEAR_BACKWARD 1
+#define FP8GMM_MLP_FORWARD 2
+#define FP8GMM_MLP_BACKWARD 3
+#define FP8GMM_PASS_MAX_EXPERTS 384
+#define FP8GMM_PASS_MAX_GRID 512
+#define FP8GMM_PASS_TABLES_BYTES 4032
+int fp8gmm_lay_out_pass(int which, const void* pass, fp8gmm_pass_plan* out, void* tables);
+int fp8gmm_build_pass(const void* tables, void* blob_dev, const fp8gmm_scaling_update* updates, int n_updates,
+                      const float* copy_src, float* copy_dst, int copy_n, void* stream);
 
 /*
  * Page-locked host memory that the device can read (for fp8gmm_upload's source), allocated also while a stream is

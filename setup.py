@@ -1,8 +1,8 @@
-"""Packaging of fp8_gmm_amd: ``pip install -e .`` (or ``pip install .``) builds ``libfp8gmm_hip.so`` with the
-Makefile under ``fp8_gmm_amd/csrc`` (hipcc, gfx950) and ships it inside the package, next to ``_lib.py`` that loads
-it.  Takes the place of the reference's ``setup.py`` (a torch CUDAExtension named ``fp8_gmm_backend``, setup.py:26-44)
-and ``reinstall.sh``: the library here is a plain C-ABI shared object, not a Python extension module, so no torch
-headers are involved in building it."""
+"""Packaging of fp8_gmm_amd: ``pip install -e .`` (or ``pip install .``) builds ``libfp8gmm_hip.so`` (hipcc, gfx950) and
+``_host.so`` (the modules' host path, on torch's C++ interface) with the Makefile under ``fp8_gmm_amd/csrc`` and ships
+them inside the package, next to ``_lib.py`` and ``native.py`` that load them.  Takes the place of the reference's
+``setup.py`` (a torch CUDAExtension named ``fp8_gmm_backend``, setup.py:26-44) and ``reinstall.sh``: the kernels' library
+is a plain C-ABI shared object that knows nothing of torch."""
 import os
 import subprocess
 
@@ -20,7 +20,7 @@ def make_library():
 
 
 class BuildHip(Command):
-    description = "build libfp8gmm_hip.so (hipcc, --offload-arch=gfx950)"
+    description = "build libfp8gmm_hip.so and _host.so (hipcc, --offload-arch=gfx950)"
     user_options = []
 
     def initialize_options(self):
@@ -50,7 +50,7 @@ setup(
     version="0.3.0",
     description="FP8 grouped GEMM modules for MoE expert layers on MI355X (gfx950): hand-written HIP behind a C ABI",
     packages=find_packages(include=["fp8_gmm_amd", "fp8_gmm_amd.*"]),
-    package_data={"fp8_gmm_amd": ["libfp8gmm_hip.so"]},
+    package_data={"fp8_gmm_amd": ["libfp8gmm_hip.so", "_host.so"]},
     python_requires=">=3.10",
     install_requires=["numpy"],   # torch is expected to be the ROCm build already present
     cmdclass={"build_hip": BuildHip, "build_py": BuildPy, "develop": Develop},
