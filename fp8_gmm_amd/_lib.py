@@ -19,6 +19,7 @@ E5M2 = 1
 OUT_BF16 = 2
 EPI_GELU = 1
 EPI_DGELU = 8
+EPI_TWO_ROUNDINGS = 32
 GEMM_B_KMAJOR = 2
 GEMM_A_KMAJOR = 4
 GEMM_TILE_128 = 0x100   # planning flag: 128 x 128 tiles, two workgroups per compute unit
@@ -119,7 +120,7 @@ class LinearPass(ctypes.Structure):
     _fields_ = [("experts", ctypes.c_int32), ("in_features", ctypes.c_int32), ("out_features", ctypes.c_int32),
                 ("fwd_fmt", ctypes.c_int32), ("bwd_fmt", ctypes.c_int32), ("cast_weights", ctypes.c_int32),
                 ("dgrad", ctypes.c_int32), ("wgrad", ctypes.c_int32), ("grid", ctypes.c_int32),
-                ("stream_k", ctypes.c_int32), ("tile_policy", ctypes.c_int32), ("reserved", ctypes.c_int32),
+                ("stream_k", ctypes.c_int32), ("tile_policy", ctypes.c_int32), ("two_roundings", ctypes.c_int32),
                 ("tokens", ctypes.c_int64), ("group_sizes", ctypes.c_void_p),
                 ("x", ctypes.c_void_p), ("x_fp8", ctypes.c_void_p), ("w", ctypes.c_void_p), ("w_fp8", ctypes.c_void_p),
                 ("y", ctypes.c_void_p), ("dy", ctypes.c_void_p), ("dy_fp8", ctypes.c_void_p), ("dx", ctypes.c_void_p),

@@ -779,7 +779,8 @@ def multi_cast_dgelu(inputs, gelu_inputs, outputs, scales, amaxes):
 # ------------------------------------------------------------------------------------------------
 # GEMMs
 # ------------------------------------------------------------------------------------------------
-def _launch_gemm(table, a_dtype, b_dtype, c_dtype, gelu, device, keep, b_kmajor=False, a_kmajor=False, dgelu=False):
+def _launch_gemm(table, a_dtype, b_dtype, c_dtype, gelu, device, keep, b_kmajor=False, a_kmajor=False, dgelu=False,
+                 two_roundings=False):
     if a_dtype not in _FP8_DTYPES or b_dtype not in _FP8_DTYPES:
         _fail("fp8_gmm_amd: GEMM operands must be fp8")
     if a_dtype == torch.float8_e5m2 and b_dtype == torch.float8_e5m2:
@@ -800,7 +801,8 @@ def _launch_gemm(table, a_dtype, b_dtype, c_dtype, gelu, device, keep, b_kmajor=
     if plan.total_tiles == 0:
         return
     n = len(table)
-    fmts = (_FMT[a_dtype], _FMT[b_dtype], _OUT_KIND[c_dtype], epi | layout)
+    fmts = (_FMT[a_dtype], _FMT[b_dtype], _OUT_KIND[c_dtype],
+            epi | layout | (_lib.EPI_TWO_ROUNDINGS if two_roundings else 0))
 
     def launch(dev_ptr):
         with _on_device(device):
@@ -1204,9 +1206,9 @@ def fp8_gmm(a, b, group_sizes, a_scale_invs, b_scale_invs, c=None, c_dtype=torch
     ``[sum(group_sizes[:i]), sum(group_sizes[:i+1]))`` of ``a[tokens, k]`` with ``b[i][n, k]^T``.
 
     One persistent kernel launch for all experts.  ``cutlass=True`` reproduces the data
-    flow of the reference's CUTLASS path (backend.py:78-82): an unscaled GEMM to bf16
-    followed by ``multi_scale_mul`` (two roundings); the default applies the scales to
-    the fp32 accumulator in the GEMM epilogue (one rounding), like its cuBLASLt path.
+    flow of the reference's CUTLASS path (backend.py:78-82): the product rounded to bf16,
+    then scaled as ``multi_scale_mul`` does and rounded again, both in the GEMM's epilogue;
+    the default applies the scales to the fp32 accumulator (one rounding), like its cuBLASLt path.
     Experts with zero rows are allowed.
 
     ``b_transposed=True`` (not in the reference): ``b`` is ``[experts, k, n]`` and expert i multiplies with
@@ -1269,15 +1271,12 @@ def fp8_gmm(a, b, group_sizes, a_scale_invs, b_scale_invs, c=None, c_dtype=torch
     table["lda"] = k
     table["ldb"] = nn if b_transposed else k
     table["ldc"] = nn
-    if not cutlass:
-        table["a_scale_inv"] = _scalar_ptrs(a_scale_invs, e, "a_scale_invs")
-        table["b_scale_inv"] = _scalar_ptrs(b_scale_invs, e, "b_scale_invs")
+    table["a_scale_inv"] = _scalar_ptrs(a_scale_invs, e, "a_scale_invs")
+    table["b_scale_inv"] = _scalar_ptrs(b_scale_invs, e, "b_scale_invs")
     if fp8_out:
         table["c_scale"] = _scalar_ptrs(c_scales, e, "c_scales")
         table["c_amax"] = _scalar_ptrs(c_amaxes, e, "c_amaxes")
     _launch_gemm(table, a.dtype, b.dtype, c.dtype, pre_gelu_out is not None, dev,
                  (a, b, c, pre_gelu_out, dgelu_pre, a_scale_invs, b_scale_invs, c_scales, c_amaxes),
-                 b_kmajor=b_transposed, dgelu=dgelu_pre is not None)
-    if cutlass:
-        multi_scale_mul(TensorBatch.rows_of(c, starts), a_scale_invs, b_scale_invs)
+                 b_kmajor=b_transposed, dgelu=dgelu_pre is not None, two_roundings=cutlass)
     return c

@@ -65,6 +65,7 @@ __global__ __launch_bounds__(kFixupThreads) void grouped_gemm_fixup_kernel(
   const float s = sa_inv * sb_inv;
   const bool gelu = (epilogue & FP8GMM_EPI_GELU) != 0;
   const bool dgelu_in = (epilogue & FP8GMM_EPI_DGELU) != 0 && pr.aux != nullptr;   // aux is then an input
+  const bool two = (epilogue & FP8GMM_EPI_TWO_ROUNDINGS) != 0;
   const int64_t ldc = pr.ldc;
   uint16_t* __restrict__ AUX = static_cast<uint16_t*>(pr.aux);
   const bool aux_ok = AUX == nullptr || (reinterpret_cast<uintptr_t>(AUX) & 7) == 0;
@@ -79,7 +80,7 @@ __global__ __launch_bounds__(kFixupThreads) void grouped_gemm_fixup_kernel(
     float v[4], r[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      v[e] = sum[q][e] * s;
+      v[e] = two ? scaled_twice(sum[q][e], sa_inv, sb_inv) : sum[q][e] * s;
       r[e] = gelu ? gelu_tanh_fast(v[e]) : v[e];
     }
     const int64_t off = (int64_t)m * ldc + n;
@@ -199,7 +200,10 @@ int launch_checked(const fp8gmm_gemm_problem* probs_dev, int n, const fp8gmm_gem
   if (n < 0 || plan->total_tiles < 0 || plan->rounds < 0 || plan->n_fixups < 0 || plan->n_slots < 0)
     return FP8GMM_ERR_BAD_ARGUMENT;
   if (out_kind != FP8GMM_OUT_BF16 && out_kind != FP8GMM_E4M3 && out_kind != FP8GMM_E5M2) return FP8GMM_ERR_BAD_FORMAT;
-  if (epilogue & ~(FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU | FP8GMM_GEMM_A_KMAJOR | FP8GMM_GEMM_B_KMAJOR))
+  constexpr int kEpilogues = FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU | FP8GMM_EPI_TWO_ROUNDINGS;
+  if (epilogue & ~(kEpilogues | FP8GMM_GEMM_A_KMAJOR | FP8GMM_GEMM_B_KMAJOR)) return FP8GMM_ERR_BAD_ARGUMENT;
+  if ((epilogue & FP8GMM_EPI_TWO_ROUNDINGS) &&
+      (out_kind != FP8GMM_OUT_BF16 || (epilogue & (FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU))))
     return FP8GMM_ERR_BAD_ARGUMENT;
   if ((epilogue & FP8GMM_EPI_GELU) && (epilogue & FP8GMM_EPI_DGELU)) return FP8GMM_ERR_BAD_ARGUMENT;
   const bool a_kmajor = (epilogue & FP8GMM_GEMM_A_KMAJOR) != 0;
@@ -231,12 +235,12 @@ int launch_checked(const fp8gmm_gemm_problem* probs_dev, int n, const fp8gmm_gem
                             (reinterpret_cast<uintptr_t>(workspace) & 255) != 0))
     return FP8GMM_ERR_WORKSPACE;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int rc = launch(probs_dev, items_dev, plan->grid, out_kind, epilogue & (FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU),
+  const int rc = launch(probs_dev, items_dev, plan->grid, out_kind, epilogue & kEpilogues,
                         static_cast<uint8_t*>(workspace), merge_descs, merge_n, s);
   if (rc != FP8GMM_OK) return rc;
   if (plan->n_fixups > 0) {
     hipLaunchKernelGGL(grouped_gemm_fixup_kernel, dim3(plan->n_fixups * kFixupSplit), dim3(kFixupThreads), 0, s, probs_dev,
-                       fixups_dev, out_kind, epilogue & (FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU),
+                       fixups_dev, out_kind, epilogue & kEpilogues,
                        static_cast<const uint8_t*>(workspace));
     if (hipGetLastError() != hipSuccess) return FP8GMM_ERR_LAUNCH;
   }

@@ -56,7 +56,8 @@ __device__ __forceinline__ f32x4 acc_quad() {   // four consecutive accumulators
 #define FP8GMM_DUAL_MFMA_Z(S, i, j, FB, FA) ((void)(FB), (void)(FA))
 #endif
 
-template <int A_FMT, int B_FMT, bool A_TR, bool B_TR>
+// TWO: FP8GMM_EPI_TWO_ROUNDINGS, a kernel of its own (a branch between the products would cost the other one).
+template <int A_FMT, int B_FMT, bool A_TR, bool B_TR, bool TWO>
 __global__ __launch_bounds__(NTHREADS, 1) void grouped_gemm_dual_kernel(
     const fp8gmm_gemm_problem* __restrict__ probs, const fp8gmm_gemm_item* __restrict__ items,
     const fp8gmm_tensor_desc* __restrict__ merge_descs, int merge_n) {
@@ -281,7 +282,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void grouped_gemm_dual_kernel(
   bool pe_on = false;
   __amdgpu_buffer_rsrc_t pe_rc = make_rsrc(nullptr, 0);
   int pe_ldc = 0, pe_cv = 0;
-  float pe_s = 1.f;
+  float pe_s = 1.f, pe_s2 = 1.f;   // two roundings: the two factors; else pe_s is their product
   // per-lane constants of the staged store: a lane holds 4 consecutive columns of row l32 of an MFMA block; a piece
   // (32 rows x 64 columns, two blocks) is staged as 32 rows x 128 B with 16-byte chunk c of row r at chunk
   // c ^ ((r >> 1) & 7) and read back 8 rows x 128 contiguous bytes per instruction
@@ -292,7 +293,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void grouped_gemm_dual_kernel(
     constexpr int P = decltype(set_c)::value, u = decltype(u_c)::value, q = decltype(q_c)::value;
     constexpr int i = u / 2, jj = u % 2, jl = q / 4, g = q % 4;
     const f32x4 t = acc_quad<16 * (4 * (i + 2 * P) + 2 * jj + jl) + 4 * g>();
-    const u32x2 o = {pack_bf16x2(t[0] * pe_s, t[1] * pe_s), pack_bf16x2(t[2] * pe_s, t[3] * pe_s)};
+    const u32x2 o = {scaled_bf16x2<TWO>(t[0], t[1], pe_s, pe_s2), scaled_bf16x2<TWO>(t[2], t[3], pe_s, pe_s2)};
     *reinterpret_cast<u32x2*>(buf + st_wr + (((4 * jl + g) ^ fsw) << 4)) = o;
   };
   auto piece_read_back = [&](u32x4 (&v)[4], const uint8_t* buf) {
@@ -456,7 +457,8 @@ __global__ __launch_bounds__(NTHREADS, 1) void grouped_gemm_dual_kernel(
     if (g.prob < 0) return false;
     cp_next = item_tile(++r_cp);
     const fp8gmm_gemm_problem pr = probs[g.prob];
-    const float scale_ab = load_scale(pr.a_scale_inv) * load_scale(pr.b_scale_inv);
+    const float scale_a = load_scale(pr.a_scale_inv), scale_b = load_scale(pr.b_scale_inv);
+    const float scale_ab = TWO ? scale_a : scale_a * scale_b;
     const int nk = g.nk;
     if (nk == 0) static_for<MT * NT>([&](auto tc) { acc_tile_clear<16 * (4 * 2 * S + decltype(tc)::value)>(); });
     // the steps, one run per kind and the runs one after the other (alternatives behind a branch make the compiler
@@ -487,6 +489,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void grouped_gemm_dual_kernel(
       pe_ldc = ldc;
       pe_cv = cv;
       pe_s = scale_ab;
+      if constexpr (TWO) pe_s2 = scale_b;
       pe_on = true;
     } else {
       // element by element (a pitch or base address that 16-byte stores cannot take)
@@ -502,14 +505,15 @@ __global__ __launch_bounds__(NTHREADS, 1) void grouped_gemm_dual_kernel(
         for (int q = 0; q < 4; ++q) {
           const int n = n0 + wave_n * 128 + j * 32 + q * 8 + khalf * 4;
           if (m >= M || n >= N) continue;
-          const float r0 = t[4 * q + 0] * scale_ab, r1 = t[4 * q + 1] * scale_ab, r2 = t[4 * q + 2] * scale_ab,
-                      r3 = t[4 * q + 3] * scale_ab;
+          float r[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            r[e] = TWO ? scaled_twice(t[4 * q + e], scale_a, scale_b) : t[4 * q + e] * scale_ab;
           const int64_t off = (int64_t)m * ldc + n;
           if (vec && n + 3 < N) {
-            const u32x2 o = {pack_bf16x2(r0, r1), pack_bf16x2(r2, r3)};
+            const u32x2 o = {pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3])};
             global_store(C + off, o);
           } else {
-            const float r[4] = {r0, r1, r2, r3};
 #pragma unroll
             for (int e = 0; e < 4; ++e)
               if (n + e < N) global_store(C + off + e, (uint16_t)f32_to_bf16_bits(r[e]));

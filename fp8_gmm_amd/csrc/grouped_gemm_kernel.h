@@ -186,6 +186,23 @@ __device__ __forceinline__ void merge_amax(float* slot, float wave_amax, int lan
     atomic_max_nonneg(slot, wave_amax);
 }
 
+// FP8GMM_EPI_TWO_ROUNDINGS: the product rounded to bf16, then multiplied by the factors one after the other, as
+// multi_scale_mul does with the result of an unscaled launch (the caller rounds once more).  In the epilogue the second
+// rounding costs three vector instructions per pair of values; as a pass of its own it read and wrote the result once
+// more and took a launch (8 experts, 4001 x 1024 -> 4096: 12.8 us behind a GEMM of 29, 5.2 behind the data gradient).
+__device__ __forceinline__ float scaled_twice(float acc, float s1, float s2) {
+  return bf16_to_f32((uint16_t)f32_to_bf16_bits(acc)) * s1 * s2;
+}
+// two neighbouring results as bf16: x * s, or with TWO the product rounded first and then multiplied by s and s2
+template <bool TWO>
+__device__ __forceinline__ uint32_t scaled_bf16x2(float x0, float x1, float s, float s2) {
+  if constexpr (TWO) {
+    const uint32_t r = pack_bf16x2(x0, x1);
+    return pack_bf16x2(bf16_lo_to_f32(r) * s * s2, bf16_hi_to_f32(r) * s * s2);
+  }
+  return pack_bf16x2(x0 * s, x1 * s);
+}
+
 // Epilogue of one 256 x 256 tile whose accumulators are complete: scales, optional GELU, conversion,
 // stores, amax.  Returns true when the staged bf16 path ran (exactly kFastStores stores per wavefront).
 // `stage`: 32 KB of LDS that no wavefront reads or loads into until the barrier at the end of the staged path.
@@ -200,7 +217,8 @@ __device__ __forceinline__ void merge_amax(float* slot, float wave_amax, int lan
 // and the workgroups that drew those tiles set the duration of the launch).
 constexpr uint32_t kMaskedOffset = 0x80000000u;  // + any row offset of a tile (< 2^30) stays out of range
 
-// `s` = a_scale_inv * b_scale_inv and `cs` = c_scale of the problem, read by the caller ahead of time.
+// `s` = a_scale_inv * b_scale_inv and `cs` = c_scale of the problem, read by the caller ahead of time.  With
+// FP8GMM_EPI_TWO_ROUNDINGS (bf16 results only, hence without a c_scale) they are a_scale_inv and b_scale_inv.
 // TILE: 256 (the namespace's constants) or 128 (the small tile: 64 x 64 per wavefront, 16 KB of staging).
 // `released(i, j)` (integral constants) is called right after MFMA tile (i, j) of the staged bf16 path has been read
 // out of its accumulators: from there on they may receive the next tile's products.
@@ -241,6 +259,7 @@ __device__ __forceinline__ int tile_epilogue(const fp8gmm_gemm_problem& pr, int 
   int fast = 0;
     const bool gelu = (epilogue & FP8GMM_EPI_GELU) != 0;
     const bool dgelu_in = (epilogue & FP8GMM_EPI_DGELU) != 0 && pr.aux != nullptr;   // aux is then an INPUT
+    const bool two = (epilogue & FP8GMM_EPI_TWO_ROUNDINGS) != 0;
     const int64_t ldc = pr.ldc;
     float amax = 0.f;
     const bool interior = (m0 + BM <= M) && (n0 + BN <= N);
@@ -275,31 +294,35 @@ __device__ __forceinline__ int tile_epilogue(const fp8gmm_gemm_problem& pr, int 
           buf_store16_stream(v[it], rc, lane_off + row_off);
         }
       };
-      static_for<MT * kUnitsPerRow>([&](auto uc) {
-        constexpr int u = decltype(uc)::value;
-        constexpr int i = u / kUnitsPerRow, jj = u % kUnitsPerRow;
-        if (i >= mt) return;
-        uint8_t* buf = mine + (kStageBytes >= 8192 ? (u & 1) * 4096 : 0);
-        static_for<2>([&](auto jlc) {
-          constexpr int jl = decltype(jlc)::value;
-          const f32x16 t = acc_tile<16 * (NT * i + 2 * jj + jl)>();
-          released(std::integral_constant<int, i>{}, std::integral_constant<int, 2 * jj + jl>{});
-#pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            const u32x2 o = {pack_bf16x2(t[4 * g + 0] * s, t[4 * g + 1] * s),
-                             pack_bf16x2(t[4 * g + 2] * s, t[4 * g + 3] * s)};
-            *reinterpret_cast<u32x2*>(buf + wr + (((4 * jl + g) ^ ((l32 >> 1) & 7)) << 4)) = o;
+      auto units = [&](auto two_c) {
+        static_for<MT * kUnitsPerRow>([&](auto uc) {
+          constexpr int u = decltype(uc)::value;
+          constexpr int i = u / kUnitsPerRow, jj = u % kUnitsPerRow;
+          if (i >= mt) return;
+          uint8_t* buf = mine + (kStageBytes >= 8192 ? (u & 1) * 4096 : 0);
+          static_for<2>([&](auto jlc) {
+            constexpr int jl = decltype(jlc)::value;
+            const f32x16 t = acc_tile<16 * (NT * i + 2 * jj + jl)>();
+            released(std::integral_constant<int, i>{}, std::integral_constant<int, 2 * jj + jl>{});
+  #pragma unroll
+            for (int g = 0; g < 4; ++g) {
+              const u32x2 o = {scaled_bf16x2<decltype(two_c)::value>(t[4 * g + 0], t[4 * g + 1], s, cs),
+                               scaled_bf16x2<decltype(two_c)::value>(t[4 * g + 2], t[4 * g + 3], s, cs)};
+              *reinterpret_cast<u32x2*>(buf + wr + (((4 * jl + g) ^ ((l32 >> 1) & 7)) << 4)) = o;
+            }
+          });
+          // the previous unit's read-back was issued before this unit's conversion: store it now
+          if (u > 0) store_unit((u - 1) / kUnitsPerRow, (u - 1) % kUnitsPerRow);
+          // only this wavefront touches `mine`, and its LDS operations complete in order
+  #pragma unroll
+          for (int it = 0; it < 4; ++it) {
+            const int r = 8 * it + rrow;
+            v[it] = *reinterpret_cast<const u32x4*>(buf + r * 128 + ((rchunk ^ ((r >> 1) & 7)) << 4));
           }
         });
-        // the previous unit's read-back was issued before this unit's conversion: store it now
-        if (u > 0) store_unit((u - 1) / kUnitsPerRow, (u - 1) % kUnitsPerRow);
-        // only this wavefront touches `mine`, and its LDS operations complete in order
-#pragma unroll
-        for (int it = 0; it < 4; ++it) {
-          const int r = 8 * it + rrow;
-          v[it] = *reinterpret_cast<const u32x4*>(buf + r * 128 + ((rchunk ^ ((r >> 1) & 7)) << 4));
-        }
-      });
+      };
+      // one straight line each: a branch inside would make every wait behind it a wait for everything
+      if (two) units(std::true_type{}); else units(std::false_type{});
       store_unit(mt - 1, kUnitsPerRow - 1);
       __builtin_amdgcn_s_barrier();  // the staging area goes back to the operand ring
       fast = mt * kUnitsPerRow * 4;
@@ -502,7 +525,7 @@ __device__ __forceinline__ int tile_epilogue(const fp8gmm_gemm_problem& pr, int 
             float v[4], r[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-              v[q] = t[g * 4 + q] * s;
+              v[q] = two ? scaled_twice(t[g * 4 + q], s, cs) : t[g * 4 + q] * s;
               r[q] = gelu ? gelu_tanh_fast(v[q]) : v[q];
             }
             const int64_t off = (int64_t)m * ldc + n;
@@ -969,8 +992,11 @@ __global__ __launch_bounds__(NTHREADS, TILE == 256 ? 1 : 2) void grouped_gemm_ke
     cp_next = item_tile(r_cp + 1);
     // only the epilogue needs the problem's record and its scaling factors: the main loop hides the reads
     const fp8gmm_gemm_problem pr = probs[g.prob];
-    const float scale_ab = load_scale(pr.a_scale_inv) * load_scale(pr.b_scale_inv);
-    const float scale_c = load_scale(pr.c_scale);
+    // (two roundings: the factors one by one)
+    const bool two = (epilogue & FP8GMM_EPI_TWO_ROUNDINGS) != 0;
+    const float scale_a = load_scale(pr.a_scale_inv), scale_b = load_scale(pr.b_scale_inv);
+    const float scale_ab = two ? scale_a : scale_a * scale_b;
+    const float scale_c = two ? scale_b : load_scale(pr.c_scale);
     const int m0 = g.m0, n0 = g.n0;
     const bool cur_half = TILE == 256 && (g.flags & FP8GMM_ITEM_HALF_HEIGHT) != 0;   // this tile's height
     bool read_half_next = cur_half;   // height of the tile that the NEXT step belongs to
@@ -1292,17 +1318,20 @@ int prepare_variant(int dev) {
   static std::atomic<bool> attr_set[kMaxDevices];
   if (dev < 0 || dev >= kMaxDevices) return FP8GMM_ERR_NO_DEVICE;
   if (!attr_set[dev].load(std::memory_order_acquire)) {
-    const void* kernel = nullptr;
+    const void* kernels[2] = {};
     int lds_bytes = 0;
     if constexpr (TILE == kTileDual) {
-      kernel = reinterpret_cast<const void*>(grouped_gemm_dual_kernel<A_FMT, B_FMT, A_TR, B_TR>);
+      kernels[0] = reinterpret_cast<const void*>(grouped_gemm_dual_kernel<A_FMT, B_FMT, A_TR, B_TR, false>);
+      kernels[1] = reinterpret_cast<const void*>(grouped_gemm_dual_kernel<A_FMT, B_FMT, A_TR, B_TR, true>);
       lds_bytes = RING * BN * BK;
     } else {
-      kernel = reinterpret_cast<const void*>(grouped_gemm_kernel<A_FMT, B_FMT, A_TR, B_TR, TILE>);
+      kernels[0] = reinterpret_cast<const void*>(grouped_gemm_kernel<A_FMT, B_FMT, A_TR, B_TR, TILE>);
       lds_bytes = RING * TILE * BK;
     }
-    if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess)
-      return FP8GMM_ERR_LAUNCH;
+    for (const void* kernel : kernels)
+      if (kernel != nullptr &&
+          hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess)
+        return FP8GMM_ERR_LAUNCH;
     attr_set[dev].store(true, std::memory_order_release);
   }
   return FP8GMM_OK;
@@ -1317,9 +1346,13 @@ int launch_variant(const fp8gmm_gemm_problem* probs_dev, const fp8gmm_gemm_item*
   const int rc = prepare_variant<A_FMT, B_FMT, A_TR, B_TR, TILE>(dev);
   if (rc != FP8GMM_OK) return rc;
   if constexpr (TILE == kTileDual) {
-    // bf16 results without a fused epilogue only (the caller has checked)
-    hipLaunchKernelGGL((grouped_gemm_dual_kernel<A_FMT, B_FMT, A_TR, B_TR>), dim3(grid), dim3(NTHREADS), RING * BN * BK,
-                       stream, probs_dev, items_dev, merge_descs, merge_n);
+    // bf16 results without a fused activation only (the caller has checked)
+    if (epilogue & FP8GMM_EPI_TWO_ROUNDINGS)
+      hipLaunchKernelGGL((grouped_gemm_dual_kernel<A_FMT, B_FMT, A_TR, B_TR, true>), dim3(grid), dim3(NTHREADS),
+                         RING * BN * BK, stream, probs_dev, items_dev, merge_descs, merge_n);
+    else
+      hipLaunchKernelGGL((grouped_gemm_dual_kernel<A_FMT, B_FMT, A_TR, B_TR, false>), dim3(grid), dim3(NTHREADS),
+                         RING * BN * BK, stream, probs_dev, items_dev, merge_descs, merge_n);
   } else {
     hipLaunchKernelGGL((grouped_gemm_kernel<A_FMT, B_FMT, A_TR, B_TR, TILE>), dim3(grid), dim3(NTHREADS),
                        RING * TILE * BK, stream, probs_dev, items_dev, out_kind, epilogue, workspace, merge_descs, merge_n);

@@ -9,6 +9,7 @@
 // What a pass computes is stated in fp8gmm.h and grouped_linear.py / grouped_mlp.py (reference fp8_gmm/grouped_linear.py:11-183,
 // fp8_gmm/grouped_mlp.py:18-325); the Python functions there launch the same kernels with the same tables and serve
 // the layouts and options that this file leaves to them.
+#include <torch/csrc/autograd/VariableTypeUtils.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -54,6 +55,7 @@ std::vector<int64_t> sizes_of(const py::object& group_sizes) {
 struct Setup {
   int fwd_fmt = 0, bwd_fmt = 0;
   int grid = 0, stream_k = 0, tile_policy = 0;
+  bool two_roundings = false;   // GroupedLinear(cutlass=True)
   Tensor fwd_scale, fwd_scale_inv, fwd_amax, bwd_scale, bwd_scale_inv, bwd_amax;
   at::ScalarType fwd_type() const { return fwd_fmt == FP8GMM_E4M3 ? at::kFloat8_e4m3fn : at::kFloat8_e5m2; }
   at::ScalarType bwd_type() const { return bwd_fmt == FP8GMM_E4M3 ? at::kFloat8_e4m3fn : at::kFloat8_e5m2; }
@@ -115,6 +117,14 @@ void check_rows(const std::vector<int64_t>& sizes, const Tensor& x) {
   TORCH_CHECK(rows == x.size(0), "group_sizes must sum to the number of input rows");
 }
 
+// Forward-mode differentiation has no rule here and is refused, as the Python functions refuse it: a tangent that is
+// silently dropped would be a wrong derivative.
+void check_no_tangent(at::TensorList inputs) {
+  if (!at::GradMode::is_enabled()) return;
+  for (const Tensor& t : inputs)
+    TORCH_CHECK(!torch::autograd::isFwGradDefined(t), "fp8_gmm_amd: the grouped modules do not support forward-mode AD");
+}
+
 // ---- GroupedLinear ------------------------------------------------------------------------------------------------
 fp8gmm_linear_pass linear_desc(const Setup& s, const std::vector<int64_t>& sizes, int64_t tokens, int64_t in, int64_t out) {
   fp8gmm_linear_pass d{};
@@ -126,6 +136,7 @@ fp8gmm_linear_pass linear_desc(const Setup& s, const std::vector<int64_t>& sizes
   d.grid = s.grid;
   d.stream_k = s.stream_k;
   d.tile_policy = s.tile_policy;
+  d.two_roundings = s.two_roundings;
   d.tokens = tokens;
   d.group_sizes = sizes.data();
   return d;
@@ -177,6 +188,7 @@ Tensor linear_step(const Tensor& x, const Tensor& w, const py::object& group_siz
   std::vector<int64_t> sizes = sizes_of(group_sizes);
   py::gil_scoped_release no_gil;
   check_rows(sizes, x);
+  check_no_tangent({x, w});
   const c10::OptionalDeviceGuard guard(x.device());
   const bool grad = at::GradMode::is_enabled();
   const bool dgrad = grad && x.requires_grad(), wgrad = grad && w.requires_grad();
@@ -292,6 +304,7 @@ Tensor mlp_step(const Tensor& x, const Tensor& w1, const Tensor& w2, const py::o
   std::vector<int64_t> sizes = sizes_of(group_sizes);
   py::gil_scoped_release no_gil;
   check_rows(sizes, x);
+  check_no_tangent({x, w1, w2});
   const c10::OptionalDeviceGuard guard(x.device());
   const bool grad = at::GradMode::is_enabled();
   const bool dgrad = grad && x.requires_grad(), wgrad = grad && w1.requires_grad();
@@ -367,6 +380,7 @@ PYBIND11_MODULE(_host, m) {
       }))
       .def_readonly("fwd_fmt", &Setup::fwd_fmt)
       .def_readwrite("stream_k", &Setup::stream_k)
+      .def_readwrite("two_roundings", &Setup::two_roundings)
       .def_readwrite("tile_policy", &Setup::tile_policy);
   py::class_<Due>(m, "Due")
       .def(py::init<>())

@@ -39,6 +39,7 @@ struct Pass {
     CastSpec cast;
     GemmSpec gemm;
     int a_fmt, b_fmt, out_kind, epi;
+    bool two_roundings;   // a flag of the launch that its plan does not see
   };
   Launch launch[8];
   int n_launches = 0;
@@ -177,7 +178,7 @@ void describe_gemm(const Pass& pass, const Pass::Launch& l, const fp8gmm_gemm_pr
   rec->a_fmt = l.a_fmt;
   rec->b_fmt = l.b_fmt;
   rec->out_kind = l.out_kind;
-  rec->epilogue = l.gemm.layout | l.epi;
+  rec->epilogue = l.gemm.layout | l.epi | (l.two_roundings ? FP8GMM_EPI_TWO_ROUNDINGS : 0);
   rec->kind = rec->plan.total_tiles > 0 ? FP8GMM_PASS_GEMM : FP8GMM_PASS_NOTHING;
   double flops = 0, bytes = 0;
   for (int i = 0; i < pass.experts; ++i) {
@@ -392,7 +393,7 @@ int linear_forward(const fp8gmm_linear_pass* s, Pass& p) {
   if (s->cast_weights) Pass::stack(cast, s->w, s->w_fp8, (int64_t)N * K, s->fwd_scale + 1, s->fwd_amax + 1);
   // y[rows of expert i] = x_fp8[rows] . w_fp8[i]^T
   p.row_gemm(s->x_fp8, s->w_fp8, s->y, 2, nullptr, N, K, false, s->fwd_fmt, s->fwd_fmt, s->fwd_scale_inv, 3,
-             s->fwd_scale_inv + 1);
+             s->fwd_scale_inv + 1).two_roundings = s->two_roundings != 0;
   return FP8GMM_OK;
 }
 
@@ -416,7 +417,7 @@ int linear_backward(const fp8gmm_linear_pass* s, Pass& p) {
   // dx[rows] = dy_fp8[rows] . w_fp8[i]: the forward weight [N, K] read in place as b[k = N][n = K]
   if (s->dgrad)
     p.row_gemm(s->dy_fp8, s->w_fp8, s->dx, 2, nullptr, K, N, true, s->bwd_fmt, s->fwd_fmt, s->bwd_scale_inv, 2,
-               s->fwd_scale_inv + 1);
+               s->fwd_scale_inv + 1).two_roundings = s->two_roundings != 0;
   return FP8GMM_OK;
 }
 

@@ -17,7 +17,7 @@ backward  one cast launch over the E slices of grad_out (e5m2), a grouped dgrad 
 Differences from the reference: experts with zero tokens are allowed (their weight
 gradient is zero), wgrad is a single launch instead of a per-expert loop, and the
 grouped GEMM is the same HIP kernel whatever ``cutlass`` says (``cutlass=True`` keeps
-the two-rounding data flow of the reference's CUTLASS path, see ``backend.fp8_gmm``).
+the two-rounding data flow of the reference's CUTLASS path in its epilogue, see ``backend.fp8_gmm``).
 """
 import math
 
@@ -131,8 +131,8 @@ class _GroupedLinear(torch.autograd.Function):
         fp8_dtype = to_torch_dtype(fwd_dtype)
         dev = input.device
 
-        if fp8_meta.get("planned_passes", True) and not reference_layout and not cutlass and input.is_cuda \
-                and input.is_contiguous() and weight.is_contiguous() \
+        if fp8_meta.get("planned_passes", True) and not reference_layout and input.is_cuda and input.is_contiguous() \
+                and weight.is_contiguous() \
                 and input.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16:
             # The default data flow as one planned pass: every table of the cast launch and of the GEMM comes out of
             # one library call (with 64 experts the array arithmetic below costs more host time than the kernels run).
@@ -153,7 +153,7 @@ class _GroupedLinear(torch.autograd.Function):
                         experts=num_groups, in_features=weight.size(2), out_features=weight.size(1),
                         fwd_fmt=_lib.E4M3 if fp8_dtype == torch.float8_e4m3fn else _lib.E5M2, cast_weights=cast_weights,
                         tokens=input.size(0), group_sizes=sizes, x=input, x_fp8=input_fp8, w=weight, w_fp8=weight_fp8,
-                        y=out, fwd_scale=fwd.scale, fwd_scale_inv=fwd.scale_inv, fwd_amax=fwd.amax_history)
+                        y=out, two_roundings=int(cutlass), fwd_scale=fwd.scale, fwd_scale_inv=fwd.scale_inv, fwd_amax=fwd.amax_history)
             if is_grad_enabled:
                 ctx.save_for_backward(input_fp8 if wgrad_needed else None, weight_fp8 if dgrad_needed else None)
                 ctx.reference_layout = False
@@ -256,6 +256,7 @@ class _GroupedLinear(torch.autograd.Function):
                         dgrad=int(ctx.input_requires_grad), wgrad=int(ctx.weight_requires_grad),
                         tokens=grad_out.size(0), group_sizes=ctx.sizes, dy=grad_out, dy_fp8=grad_out_fp8,
                         x_fp8=input_for_wgrad, w_fp8=weight_for_dgrad, dx=grad_input, dw=grad_weight,
+                        two_roundings=int(ctx.cutlass),
                         fwd_scale_inv=meta._forward_scale_inv_cloned, bwd_scale=bwd.scale,
                         bwd_scale_inv=bwd.scale_inv, bwd_amax=bwd.amax_history)
             return grad_input, grad_weight, None, None, None, None, None, None
@@ -374,8 +375,9 @@ class GroupedLinear(Fp8GroupedModuleBase):
         elif is_first_microbatch is not None:
             cache, refresh = self._weight_cache, bool(is_first_microbatch)
         weight = self.weight_tensor
-        if not self.cutlass and self._native(input, weight):
+        if self._native(input, weight):
             setup = self._native_setup(input.device)
+            setup.two_roundings = bool(self.cutlass)
             held = cache.take(weight, setup, refresh) if cache is not None else None
             return linear_step(input, weight, group_sizes, held, refresh, setup, self._native_due(due))
         self._run_update(due)

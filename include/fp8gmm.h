@@ -145,6 +145,11 @@ typedef struct fp8gmm_gemm_problem {
  * missing fusion (:252-253); here v stays in fp32 until the one rounding to fp8.  Not together with
  * FP8GMM_EPI_GELU. */
 #define FP8GMM_EPI_DGELU 8
+/* The data flow of the reference's CUTLASS path (fp8_gmm/backend.py:78-82: an unscaled grouped GEMM to bf16, then
+ * multi_scale_mul) in one launch: c = bf16(bf16(sum) * *a_scale_inv * *b_scale_inv), the factors multiplied one after
+ * the other; the same bits as the two launches.  bf16 results without the other FP8GMM_EPI_* only.  A flag of the
+ * launch, not of its plan. */
+#define FP8GMM_EPI_TWO_ROUNDINGS 32
 /* b is stored contraction-major: b[k, n] with n contiguous and ldb >= n its row pitch, i.e.
  * c[m, n] = epilogue( a[m, k] . b[k, n] ).  This is a forward weight [N_fwd = k, K_fwd = n] as the data-gradient
  * GEMM needs it, read in place: the reference casts a transposed copy of every weight for that GEMM instead
@@ -307,7 +312,7 @@ int fp8gmm_plan_grouped_gemm_launch(fp8gmm_gemm_problem* probs, int n, int layou
  *   plan         : the host struct fp8gmm_plan_grouped_gemm_launch filled
  *   a_fmt, b_fmt : FP8GMM_E4M3 / FP8GMM_E5M2 (e5m2 x e5m2 is rejected, as cuBLASLt does)
  *   out_kind     : FP8GMM_OUT_BF16, or FP8GMM_E4M3 / FP8GMM_E5M2 for an fp8 `c`
- *   epilogue     : FP8GMM_EPI_GELU or FP8GMM_EPI_DGELU, and the layout flags the table was planned with
+ *   epilogue     : one of FP8GMM_EPI_*, or none, and the layout flags the table was planned with
  *   workspace    : device memory, workspace_bytes >= plan->n_slots * FP8GMM_GEMM_SLOT_BYTES, 256-byte aligned,
  *                  contents irrelevant; may be NULL when n_slots == 0.  Launches that overlap in time (different
  *                  streams) need different workspaces.  Too small: FP8GMM_ERR_WORKSPACE, nothing is launched.
@@ -355,7 +360,7 @@ typedef struct fp8gmm_linear_pass {
   int32_t stream_k;                  /* as for fp8gmm_plan_grouped_gemm_launch */
   int32_t tile_policy;               /* 0: the library chooses per launch; 256 or 128: that tile for every launch;
                                         FP8GMM_GEMM_TILE_DUAL: the 128 x 256 form for every launch that can take it */
-  int32_t reserved;
+  int32_t two_roundings;             /* != 0: y and dx are formed with FP8GMM_EPI_TWO_ROUNDINGS */
   int64_t tokens;                    /* rows of x / dy: must equal the sum of group_sizes */
   const int64_t* group_sizes;        /* HOST array [experts] */
   const void* x;                     /* bf16 [tokens, in_features] */

@@ -385,6 +385,29 @@ def test_batched_uploads_runs_the_queued_launches_in_order(dev):
     assert c2.any()
 
 
+@pytest.mark.parametrize("tile", ["256", "128", "dual", "auto"])
+@pytest.mark.parametrize("b_transposed", [False, True])
+def test_two_roundings_in_the_epilogue_equal_the_separate_scaling(dev, tile, b_transposed):
+    """``cutlass=True`` rounds the product to bf16, multiplies by both factors and rounds again inside the GEMM: the same
+    bits as an unscaled launch followed by ``multi_scale_mul``, in every tile form, on edge tiles, on pitches that only
+    take element stores, on tiles shared along K, with NaN and saturated products, and for experts without rows."""
+    backend = _backend()
+    g = gen(4711)
+    for sizes, k, n in [([137, 0, 259, 60], 256, 272), ([1], 16, 16), ([513, 40], 2048, 144 if b_transposed else 150),
+                        ([300, 2, 700], 4096, 1024)]:
+        m, e = sum(sizes), len(sizes)
+        a = _q(randn_bf16((m, k), g, 4.0), E4M3).to(dev)
+        b = _q(randn_bf16((e, k, n) if b_transposed else (e, n, k), g, 4.0), E4M3).to(dev)
+        a.view(torch.uint8)[m // 2, 3] = 0x7F   # a row of NaN
+        sa = torch.rand(e, generator=g).to(dev) * 1e-3
+        sb = torch.full((e,), 3e38, device=dev) if n == 1024 else torch.rand(e, generator=g).to(dev)
+        with backend.gemm_options(tile=tile):
+            want = backend.fp8_gmm(a, b, torch.tensor(sizes), None, None, b_transposed=b_transposed)
+            backend.multi_scale_mul(list(torch.split(want, sizes)), sa, sb)
+            got = backend.fp8_gmm(a, b, torch.tensor(sizes), sa, sb, cutlass=True, b_transposed=b_transposed)
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (sizes, k, n)
+
+
 def test_random_problem_lists_are_exact(dev):
     """Sixty random grouped problems (ragged and empty experts, K and N that are not tile multiples, both operand
     formats, the stacked and the list calling form).  Operands come from {0, +-0.25 .. +-2} and the scales are

@@ -421,6 +421,36 @@ def test_weights_cast_ahead_of_the_pass_give_the_same_bits(dev, kind):
         mods[0](data[0][0], torch.tensor(data[0][1]), is_first_microbatch=True)
 
 
+def test_cutlass_passes_equal_the_per_launch_path(dev):
+    """GroupedLinear(cutlass=True) runs its passes from native code like the default: the bits of the per-launch entry
+    points, cached weights and a frozen weight included; forward-mode differentiation is refused."""
+    pkg = _pkg()
+    e, h, f = 4, 160, 336
+    g = gen(515)
+    mods = [pkg.GroupedLinear(h, f, e, torch.bfloat16, device=dev, cutlass=True, planned_passes=p) for p in (True, False)]
+    mods[1].load_state_dict(mods[0].state_dict())
+    for step, (sizes, first) in enumerate([([70, 0, 301, 5], None), ([1, 1, 1, 1], True), ([40, 300, 0, 90], False)]):
+        x, dy = randn_bf16((sum(sizes), h), g).to(dev), randn_bf16((sum(sizes), f), g, 1e-2).to(dev)
+        res = []
+        for mod in mods:
+            mod.zero_grad()
+            mod.weight_tensor.requires_grad_(step != 2)
+            xi = x.clone().requires_grad_()
+            out = mod(xi, torch.tensor(sizes), is_first_microbatch=first)
+            out.backward(dy)
+            res.append([out, xi.grad] + ([mod.weight_tensor.grad] if step != 2 else []))
+        for a, b in zip(*res):
+            assert torch.equal(a.view(torch.int16), b.view(torch.int16)), step
+        for name in ("scaling_fwd", "scaling_bwd"):
+            for a, b in zip(mods[0].fp8_meta[name].state().values(), mods[1].fp8_meta[name].state().values()):
+                assert torch.equal(a, b), (step, name)
+    with torch.autograd.forward_ad.dual_level():
+        for mod in mods:
+            dual = torch.autograd.forward_ad.make_dual(x.clone(), torch.ones_like(x))
+            with pytest.raises(RuntimeError):
+                mod(dual, torch.tensor(sizes))
+
+
 def test_grouped_mlp_frozen_weights_against_the_oracle(dev):
     """No weight gradients: padded transposes are skipped and d(pre-GELU) goes through the cast-only dGELU
     kernel; output and grad_input must still be the oracle's."""
