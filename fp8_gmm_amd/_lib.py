@@ -24,6 +24,8 @@ GEMM_B_KMAJOR = 2
 GEMM_A_KMAJOR = 4
 GEMM_TILE_128 = 0x100   # planning flag: 128 x 128 tiles, two workgroups per compute unit
 GEMM_TILE_DUAL = 0x200  # planning flag: 128 x 256 tiles for the kernel form with two sets of accumulators
+GEMM_TILE_ROWS = 0x400
+GEMM_ROWS_TILE_M = 64
 
 OP_QUANTIZE = 0
 OP_SCALE_MUL = 1

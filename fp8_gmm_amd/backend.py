@@ -103,7 +103,9 @@ def gemm_form(a_fmt, flags, plan=None):
     also the tile where it is not the 256 x 256 one."""
     fmt = "e5m2" if a_fmt == _lib.E5M2 else "e4m3"
     tile = ""
-    if plan is not None and plan.tile_m not in (0, plan.tile):
+    if plan is not None and plan.tile_m == _lib.GEMM_ROWS_TILE_M:
+        tile = f"; {plan.tile_m} x {plan.tile} tiles, few rows"
+    elif plan is not None and plan.tile_m not in (0, plan.tile):
         tile = f"; {plan.tile_m} x {plan.tile} tiles, two sets of accumulators"
     elif plan is not None and plan.tile not in (0, 256):
         tile = f"; {plan.tile} x {plan.tile} tiles"
@@ -792,7 +794,9 @@ def _launch_gemm(table, a_dtype, b_dtype, c_dtype, gelu, device, keep, b_kmajor=
     layout = (_lib.GEMM_B_KMAJOR if b_kmajor else 0) | (_lib.GEMM_A_KMAJOR if a_kmajor else 0)
     grid = _lib.gemm_grid(_lib.init(device.index if device.index is not None else torch.cuda.current_device()))
     epi = _lib.EPI_GELU if gelu else _lib.EPI_DGELU if dgelu else 0
-    if not epi and _small_tiles(table):
+    if not dgelu and not layout and _rows_tiles(table):
+        plan, blob, off_items, off_fix = _lib.plan_grouped_gemm_blob(table, epi | _lib.GEMM_TILE_ROWS, 2 * grid, False)
+    elif not epi and _small_tiles(table):
         plan, blob, off_items, off_fix = _lib.plan_grouped_gemm_blob(table, layout | _lib.GEMM_TILE_128, 2 * grid, False)
     elif not epi and c_dtype == torch.bfloat16 and _dual_tiles(table, a_kmajor):
         plan, blob, off_items, off_fix = _lib.plan_grouped_gemm_blob(table, layout | _lib.GEMM_TILE_DUAL, grid, False)
@@ -838,7 +842,7 @@ def _launch_gemm(table, a_dtype, b_dtype, c_dtype, gelu, device, keep, b_kmajor=
 # Tail balancing of the grouped GEMM (the workgroups of an XCD share their range's last tiles along K) needs
 # scratch memory for partial sums and a second, small launch; options.stream_k = False plans every launch without it.
 class GemmOptions:
-    """Launch policy of the grouped GEMMs of this process: ``tile`` "auto" | "256" | "128" | "dual", ``stream_k`` (share the
+    """Launch policy of the grouped GEMMs of this process: ``tile`` "auto" | "256" | "128" | "dual" | "rows", ``stream_k`` (share the
     tail tiles of a launch along K), ``wgrad`` "in_place" | "copy", ``upload`` "kernel" (tables reach the device
     through staging memory and a copy kernel of the library) | "copy" (a pinned buffer per upload and torch's
     asynchronous copy; while a stream is being captured into a graph the tables always take the first way, from
@@ -856,7 +860,7 @@ class GemmOptions:
 
 
 options = GemmOptions()
-TILE_POLICIES = {"auto": 0, "256": 256, "128": 128, "dual": _lib.GEMM_TILE_DUAL}
+TILE_POLICIES = {"auto": 0, "256": 256, "128": 128, "dual": _lib.GEMM_TILE_DUAL, "rows": _lib.GEMM_TILE_ROWS}
 
 
 @contextlib.contextmanager
@@ -894,6 +898,22 @@ def _dual_tiles(table, a_kmajor):
         return False
     m, n, k = (table[f].astype(np.int64) for f in ("m", "n", "k"))
     return int(k.max()) <= _DUAL_MAX_K and int(((m + n) * k + 2 * m * n).sum()) <= _DUAL_MAX_BYTES
+
+
+# The form for few rows per problem (64 x 128 tiles, weights passing by once): csrc/pass_plan.cpp, rows_pay, has the rule
+# and its measurements.
+def _rows_tiles(table):
+    if options.tile != "auto":
+        return options.tile == "rows"
+    m, n, k = (table[f].astype(np.int64) for f in ("m", "n", "k"))
+    used = m > 0
+    problems = int(used.sum())
+    if problems == 0:
+        return False
+    longest = int(k[used].max())
+    most = 64 if longest >= 4096 else 32 if longest >= 1024 else 16 if longest >= 512 else 0
+    return int((n * k)[used].sum()) >= 64 << 20 and 8 * int(((m + 63) // 64).sum()) <= 9 * problems \
+        and int(m.sum()) <= most * problems
 
 
 def _small_tiles(table):

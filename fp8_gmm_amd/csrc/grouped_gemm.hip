@@ -4,7 +4,7 @@
 // Replaces the reference's CUTLASS grouped GEMM (csrc/fp8_gmm.cu:82-205) and its per-expert cuBLASLt loops
 // (fp8_gmm/backend.py:84-96, grouped_linear.py:173-182, grouped_mlp.py:234-242,313-322) with ONE launch over
 // device-side tables written by the host planner (plan.cpp).
-#include "grouped_gemm_kernel.h"
+#include "grouped_gemm_rows.h"
 #include "internal.h"
 
 // Scratch of fp8gmm_grouped_gemm_static: the tail-balancing workspace for callers that cannot allocate one.
@@ -178,6 +178,20 @@ int scratch_for(int dev, uint8_t** out) {
   return FP8GMM_OK;
 }
 
+// "may use its LDS" of the form for few rows, as prepare_variant sets it for the others
+template <int A_FMT, int B_FMT>
+int prepare_rows(int dev) {
+  static std::atomic<bool> attr_set[kMaxDevices];
+  if (dev < 0 || dev >= kMaxDevices) return FP8GMM_ERR_NO_DEVICE;
+  if (!attr_set[dev].load(std::memory_order_acquire)) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(grouped_gemm_rows_kernel<A_FMT, B_FMT>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, kRowsLds) != hipSuccess)
+      return FP8GMM_ERR_LAUNCH;
+    attr_set[dev].store(true, std::memory_order_release);
+  }
+  return FP8GMM_OK;
+}
+
 typedef int (*launch_fn)(const fp8gmm_gemm_problem*, const fp8gmm_gemm_item*, int, int, int, uint8_t*,
                          const fp8gmm_tensor_desc*, int, hipStream_t);
 
@@ -188,6 +202,26 @@ launch_fn variant_for(int a_fmt, int b_fmt, bool a_kmajor, bool b_kmajor, int ti
     return &launch_variant<AF, BF, AT, BT, TL>;
   FP8GMM_FOR_EACH_GEMM_VARIANT(FP8GMM_PICK)
 #undef FP8GMM_PICK
+  return nullptr;
+}
+
+// the form for few rows (grouped_gemm_rows.h), or null
+template <int A_FMT, int B_FMT>
+int launch_rows(const fp8gmm_gemm_problem* probs_dev, const fp8gmm_gemm_item* items_dev, int grid, int out_kind, int epilogue,
+                uint8_t*, const fp8gmm_tensor_desc* merge_descs, int merge_n, hipStream_t stream) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return FP8GMM_ERR_NO_DEVICE;
+  const int rc = prepare_rows<A_FMT, B_FMT>(dev);
+  if (rc != FP8GMM_OK) return rc;
+  hipLaunchKernelGGL((grouped_gemm_rows_kernel<A_FMT, B_FMT>), dim3(grid), dim3(NTHREADS), kRowsLds, stream, probs_dev,
+                     items_dev, out_kind, epilogue, merge_descs, merge_n);
+  return hipGetLastError() == hipSuccess ? FP8GMM_OK : FP8GMM_ERR_LAUNCH;
+}
+launch_fn rows_variant_for(int a_fmt, int b_fmt, bool b_kmajor) {
+  if (b_kmajor) return nullptr;
+  if (a_fmt == FP8GMM_E4M3 && b_fmt == FP8GMM_E4M3) return &launch_rows<FP8GMM_E4M3, FP8GMM_E4M3>;
+  if (a_fmt == FP8GMM_E5M2 && b_fmt == FP8GMM_E4M3) return &launch_rows<FP8GMM_E5M2, FP8GMM_E4M3>;
+  if (a_fmt == FP8GMM_E4M3 && b_fmt == FP8GMM_E5M2) return &launch_rows<FP8GMM_E4M3, FP8GMM_E5M2>;
   return nullptr;
 }
 
@@ -214,18 +248,20 @@ int launch_checked(const fp8gmm_gemm_problem* probs_dev, int n, const fp8gmm_gem
   // e5m2 x e5m2 does not exist (cuBLASLt rejects it too); the contraction-major forms are the gradient GEMMs,
   // whose b is a forward tensor (weight or activation), always e4m3
   int tile = plan->tile == 0 ? kGemmTileN : plan->tile;
+  const bool rows_form = tile == FP8GMM_GEMM_ROWS_TILE_N && plan->tile_m == FP8GMM_GEMM_ROWS_TILE_M;
   if (tile != kGemmTileN && tile != FP8GMM_GEMM_SMALL_TILE) return FP8GMM_ERR_BAD_ARGUMENT;
-  if (plan->tile_m != 0 && plan->tile_m != tile) {
+  if (!rows_form && plan->tile_m != 0 && plan->tile_m != tile) {
     // the form with two sets of accumulators: bf16 results only
     if (tile != kGemmTileN || plan->tile_m != FP8GMM_GEMM_DUAL_TILE_M || out_kind != FP8GMM_OUT_BF16)
       return FP8GMM_ERR_BAD_ARGUMENT;
     tile = kTileDual;
   }
-  // only the large tile is ever shared along K or has the fused epilogues
-  if (tile != kGemmTileM &&
-      (plan->n_slots != 0 || plan->n_fixups != 0 || (epilogue & (FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU))))
+  // only the large tile is ever shared along K or has all the fused epilogues
+  if (tile != kGemmTileM && (plan->n_slots != 0 || plan->n_fixups != 0 || (epilogue & FP8GMM_EPI_DGELU) ||
+                             ((epilogue & FP8GMM_EPI_GELU) && !rows_form)))
     return FP8GMM_ERR_BAD_ARGUMENT;
-  const launch_fn launch = variant_for(a_fmt, b_fmt, a_kmajor, b_kmajor, tile);
+  if (rows_form && a_kmajor) return FP8GMM_ERR_BAD_ARGUMENT;
+  const launch_fn launch = rows_form ? rows_variant_for(a_fmt, b_fmt, b_kmajor) : variant_for(a_fmt, b_fmt, a_kmajor, b_kmajor, tile);
   if (launch == nullptr) return FP8GMM_ERR_BAD_FORMAT;
   if (n == 0 || plan->total_tiles == 0) return merge_n > 0 ? FP8GMM_ERR_BAD_ARGUMENT : FP8GMM_OK;   // nothing would merge
   if (plan->grid <= 0 || (plan->grid % kNumXcd) != 0 || plan->rounds < 1) return FP8GMM_ERR_BAD_ARGUMENT;

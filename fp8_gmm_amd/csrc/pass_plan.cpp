@@ -141,7 +141,36 @@ bool dual_tiles_pay(const fp8gmm_gemm_problem* p, int n, int layout) {
   return k_max <= 2048 && bytes <= ((int64_t)320 << 20);
 }
 
+// ... and the form for few rows (FP8GMM_GEMM_TILE_ROWS): row-major weights of 64 MB or more that (nearly) every problem
+// reads for one tile of up to 64 rows.  The shorter the contraction, the more of a tile is its start and its result, and
+// the fewer rows it takes for the other forms to be as fast.  Measured, other forms -> this one in us, at 8 / 32 / 64 rows
+// per expert: K = 14336 (8 experts, 4096 columns) 104 / 105 / 106 -> 73 / 74 / 80; K = 4096 (16, 6400) 94 / 96 / 100 ->
+// 83 / 86 / 99; K = 2048 (64, 1024) 32 / 32 / 32 -> 27 / 28 / 33; K = 768 (128, 2048) 46 / 49 / 53 -> 41 / 49 / 60; K = 256
+// (64, 4096) 25 -> 25 and worse; with 34 MB of weights (16, K = 1024, 2048) 12.7 -> 13.5.
+bool rows_pay(const fp8gmm_gemm_problem* p, int n, int layout) {
+  if (layout != 0) return false;
+  int64_t weights = 0, rows = 0, tiles = 0, problems = 0;
+  int32_t k = 0;
+  for (int i = 0; i < n; ++i) {
+    if (p[i].m == 0) continue;
+    ++problems;
+    rows += p[i].m;
+    tiles += (p[i].m + FP8GMM_GEMM_ROWS_TILE_M - 1) / FP8GMM_GEMM_ROWS_TILE_M;
+    weights += (int64_t)p[i].n * p[i].k;
+    if (p[i].k > k) k = p[i].k;
+  }
+  const int64_t most = k >= 4096 ? 64 : k >= 1024 ? 32 : k >= 512 ? 16 : 0;   // rows per problem
+  return weights >= ((int64_t)64 << 20) && 8 * tiles <= 9 * problems && rows <= most * problems;
+}
+
+// what the forms with two workgroups per compute unit multiply the grid by
+int grid_of(int flag, int grid) { return flag == FP8GMM_GEMM_TILE_128 || flag == FP8GMM_GEMM_TILE_ROWS ? 2 * grid : grid; }
+
 int tile_flag(const fp8gmm_gemm_problem* probs, int n, const Pass& pass, const Pass::Launch& l) {
+  // (a pass's fused GELU stores e4m3 and its argument: what the form for few rows takes)
+  if ((l.epi & FP8GMM_EPI_DGELU) == 0 &&
+      (pass.tile_policy == FP8GMM_GEMM_TILE_ROWS ? l.gemm.layout == 0 : pass.tile_policy == 0 && rows_pay(probs, n, l.gemm.layout)))
+    return FP8GMM_GEMM_TILE_ROWS;
   const bool small = l.epi == 0 && (pass.tile_policy == 128 || (pass.tile_policy == 0 && small_tiles_pay(probs, n)));
   const bool dual = !small && l.epi == 0 && l.out_kind == FP8GMM_OUT_BF16 &&
                     (pass.tile_policy == FP8GMM_GEMM_TILE_DUAL ||
@@ -268,7 +297,7 @@ int write_pass(Pass& pass, void* blob, size_t blob_bytes, fp8gmm_pass_plan* out)
     // shared-tile records are few (at most one per workgroup): planned into a local array, appended afterwards
     static thread_local fp8gmm_gemm_fixup_desc fix[4096];
     const int rc = fp8gmm_plan_grouped_gemm_launch(
-        probs, e, l.gemm.layout | l.epi | flag, flag == FP8GMM_GEMM_TILE_128 ? 2 * pass.grid : pass.grid,
+        probs, e, l.gemm.layout | l.epi | flag, grid_of(flag, pass.grid),
         flag != 0 ? 0 : pass.stream_k, items, (int)room, fix, 4096, &rec->plan);
     if (rc != FP8GMM_OK && rc != FP8GMM_ERR_BUFFER_TOO_SMALL) return rc;
     if (rc == FP8GMM_ERR_BUFFER_TOO_SMALL) w.fits = false;
@@ -320,11 +349,11 @@ int lay_out_pass(Pass& pass, fp8gmm_pass_plan* out, PassTables* t) {
     const int flag = tile_flag(probs, e, pass, l);
     fp8gmm::GemmRanges* ranges = &t->ranges[t->n_gemms];
     const int rc = fp8gmm::plan_gemm_ranges(probs, e, l.gemm.layout | l.epi | flag,
-                                            flag == FP8GMM_GEMM_TILE_128 ? 2 * pass.grid : pass.grid,
+                                            grid_of(flag, pass.grid),
                                             flag != 0 ? 0 : pass.stream_k, &rec->plan, ranges);
     if (rc != FP8GMM_OK) return rc;
-    l.gemm.tile_n = flag == FP8GMM_GEMM_TILE_128 ? FP8GMM_GEMM_SMALL_TILE : fp8gmm::kGemmTileN;
-    l.gemm.tile_m = flag == 0 ? fp8gmm::kGemmTileM : 128;
+    l.gemm.tile_n = rec->plan.tile != 0 ? rec->plan.tile : fp8gmm::kGemmTileN;
+    l.gemm.tile_m = rec->plan.tile_m != 0 ? rec->plan.tile_m : l.gemm.tile_n;
     rec->table_offset = l.gemm.table_offset = take((int64_t)e * (int64_t)sizeof(fp8gmm_gemm_problem));
     rec->items_offset = l.gemm.items_offset = take((int64_t)ranges->rounds * ranges->grid * (int64_t)sizeof(fp8gmm_gemm_item));
     rec->fixups_offset = l.gemm.fixups_offset = take((int64_t)ranges->n_fixups * (int64_t)sizeof(fp8gmm_gemm_fixup_desc));
@@ -355,7 +384,7 @@ int check_sizes(int experts, const int64_t* group_sizes, int64_t tokens) {
   }
   return rows == tokens ? FP8GMM_OK : FP8GMM_ERR_BAD_SHAPE;
 }
-bool tile_policy_ok(int p) { return p == 0 || p == 128 || p == 256 || p == FP8GMM_GEMM_TILE_DUAL; }
+bool tile_policy_ok(int p) { return p == 0 || p == 128 || p == 256 || p == FP8GMM_GEMM_TILE_DUAL || p == FP8GMM_GEMM_TILE_ROWS; }
 
 void begin_pass(Pass& p, int experts, const int64_t* sizes, int grid, int stream_k, int tile_policy) {
   p.experts = experts;

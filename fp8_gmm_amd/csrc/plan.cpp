@@ -186,10 +186,31 @@ int fp8gmm_plan_grouped_gemm_layout(fp8gmm_gemm_problem* probs, int n, int layou
 // The work list of a launch: the schedule of gemm_schedule.h written out, one record per (workgroup, item), in
 // the order items[r * grid + workgroup]; the slots in use are renumbered from 0 in the order the workgroups
 // are walked, and the fix-up records name them by their new numbers.
-// The same launch cut into 128 x 128 tiles (FP8GMM_GEMM_TILE_128) or into 128 x 256 tiles for the kernel with two
-// sets of accumulators (FP8GMM_GEMM_TILE_DUAL): whole tiles only, the tile list in 8 contiguous ranges of equal
+// The same launch cut into 128 x 128 tiles (FP8GMM_GEMM_TILE_128), into 128 x 256 tiles for the kernel with two
+// sets of accumulators (FP8GMM_GEMM_TILE_DUAL), or into 64 x 128 tiles for few rows (FP8GMM_GEMM_TILE_ROWS): whole tiles only, the tile list in 8 contiguous ranges of equal
 // work, the workgroups of an XCD striding through their range.
-constexpr int kSmallTileOverhead = 3, kDualTileOverhead = 2;
+constexpr int kSmallTileOverhead = 3, kDualTileOverhead = 2, kRowsTileOverhead = 1;
+constexpr int kWholeTileForms = FP8GMM_GEMM_TILE_128 | FP8GMM_GEMM_TILE_DUAL | FP8GMM_GEMM_TILE_ROWS;
+// Tile and overhead of the form that `layout` asks for; false when it names none that exists with its other flags.
+static bool whole_tile_form(int layout, int* tm, int* tn, int* overhead) {
+  switch (layout & kWholeTileForms) {
+    case FP8GMM_GEMM_TILE_128:
+      *tm = *tn = FP8GMM_GEMM_SMALL_TILE;
+      *overhead = kSmallTileOverhead;
+      return (layout & (FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU)) == 0;
+    case FP8GMM_GEMM_TILE_DUAL:
+      *tm = FP8GMM_GEMM_DUAL_TILE_M;
+      *tn = fp8gmm::kGemmTileN;
+      *overhead = kDualTileOverhead;
+      return (layout & (FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU)) == 0;
+    case FP8GMM_GEMM_TILE_ROWS:
+      *tm = FP8GMM_GEMM_ROWS_TILE_M;
+      *tn = FP8GMM_GEMM_ROWS_TILE_N;
+      *overhead = kRowsTileOverhead;
+      return (layout & (FP8GMM_EPI_DGELU | FP8GMM_GEMM_A_KMAJOR | FP8GMM_GEMM_B_KMAJOR)) == 0;
+  }
+  return false;
+}
 // kOverhead: what a tile costs besides its steps, in K = 128 steps: epilogue and switch of a small tile on a
 // workgroup that shares its compute unit; with two sets of accumulators, the slower steps that carry the result.
 struct WholeTileCuts {
@@ -292,14 +313,10 @@ int fp8gmm_plan_grouped_gemm_launch(fp8gmm_gemm_problem* probs, int n, int layou
   if (plan == nullptr) return FP8GMM_ERR_NULL_POINTER;
   *plan = fp8gmm_gemm_plan{};
   if (grid <= 0 || (grid % kNumXcd) != 0 || max_items < 0 || max_fixups < 0) return FP8GMM_ERR_BAD_ARGUMENT;
-  if (layout & (FP8GMM_GEMM_TILE_128 | FP8GMM_GEMM_TILE_DUAL)) {
-    if (layout & (FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU)) return FP8GMM_ERR_BAD_ARGUMENT;
-    if ((layout & FP8GMM_GEMM_TILE_128) && (layout & FP8GMM_GEMM_TILE_DUAL)) return FP8GMM_ERR_BAD_ARGUMENT;
-    const int operands = layout & ~(FP8GMM_GEMM_TILE_128 | FP8GMM_GEMM_TILE_DUAL);
-    if (layout & FP8GMM_GEMM_TILE_128)
-      return plan_whole_tiles(FP8GMM_GEMM_SMALL_TILE, FP8GMM_GEMM_SMALL_TILE, kSmallTileOverhead, probs, n, operands, grid, items,
-                              max_items, plan);
-    return plan_whole_tiles(FP8GMM_GEMM_DUAL_TILE_M, kGemmTileN, kDualTileOverhead, probs, n, operands, grid, items, max_items,
+  if (layout & kWholeTileForms) {
+    int tm = 0, tn = 0, overhead = 0;
+    if (!whole_tile_form(layout, &tm, &tn, &overhead)) return FP8GMM_ERR_BAD_ARGUMENT;
+    return plan_whole_tiles(tm, tn, overhead, probs, n, layout & ~(kWholeTileForms | FP8GMM_EPI_GELU), grid, items, max_items,
                             plan);
   }
   plan->tile = kGemmTileM;
@@ -475,12 +492,12 @@ int plan_gemm_ranges(fp8gmm_gemm_problem* probs, int n, int layout, int grid, in
   *plan = fp8gmm_gemm_plan{};
   *out = GemmRanges{};
   if (grid <= 0 || (grid % kNumXcd) != 0) return FP8GMM_ERR_BAD_ARGUMENT;
-  if (layout & (FP8GMM_GEMM_TILE_128 | FP8GMM_GEMM_TILE_DUAL)) {
-    const bool small = (layout & FP8GMM_GEMM_TILE_128) != 0;
+  if (layout & kWholeTileForms) {
+    int tm = 0, tn = 0, overhead = 0;
+    if (!whole_tile_form(layout, &tm, &tn, &overhead)) return FP8GMM_ERR_BAD_ARGUMENT;
     WholeTileCuts cuts;
-    const int rc = cut_whole_tiles(small ? FP8GMM_GEMM_SMALL_TILE : FP8GMM_GEMM_DUAL_TILE_M, small ? FP8GMM_GEMM_SMALL_TILE : kGemmTileN,
-                                   small ? kSmallTileOverhead : kDualTileOverhead, probs, n,
-                                   layout & (FP8GMM_GEMM_A_KMAJOR | FP8GMM_GEMM_B_KMAJOR), grid, &cuts, plan);
+    const int rc = cut_whole_tiles(tm, tn, overhead, probs, n, layout & (FP8GMM_GEMM_A_KMAJOR | FP8GMM_GEMM_B_KMAJOR), grid,
+                                   &cuts, plan);
     if (rc != FP8GMM_OK || plan->total_tiles == 0) return rc;
     for (int x = 0; x < kNumXcd; ++x) {
       out->xcd[x].begin = cuts.cut[x];

@@ -182,6 +182,13 @@ typedef struct fp8gmm_gemm_problem {
  * shares tiles along K (stream_k is ignored).  No counterpart in the reference. */
 #define FP8GMM_GEMM_TILE_DUAL 0x200
 #define FP8GMM_GEMM_DUAL_TILE_M 128
+/* Planning flag (`layout` of fp8gmm_plan_grouped_gemm_launch only): cut the outputs into tiles of 64 rows x 128 columns for the
+ * form that streams the weights of problems with few rows (two workgroups per compute unit: pass a grid of
+ * 2 * fp8gmm_gemm_grid()).  For launches bound by reading b once.  Both operands row-major; any result,
+ * FP8GMM_EPI_DGELU excepted; never shares tiles along K (stream_k is ignored).  No counterpart in the reference. */
+#define FP8GMM_GEMM_TILE_ROWS 0x400
+#define FP8GMM_GEMM_ROWS_TILE_M 64
+#define FP8GMM_GEMM_ROWS_TILE_N 128
 
 /*
  * Work list of a grouped-GEMM launch, written by fp8gmm_plan_grouped_gemm_launch on the host and read by the
@@ -359,7 +366,8 @@ typedef struct fp8gmm_linear_pass {
   int32_t grid;                      /* fp8gmm_gemm_grid() of the device */
   int32_t stream_k;                  /* as for fp8gmm_plan_grouped_gemm_launch */
   int32_t tile_policy;               /* 0: the library chooses per launch; 256 or 128: that tile for every launch;
-                                        FP8GMM_GEMM_TILE_DUAL: the 128 x 256 form for every launch that can take it */
+                                        FP8GMM_GEMM_TILE_DUAL / FP8GMM_GEMM_TILE_ROWS: that form for every launch
+                                        that can take it */
   int32_t two_roundings;             /* != 0: y and dx are formed with FP8GMM_EPI_TWO_ROUNDINGS */
   int64_t tokens;                    /* rows of x / dy: must equal the sum of group_sizes */
   const int64_t* group_sizes;        /* HOST array [experts] */

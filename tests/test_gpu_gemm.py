@@ -408,6 +408,35 @@ def test_two_roundings_in_the_epilogue_equal_the_separate_scaling(dev, tile, b_t
         assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (sizes, k, n)
 
 
+@pytest.mark.parametrize("out", ["bf16", "two-roundings", "gelu-e4m3", "e5m2"])
+def test_the_form_for_few_rows_gives_the_same_bits(dev, out):
+    """64 x 128 tiles with streamed weights against the other forms: row counts around its blocks and tiles, column and
+    contraction remainders, pitches that take element stores only, empty experts, both operand formats, a NaN row."""
+    backend = _backend()
+    g = gen(88)
+    for sizes, k, n, fmt in [([1], 16, 16, E4M3), ([7, 0, 32, 33, 64], 256, 128, E4M3), ([65, 128, 2, 31], 400, 200, E5M2),
+                             ([5, 90, 63], 272, 150, E4M3), ([3] * 40, 1024, 768, E4M3)]:
+        m, e = sum(sizes), len(sizes)
+        a = _q(randn_bf16((m, k), g, 4.0), fmt).to(dev)
+        b = _q(randn_bf16((e, n, k), g, 4.0), E4M3).to(dev)
+        a.view(torch.uint8)[m // 2, 3] = 0x7F
+        sa, sb = torch.rand(e, generator=g).to(dev), torch.rand(e, generator=g).to(dev)
+        results = []
+        for tile in ("256", "rows"):
+            with backend.gemm_options(tile=tile, stream_k=False):
+                if out in ("bf16", "two-roundings"):
+                    c = backend.fp8_gmm(a, b, torch.tensor(sizes), sa, sb, cutlass=out == "two-roundings")
+                    results.append([c.view(torch.int16)])
+                    continue
+                pre = torch.zeros(m, n, dtype=torch.bfloat16, device=dev) if out == "gelu-e4m3" else None
+                c = torch.zeros(m, n, dtype=torch.uint8, device=dev).view(E4M3 if out == "gelu-e4m3" else E5M2)
+                amax = torch.zeros(e, device=dev)
+                backend.fp8_gmm(a, b, torch.tensor(sizes), sa, sb, c, pre_gelu_out=pre, c_scales=sb, c_amaxes=amax)
+                results.append([c.view(torch.uint8), amax] + ([pre.view(torch.int16)] if pre is not None else []))
+        for x, y in zip(*results):
+            assert torch.equal(x, y), (sizes, k, n)
+
+
 def test_random_problem_lists_are_exact(dev):
     """Sixty random grouped problems (ragged and empty experts, K and N that are not tile multiples, both operand
     formats, the stacked and the list calling form).  Operands come from {0, +-0.25 .. +-2} and the scales are

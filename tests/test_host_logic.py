@@ -265,3 +265,33 @@ def test_tensor_batch_describes_the_same_memory_as_views():
         TensorBatch.concat([b, s])  # dtypes differ
     with pytest.raises(RuntimeError):
         TensorBatch.rows_of(x.t(), [0, 1])  # not contiguous
+
+
+def test_the_rule_for_few_rows_is_the_same_in_both_planners():
+    """backend._rows_tiles and the pass planner's rows_pay choose the same launches, on either side of every bound."""
+    import numpy as np
+
+    from fp8_gmm_amd import _lib, backend
+
+    lib = _lib.load()
+    rng = np.random.default_rng(5)
+    taken = 0
+    for case in range(300):
+        experts = int(rng.choice([1, 8, 32, 64, 128]))
+        k, n = 16 * int(rng.integers(16, 400)), 16 * int(rng.integers(16, 400))
+        sizes = rng.integers(0, int(rng.choice([2, 17, 34, 66, 130])), size=experts).astype(np.int64)
+        sizes[rng.random(experts) < 0.2] = 0
+        d = _lib.LinearPass()
+        d.experts, d.in_features, d.out_features, d.grid, d.stream_k = experts, k, n, 256, 1
+        d.tokens, d.group_sizes = int(sizes.sum()), sizes.ctypes.data
+        for f in ("x", "x_fp8", "w_fp8", "y", "fwd_scale", "fwd_scale_inv", "fwd_amax"):
+            setattr(d, f, 1 << 20)
+        plan = _lib.PassPlan()
+        assert lib.fp8gmm_plan_linear_forward(d, None, 0, plan) == -8 or d.tokens == 0
+        table = np.zeros(experts, dtype=_lib.GEMM_PROBLEM)
+        table["m"], table["n"], table["k"] = sizes, n, k
+        want = backend._rows_tiles(table)
+        if d.tokens:
+            assert (plan.launch[1].plan.tile_m == _lib.GEMM_ROWS_TILE_M) == want, (experts, k, n, sizes)
+        taken += want
+    assert 20 < taken < 280
