@@ -111,10 +111,18 @@ void run_pass(int which, const void* desc, const at::Device& device, const Setup
                              (size_t)slots * FP8GMM_GEMM_SLOT_BYTES, stream));
 }
 
-void check_rows(const std::vector<int64_t>& sizes, const Tensor& x) {
+// The kernels follow addresses: what they read has to be there.  `w` [experts, out, x's columns].
+void check_shapes(const std::vector<int64_t>& sizes, const Tensor& x, const Tensor& w, const Setup& s, int gemms) {
   int64_t rows = 0;
-  for (const int64_t s : sizes) rows += s;
+  for (const int64_t n : sizes) rows += n;
   TORCH_CHECK(rows == x.size(0), "group_sizes must sum to the number of input rows");
+  TORCH_CHECK((int64_t)sizes.size() <= w.size(0), "fp8_gmm_amd: group_sizes has ", sizes.size(), " entries for ", w.size(0),
+              " weights");
+  TORCH_CHECK(x.size(1) == w.size(2), "fp8_gmm_amd: the input has ", x.size(1), " columns, the weights expect ", w.size(2));
+  const int64_t n = (int64_t)sizes.size() * gemms;   // scaling slots: 3 a GEMM forward, 2 backward
+  TORCH_CHECK(s.fwd_scale.numel() >= 3 * n && s.fwd_scale_inv.numel() >= 3 * n && s.fwd_amax.size(-1) >= 3 * n &&
+                  s.bwd_scale.numel() >= 2 * n && s.bwd_scale_inv.numel() >= 2 * n && s.bwd_amax.size(-1) >= 2 * n,
+              "fp8_gmm_amd: the scaling state has too few slots");
 }
 
 // Forward-mode differentiation has no rule here and is refused, as the Python functions refuse it: a tangent that is
@@ -187,7 +195,7 @@ Tensor linear_step(const Tensor& x, const Tensor& w, const py::object& group_siz
                    bool cast_weights, const Setup& setup, const Due& due) {
   std::vector<int64_t> sizes = sizes_of(group_sizes);
   py::gil_scoped_release no_gil;
-  check_rows(sizes, x);
+  check_shapes(sizes, x, w, setup, 1);
   check_no_tangent({x, w});
   const c10::OptionalDeviceGuard guard(x.device());
   const bool grad = at::GradMode::is_enabled();
@@ -303,7 +311,9 @@ Tensor mlp_step(const Tensor& x, const Tensor& w1, const Tensor& w2, const py::o
                 const Setup& setup, const Due& due) {
   std::vector<int64_t> sizes = sizes_of(group_sizes);
   py::gil_scoped_release no_gil;
-  check_rows(sizes, x);
+  check_shapes(sizes, x, w1, setup, 2);
+  TORCH_CHECK(w2.size(0) == w1.size(0) && w2.size(1) == w1.size(2) && w2.size(2) == w1.size(1),
+              "fp8_gmm_amd: fc2's weights do not follow fc1's");
   check_no_tangent({x, w1, w2});
   const c10::OptionalDeviceGuard guard(x.device());
   const bool grad = at::GradMode::is_enabled();

@@ -295,3 +295,27 @@ def test_the_rule_for_few_rows_is_the_same_in_both_planners():
             assert (plan.launch[1].plan.tile_m == _lib.GEMM_ROWS_TILE_M) == want, (experts, k, n, sizes)
         taken += want
     assert 20 < taken < 280
+
+
+def test_native_passes_refuse_operands_that_do_not_fit():
+    """The kernels follow addresses: widths, group counts and scaling slots that do not fit are refused on the host,
+    before anything is launched."""
+    from fp8_gmm_amd.native import Due, Setup, linear_step, mlp_step
+
+    def setup(experts, gemms):
+        f, b = torch.ones(3 * experts * gemms), torch.ones(2 * experts * gemms)
+        return Setup(0, 1, 256, f, f, f.reshape(1, -1), b, b, b.reshape(1, -1))
+
+    def bf16(*shape):
+        return torch.zeros(shape, dtype=torch.bfloat16)
+
+    with pytest.raises(RuntimeError, match="columns"):
+        linear_step(bf16(3, 16), bf16(2, 16, 32), [1, 2], None, True, setup(2, 1), Due())
+    with pytest.raises(RuntimeError, match="entries"):
+        linear_step(bf16(3, 16), bf16(2, 16, 16), [1, 1, 1], None, True, setup(3, 1), Due())
+    with pytest.raises(RuntimeError, match="slots"):
+        linear_step(bf16(3, 16), bf16(2, 16, 16), [1, 2], None, True, setup(1, 1), Due())
+    with pytest.raises(RuntimeError, match="columns"):
+        mlp_step(bf16(3, 32), bf16(2, 32, 16), bf16(2, 16, 32), [1, 2], None, None, True, setup(2, 2), Due())
+    with pytest.raises(RuntimeError, match="fc2"):
+        mlp_step(bf16(3, 16), bf16(2, 32, 16), bf16(2, 16, 16), [1, 2], None, None, True, setup(2, 2), Due())
