@@ -40,7 +40,7 @@ T* ptr(const Tensor& t) {
   return t.defined() ? static_cast<T*>(t.data_ptr()) : nullptr;
 }
 
-// Rows per expert, from a CPU tensor or a sequence.
+// Rows per expert, from a CPU tensor or anything that iterates over numbers.
 std::vector<int64_t> sizes_of(const py::object& group_sizes) {
   if (THPVariable_Check(group_sizes.ptr())) {
     const Tensor t = THPVariable_Unpack(group_sizes.ptr()).to(at::kCPU, at::kLong).contiguous();
@@ -48,7 +48,9 @@ std::vector<int64_t> sizes_of(const py::object& group_sizes) {
     const int64_t* p = t.const_data_ptr<int64_t>();
     return std::vector<int64_t>(p, p + t.numel());
   }
-  return py::cast<std::vector<int64_t>>(group_sizes);
+  std::vector<int64_t> sizes;
+  for (const py::handle n : py::iter(group_sizes)) sizes.push_back(py::cast<int64_t>(py::int_(py::reinterpret_borrow<py::object>(n))));
+  return sizes;
 }
 
 // How the launches of a module are planned, and its scaling state of both directions.

@@ -319,3 +319,15 @@ def test_native_passes_refuse_operands_that_do_not_fit():
         mlp_step(bf16(3, 32), bf16(2, 32, 16), bf16(2, 16, 32), [1, 2], None, None, True, setup(2, 2), Due())
     with pytest.raises(RuntimeError, match="fc2"):
         mlp_step(bf16(3, 16), bf16(2, 32, 16), bf16(2, 16, 16), [1, 2], None, None, True, setup(2, 2), Due())
+
+
+def test_native_passes_take_group_sizes_of_any_iterable():
+    """As ``cumsum_group_sizes`` does: every entry through ``int``."""
+    from fp8_gmm_amd.native import Due, Setup, linear_step
+
+    z = torch.ones(12).reshape(1, -1)
+    x, w = torch.zeros(4, 16, dtype=torch.bfloat16), torch.zeros(2, 16, 16, dtype=torch.bfloat16)
+    for sizes in ([1, 2], (1, 2), iter([1, 2]), [1.0, 2.0], torch.tensor([1, 2]).numpy(), [torch.tensor(1), 2],
+                  torch.tensor([1, 2], dtype=torch.int32)):
+        with pytest.raises(RuntimeError, match="must sum"):   # read, and not the input's four rows
+            linear_step(x, w, sizes, None, True, Setup(0, 1, 256, z, z, z, z, z, z), Due())
