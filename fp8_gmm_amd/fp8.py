@@ -96,6 +96,9 @@ class fp8_autocast(contextlib.ContextDecorator):  # noqa: N801 - TransformerEngi
         self.enabled, self.recipe = enabled, (fp8_recipe or DelayedScaling()) if enabled else None
         self.outer = []
 
+    def _recreate_cm(self):   # a block of its own for every call of a decorated function, which threads may share
+        return fp8_autocast(self.enabled, self.recipe)
+
     def __enter__(self):
         self.outer.append((_STATE.enabled, _STATE.recipe))
         _STATE.enabled, _STATE.recipe = self.enabled, self.recipe

@@ -331,3 +331,32 @@ def test_native_passes_take_group_sizes_of_any_iterable():
                   torch.tensor([1, 2], dtype=torch.int32)):
         with pytest.raises(RuntimeError, match="must sum"):   # read, and not the input's four rows
             linear_step(x, w, sizes, None, True, Setup(0, 1, 256, z, z, z, z, z, z), Due())
+
+
+def test_fp8_autocast_as_a_decorator_keeps_every_call_apart():
+    """A decorated function may run in two threads at once: each restores what its own thread had before."""
+    import threading
+
+    from fp8_gmm_amd.fp8 import _STATE, DelayedScaling, fp8_autocast
+
+    inside, leave, seen = threading.Barrier(2), [threading.Event(), threading.Event()], [None, None]
+
+    @fp8_autocast(enabled=True)
+    def body(i):
+        inside.wait(30)
+        leave[i].wait(30)
+
+    outer = [DelayedScaling(margin=1), DelayedScaling(margin=2)]
+
+    def thread(i):
+        with fp8_autocast(fp8_recipe=outer[i]):
+            body(i)
+            seen[i] = _STATE.recipe
+
+    threads = [threading.Thread(target=thread, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for i in range(2):
+        leave[i].set()
+        threads[i].join(30)
+    assert seen[0] is outer[0] and seen[1] is outer[1]
