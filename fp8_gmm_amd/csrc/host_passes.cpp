@@ -161,10 +161,12 @@ struct GroupedLinearBackward : public Node {
 
   std::string name() const override { return "GroupedLinearBackward"; }
   void release_variables() override {
+    const std::lock_guard<std::mutex> lock(mutex_);   // backward passes of several threads may meet in one graph
     x_fp8.reset_data();
     w_fp8.reset_data();
   }
   variable_list apply(variable_list&& grads) override {
+    const std::lock_guard<std::mutex> lock(mutex_);
     at::AutoGradMode no_grad(false);
     variable_list result(2);
     const bool dgrad = task_should_compute_output(0), wgrad = task_should_compute_output(1);
@@ -264,9 +266,11 @@ struct GroupedMlpBackward : public Node {
 
   std::string name() const override { return "GroupedMlpBackward"; }
   void release_variables() override {
+    const std::lock_guard<std::mutex> lock(mutex_);   // backward passes of several threads may meet in one graph
     for (SavedVariable* v : {&x_fp8, &w1_fp8, &w2_fp8, &pre, &act_fp8}) v->reset_data();
   }
   variable_list apply(variable_list&& grads) override {
+    const std::lock_guard<std::mutex> lock(mutex_);
     at::AutoGradMode no_grad(false);
     variable_list result(3);
     const bool want_x = dgrad && task_should_compute_output(0);
