@@ -53,6 +53,18 @@ std::vector<int64_t> sizes_of(const py::object& group_sizes) {
   return sizes;
 }
 
+// An exception of Python code that a pass calls - saved-tensor hooks; activation checkpointing ends its recomputation
+// with one - reaches the caller as it is.
+template <class F>
+Tensor with_python_errors(F&& pass) {
+  try {
+    return pass();
+  } catch (python_error& e) {
+    e.restore();
+    throw py::error_already_set();
+  }
+}
+
 // How the launches of a module are planned, and its scaling state of both directions.
 struct Setup {
   int fwd_fmt = 0, bwd_fmt = 0;
@@ -197,47 +209,48 @@ struct GroupedLinearBackward : public Node {
 
 Tensor linear_step(const Tensor& x, const Tensor& w, const py::object& group_sizes, const std::optional<Tensor>& cached,
                    bool cast_weights, const Setup& setup, const Due& due) {
-  std::vector<int64_t> sizes = sizes_of(group_sizes);
-  py::gil_scoped_release no_gil;
-  check_shapes(sizes, x, w, setup, 1);
-  check_no_tangent({x, w});
-  const c10::OptionalDeviceGuard guard(x.device());
-  const bool grad = at::GradMode::is_enabled();
-  const bool dgrad = grad && x.requires_grad(), wgrad = grad && w.requires_grad();
-  Tensor y, x_fp8, w_fp8, scale_inv;
-  {
-    at::AutoGradMode no_grad(false);
-    const auto fp8 = x.options().dtype(setup.fwd_type());
-    x_fp8 = at::empty(x.sizes(), fp8);
-    w_fp8 = cached.has_value() ? *cached : at::empty(w.sizes(), fp8);
-    y = at::empty({x.size(0), w.size(1)}, x.options());
-    if (dgrad || wgrad) scale_inv = at::empty_like(setup.fwd_scale_inv);
-    fp8gmm_linear_pass d = linear_desc(setup, sizes, x.size(0), w.size(2), w.size(1));
-    d.cast_weights = cast_weights;
-    d.x = ptr<void>(x);
-    d.x_fp8 = ptr<void>(x_fp8);
-    d.w = ptr<void>(w);
-    d.w_fp8 = ptr<void>(w_fp8);
-    d.y = ptr<void>(y);
-    d.fwd_scale = ptr<float>(setup.fwd_scale);
-    d.fwd_scale_inv = ptr<float>(setup.fwd_scale_inv);
-    d.fwd_amax = ptr<float>(setup.fwd_amax);
-    run_pass(FP8GMM_LINEAR_FORWARD, &d, x.device(), &setup, &due, scale_inv.defined() ? setup.fwd_scale_inv : Tensor(),
-             scale_inv);
-  }
-  if (dgrad || wgrad) {
-    auto node = std::shared_ptr<GroupedLinearBackward>(new GroupedLinearBackward(), torch::autograd::deleteNode);
-    node->set_next_edges(torch::autograd::collect_next_edges(x, w));
-    node->setup = setup;
-    node->sizes = std::move(sizes);
-    node->in = w.size(2);
-    node->out = w.size(1);
-    if (wgrad) node->x_fp8 = SavedVariable(x_fp8, false);
-    if (dgrad) node->w_fp8 = SavedVariable(w_fp8, false);
-    node->scale_inv = scale_inv;
-    torch::autograd::set_history(y, node);
-  }
-  return y;
+  return with_python_errors([&, sizes = sizes_of(group_sizes)]() mutable {
+    py::gil_scoped_release no_gil;
+    check_shapes(sizes, x, w, setup, 1);
+    check_no_tangent({x, w});
+    const c10::OptionalDeviceGuard guard(x.device());
+    const bool grad = at::GradMode::is_enabled();
+    const bool dgrad = grad && x.requires_grad(), wgrad = grad && w.requires_grad();
+    Tensor y, x_fp8, w_fp8, scale_inv;
+    {
+      at::AutoGradMode no_grad(false);
+      const auto fp8 = x.options().dtype(setup.fwd_type());
+      x_fp8 = at::empty(x.sizes(), fp8);
+      w_fp8 = cached.has_value() ? *cached : at::empty(w.sizes(), fp8);
+      y = at::empty({x.size(0), w.size(1)}, x.options());
+      if (dgrad || wgrad) scale_inv = at::empty_like(setup.fwd_scale_inv);
+      fp8gmm_linear_pass d = linear_desc(setup, sizes, x.size(0), w.size(2), w.size(1));
+      d.cast_weights = cast_weights;
+      d.x = ptr<void>(x);
+      d.x_fp8 = ptr<void>(x_fp8);
+      d.w = ptr<void>(w);
+      d.w_fp8 = ptr<void>(w_fp8);
+      d.y = ptr<void>(y);
+      d.fwd_scale = ptr<float>(setup.fwd_scale);
+      d.fwd_scale_inv = ptr<float>(setup.fwd_scale_inv);
+      d.fwd_amax = ptr<float>(setup.fwd_amax);
+      run_pass(FP8GMM_LINEAR_FORWARD, &d, x.device(), &setup, &due, scale_inv.defined() ? setup.fwd_scale_inv : Tensor(),
+               scale_inv);
+    }
+    if (dgrad || wgrad) {
+      auto node = std::shared_ptr<GroupedLinearBackward>(new GroupedLinearBackward(), torch::autograd::deleteNode);
+      node->set_next_edges(torch::autograd::collect_next_edges(x, w));
+      node->setup = setup;
+      node->sizes = std::move(sizes);
+      node->in = w.size(2);
+      node->out = w.size(1);
+      if (wgrad) node->x_fp8 = SavedVariable(x_fp8, false);
+      if (dgrad) node->w_fp8 = SavedVariable(w_fp8, false);
+      node->scale_inv = scale_inv;
+      torch::autograd::set_history(y, node);
+    }
+    return y;
+  });
 }
 
 // ---- GroupedMlp ---------------------------------------------------------------------------------------------------
@@ -315,64 +328,65 @@ struct GroupedMlpBackward : public Node {
 Tensor mlp_step(const Tensor& x, const Tensor& w1, const Tensor& w2, const py::object& group_sizes,
                 const std::optional<Tensor>& cached1, const std::optional<Tensor>& cached2, bool cast_weights,
                 const Setup& setup, const Due& due) {
-  std::vector<int64_t> sizes = sizes_of(group_sizes);
-  py::gil_scoped_release no_gil;
-  check_shapes(sizes, x, w1, setup, 2);
-  TORCH_CHECK(w2.size(0) == w1.size(0) && w2.size(1) == w1.size(2) && w2.size(2) == w1.size(1),
-              "fp8_gmm_amd: fc2's weights do not follow fc1's");
-  check_no_tangent({x, w1, w2});
-  const c10::OptionalDeviceGuard guard(x.device());
-  const bool grad = at::GradMode::is_enabled();
-  const bool dgrad = grad && x.requires_grad(), wgrad = grad && w1.requires_grad();
-  const int64_t tokens = x.size(0), hidden = x.size(1), ffn = w1.size(1);
-  Tensor y, x_fp8, w1_fp8, w2_fp8, pre, act_fp8, scale_inv;
-  {
-    at::AutoGradMode no_grad(false);
-    const auto fp8 = x.options().dtype(setup.fwd_type());
-    x_fp8 = at::empty(x.sizes(), fp8);
-    w1_fp8 = cached1.has_value() ? *cached1 : at::empty(w1.sizes(), fp8);
-    w2_fp8 = cached2.has_value() ? *cached2 : at::empty(w2.sizes(), fp8);
-    pre = at::empty({tokens, ffn}, x.options());
-    act_fp8 = at::empty({tokens, ffn}, fp8);
-    y = at::empty(x.sizes(), x.options());
-    if (dgrad || wgrad) scale_inv = at::empty_like(setup.fwd_scale_inv);
-    fp8gmm_mlp_pass d = mlp_desc(setup, sizes, tokens, hidden, ffn);
-    d.cast_weights = cast_weights;
-    d.x = ptr<void>(x);
-    d.x_fp8 = ptr<void>(x_fp8);
-    d.w1 = ptr<void>(w1);
-    d.w1_fp8 = ptr<void>(w1_fp8);
-    d.w2 = ptr<void>(w2);
-    d.w2_fp8 = ptr<void>(w2_fp8);
-    d.pre = ptr<void>(pre);
-    d.act_fp8 = ptr<void>(act_fp8);
-    d.y = ptr<void>(y);
-    d.fwd_scale = ptr<float>(setup.fwd_scale);
-    d.fwd_scale_inv = ptr<float>(setup.fwd_scale_inv);
-    d.fwd_amax = ptr<float>(setup.fwd_amax);
-    run_pass(FP8GMM_MLP_FORWARD, &d, x.device(), &setup, &due, scale_inv.defined() ? setup.fwd_scale_inv : Tensor(),
-             scale_inv);
-  }
-  if (dgrad || wgrad) {
-    auto node = std::shared_ptr<GroupedMlpBackward>(new GroupedMlpBackward(), torch::autograd::deleteNode);
-    node->set_next_edges(torch::autograd::collect_next_edges(x, w1, w2));
-    node->setup = setup;
-    node->sizes = std::move(sizes);
-    node->dgrad = dgrad;
-    node->wgrad = wgrad;
-    node->hidden = hidden;
-    node->ffn = ffn;
-    node->pre = SavedVariable(pre, false);
-    node->w2_fp8 = SavedVariable(w2_fp8, false);
-    if (dgrad) node->w1_fp8 = SavedVariable(w1_fp8, false);
-    if (wgrad) {
-      node->x_fp8 = SavedVariable(x_fp8, false);
-      node->act_fp8 = SavedVariable(act_fp8, false);
+  return with_python_errors([&, sizes = sizes_of(group_sizes)]() mutable {
+    py::gil_scoped_release no_gil;
+    check_shapes(sizes, x, w1, setup, 2);
+    TORCH_CHECK(w2.size(0) == w1.size(0) && w2.size(1) == w1.size(2) && w2.size(2) == w1.size(1),
+                "fp8_gmm_amd: fc2's weights do not follow fc1's");
+    check_no_tangent({x, w1, w2});
+    const c10::OptionalDeviceGuard guard(x.device());
+    const bool grad = at::GradMode::is_enabled();
+    const bool dgrad = grad && x.requires_grad(), wgrad = grad && w1.requires_grad();
+    const int64_t tokens = x.size(0), hidden = x.size(1), ffn = w1.size(1);
+    Tensor y, x_fp8, w1_fp8, w2_fp8, pre, act_fp8, scale_inv;
+    {
+      at::AutoGradMode no_grad(false);
+      const auto fp8 = x.options().dtype(setup.fwd_type());
+      x_fp8 = at::empty(x.sizes(), fp8);
+      w1_fp8 = cached1.has_value() ? *cached1 : at::empty(w1.sizes(), fp8);
+      w2_fp8 = cached2.has_value() ? *cached2 : at::empty(w2.sizes(), fp8);
+      pre = at::empty({tokens, ffn}, x.options());
+      act_fp8 = at::empty({tokens, ffn}, fp8);
+      y = at::empty(x.sizes(), x.options());
+      if (dgrad || wgrad) scale_inv = at::empty_like(setup.fwd_scale_inv);
+      fp8gmm_mlp_pass d = mlp_desc(setup, sizes, tokens, hidden, ffn);
+      d.cast_weights = cast_weights;
+      d.x = ptr<void>(x);
+      d.x_fp8 = ptr<void>(x_fp8);
+      d.w1 = ptr<void>(w1);
+      d.w1_fp8 = ptr<void>(w1_fp8);
+      d.w2 = ptr<void>(w2);
+      d.w2_fp8 = ptr<void>(w2_fp8);
+      d.pre = ptr<void>(pre);
+      d.act_fp8 = ptr<void>(act_fp8);
+      d.y = ptr<void>(y);
+      d.fwd_scale = ptr<float>(setup.fwd_scale);
+      d.fwd_scale_inv = ptr<float>(setup.fwd_scale_inv);
+      d.fwd_amax = ptr<float>(setup.fwd_amax);
+      run_pass(FP8GMM_MLP_FORWARD, &d, x.device(), &setup, &due, scale_inv.defined() ? setup.fwd_scale_inv : Tensor(),
+               scale_inv);
     }
-    node->scale_inv = scale_inv;
-    torch::autograd::set_history(y, node);
-  }
-  return y;
+    if (dgrad || wgrad) {
+      auto node = std::shared_ptr<GroupedMlpBackward>(new GroupedMlpBackward(), torch::autograd::deleteNode);
+      node->set_next_edges(torch::autograd::collect_next_edges(x, w1, w2));
+      node->setup = setup;
+      node->sizes = std::move(sizes);
+      node->dgrad = dgrad;
+      node->wgrad = wgrad;
+      node->hidden = hidden;
+      node->ffn = ffn;
+      node->pre = SavedVariable(pre, false);
+      node->w2_fp8 = SavedVariable(w2_fp8, false);
+      if (dgrad) node->w1_fp8 = SavedVariable(w1_fp8, false);
+      if (wgrad) {
+        node->x_fp8 = SavedVariable(x_fp8, false);
+        node->act_fp8 = SavedVariable(act_fp8, false);
+      }
+      node->scale_inv = scale_inv;
+      torch::autograd::set_history(y, node);
+    }
+    return y;
+  });
 }
 
 }  // namespace

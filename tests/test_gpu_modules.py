@@ -921,3 +921,36 @@ def test_tables_built_on_the_device_are_those_of_the_host_planner(dev, sizes, h,
                 used[off: off + nbytes] = True
         assert np.all(got[~used] == 0xAB)
         assert dst.tolist() == [0.0, 1.0, 2.0, 3.0, 4.0, 0.0]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["linear", "mlp"])
+def test_passes_under_activation_checkpointing_and_saved_tensor_hooks(dev, kind):
+    """Checkpointing ends its recomputation with an exception out of the last saved tensor's hook: the bits of the
+    per-launch path under the same checkpoint.  An exception of a user's hook arrives as it was raised."""
+    from torch.utils.checkpoint import checkpoint
+
+    pkg = _pkg()
+    sizes, g = torch.tensor([70, 0, 33]), gen(77)
+    mods = [pkg.GroupedLinear(64, 64, 3, torch.bfloat16, device=dev) if kind == "linear" else
+            pkg.GroupedMlp(64, 96, 3, torch.bfloat16, device=dev) for _ in range(2)]
+    mods[1].load_state_dict(mods[0].state_dict())
+    mods[1].fp8_meta["planned_passes"] = False
+    x, dy = randn_bf16((103, 64), g).to(dev), randn_bf16((103, 64), g, 1e-2).to(dev)
+    res = []
+    for mod in mods:
+        xi = x.clone().requires_grad_()
+        out = checkpoint(mod, xi, sizes, use_reentrant=False)
+        out.backward(dy)
+        res.append([out, xi.grad] + [p.grad for p in mod.parameters()])
+    for a, b in zip(*res):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+    class Stop(Exception):
+        pass
+
+    def pack(t):
+        raise Stop
+
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t), pytest.raises(Stop):
+        mods[0](x.clone().requires_grad_(), sizes)
