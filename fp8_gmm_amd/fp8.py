@@ -195,6 +195,13 @@ class Fp8WeightCache:
                 "weights" + (" with their transposes (it ran without gradients)" if self.valid else ""))
 
 
+def refuse_tracing():
+    """A recorded graph would hold the allocation of a pass's result and not the launches that write it."""
+    if torch.jit.is_tracing() or torch._C._get_dispatch_mode(torch._C._TorchDispatchModeKey.PROXY) is not None:
+        raise RuntimeError("fp8_gmm_amd: the grouped modules cannot be traced (torch.jit.trace, make_fx): a tracer does not "
+                           "see their kernels")
+
+
 class Fp8GroupedModuleBase(torch.nn.Module):
     """The slice of ``TransformerEngineBaseModule`` the grouped modules rely on."""
 

@@ -27,7 +27,7 @@ import torch
 from . import _lib
 from .backend import (TensorBatch, batched_uploads, fp8_gmm, grouped_gemm, linear_pass, multi_cast_transpose,
                       multi_quantize, wgrad_wants_transposed_gradient)
-from .fp8 import Fp8GroupedModuleBase, Fp8WeightCache, get_fp8_te_dtype
+from .fp8 import Fp8GroupedModuleBase, Fp8WeightCache, get_fp8_te_dtype, refuse_tracing
 from .native import linear_step
 from .utils import PAD_MULTIPLE, Fp8MetaWrapper, Fp8TensorType, MetaTensorType, cumsum_group_sizes, to_torch_dtype
 
@@ -365,6 +365,7 @@ class GroupedLinear(Fp8GroupedModuleBase):
 
     def forward(self, input, group_sizes, is_first_microbatch=None):
         ahead = self._take_ahead(is_first_microbatch)
+        refuse_tracing()
         due = None
         if ahead is None:
             due = self._prepare(input.device, is_first_microbatch, self.num_groups)

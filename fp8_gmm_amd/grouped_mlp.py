@@ -41,7 +41,7 @@ from .backend import (
     multi_transpose,
     wgrad_wants_transposed_gradient,
 )
-from .fp8 import Fp8GroupedModuleBase, Fp8WeightCache, get_fp8_te_dtype
+from .fp8 import Fp8GroupedModuleBase, Fp8WeightCache, get_fp8_te_dtype, refuse_tracing
 from .grouped_linear import MODULE_PAD_MULTIPLE, alloc_transposed, row_slices, stage_weight_cast, transposed_views
 from .native import mlp_step
 from .utils import PAD_MULTIPLE, Fp8MetaWrapper, Fp8TensorType, MetaTensorType, cumsum_group_sizes, to_torch_dtype
@@ -449,6 +449,7 @@ class GroupedMlp(Fp8GroupedModuleBase):
 
     def forward(self, input, group_sizes, has_tp=False, tp_group=None, is_first_microbatch=None):
         ahead = self._take_ahead(is_first_microbatch)
+        refuse_tracing()
         due = None
         if ahead is None:
             due = self._prepare(input.device, is_first_microbatch, self.num_groups * 2)

@@ -360,3 +360,22 @@ def test_fp8_autocast_as_a_decorator_keeps_every_call_apart():
         leave[i].set()
         threads[i].join(30)
     assert seen[0] is outer[0] and seen[1] is outer[1]
+
+
+@pytest.mark.parametrize("grad", [True, False])
+@pytest.mark.parametrize("kind", ["linear", "mlp"])
+def test_modules_refuse_to_be_traced(kind, grad):
+    """A tracer sees the allocation of a pass's result and none of the launches that write it: the recorded graph would
+    return uninitialised memory.  With and without gradients, before anything of the module has changed."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    from fp8_gmm_amd import GroupedLinear, GroupedMlp
+
+    module = (GroupedLinear if kind == "linear" else GroupedMlp)(16, 32, 2, torch.bfloat16, device="cpu")
+    x = torch.zeros(3, 16, dtype=torch.bfloat16, requires_grad=grad)
+    with torch.set_grad_enabled(grad):
+        with pytest.raises(RuntimeError, match="cannot be traced"):
+            torch.jit.trace(module, (x, torch.tensor([1, 2])), check_trace=False)
+        with pytest.raises(RuntimeError, match="cannot be traced"):
+            make_fx(lambda t: module(t, [1, 2]))(x)
+    assert module._fp8_steps == 0
