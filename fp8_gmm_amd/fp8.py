@@ -180,10 +180,11 @@ class Fp8WeightCache:
         return self.fp8, self.fp8_t
 
     def take(self, weight, setup, refresh):
-        """The row-major buffer for a pass that casts into it (``refresh``) or reuses it."""
+        """The row-major buffer for a pass that casts into it (``refresh``) or reuses it.  A refreshed one is valid once
+        the caller says so, behind the pass: one that was refused or failed has cast nothing."""
         fp8, _ = self.buffers(weight, torch.float8_e4m3fn if setup.fwd_fmt == 0 else torch.float8_e5m2, False)
         if refresh:
-            self.valid, self.valid_t = True, False
+            self.valid = self.valid_t = False
         else:
             self.require(False)
         return fp8

@@ -380,7 +380,10 @@ class GroupedLinear(Fp8GroupedModuleBase):
             setup = self._native_setup(input.device)
             setup.two_roundings = bool(self.cutlass)
             held = cache.take(weight, setup, refresh) if cache is not None else None
-            return linear_step(input, weight, group_sizes, held, refresh, setup, self._native_due(due))
+            out = linear_step(input, weight, group_sizes, held, refresh, setup, self._native_due(due))
+            if held is not None:
+                cache.valid = True
+            return out
         self._run_update(due)
         grad = torch.is_grad_enabled()
         args = (input, weight, group_sizes, self.fp8_meta, grad, self.cutlass)

@@ -464,7 +464,10 @@ class GroupedMlp(Fp8GroupedModuleBase):
             setup = self._native_setup(input.device)
             held1, held2 = (c.take(w, setup, refresh) for c, w in zip(caches, (w1, w2))) if caches is not None \
                 else (None, None)
-            return mlp_step(input, w1, w2, group_sizes, held1, held2, refresh, setup, self._native_due(due))
+            out = mlp_step(input, w1, w2, group_sizes, held1, held2, refresh, setup, self._native_due(due))
+            if caches is not None:
+                caches[0].valid = caches[1].valid = True
+            return out
         self._run_update(due)
         grad = torch.is_grad_enabled()
         args = (input, w1, w2, group_sizes, self.fp8_meta, grad, has_tp, tp_group)

@@ -379,3 +379,28 @@ def test_modules_refuse_to_be_traced(kind, grad):
         with pytest.raises(RuntimeError, match="cannot be traced"):
             make_fx(lambda t: module(t, [1, 2]))(x)
     assert module._fp8_steps == 0
+
+
+def _native_module_on_the_cpu(monkeypatch, kind):
+    """A module that takes the native path with CPU tensors: good for calls that are refused before any launch."""
+    from fp8_gmm_amd import GroupedLinear, GroupedMlp, _lib
+
+    cls = GroupedLinear if kind == "linear" else GroupedMlp
+    monkeypatch.setattr(cls, "_native", lambda self, *tensors: True)
+    monkeypatch.setattr(_lib, "device_grid", lambda index: 256)
+    return cls(16, 32, 2, torch.bfloat16, device="cpu")
+
+
+@pytest.mark.parametrize("kind", ["linear", "mlp"])
+def test_a_refused_first_microbatch_leaves_no_valid_weight_cache(monkeypatch, kind):
+    """A first micro-batch that raises has cast nothing: the next one must not compute with what the buffer holds, neither
+    uninitialised memory nor the weights of the step before."""
+    module = _native_module_on_the_cpu(monkeypatch, kind)
+    x = torch.zeros(3, 16, dtype=torch.bfloat16)
+    for earlier in (False, True):
+        for cache in module._weight_caches:
+            cache.valid = earlier
+        with pytest.raises(RuntimeError, match="must sum"):
+            module(x, [1, 1], is_first_microbatch=True)
+        with pytest.raises(RuntimeError, match="no earlier pass"):
+            module(x, [1, 2], is_first_microbatch=False)
