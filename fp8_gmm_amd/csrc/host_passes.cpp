@@ -75,7 +75,7 @@ struct Setup {
   at::ScalarType bwd_type() const { return bwd_fmt == FP8GMM_E4M3 ? at::kFloat8_e4m3fn : at::kFloat8_e5m2; }
 };
 
-// The scaling update that is due in front of a pass.
+// The scaling update that is due in front of a pass; not any more once it is enqueued.
 struct Due {
   bool due = false;
   double fwd_max = 0, bwd_max = 0;
@@ -84,7 +84,7 @@ struct Due {
 };
 
 // Builds the tables of a pass and enqueues its launches on the current stream.
-void run_pass(int which, const void* desc, const at::Device& device, const Setup* update, const Due* due, const Tensor& snapshot_of,
+void run_pass(int which, const void* desc, const at::Device& device, const Setup* update, Due* due, const Tensor& snapshot_of,
               const Tensor& snapshot) {
   fp8gmm_pass_plan plan;
   alignas(16) unsigned char tables[FP8GMM_PASS_TABLES_BYTES];
@@ -115,6 +115,7 @@ void run_pass(int which, const void* desc, const at::Device& device, const Setup
   }
   check(fp8gmm_build_pass(tables, blob.data_ptr(), updates, n, ptr<const float>(snapshot_of), ptr<float>(snapshot),
                           snapshot.defined() ? (int)snapshot.numel() : 0, stream));
+  if (due != nullptr) due->due = false;
   int slots = 0;
   for (int i = 0; i < plan.n_launches; ++i) slots = std::max(slots, plan.launch[i].plan.n_slots);
   // partial sums of tiles shared along K: from the caching allocator, which hands memory out again in stream order
@@ -208,7 +209,7 @@ struct GroupedLinearBackward : public Node {
 };
 
 Tensor linear_step(const Tensor& x, const Tensor& w, const py::object& group_sizes, const std::optional<Tensor>& cached,
-                   bool cast_weights, const Setup& setup, const Due& due) {
+                   bool cast_weights, const Setup& setup, Due& due) {
   return with_python_errors([&, sizes = sizes_of(group_sizes)]() mutable {
     py::gil_scoped_release no_gil;
     check_shapes(sizes, x, w, setup, 1);
@@ -327,7 +328,7 @@ struct GroupedMlpBackward : public Node {
 
 Tensor mlp_step(const Tensor& x, const Tensor& w1, const Tensor& w2, const py::object& group_sizes,
                 const std::optional<Tensor>& cached1, const std::optional<Tensor>& cached2, bool cast_weights,
-                const Setup& setup, const Due& due) {
+                const Setup& setup, Due& due) {
   return with_python_errors([&, sizes = sizes_of(group_sizes)]() mutable {
     py::gil_scoped_release no_gil;
     check_shapes(sizes, x, w1, setup, 2);
@@ -416,7 +417,8 @@ PYBIND11_MODULE(_host, m) {
       .def(py::init<>())
       .def(py::init([](double fwd_max, double bwd_max, int margin, bool most_recent, bool keep_weights) {
         return Due{true, fwd_max, bwd_max, margin, most_recent, keep_weights};
-      }));
+      }))
+      .def_readonly("due", &Due::due);
   m.def("linear_step", &linear_step);
   m.def("mlp_step", &mlp_step);
 }

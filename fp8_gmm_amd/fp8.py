@@ -317,14 +317,25 @@ class Fp8GroupedModuleBase(torch.nn.Module):
         setup.tile_policy = backend.TILE_POLICIES[backend.options.tile]
         return setup
 
-    def _native_due(self, due):
+    def _native_pass(self, step, input, weights, group_sizes, caches, refresh, setup, due):
+        """A pass of the native host path, ``step``, behind the scaling update that ``_prepare`` found due, with the fp8
+        weights of ``caches`` (None: temporaries).  A refused pass leaves the scaling state as the other paths do: updated."""
         from .native import Due
 
-        if due is None:
-            return Due()
         meta = self.fp8_meta
         r = meta["recipe"]
-        return Due(meta["fp8_max_fwd"], meta["fp8_max_bwd"], int(r.margin), r.amax_compute_algo != "max", due[0])
+        native_due = Due() if due is None else Due(meta["fp8_max_fwd"], meta["fp8_max_bwd"], int(r.margin),
+                                                   r.amax_compute_algo != "max", due[0])
+        try:
+            held = [None] * len(weights) if caches is None else [c.take(w, setup, refresh) for c, w in zip(caches, weights)]
+            out = step(input, *weights, group_sizes, *held, refresh, setup, native_due)
+        except BaseException:
+            if native_due.due:
+                self._run_update(due)
+            raise
+        for cache in caches or ():
+            cache.valid = True
+        return out
 
     def _cast_ahead(self, weights_and_groups):
         """The part of a forward pass that needs no group sizes, run now: the delayed-scaling update and the cast of

@@ -370,25 +370,21 @@ class GroupedLinear(Fp8GroupedModuleBase):
         if ahead is None:
             due = self._prepare(input.device, is_first_microbatch, self.num_groups)
         # the fp8 weights: temporaries of the pass, or the buffers of a cache that the pass refreshes or reuses
-        cache, refresh = None, True
+        caches, refresh = None, True
         if ahead is not None:
-            cache, refresh = ahead[0], False
+            caches, refresh = ahead, False
         elif is_first_microbatch is not None:
-            cache, refresh = self._weight_cache, bool(is_first_microbatch)
+            caches, refresh = (self._weight_cache,), bool(is_first_microbatch)
         weight = self.weight_tensor
         if self._native(input, weight):
             setup = self._native_setup(input.device)
             setup.two_roundings = bool(self.cutlass)
-            held = cache.take(weight, setup, refresh) if cache is not None else None
-            out = linear_step(input, weight, group_sizes, held, refresh, setup, self._native_due(due))
-            if held is not None:
-                cache.valid = True
-            return out
+            return self._native_pass(linear_step, input, (weight,), group_sizes, caches, refresh, setup, due)
         self._run_update(due)
         grad = torch.is_grad_enabled()
         args = (input, weight, group_sizes, self.fp8_meta, grad, self.cutlass)
-        if cache is not None:
-            args += (cache, refresh)
+        if caches is not None:
+            args += (caches[0], refresh)
         if grad:
             return _GroupedLinear.apply(*args)
         return _GroupedLinear.forward(None, *args)

@@ -462,12 +462,7 @@ class GroupedMlp(Fp8GroupedModuleBase):
         w1, w2 = self.fc1_weight, self.fc2_weight
         if not has_tp and not self.fp8_meta["fused_dgelu"] and "capture" not in self.fp8_meta and self._native(input, w1, w2):
             setup = self._native_setup(input.device)
-            held1, held2 = (c.take(w, setup, refresh) for c, w in zip(caches, (w1, w2))) if caches is not None \
-                else (None, None)
-            out = mlp_step(input, w1, w2, group_sizes, held1, held2, refresh, setup, self._native_due(due))
-            if caches is not None:
-                caches[0].valid = caches[1].valid = True
-            return out
+            return self._native_pass(mlp_step, input, (w1, w2), group_sizes, caches, refresh, setup, due)
         self._run_update(due)
         grad = torch.is_grad_enabled()
         args = (input, w1, w2, group_sizes, self.fp8_meta, grad, has_tp, tp_group)

@@ -404,3 +404,21 @@ def test_a_refused_first_microbatch_leaves_no_valid_weight_cache(monkeypatch, ki
             module(x, [1, 1], is_first_microbatch=True)
         with pytest.raises(RuntimeError, match="no earlier pass"):
             module(x, [1, 2], is_first_microbatch=False)
+
+
+@pytest.mark.parametrize("reuse", [False, True])
+@pytest.mark.parametrize("kind", ["linear", "mlp"])
+def test_a_refused_native_pass_keeps_its_scaling_update(monkeypatch, kind, reuse):
+    """The update that is due in front of a pass has taken its turn (``interval`` counts passes): where the pass is refused
+    it is run all the same, once, as it is in front of the other paths."""
+    module = _native_module_on_the_cpu(monkeypatch, kind)
+    x = torch.zeros(3, 16, dtype=torch.bfloat16)
+    recipe = fp8.DelayedScaling(amax_history_len=3, interval=2)
+    passes = [(1.0, 1.0, [0.0, 0.0, 0.0]), (1.0, 1.0, [2.0, 0.0, 0.0]), (224.0, 28672.0, [0.0, 0.0, 2.0]),
+              (224.0, 28672.0, [2.0, 0.0, 2.0])]   # due in front of the third pass alone
+    for want in passes:
+        with fp8.fp8_autocast(fp8_recipe=recipe), pytest.raises(RuntimeError, match="no earlier pass" if reuse else "must sum"):
+            module(x, [1, 1], is_first_microbatch=False if reuse else None)
+        fwd, bwd = module.fp8_meta["scaling_fwd"], module.fp8_meta["scaling_bwd"]
+        assert (fwd.scale[0].item(), bwd.scale[0].item(), fwd.amax_history[:, 0].tolist()) == want
+        fwd.amax_history[0] = bwd.amax_history[0] = 2.0
