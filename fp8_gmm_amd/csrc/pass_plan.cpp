@@ -11,6 +11,7 @@
 #include <stdint.h>
 #include <string.h>
 
+#include <initializer_list>
 #include <vector>
 
 #include "../../include/fp8gmm.h"
@@ -384,6 +385,14 @@ int check_sizes(int experts, const int64_t* group_sizes, int64_t tokens) {
   }
   return rows == tokens ? FP8GMM_OK : FP8GMM_ERR_BAD_SHAPE;
 }
+// Token-major tensors of a pass: one without rows has no memory, and none of it is touched.
+template <class Desc>
+bool rows_missing(const Desc* s, std::initializer_list<const void*> tensors) {
+  if (s->tokens == 0) return false;
+  for (const void* t : tensors)
+    if (t == nullptr) return true;
+  return false;
+}
 bool tile_policy_ok(int p) { return p == 0 || p == 128 || p == 256 || p == FP8GMM_GEMM_TILE_DUAL || p == FP8GMM_GEMM_TILE_ROWS; }
 
 void begin_pass(Pass& p, int experts, const int64_t* sizes, int grid, int stream_k, int tile_policy) {
@@ -410,7 +419,7 @@ int check_common(const fp8gmm_linear_pass* s) {
 int linear_forward(const fp8gmm_linear_pass* s, Pass& p) {
   const int rc = check_common(s);
   if (rc != FP8GMM_OK) return rc;
-  if (s->x == nullptr || s->x_fp8 == nullptr || s->w_fp8 == nullptr || s->y == nullptr || s->fwd_scale == nullptr ||
+  if (rows_missing(s, {s->x, s->x_fp8, s->y}) || s->w_fp8 == nullptr || s->fwd_scale == nullptr ||
       s->fwd_scale_inv == nullptr || s->fwd_amax == nullptr || (s->cast_weights && s->w == nullptr))
     return FP8GMM_ERR_NULL_POINTER;
   const int K = s->in_features, N = s->out_features;
@@ -429,10 +438,11 @@ int linear_forward(const fp8gmm_linear_pass* s, Pass& p) {
 int linear_backward(const fp8gmm_linear_pass* s, Pass& p) {
   const int rc = check_common(s);
   if (rc != FP8GMM_OK) return rc;
-  if (s->dy == nullptr || s->dy_fp8 == nullptr || s->bwd_scale == nullptr || s->bwd_scale_inv == nullptr ||
+  if (rows_missing(s, {s->dy, s->dy_fp8}) || s->bwd_scale == nullptr || s->bwd_scale_inv == nullptr ||
       s->bwd_amax == nullptr || s->fwd_scale_inv == nullptr)
     return FP8GMM_ERR_NULL_POINTER;
-  if ((s->dgrad && (s->dx == nullptr || s->w_fp8 == nullptr)) || (s->wgrad && (s->dw == nullptr || s->x_fp8 == nullptr)))
+  if ((s->dgrad && (rows_missing(s, {s->dx}) || s->w_fp8 == nullptr)) ||
+      (s->wgrad && (s->dw == nullptr || rows_missing(s, {s->x_fp8}))))
     return FP8GMM_ERR_NULL_POINTER;
   const int K = s->in_features, N = s->out_features;
   begin_pass(p, s->experts, s->group_sizes, s->grid, s->stream_k, s->tile_policy);
@@ -469,9 +479,9 @@ int check_mlp(const fp8gmm_mlp_pass* s) {
 int mlp_forward(const fp8gmm_mlp_pass* s, Pass& p) {
   const int rc = check_mlp(s);
   if (rc != FP8GMM_OK) return rc;
-  if (s->x == nullptr || s->x_fp8 == nullptr || s->w1_fp8 == nullptr || s->w2_fp8 == nullptr || s->pre == nullptr ||
-      s->act_fp8 == nullptr || s->y == nullptr || s->fwd_scale == nullptr || s->fwd_scale_inv == nullptr ||
-      s->fwd_amax == nullptr || (s->cast_weights && (s->w1 == nullptr || s->w2 == nullptr)))
+  if (rows_missing(s, {s->x, s->x_fp8, s->pre, s->act_fp8, s->y}) || s->w1_fp8 == nullptr || s->w2_fp8 == nullptr ||
+      s->fwd_scale == nullptr || s->fwd_scale_inv == nullptr || s->fwd_amax == nullptr ||
+      (s->cast_weights && (s->w1 == nullptr || s->w2 == nullptr)))
     return FP8GMM_ERR_NULL_POINTER;
   const int H = s->hidden, F = s->ffn;
   const int64_t g2 = 3 * (int64_t)s->experts;   // first forward slot of the fc2 GEMMs
@@ -499,12 +509,11 @@ int mlp_forward(const fp8gmm_mlp_pass* s, Pass& p) {
 int mlp_backward(const fp8gmm_mlp_pass* s, Pass& p) {
   const int rc = check_mlp(s);
   if (rc != FP8GMM_OK) return rc;
-  if (s->dy == nullptr || s->dy_fp8 == nullptr || s->w2_fp8 == nullptr || s->pre == nullptr || s->dact == nullptr ||
-      s->dpre_fp8 == nullptr || s->bwd_scale == nullptr || s->bwd_scale_inv == nullptr || s->bwd_amax == nullptr ||
-      s->fwd_scale_inv == nullptr)
+  if (rows_missing(s, {s->dy, s->dy_fp8, s->pre, s->dact, s->dpre_fp8}) || s->w2_fp8 == nullptr ||
+      s->bwd_scale == nullptr || s->bwd_scale_inv == nullptr || s->bwd_amax == nullptr || s->fwd_scale_inv == nullptr)
     return FP8GMM_ERR_NULL_POINTER;
-  if ((s->dgrad && (s->dx == nullptr || s->w1_fp8 == nullptr)) ||
-      (s->wgrad && (s->dw1 == nullptr || s->dw2 == nullptr || s->x_fp8 == nullptr || s->act_fp8 == nullptr)))
+  if ((s->dgrad && (rows_missing(s, {s->dx}) || s->w1_fp8 == nullptr)) ||
+      (s->wgrad && (s->dw1 == nullptr || s->dw2 == nullptr || rows_missing(s, {s->x_fp8, s->act_fp8}))))
     return FP8GMM_ERR_NULL_POINTER;
   const int H = s->hidden, F = s->ffn;
   const int64_t f2 = 3 * (int64_t)s->experts, b2 = 2 * (int64_t)s->experts;   // first slots of the fc2 GEMMs

@@ -356,7 +356,8 @@ int fp8gmm_grouped_gemm_static(const fp8gmm_gemm_problem* probs_dev, int n, cons
  * through the bases of the flat fp32 arrays in TransformerEngine's slot layout, which the reference indexes in
  * fp8_gmm/utils.py:98-103: forward slots 3 i (input of expert i) and 3 i + 1 (its weight), backward slot 2 i (its
  * output gradient).  For the backward pass fwd_scale_inv is the copy of the forward scale_inv taken after the
- * forward pass.  All data pointers are device pointers that are only stored, never dereferenced, by the planner.
+ * forward pass.  All data pointers are device pointers that are only stored, never dereferenced, by the planner.  With
+ * tokens == 0 the token-major tensors may be NULL: the weights are cast, the weight gradients are zeros.
  */
 typedef struct fp8gmm_linear_pass {
   int32_t experts, in_features, out_features;

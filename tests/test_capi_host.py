@@ -399,3 +399,37 @@ def test_mlp_pass_planner_options_and_errors():
     d, _, _ = _mlp_pass([-1, 1], h, f)
     assert run(fwd, d) == -2
     assert lib.fp8gmm_plan_mlp_forward(None, blob.ctypes.data, blob.nbytes, ctypes.byref(plan)) == -1
+
+
+def test_passes_without_rows_need_no_row_tensors():
+    """An input without rows has no memory (torch reports a null address): its pass casts the weights forward and writes
+    zero weight gradients backward.  With rows, every one of those tensors is needed; the weights always are."""
+    lib = _lib.load()
+    h, f = 64, 96
+    plan, tables = _lib.PassPlan(), _lib.PassTables()
+    forward, backward = ("x", "x_fp8", "y", "pre", "act_fp8"), ("dy", "dy_fp8", "dx", "x_fp8", "pre", "act_fp8", "dact", "dpre_fp8")
+
+    def linear(sizes, **over):
+        _, _, gs = _mlp_pass(sizes, h, f)
+        fields = {n: (i + 1) << 36 for i, (n, _) in enumerate(_lib.LinearPass._fields_[14:])}
+        fields.update(experts=len(sizes), in_features=h, out_features=f, fwd_fmt=_lib.E4M3, bwd_fmt=_lib.E5M2, cast_weights=1,
+                      dgrad=1, wgrad=1, grid=64, stream_k=1, tokens=int(gs.sum()), group_sizes=gs.ctypes.data)
+        fields.update(over)
+        return _lib.LinearPass(**fields), gs
+
+    for which, describe, kinds, row_tensors, always in (
+            (_lib.LINEAR_FORWARD, linear, [_lib.PASS_CAST, 0], forward[:3], "w_fp8"),
+            (_lib.LINEAR_BACKWARD, linear, [0, _lib.PASS_GEMM, 0], backward[:4], "dw"),
+            (_lib.MLP_FORWARD, _mlp_pass, [_lib.PASS_CAST, 0, 0], forward, "w2_fp8"),
+            (_lib.MLP_BACKWARD, _mlp_pass, [0, _lib.PASS_GEMM, 0, 0, 0, _lib.PASS_GEMM], backward, "dw1")):
+        shape = () if describe is linear else (h, f)
+
+        def rc(sizes, missing):
+            made = describe(sizes, *shape, **dict.fromkeys(missing, 0))   # keeps the sizes alive
+            return lib.fp8gmm_lay_out_pass(which, ctypes.byref(made[0]), ctypes.byref(plan), tables)
+
+        assert rc([0, 0], row_tensors) == 0
+        assert [plan.launch[i].kind for i in range(plan.n_launches)] == kinds
+        assert rc([0, 0], row_tensors + (always,)) == -1
+        for name in row_tensors:
+            assert rc([0, 3], (name,)) == -1, (which, name)

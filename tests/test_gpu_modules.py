@@ -954,3 +954,30 @@ def test_passes_under_activation_checkpointing_and_saved_tensor_hooks(dev, kind)
 
     with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t), pytest.raises(Stop):
         mods[0](x.clone().requires_grad_(), sizes)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["linear", "cutlass", "mlp"])
+def test_passes_without_rows(dev, kind):
+    """A rank or a micro-batch without tokens: empty results, zero weight gradients, and the weights' maxima in the scaling
+    state as any pass leaves them, through several passes and next to one with rows."""
+    pkg = _pkg()
+    g = gen(606)
+    mod = pkg.GroupedMlp(64, 96, 3, torch.bfloat16, device=dev) if kind == "mlp" else \
+        pkg.GroupedLinear(64, 96, 3, torch.bfloat16, device=dev, cutlass=kind == "cutlass")
+    out_features = 64 if kind == "mlp" else 96
+    for rows in (0, 7, 0):
+        mod.zero_grad()
+        x = randn_bf16((rows, 64), g).to(dev).requires_grad_()
+        out = mod(x, torch.tensor([0, rows, 0]))
+        out.backward(torch.ones_like(out))
+        assert out.shape == (rows, out_features) and x.grad.shape == x.shape
+        for p in mod.parameters():
+            assert p.grad.shape == p.shape and p.grad.isfinite().all()
+            assert bool(p.grad.any()) == (rows > 0)
+    fwd, bwd = mod.fp8_meta["scaling_fwd"].amax_history[0].cpu(), mod.fp8_meta["scaling_bwd"].amax_history[0]
+    assert not bwd.any() and not fwd[0::3].any()   # nothing was cast but the weights
+    want = torch.cat([p.detach().abs().amax(dim=(1, 2)).float() for p in mod.parameters()]).cpu()
+    assert torch.equal(fwd[1::3], want)
+    with torch.no_grad():
+        assert mod(torch.empty(0, 64, dtype=torch.bfloat16, device=dev), [0, 0, 0]).shape == (0, out_features)
