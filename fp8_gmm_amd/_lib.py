@@ -179,6 +179,7 @@ PASS_CAST = 1
 PASS_GEMM = 2
 LINEAR_FORWARD, LINEAR_BACKWARD, MLP_FORWARD, MLP_BACKWARD = range(4)
 PASS_MAX_EXPERTS = 384
+PASS_MAX_ROWS = 0x7FFFFFFF
 PASS_MAX_GRID = 512
 PassTables = ctypes.c_uint64 * (4032 // 8)   # FP8GMM_PASS_TABLES_BYTES, opaque
 

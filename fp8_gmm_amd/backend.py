@@ -977,7 +977,7 @@ def warm_up(device=None):
 def _run_pass(device, which, desc, fields, snapshot, host_planned):
     """Fill the pass description `desc` from `fields`, have its tables built and enqueue its launches.  The tables are
     written by a kernel of the library from a description of the pass (fp8gmm_build_pass), which also takes the
-    `snapshot` (source, destination) of fp32 values; a pass of more experts than fit a kernel argument is planned on
+    `snapshot` (source, destination) of fp32 values; a pass of more experts or rows than the kernel takes is planned on
     the host (`host_planned`: planning function, bound on its bytes) and uploaded."""
     L = _lib.load()
     flush_uploads()   # launches queued before this pass come first
@@ -996,7 +996,7 @@ def _run_pass(device, which, desc, fields, snapshot, host_planned):
     desc.stream_k = int(bool(options.stream_k))
     desc.tile_policy = TILE_POLICIES[options.tile]
     plan = _lib.PassPlan()
-    if desc.experts <= _lib.PASS_MAX_EXPERTS and 2 * grid <= _lib.PASS_MAX_GRID:
+    if desc.experts <= _lib.PASS_MAX_EXPERTS and desc.tokens <= _lib.PASS_MAX_ROWS and 2 * grid <= _lib.PASS_MAX_GRID:
         tables = _lib.PassTables()
         _lib.check(L.fp8gmm_lay_out_pass(which, ctypes.byref(desc), ctypes.byref(plan), tables))
         with _on_device(device):

@@ -323,8 +323,10 @@ int lay_out_pass(Pass& pass, fp8gmm_pass_plan* out, PassTables* t) {
     return FP8GMM_ERR_BAD_ARGUMENT;
   t->experts = e;
   t->n_casts = t->n_gemms = 0;
+  int64_t rows = 0;
   for (int i = 0; i < e; ++i) {
-    if (pass.group_sizes[i] > INT32_MAX / 2) return FP8GMM_ERR_BAD_SHAPE;
+    rows += pass.group_sizes[i];
+    if (pass.group_sizes[i] > INT32_MAX / 2 || rows > FP8GMM_PASS_MAX_ROWS) return FP8GMM_ERR_BAD_SHAPE;
     t->rows[i] = (int32_t)pass.group_sizes[i];
   }
   static thread_local std::vector<fp8gmm_gemm_problem> scratch;

@@ -295,7 +295,8 @@ class Fp8GroupedModuleBase(torch.nn.Module):
                 and backend.options.wgrad == "in_place" and self.num_groups <= _lib.PASS_MAX_EXPERTS
                 and getattr(backend._pending, "items", None) is None):
             return False
-        if not (input.is_cuda and input.dtype == torch.bfloat16 and input.dim() == 2 and input.is_contiguous()):
+        if not (input.is_cuda and input.dtype == torch.bfloat16 and input.dim() == 2 and input.is_contiguous()
+                and input.size(0) <= _lib.PASS_MAX_ROWS):
             return False
         for w in weights:
             if not (w.dtype == torch.bfloat16 and w.is_contiguous() and w.device == input.device

@@ -524,14 +524,15 @@ int fp8gmm_delayed_scaling_updates(const fp8gmm_scaling_update* updates, int n, 
  *            read the new scales), as fp8gmm_delayed_scaling_updates would
  *   copy_* : copy_n floats (0: none) that the same launch copies on the side, e.g. the snapshot of the forward
  *            scale_inv that the backward pass wants; a copy of an updated scale_inv (all of it) holds the new values
- * More than FP8GMM_PASS_MAX_EXPERTS experts do not fit a kernel argument (FP8GMM_ERR_BAD_ARGUMENT): plan those passes on
- * the host.
+ * More than FP8GMM_PASS_MAX_EXPERTS experts do not fit a kernel argument (FP8GMM_ERR_BAD_ARGUMENT), and the kernel counts
+ * rows in 32 bits (more than FP8GMM_PASS_MAX_ROWS in all: FP8GMM_ERR_BAD_SHAPE): plan those passes on the host.
  */
 #define FP8GMM_LINEAR_FORWARD 0
 #define FP8GMM_LINEAR_BACKWARD 1
 #define FP8GMM_MLP_FORWARD 2
 #define FP8GMM_MLP_BACKWARD 3
 #define FP8GMM_PASS_MAX_EXPERTS 384
+#define FP8GMM_PASS_MAX_ROWS 0x7fffffff
 #define FP8GMM_PASS_MAX_GRID 512
 #define FP8GMM_PASS_TABLES_BYTES 4032
 int fp8gmm_lay_out_pass(int which, const void* pass, fp8gmm_pass_plan* out, void* tables);

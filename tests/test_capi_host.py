@@ -401,6 +401,42 @@ def test_mlp_pass_planner_options_and_errors():
     assert lib.fp8gmm_plan_mlp_forward(None, blob.ctypes.data, blob.nbytes, ctypes.byref(plan)) == -1
 
 
+def _linear_pass(sizes, k, n, **over):
+    gs = np.asarray(sizes, dtype=np.int64)
+    fields = {name: (i + 1) << 40 for i, (name, _) in enumerate(_lib.LinearPass._fields_[14:])}
+    fields.update(experts=len(sizes), in_features=k, out_features=n, fwd_fmt=_lib.E4M3, bwd_fmt=_lib.E5M2, cast_weights=1,
+                  dgrad=1, wgrad=1, grid=64, stream_k=1, tokens=int(gs.sum()), group_sizes=gs.ctypes.data)
+    fields.update(over)
+    return _lib.LinearPass(**fields), None, gs
+
+
+def test_device_tables_are_refused_past_the_rows_that_32_bits_count():
+    """The table kernel adds the rows up in 32 bits: a pass of more rows is refused on the host (narrow widths only: every
+    expert keeps below 2^31 elements), where the host planner, which counts in 64, takes it; the binding goes there."""
+    from types import SimpleNamespace
+
+    import torch
+
+    from fp8_gmm_amd import GroupedLinear
+
+    lib = _lib.load()
+    plan, tables = _lib.PassPlan(), _lib.PassTables()
+    full = [(1 << 27) - 1] * 16
+    for rows, status in ((15, 0), (16, -2), (1 << 20, -2)):
+        for which, describe in ((_lib.LINEAR_FORWARD, _linear_pass), (_lib.LINEAR_BACKWARD, _linear_pass),
+                                (_lib.MLP_FORWARD, _mlp_pass), (_lib.MLP_BACKWARD, _mlp_pass)):
+            d = describe(full + [rows], 16, 16)
+            assert lib.fp8gmm_lay_out_pass(which, ctypes.byref(d[0]), ctypes.byref(plan), tables) == status
+    d = _linear_pass(full + [16], 16, 16)
+    assert lib.fp8gmm_plan_linear_forward(ctypes.byref(d[0]), None, 0, ctypes.byref(plan)) == -8   # sized, not refused
+    module = GroupedLinear(16, 16, 2, torch.bfloat16, device="cpu")
+    module._prepare(torch.device("cpu"), None, 2)
+    for rows in ((1 << 31) - 1, 1 << 31):
+        x = SimpleNamespace(is_cuda=True, dtype=torch.bfloat16, dim=lambda: 2, is_contiguous=lambda: True, size=lambda i: rows,
+                            device=module.weight_tensor.device)
+        assert module._native(x, module.weight_tensor) == (rows < 1 << 31)
+
+
 def test_passes_without_rows_need_no_row_tensors():
     """An input without rows has no memory (torch reports a null address): its pass casts the weights forward and writes
     zero weight gradients backward.  With rows, every one of those tensors is needed; the weights always are."""
@@ -409,23 +445,13 @@ def test_passes_without_rows_need_no_row_tensors():
     plan, tables = _lib.PassPlan(), _lib.PassTables()
     forward, backward = ("x", "x_fp8", "y", "pre", "act_fp8"), ("dy", "dy_fp8", "dx", "x_fp8", "pre", "act_fp8", "dact", "dpre_fp8")
 
-    def linear(sizes, **over):
-        _, _, gs = _mlp_pass(sizes, h, f)
-        fields = {n: (i + 1) << 36 for i, (n, _) in enumerate(_lib.LinearPass._fields_[14:])}
-        fields.update(experts=len(sizes), in_features=h, out_features=f, fwd_fmt=_lib.E4M3, bwd_fmt=_lib.E5M2, cast_weights=1,
-                      dgrad=1, wgrad=1, grid=64, stream_k=1, tokens=int(gs.sum()), group_sizes=gs.ctypes.data)
-        fields.update(over)
-        return _lib.LinearPass(**fields), gs
-
     for which, describe, kinds, row_tensors, always in (
-            (_lib.LINEAR_FORWARD, linear, [_lib.PASS_CAST, 0], forward[:3], "w_fp8"),
-            (_lib.LINEAR_BACKWARD, linear, [0, _lib.PASS_GEMM, 0], backward[:4], "dw"),
+            (_lib.LINEAR_FORWARD, _linear_pass, [_lib.PASS_CAST, 0], forward[:3], "w_fp8"),
+            (_lib.LINEAR_BACKWARD, _linear_pass, [0, _lib.PASS_GEMM, 0], backward[:4], "dw"),
             (_lib.MLP_FORWARD, _mlp_pass, [_lib.PASS_CAST, 0, 0], forward, "w2_fp8"),
             (_lib.MLP_BACKWARD, _mlp_pass, [0, _lib.PASS_GEMM, 0, 0, 0, _lib.PASS_GEMM], backward, "dw1")):
-        shape = () if describe is linear else (h, f)
-
         def rc(sizes, missing):
-            made = describe(sizes, *shape, **dict.fromkeys(missing, 0))   # keeps the sizes alive
+            made = describe(sizes, h, f, **dict.fromkeys(missing, 0))   # keeps the sizes alive
             return lib.fp8gmm_lay_out_pass(which, ctypes.byref(made[0]), ctypes.byref(plan), tables)
 
         assert rc([0, 0], row_tensors) == 0
