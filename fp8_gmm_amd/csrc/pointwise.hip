@@ -210,7 +210,8 @@ extern "C" {
 int fp8gmm_delayed_scaling_update(float* amax_history, float* scale, float* scale_inv, int history_len, int slots,
                                   float fp8_max, int margin, int most_recent, int keep_period, int keep_phase,
                                   void* stream) {
-  if (history_len < 1 || slots < 0 || slots > (1 << 20) - 1 || margin < -126 || margin > 126) return FP8GMM_ERR_BAD_ARGUMENT;
+  if (history_len < 1 || slots < 0 || slots > INT32_MAX - fp8gmm::kScalingCols || margin < -126 || margin > 126)
+    return FP8GMM_ERR_BAD_ARGUMENT;
   if (keep_period < 0 || (keep_period > 0 && (keep_phase < 0 || keep_phase >= keep_period)))
     return FP8GMM_ERR_BAD_ARGUMENT;
   if (slots == 0) return FP8GMM_OK;

@@ -29,6 +29,7 @@ constexpr int kScalingThreads = 256;
 constexpr int kScalingLanes = kScalingThreads / kScalingCols;   // rows side by side: 16
 constexpr int kScalingPerLane = 64;
 constexpr int kScalingRows = kScalingLanes * kScalingPerLane;   // 1024
+constexpr int kScalingChunkSlots = 0xffffffffu / 4 / kScalingRows;   // columns of a chunk that 32-bit offsets reach: 2^20 - 1
 
 // torch.max semantics: a NaN anywhere in the column wins
 __device__ __forceinline__ float history_max(float a, float b) { return (b > a || b != b) ? b : a; }
@@ -44,38 +45,48 @@ __device__ __forceinline__ void delayed_scaling_update_columns(float* __restrict
   float* col = history + c;
   const float first = live ? col[0] : 0.f;
   float amax = first;
-  const uint32_t pitch = (uint32_t)slots * 4;
-  const uint32_t lane_off = live ? (uint32_t)lane_row * pitch + (uint32_t)c * 4 : kOobOffset;
-  for (int base = 0; base < history_len; base += kScalingRows) {
-    // rows past the history read as zeros, which never raise a maximum of magnitudes, and are not stored; the
-    // descriptor of the stores begins one row above that of the loads
-    const int rows = history_len - base < kScalingRows ? history_len - base : kScalingRows;
-    float* const chunk = history + (int64_t)base * slots;
-    const __amdgpu_buffer_rsrc_t from = make_rsrc(chunk, (uint32_t)rows * pitch);
-    const __amdgpu_buffer_rsrc_t to = make_rsrc(chunk - slots, (uint32_t)rows * pitch);
-    uint32_t v[kScalingPerLane];
-    uint32_t off = lane_off;
-#pragma unroll
-    for (int j = 0; j < kScalingPerLane; ++j) {
-      v[j] = __builtin_amdgcn_raw_buffer_load_b32(from, (int)off, 0, 0);
-      off = live ? off + kScalingLanes * pitch : kOobOffset;
+  if (slots > kScalingChunkSlots) {
+    // a chunk of so wide a table is out of a buffer descriptor's reach: a lane per column, row by row
+    if (threadIdx.x >= kScalingCols || !live) return;
+    for (int r = 1; r < history_len; ++r) {
+      const float v = col[(size_t)r * slots];
+      amax = history_max(amax, v);
+      col[(size_t)(r - 1) * slots] = v;
     }
+  } else {
+    const uint32_t pitch = (uint32_t)slots * 4;
+    const uint32_t lane_off = live ? (uint32_t)lane_row * pitch + (uint32_t)c * 4 : kOobOffset;
+    for (int base = 0; base < history_len; base += kScalingRows) {
+      // rows past the history read as zeros, which never raise a maximum of magnitudes, and are not stored; the
+      // descriptor of the stores begins one row above that of the loads
+      const int rows = history_len - base < kScalingRows ? history_len - base : kScalingRows;
+      float* const chunk = history + (int64_t)base * slots;
+      const __amdgpu_buffer_rsrc_t from = make_rsrc(chunk, (uint32_t)rows * pitch);
+      const __amdgpu_buffer_rsrc_t to = make_rsrc(chunk - slots, (uint32_t)rows * pitch);
+      uint32_t v[kScalingPerLane];
+      uint32_t off = lane_off;
 #pragma unroll
-    for (int j = 0; j < kScalingPerLane; ++j) amax = history_max(amax, __uint_as_float(v[j]));
-    __syncthreads();
-    off = base == 0 && lane_row < 2 ? kOobOffset : lane_off;   // row 1 falls on row 0, which is cleared below
+      for (int j = 0; j < kScalingPerLane; ++j) {
+        v[j] = __builtin_amdgcn_raw_buffer_load_b32(from, (int)off, 0, 0);
+        off = live ? off + kScalingLanes * pitch : kOobOffset;
+      }
 #pragma unroll
-    for (int j = 0; j < kScalingPerLane; ++j) {
-      __builtin_amdgcn_raw_buffer_store_b32(v[j], to, (int)off, 0, 0);
-      off = live ? lane_off + (uint32_t)(j + 1) * (kScalingLanes * pitch) : kOobOffset;
+      for (int j = 0; j < kScalingPerLane; ++j) amax = history_max(amax, __uint_as_float(v[j]));
+      __syncthreads();
+      off = base == 0 && lane_row < 2 ? kOobOffset : lane_off;   // row 1 falls on row 0, which is cleared below
+#pragma unroll
+      for (int j = 0; j < kScalingPerLane; ++j) {
+        __builtin_amdgcn_raw_buffer_store_b32(v[j], to, (int)off, 0, 0);
+        off = live ? lane_off + (uint32_t)(j + 1) * (kScalingLanes * pitch) : kOobOffset;
+      }
     }
+    // lanes 16 apart hold the same column
+    for (int off = kScalingCols; off < kWaveSize; off <<= 1) amax = history_max(amax, __shfl_xor(amax, off));
+    if (threadIdx.x % kWaveSize < kScalingCols) stage[threadIdx.x / kWaveSize][lane_col] = amax;
+    __syncthreads();   // (the last rows have been read by now, too: the row written below is one of them)
+    if (threadIdx.x >= kScalingCols || !live) return;
+    for (int w = 1; w < kScalingThreads / kWaveSize; ++w) amax = history_max(amax, stage[w][lane_col]);
   }
-  // lanes 16 apart hold the same column
-  for (int off = kScalingCols; off < kWaveSize; off <<= 1) amax = history_max(amax, __shfl_xor(amax, off));
-  if (threadIdx.x % kWaveSize < kScalingCols) stage[threadIdx.x / kWaveSize][lane_col] = amax;
-  __syncthreads();   // (the last rows have been read by now, too: the row written below is one of them)
-  if (threadIdx.x >= kScalingCols || !live) return;
-  for (int w = 1; w < kScalingThreads / kWaveSize; ++w) amax = history_max(amax, stage[w][lane_col]);
   if (most_recent) amax = first;
   float sc = scale[c];
   if (amax > 0.f && amax <= 3.4028234663852886e38f) sc = ((1.0f / amax) * fp8_max) * margin_factor;
@@ -118,8 +129,7 @@ int collect_scaling_updates(const fp8gmm_scaling_update* updates, int n, Scaling
   int blocks = 0;
   for (int i = 0; i < n; ++i) {
     const fp8gmm_scaling_update& u = updates[i];
-    // (a chunk of the history is addressed through one buffer descriptor)
-    if (u.history_len < 1 || u.slots < 0 || u.slots > (1 << 20) - 1 || u.margin < -126 || u.margin > 126) return FP8GMM_ERR_BAD_ARGUMENT;
+    if (u.history_len < 1 || u.slots < 0 || u.slots > INT32_MAX - kScalingCols || u.margin < -126 || u.margin > 126) return FP8GMM_ERR_BAD_ARGUMENT;
     if (u.keep_period < 0 || (u.keep_period > 0 && (u.keep_phase < 0 || u.keep_phase >= u.keep_period)))
       return FP8GMM_ERR_BAD_ARGUMENT;
     if (u.slots > 0 && (u.amax_history == nullptr || u.scale == nullptr || u.scale_inv == nullptr))

@@ -383,6 +383,24 @@ def test_delayed_scaling_update_at_the_edges_of_its_pieces(dev, history_len, slo
             assert torch.equal(a.view(torch.int32), b.view(torch.int32)), f"{name} differs at step {step}"
 
 
+@pytest.mark.parametrize("slots", [(1 << 20) - 1, 1 << 20, (1 << 20) + 3])
+@pytest.mark.parametrize("history_len", [1, 3])
+def test_delayed_scaling_update_of_very_wide_tables(dev, slots, history_len):
+    """Either side of the width at which a chunk of 1024 rows outgrows 32-bit offsets, bit for bit against the torch rule."""
+    from fp8_gmm_amd import fp8
+
+    hist = torch.rand(history_len, slots, generator=gen(slots))
+    hist[0, 0], hist[history_len - 1, slots - 1], hist[history_len // 2, 16] = 0.0, 7.0, float("nan")
+    recipe = fp8.DelayedScaling(amax_history_len=history_len)
+    cpu, gpu = (fp8.Fp8MetaTensors(slots, history_len, d) for d in (torch.device("cpu"), dev))
+    cpu.amax_history.copy_(hist), gpu.amax_history.copy_(hist)
+    for meta in (cpu, gpu):
+        fp8.amax_and_scale_update(meta, 448.0, recipe, keep_scale_inv=(3, 1))
+    for name in ("scale", "scale_inv", "amax_history"):
+        a, b = getattr(gpu, name).cpu(), getattr(cpu, name)
+        assert torch.equal(a.view(torch.int32), b.view(torch.int32)), name
+
+
 def test_several_scaling_updates_in_one_launch_equal_one_launch_each(dev):
     """fp8gmm_delayed_scaling_updates: up to four directions in one kernel launch (a module's forward and backward
     state go together) must leave every tensor exactly as one launch per direction does: different history
