@@ -148,6 +148,12 @@ void check_no_tangent(at::TensorList inputs) {
     TORCH_CHECK(!torch::autograd::isFwGradDefined(t), "fp8_gmm_amd: the grouped modules do not support forward-mode AD");
 }
 
+// What a backward pass starts from.  A node behind the pass that returned no gradient stands for zeros, as it does for a
+// Python autograd function.
+Tensor gradient_of_result(const Node& node, const variable_list& grads) {
+  return grads[0].defined() ? grads[0].contiguous() : node.input_metadata(0).zeros_like();
+}
+
 // ---- GroupedLinear ------------------------------------------------------------------------------------------------
 fp8gmm_linear_pass linear_desc(const Setup& s, const std::vector<int64_t>& sizes, int64_t tokens, int64_t in, int64_t out) {
   fp8gmm_linear_pass d{};
@@ -183,8 +189,7 @@ struct GroupedLinearBackward : public Node {
     at::AutoGradMode no_grad(false);
     variable_list result(2);
     const bool dgrad = task_should_compute_output(0), wgrad = task_should_compute_output(1);
-    if (!grads[0].defined() || !(dgrad || wgrad)) return result;
-    const Tensor dy = grads[0].contiguous();
+    const Tensor dy = gradient_of_result(*this, grads);
     const c10::OptionalDeviceGuard guard(dy.device());
     const Tensor x = wgrad ? x_fp8.unpack() : Tensor(), w = dgrad ? w_fp8.unpack() : Tensor();
     const Tensor dy_fp8 = at::empty(dy.sizes(), dy.options().dtype(setup.bwd_type()));
@@ -289,8 +294,7 @@ struct GroupedMlpBackward : public Node {
     variable_list result(3);
     const bool want_x = dgrad && task_should_compute_output(0);
     const bool want_w = wgrad && (task_should_compute_output(1) || task_should_compute_output(2));
-    if (!grads[0].defined() || !(want_x || want_w)) return result;
-    const Tensor dy = grads[0].contiguous();
+    const Tensor dy = gradient_of_result(*this, grads);
     const c10::OptionalDeviceGuard guard(dy.device());
     const int64_t tokens = dy.size(0), e = (int64_t)sizes.size();
     const auto bf16 = dy.options(), fp8 = dy.options().dtype(setup.bwd_type());

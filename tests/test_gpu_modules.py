@@ -981,3 +981,30 @@ def test_passes_without_rows(dev, kind):
     assert torch.equal(fwd[1::3], want)
     with torch.no_grad():
         assert mod(torch.empty(0, 64, dtype=torch.bfloat16, device=dev), [0, 0, 0]).shape == (0, out_features)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["linear", "mlp"])
+def test_a_result_whose_gradient_is_dropped_has_gradients_of_zero(dev, kind):
+    """A function behind the module that returns None for its gradient: zeros for the input and the weights, and the scaling
+    state, are what the per-launch path's autograd function leaves."""
+    class Drop(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, t):
+            return t.clone()
+
+        @staticmethod
+        def backward(ctx, grad):
+            return None
+
+    pkg = _pkg()
+    sizes, x, res = torch.tensor([5, 0, 28]), randn_bf16((33, 64), gen(91)).to(dev), []
+    for planned in (True, False):
+        mod = (pkg.GroupedLinear if kind == "linear" else pkg.GroupedMlp)(64, 96, 3, torch.bfloat16, device=dev,
+                                                                          planned_passes=planned)
+        xi = x.clone().requires_grad_()
+        Drop.apply(mod(xi, sizes)).sum().backward()
+        res.append([xi.grad] + [p.grad for p in mod.parameters()] + list(mod.fp8_meta["scaling_bwd"].state().values()))
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
+    assert not any(t.any() for t in res[0][: 2 if kind == "linear" else 3])
