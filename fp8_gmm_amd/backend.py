@@ -1262,6 +1262,10 @@ def fp8_gmm(a, b, group_sizes, a_scale_invs, b_scale_invs, c=None, c_dtype=torch
         _fail("fp8_gmm_amd: an fp8 output needs c_scales and c_amaxes")
     if cutlass and (c.dtype != torch.bfloat16 or pre_gelu_out is not None):
         _fail("fp8_gmm_amd: cutlass=True supports a bf16 output without GELU only")
+    if cutlass and e:
+        if a_scale_invs is None or b_scale_invs is None:
+            _fail("fp8_gmm_amd: cutlass=True needs a_scale_invs and b_scale_invs")
+        _check_counts(e, a_scale_invs=a_scale_invs, b_scale_invs=b_scale_invs)
     if pre_gelu_out is not None and (
         pre_gelu_out.dtype != torch.bfloat16 or tuple(pre_gelu_out.shape) != (tokens, nn)
         or not pre_gelu_out.is_contiguous()

@@ -422,3 +422,17 @@ def test_a_refused_native_pass_keeps_its_scaling_update(monkeypatch, kind, reuse
         fwd, bwd = module.fp8_meta["scaling_fwd"], module.fp8_meta["scaling_bwd"]
         assert (fwd.scale[0].item(), bwd.scale[0].item(), fwd.amax_history[:, 0].tolist()) == want
         fwd.amax_history[0] = bwd.amax_history[0] = 2.0
+
+
+def test_cutlass_products_need_their_factors():
+    """``multi_scale_mul`` refuses a missing factor, and the form that scales in the GEMM's epilogue does too."""
+    from fp8_gmm_amd import backend
+
+    a = torch.zeros(3, 16, dtype=torch.uint8).view(torch.float8_e4m3fn)
+    b = torch.zeros(2, 16, 16, dtype=torch.uint8).view(torch.float8_e4m3fn)
+    ones = torch.ones(2)
+    for sa, sb in ((None, ones), (ones, None)):
+        with pytest.raises(RuntimeError, match="needs a_scale_invs"):
+            backend.fp8_gmm(a, b, [1, 2], sa, sb, cutlass=True)
+    with pytest.raises(RuntimeError, match="entries"):
+        backend.fp8_gmm(a, b, [1, 2], ones, ones.reshape(1, 2), cutlass=True)
