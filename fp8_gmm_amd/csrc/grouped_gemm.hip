@@ -178,7 +178,10 @@ int scratch_for(int dev, uint8_t** out) {
   return FP8GMM_OK;
 }
 
-// "may use its LDS" of the form for few rows, as prepare_variant sets it for the others
+// operand formats of the form for few rows
+#define FP8GMM_FOR_EACH_ROWS_FORM(X) X(FP8GMM_E4M3, FP8GMM_E4M3) X(FP8GMM_E5M2, FP8GMM_E4M3) X(FP8GMM_E4M3, FP8GMM_E5M2)
+
+// "may use its LDS" of that form, as prepare_variant sets it for the others
 template <int A_FMT, int B_FMT>
 int prepare_rows(int dev) {
   static std::atomic<bool> attr_set[kMaxDevices];
@@ -219,9 +222,10 @@ int launch_rows(const fp8gmm_gemm_problem* probs_dev, const fp8gmm_gemm_item* it
 }
 launch_fn rows_variant_for(int a_fmt, int b_fmt, bool b_kmajor) {
   if (b_kmajor) return nullptr;
-  if (a_fmt == FP8GMM_E4M3 && b_fmt == FP8GMM_E4M3) return &launch_rows<FP8GMM_E4M3, FP8GMM_E4M3>;
-  if (a_fmt == FP8GMM_E5M2 && b_fmt == FP8GMM_E4M3) return &launch_rows<FP8GMM_E5M2, FP8GMM_E4M3>;
-  if (a_fmt == FP8GMM_E4M3 && b_fmt == FP8GMM_E5M2) return &launch_rows<FP8GMM_E4M3, FP8GMM_E5M2>;
+#define FP8GMM_SELECT_ROWS(AF, BF) \
+  if (a_fmt == AF && b_fmt == BF) return &launch_rows<AF, BF>;
+  FP8GMM_FOR_EACH_ROWS_FORM(FP8GMM_SELECT_ROWS)
+#undef FP8GMM_SELECT_ROWS
   return nullptr;
 }
 
@@ -316,6 +320,13 @@ int fp8gmm_init(int device) {
   }
   FP8GMM_FOR_EACH_GEMM_VARIANT(FP8GMM_PREPARE)
 #undef FP8GMM_PREPARE
+#define FP8GMM_PREPARE_ROWS(AF, BF)          \
+  if (rc > 0) {                              \
+    const int e = prepare_rows<AF, BF>(dev); \
+    if (e != FP8GMM_OK) rc = e;              \
+  }
+  FP8GMM_FOR_EACH_ROWS_FORM(FP8GMM_PREPARE_ROWS)
+#undef FP8GMM_PREPARE_ROWS
   if (rc > 0) {
     uint8_t* unused = nullptr;
     const int e = scratch_for(dev, &unused);
