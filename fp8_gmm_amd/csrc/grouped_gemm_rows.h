@@ -12,7 +12,7 @@
 // runs on across tile boundaries.  Unit layout, K order and products are those of the other forms: the same bits.
 //
 // Back to back, other forms -> this one (us, table upload of 3 - 4 included): 8 experts, 8 rows each, K = 14336 to 4096
-// columns 104 -> 73, K = 4096 to 14336 columns 108 -> 90; 128 experts, 8 rows each, K = 2048 to 768 columns 45 -> 39.
+// columns 104 -> 73, K = 4096 to 14336 columns 108 -> 90 (with the GELU and an fp8 result 128 -> 94); 128 experts, 8 rows each, K = 2048 to 768 columns 45 -> 39.
 // Tiles of 64 columns (ring of five) move the tokens twice as often: 85 against 73, 84 against 89 at 896 tiles, where
 // their balance is better; one workgroup per compute unit with a ring of six: 74, 96.
 #pragma once
@@ -194,6 +194,12 @@ __global__ __launch_bounds__(NTHREADS, 2) void grouped_gemm_rows_kernel(
   for (int s = 0; s < kRowsStages - 1; ++s) load_step(s);
   int cur = 0;
   ItemTile cp_next = item_tile(0);
+  // The running maximum of an fp8 result goes to its slot once per workgroup and run of tiles of one problem.  The slots of
+  // a pass share a cache line or two, and 512 workgroups that look at one line are served one after the other: with a look
+  // per wavefront and tile, 8 experts of 4096 -> 14336 columns took 137 us where slots of their own lines take 84.
+  __shared__ float wave_amax[2][NWAVES];   // in turn: two runs may end without a K step's barrier in between
+  int turn = 0;
+  float amax = 0.f;
 #pragma unroll 1
   for (int r_cp = 0;;) {
     const ItemTile g = cp_next;
@@ -224,13 +230,26 @@ __global__ __launch_bounds__(NTHREADS, 2) void grouped_gemm_rows_kernel(
       }
       cur = cur + 1 == kRowsStages ? 0 : cur + 1;
     }
-    float amax = 0.f;
 #pragma unroll
     for (int i = 0; i < MB; ++i)
       if (i < blocks)
         amax = fmaxf(amax, store_rows_block(pr, g.m0 + i * 32 + l32, g.n0 + wave * 32 + khalf * 4, acc[i], out_kind,
                                             epilogue, sa, sb, cs));
-    if (out_kind != FP8GMM_OUT_BF16) merge_amax(pr.c_amax, wave_max(amax), lane);
+    if (out_kind != FP8GMM_OUT_BF16 && cp_next.prob != g.prob) {
+      const float own = wave_max(amax);
+      if (lane == 0) wave_amax[turn][wave] = own;
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      if (wave == 0) {
+        float most = wave_amax[turn][0];
+#pragma unroll
+        for (int w = 1; w < NWAVES; ++w) most = fmaxf(most, wave_amax[turn][w]);
+        merge_amax(pr.c_amax, most, lane);
+      }
+      turn ^= 1;
+      amax = 0.f;
+    }
   }
   // zero-fill loads issued past the end of the stream still target this workgroup's LDS
   FP8GMM_WAIT_VM(0);

@@ -147,7 +147,12 @@ bool dual_tiles_pay(const fp8gmm_gemm_problem* p, int n, int layout) {
 // the fewer rows it takes for the other forms to be as fast.  Measured, other forms -> this one in us, at 8 / 32 / 64 rows
 // per expert: K = 14336 (8 experts, 4096 columns) 104 / 105 / 106 -> 73 / 74 / 80; K = 4096 (16, 6400) 94 / 96 / 100 ->
 // 83 / 86 / 99; K = 2048 (64, 1024) 32 / 32 / 32 -> 27 / 28 / 33; K = 768 (128, 2048) 46 / 49 / 53 -> 41 / 49 / 60; K = 256
-// (64, 4096) 25 -> 25 and worse; with 34 MB of weights (16, K = 1024, 2048) 12.7 -> 13.5.
+// (64, 4096) 25 -> 25 and worse; with 34 MB of weights (16, K = 1024, 2048) 12.7 -> 13.5.  With the GELU and an fp8 result,
+// which the 128 x 128 form does not have, every set of weights from HBM (1.2 GB in turn): 8 / 32 / 64 rows, K = 14336 (8, 4096)
+// 153 -> 84 at 8, 146 -> 86 at 64; K = 4096 (8, 14336) 128 -> 94, 126 -> 113 at 64, (32, 2048) 81 / 81 / 82 -> 64 / 65 / 68;
+// K = 2048 (32, 2048) 42 / 43 -> 32 / 33, (128, 768) 62 / 62 -> 42 / 46; K = 1024 (64, 1024) 29 / 29 -> 21 / 22; K = 768
+// (128, 2048) 74 -> 46 at 8, 75 -> 50 at 16; under a skewed split of 64 rows (8, K = 4096, 14336) 138 -> 147, which is more
+// tiles than the rule takes.
 bool rows_pay(const fp8gmm_gemm_problem* p, int n, int layout) {
   if (layout != 0) return false;
   int64_t weights = 0, rows = 0, tiles = 0, problems = 0;

@@ -437,6 +437,30 @@ def test_the_form_for_few_rows_gives_the_same_bits(dev, out):
             assert torch.equal(x, y), (sizes, k, n)
 
 
+def test_the_form_for_few_rows_merges_maxima_over_runs_of_tiles(dev):
+    """More tiles than workgroups: a workgroup's maximum of an fp8 result is merged where the next tile is another
+    problem's (or none), over runs of one tile and of several, whichever wavefront holds it; the large tiles' bits."""
+    backend = _backend()
+    g = gen(89)
+    sizes, k, n = [1, 0, 65, 2, 64], 16, 24600   # 193 x (1 + 2 + 1 + 1) tiles for 512 workgroups
+    m, e = sum(sizes), len(sizes)
+    a = _q(randn_bf16((m, k), g, 4.0), E4M3).to(dev)
+    b = _q(randn_bf16((e, n, k), g, 1.0), E4M3).to(dev)
+    for expert, column in ((0, 0), (2, 24599), (3, 12345), (4, 40)):   # the largest products, in one column each
+        b.view(torch.uint8)[expert, column] = 0x70   # 128
+    ones, results = torch.ones(e, device=dev), []
+    for tile in ("256", "rows"):
+        c = torch.zeros(m, n, dtype=torch.uint8, device=dev).view(E4M3)
+        pre, amax = torch.zeros(m, n, dtype=torch.bfloat16, device=dev), torch.zeros(3 * e, device=dev)
+        with backend.gemm_options(tile=tile, stream_k=False):
+            backend.fp8_gmm(a, b, torch.tensor(sizes), ones, ones, c, pre_gelu_out=pre, c_scales=ones,
+                            c_amaxes=[amax[3 * i] for i in range(e)])
+        results.append([c.view(torch.uint8), pre.view(torch.int16), amax])
+    for x, y in zip(*results):
+        assert torch.equal(x, y)
+    assert results[0][2][0::3].tolist()[1] == 0 and (results[0][2][0::3] > 0).sum() >= 3
+
+
 def test_random_problem_lists_are_exact(dev):
     """Sixty random grouped problems (ragged and empty experts, K and N that are not tile multiples, both operand
     formats, the stacked and the list calling form).  Operands come from {0, +-0.25 .. +-2} and the scales are
