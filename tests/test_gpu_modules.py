@@ -875,7 +875,8 @@ def test_fused_dgelu_backward_against_the_oracle(dev):
 @pytest.mark.parametrize("sizes,h,f,policy", [
     ([700, 0, 33, 1291, 5, 256], 512, 768, 0), ([300], 4096, 7168, 256), ([0, 513, 90, 0], 4112, 2064, 256),
     ([1, 0, 2] * 127 + [3], 64, 48, 0), ([128, 129, 0, 256, 257, 1], 272, 1408, 512), ([64] * 9 + [0], 256, 128, 128),
-    ([0, 0], 64, 64, 0)])
+    ([0, 0], 64, 64, 0), ([31, 0, 64, 1, 65, 128, 32, 0], 272, 400, 1024), ([3] * 9, 2048, 16400, 1024),
+    ([2, 0, 1] * 128, 64, 48, 1024), ([5, 0, 70] * 128, 80, 272, 0), ([8, 2, 1, 9] * 16, 1024, 1040, 0)])
 def test_tables_built_on_the_device_are_those_of_the_host_planner(dev, sizes, h, f, policy):
     """fp8gmm_build_pass writes a pass's tables into device memory from a kernel argument: descriptors, problem tables,
     work lists and shared-tile records must be the host planner's, byte for byte, at the same offsets, and nothing else
@@ -913,6 +914,8 @@ def test_tables_built_on_the_device_are_those_of_the_host_planner(dev, sizes, h,
         used = np.zeros(got.size, dtype=bool)
         for i in range(plan.n_launches):
             rec = plan.launch[i]
+            if rec.plan.tile and (policy == 1024 or h == 1024) and which in (_lib.LINEAR_FORWARD, _lib.MLP_FORWARD):
+                assert rec.plan.tile_m == _lib.GEMM_ROWS_TILE_M   # the form for few rows, asked for or chosen by the rule
             parts = [(rec.table_offset, rec.n * (96 if rec.plan.tile else 128))]
             if rec.plan.tile:
                 parts += [(rec.items_offset, rec.plan.rounds * rec.plan.grid * 64), (rec.fixups_offset, rec.plan.n_fixups * 32)]
@@ -1008,3 +1011,74 @@ def test_a_result_whose_gradient_is_dropped_has_gradients_of_zero(dev, kind):
     for a, b in zip(*res):
         assert torch.equal(a, b)
     assert not any(t.any() for t in res[0][: 2 if kind == "linear" else 3])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["linear", "mlp"])
+def test_native_passes_in_the_form_for_few_rows(dev, kind):
+    """The path of a decoding pass: tables of 64 x 128 tiles built on the device, the GELU with its fp8 result, the casts'
+    maxima merged by the GEMM.  Results, gradients and scaling state of the per-launch path, which plans on the host."""
+    from fp8_gmm_amd import backend
+
+    pkg = _pkg()
+    g, e, h, f = gen(93), 6, 160, 336
+    mods = [(pkg.GroupedLinear if kind == "linear" else pkg.GroupedMlp)(h, f, e, torch.bfloat16, device=dev, planned_passes=p)
+            for p in (True, False)]
+    mods[1].load_state_dict(mods[0].state_dict())
+    for sizes, first in (([31, 0, 64, 1, 65, 32], None), ([1] * 6, True), ([0, 70, 0, 2, 3, 33], False)):
+        x = randn_bf16((sum(sizes), h), g).to(dev)
+        dy, res = randn_bf16((sum(sizes), f if kind == "linear" else h), g, 1e-2).to(dev), []
+        for mod in mods:
+            mod.zero_grad()
+            xi = x.clone().requires_grad_()
+            with backend.gemm_options(tile="rows"):
+                out = mod(xi, torch.tensor(sizes), is_first_microbatch=first)
+                out.backward(dy)
+            res.append([out, xi.grad] + [p.grad for p in mod.parameters()])
+        for a, b in zip(*res):
+            assert torch.equal(a.view(torch.int16), b.view(torch.int16)), sizes
+        for name in ("scaling_fwd", "scaling_bwd"):
+            for a, b in zip(mods[0].fp8_meta[name].state().values(), mods[1].fp8_meta[name].state().values()):
+                assert torch.equal(a, b), (sizes, name)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["linear", "mlp"])
+def test_native_passes_on_a_side_stream_with_the_backward_in_another_thread(dev, kind):
+    """A forward pass on a stream of its own, its backward pass started from another thread on the default stream, over
+    several steps with the temporaries' memory handed out again in between: the bits of the plain order."""
+    import threading
+
+    pkg = _pkg()
+    g, sizes = gen(94), torch.tensor([70, 0, 301, 5])
+    mods = [(pkg.GroupedLinear if kind == "linear" else pkg.GroupedMlp)(160, 336, 4, torch.bfloat16, device=dev)
+            for _ in range(2)]
+    mods[1].load_state_dict(mods[0].state_dict())
+    side, failed = torch.cuda.Stream(), []
+    for _ in range(3):
+        x = randn_bf16((376, 160), g).to(dev)
+        dy, res = randn_bf16((376, 336 if kind == "linear" else 160), g, 1e-2).to(dev), []
+        for mod, stream in zip(mods, (torch.cuda.current_stream(), side)):
+            mod.zero_grad()
+            xi = x.clone().requires_grad_()
+            stream.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(stream):
+                out = mod(xi, sizes)
+            if stream is side:
+                def backward():
+                    try:
+                        out.backward(dy)
+                    except BaseException as exc:   # noqa: BLE001 - reported by the main thread
+                        failed.append(exc)
+
+                thread = threading.Thread(target=backward)
+                thread.start()
+                thread.join(60)
+                assert not thread.is_alive() and not failed, failed
+            else:
+                out.backward(dy)
+            torch.cuda.current_stream().wait_stream(stream)
+            res.append([out, xi.grad] + [p.grad for p in mod.parameters()])
+        for a, b in zip(*res):
+            assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+        torch.cuda.synchronize()

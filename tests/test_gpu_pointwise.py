@@ -360,10 +360,10 @@ def test_delayed_scaling_update_matches_the_torch_rule(dev, history_len, slots, 
         gpu.amax_history[0] += bump.to(dev)
 
 
-@pytest.mark.parametrize("history_len", [2, 63, 65, 1023, 1025, 2049])
+@pytest.mark.parametrize("history_len", [2, 15, 16, 17, 63, 65, 1023, 1025, 2049])
 @pytest.mark.parametrize("slots", [15, 17, 40])
 def test_delayed_scaling_update_at_the_edges_of_its_pieces(dev, history_len, slots):
-    """A workgroup moves 16 columns by 1024 rows at once, 64 rows side by side: histories and slot counts around those
+    """A workgroup moves 16 columns by 1024 rows at once, 16 rows side by side: histories and slot counts around those
     numbers, the row that carries the maximum walking through all of them, bit for bit against the torch rule."""
     from fp8_gmm_amd import fp8
 
