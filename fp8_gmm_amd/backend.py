@@ -20,6 +20,7 @@ import torch
 
 from . import _lib
 from ._lib import GEMM_PROBLEM, TENSOR_DESC
+from .native import set_kernel_timing
 import os
 
 _lib.load()  # fail at import time, loudly, when the extension is missing
@@ -69,10 +70,12 @@ class kernel_timing:
 
     def __enter__(self):
         kernel_timing._active = self
+        set_kernel_timing(True)
         return self
 
     def __exit__(self, *exc):
         kernel_timing._active = None
+        set_kernel_timing(False)
         return False
 
     def summary(self):
@@ -848,7 +851,8 @@ class GemmOptions:
     asynchronous copy; while a stream is being captured into a graph the tables always take the first way, from
     memory that is kept for the replays).  The defaults can be preset with the environment variables FP8GMM_TILE, FP8GMM_STREAMK
     (0 turns sharing off), FP8GMM_WGRAD and FP8GMM_UPLOAD, read once when the module is imported; afterwards assign
-    the attributes or use ``gemm_options(...)`` for a block."""
+    the attributes or use ``gemm_options(...)`` for a block.  A module's backward pass keeps the policy that its forward
+    pass was made under."""
 
     __slots__ = ("tile", "stream_k", "wgrad", "upload")
 
@@ -1025,6 +1029,13 @@ def _run_pass(device, which, desc, fields, snapshot, host_planned):
                 rc = L.fp8gmm_run_planned(base, ctypes.byref(rec), ws_ptr, ws_bytes, stream)
             _lib.check(rc)
     return plan
+
+
+def run_described_pass(which, device_index, desc):
+    """A backward pass as the native host path describes it (the bytes of its C structure), launch by launch: where
+    ``kernel_timing`` wants every launch bracketed with events."""
+    desc = (_lib.LinearPass if which == _lib.LINEAR_BACKWARD else _lib.MlpPass).from_buffer_copy(desc)
+    _run_pass(torch.device("cuda", device_index), which, desc, {}, None, None)
 
 
 def _plan_on_host(device, desc, plan, plan_fn, bound_fn, grid):

@@ -20,6 +20,8 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
+#include <atomic>
+
 #include "fp8gmm.h"
 
 namespace {
@@ -83,9 +85,21 @@ struct Due {
   bool most_recent = false, keep_weights = false;
 };
 
+// Whether a block of backend.kernel_timing is open (set_kernel_timing).
+std::atomic<bool> kernel_timing{false};
+
 // Builds the tables of a pass and enqueues its launches on the current stream.
 void run_pass(int which, const void* desc, const at::Device& device, const Setup* update, Due* due, const Tensor& snapshot_of,
               const Tensor& snapshot) {
+  const bool backward = which == FP8GMM_LINEAR_BACKWARD || which == FP8GMM_MLP_BACKWARD;
+  if (backward && kernel_timing.load(std::memory_order_relaxed)) {
+    // the same launches one by one, each between two events (a module does not come here for such a forward pass)
+    const size_t bytes = which == FP8GMM_LINEAR_BACKWARD ? sizeof(fp8gmm_linear_pass) : sizeof(fp8gmm_mlp_pass);
+    py::gil_scoped_acquire gil;
+    py::module_::import("fp8_gmm_amd.backend")
+        .attr("run_described_pass")(which, (int)device.index(), py::bytes(static_cast<const char*>(desc), bytes));
+    return;
+  }
   fp8gmm_pass_plan plan;
   alignas(16) unsigned char tables[FP8GMM_PASS_TABLES_BYTES];
   check(fp8gmm_lay_out_pass(which, desc, &plan, tables));
@@ -425,4 +439,5 @@ PYBIND11_MODULE(_host, m) {
       .def_readonly("due", &Due::due);
   m.def("linear_step", &linear_step);
   m.def("mlp_step", &mlp_step);
+  m.def("set_kernel_timing", [](bool on) { kernel_timing.store(on, std::memory_order_relaxed); });
 }

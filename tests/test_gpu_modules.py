@@ -1082,3 +1082,30 @@ def test_native_passes_on_a_side_stream_with_the_backward_in_another_thread(dev,
         for a, b in zip(*res):
             assert torch.equal(a.view(torch.int16), b.view(torch.int16))
         torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["linear", "mlp"])
+def test_kernel_timing_around_a_backward_pass_alone(dev, kind):
+    """Every launch of the backward pass is recorded although its forward pass ran outside the block, with the bits of an
+    untimed pass."""
+    from fp8_gmm_amd import backend
+
+    pkg = _pkg()
+    g, sizes, res = gen(95), torch.tensor([70, 0, 33]), []
+    x, dy = randn_bf16((103, 64), g).to(dev), randn_bf16((103, 96 if kind == "linear" else 64), g, 1e-2).to(dev)
+    mod = (pkg.GroupedLinear if kind == "linear" else pkg.GroupedMlp)(64, 96, 3, torch.bfloat16, device=dev).eval()
+    for timed in (False, True):
+        mod.zero_grad()
+        xi = x.clone().requires_grad_()
+        out = mod(xi, sizes)
+        if timed:
+            with backend.kernel_timing() as timing:
+                out.backward(dy)
+        else:
+            out.backward(dy)
+        res.append([xi.grad] + [p.grad for p in mod.parameters()])
+    for a, b in zip(*res):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    counts = {name: rec["launches"] for name, rec in timing.summary().items()}
+    assert counts["grouped_gemm"] == (2 if kind == "linear" else 4) and sum(counts.values()) == (3 if kind == "linear" else 6)
