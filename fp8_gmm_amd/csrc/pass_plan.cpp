@@ -1,12 +1,14 @@
-// One call that plans a whole pass of a grouped linear layer or of a grouped MLP: the tensor descriptors of its cast
-// launches, the problem tables of its grouped GEMMs and their work lists, written straight into the (pinned) buffer
-// that the caller uploads, plus a second call that runs one planned launch.  Host only.
+// Plans a whole pass of a grouped linear layer or of a grouped MLP in one call: the tensor descriptors of its cast launches,
+// the problem tables of its grouped GEMMs and their work lists.  A pass is described launch by launch (pass_spec.h); the
+// planning calls write its tables into host memory (fp8gmm_plan_*: staging memory, a kernel copies it), or the description
+// itself becomes the argument of the kernel that writes them on the device (fp8gmm_lay_out_pass, fp8gmm_build_pass;
+// pass_tables.hip).  fp8gmm_run_planned runs one planned launch.  Host code; the kernels are elsewhere.
 //
 // The reference does the equivalent host work per call in C++: CutlassFp8GroupedGemm builds the problem sizes,
 // pointers and strides of every expert (csrc/fp8_gmm.cu:115-135) and MultiPadCastTranspose packs the tensor list
 // into its kernel arguments (csrc/multi_pad_fusion.cu:455-502), driven by a Python loop over the experts
-// (fp8_gmm/grouped_linear.py:109-188, fp8_gmm/grouped_mlp.py:60-318).  With 64 experts that loop - here: the array arithmetic that replaced it -
-// costs more host time than the kernels run; from (group_sizes, base pointers, scaling-metadata bases) the whole
+// (fp8_gmm/grouped_linear.py:109-188, fp8_gmm/grouped_mlp.py:60-318).  With 64 experts that loop (here: the array
+// arithmetic that replaced it) costs more host time than the kernels run; from (group_sizes, base pointers, scaling-metadata bases) the whole
 // pass is a few microseconds of C.
 #include <stdint.h>
 #include <string.h>
@@ -368,13 +370,13 @@ int lay_out_pass(Pass& pass, fp8gmm_pass_plan* out, PassTables* t) {
     describe_gemm(pass, l, probs, rec);
     t->gemm[t->n_gemms++] = l.gemm;
   }
-  // the table kernel's workgroups: one per cast, one per 256 records of a work list
+  // the table kernel's workgroups: one per cast, one per kPassRecordsPerBlock records of a work list
   int blocks = 0;
   for (int c = 0; c < t->n_casts; ++c) t->first_block[c] = blocks++;
   for (int g = 0; g < t->n_gemms; ++g) {
     t->first_block[t->n_casts + g] = blocks;
     const int records = t->ranges[g].rounds * t->ranges[g].grid;
-    blocks += records > 0 ? (records + 255) / 256 : 1;
+    blocks += records > 0 ? (records + fp8gmm::kPassRecordsPerBlock - 1) / fp8gmm::kPassRecordsPerBlock : 1;
   }
   t->blocks = e > 0 ? blocks : 0;
   out->n_launches = pass.n_launches;

@@ -73,6 +73,7 @@ struct GemmRanges {
 
 constexpr int kPassMaxExperts = FP8GMM_PASS_MAX_EXPERTS;
 constexpr int kPassMaxCasts = 2, kPassMaxGemms = 4;
+constexpr int kPassRecordsPerBlock = 256;   // records of a work list that a workgroup of the table kernel writes
 
 // The table kernel's argument (and the opaque `tables` of the C ABI).  A kernel's arguments may take 4 KB.
 struct PassTables {

@@ -24,7 +24,7 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kExperts = kPassMaxExperts;
-constexpr int kRecordsPerBlock = kThreads;
+static_assert(kPassRecordsPerBlock == kThreads, "a lane per record");
 
 // exclusive prefix sums of v[0 .. n) in place, their total in v[n]; all threads of the workgroup
 __device__ void exclusive_scan(int* v, int n, int* wave_sums) {
@@ -181,7 +181,7 @@ __device__ void write_gemm(const PassTables& t, int g, int block, uint8_t* blob,
       }
     }
   }
-  const int index = block * kRecordsPerBlock + (int)threadIdx.x;
+  const int index = block * kPassRecordsPerBlock + (int)threadIdx.x;
   if (index >= ranges.rounds * ranges.grid) return;
   const int wg = index % ranges.grid, x = wg % kNumXcd, j = wg / kNumXcd;
   const GemmRanges::Xcd& xc = ranges.xcd[x];

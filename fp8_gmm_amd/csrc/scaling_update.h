@@ -21,7 +21,7 @@ namespace fp8gmm {
 // read and to write, a few microseconds of memory traffic.  With one lane per column the rows are a chain of dependent
 // round trips (61 us for 20 columns, 111 us for 1280 with the rows read eight at a time).  Here a workgroup owns
 // kScalingCols neighbouring columns (one 64-byte piece of every row) and moves kScalingRows rows at once: every lane
-// has its sixteen rows in flight together, all of them are read before the barrier and written one place up behind it, so the
+// has its 64 rows in flight together, all of them are read before the barrier and written one place up behind it, so the
 // shift can be done in place; longer histories take the next rows in turn.  A workgroup per column piece and not per
 // row range: the row that one range writes is the row its neighbour still has to read.
 constexpr int kScalingCols = 16;
