@@ -995,10 +995,11 @@ def _run_pass(device, which, desc, fields, snapshot, host_planned):
             value = value.ctypes.data
         setattr(desc, name, value)
     index = device.index if device.index is not None else torch.cuda.current_device()
-    grid = _lib.gemm_grid(_lib.init(index))
-    desc.grid = grid
-    desc.stream_k = int(bool(options.stream_k))
-    desc.tile_policy = TILE_POLICIES[options.tile]
+    if not desc.grid:   # else described with its launch policy (run_described_pass)
+        desc.grid = _lib.gemm_grid(_lib.init(index))
+        desc.stream_k = int(bool(options.stream_k))
+        desc.tile_policy = TILE_POLICIES[options.tile]
+    grid = desc.grid
     plan = _lib.PassPlan()
     if desc.experts <= _lib.PASS_MAX_EXPERTS and desc.tokens <= _lib.PASS_MAX_ROWS and 2 * grid <= _lib.PASS_MAX_GRID:
         tables = _lib.PassTables()
@@ -1033,7 +1034,7 @@ def _run_pass(device, which, desc, fields, snapshot, host_planned):
 
 def run_described_pass(which, device_index, desc):
     """A backward pass as the native host path describes it (the bytes of its C structure), launch by launch: where
-    ``kernel_timing`` wants every launch bracketed with events."""
+    ``kernel_timing`` wants every launch bracketed with events.  The launch policy is the description's."""
     desc = (_lib.LinearPass if which == _lib.LINEAR_BACKWARD else _lib.MlpPass).from_buffer_copy(desc)
     _run_pass(torch.device("cuda", device_index), which, desc, {}, None, None)
 

@@ -1109,3 +1109,22 @@ def test_kernel_timing_around_a_backward_pass_alone(dev, kind):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16))
     counts = {name: rec["launches"] for name, rec in timing.summary().items()}
     assert counts["grouped_gemm"] == (2 if kind == "linear" else 4) and sum(counts.values()) == (3 if kind == "linear" else 6)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["linear", "mlp"])
+def test_a_timed_backward_pass_keeps_the_policy_of_its_forward_pass(dev, kind):
+    """The tile that was in force for the forward pass also cuts the GEMMs of a backward pass under ``kernel_timing``."""
+    from fp8_gmm_amd import backend
+
+    pkg = _pkg()
+    g = gen(96)
+    x = randn_bf16((103, 64), g).to(dev).requires_grad_()
+    mod = (pkg.GroupedLinear if kind == "linear" else pkg.GroupedMlp)(64, 96, 3, torch.bfloat16, device=dev)
+    for tile in ("128", "256"):
+        with backend.gemm_options(tile=tile):
+            out = mod(x, torch.tensor([70, 0, 33]))
+        with backend.gemm_options(tile="256" if tile == "128" else "128"), backend.kernel_timing() as timing:
+            out.sum().backward()
+        forms = timing.summary()["grouped_gemm"]["forms"]
+        assert forms and all(("128 x 128 tiles" in f) == (tile == "128") for f in forms), forms
