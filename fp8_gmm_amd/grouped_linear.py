@@ -364,8 +364,8 @@ class GroupedLinear(Fp8GroupedModuleBase):
         return self._cast_ahead([(self.weight_tensor, Fp8TensorType.kWeightGroup1)])
 
     def forward(self, input, group_sizes, is_first_microbatch=None):
-        ahead = self._take_ahead(is_first_microbatch)
         refuse_tracing()
+        ahead = self._take_ahead(is_first_microbatch)
         due = None
         if ahead is None:
             due = self._prepare(input.device, is_first_microbatch, self.num_groups)

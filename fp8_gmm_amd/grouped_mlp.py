@@ -448,8 +448,8 @@ class GroupedMlp(Fp8GroupedModuleBase):
         return self._cast_ahead([(self.fc1_weight, _T.kWeightGroup1), (self.fc2_weight, _T.kWeightGroup2)])
 
     def forward(self, input, group_sizes, has_tp=False, tp_group=None, is_first_microbatch=None):
-        ahead = self._take_ahead(is_first_microbatch)
         refuse_tracing()
+        ahead = self._take_ahead(is_first_microbatch)
         due = None
         if ahead is None:
             due = self._prepare(input.device, is_first_microbatch, self.num_groups * 2)

@@ -373,12 +373,13 @@ def test_modules_refuse_to_be_traced(kind, grad):
 
     module = (GroupedLinear if kind == "linear" else GroupedMlp)(16, 32, 2, torch.bfloat16, device="cpu")
     x = torch.zeros(3, 16, dtype=torch.bfloat16, requires_grad=grad)
+    module._ahead = ahead = ()   # what cast_weights_ahead() leaves for the next forward pass
     with torch.set_grad_enabled(grad):
         with pytest.raises(RuntimeError, match="cannot be traced"):
             torch.jit.trace(module, (x, torch.tensor([1, 2])), check_trace=False)
         with pytest.raises(RuntimeError, match="cannot be traced"):
             make_fx(lambda t: module(t, [1, 2]))(x)
-    assert module._fp8_steps == 0
+    assert module._fp8_steps == 0 and module._ahead is ahead
 
 
 def _native_module_on_the_cpu(monkeypatch, kind):
