@@ -17,47 +17,58 @@ static __device__ __align__(256) uint8_t scratch[(size_t)kStaticSlots * FP8GMM_G
 namespace fp8gmm {
 namespace {
 
-// Completes the tiles that the main kernel shared along K.  MT workgroups per such tile (one record of the
+// Completes the tiles that the main kernel shared along K.  Eight workgroups per such tile (one record of the
 // fix-up list): together they add the tile's pieces, which lie in consecutive workspace slots in K order, and
-// apply the epilogue.  A launch has few shared tiles (64 at most on 256 compute units), each with a megabyte of
-// partial sums to read: four workgroups per tile put the whole chip to it.
-// 1024 threads: thread T owns the 16-byte groups T + 1024 q of a slot, i.e. register group g = T / 256 of the
-// MFMA tiles (i, j) = q of main-kernel thread T % 256: 4 consecutive columns of one row each; workgroup `part`
-// of a tile takes i = part (q = part * NT .. part * NT + NT - 1).  The sums and the arithmetic are those of
+// apply the epilogue.
+// 512 threads: workgroup `part` of a tile takes the MFMA tiles (i, j) with i = part / 2 and j = 2 (part % 2) and the one
+// beside it - whole 128-byte lines of the result -, thread T the four 16-byte register groups of the tile with
+// j = 2 (part % 2) + T / 256 that main-kernel thread T % 256 stored.  The sums and the arithmetic are those of
 // tile_epilogue's general paths, so a shared tile gets the same bits as a whole one.
-constexpr int kFixupThreads = 1024;
-constexpr int kFixupSplit = MT;  // workgroups per shared tile
-static_assert(kFixupThreads == 4 * NTHREADS, "one register group of every MFMA tile per thread");
+// Bound: a megabyte of partial sums per shared tile and what it takes to ask for it.  kFixupAhead pieces are under way
+// at once behind the first one.  (Four workgroups of 1024 threads
+// per tile that asked for one piece at a time -> this: 20 slots of one XCD 10.1 -> 7.5 us; four launches of 256 - 336
+// slots 87 -> 83; 320 slots 26, either way: 84 MB that come back from memory.)
+constexpr int kFixupSplit = MT * NT / 2;     // workgroups per shared tile
+constexpr int kFixupThreads = 2 * NTHREADS;
+constexpr int kFixupAhead = 3;
+constexpr int kGroups = 4;                   // 16-byte register groups of an MFMA tile
 
 __global__ __launch_bounds__(kFixupThreads) void grouped_gemm_fixup_kernel(
     const fp8gmm_gemm_problem* __restrict__ probs, const fp8gmm_gemm_fixup_desc* __restrict__ fixups, int out_kind,
     int epilogue, const uint8_t* __restrict__ workspace) {
   const fp8gmm_gemm_fixup_desc fx = fixups[blockIdx.x / kFixupSplit];
   const int part = blockIdx.x % kFixupSplit;
+  const int t = threadIdx.x % NTHREADS;
+  const int i = part / (NT / 2), jj = 2 * (part % (NT / 2)) + threadIdx.x / NTHREADS;
+
+  const f32x4* const own = reinterpret_cast<const f32x4*>(workspace + (size_t)fx.first_slot * kPartialBytes) +
+                           (size_t)(i * NT + jj) * kGroups * NTHREADS + t;
+  constexpr int kSlotGroups = kPartialBytes / (int)sizeof(f32x4);
+  f32x4 sum[kGroups];
+#pragma unroll
+  for (int g = 0; g < kGroups; ++g) sum[g] = __builtin_nontemporal_load(own + g * NTHREADS);
+  for (int w = 1; w < fx.n_pieces; w += kFixupAhead) {
+    f32x4 piece[kFixupAhead][kGroups];
+#pragma unroll
+    for (int u = 0; u < kFixupAhead; ++u) {
+      if (w + u >= fx.n_pieces) break;
+#pragma unroll
+      for (int g = 0; g < kGroups; ++g)
+        piece[u][g] = __builtin_nontemporal_load(own + (size_t)(w + u) * kSlotGroups + g * NTHREADS);
+    }
+#pragma unroll
+    for (int u = 0; u < kFixupAhead; ++u) {
+      if (w + u >= fx.n_pieces) break;
+#pragma unroll
+      for (int g = 0; g < kGroups; ++g) sum[g] += piece[u][g];
+    }
+  }
+
   const fp8gmm_gemm_problem pr = probs[fx.prob];
   const int m0 = fx.m0, n0 = fx.n0;
-
-  const int t = threadIdx.x % NTHREADS, g = threadIdx.x / NTHREADS;
   const int lane = t & 63, wave = t >> 6;
   const int wave_m = wave / WAVES_N, wave_n = wave % WAVES_N;
   const int l32 = lane & 31, khalf = lane >> 5;
-
-  f32x4 sum[NT];
-  {
-    const f32x4* first = reinterpret_cast<const f32x4*>(workspace + (size_t)fx.first_slot * kPartialBytes) +
-                         (size_t)part * NT * kFixupThreads + threadIdx.x;
-#pragma unroll
-    for (int q = 0; q < NT; ++q) sum[q] = __builtin_nontemporal_load(first + q * kFixupThreads);
-  }
-  for (int w = 1; w < fx.n_pieces; ++w) {
-    const f32x4* next = reinterpret_cast<const f32x4*>(workspace + (size_t)(fx.first_slot + w) * kPartialBytes) +
-                        (size_t)part * NT * kFixupThreads + threadIdx.x;
-    f32x4 piece[NT];
-#pragma unroll
-    for (int q = 0; q < NT; ++q) piece[q] = __builtin_nontemporal_load(next + q * kFixupThreads);
-#pragma unroll
-    for (int q = 0; q < NT; ++q) sum[q] += piece[q];
-  }
 
   const int M = pr.m, N = pr.n;
   const float sa_inv = pr.a_scale_inv ? *pr.a_scale_inv : 1.f;
@@ -72,15 +83,14 @@ __global__ __launch_bounds__(kFixupThreads) void grouped_gemm_fixup_kernel(
   const float cs = pr.c_scale ? *pr.c_scale : 1.f;
   float amax = 0.f;
 #pragma unroll
-  for (int q = 0; q < NT; ++q) {
-    const int i = part, jj = q;
+  for (int g = 0; g < kGroups; ++g) {
     const int m = m0 + wave_m * WM + i * 32 + l32;
     const int n = n0 + wave_n * WN + jj * 32 + g * 8 + khalf * 4;
     if (m >= M || n >= N) continue;
     float v[4], r[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      v[e] = two ? scaled_twice(sum[q][e], sa_inv, sb_inv) : sum[q][e] * s;
+      v[e] = two ? scaled_twice(sum[g][e], sa_inv, sb_inv) : sum[g][e] * s;
       r[e] = gelu ? gelu_tanh_fast(v[e]) : v[e];
     }
     const int64_t off = (int64_t)m * ldc + n;

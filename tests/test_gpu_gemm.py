@@ -116,6 +116,37 @@ def test_tiles_shared_along_k_are_exact(dev, a_dtype, sizes, n, k, monkeypatch):
             row += m
 
 
+@pytest.mark.parametrize("pieces", [3, 4, 5, 7, 8])
+def test_shared_tiles_of_every_number_of_pieces_are_exact(dev, pieces, monkeypatch):
+    """One tile, cut into as many pieces as its K = 128 steps allow (four each): the fix-up launch reads the first piece
+    and the following ones three at a time, with one, two or three of them in the last turn.  Exact sums, as above; the
+    tile's last row and columns are missing."""
+    from fp8_gmm_amd import _lib
+
+    backend = _backend()
+    monkeypatch.setattr(backend.options, "tile", "256")
+    m, n, k = 251, 200, 512 * pieces
+    import numpy as np
+
+    table = np.zeros(1, dtype=_lib.GEMM_PROBLEM)
+    table[0]["a"] = table[0]["b"] = table[0]["c"] = 0x1000
+    table[0]["m"], table[0]["n"], table[0]["k"] = m, n, k
+    table[0]["lda"] = table[0]["ldb"] = k
+    table[0]["ldc"] = n
+    grid = _lib.gemm_grid(torch.cuda.get_device_properties(dev).multi_processor_count)
+    plan, _, fixups = _lib.plan_grouped_gemm_launch(table, 0, grid, True)
+    assert len(fixups) == 1 and fixups[0]["n_pieces"] == pieces
+
+    g = gen(pieces)
+    vals = torch.tensor([0.0, 0.5, -0.5, 1.0, -1.0, 2.0, -2.0, 0.25])
+    a = _q(vals[torch.randint(0, 8, (m, k), generator=g)].to(torch.bfloat16), E4M3)
+    b = _q(vals[torch.randint(0, 8, (1, n, k), generator=g)].to(torch.bfloat16), E4M3)
+    one = torch.ones(1, device=dev)
+    got = backend.fp8_gmm(a.to(dev), b.to(dev), torch.tensor([m]), one, one)
+    want = (a.float() @ b[0].float().t()).to(torch.bfloat16)
+    assert torch.equal(got.cpu().view(torch.int16), want.view(torch.int16))
+
+
 def test_identity_weights_reproduce_a(dev):
     backend = _backend()
     g = gen(7)
