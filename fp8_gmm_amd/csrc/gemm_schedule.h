@@ -26,12 +26,16 @@ namespace fp8gmm {
 constexpr int kSkMinPairs = 4;        // never cut pieces shorter than this many K = 128 steps
 constexpr int kSkMaxPieces = 8;       // average pieces per tile the region may be cut into
 constexpr int kSkMaxRounds = 24;      // with more full rounds than this the tail cannot cost enough to share it
-// The second launch, which completes the shared tiles, costs about kSkFixupLaunch K = 128 steps of time (5 us:
-// the gap between two launches) plus kSkFixupPerTile / 100 steps per shared tile of the XCD (four workgroups per
-// tile on 256 compute units, a megabyte of partial sums each), three times that when it has the GELU epilogue to
-// apply; sharing has to save half as much again.
+// What sharing costs, in K = 128 steps of time: kSkFixupLaunch for the second launch, which completes the shared tiles
+// (5 us: the gap between two launches), and one step per workspace slot of an XCD while all eight of them share - a slot
+// is 256 KB to write and to read again, 4 MB for the chip.  Measured with the pieces forced, 8 experts, K = 4096, 10
+// remainder tiles on 32 workgroups: 2 pieces a tile 147 us, 3 154, 32 pieces over the ten tiles (40 slots) 161, not
+// shared 146; 6 tiles: 135, 136 and, 5 pieces a tile, 139, 141 (36 slots), not shared 138; K = 14336, 8 tiles: 2, 3 or 4
+// pieces 5536 - 5555 us for an MLP's step, not shared 5608; one XCD of the eight sharing 4 tiles of 17 steps: 17 pieces
+// 164 us for a layer's step, 12 164, 8 171, not shared 171.  With the GELU epilogue to apply, a shared tile costs
+// kSkGeluPerTile / 100 steps more.
 constexpr int kSkFixupLaunch = 4;
-constexpr int kSkFixupPerTile = 75;
+constexpr int kSkGeluPerTile = 150;
 constexpr int kPartialBytes = BM * BN * 4;  // one slot: the fp32 accumulators of one tile
 constexpr int kTileOverhead = 4;      // fixed cost of a tile (epilogue, switch) in K = 128 steps, measured
 constexpr int kSlotsPerWg = 2;        // a piece that starts inside a tile, one that ends inside a tile
@@ -46,7 +50,7 @@ struct Sched {
   int sk_wgs;                  // workgroups that take a piece of the region
   int64_t sk_c0, sk_cost;      // cost before the region, cost of the region (K = 128 steps)
   int64_t total_cost;          // cost of all tiles
-  int fixup_weight;            // 1, or 3 when completing a shared tile includes the GELU epilogue
+  bool gelu;                   // completing a shared tile includes the GELU epilogue
 };
 
 FP8GMM_HD int problem_end_tile(const Sched& s, int p) {
@@ -95,25 +99,37 @@ FP8GMM_HD int first_tile_at_work(const Sched& s, int64_t c, int ov) {
   return work_before(s, t, ov) == c ? t : t + 1;
 }
 
+// first tile of XCD x's range (x = 8: the end of the last one)
+FP8GMM_HD int range_start(const Sched& s, int x) {
+  const int64_t total_work = s.total_cost + (int64_t)kTileOverhead * s.total_tiles;
+  return first_tile_at_work(s, (total_work * x + kNumXcd - 1) / kNumXcd, kTileOverhead);
+}
+// Striding takes a range of n tiles full + 1 rounds, sharing the remainder full + rem / W: worth a thought when that saves
+// a twelfth of the launch by this count.  Measured, sharing returns about half of what the count promises (workgroups do
+// not finish their rounds in step, so part of a last round is hidden anyway), and it costs the second launch and a
+// round trip of the partial sums through memory: config 2's 4.25 rounds (15 % by the count) gain 6.5 %, launches
+// of 14 rounds with a short tail (4 - 6.5 % by the count; the reference's example layer) lost 1 % of their step.
+FP8GMM_HD bool remainder_may_share(int n_tiles, int W) {
+  const int full = n_tiles / W, rem = n_tiles % W;
+  return rem != 0 && full <= kSkMaxRounds && (int64_t)(W - rem) * 12 >= (int64_t)W * (full + 1);
+}
+
 // Workgroup i runs on XCD i % 8.  The tile list is cut into 8 contiguous ranges of equal WORK, one per XCD,
 // so that workgroups that share an L2 work on neighbouring tiles; the workgroups of an XCD stride through the
 // range, and share its remainder along K when that pays.  k differs per problem in the wgrad form, and a
 // tile costs its K steps plus a fixed part (epilogue, tile switch) worth about kTileOverhead steps: balancing
 // K steps alone left the XCDs that hold the short-K problems 17 % more work than the others.
 FP8GMM_HD void sched_init(Sched& s, const fp8gmm_gemm_problem* probs, int nprob, int total_tiles,
-                                           int xcd, int wgs_per_xcd, bool sk_enable, int fixup_weight = 1) {
-  s.fixup_weight = fixup_weight;
+                                           int xcd, int wgs_per_xcd, bool sk_enable, bool gelu = false) {
+  s.gelu = gelu;
   s.probs = probs;
   s.nprob = nprob;
   s.total_tiles = total_tiles;
   s.wgs = wgs_per_xcd;
   s.total_cost = 0;
   s.total_cost = cost_before(s, total_tiles);
-  const int64_t total_work = s.total_cost + (int64_t)kTileOverhead * total_tiles;
-  const int64_t lo = (total_work * xcd + kNumXcd - 1) / kNumXcd;
-  const int64_t hi = (total_work * (xcd + 1) + kNumXcd - 1) / kNumXcd;
-  s.range_begin = first_tile_at_work(s, lo, kTileOverhead);
-  s.range_end = first_tile_at_work(s, hi, kTileOverhead);
+  s.range_begin = range_start(s, xcd);
+  s.range_end = range_start(s, xcd + 1);
   const int n_x = s.range_end - s.range_begin;
   const int W = wgs_per_xcd;
   s.dp_rounds = (n_x + W - 1) / W;  // plain striding: the last round may be partial
@@ -121,31 +137,37 @@ FP8GMM_HD void sched_init(Sched& s, const fp8gmm_gemm_problem* probs, int nprob,
   s.sk_wgs = 0;
   s.sk_c0 = 0;
   s.sk_cost = 0;
-  const int full = n_x / W, rem = n_x % W;
-  if (!sk_enable || rem == 0 || full > kSkMaxRounds) return;
-  // striding needs full + 1 rounds, sharing the remainder full + rem / W: take it when that saves a twelfth of the
-  // launch by this count.  Measured, sharing returns about half of what the count promises (workgroups do not
-  // finish their rounds in step, so part of a last round is hidden anyway), and it costs the second launch and a
-  // round trip of the partial sums through memory: config 2's 4.25 rounds (15 % by the count) gain 6.5 %, launches
-  // of 14 rounds with a short tail (4 - 6.5 % by the count; the reference's example layer) lost 1 % of their step.
-  if ((int64_t)(W - rem) * 12 < (int64_t)W * (full + 1)) return;
-  const int n_sk = rem;
-  const int rounds = full;
+  if (!sk_enable || !remainder_may_share(n_x, W)) return;
+  const int rounds = n_x / W, n_sk = n_x % W;
   const int sk_begin = s.range_begin + rounds * W;
   const int64_t c0 = cost_before(s, sk_begin);
   const int64_t cost = cost_before(s, s.range_end) - c0;
-  int64_t w = W;
-  if (w > cost / kSkMinPairs) w = cost / kSkMinPairs;
-  if (w > (int64_t)n_sk * kSkMaxPieces) w = (int64_t)n_sk * kSkMaxPieces;
-  if (w <= n_sk) return;  // nothing to gain: at most one piece per tile
-  // ... and more time than the launch that completes the shared tiles takes: the last round shrinks from one
-  // tile's duration to that of one piece.  (128 experts x 768 outputs x 2048 inputs with the GELU epilogue: 24
-  // shared tiles of 16 steps per XCD, the second launch took 75 us to save 10.)
-  {
-    const int64_t saved_x100 = (cost / n_sk - cost / w) * 100;
-    const int64_t fixup_x100 = kSkFixupLaunch * 100 + (int64_t)n_sk * kSkFixupPerTile * s.fixup_weight;
-    if (saved_x100 * 2 < fixup_x100 * 3) return;
+  int sharing = 0;   // XCDs whose partial sums travel at the same time
+  for (int x = 0, begin = 0; x < kNumXcd; ++x) {
+    const int end = range_start(s, x + 1);
+    sharing += remainder_may_share(end - begin, W) ? 1 : 0;
+    begin = end;
   }
+  // The last round shrinks from a tile's duration to a piece's; every piece is a slot to write and to read again.  Pieces
+  // that end where tiles end (so many per tile) leave one slot each; W pieces over n tiles cut up to n - 1 of them in two.
+  int64_t most = W;
+  if (most > cost / kSkMinPairs) most = cost / kSkMinPairs;
+  if (most > (int64_t)n_sk * kSkMaxPieces) most = (int64_t)n_sk * kSkMaxPieces;
+  int64_t best_x100 = cost * 100 / n_sk, w = 0;   // what not sharing takes
+  for (int per_tile = 2;; ++per_tile) {
+    const bool aligned = (int64_t)per_tile * n_sk <= most;
+    const int64_t pieces = aligned ? (int64_t)per_tile * n_sk : most;
+    if (pieces <= n_sk) break;   // at most one piece per tile: nothing to gain
+    const int64_t slots = pieces % n_sk == 0 ? pieces : pieces + n_sk - 1;
+    const int64_t takes_x100 = cost * 100 / pieces + kSkFixupLaunch * 100 + slots * 100 * sharing / kNumXcd +
+                               (s.gelu ? (int64_t)n_sk * kSkGeluPerTile * sharing / kNumXcd : 0);
+    if (takes_x100 < best_x100) {
+      best_x100 = takes_x100;
+      w = pieces;
+    }
+    if (!aligned) break;
+  }
+  if (w == 0) return;
   s.dp_rounds = rounds;
   s.sk_begin = sk_begin;
   s.sk_wgs = (int)w;

@@ -336,7 +336,7 @@ int fp8gmm_plan_grouped_gemm_launch(fp8gmm_gemm_problem* probs, int n, int layou
   // pass 1: sizes.  The tiles that were shared along K first: the pieces of such a tile get consecutive
   // workspace slots, numbered from 0 over the launch, in K order.
   std::vector<Sched> sched(kNumXcd);
-  for (int x = 0; x < kNumXcd; ++x) sched_init(sched[x], probs, n, total_tiles, x, wgs, sk, gelu ? 3 : 1);
+  for (int x = 0; x < kNumXcd; ++x) sched_init(sched[x], probs, n, total_tiles, x, wgs, sk, gelu);
   std::vector<int32_t> slot_map((size_t)kSlotsPerWg * grid, -1);
   std::vector<fp8gmm_gemm_fixup_desc> fix;
   int n_slots = 0;
@@ -516,7 +516,7 @@ int plan_gemm_ranges(fp8gmm_gemm_problem* probs, int n, int layout, int grid, in
     plan->grid = grid;
     for (int x = 0; x < kNumXcd; ++x) {
       Sched s;
-      sched_init(s, probs, n, total_tiles, x, wgs, sk, gelu ? 3 : 1);
+      sched_init(s, probs, n, total_tiles, x, wgs, sk, gelu);
       GemmRanges::Xcd& o = out->xcd[x];
       o.begin = s.range_begin;
       o.end = s.range_end;

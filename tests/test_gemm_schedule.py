@@ -211,6 +211,21 @@ def test_tail_balancing_is_off_when_it_cannot_pay():
     assert check_schedule([(2048, 4096, 4096)] * 8, 256, True) == 0
 
 
+def test_pieces_end_where_tiles_end_unless_whole_tiles_are_faster():
+    """Every slot of partial sums is 256 KB to write and to read again: with remainder tiles of one K the pieces are so
+    many per tile, one slot each, and a remainder that would cost more slots than it saves steps is not shared."""
+    for m_tiles, k, per_tile in [(66, 14336, (2, 8)), (70, 4096, None), (76, 14336, (2, 2)), (74, 4096, None)]:
+        # 8 XCDs of m_tiles tiles on 32 workgroups each: a remainder of 2, 6, 12 or 10 tiles
+        table, total = make_table([(256 * m_tiles, 256, k)] * 8)
+        plan, _, fixups = _lib.plan_grouped_gemm_launch(table, 0, 256, True)
+        if per_tile is None:
+            assert plan.n_slots == 0
+            continue
+        assert len(fixups) == 8 * (m_tiles - 64)
+        assert per_tile[0] <= fixups["n_pieces"].min() and fixups["n_pieces"].max() <= per_tile[1]
+        assert fixups["n_pieces"].min() == fixups["n_pieces"].max()
+
+
 @pytest.mark.parametrize("shapes", [
     [(1, 1, 16)],
     [(256, 256, 128)],
