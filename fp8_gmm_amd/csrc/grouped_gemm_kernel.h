@@ -61,14 +61,6 @@
 
 namespace fp8gmm {
 
-// The result of a tile is written once and not read again by this launch: stored with the streaming hint, it does
-// not push the operand slabs that neighbouring workgroups are about to re-read out of the L2, and the loads that
-// follow the epilogue in the memory pipeline are not held up as long behind its stores (a dense 16384 x 14336 x
-// 4096 launch: 1.14 -> 1.09 million cycles; without any stores it would be 1.06).
-__device__ __forceinline__ void buf_store16_stream(u32x4 v, __amdgpu_buffer_rsrc_t r, uint32_t off) {
-  __builtin_amdgcn_raw_buffer_store_b128(v, r, (int)off, 0, 2);
-}
-
 // A buffer descriptor of a tile's result, made of values that are the same in every lane.  The compiler does not
 // always know that: when it has moved the address arithmetic of a tile to the vector unit (it does, where scalar
 // registers are short), a descriptor built from the outcome sits in vector registers, and every store through it

@@ -467,3 +467,32 @@ def test_tables_reach_the_device_through_the_staging_memory(dev, monkeypatch):
         got = on_device.cpu().numpy()
         assert np.array_equal(got[: len(table)], table), f"upload {i} of {len(table)} bytes"
         assert not got[len(table):].any()
+
+
+@pytest.mark.parametrize("shapes", [
+    [(120, 40)],                           # one workgroup
+    [(31 * 128 - 5, 120)],                 # 31: short of a group
+    [(8 * 128, 512)],                      # 32: one whole group
+    [(300, 11 * 128)],                     # 33
+    [(1000, 256), (7, 136), (515, 1024)],  # 16 + 2 + 40 = 58: a group that spans three tensors, a partial one behind it
+], ids=["1", "31", "32", "33", "58"])
+def test_every_tile_is_taken_once_whatever_the_number_of_workgroups(dev, shapes):
+    """Workgroups are dealt to the tiles in groups of 32, four neighbouring tiles per XCD, the last partial group in order:
+    a tile that two of them took, or none, leaves the filler byte behind."""
+    backend = _backend()
+    g = gen(41)
+    dtype = torch.float8_e4m3fn
+    ins = [randn_bf16(s, g) for s in shapes]
+    scales = _scales(len(shapes), g, positive=True)
+    t_shapes = transpose_shapes(shapes, True)
+    outs, touts = [torch.empty(s, dtype=dtype) for s in shapes], [torch.empty(s, dtype=dtype) for s in t_shapes]
+    amaxes = [torch.zeros(1) for _ in shapes]
+    ref.multi_cast_transpose(ins, outs, touts, scales, amaxes)
+    d_outs = [torch.full(s, 0x55, dtype=torch.uint8, device=dev).view(dtype) for s in shapes]
+    d_touts = [torch.full(s, 0x55, dtype=torch.uint8, device=dev).view(dtype) for s in t_shapes]
+    d_amaxes = [torch.zeros(1, device=dev) for _ in shapes]
+    backend.multi_cast_transpose(_to_dev(ins, dev), d_outs, d_touts, _to_dev(scales, dev), d_amaxes)
+    for i, s in enumerate(shapes):
+        assert_bytes_equal(d_outs[i], outs[i], f"cast {i} {s}")
+        assert_bytes_equal(d_touts[i], touts[i], f"transpose {i} {s}")
+        assert_scalar_bits_equal(d_amaxes[i].cpu(), amaxes[i], f"amax {i}")
