@@ -408,6 +408,50 @@ Tensor mlp_step(const Tensor& x, const Tensor& w1, const Tensor& w2, const py::o
   });
 }
 
+// ---- weights ahead of a pass --------------------------------------------------------------------------------------
+// What a forward pass does before its rows are known: a pass without rows, which is the scaling update and the casts of
+// one weight stack (GroupedLinear) or two (GroupedMlp) into `fp8`.
+void cast_weights(const std::vector<Tensor>& weights, const std::vector<Tensor>& fp8, const Setup& setup, Due& due) {
+  py::gil_scoped_release no_gil;
+  TORCH_CHECK((weights.size() == 1 || weights.size() == 2) && fp8.size() == weights.size(),
+              "fp8_gmm_amd: one or two weight stacks and a result for each");
+  const Tensor& w = weights[0];
+  for (size_t i = 0; i < weights.size(); ++i)
+    TORCH_CHECK(weights[i].dim() == 3 && weights[i].sizes() == fp8[i].sizes() && weights[i].is_contiguous() &&
+                    fp8[i].is_contiguous() && weights[i].size(0) == w.size(0) && weights[i].device() == w.device() &&
+                    fp8[i].device() == w.device() && weights[i].scalar_type() == at::kBFloat16 &&
+                    fp8[i].scalar_type() == setup.fwd_type(),
+                "fp8_gmm_amd: weight stacks and results that do not fit together");
+  if (weights.size() == 2)
+    TORCH_CHECK(weights[1].size(1) == w.size(2) && weights[1].size(2) == w.size(1),
+                "fp8_gmm_amd: fc2's weights do not follow fc1's");
+  const std::vector<int64_t> sizes((size_t)w.size(0), 0);
+  const int64_t slots = 3 * w.size(0) * (int64_t)weights.size();
+  TORCH_CHECK(setup.fwd_scale.numel() >= slots && setup.fwd_scale_inv.numel() >= slots && setup.fwd_amax.size(-1) >= slots,
+              "fp8_gmm_amd: the scaling state has too few slots");
+  const c10::OptionalDeviceGuard guard(w.device());
+  auto run = [&](int which, auto& d) {
+    d.cast_weights = 1;
+    d.fwd_scale = ptr<float>(setup.fwd_scale);
+    d.fwd_scale_inv = ptr<float>(setup.fwd_scale_inv);
+    d.fwd_amax = ptr<float>(setup.fwd_amax);
+    run_pass(which, &d, w.device(), &setup, &due, Tensor(), Tensor());
+  };
+  if (weights.size() == 1) {
+    fp8gmm_linear_pass d = linear_desc(setup, sizes, 0, w.size(2), w.size(1));
+    d.w = ptr<void>(w);
+    d.w_fp8 = ptr<void>(fp8[0]);
+    run(FP8GMM_LINEAR_FORWARD, d);
+  } else {
+    fp8gmm_mlp_pass d = mlp_desc(setup, sizes, 0, w.size(2), w.size(1));
+    d.w1 = ptr<void>(w);
+    d.w1_fp8 = ptr<void>(fp8[0]);
+    d.w2 = ptr<void>(weights[1]);
+    d.w2_fp8 = ptr<void>(fp8[1]);
+    run(FP8GMM_MLP_FORWARD, d);
+  }
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_host, m) {
@@ -439,5 +483,6 @@ PYBIND11_MODULE(_host, m) {
       .def_readonly("due", &Due::due);
   m.def("linear_step", &linear_step);
   m.def("mlp_step", &mlp_step);
+  m.def("cast_weights", &cast_weights);
   m.def("set_kernel_timing", [](bool on) { kernel_timing.store(on, std::memory_order_relaxed); });
 }

@@ -421,6 +421,33 @@ def test_weights_cast_ahead_of_the_pass_give_the_same_bits(dev, kind):
         mods[0](data[0][0], torch.tensor(data[0][1]), is_first_microbatch=True)
 
 
+@pytest.mark.parametrize("shape", [(1, 16, 16), (5, 48, 272), (3, 256, 2064)])
+@pytest.mark.parametrize("kind", ["linear", "mlp"])
+def test_weights_cast_ahead_from_native_code_equal_the_per_launch_path(dev, kind, shape):
+    """The native call is a pass without rows; ``planned_passes=False`` runs the update and the cast one by one.  The same
+    fp8 weights, maxima and scales, with an update due (second and third turn) and without (first, and in evaluation)."""
+    pkg = _pkg()
+    e, h, f = shape
+    cls = pkg.GroupedMlp if kind == "mlp" else pkg.GroupedLinear
+    mods = [cls(h, f, e, torch.bfloat16, device=dev, planned_passes=p) for p in (True, False)]
+    mods[1].load_state_dict(mods[0].state_dict())
+    fp8_recipe = pkg.DelayedScaling(amax_history_len=3, margin=1)
+    for turn in range(4):
+        for mod in mods:
+            mod.train(turn < 3)
+            with pkg.fp8_autocast(fp8_recipe=fp8_recipe):
+                assert mod.cast_weights_ahead()
+        for a, b in zip(mods[0]._ahead, mods[1]._ahead):
+            assert a.valid and b.valid and torch.equal(a.fp8.view(torch.uint8), b.fp8.view(torch.uint8)), turn
+        for name in ("scaling_fwd", "scaling_bwd"):
+            for x, y in zip(*(m.fp8_meta[name].state().values() for m in mods)):
+                assert torch.equal(x, y), (turn, name)
+        with torch.no_grad():
+            for pa, pb in zip(mods[0].parameters(), mods[1].parameters()):
+                pa.mul_(1.5)
+                pb.copy_(pa)
+
+
 def test_cutlass_passes_equal_the_per_launch_path(dev):
     """GroupedLinear(cutlass=True) runs its passes from native code like the default: the bits of the per-launch entry
     points, cached weights and a frozen weight included; forward-mode differentiation is refused."""
