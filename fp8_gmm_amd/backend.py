@@ -799,7 +799,7 @@ def _launch_gemm(table, a_dtype, b_dtype, c_dtype, gelu, device, keep, b_kmajor=
     epi = _lib.EPI_GELU if gelu else _lib.EPI_DGELU if dgelu else 0
     if not dgelu and not layout and _rows_tiles(table):
         plan, blob, off_items, off_fix = _lib.plan_grouped_gemm_blob(table, epi | _lib.GEMM_TILE_ROWS, 2 * grid, False)
-    elif not epi and _small_tiles(table):
+    elif not epi and _small_tiles(table, a_kmajor, c_dtype == torch.bfloat16):
         plan, blob, off_items, off_fix = _lib.plan_grouped_gemm_blob(table, layout | _lib.GEMM_TILE_128, 2 * grid, False)
     elif not epi and c_dtype == torch.bfloat16 and _dual_tiles(table, a_kmajor):
         plan, blob, off_items, off_fix = _lib.plan_grouped_gemm_blob(table, layout | _lib.GEMM_TILE_DUAL, grid, False)
@@ -836,9 +836,9 @@ def _launch_gemm(table, a_dtype, b_dtype, c_dtype, gelu, device, keep, b_kmajor=
 #
 # Tile size of a grouped GEMM.  The 256 x 256 tile is the fast one per flop.  The 128 x 128 tile (two workgroups per
 # compute unit, twice the operand traffic from L2) wins where the large tile leaves the machine idle: launches with
-# fewer large tiles than about half the compute units, and launches whose problems are so short or narrow that the
-# large tiles are mostly padding (measured 1.1 - 1.7 x there, 0.8 - 0.9 x on launches that fill the machine with
-# full tiles).  Whole tiles get the same bits from either size; a tile that the large-tile launch shares along K is
+# fewer large tiles than about half the compute units, launches whose problems are so short or narrow that the
+# large tiles are mostly padding, and launches of a few rounds, which are mostly starts, results and tile switches
+# (measured 1.1 - 1.7 x there, 0.8 - 0.9 x on launches that fill the machine with full tiles for long).  Whole tiles get the same bits from either size; a tile that the large-tile launch shares along K is
 # summed from fp32 partial sums, a deterministic but differently associated sum.  options.tile = "256" / "128"
 # forces one size.
 #
@@ -920,15 +920,34 @@ def _rows_tiles(table):
         and int(m.sum()) <= most * problems
 
 
-def _small_tiles(table):
+# The 128 x 128 tile: csrc/pass_plan.cpp, small_tiles_pay and small_tiles_beat_dual, has the rules and their measurements.
+def _small_tiles(table, a_kmajor, c_bf16):
     if options.tile != "auto":
         return options.tile == "128"
     m, n = table["m"].astype(np.int64), table["n"].astype(np.int64)
-    large = int((((m + 255) // 256) * ((n + 255) // 256)).sum())
+    tiles = ((m + 255) // 256) * ((n + 255) // 256)
+    large = int(tiles.sum())
     if large == 0:
         return False
-    small = int((((m + 127) // 128) * ((n + 127) // 128)).sum())
-    return large <= 160 or 2 * small <= 5 * large
+    if large <= 160 or 2 * int((((m + 127) // 128) * ((n + 127) // 128)).sum()) <= 5 * large:
+        return True
+    k = table["k"].astype(np.int64)
+    if not a_kmajor:
+        return c_bf16 and _dual_tiles(table, False) and _small_beat_dual(m, n, k, large)
+    own = np.maximum((k + 127) // 128, 1)
+    steps, longest = int((tiles * own).sum()), int(own[tiles > 0].max())
+    if large <= 2600 and steps <= 9000 and 2 * steps <= 17 * large and (large <= 800 or 2 * steps >= 3 * large):
+        return True
+    return 1024 * longest >= 3 * steps and 4096 < steps <= 13000 and steps <= 16 * large
+
+
+def _small_beat_dual(m, n, k, large):
+    if int(n.min()) < 512:
+        return False
+    dual = int((((m + 127) // 128) * ((n + 255) // 256)).sum())
+    if int(k.max()) <= 1152:
+        return large <= 600
+    return large <= 300 and 100 * dual <= 95 * (-(-dual // 256) * 256)
 
 
 # The partial sums of tiles shared along K go to a workspace that the library takes from the caller.  One buffer

@@ -118,15 +118,33 @@ struct Pass {
 };
 
 // Which tile a launch takes when the caller leaves the choice to the library: the 128 x 128 tile where the
-// 256 x 256 tiles would be fewer than about half the compute units or mostly padding (see FP8GMM_GEMM_TILE_128).
-bool small_tiles_pay(const fp8gmm_gemm_problem* p, int n) {
-  int64_t large = 0, small = 0;
+// 256 x 256 tiles would be fewer than about half the compute units or mostly padding (see FP8GMM_GEMM_TILE_128), and
+// where the launch is short for other reasons: two workgroups per compute unit hide each other's starts, results and tile
+// switches, which are most of a short launch, and a range's end is spread over tiles a quarter of the size.  What the form
+// pays, twice the operand bytes from L2 per flop, grows with the K = 128 steps of the large tiles ("steps" below).
+// Weight gradients, measured inside a layer's step, large tiles -> this form in us (experts, result, rows each): 16 of
+// 1024 x 2048, 250 30.3 -> 23.2, 1000 48 -> 39; 8 of 4096 x 4096, 500 90 -> 86; 48 of 1536 x 1536, 400 76 -> 76; 1024 tiles
+// of one step, stores only, 36 -> 42; 128 of 2048 x 768, 512 (12288 steps) 156 -> 182; 2 of 4096 x 4096, 2000 (16 steps a
+// tile) 65 -> 68.  Under a skewed split large tiles wait for the longest contraction: 96 of 512 x 1024, 700 146 -> 98, 64 of
+// 1024 x 1408, 1000 127 -> 107, 64 of 2048 x 1408, 384 158 -> 146; 32 of 2048 x 4096, 300 (half a share) 148 -> 162.  Over
+// 190 launches that this rule changes, 17 % less time in the mean; 2 of them lose more than a twentieth.
+bool small_tiles_pay(const fp8gmm_gemm_problem* p, int n, int layout) {
+  int64_t large = 0, small = 0, steps = 0, longest = 0;
   for (int i = 0; i < n; ++i) {
     const int64_t m = p[i].m, nn = p[i].n;
-    large += ((m + 255) / 256) * ((nn + 255) / 256);
+    const int64_t tiles = ((m + 255) / 256) * ((nn + 255) / 256);
+    const int64_t own = p[i].k > 128 ? (p[i].k + 127) / 128 : 1;
+    large += tiles;
     small += ((m + 127) / 128) * ((nn + 127) / 128);
+    steps += tiles * own;
+    if (tiles > 0 && own > longest) longest = own;
   }
-  return large != 0 && (large <= 160 || 2 * small <= 5 * large);
+  if (large == 0) return false;
+  if (large <= 160 || 2 * small <= 5 * large) return true;
+  if (!(layout & FP8GMM_GEMM_A_KMAJOR)) return false;
+  if (large <= 2600 && steps <= 9000 && 2 * steps <= 17 * large && (large <= 800 || 2 * steps >= 3 * large)) return true;
+  // one expert's contraction takes three quarters of a compute unit's share of the launch
+  return 1024 * longest >= 3 * steps && steps > 4096 && steps <= 13000 && steps <= 16 * large;
 }
 
 // ... and the form with two sets of accumulators (FP8GMM_GEMM_TILE_DUAL): a contraction of up to 2048 whose
@@ -142,6 +160,26 @@ bool dual_tiles_pay(const fp8gmm_gemm_problem* p, int n, int layout) {
     if (p[i].k > k_max) k_max = p[i].k;
   }
   return k_max <= 2048 && bytes <= ((int64_t)320 << 20);
+}
+
+// Which of those launches the 128 x 128 tile is the better one for all the same: the short ones, up to two rounds of large
+// tiles; at more than nine K steps, up to one round and not where the 128 x 256 tiles come out as whole rounds; not results
+// of a column or two of tiles, whose operand a it reads twice as often.  Measured as above, two sets -> this form: K = 1024, 8
+// experts of 4096 columns, 500 rows 30.4 -> 25.8, 1000 44.5 -> 39.4, 2000 (1056 large tiles) 73 -> 74; K = 880, 10 of 2160,
+// 600 27 -> 25; K = 1632, 9 of 1632, 1000 44 -> 36, 2000 58 -> 66; K = 2048, 16 of 2048, 500 43 -> 39, 32 of 1024, 250 32 ->
+// 27; K = 2048, 8 of 256, 6000 34 -> 35; K = 2032 with 1.97 rounds 42.6 -> 46.4.
+bool small_tiles_beat_dual(const fp8gmm_gemm_problem* p, int n) {
+  int64_t large = 0, dual = 0;
+  int32_t k = 0, narrowest = INT32_MAX;
+  for (int i = 0; i < n; ++i) {
+    const int64_t columns = ((int64_t)p[i].n + 255) / 256;
+    large += (((int64_t)p[i].m + 255) / 256) * columns;
+    dual += (((int64_t)p[i].m + 127) / 128) * columns;
+    if (p[i].k > k) k = p[i].k;
+    if (p[i].n < narrowest) narrowest = p[i].n;
+  }
+  if (narrowest < 512) return false;
+  return k <= 1152 ? large <= 600 : large <= 300 && 100 * dual <= 95 * ((dual + 255) / 256 * 256);
 }
 
 // ... and the form for few rows (FP8GMM_GEMM_TILE_ROWS): row-major weights of 64 MB or more that (nearly) every problem
@@ -179,10 +217,14 @@ int tile_flag(const fp8gmm_gemm_problem* probs, int n, const Pass& pass, const P
   if ((l.epi & FP8GMM_EPI_DGELU) == 0 &&
       (pass.tile_policy == FP8GMM_GEMM_TILE_ROWS ? l.gemm.layout == 0 : pass.tile_policy == 0 && rows_pay(probs, n, l.gemm.layout)))
     return FP8GMM_GEMM_TILE_ROWS;
-  const bool small = l.epi == 0 && (pass.tile_policy == 128 || (pass.tile_policy == 0 && small_tiles_pay(probs, n)));
-  const bool dual = !small && l.epi == 0 && l.out_kind == FP8GMM_OUT_BF16 &&
-                    (pass.tile_policy == FP8GMM_GEMM_TILE_DUAL ||
-                     (pass.tile_policy == 0 && dual_tiles_pay(probs, n, l.gemm.layout)));
+  bool small = l.epi == 0 && (pass.tile_policy == 128 || (pass.tile_policy == 0 && small_tiles_pay(probs, n, l.gemm.layout)));
+  bool dual = !small && l.epi == 0 && l.out_kind == FP8GMM_OUT_BF16 &&
+              (pass.tile_policy == FP8GMM_GEMM_TILE_DUAL ||
+               (pass.tile_policy == 0 && dual_tiles_pay(probs, n, l.gemm.layout)));
+  if (dual && pass.tile_policy == 0 && small_tiles_beat_dual(probs, n)) {
+    small = true;
+    dual = false;
+  }
   return small ? FP8GMM_GEMM_TILE_128 : dual ? FP8GMM_GEMM_TILE_DUAL : 0;
 }
 

@@ -292,12 +292,10 @@ class Fp8GroupedModuleBase(torch.nn.Module):
 
         return (input.is_cuda and input.dtype == torch.bfloat16 and input.dim() == 2 and input.is_contiguous()
                 and input.size(0) <= _lib.PASS_MAX_ROWS and backend.options.wgrad == "in_place"
-                and self._native_weights(input.device, *weights))
+                and self._native_weights(_lib, backend, input.device, weights))
 
-    def _native_weights(self, device, *weights):
-        """What ``_native`` asks of everything but the input."""
-        from . import _lib, backend
-
+    def _native_weights(self, _lib, backend, device, weights):
+        """What ``_native`` asks of everything but the input (``_lib``, ``backend``: the caller has imported them)."""
         meta = self.fp8_meta
         if not (meta["planned_passes"] and not meta["reference_layout"] and backend.kernel_timing._active is None
                 and self.num_groups <= _lib.PASS_MAX_EXPERTS and getattr(backend._pending, "items", None) is None):
@@ -351,9 +349,7 @@ class Fp8GroupedModuleBase(torch.nn.Module):
         """The part of a forward pass that needs no group sizes, run now: the delayed-scaling update and the cast of
         the weight stacks ``[(weight, Fp8TensorType of its scaling slots), ...]`` into fp8 tensors of their own, one
         launch.  Returns False (and does nothing) where the pass would use the reference's transposed layout."""
-        from .backend import TensorBatch, multi_quantize
-        from .grouped_linear import stage_weight_cast
-        from .utils import Fp8MetaWrapper, MetaTensorType, to_torch_dtype
+        from . import _lib, backend
 
         first = weights_and_groups[0][0]
         if self.fp8_meta.get("reference_layout") or not first.is_cuda \
@@ -363,7 +359,7 @@ class Fp8GroupedModuleBase(torch.nn.Module):
         weights = [w for w, _ in weights_and_groups]
         due = self._prepare(first.device, None, self.num_groups * len(weights))
         caches = tuple(Fp8WeightCache() for _ in weights)
-        if self._native_weights(first.device, *weights) \
+        if self._native_weights(_lib, backend, first.device, weights) \
                 and all(w.size(0) == self.num_groups and w.size(1) * w.size(2) < 2 ** 31 for w in weights):
             from .native import cast_weights
 
@@ -378,6 +374,10 @@ class Fp8GroupedModuleBase(torch.nn.Module):
             for cache in caches:
                 cache.valid = True
         else:
+            from .backend import TensorBatch, multi_quantize
+            from .grouped_linear import stage_weight_cast
+            from .utils import Fp8MetaWrapper, MetaTensorType, to_torch_dtype
+
             self._run_update(due)
             meta = Fp8MetaWrapper(self.num_groups, self.fp8_meta)
             fp8_dtype = to_torch_dtype(get_fp8_te_dtype(self.fp8_meta["recipe"], fprop_tensor=True))

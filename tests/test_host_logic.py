@@ -297,6 +297,55 @@ def test_the_rule_for_few_rows_is_the_same_in_both_planners():
     assert 20 < taken < 280
 
 
+def test_the_rules_for_tiles_are_the_same_in_both_planners():
+    """backend._small_tiles / _dual_tiles and the pass planner choose the same tile for the three launches of a linear
+    layer, on either side of every bound."""
+    import numpy as np
+
+    from fp8_gmm_amd import _lib, backend
+
+    lib = _lib.load()
+    rng = np.random.default_rng(6)
+    taken = {}
+
+    def tile_of(plan):
+        return (plan.tile_m or plan.tile or 256, plan.tile or 256)
+
+    def want(m, n, k, a_kmajor, layout):
+        table = np.zeros(len(m), dtype=_lib.GEMM_PROBLEM)
+        table["m"], table["n"], table["k"] = m, n, k
+        if not layout and backend._rows_tiles(table):
+            return (_lib.GEMM_ROWS_TILE_M, 128)
+        if backend._small_tiles(table, a_kmajor, True):
+            return (128, 128)
+        return (128, 256) if backend._dual_tiles(table, a_kmajor) else (256, 256)
+
+    for case in range(400):
+        experts = int(rng.choice([1, 3, 8, 16, 48, 128]))
+        k, n = (16 * int(rng.choice([rng.integers(4, 20), rng.integers(16, 130), rng.integers(100, 300)])) for _ in range(2))
+        mean = int(rng.choice([40, 150, 500, 1200, 2500]))
+        sizes = rng.multinomial(experts * mean, rng.dirichlet(np.full(experts, float(rng.choice([0.4, 1, 1000])))))
+        sizes = np.ascontiguousarray(sizes.astype(np.int64))
+        d = _lib.LinearPass()
+        d.experts, d.in_features, d.out_features, d.grid, d.stream_k = experts, k, n, 256, 1
+        d.tokens, d.group_sizes = int(sizes.sum()), sizes.ctypes.data
+        d.dgrad = d.wgrad = 1
+        for f in ("x", "x_fp8", "w_fp8", "y", "dy", "dy_fp8", "dx", "dw", "fwd_scale", "fwd_scale_inv", "fwd_amax",
+                  "bwd_scale", "bwd_scale_inv", "bwd_amax"):
+            setattr(d, f, 1 << 20)
+        fwd, bwd = _lib.PassPlan(), _lib.PassPlan()
+        assert lib.fp8gmm_plan_linear_forward(d, None, 0, fwd) == -8
+        assert lib.fp8gmm_plan_linear_backward(d, None, 0, bwd) == -8
+        got = [tile_of(fwd.launch[1].plan), tile_of(bwd.launch[1].plan), tile_of(bwd.launch[2].plan)]
+        full = np.full(experts, n), np.full(experts, k)
+        assert got == [want(sizes, n, k, False, 0), want(full[0], k, sizes, True, 3), want(sizes, k, n, False, 1)], \
+            (experts, k, n, sizes)
+        for i, g in enumerate(got):
+            taken[i, g] = taken.get((i, g), 0) + 1
+    assert all(taken.get((i, g), 0) > 10 for i in (0, 2) for g in ((128, 128), (128, 256), (256, 256))), taken
+    assert all(taken.get((1, g), 0) > 10 for g in ((128, 128), (256, 256))), taken
+
+
 def test_native_passes_refuse_operands_that_do_not_fit():
     """The kernels follow addresses: widths, group counts and scaling slots that do not fit are refused on the host,
     before anything is launched."""
