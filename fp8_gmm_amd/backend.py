@@ -837,10 +837,10 @@ def _launch_gemm(table, a_dtype, b_dtype, c_dtype, gelu, device, keep, b_kmajor=
 # Tile size of a grouped GEMM.  The 256 x 256 tile is the fast one per flop.  The 128 x 128 tile (two workgroups per
 # compute unit, twice the operand traffic from L2) wins where the large tile leaves the machine idle: launches with
 # fewer large tiles than about half the compute units, launches whose problems are so short or narrow that the
-# large tiles are mostly padding, and launches of a few rounds, which are mostly starts, results and tile switches
-# (measured 1.1 - 1.7 x there, 0.8 - 0.9 x on launches that fill the machine with full tiles for long).  Whole tiles get the same bits from either size; a tile that the large-tile launch shares along K is
-# summed from fp32 partial sums, a deterministic but differently associated sum.  options.tile = "256" / "128"
-# forces one size.
+# large tiles are mostly padding, and launches of a few rounds or of a few steps per tile, which are mostly starts,
+# results and tile switches (measured 1.1 - 1.7 x there, 0.6 - 0.9 x on launches that fill the machine with long, full
+# tiles).  Whole tiles get the same bits from either size; a tile that the large-tile launch shares along K is summed
+# from fp32 partial sums, a deterministic but differently associated sum.  options.tile = "256" / "128" forces one size.
 #
 # Tail balancing of the grouped GEMM (the workgroups of an XCD share their range's last tiles along K) needs
 # scratch memory for partial sums and a second, small launch; options.stream_k = False plans every launch without it.
@@ -936,9 +936,9 @@ def _small_tiles(table, a_kmajor, c_bf16):
         return c_bf16 and _dual_tiles(table, False) and _small_beat_dual(m, n, k, large)
     own = np.maximum((k + 127) // 128, 1)
     steps, longest = int((tiles * own).sum()), int(own[tiles > 0].max())
-    if large <= 2600 and steps <= 9000 and 2 * steps <= 17 * large and (large <= 800 or 2 * steps >= 3 * large):
-        return True
-    return 1024 * longest >= 3 * steps and 4096 < steps <= 13000 and steps <= 16 * large
+    if steps <= 9000 and 2 * steps <= 17 * large:
+        return large <= 1800 or int(n.max()) > 144
+    return (1024 * longest >= 3 * steps and steps <= 16 * large) or (1024 * longest >= 9 * steps and steps <= 24 * large)
 
 
 def _small_beat_dual(m, n, k, large):

@@ -122,14 +122,22 @@ struct Pass {
 // where the launch is short for other reasons: two workgroups per compute unit hide each other's starts, results and tile
 // switches, which are most of a short launch, and a range's end is spread over tiles a quarter of the size.  What the form
 // pays, twice the operand bytes from L2 per flop, grows with the K = 128 steps of the large tiles ("steps" below).
-// Weight gradients, measured inside a layer's step, large tiles -> this form in us (experts, result, rows each): 16 of
-// 1024 x 2048, 250 30.3 -> 23.2, 1000 48 -> 39; 8 of 4096 x 4096, 500 90 -> 86; 48 of 1536 x 1536, 400 76 -> 76; 1024 tiles
-// of one step, stores only, 36 -> 42; 128 of 2048 x 768, 512 (12288 steps) 156 -> 182; 2 of 4096 x 4096, 2000 (16 steps a
-// tile) 65 -> 68.  Under a skewed split large tiles wait for the longest contraction: 96 of 512 x 1024, 700 146 -> 98, 64 of
-// 1024 x 1408, 1000 127 -> 107, 64 of 2048 x 1408, 384 158 -> 146; 32 of 2048 x 4096, 300 (half a share) 148 -> 162.  Over
-// 190 launches that this rule changes, 17 % less time in the mean; 2 of them lose more than a twentieth.
+// Weight gradients, traced inside a layer's step, large tiles -> this form in us (profiles/tile_rules.md has all of 462):
+//   * Up to 9000 steps, 8.5 a tile, whatever the number of tiles: 2048 tiles of 3.4 steps 88 -> 80, of 6.3 (12800 steps) 107 ->
+//     117; 4096 of 2.0 127 -> 115, of 2.7 (10880) 143 -> 148; 8330 of one step 178 -> 137; 448 of 27 (12012) 93 -> 133.  Not
+//     results of up to 144 columns in many tiles: their second column of tiles stores pieces of 32 bytes (144 columns, 1988,
+//     3478 and 4750 tiles of 1.3 - 2.4 steps 81 -> 87, 132 -> 142, 177 -> 210; 160 columns, 2444 64 -> 61).
+//   * Under a skewed split large tiles wait for the longest contraction, the more the larger it is against a compute unit's
+//     share of the launch, at any number of steps: at 0.75 of a share and more 64 of 1408 x 2048 with 10608 / 13536 / 16416 /
+//     20064 steps 158 / 167 / 212 / 242 -> 154 / 158 / 179 / 239, 8 of 2048 x 1024 with 2368 steps 38 -> 28, 16 of 2048 x 2048 with
+//     12.5 / 16.5 / 20 / 24.5 steps a tile 144 / 180 / 159 / 248 -> 110 / 157 / 200 / 241; at half a share 32 of 4096 x 2048 143 ->
+//     148 and 260 -> 370.  At 2.25 shares and more also with 16 to 24 steps a tile, where six launches took 21 % less; past 24 it
+//     depends on how the long contraction falls into the XCDs' ranges (0.76 - 1.64 x).
+// The 386 launches that the rule takes take 16 % less time in the mean.  12 lose more than a twentieth, all but one of them skewed and
+// with 6 to 12 steps a tile; the most: 19 of 1360 x 1392, 26955 rows 83 -> 104; 8 of 2192 x 1264, 8875 43 -> 51; 3 of 5744 x
+// 912, 3178 32 -> 38.  Steps a tile, share and tiles do not tell them from launches that gain as much.
 bool small_tiles_pay(const fp8gmm_gemm_problem* p, int n, int layout) {
-  int64_t large = 0, small = 0, steps = 0, longest = 0;
+  int64_t large = 0, small = 0, steps = 0, longest = 0, widest = 0;
   for (int i = 0; i < n; ++i) {
     const int64_t m = p[i].m, nn = p[i].n;
     const int64_t tiles = ((m + 255) / 256) * ((nn + 255) / 256);
@@ -138,13 +146,14 @@ bool small_tiles_pay(const fp8gmm_gemm_problem* p, int n, int layout) {
     small += ((m + 127) / 128) * ((nn + 127) / 128);
     steps += tiles * own;
     if (tiles > 0 && own > longest) longest = own;
+    if (nn > widest) widest = nn;
   }
   if (large == 0) return false;
   if (large <= 160 || 2 * small <= 5 * large) return true;
   if (!(layout & FP8GMM_GEMM_A_KMAJOR)) return false;
-  if (large <= 2600 && steps <= 9000 && 2 * steps <= 17 * large && (large <= 800 || 2 * steps >= 3 * large)) return true;
-  // one expert's contraction takes three quarters of a compute unit's share of the launch
-  return 1024 * longest >= 3 * steps && steps > 4096 && steps <= 13000 && steps <= 16 * large;
+  if (steps <= 9000 && 2 * steps <= 17 * large) return large <= 1800 || widest > 144;
+  // one expert's contraction takes three quarters of a compute unit's share of the launch, or more than twice that
+  return (1024 * longest >= 3 * steps && steps <= 16 * large) || (1024 * longest >= 9 * steps && steps <= 24 * large);
 }
 
 // ... and the form with two sets of accumulators (FP8GMM_GEMM_TILE_DUAL): a contraction of up to 2048 whose

@@ -346,6 +346,35 @@ def test_the_rules_for_tiles_are_the_same_in_both_planners():
     assert all(taken.get((1, g), 0) > 10 for g in ((128, 128), (256, 256))), taken
 
 
+def test_tiles_of_weight_gradients_follow_the_split_not_its_size():
+    """A split of one skew keeps its tile as the batch grows: the rule asks for the longest contraction in shares of the
+    launch.  Even splits take the small tile up to a number of steps, whatever the number of tiles."""
+    import numpy as np
+
+    from fp8_gmm_amd import backend
+
+    def small(experts, m, n, sizes):
+        table = np.zeros(experts, dtype=backend._lib.GEMM_PROBLEM)
+        table["m"], table["n"], table["k"] = m, n, sizes
+        return backend._small_tiles(table, True, True)
+
+    zipf = 1.0 / np.arange(1, 65) ** 1.1
+    zipf /= zipf.sum()
+    # 64 experts, a quarter of the rows in one: 3 to 40 thousand steps
+    for rows in (9000, 18000, 24576, 30000, 32768, 40000, 49152, 98304):
+        assert small(64, 1408, 2048, np.round(rows * zipf).astype(np.int64)), rows
+    # 8 experts: a contraction of more than two shares, 800 to 6000 steps
+    first = zipf[:8] / zipf[:8].sum()
+    for rows in (3000, 6000, 9000, 12000, 18000, 23000):
+        assert small(8, 2048, 1024, np.round(rows * first).astype(np.int64)), rows
+    # tiles of one step, 1024 to 8192 of them; as many rows under a long even contraction
+    for experts in (16, 64, 128):
+        assert small(experts, 2048, 2048, np.full(experts, 100))
+    assert not small(64, 2048, 2048, np.full(64, 600))
+    # narrow results in many tiles
+    assert small(40, 9600, 144, np.full(40, 100)) and not small(125, 9600, 144, np.full(125, 100))
+
+
 def test_native_passes_refuse_operands_that_do_not_fit():
     """The kernels follow addresses: widths, group counts and scaling slots that do not fit are refused on the host,
     before anything is launched."""
