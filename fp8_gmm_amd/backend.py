@@ -947,7 +947,7 @@ def _small_beat_dual(m, n, k, large):
     dual = int((((m + 127) // 128) * ((n + 255) // 256)).sum())
     if int(k.max()) <= 1152:
         return large <= 600
-    return large <= 300 and 100 * dual <= 95 * (-(-dual // 256) * 256)
+    return large <= 300 and 100 * dual <= 77 * (-(-dual // 256) * 256)
 
 
 # The partial sums of tiles shared along K go to a workspace that the library takes from the caller.  One buffer

@@ -375,6 +375,24 @@ def test_tiles_of_weight_gradients_follow_the_split_not_its_size():
     assert small(40, 9600, 144, np.full(40, 100)) and not small(125, 9600, 144, np.full(125, 100))
 
 
+def test_row_sliced_launches_of_nearly_whole_rounds_keep_two_sets_of_accumulators():
+    """More than nine K steps: the small tile where the last round of 128 x 256 tiles is half empty, not where it is nearly
+    full."""
+    import numpy as np
+
+    from fp8_gmm_amd import backend
+
+    def small(experts, rows, n, k):
+        table = np.zeros(experts, dtype=backend._lib.GEMM_PROBLEM)
+        table["m"], table["n"], table["k"] = rows, n, k
+        return backend._small_tiles(table, False, True)
+
+    for k in (1168, 1600, 2048):
+        assert small(11, 120, 6144, k) and small(12, 300, 2560, k)           # 1.03 and 1.41 rounds
+        assert not small(13, 300, 2816, k) and not small(12, 500, 2560, k)   # 1.68 and 1.88
+    assert small(13, 300, 2816, 1024) and small(12, 500, 2560, 1024)
+
+
 def test_native_passes_refuse_operands_that_do_not_fit():
     """The kernels follow addresses: widths, group counts and scaling slots that do not fit are refused on the host,
     before anything is launched."""
