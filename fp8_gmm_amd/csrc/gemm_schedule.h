@@ -6,6 +6,8 @@
 
 #include <stdint.h>
 
+#include <vector>
+
 #include "fp8gmm.h"
 #include "tiling.h"
 
@@ -27,14 +29,17 @@ constexpr int kSkMinPairs = 4;        // never cut pieces shorter than this many
 constexpr int kSkMaxPieces = 8;       // average pieces per tile the region may be cut into
 constexpr int kSkMaxRounds = 24;      // with more full rounds than this the tail cannot cost enough to share it
 // What sharing costs, in K = 128 steps of time: kSkFixupLaunch for the second launch, which completes the shared tiles
-// (5 us: the gap between two launches), and one step per workspace slot of an XCD while all eight of them share - a slot
-// is 256 KB to write and to read again, 4 MB for the chip.  Measured with the pieces forced, 8 experts, K = 4096, 10
+// (5 us: the gap between two launches), and kSkPerSlot / 100 per workspace slot of an XCD while all eight of them share - a
+// slot is 256 KB to write and to read again, 4 MB for the chip.  Measured with the pieces forced, 8 experts, K = 4096, 10
 // remainder tiles on 32 workgroups: 2 pieces a tile 147 us, 3 154, 32 pieces over the ten tiles (40 slots) 161, not
-// shared 146; 6 tiles: 135, 136 and, 5 pieces a tile, 139, 141 (36 slots), not shared 138; K = 14336, 8 tiles: 2, 3 or 4
-// pieces 5536 - 5555 us for an MLP's step, not shared 5608; one XCD of the eight sharing 4 tiles of 17 steps: 17 pieces
-// 164 us for a layer's step, 12 164, 8 171, not shared 171.  With the GELU epilogue to apply, a shared tile costs
-// kSkGeluPerTile / 100 steps more.
+// shared 146; 6 tiles: 135, 136 and, 5 pieces a tile, 139, 141 (36 slots), not shared 138 (to the rule a draw: not shared);
+// K = 14336, 8 tiles: 2, 3 or 4 pieces 5536 - 5555 us for an MLP's step, not shared 5608; one XCD of the eight sharing 4
+// tiles of 17 steps: 17 pieces 164 us for a layer's step, 12 164, 8 171, not shared 171.  Three quarters of a step per slot
+// fit these figures better, but over the 181 launches of drawn layers that would then be planned otherwise 43 got faster
+// and 42 slower by more than 3 %, 0.9 % faster in the mean: the price stays.  With the GELU epilogue to apply, a shared tile
+// costs kSkGeluPerTile / 100 steps more.
 constexpr int kSkFixupLaunch = 4;
+constexpr int kSkPerSlot = 100;
 constexpr int kSkGeluPerTile = 150;
 constexpr int kPartialBytes = BM * BN * 4;  // one slot: the fp32 accumulators of one tile
 constexpr int kTileOverhead = 4;      // fixed cost of a tile (epilogue, switch) in K = 128 steps, measured
@@ -114,65 +119,202 @@ FP8GMM_HD bool remainder_may_share(int n_tiles, int W) {
   return rem != 0 && full <= kSkMaxRounds && (int64_t)(W - rem) * 12 >= (int64_t)W * (full + 1);
 }
 
+// The tile that workgroup j of the XCD takes in round i of the strided part.  The position inside the round
+// rotates from round to round: how fast a workgroup's steps run depends on where its tile sits in the round's
+// 8 x 4 block (which operand slabs it shares with its neighbours, which memory channels those fall into - up to
+// 6 % between columns of a weight-gradient problem), and a workgroup that kept one position for the whole launch
+// would finish that much earlier or later than the others.
+constexpr int kRoundRotation = 5;  // coprime to every workgroup count in use (multiples of 8 per XCD: 32, 38, ...)
+FP8GMM_HD int dp_tile(const Sched& s, int j, int i) {
+  return s.range_begin + s.wgs * i + (j + kRoundRotation * i) % s.wgs;
+}
+
+// One way to share a remainder: so many equal pieces, and the workspace slots that they leave.
+struct SkSplit {
+  int pieces, slots;
+};
+// The remainder of an XCD's range and the ways to share it.
+struct SkRemainder {
+  int begin, tiles;      // first tile, how many
+  int64_t c0, cost;      // cost before it, its own
+  int n_splits;          // 0: not worth a thought
+  SkSplit split[kSkMaxPieces];
+  // when the last workgroup is through, in hundredths of a K = 128 step: the remainder as whole tiles, and each split (under
+  // one K from when they come to it, otherwise from the launch's start)
+  int64_t whole_x100, shared_x100[kSkMaxPieces];
+};
+
+// A tile that k piece ends fall inside of is left in k + 1 slots; one that no end falls inside of needs none.
+inline int sk_slots(const Sched& s, const SkRemainder& r, int pieces) {
+  int slots = 0, p = problem_of_tile(s, r.begin), problem_end = problem_end_tile(s, p), tile = r.begin;
+  int64_t k = tile_cost(s, p), first = 0;   // the tile's steps, and those of the region before it
+  bool cut = false;
+  const int64_t length = r.cost / pieces;   // the end of piece j is at r.cost * j / pieces, without a division for each
+  const int over = (int)(r.cost % pieces);
+  int64_t at = 0;
+  for (int j = 1, rest = 0; j < pieces; ++j) {
+    at += length;
+    rest += over;
+    if (rest >= pieces) {
+      rest -= pieces;
+      ++at;
+    }
+    while (at >= first + k) {
+      first += k;
+      cut = false;
+      if (++tile < problem_end) continue;
+      do problem_end = problem_end_tile(s, ++p); while (tile >= problem_end);
+      k = tile_cost(s, p);
+    }
+    if (at > first) {
+      slots += cut ? 1 : 2;
+      cut = true;
+    }
+  }
+  return slots;
+}
+
+// Every tile of XCD s's range contracts over the same number of steps.
+inline bool range_has_one_k(const Sched& s) {
+  const int last = problem_of_tile(s, s.range_end - 1);
+  const int64_t k = tile_cost(s, last);
+  for (int p = problem_of_tile(s, s.range_begin); p < last; ++p)
+    if (problem_end_tile(s, p) > s.probs[p].tile_begin && tile_cost(s, p) != k) return false;
+  return true;
+}
+
+// The ways to share a remainder, and how long each takes but for the partial sums.  Pieces that end where tiles end (so many
+// per tile) leave one slot each if all tiles have one K; the most pieces that may be cut end anywhere.  Under one K the
+// workgroups come to the remainder together; otherwise one that its whole tiles keep longer than the others begins later, and
+// whether it gets a tile, a piece or nothing of the remainder decides when the range is through.  Measured on the weight
+// gradients of drawn layers, against the mean remainder tile as the time of whole tiles, one slot a piece throughout and all
+// XCDs that might share as sharing: 196 launches planned otherwise take 4.4 % less time in the mean (6 experts of 2464 x 576,
+// 48592 rows 226 -> 130 us; 75 gain more than 3 %, 31 lose as much, 22 % at most).  With the slots and the XCDs counted but
+// the mean tile kept, 105 launches took 1.4 % more.
+inline void sk_splits(const Sched& s, SkRemainder& r) {
+  const int W = s.wgs, full = (s.range_end - s.range_begin) / W;
+  const bool one_k = range_has_one_k(s);
+  int64_t most = W;
+  if (most > r.cost / kSkMinPairs) most = r.cost / kSkMinPairs;
+  if (most > (int64_t)r.tiles * kSkMaxPieces) most = (int64_t)r.tiles * kSkMaxPieces;
+  for (int per_tile = 2; r.n_splits < kSkMaxPieces; ++per_tile) {
+    const bool per_tile_fits = (int64_t)per_tile * r.tiles <= most;
+    const int pieces = per_tile_fits ? per_tile * r.tiles : (int)most;
+    if (pieces <= r.tiles) break;   // at most one piece per tile: nothing to gain
+    r.split[r.n_splits++] = SkSplit{pieces, one_k && pieces % r.tiles == 0 ? pieces : sk_slots(s, r, pieces)};
+    if (!per_tile_fits) break;
+  }
+  if (r.n_splits == 0) return;
+  if (one_k) {
+    r.whole_x100 = r.cost * 100 / r.tiles;
+    for (int i = 0; i < r.n_splits; ++i) r.shared_x100[i] = r.cost * 100 / r.split[i].pieces;
+    return;
+  }
+  // steps of each workgroup's whole tiles (without a full round, of those that a remainder tile goes to: none yet)
+  const int workgroups = full > 0 ? W : r.tiles;
+  std::vector<int64_t> load(workgroups, 0);
+  int tile = s.range_begin, p = problem_of_tile(s, tile);
+  r.whole_x100 = 0;
+  for (int round = 0; round <= full; ++round) {
+    int j = (int)((int64_t)kRoundRotation * round % W);   // position 0 of the round is workgroup -j's
+    j = j == 0 ? 0 : W - j;
+    for (int at = 0; at < W && tile < s.range_end; ++at, ++tile) {
+      while (tile >= problem_end_tile(s, p)) ++p;
+      const int64_t through = load[j] + tile_cost(s, p) + kTileOverhead;
+      if (round < full) load[j] = through;
+      else r.whole_x100 = r.whole_x100 < through * 100 ? through * 100 : r.whole_x100;
+      if (++j == W) j = 0;
+    }
+  }
+  int64_t longest = 0;
+  for (int j = 0; j < workgroups; ++j) longest = longest < load[j] ? load[j] : longest;
+  if (r.whole_x100 < longest * 100) r.whole_x100 = longest * 100;
+  int64_t first = 0;   // the longest of the workgroups that get a piece
+  for (int i = 0, j = 0; i < r.n_splits; ++i) {
+    for (; j < r.split[i].pieces && j < workgroups; ++j) first = first < load[j] ? load[j] : first;
+    const int64_t through_x100 = (first + kTileOverhead) * 100 + r.cost * 100 / r.split[i].pieces;
+    r.shared_x100[i] = through_x100 < longest * 100 ? longest * 100 : through_x100;
+  }
+}
+
+// The pieces that take the least time while `sharing` XCDs share (0: whole tiles do).  Every slot is written and read again.
+inline int sk_pieces(const Sched& s, const SkRemainder& r, int sharing) {
+  if (r.n_splits == 0) return 0;
+  int64_t best_x100 = r.whole_x100;
+  int pieces = 0;
+  for (int i = 0; i < r.n_splits; ++i) {
+    const int64_t price_x100 = (int64_t)r.split[i].slots * kSkPerSlot + (s.gelu ? (int64_t)r.tiles * kSkGeluPerTile : 0);
+    const int64_t takes_x100 = r.shared_x100[i] + kSkFixupLaunch * 100 + price_x100 * sharing / kNumXcd;
+    if (takes_x100 < best_x100) {
+      best_x100 = takes_x100;
+      pieces = r.split[i].pieces;
+    }
+  }
+  return pieces;
+}
+
 // Workgroup i runs on XCD i % 8.  The tile list is cut into 8 contiguous ranges of equal WORK, one per XCD,
 // so that workgroups that share an L2 work on neighbouring tiles; the workgroups of an XCD stride through the
 // range, and share its remainder along K when that pays.  k differs per problem in the wgrad form, and a
 // tile costs its K steps plus a fixed part (epilogue, tile switch) worth about kTileOverhead steps: balancing
 // K steps alone left the XCDs that hold the short-K problems 17 % more work than the others.
-FP8GMM_HD void sched_init(Sched& s, const fp8gmm_gemm_problem* probs, int nprob, int total_tiles,
-                                           int xcd, int wgs_per_xcd, bool sk_enable, bool gelu = false) {
-  s.gelu = gelu;
-  s.probs = probs;
-  s.nprob = nprob;
-  s.total_tiles = total_tiles;
-  s.wgs = wgs_per_xcd;
-  s.total_cost = 0;
-  s.total_cost = cost_before(s, total_tiles);
-  s.range_begin = range_start(s, xcd);
-  s.range_end = range_start(s, xcd + 1);
-  const int n_x = s.range_end - s.range_begin;
+inline void sched_init(Sched (&all)[kNumXcd], const fp8gmm_gemm_problem* probs, int nprob, int total_tiles, int wgs_per_xcd,
+                       bool sk_enable, bool gelu = false) {
   const int W = wgs_per_xcd;
-  s.dp_rounds = (n_x + W - 1) / W;  // plain striding: the last round may be partial
-  s.sk_begin = s.range_end;
-  s.sk_wgs = 0;
-  s.sk_c0 = 0;
-  s.sk_cost = 0;
-  if (!sk_enable || !remainder_may_share(n_x, W)) return;
-  const int rounds = n_x / W, n_sk = n_x % W;
-  const int sk_begin = s.range_begin + rounds * W;
-  const int64_t c0 = cost_before(s, sk_begin);
-  const int64_t cost = cost_before(s, s.range_end) - c0;
+  SkRemainder rem[kNumXcd];
   int sharing = 0;   // XCDs whose partial sums travel at the same time
-  for (int x = 0, begin = 0; x < kNumXcd; ++x) {
-    const int end = range_start(s, x + 1);
-    sharing += remainder_may_share(end - begin, W) ? 1 : 0;
-    begin = end;
+  for (int x = 0; x < kNumXcd; ++x) {
+    Sched& s = all[x];
+    s.gelu = gelu;
+    s.probs = probs;
+    s.nprob = nprob;
+    s.total_tiles = total_tiles;
+    s.wgs = W;
+    s.total_cost = x > 0 ? all[0].total_cost : 0;
+    if (x == 0) s.total_cost = cost_before(s, total_tiles);
+    s.range_begin = x > 0 ? all[x - 1].range_end : 0;
+    s.range_end = range_start(s, x + 1);
+    const int n_x = s.range_end - s.range_begin;
+    s.dp_rounds = (n_x + W - 1) / W;  // plain striding: the last round may be partial
+    s.sk_begin = s.range_end;
+    s.sk_wgs = 0;
+    s.sk_c0 = 0;
+    s.sk_cost = 0;
+    SkRemainder& r = rem[x];
+    r.n_splits = 0;
+    if (!sk_enable || !remainder_may_share(n_x, W)) continue;
+    r.tiles = n_x % W;
+    r.begin = s.range_end - r.tiles;
+    r.c0 = cost_before(s, r.begin);
+    r.cost = cost_before(s, s.range_end) - r.c0;
+    sk_splits(s, r);
+    sharing += r.n_splits > 0 ? 1 : 0;
   }
-  // The last round shrinks from a tile's duration to a piece's; every piece is a slot to write and to read again.  Pieces
-  // that end where tiles end (so many per tile) leave one slot each; W pieces over n tiles cut up to n - 1 of them in two.
-  int64_t most = W;
-  if (most > cost / kSkMinPairs) most = cost / kSkMinPairs;
-  if (most > (int64_t)n_sk * kSkMaxPieces) most = (int64_t)n_sk * kSkMaxPieces;
-  int64_t best_x100 = cost * 100 / n_sk, w = 0;   // what not sharing takes
-  for (int per_tile = 2;; ++per_tile) {
-    const bool aligned = (int64_t)per_tile * n_sk <= most;
-    const int64_t pieces = aligned ? (int64_t)per_tile * n_sk : most;
-    if (pieces <= n_sk) break;   // at most one piece per tile: nothing to gain
-    const int64_t slots = pieces % n_sk == 0 ? pieces : pieces + n_sk - 1;
-    const int64_t takes_x100 = cost * 100 / pieces + kSkFixupLaunch * 100 + slots * 100 * sharing / kNumXcd +
-                               (s.gelu ? (int64_t)n_sk * kSkGeluPerTile * sharing / kNumXcd : 0);
-    if (takes_x100 < best_x100) {
-      best_x100 = takes_x100;
-      w = pieces;
+  if (sharing == 0) return;
+  int pieces[kNumXcd];
+  auto decide = [&](int at_once) {
+    int count = 0;
+    for (int x = 0; x < kNumXcd; ++x) {
+      pieces[x] = sk_pieces(all[x], rem[x], at_once);
+      count += pieces[x] > 0 ? 1 : 0;
     }
-    if (!aligned) break;
+    return count;
+  };
+  // Where fewer share than might, the price of those that do is lower, and with it more may share: the smallest number
+  // from there on that no more than that many share at.
+  int count = decide(sharing);
+  if (count > 0 && count < sharing)
+    for (sharing = count; (count = decide(sharing)) > sharing; ++sharing) {
+    }
+  for (int x = 0; x < kNumXcd; ++x) {
+    if (pieces[x] == 0) continue;
+    Sched& s = all[x];
+    s.dp_rounds = (s.range_end - s.range_begin) / W;
+    s.sk_begin = rem[x].begin;
+    s.sk_wgs = pieces[x];
+    s.sk_c0 = rem[x].c0;
+    s.sk_cost = rem[x].cost;
   }
-  if (w == 0) return;
-  s.dp_rounds = rounds;
-  s.sk_begin = sk_begin;
-  s.sk_wgs = (int)w;
-  s.sk_c0 = c0;
-  s.sk_cost = cost;
 }
 
 // piece boundaries of the stream-K region, relative to sk_c0
@@ -202,16 +344,6 @@ struct Cursor {
   int dp_i;     // strided tiles already taken
   int sk_tile;  // next tile of this workgroup's stream-K piece, -1: none left
 };
-
-// The tile that workgroup j of the XCD takes in round i of the strided part.  The position inside the round
-// rotates from round to round: how fast a workgroup's steps run depends on where its tile sits in the round's
-// 8 x 4 block (which operand slabs it shares with its neighbours, which memory channels those fall into - up to
-// 6 % between columns of a weight-gradient problem), and a workgroup that kept one position for the whole launch
-// would finish that much earlier or later than the others.
-constexpr int kRoundRotation = 5;  // coprime to every workgroup count in use (multiples of 8 per XCD: 32, 38, ...)
-FP8GMM_HD int dp_tile(const Sched& s, int j, int i) {
-  return s.range_begin + s.wgs * i + (j + kRoundRotation * i) % s.wgs;
-}
 
 FP8GMM_HD void cursor_init(const Sched& s, int j, Cursor& c) {
   c.dp_i = 0;

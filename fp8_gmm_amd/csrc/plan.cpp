@@ -92,8 +92,9 @@ int fp8gmm_gemm_schedule(const fp8gmm_gemm_problem* probs, int n, int total_tile
   if ((n > 0 && probs == nullptr) || (max_items > 0 && items == nullptr)) return FP8GMM_ERR_NULL_POINTER;
   if (n == 0 || total_tiles == 0) return 0;
   const int xcd = wg % kNumXcd, j = wg / kNumXcd;
-  Sched s;
-  sched_init(s, probs, n, total_tiles, xcd, grid / kNumXcd, stream_k != 0);
+  Sched all[kNumXcd];
+  sched_init(all, probs, n, total_tiles, grid / kNumXcd, stream_k != 0);
+  const Sched& s = all[xcd];
   Cursor c;
   cursor_init(s, j, c);
   int count = 0;
@@ -119,8 +120,9 @@ int fp8gmm_gemm_fixup(const fp8gmm_gemm_problem* probs, int n, int total_tiles, 
   *tile = -1;
   if (n == 0 || total_tiles == 0) return 0;
   const int xcd = wg % kNumXcd, j = wg / kNumXcd + 1, wgs = grid / kNumXcd;
-  Sched s;
-  sched_init(s, probs, n, total_tiles, xcd, wgs, true);
+  Sched all[kNumXcd];
+  sched_init(all, probs, n, total_tiles, wgs, true);
+  const Sched& s = all[xcd];
   int n_following = 0;
   const int t = fixup_tile(s, j, &n_following);
   if (t < 0) return 0;
@@ -335,8 +337,8 @@ int fp8gmm_plan_grouped_gemm_launch(fp8gmm_gemm_problem* probs, int n, int layou
 
   // pass 1: sizes.  The tiles that were shared along K first: the pieces of such a tile get consecutive
   // workspace slots, numbered from 0 over the launch, in K order.
-  std::vector<Sched> sched(kNumXcd);
-  for (int x = 0; x < kNumXcd; ++x) sched_init(sched[x], probs, n, total_tiles, x, wgs, sk, gelu);
+  Sched sched[kNumXcd];
+  sched_init(sched, probs, n, total_tiles, wgs, sk, gelu);
   std::vector<int32_t> slot_map((size_t)kSlotsPerWg * grid, -1);
   std::vector<fp8gmm_gemm_fixup_desc> fix;
   int n_slots = 0;
@@ -514,9 +516,10 @@ int plan_gemm_ranges(fp8gmm_gemm_problem* probs, int n, int layout, int grid, in
     const bool sk = share_tail(stream_k, total_tiles, &grid);
     const int wgs = grid / kNumXcd;
     plan->grid = grid;
+    Sched sched[kNumXcd];
+    sched_init(sched, probs, n, total_tiles, wgs, sk, gelu);
     for (int x = 0; x < kNumXcd; ++x) {
-      Sched s;
-      sched_init(s, probs, n, total_tiles, x, wgs, sk, gelu);
+      const Sched& s = sched[x];
       GemmRanges::Xcd& o = out->xcd[x];
       o.begin = s.range_begin;
       o.end = s.range_end;

@@ -226,6 +226,84 @@ def test_pieces_end_where_tiles_end_unless_whole_tiles_are_faster():
         assert fixups["n_pieces"].min() == fixups["n_pieces"].max()
 
 
+# The rule for sharing, with everything counted from its definition: K = 128 steps of time, in hundredths.
+LAUNCH, PER_SLOT, GELU_PER_TILE = 400, 100, 150
+
+
+def shared_pieces(costs, wgs, gelu):
+    """costs: K steps of the tiles, in order.  Slots and shared tiles of a launch, if an XCD takes the number of pieces with
+    which its last workgroup is through first, at the price of the XCDs that share."""
+    n = len(costs)
+    before = np.concatenate([[0], np.cumsum(costs)])
+    work = before + 4 * np.arange(n + 1)
+    cut = [int(np.searchsorted(work, -(-int(work[-1]) * x // 8))) for x in range(9)]
+    options = []   # per XCD: (time with whole tiles, [(time but for the slots, slots, tiles cut, tiles)])
+    for x in range(8):
+        own = costs[cut[x]: cut[x + 1]]
+        full, rem = divmod(len(own), wgs)
+        if rem == 0 or full > 24 or (wgs - rem) * 12 < wgs * (full + 1):
+            continue
+        ends = np.concatenate([[0], np.cumsum(own[full * wgs:])])
+        cost, most, ways = int(ends[-1]), min(wgs, int(ends[-1]) // 4, 8 * rem), []
+        load = np.zeros(wgs, dtype=int)
+        for i in range(full):   # workgroup j's place in round i is j + 5 i
+            load += own[i * wgs + (np.arange(wgs) + 5 * i) % wgs] + 4
+        last = {j: int(own[full * wgs + p]) for j in range(wgs) for p in [(j + 5 * full) % wgs] if p < rem}
+        whole = max([int(load.max())] + [int(load[j]) + c + 4 for j, c in last.items()]) * 100
+        if len(set(own.tolist())) == 1:
+            whole = cost * 100 // rem
+        for pieces in sorted({p * rem for p in range(2, 9) if p * rem <= most} | ({most} if most > rem else set())):
+            inside = [t for j in range(1, pieces) for t in [int(np.searchsorted(ends, cost * j // pieces, "right")) - 1]
+                      if ends[t] != cost * j // pieces]
+            through = cost * 100 // pieces
+            if len(set(own.tolist())) > 1:
+                through = max(int(load.max()) * 100, (int(load[:pieces].max()) + 4) * 100 + through)
+            ways.append((through, len(inside) + len(set(inside)), len(set(inside)), rem, pieces))
+        if ways:
+            options.append((whole, ways))
+
+    def decide(sharing):
+        chosen = []
+        for whole, ways in options:
+            takes = [t + LAUNCH + (slots * PER_SLOT + (rem * GELU_PER_TILE if gelu else 0)) * sharing // 8
+                     for t, slots, _, rem, _ in ways]
+            if min(takes) < whole:
+                chosen.append(ways[takes.index(min(takes))])
+        return chosen
+
+    sharing = len(options)
+    chosen = decide(sharing)
+    if chosen and len(chosen) < sharing:
+        sharing = len(chosen)
+        chosen = decide(sharing)
+        while len(chosen) > sharing:
+            sharing += 1
+            chosen = decide(sharing)
+    return sum(c[1] for c in chosen), sum(c[2] for c in chosen)
+
+
+def test_sharing_is_priced_by_the_slots_and_the_xcds_that_there_are():
+    """Contractions of several lengths: equal pieces then end inside tiles, some ranges share while others that might do
+    not, and the workgroups come to the remainder one after the other."""
+    rng = np.random.default_rng(11)
+    seen = {"mixed": 0, "some": 0}
+    for case in range(300):
+        e = int(rng.choice([2, 4, 8, 16, 64]))
+        tiles = int(rng.integers(1, 2 + 1200 // e))
+        k = rng.multinomial(int(rng.choice([4000, 12000, 40000])), rng.dirichlet(np.full(e, float(rng.choice([0.5, 1, 20])))))
+        gelu = bool(case % 3 == 0)
+        table, total = make_table([(256 * tiles, 256, 16 * int((v + 15) // 16)) for v in k])
+        plan, items, fixups = _lib.plan_grouped_gemm_launch(table, _lib.EPI_GELU if gelu else 0, 256, True)
+        costs = np.repeat([max(1, -(-int(v) // 128)) for v in k], tiles)
+        assert (plan.n_slots, len(fixups)) == shared_pieces(costs, 32, gelu), (case, e, tiles, k.tolist())
+        if len(fixups):
+            recs = items[items["prob"] >= 0]
+            shared = recs[recs["slot"] >= 0]
+            seen["mixed"] += len(set(shared["prob"].tolist())) > 1
+            seen["some"] += len({int(w) % 8 for w in np.flatnonzero(items["slot"].reshape(-1) * (items["prob"] >= 0) > 0)}) < 8
+    assert seen["mixed"] > 30 and seen["some"] > 30, seen
+
+
 @pytest.mark.parametrize("shapes", [
     [(1, 1, 16)],
     [(256, 256, 128)],
