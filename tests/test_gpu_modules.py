@@ -423,11 +423,15 @@ def test_weights_cast_ahead_of_the_pass_give_the_same_bits(dev, kind):
 
 @pytest.mark.parametrize("shape", [(1, 16, 16), (5, 48, 272), (3, 256, 2064)])
 @pytest.mark.parametrize("kind", ["linear", "mlp"])
-def test_weights_cast_ahead_from_native_code_equal_the_per_launch_path(dev, kind, shape):
+def test_weights_cast_ahead_from_native_code_equal_the_per_launch_path(dev, kind, shape, monkeypatch):
     """The native call is a pass without rows; ``planned_passes=False`` runs the update and the cast one by one.  The same
     fp8 weights, maxima and scales, with an update due (second and third turn) and without (first, and in evaluation)."""
+    from fp8_gmm_amd import native
+
     pkg = _pkg()
     e, h, f = shape
+    calls, cast_weights = [], native.cast_weights
+    monkeypatch.setattr(native, "cast_weights", lambda *a: (calls.append(len(a[0])), cast_weights(*a))[1])
     cls = pkg.GroupedMlp if kind == "mlp" else pkg.GroupedLinear
     mods = [cls(h, f, e, torch.bfloat16, device=dev, planned_passes=p) for p in (True, False)]
     mods[1].load_state_dict(mods[0].state_dict())
@@ -437,6 +441,7 @@ def test_weights_cast_ahead_from_native_code_equal_the_per_launch_path(dev, kind
             mod.train(turn < 3)
             with pkg.fp8_autocast(fp8_recipe=fp8_recipe):
                 assert mod.cast_weights_ahead()
+        assert calls == [2 if kind == "mlp" else 1] * (turn + 1)   # the first module's call, and no other
         for a, b in zip(mods[0]._ahead, mods[1]._ahead):
             assert a.valid and b.valid and torch.equal(a.fp8.view(torch.uint8), b.fp8.view(torch.uint8)), turn
         for name in ("scaling_fwd", "scaling_bwd"):
@@ -446,6 +451,37 @@ def test_weights_cast_ahead_from_native_code_equal_the_per_launch_path(dev, kind
             for pa, pb in zip(mods[0].parameters(), mods[1].parameters()):
                 pa.mul_(1.5)
                 pb.copy_(pa)
+
+
+@pytest.mark.parametrize("kind", ["linear", "mlp"])
+def test_a_refused_cast_ahead_leaves_the_scaling_state_updated_once(dev, kind, monkeypatch):
+    """The native call refuses (before it launches anything) while an update is due: the error is passed on, the update has
+    run, once, and nothing is kept for the pass."""
+    from fp8_gmm_amd import native
+
+    pkg = _pkg()
+    cls = pkg.GroupedMlp if kind == "mlp" else pkg.GroupedLinear
+    mods = [cls(48, 80, 3, torch.bfloat16, device=dev) for _ in range(2)]
+    mods[1].load_state_dict(mods[0].state_dict())
+    fp8_recipe = pkg.DelayedScaling(amax_history_len=4)
+    with pkg.fp8_autocast(fp8_recipe=fp8_recipe):
+        for mod in mods:
+            assert mod.cast_weights_ahead()
+        assert mods[0].cast_weights_ahead()   # the update, and the weights' maxima in the new row
+
+        def refuse(*args):
+            raise RuntimeError("refused")
+
+        monkeypatch.setattr(native, "cast_weights", refuse)
+        with pytest.raises(RuntimeError, match="refused"):
+            mods[1].cast_weights_ahead()
+    assert mods[1]._ahead is None
+    for name in ("scaling_fwd", "scaling_bwd"):
+        want, got = (m.fp8_meta[name] for m in mods)
+        assert torch.equal(want.scale, got.scale) and torch.equal(want.scale_inv, got.scale_inv), name
+        assert torch.equal(want.amax_history[1:], got.amax_history[1:]), name
+        assert not got.amax_history[0].any(), name
+    assert mods[0].fp8_meta["scaling_fwd"].amax_history[0].any()
 
 
 def test_cutlass_passes_equal_the_per_launch_path(dev):
