@@ -133,14 +133,13 @@ FP8GMM_HD int dp_tile(const Sched& s, int j, int i) {
 struct SkSplit {
   int pieces, slots;
 };
-// The remainder of an XCD's range and the ways to share it.
+// The remainder of an XCD's range, the ways to share it, and when the range's last workgroup is through, from the launch's
+// start and in hundredths of a K = 128 step: with whole tiles, and with each split but for its partial sums.
 struct SkRemainder {
   int begin, tiles;      // first tile, how many
   int64_t c0, cost;      // cost before it, its own
   int n_splits;          // 0: not worth a thought
   SkSplit split[kSkMaxPieces];
-  // when the last workgroup is through, in hundredths of a K = 128 step: the remainder as whole tiles, and each split (under
-  // one K from when they come to it, otherwise from the launch's start)
   int64_t whole_x100, shared_x100[kSkMaxPieces];
 };
 
@@ -183,18 +182,11 @@ inline bool range_has_one_k(const Sched& s) {
   return true;
 }
 
-// The ways to share a remainder, and how long each takes but for the partial sums.  Pieces that end where tiles end (so many
-// per tile) leave one slot each if all tiles have one K; the most pieces that may be cut end anywhere.  Under one K the
-// workgroups come to the remainder together; otherwise one that its whole tiles keep longer than the others begins later, and
-// whether it gets a tile, a piece or nothing of the remainder decides when the range is through.  Measured on the weight
-// gradients of drawn layers, against the mean remainder tile as the time of whole tiles, one slot a piece throughout and all
-// XCDs that might share as sharing: 196 launches planned otherwise take 4.4 % less time in the mean (6 experts of 2464 x 576,
-// 48592 rows 226 -> 130 us; 75 gain more than 3 %, 31 lose as much, 22 % at most).  With the slots and the XCDs counted but
-// the mean tile kept, 105 launches took 1.4 % more.
+// Pieces that end where tiles end (so many per tile) leave one slot each if all tiles have one K; the most pieces that may be
+// cut end anywhere.
 inline void sk_splits(const Sched& s, SkRemainder& r) {
-  const int W = s.wgs, full = (s.range_end - s.range_begin) / W;
   const bool one_k = range_has_one_k(s);
-  int64_t most = W;
+  int64_t most = s.wgs;
   if (most > r.cost / kSkMinPairs) most = r.cost / kSkMinPairs;
   if (most > (int64_t)r.tiles * kSkMaxPieces) most = (int64_t)r.tiles * kSkMaxPieces;
   for (int per_tile = 2; r.n_splits < kSkMaxPieces; ++per_tile) {
@@ -204,31 +196,43 @@ inline void sk_splits(const Sched& s, SkRemainder& r) {
     r.split[r.n_splits++] = SkSplit{pieces, one_k && pieces % r.tiles == 0 ? pieces : sk_slots(s, r, pieces)};
     if (!per_tile_fits) break;
   }
-  if (r.n_splits == 0) return;
-  if (one_k) {
-    r.whole_x100 = r.cost * 100 / r.tiles;
-    for (int i = 0; i < r.n_splits; ++i) r.shared_x100[i] = r.cost * 100 / r.split[i].pieces;
+}
+
+// Under one K the workgroups come to the remainder together; otherwise one that its whole tiles keep longer than the others
+// begins later, and whether it gets a tile, a piece or nothing of the remainder decides when the range is through.
+inline void sk_times(const Sched& s, SkRemainder& r) {
+  const int W = s.wgs, full = (s.range_end - s.range_begin) / W;
+  if (range_has_one_k(s)) {
+    const int64_t round = tile_cost(s, problem_of_tile(s, s.range_begin)) + kTileOverhead;
+    r.whole_x100 = (full + (r.tiles > 0 ? 1 : 0)) * round * 100;
+    for (int i = 0; i < r.n_splits; ++i)
+      r.shared_x100[i] = (full * round + kTileOverhead) * 100 + r.cost * 100 / r.split[i].pieces;
     return;
   }
   // steps of each workgroup's whole tiles (without a full round, of those that a remainder tile goes to: none yet)
   const int workgroups = full > 0 ? W : r.tiles;
   std::vector<int64_t> load(workgroups, 0);
   int tile = s.range_begin, p = problem_of_tile(s, tile);
-  r.whole_x100 = 0;
+  int64_t steps = tile_cost(s, p) + kTileOverhead, last = 0;
   for (int round = 0; round <= full; ++round) {
     int j = (int)((int64_t)kRoundRotation * round % W);   // position 0 of the round is workgroup -j's
     j = j == 0 ? 0 : W - j;
-    for (int at = 0; at < W && tile < s.range_end; ++at, ++tile) {
-      while (tile >= problem_end_tile(s, p)) ++p;
-      const int64_t through = load[j] + tile_cost(s, p) + kTileOverhead;
-      if (round < full) load[j] = through;
-      else r.whole_x100 = r.whole_x100 < through * 100 ? through * 100 : r.whole_x100;
-      if (++j == W) j = 0;
+    const int end = tile + W < s.range_end ? tile + W : s.range_end;
+    while (tile < end) {
+      while (tile >= problem_end_tile(s, p)) steps = tile_cost(s, ++p) + kTileOverhead;
+      int n = problem_end_tile(s, p) < end ? problem_end_tile(s, p) - tile : end - tile;   // tiles of one K side by side
+      if (n > W - j) n = W - j;
+      for (int i = 0; i < n; ++i) {
+        if (round < full) load[j + i] += steps;
+        else if (last < load[j + i] + steps) last = load[j + i] + steps;
+      }
+      tile += n;
+      j = j + n == W ? 0 : j + n;
     }
   }
   int64_t longest = 0;
-  for (int j = 0; j < workgroups; ++j) longest = longest < load[j] ? load[j] : longest;
-  if (r.whole_x100 < longest * 100) r.whole_x100 = longest * 100;
+  for (const int64_t l : load) longest = longest < l ? l : longest;
+  r.whole_x100 = (longest < last ? last : longest) * 100;
   int64_t first = 0;   // the longest of the workgroups that get a piece
   for (int i = 0, j = 0; i < r.n_splits; ++i) {
     for (; j < r.split[i].pieces && j < workgroups; ++j) first = first < load[j] ? load[j] : first;
@@ -237,20 +241,66 @@ inline void sk_splits(const Sched& s, SkRemainder& r) {
   }
 }
 
-// The pieces that take the least time while `sharing` XCDs share (0: whole tiles do).  Every slot is written and read again.
-inline int sk_pieces(const Sched& s, const SkRemainder& r, int sharing) {
-  if (r.n_splits == 0) return 0;
-  int64_t best_x100 = r.whole_x100;
+// The pieces with which a range is through first while `sharing` XCDs share (0: whole tiles), and when.  Every slot is written
+// and read again.
+inline int sk_pieces(const Sched& s, const SkRemainder& r, int sharing, int64_t* through_x100) {
   int pieces = 0;
+  *through_x100 = r.whole_x100;
   for (int i = 0; i < r.n_splits; ++i) {
     const int64_t price_x100 = (int64_t)r.split[i].slots * kSkPerSlot + (s.gelu ? (int64_t)r.tiles * kSkGeluPerTile : 0);
     const int64_t takes_x100 = r.shared_x100[i] + kSkFixupLaunch * 100 + price_x100 * sharing / kNumXcd;
-    if (takes_x100 < best_x100) {
-      best_x100 = takes_x100;
+    if (takes_x100 < *through_x100) {
+      *through_x100 = takes_x100;
       pieces = r.split[i].pieces;
     }
   }
   return pieces;
+}
+
+// Which remainders of a launch are shared, and in how many pieces each.  A range shares where that is faster for it, at the
+// price of the XCDs that share; the launch does if its last range is through sooner for it, the second launch included, which
+// also those wait for that do not share; and a range that with whole tiles is through before that keeps them.  Measured on the
+// launches of drawn layers that are planned otherwise, against ranges that decide for themselves by the mean remainder tile,
+// one slot a piece and all XCDs that might share: 269 take 6.7 % less time in the mean, 167 gain more than 3 %, 14 lose as much
+// (a weight gradient of 7 x 3088 x 416, 37005 rows 154 -> 102 us, of 11 x 1552 x 1632, 51592 272 -> 211; GELU launches of about a
+// round 38.7 -> 29.9 and 44.1 -> 34.6).  By the workgroups' times but each range for itself 3.2 %; with the slots and the XCDs
+// counted but by the mean tile 105 launches took 1.4 % more.
+inline void sk_decide(const Sched (&all)[kNumXcd], SkRemainder (&rem)[kNumXcd], int (&pieces)[kNumXcd]) {
+  int sharing = 0;
+  int64_t through[kNumXcd];
+  for (int x = 0; x < kNumXcd; ++x) {
+    pieces[x] = 0;
+    if (rem[x].n_splits == 0) continue;
+    ++sharing;
+    sk_times(all[x], rem[x]);
+  }
+  if (sharing == 0) return;
+  auto decide = [&](int at_once) {
+    int count = 0;
+    for (int x = 0; x < kNumXcd; ++x) {
+      if (rem[x].n_splits == 0) continue;
+      pieces[x] = sk_pieces(all[x], rem[x], at_once, &through[x]);
+      count += pieces[x] > 0 ? 1 : 0;
+    }
+    return count;
+  };
+  // Where fewer share than might, the price of those that do is lower, and with it more may share: the smallest number
+  // from there on that no more than that many share at.
+  int count = decide(sharing);
+  if (count == 0) return;
+  if (count < sharing)
+    for (sharing = count; (count = decide(sharing)) > sharing; ++sharing) {
+    }
+  int64_t whole = 0, last = 0;
+  for (int x = 0; x < kNumXcd; ++x) {
+    if (all[x].range_begin == all[x].range_end) continue;
+    if (rem[x].n_splits == 0) sk_times(all[x], rem[x]);
+    const int64_t own = pieces[x] > 0 ? through[x] : rem[x].whole_x100 + kSkFixupLaunch * 100;
+    whole = whole < rem[x].whole_x100 ? rem[x].whole_x100 : whole;
+    last = last < own ? own : last;
+  }
+  for (int x = 0; x < kNumXcd; ++x)
+    if (last >= whole || rem[x].whole_x100 + kSkFixupLaunch * 100 <= last) pieces[x] = 0;
 }
 
 // Workgroup i runs on XCD i % 8.  The tile list is cut into 8 contiguous ranges of equal WORK, one per XCD,
@@ -262,7 +312,6 @@ inline void sched_init(Sched (&all)[kNumXcd], const fp8gmm_gemm_problem* probs, 
                        bool sk_enable, bool gelu = false) {
   const int W = wgs_per_xcd;
   SkRemainder rem[kNumXcd];
-  int sharing = 0;   // XCDs whose partial sums travel at the same time
   for (int x = 0; x < kNumXcd; ++x) {
     Sched& s = all[x];
     s.gelu = gelu;
@@ -282,30 +331,17 @@ inline void sched_init(Sched (&all)[kNumXcd], const fp8gmm_gemm_problem* probs, 
     s.sk_cost = 0;
     SkRemainder& r = rem[x];
     r.n_splits = 0;
-    if (!sk_enable || !remainder_may_share(n_x, W)) continue;
+    r.whole_x100 = 0;
     r.tiles = n_x % W;
     r.begin = s.range_end - r.tiles;
+    if (!sk_enable || !remainder_may_share(n_x, W)) continue;
     r.c0 = cost_before(s, r.begin);
     r.cost = cost_before(s, s.range_end) - r.c0;
     sk_splits(s, r);
-    sharing += r.n_splits > 0 ? 1 : 0;
   }
-  if (sharing == 0) return;
+  if (!sk_enable) return;
   int pieces[kNumXcd];
-  auto decide = [&](int at_once) {
-    int count = 0;
-    for (int x = 0; x < kNumXcd; ++x) {
-      pieces[x] = sk_pieces(all[x], rem[x], at_once);
-      count += pieces[x] > 0 ? 1 : 0;
-    }
-    return count;
-  };
-  // Where fewer share than might, the price of those that do is lower, and with it more may share: the smallest number
-  // from there on that no more than that many share at.
-  int count = decide(sharing);
-  if (count > 0 && count < sharing)
-    for (sharing = count; (count = decide(sharing)) > sharing; ++sharing) {
-    }
+  sk_decide(all, rem, pieces);
   for (int x = 0; x < kNumXcd; ++x) {
     if (pieces[x] == 0) continue;
     Sched& s = all[x];

@@ -232,54 +232,57 @@ LAUNCH, PER_SLOT, GELU_PER_TILE = 400, 100, 150
 
 def shared_pieces(costs, wgs, gelu):
     """costs: K steps of the tiles, in order.  Slots and shared tiles of a launch, if an XCD takes the number of pieces with
-    which its last workgroup is through first, at the price of the XCDs that share."""
+    which its last workgroup is through first, at the price of the XCDs that share, and the launch shares where its last XCD
+    is through sooner for it."""
     n = len(costs)
     before = np.concatenate([[0], np.cumsum(costs)])
     work = before + 4 * np.arange(n + 1)
     cut = [int(np.searchsorted(work, -(-int(work[-1]) * x // 8))) for x in range(9)]
-    options = []   # per XCD: (time with whole tiles, [(time but for the slots, slots, tiles cut, tiles)])
+    ranges = []   # per XCD: (time with whole tiles, [(time but for the slots, slots, tiles cut, tiles)])
     for x in range(8):
         own = costs[cut[x]: cut[x + 1]]
-        full, rem = divmod(len(own), wgs)
-        if rem == 0 or full > 24 or (wgs - rem) * 12 < wgs * (full + 1):
+        if len(own) == 0:
             continue
-        ends = np.concatenate([[0], np.cumsum(own[full * wgs:])])
-        cost, most, ways = int(ends[-1]), min(wgs, int(ends[-1]) // 4, 8 * rem), []
+        full, rem = divmod(len(own), wgs)
         load = np.zeros(wgs, dtype=int)
         for i in range(full):   # workgroup j's place in round i is j + 5 i
             load += own[i * wgs + (np.arange(wgs) + 5 * i) % wgs] + 4
-        last = {j: int(own[full * wgs + p]) for j in range(wgs) for p in [(j + 5 * full) % wgs] if p < rem}
-        whole = max([int(load.max())] + [int(load[j]) + c + 4 for j, c in last.items()]) * 100
-        if len(set(own.tolist())) == 1:
-            whole = cost * 100 // rem
-        for pieces in sorted({p * rem for p in range(2, 9) if p * rem <= most} | ({most} if most > rem else set())):
-            inside = [t for j in range(1, pieces) for t in [int(np.searchsorted(ends, cost * j // pieces, "right")) - 1]
-                      if ends[t] != cost * j // pieces]
-            through = cost * 100 // pieces
-            if len(set(own.tolist())) > 1:
-                through = max(int(load.max()) * 100, (int(load[:pieces].max()) + 4) * 100 + through)
-            ways.append((through, len(inside) + len(set(inside)), len(set(inside)), rem, pieces))
-        if ways:
-            options.append((whole, ways))
+        last = [int(load[j] + own[full * wgs + p]) + 4 for j in range(wgs) for p in [(j + 5 * full) % wgs] if p < rem]
+        whole, ways = max([int(load.max())] + last) * 100, []
+        ends = np.concatenate([[0], np.cumsum(own[full * wgs:])])
+        cost, most = int(ends[-1]), min(wgs, int(ends[-1]) // 4, 8 * rem)
+        if rem and full <= 24 and (wgs - rem) * 12 >= wgs * (full + 1):
+            for pieces in sorted({p * rem for p in range(2, 9) if p * rem <= most} | ({most} if most > rem else set())):
+                inside = [t for j in range(1, pieces) for t in [int(np.searchsorted(ends, cost * j // pieces, "right")) - 1]
+                          if ends[t] != cost * j // pieces]
+                through = max(int(load.max()) * 100, (int(load[:pieces].max()) + 4) * 100 + cost * 100 // pieces)
+                ways.append((through, len(inside) + len(set(inside)), len(set(inside)), rem))
+        ranges.append((whole, ways))
 
     def decide(sharing):
-        chosen = []
-        for whole, ways in options:
+        chosen = []   # per range: (when it is through, slots, tiles), None for whole tiles
+        for whole, ways in ranges:
             takes = [t + LAUNCH + (slots * PER_SLOT + (rem * GELU_PER_TILE if gelu else 0)) * sharing // 8
-                     for t, slots, _, rem, _ in ways]
-            if min(takes) < whole:
-                chosen.append(ways[takes.index(min(takes))])
-        return chosen
+                     for t, slots, _, rem in ways]
+            best = takes.index(min(takes)) if takes else 0
+            chosen.append((takes[best],) + ways[best][1:3] if takes and takes[best] < whole else None)
+        return chosen, sum(c is not None for c in chosen)
 
-    sharing = len(options)
-    chosen = decide(sharing)
-    if chosen and len(chosen) < sharing:
-        sharing = len(chosen)
-        chosen = decide(sharing)
-        while len(chosen) > sharing:
+    sharing = sum(bool(ways) for _, ways in ranges)
+    chosen, count = decide(sharing)
+    if 0 < count < sharing:
+        sharing = count
+        chosen, count = decide(sharing)
+        while count > sharing:
             sharing += 1
-            chosen = decide(sharing)
-    return sum(c[1] for c in chosen), sum(c[2] for c in chosen)
+            chosen, count = decide(sharing)
+    if count == 0:
+        return 0, 0
+    last = max(c[0] if c else whole + LAUNCH for c, (whole, _) in zip(chosen, ranges))
+    if last >= max(whole for whole, _ in ranges):
+        return 0, 0
+    kept = [c for c, (whole, _) in zip(chosen, ranges) if c and whole + LAUNCH > last]
+    return sum(c[1] for c in kept), sum(c[2] for c in kept)
 
 
 def test_sharing_is_priced_by_the_slots_and_the_xcds_that_there_are():
