@@ -120,8 +120,8 @@ __device__ __forceinline__ void buf_store16(u32x4 v, __amdgpu_buffer_rsrc_t r, u
 // A store with the streaming hint.  The result of a GEMM's tile is written once and not read again by its launch: stored
 // this way it does not push the operand slabs that neighbouring workgroups are about to re-read out of the L2, and the
 // loads that follow the epilogue in the memory pipeline are not held up as long behind its stores (a dense 16384 x 14336
-// x 4096 launch: 1.14 -> 1.09 million cycles; without any stores it would be 1.06).  The transposed copy of a cast: see
-// pad_fusion.hip.
+// x 4096 launch: 1.14 -> 1.09 million cycles; without any stores it would be 1.06).  The transposed copy of a large cast:
+// pad_fusion.hip, kStreamTiles.
 __device__ __forceinline__ void buf_store16_stream(u32x4 v, __amdgpu_buffer_rsrc_t r, uint32_t off) {
   __builtin_amdgcn_raw_buffer_store_b128(v, r, (int)off, 0, 2);
 }

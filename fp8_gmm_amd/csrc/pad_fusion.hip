@@ -16,12 +16,8 @@
 //     to a 128 x 128-byte LDS tile (column-major, 8-byte granules XOR-swizzled by the
 //     column group so that the 64 lanes of a store hit distinct banks);
 //   * the tile is read back 16 bytes at a time and stored to the transposed output
-//     with 128-bit stores: 8 lanes cover 128 contiguous bytes of one output row.  They carry the streaming
-//     hint: the transposed copy waits for the backward pass, the row-major one is read by the next launch and
-//     should be what the memory-side cache keeps.  Measured with new buffers every time, cast / cast and the GEMM
-//     that reads its result, 8 tensors: 196 million elements (rows of 2880) 166 / 649 us plain, 158 / 600 with the
-//     hint, 153 / 642 with the hint on both copies; 114 million (rows of 4096) 97 / 443, 95 / 431, 93 / 444; 57
-//     million 250 with the GEMM, 241, 246.
+//     with 128-bit stores: 8 lanes cover 128 contiguous bytes of one output row.  In large launches of the casts they
+//     carry the streaming hint, see kStreamTiles;
 //   * amax: per-lane running max -> wave shuffle reduction -> one integer atomic max
 //     per workgroup.
 // HBM-bound: per element 2 B (bf16) or 1 B (fp8) read, 1 B + Mpad/m B written.
@@ -66,6 +62,21 @@ __device__ __forceinline__ int tile_of_block(int block, int blocks) {
   const int within = block % kGroup, first = block - within;
   return first + kGroup <= blocks ? first + within % kNumXcd * kXcdRun + within / kNumXcd : block;
 }
+
+// From this many tiles on (48 MB of transposed copy) the casts store the transposed copy with the streaming hint: a fifth of
+// what the memory-side cache holds is then more than the next launches of a step find again, and the row-major copy should be
+// what stays.  Below, the copy is still there for a launch that reads it at once, as the weight gradient reads that of a
+// gradient in the reference's layout and under wgrad = "copy".  Measured with new buffers every time, time with the hint over
+// time without, means of 20 launches of 16 - 224 MB: the launch alone, with the GEMM that reads the row-major copy, with the
+// weight gradient that reads the transposed one.
+//   * Cast, 16 - 43 MB: 0.99, 0.98, 1.08 (64 experts, 24576 skewed rows of 1408 37 / 37 us, 136 / 138, 249 / 197; 8 experts, 4001
+//     rows of 4096 25.8 / 26.2, 65 / 66, 69 / 64); 48 - 73 MB: 0.97, 0.98, 1.00; 98 MB and more: 0.90, 0.97, 0.97 (128 of 512
+//     rows of 2048 95 / 110, 211 / 221, 269 / 284).  With the hint on the row-major copy as well the cast alone is another 1 -
+//     3 % faster and the GEMM behind it 3 - 7 % slower.
+//   * Cast + dGELU: 0.99, 0.98, 1.07; 0.97, 0.98, 1.00; 0.92, 0.98, 0.97.
+//   * The transpose alone, whose only result the next launch reads, takes plain stores at any size: 1.02 alone, 1.08 with the
+//     weight gradient (16 of 750 rows of 6400 169 / 138; the only one more than 2 % the other way 128 of 512 rows of 2048, 228 / 236).
+constexpr int kStreamTiles = 3072;
 
 template <int OP, int FMT>
 __global__ __launch_bounds__(kPtThreads) void multi_pad_kernel(fp8gmm_tensor_desc* __restrict__ descs, int n) {
@@ -230,6 +241,7 @@ __global__ __launch_bounds__(kPtThreads) void multi_pad_kernel(fp8gmm_tensor_des
   __syncthreads();
 
   // ---- LDS tile -> transposed output: 16 token rows of one column per lane and step ----
+  const bool stream = OP != OP_TRANSPOSE && (int)gridDim.x >= kStreamTiles;
   const __amdgpu_buffer_rsrc_t rt = make_rsrc(out_t, fast ? (uint32_t)((int64_t)ncols * mpad) : 0u);
 #pragma unroll
   for (int q = 0; q < (TN * TM / 16) / kPtThreads; ++q) {
@@ -244,7 +256,9 @@ __global__ __launch_bounds__(kPtThreads) void multi_pad_kernel(fp8gmm_tensor_des
     const int grow = r0 + 16 * piece;
     const bool ok = gcol < ncols && grow < mpad;
     if (fast) {
-      buf_store16_stream(v, rt, ok ? (uint32_t)gcol * (uint32_t)mpad + (uint32_t)grow : kOobOffset);
+      const uint32_t off = ok ? (uint32_t)gcol * (uint32_t)mpad + (uint32_t)grow : kOobOffset;
+      if (stream) buf_store16_stream(v, rt, off);
+      else buf_store16(v, rt, off);
     } else if (ok) {
       uint8_t* dst = out_t + (int64_t)gcol * mpad + grow;
       if (vec_t) {

@@ -496,3 +496,38 @@ def test_every_tile_is_taken_once_whatever_the_number_of_workgroups(dev, shapes)
         assert_bytes_equal(d_outs[i], outs[i], f"cast {i} {s}")
         assert_bytes_equal(d_touts[i], touts[i], f"transpose {i} {s}")
         assert_scalar_bits_equal(d_amaxes[i].cpu(), amaxes[i], f"amax {i}")
+
+
+@pytest.mark.parametrize("op", ["cast", "dgelu", "transpose"])
+@pytest.mark.parametrize("shapes", [
+    [(12 * 128 - 7, 256 * 128 - 120)],                          # 3072 tiles, partial ones among them
+    [(12 * 128 - 7, 255 * 128), (5, 1024), (3 * 128 + 1, 96)],  # 3060 + 8 + 4: 3072 as well
+    [(11 * 128, 279 * 128), (200, 8)],                          # 3069 + 2: one short
+], ids=["3072", "3072 in three", "3071"])
+def test_transposed_copies_of_either_store_form(dev, shapes, op):
+    """From 3072 tiles on a cast stores its transposed copy with the streaming hint.  The bytes are those of the launch
+    without a transpose and of its result transposed by torch; the padding is zero."""
+    backend = _backend()
+    g = torch.Generator(device="cuda").manual_seed(43)
+    dtype = torch.float8_e4m3fn
+    ins = [torch.randn(s, generator=g, dtype=torch.bfloat16, device=dev) for s in shapes]
+    pre = [torch.randn(s, generator=g, dtype=torch.bfloat16, device=dev) for s in shapes]
+    scales = [torch.full((1,), 3.5, device=dev) for _ in shapes]
+    want = [torch.empty(s, dtype=dtype, device=dev) for s in shapes]
+    want_amax, amax = ([torch.zeros(1, device=dev) for _ in shapes] for _ in range(2))
+    outs = [torch.full(s, 0x55, dtype=torch.uint8, device=dev).view(dtype) for s in shapes]
+    touts = [torch.full(s, 0x55, dtype=torch.uint8, device=dev).view(dtype) for s in transpose_shapes(shapes, True)]
+    if op == "dgelu":
+        backend.multi_cast_dgelu(ins, pre, want, scales, want_amax)
+        backend.multi_cast_transpose_dgelu(ins, pre, outs, touts, scales, amax)
+    else:
+        backend.multi_quantize(ins, want, scales, want_amax)
+        if op == "cast":
+            backend.multi_cast_transpose(ins, outs, touts, scales, amax)
+        else:
+            outs, amax = want, want_amax
+            backend.multi_transpose(want, touts)
+    for i, (rows, _) in enumerate(shapes):
+        assert torch.equal(outs[i].view(torch.uint8), want[i].view(torch.uint8)) and torch.equal(amax[i], want_amax[i]), i
+        t = touts[i].view(torch.uint8)
+        assert torch.equal(t[:, :rows], want[i].view(torch.uint8).t()) and not t[:, rows:].any(), i
