@@ -299,10 +299,12 @@ int fp8gmm_multi_cast_dgelu(fp8gmm_tensor_desc* descs_dev, int n, int total_bloc
  * Validates `probs[0..n)` like fp8gmm_plan_grouped_gemm_layout, fills tile_begin / cost_begin, and writes the work
  * list of a launch with `grid` workgroups (fp8gmm_gemm_grid) into items[0 .. rounds * grid) and
  * fixups[0 .. n_fixups).  `layout` takes the launch's flags: the KMAJOR flags as for the plain plan, and
- * FP8GMM_EPI_GELU / FP8GMM_EPI_DGELU, which only weigh the decision below (completing a shared tile costs more with that epilogue).  stream_k != 0: the workgroups of an XCD share the tail tiles of their range along K when
- * the last round would otherwise be mostly idle and the time it saves is more than the partial sums cost; the launch then needs plan->n_slots workspace slots (never more
- * than 2 * grid).  stream_k > 1: the same, but with at most stream_k slots - a launch whose sharing would need more
- * is planned with whole tiles instead (callers of fp8gmm_grouped_gemm_static pass FP8GMM_GEMM_STATIC_SLOTS and never
+ * FP8GMM_EPI_GELU / FP8GMM_EPI_DGELU, which only weigh the decision below (completing a shared tile costs more with
+ * that epilogue).  stream_k != 0: the workgroups of an XCD share the tail tiles of their range along K when the last
+ * round would otherwise be mostly idle and the launch is through sooner for it, the cost of the partial sums included;
+ * it then needs plan->n_slots workspace slots (never more than 2 * grid).  stream_k > 1: the same, but with at most
+ * stream_k slots - a launch whose sharing would need more is planned with whole tiles instead (callers of
+ * fp8gmm_grouped_gemm_static pass FP8GMM_GEMM_STATIC_SLOTS and never
  * see FP8GMM_ERR_WORKSPACE).  stream_k == 0: every record is a whole tile, no workspace, no fix-up launch.
  * The sizes are returned in *plan even when max_items / max_fixups are too small (FP8GMM_ERR_BUFFER_TOO_SMALL;
  * the arrays then hold the part of the list that fitted and are not to be used): call again with larger arrays.  Host only, no GPU needed.
