@@ -123,19 +123,19 @@ struct Pass {
 // switches, which are most of a short launch, and a range's end is spread over tiles a quarter of the size.  What the form
 // pays, twice the operand bytes from L2 per flop, grows with the K = 128 steps of the large tiles ("steps" below).
 // Weight gradients, traced inside a layer's step, large tiles -> this form in us (profiles/tile_rules.md has all of 462):
-//   * Up to 9000 steps, 8.5 a tile, whatever the number of tiles: 2048 tiles of 3.4 steps 88 -> 80, of 6.3 (12800 steps) 107 ->
-//     117; 4096 of 2.0 127 -> 115, of 2.7 (10880) 143 -> 148; 8330 of one step 178 -> 137; 448 of 27 (12012) 93 -> 133.  Not
-//     results of up to 144 columns in many tiles: their second column of tiles stores pieces of 32 bytes (144 columns, 1988,
-//     3478 and 4750 tiles of 1.3 - 2.4 steps 81 -> 87, 132 -> 142, 177 -> 210; 160 columns, 2444 64 -> 61).
+//   * Up to 9000 steps, 8.5 a tile, whatever the number of tiles: 2048 tiles of 3.5 steps 82 -> 85, of 6.2 (12800 steps) 113 ->
+//     121; 4096 of 2.0 128 -> 117, of 2.7 (10880) 144 -> 145, of 3.5 (14208) 160 -> 176; 8330 of one step 169 -> 133; 448 of 27
+//     (12012) 93 -> 150.  Not results of up to 144 columns in many tiles: their second column of tiles stores pieces of 32
+//     bytes (144 columns, 1988, 3478 and 4750 tiles of 1.3 - 2.3 steps 93 -> 90, 125 -> 141, 149 -> 168; 160 columns, 2444 59 -> 56).
 //   * Under a skewed split large tiles wait for the longest contraction, the more the larger it is against a compute unit's
-//     share of the launch, at any number of steps: at 0.75 of a share and more 64 of 1408 x 2048 with 10608 / 13536 / 16416 /
-//     20064 steps 158 / 167 / 212 / 242 -> 154 / 158 / 179 / 239, 8 of 2048 x 1024 with 2368 steps 38 -> 28, 16 of 2048 x 2048 with
-//     12.5 / 16.5 / 20 / 24.5 steps a tile 144 / 180 / 159 / 248 -> 110 / 157 / 200 / 241; at half a share 32 of 4096 x 2048 143 ->
-//     148 and 260 -> 370.  At 2.25 shares and more also with 16 to 24 steps a tile, where six launches took 21 % less; past 24 it
-//     depends on how the long contraction falls into the XCDs' ranges (0.76 - 1.64 x).
-// The 386 launches that the rule takes take 16 % less time in the mean.  12 lose more than a twentieth, all but one of them skewed and
-// with 6 to 12 steps a tile; the most: 19 of 1360 x 1392, 26955 rows 83 -> 104; 8 of 2192 x 1264, 8875 43 -> 51; 3 of 5744 x
-// 912, 3178 32 -> 38.  Steps a tile, share and tiles do not tell them from launches that gain as much.
+//     share of the launch, at any number of steps: at 0.75 of a share and more 64 of 1408 x 2048 with 10464 / 13632 / 16560 /
+//     19872 steps 148 / 187 / 199 / 228 -> 128 / 156 / 184 / 209, 8 of 2048 x 1024 with 2400 steps 46 -> 32, 16 of 2048 x 2048 with
+//     12.6 / 16.5 / 20 / 24.4 steps a tile 150 / 182 / 174 / 250 -> 121 / 159 / 197 / 257; at half a share 32 of 4096 x 2048 186 ->
+//     204 and 261 -> 353.  At 2.25 shares and more also with 16 to 24 steps a tile, where five launches took 15 % less; past 24 it
+//     depends on how the long contraction falls into the XCDs' ranges (0.69 - 1.53 x).
+// The 385 launches that the rule takes take 15 % less time in the mean.  16 lose more than a twentieth, eleven of them skewed and
+// with 6 to 16 steps a tile; the most: 7 of 5408 x 1232, 8841 rows 79 -> 104; 28 of 11376 x 192, 12965 59 -> 73; 19 of 1360 x
+// 1392, 26955 87 -> 104.  Steps a tile, share and tiles do not tell them from launches that gain as much.
 bool small_tiles_pay(const fp8gmm_gemm_problem* p, int n, int layout) {
   int64_t large = 0, small = 0, steps = 0, longest = 0, widest = 0;
   for (int i = 0; i < n; ++i) {
