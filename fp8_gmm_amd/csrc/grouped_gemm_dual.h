@@ -79,7 +79,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void grouped_gemm_dual_kernel(
   const int wave_m = wave / WAVES_N, wave_n = wave % WAVES_N;
   const int l32 = lane & 31;
   const int khalf = lane >> 5;
-  const uint32_t lds_base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds);
+  const uint32_t lds_wave = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds) + wave * 1024;
 
   // load and fragment maps: those of grouped_gemm_kernel, the token operand's with the small tile's extents
   const int drow = lane >> 3;
@@ -139,15 +139,14 @@ __global__ __launch_bounds__(NTHREADS, 1) void grouped_gemm_dual_kernel(
   const int tr_col_b = ((lane & 15) ^ (2 * (krow_b & 7))) << 4;
   const int krow_a = wave * 8 + lane / 8;
   const int tr_col_a = ((lane & 7) ^ (krow_a & 6)) << 4;
-  auto load_setup = [&]() {
+  auto load_setup = [&]() {   // the record after this one is fetched last, as in grouped_gemm_kernel
     for (;;) {
-      const ItemLoad gl = ld_next_l;
-      const ItemTile gt = ld_next_t;
+      const ItemLoad& gl = ld_next_l;
+      const ItemTile& gt = ld_next_t;
       ld_live = gt.prob >= 0;
       if (!ld_live) break;
-      ld_next_l = item_load(r_ld + 1);
-      ld_next_t = item_tile(r_ld + 1);
-      if (gt.nk > 0) {
+      const bool take = gt.nk > 0;
+      if (take) {
         // (read back as lane-uniform words: with the two copies of the tile's code below, the compiler otherwise keeps
         // the record fetched ahead, and the descriptors made of it, in vector registers, which the loads cannot take)
         rsrc_a[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)gl.a);
@@ -176,30 +175,36 @@ __global__ __launch_bounds__(NTHREADS, 1) void grouped_gemm_dual_kernel(
         ld_kt = gt.k_begin;
         ld_nk = gt.k_begin + gt.nk;
         step_setup();
-        return;
       }
+      FP8GMM_RECORD_USED(gt);
       ++r_ld;
+      ld_next_l = item_load(r_ld);
+      ld_next_t = item_tile(r_ld);
+      if (take) return;
     }
     rsrc_a[2] = 0;
     rsrc_b[2] = 0;
   };
   // part j of the tokens / weights of the step the load cursor points at, into stage `stage`
-  auto dma_a = [&](int stage, int j) {   // j < kPartsA
+  auto dma_a = [&](int stage, auto part) {   // part < kPartsA
+    constexpr int j = decltype(part)::value;
     uint32_t v = a_k + j * a_step;
     if constexpr (!A_TR) v = k_ok ? v : 0xffffffffu;
-    const uint32_t l = lds_base + stage * kStep + (wave + NWAVES * j) * 1024;
-    FP8GMM_DMA(l, v, rsrc_a);
+    const uint32_t to = lds_wave + stage * kStep;   // (locals: a generic lambda's assembly operands do not capture)
+    const i32x4 from = rsrc_a;
+    FP8GMM_DMA(to, NWAVES * j * 1024, v, from);
   };
-  auto dma_b = [&](int stage, int j) {   // j < kPartsB
+  auto dma_b = [&](int stage, auto part) {   // part < kPartsB
+    constexpr int j = decltype(part)::value;
     uint32_t v = b_k + j * b_step;
     if constexpr (!B_TR) v = k_ok ? v : 0xffffffffu;
-    const uint32_t l = lds_base + stage * kStep + kUnitA + (wave + NWAVES * j) * 1024;
-    FP8GMM_DMA(l, v, rsrc_b);
+    const uint32_t to = lds_wave + stage * kStep;   // (locals: a generic lambda's assembly operands do not capture)
+    const i32x4 from = rsrc_b;
+    FP8GMM_DMA(to, kUnitA + NWAVES * j * 1024, v, from);
   };
   auto dma_advance = [&]() {
     if (!ld_live) return;
     if (++ld_kt == ld_nk) {
-      ++r_ld;
       load_setup();
     } else {
       step_setup();
@@ -253,20 +258,15 @@ __global__ __launch_bounds__(NTHREADS, 1) void grouped_gemm_dual_kernel(
   constexpr int kFirstLoads = kPartsA + 2;                 // of a step's 12 loads: the tokens and two parts of the weights
   constexpr int kLastLoads = kPartsB - 2;
   load_setup();
-#pragma unroll
-  for (int j = 0; j < kPartsA; ++j) dma_a(0, j);
-#pragma unroll
-  for (int j = 0; j < kPartsB; ++j) dma_b(0, j);
+  static_for<kPartsA>([&](auto j) { dma_a(0, j); });
+  static_for<kPartsB>([&](auto j) { dma_b(0, j); });
   dma_advance();
-#pragma unroll
-  for (int j = 0; j < kPartsA; ++j) dma_a(1, j);
-#pragma unroll
-  for (int j = 0; j < kPartsB; ++j) dma_b(1, j);
+  static_for<kPartsA>([&](auto j) { dma_a(1, j); });
+  static_for<kPartsB>([&](auto j) { dma_b(1, j); });
   dma_advance();
-#pragma unroll
-  for (int j = 0; j < kPartsA; ++j) dma_a(2, j);
-  dma_b(2, 0);
-  dma_b(2, 1);
+  static_for<kPartsA>([&](auto j) { dma_a(2, j); });
+  dma_b(2, kPart<0>);
+  dma_b(2, kPart<1>);
   FP8GMM_WAIT_VM(kPartsA + kPartsB + kFirstLoads);
   __builtin_amdgcn_s_barrier();
 #pragma unroll
@@ -358,27 +358,27 @@ __global__ __launch_bounds__(NTHREADS, 1) void grouped_gemm_dual_kernel(
       // previous step's barrier)
       const uint8_t* qa = lds + cur * kStep;
       const uint8_t* qb = qa + kUnitA;
-      dma_b(nn, 2);
+      dma_b(nn, kPart<2>);
       frag_b(fb1[0], qb, 0, 1);
       if constexpr (E != 0) { FP8GMM_DQ(UL, 0); FP8GMM_DQ(UL, 1); }
       FP8GMM_SB(); FP8GMM_DMF0(0, 1); FP8GMM_SB();
-      dma_b(nn, 3);
+      dma_b(nn, kPart<3>);
       frag_b(fb1[1], qb, 1, 1);
       if constexpr (E != 0) { FP8GMM_DQ(UL, 2); }
       FP8GMM_SB(); FP8GMM_DMF0(0, 2); FP8GMM_SB();
-      dma_b(nn, 4);
+      dma_b(nn, kPart<4>);
       frag_b(fb1[2], qb, 2, 1);
       if constexpr (E != 0) { FP8GMM_DQ(UL, 3); }
       FP8GMM_SB(); FP8GMM_DMF0(0, 3); FP8GMM_SB();
-      dma_b(nn, 5);
+      dma_b(nn, kPart<5>);
       frag_b(fb1[3], qb, 3, 1);
       if constexpr (E != 0) { FP8GMM_DQ(UL, 4); }
       FP8GMM_SB(); FP8GMM_DMF0(1, 0); FP8GMM_SB();
-      dma_b(nn, 6);
+      dma_b(nn, kPart<6>);
       frag_a(fa1[0], qa, 0, 1);
       if constexpr (E != 0) { FP8GMM_DQ(UL, 5); }
       FP8GMM_SB(); FP8GMM_DMF0(1, 1); FP8GMM_SB();
-      dma_b(nn, 7);
+      dma_b(nn, kPart<7>);
       frag_a(fa1[1], qa, 1, 1);
       if constexpr (E != 0) { FP8GMM_DQ(UL, 6); FP8GMM_DQ(UL, 7); }
       FP8GMM_SB(); FP8GMM_DMF0(1, 2); FP8GMM_SB();
@@ -409,27 +409,27 @@ __global__ __launch_bounds__(NTHREADS, 1) void grouped_gemm_dual_kernel(
       } else {
         dma_advance();
       }
-      dma_a(cur, 0);
+      dma_a(cur, kPart<0>);
       frag_b(fb0[0], qb, 0, 0);
       if constexpr (E != 0) { FP8GMM_DQ(UH, 0); FP8GMM_DQ(UH, 1); }
       FP8GMM_SB(); FP8GMM_DMF1(0, 1); FP8GMM_SB();
-      dma_a(cur, 1);
+      dma_a(cur, kPart<1>);
       frag_b(fb0[1], qb, 1, 0);
       if constexpr (E != 0) { FP8GMM_DQ(UH, 2); }
       FP8GMM_SB(); FP8GMM_DMF1(0, 2); FP8GMM_SB();
-      dma_a(cur, 2);
+      dma_a(cur, kPart<2>);
       frag_b(fb0[2], qb, 2, 0);
       if constexpr (E != 0) { FP8GMM_DQ(UH, 3); }
       FP8GMM_SB(); FP8GMM_DMF1(0, 3); FP8GMM_SB();
-      dma_a(cur, 3);
+      dma_a(cur, kPart<3>);
       frag_b(fb0[3], qb, 3, 0);
       if constexpr (E != 0) { FP8GMM_DQ(UH, 4); }
       FP8GMM_SB(); FP8GMM_DMF1(1, 0); FP8GMM_SB();
-      dma_b(cur, 0);
+      dma_b(cur, kPart<0>);
       frag_a(fa0[0], qa, 0, 0);
       if constexpr (E != 0) { FP8GMM_DQ(UH, 5); }
       FP8GMM_SB(); FP8GMM_DMF1(1, 1); FP8GMM_SB();
-      dma_b(cur, 1);
+      dma_b(cur, kPart<1>);
       frag_a(fa0[1], qa, 1, 0);
       if constexpr (E != 0) { FP8GMM_DQ(UH, 6); FP8GMM_DQ(UH, 7); }
       FP8GMM_SB(); FP8GMM_DMF1(1, 2); FP8GMM_SB();

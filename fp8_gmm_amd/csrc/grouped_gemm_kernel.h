@@ -116,11 +116,24 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
   "a48", "a49", "a50", "a51", "a52", "a53", "a54", "a55", "a56", "a57", "a58", "a59", "a60", "a61", "a62", "a63"
 
 #define FP8GMM_SB() __builtin_amdgcn_sched_barrier(0)
+// Behind the last use of a fetched record's words: from here on its registers may receive the next one.  (m0 is named because
+// the words around it are: k .. nk travel in a load of four words, and a word of it that nothing reads would be given to
+// another value at once - which then waits for the load.)
+#define FP8GMM_RECORD_USED(gt)            \
+  do {                                    \
+    asm volatile("" ::"s"((gt).m0));      \
+    __builtin_amdgcn_sched_barrier(0);    \
+  } while (0)
 #define FP8GMM_WAIT_VM(n) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(n) : "memory")
 #define FP8GMM_WAIT_VM_LGKM(n) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(n) : "memory")
-// global -> LDS: lane i's 16 bytes land at M0 + 16 i; out-of-range offsets deliver zeros
-#define FP8GMM_DMA(lds_addr, voff, rsrc) \
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds_addr), "v"(voff), "s"(rsrc))
+// global -> LDS: lane i's 16 bytes land at M0 + 16 i; out-of-range offsets deliver zeros.  `imm` is a constant: formed from it
+// here, an address is not a scalar register per load instruction of a step.
+#define FP8GMM_DMA(lds_addr, imm, voff, rsrc)                                                                            \
+  asm volatile("s_add_u32 m0, %0, %3\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds_addr), "v"(voff), "s"(rsrc), \
+               "n"(imm)                                                                                                  \
+               : "scc")
+template <int J>
+inline constexpr std::integral_constant<int, J> kPart{};   // part J of a unit's loads
 
 // The accumulators of a lane are the accumulation registers a0 .. a255 (a0 .. a63 for the small tile), addressed BY
 // NAME in every statement that touches them: MFMA tile (i, j) of a wavefront's sub-tile owns the 16 registers from
@@ -162,8 +175,11 @@ __device__ __forceinline__ void acc_tile_clear() {
 // and a vector load would have to be waited for with vmcnt(0), i.e. together with every operand load the
 // load stream has in flight for the next tile - thousands of cycles per tile when those come from HBM.
 typedef __attribute__((address_space(4))) const float scalar_float;
-__device__ __forceinline__ float load_scale(const float* p) {   // constant while the kernel runs; null means 1
-  return p != nullptr ? *reinterpret_cast<scalar_float*>(reinterpret_cast<uintptr_t>(p)) : 1.f;
+// Null means 1: by choice of the address, not of the value - behind a branch the value of a load meets another one, and the
+// compiler waits for it there instead of where it is used.
+__device__ const float kNoScale = 1.f;
+__device__ __forceinline__ float load_scale(const float* p) {   // constant while the kernel runs
+  return *reinterpret_cast<scalar_float*>(reinterpret_cast<uintptr_t>(p != nullptr ? p : &kNoScale));
 }
 // The running maximum another workgroup may be raising at this moment: any value read is a lower bound of it.
 __device__ __forceinline__ float peek_amax(const float* p) {
@@ -214,6 +230,8 @@ constexpr uint32_t kMaskedOffset = 0x80000000u;  // + any row offset of a tile (
 // TILE: 256 (the namespace's constants) or 128 (the small tile: 64 x 64 per wavefront, 16 KB of staging).
 // `released(i, j)` (integral constants) is called right after MFMA tile (i, j) of the staged bf16 path has been read
 // out of its accumulators: from there on they may receive the next tile's products.
+// The epilogues a kernel is compiled with: kPlain knows bf16 results without an activation, kAny every kind of result.
+constexpr int kPlain = 0, kAny = 1;
 // whether the plain bf16 epilogue through the staging area applies to this tile
 template <int TILE>
 __device__ __forceinline__ bool staged_bf16_tile(const fp8gmm_gemm_problem& pr, int m0, int n0, int out_kind,
@@ -231,9 +249,9 @@ struct NothingReleased {
 };
 // `mt`: 32-row blocks per wavefront: MT, or MT / 2 for a tile of half height, whose wavefronts stand on rows
 // wave_m * 64 + 32 i.  Returns the number of stores per wavefront that the staged bf16 form left in flight (0: another form ran).
-template <int TILE, class Released = NothingReleased>
+template <int TILE, int EPI, class Released = NothingReleased>
 __device__ __forceinline__ int tile_epilogue(const fp8gmm_gemm_problem& pr, int m0, int n0, int out_kind, int epilogue,
-                                             uint8_t* stage, int mt, bool oob_zero, bool oob_rows_zero, float s, float cs,
+                                             bool staged, uint8_t* stage, int mt, bool oob_zero, bool oob_rows_zero, float s, float cs,
                                              Released released = Released()) {
   constexpr int BM = TILE, BN = TILE, WN = TILE / 2, MT = TILE / 64, NT = WN / 32;
   const int WM = mt * 32;   // rows of a wavefront's sub-tile
@@ -249,8 +267,8 @@ __device__ __forceinline__ int tile_epilogue(const fp8gmm_gemm_problem& pr, int 
   const int l32 = lane & 31, khalf = lane >> 5;
   const int M = pr.m, N = pr.n;
   int fast = 0;
-    const bool gelu = (epilogue & FP8GMM_EPI_GELU) != 0;
-    const bool dgelu_in = (epilogue & FP8GMM_EPI_DGELU) != 0 && pr.aux != nullptr;   // aux is then an INPUT
+    const bool gelu = EPI == kAny && (epilogue & FP8GMM_EPI_GELU) != 0;
+    const bool dgelu_in = EPI == kAny && (epilogue & FP8GMM_EPI_DGELU) != 0 && pr.aux != nullptr;   // aux is then an INPUT
     const bool two = (epilogue & FP8GMM_EPI_TWO_ROUNDINGS) != 0;
     const int64_t ldc = pr.ldc;
     float amax = 0.f;
@@ -259,7 +277,7 @@ __device__ __forceinline__ int tile_epilogue(const fp8gmm_gemm_problem& pr, int 
     const int cv = N - n0 < BN ? N - n0 : BN;
     // 16-byte pieces of the tile's rows can be addressed with 32-bit offsets below 2^30
     const bool desc_ok = ((ldc & 7) == 0) && ldc < (1 << 21) && ((reinterpret_cast<uintptr_t>(pr.c) & 15) == 0);
-    if (staged_bf16_tile<TILE>(pr, m0, n0, out_kind, epilogue)) {
+    if (staged) {
       // Plain bf16 output: straight-line code with an exact store count.
       // Through LDS, so that a store instruction writes whole lines.  In the MFMA layout a lane holds 4
       // consecutive columns of one row, and a 16-byte store per lane touches 32 rows: 64 separate 32-byte
@@ -318,7 +336,7 @@ __device__ __forceinline__ int tile_epilogue(const fp8gmm_gemm_problem& pr, int 
       store_unit(mt - 1, kUnitsPerRow - 1);
       __builtin_amdgcn_s_barrier();  // the staging area goes back to the operand ring
       fast = mt * kUnitsPerRow * 4;
-    } else if (TILE == 256 && out_kind == FP8GMM_E4M3 && gelu && pr.aux != nullptr && desc_ok && ((ldc & 15) == 0) &&
+    } else if (EPI == kAny && TILE == 256 && out_kind == FP8GMM_E4M3 && gelu && pr.aux != nullptr && desc_ok && ((ldc & 15) == 0) &&
                ((reinterpret_cast<uintptr_t>(pr.aux) & 15) == 0) && (interior || (oob_zero && (cv & 15) == 0))) {
       // The fused GELU form (e4m3 gelu(v) * c_scale, bf16 v on the side, amax of gelu(v)): both outputs go
       // through the staging area like the plain form's, one 32-row block at a time, in ONE pass over the
@@ -426,7 +444,7 @@ __device__ __forceinline__ int tile_epilogue(const fp8gmm_gemm_problem& pr, int 
       });
       __builtin_amdgcn_s_barrier();  // the staging area goes back to the operand ring
       merge_amax(pr.c_amax, wave_max(tile_amax), lane);
-    } else if (TILE == 256 && out_kind != FP8GMM_OUT_BF16 && dgelu_in && desc_ok && ((ldc & 15) == 0) &&
+    } else if (EPI == kAny && TILE == 256 && out_kind != FP8GMM_OUT_BF16 && dgelu_in && desc_ok && ((ldc & 15) == 0) &&
                ((reinterpret_cast<uintptr_t>(pr.aux) & 7) == 0) && n0 + BN <= N && (interior || oob_rows_zero)) {
       // The data gradient with the GELU's derivative folded in: x = v * dgelu(pre), fp8(x * c_scale), amax of x.
       // `pre` (bf16, the layout of c) is read in the MFMA layout, 8 bytes per lane and piece, one 32-row block
@@ -498,7 +516,7 @@ __device__ __forceinline__ int tile_epilogue(const fp8gmm_gemm_problem& pr, int 
       });
       __builtin_amdgcn_s_barrier();  // the staging area goes back to the operand ring
       merge_amax(pr.c_amax, wave_max(tile_amax), lane);
-    } else if (out_kind == FP8GMM_OUT_BF16) {
+    } else if (EPI == kPlain || out_kind == FP8GMM_OUT_BF16) {
       uint16_t* __restrict__ C = static_cast<uint16_t*>(pr.c);
       uint16_t* __restrict__ AUX = static_cast<uint16_t*>(pr.aux);
       const bool vec = ((ldc & 3) == 0) && ((reinterpret_cast<uintptr_t>(C) & 7) == 0) &&
@@ -619,6 +637,14 @@ __device__ __forceinline__ void partial_store(uint8_t* slot) {
     }
   });
 }
+// A condition that is the same in every lane, as a word in one scalar register.  As a bool that lives across branches it is a
+// lane mask in two, and the main loop's scalar registers are all taken: what does not fit is parked in the lanes of a
+// vector register, and a record on its way from memory is waited for on the spot to be parked.
+__device__ __forceinline__ int as_word(bool b) {
+  int w = __builtin_amdgcn_readfirstlane(b ? 1 : 0);
+  asm("" : "+s"(w));
+  return w;
+}
 // The half of a work-list record (fp8gmm_gemm_item) that a side of the kernel needs, as scalar loads.
 struct ItemLoad {   // bytes 0..31: what the load stream needs besides ItemTile
   uint64_t a, b;
@@ -649,13 +675,15 @@ static_assert(offsetof(fp8gmm_gemm_item, k) == 32 && offsetof(fp8gmm_gemm_item, 
 // full tiles it is 10 - 20 % slower however short the contraction.  Which tile a launch takes is decided when it
 // is planned (FP8GMM_GEMM_TILE_128); the results are the same bits either way.  No sharing along K and no fused
 // GELU epilogue in this form.
-template <int A_FMT, int B_FMT, bool A_TR, bool B_TR, int TILE>
+template <int A_FMT, int B_FMT, bool A_TR, bool B_TR, int TILE, int EPI>
 __global__ __launch_bounds__(NTHREADS, TILE == 256 ? 1 : 2) void grouped_gemm_kernel(
-    const fp8gmm_gemm_problem* __restrict__ probs, const fp8gmm_gemm_item* __restrict__ items, int out_kind,
-    int epilogue, uint8_t* __restrict__ workspace, const fp8gmm_tensor_desc* __restrict__ merge_descs, int merge_n) {
+    const fp8gmm_gemm_problem* __restrict__ probs, const fp8gmm_gemm_item* __restrict__ items, int out_kind_arg,
+    int epilogue_arg, uint8_t* __restrict__ workspace, const fp8gmm_tensor_desc* __restrict__ merge_descs, int merge_n) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   // the amax merge of the cast launch in front of this one, where the pass planner has moved it here
   if (merge_n > 0 && blockIdx.x == 0) merge_amax_partials(merge_descs, merge_n, threadIdx.x, NTHREADS);
+  const int out_kind = EPI == kPlain ? FP8GMM_OUT_BF16 : out_kind_arg;
+  const int epilogue = EPI == kPlain ? epilogue_arg & FP8GMM_EPI_TWO_ROUNDINGS : epilogue_arg;
   // the tile's extents shadow the namespace's (which are those of the 256 x 256 tile)
   [[maybe_unused]] constexpr int BM = TILE;
   constexpr int BN = TILE, US = TILE * BK, WM = TILE / 2, WN = TILE / 2, MT = WM / 32, NT = WN / 32;
@@ -670,7 +698,7 @@ __global__ __launch_bounds__(NTHREADS, TILE == 256 ? 1 : 2) void grouped_gemm_ke
   const int wave_n = wave % WAVES_N;  // 0..1
   const int l32 = lane & 31;
   const int khalf = lane >> 5;   // which 32-byte half of the 64-byte MFMA K slice this lane feeds
-  const uint32_t lds_base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds);
+  const uint32_t lds_wave = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds) + wave * 1024;
 
   // DMA lane map, row-major operand: one wavefront instruction fills 8 rows x 128 B of a unit, i.e. whole
   // cache lines: lane -> row lane >> 3 of the group, slot chunk lane & 7.  Chunk c of row r is kept at chunk
@@ -719,13 +747,13 @@ __global__ __launch_bounds__(NTHREADS, TILE == 256 ? 1 : 2) void grouped_gemm_ke
   const size_t item_stride = (size_t)gridDim.x * sizeof(fp8gmm_gemm_item);
   auto item_load = [&](int r) { return *reinterpret_cast<const ItemLoad*>(my_items + r * item_stride); };
   auto item_tile = [&](int r) { return *reinterpret_cast<const ItemTile*>(my_items + r * item_stride + 32); };
-  int r_ld = 0;                         // record the load side is in
-  ItemLoad ld_next_l = item_load(0);    // ... and the record it takes next, fetched ahead
+  int r_ld = 0;                         // the record the load side takes next, fetched ahead
+  ItemLoad ld_next_l = item_load(0);
   ItemTile ld_next_t = item_tile(0);
   if (ld_next_t.prob < 0) return;
 
   // ---- load side: runs two steps ahead of the compute side, possibly in the next tile ----
-  bool ld_live = true;  // the load cursor still points at an item
+  int ld_live = 1;      // the load cursor still points at an item (flags that live long are whole words: see `as_word`)
   int ld_kt = 0, ld_nk = 0, ld_kmax = 0;
   [[maybe_unused]] int ld_lda = 0, ld_ldb = 0;  // contraction-major operands only
   i32x4 rsrc_a = {0, 0, 0, 0x00020000}, rsrc_b = {0, 0, 0, 0x00020000};  // raw buffers; empty until set up
@@ -760,16 +788,17 @@ __global__ __launch_bounds__(NTHREADS, TILE == 256 ? 1 : 2) void grouped_gemm_ke
   constexpr int kTrRows = 1024 / kTrPitch;             // contraction rows per load instruction: 4 or 8
   const int krow = wave * kTrRows + lane / (kTrPitch / 16);
   const int tr_col = TILE == 256 ? ((lane & 15) ^ (2 * (krow & 7))) << 4 : ((lane & 7) ^ (krow & 6)) << 4;
-  // Takes the record fetched ahead (r_ld), fetches the one after it, and sets up descriptors and offsets.
+  // Takes the record fetched ahead (r_ld), sets up descriptors and offsets, and only then fetches the one after it, into the
+  // same registers: fetched while the old one is still in use, it lands in other registers, and the copy back, at the end
+  // of this function, waits for memory at every tile.
   auto load_setup = [&]() {
     for (;;) {
-      const ItemLoad gl = ld_next_l;
-      const ItemTile gt = ld_next_t;
-      ld_live = gt.prob >= 0;
+      const ItemLoad& gl = ld_next_l;
+      const ItemTile& gt = ld_next_t;
+      ld_live = as_word(gt.prob >= 0);
       if (!ld_live) break;
-      ld_next_l = item_load(r_ld + 1);  // every list ends with an end record, so r_ld + 1 exists
-      ld_next_t = item_tile(r_ld + 1);
-      if (gt.nk > 0) {
+      const bool take = gt.nk > 0;   // an item without K work needs no loads
+      if (take) {
         rsrc_a[0] = (int)(uint32_t)gl.a;
         rsrc_a[1] = (int)(uint32_t)(gl.a >> 32);
         rsrc_a[2] = (int)gl.a_bytes;
@@ -796,9 +825,12 @@ __global__ __launch_bounds__(NTHREADS, TILE == 256 ? 1 : 2) void grouped_gemm_ke
         ld_kt = gt.k_begin;
         ld_nk = gt.k_begin + gt.nk;
         step_setup();
-        return;
       }
-      ++r_ld;  // an item without K work needs no loads
+      FP8GMM_RECORD_USED(gt);
+      ++r_ld;   // every list ends with an end record, so it exists
+      ld_next_l = item_load(r_ld);
+      ld_next_t = item_tile(r_ld);
+      if (take) return;
     }
     // Past the end of the stream the loads are issued all the same, against empty descriptors (zero fill),
     // which keeps the vmcnt arithmetic uniform.
@@ -806,22 +838,25 @@ __global__ __launch_bounds__(NTHREADS, TILE == 256 ? 1 : 2) void grouped_gemm_ke
     rsrc_b[2] = 0;
   };
   // One instruction of that step: part j (0..7) of the token operand into ring unit `unit`, or of the weights.
-  auto dma_a = [&](int unit, int j) {
+  auto dma_a = [&](int unit, auto part) {
+    constexpr int j = decltype(part)::value;
     uint32_t v = a_k + j * a_step;
     if constexpr (!A_TR) v = k_ok ? v : 0xffffffffu;
-    const uint32_t l = lds_base + unit * US + (wave + NWAVES * j) * 1024;
-    FP8GMM_DMA(l, v, rsrc_a);
+    const uint32_t to = lds_wave + unit * US;   // (locals: a generic lambda's assembly operands do not capture)
+    const i32x4 from = rsrc_a;
+    FP8GMM_DMA(to, NWAVES * j * 1024, v, from);
   };
-  auto dma_b = [&](int unit, int j) {
+  auto dma_b = [&](int unit, auto part) {
+    constexpr int j = decltype(part)::value;
     uint32_t v = b_k + j * b_step;
     if constexpr (!B_TR) v = k_ok ? v : 0xffffffffu;
-    const uint32_t l = lds_base + unit * US + (wave + NWAVES * j) * 1024;
-    FP8GMM_DMA(l, v, rsrc_b);
+    const uint32_t to = lds_wave + unit * US;   // (locals: a generic lambda's assembly operands do not capture)
+    const i32x4 from = rsrc_b;
+    FP8GMM_DMA(to, NWAVES * j * 1024, v, from);
   };
   auto dma_advance = [&]() {
     if (!ld_live) return;
     if (++ld_kt == ld_nk) {
-      ++r_ld;
       load_setup();
     } else {
       step_setup();
@@ -869,7 +904,7 @@ __global__ __launch_bounds__(NTHREADS, TILE == 256 ? 1 : 2) void grouped_gemm_ke
     }
   };
   // (token fragments: `half` = the tile they are read for is of half height)
-  [[maybe_unused]] auto half_a = [&](i32x8& f, const uint8_t* unit, int i, int hh, int h, bool half = false) {
+  [[maybe_unused]] auto half_a = [&](i32x8& f, const uint8_t* unit, int i, int hh, int h, int half = 0) {
     if constexpr (!A_TR) {
       read_half(f, unit - (half ? half_rows_back : 0) + fa_off + i * 32 * BK, hh, h);
     } else {
@@ -884,7 +919,7 @@ __global__ __launch_bounds__(NTHREADS, TILE == 256 ? 1 : 2) void grouped_gemm_ke
       read_frag_tr(f, (uint32_t)(uintptr_t)unit + fbt_off[j] + hh * (64 * kTrPitch));
     }
   };
-  auto read_frag_a = [&](i32x8& f, const uint8_t* unit, int i, int hh, bool half = false) {
+  auto read_frag_a = [&](i32x8& f, const uint8_t* unit, int i, int hh, int half = 0) {
     if constexpr (!A_TR) {
       read_frag(f, unit - (half ? half_rows_back : 0) + fa_off + i * 32 * BK, hh);
     } else {
@@ -894,15 +929,11 @@ __global__ __launch_bounds__(NTHREADS, TILE == 256 ? 1 : 2) void grouped_gemm_ke
 
   // ---- fill: steps 0 and 1 of the stream into units 0..3, the first fragments into registers ----
   load_setup();
-#pragma unroll
-  for (int j = 0; j < kParts; ++j) dma_a(0, j);
-#pragma unroll
-  for (int j = 0; j < kParts; ++j) dma_b(1, j);
+  static_for<kParts>([&](auto j) { dma_a(0, j); });
+  static_for<kParts>([&](auto j) { dma_b(1, j); });
   dma_advance();
-#pragma unroll
-  for (int j = 0; j < kParts; ++j) dma_a(2, j);
-#pragma unroll
-  for (int j = 0; j < kParts; ++j) dma_b(3, j);
+  static_for<kParts>([&](auto j) { dma_a(2, j); });
+  static_for<kParts>([&](auto j) { dma_b(3, j); });
   dma_advance();
   FP8GMM_WAIT_VM(2 * kParts);
   __builtin_amdgcn_s_barrier();
@@ -912,10 +943,10 @@ __global__ __launch_bounds__(NTHREADS, TILE == 256 ? 1 : 2) void grouped_gemm_ke
   // some (the planner notes it there): the load stream skips records without K steps, so the fragments read at
   // the end of a tile are those of the next tile that has any
   auto half_height = [](const ItemTile& t) {
-    return TILE == 256 && ((t.nk > 0 ? t.flags : t.flags >> 1) & FP8GMM_ITEM_HALF_HEIGHT) != 0;
+    return TILE == 256 ? as_word(((t.nk > 0 ? t.flags : t.flags >> 1) & FP8GMM_ITEM_HALF_HEIGHT) != 0) : 0;
   };
   ItemTile cp_next = item_tile(0);  // the compute side's next record, fetched ahead like the load side's
-  bool nxt_half = half_height(cp_next);   // height of the tile whose first fragments are in fa0 / fb0
+  const int nxt_half = half_height(cp_next);   // height of the tile whose first fragments are in fa0 / fb0
 #pragma unroll
   for (int i = 0; i < MT; ++i) read_frag_a(fa0[i], lds, i, 0, nxt_half);
   int ua = 0;  // ring unit of the current step's token rows; its weight rows are in the next unit
@@ -959,7 +990,7 @@ __global__ __launch_bounds__(NTHREADS, TILE == 256 ? 1 : 2) void grouped_gemm_ke
   // free: from inside the previous tile's epilogue where that is the staged bf16 form, right after it otherwise.
   // Invariant at the top of the item loop: if the item has K work, those products are under way.
   // (a tile of half height has the products i < MT / 2 only)
-  auto start_tile = [&fb0, &fa0](bool half, bool upper_only = false) {
+  auto start_tile = [&fb0, &fa0](int half, bool upper_only = false) {
     static_for<MT * NT>([&](auto tc) {
       constexpr int i = decltype(tc)::value / NT, j = decltype(tc)::value % NT;
       if ((i >= MT / 2 && half) || (i < MT / 2 && upper_only)) return;
@@ -971,7 +1002,10 @@ __global__ __launch_bounds__(NTHREADS, TILE == 256 ? 1 : 2) void grouped_gemm_ke
   // Where an epilogue cannot take the next tile's products in (every form but the staged bf16 one), it does not
   // have to carry that tile's first fragments through its arithmetic either: they are fetched again afterwards,
   // from the ring units that still hold them, which leaves the epilogue 64 more registers.
-  auto refetch_first_fragments = [&](int unit_a, bool half) {
+  // (kPlain keeps them: its epilogues need no more registers than there are, and fragments that come from two places are
+  // copied to one, 128 vector moves a tile)
+  auto refetch_first_fragments = [&]([[maybe_unused]] int unit_a, [[maybe_unused]] int half) {
+    if constexpr (EPI == kPlain) return;
     const int unit_b = ring_inc(unit_a);
 #pragma unroll
     for (int j = 0; j < NT; ++j) read_frag_b(fb0[j], lds + unit_b * US, j, 0);
@@ -982,23 +1016,31 @@ __global__ __launch_bounds__(NTHREADS, TILE == 256 ? 1 : 2) void grouped_gemm_ke
     const ItemTile g = cp_next;
     if (g.prob < 0) break;
     cp_next = item_tile(r_cp + 1);
-    // only the epilogue needs the problem's record and its scaling factors: the main loop hides the reads
-    const fp8gmm_gemm_problem pr = probs[g.prob];
-    // (two roundings: the factors one by one)
-    const bool two = (epilogue & FP8GMM_EPI_TWO_ROUNDINGS) != 0;
-    const float scale_a = load_scale(pr.a_scale_inv), scale_b = load_scale(pr.b_scale_inv);
-    const float scale_ab = two ? scale_a : scale_a * scale_b;
-    const float scale_c = two ? scale_b : load_scale(pr.c_scale);
+    // Only the epilogue needs the problem's record and its scaling factors.  What the main loop has scalar registers for is the
+    // factors' addresses here, the factors behind the tile's first step, and the rest, in lines that the scalar cache holds by
+    // then, in front of the epilogue.  With everything read here, factors included, a tile began with three reads that wait
+    // for each other, and nothing but the first products under way.
+    const fp8gmm_gemm_problem* const record = probs + g.prob;
+    const float* const a_factor = record->a_scale_inv;
+    const float* const b_factor = record->b_scale_inv;
+    const float* const c_factor = EPI == kPlain ? nullptr : record->c_scale;
+    const int rows = record->m;
+    float scale_a = 1.f, scale_b = 1.f, factor_c = 1.f;
+    auto fetch_factors = [&]() {
+      scale_a = load_scale(a_factor);
+      scale_b = load_scale(b_factor);
+      if constexpr (EPI != kPlain) factor_c = load_scale(c_factor);
+    };
     const int m0 = g.m0, n0 = g.n0;
-    const bool cur_half = TILE == 256 && (g.flags & FP8GMM_ITEM_HALF_HEIGHT) != 0;   // this tile's height
-    bool read_half_next = cur_half;   // height of the tile that the NEXT step belongs to
+    const int cur_half = TILE == 256 ? as_word((g.flags & FP8GMM_ITEM_HALF_HEIGHT) != 0) : 0;   // this tile's height
 
     // One K = 128 step.  `same_item`: the load cursor stays inside its current item after this step (the caller
     // knows), so advancing it is three additions; otherwise the general advance, which may switch items.
     // `half_height_tile`: the sequence for a tile of half height.  The two heights are two kinds of step, each
     // straight-line code: with both sequences inside one step behind a uniform branch, every wait for a fragment
     // after the join becomes a wait for all of them (6 % of a launch).
-    auto k_step = [&](auto same_item, auto first, auto half_height_tile) {
+    // `next_half`: height of the tile that the NEXT step belongs to (where `same_item` leaves that open).
+    auto k_step = [&](auto same_item, auto first, auto half_height_tile, [[maybe_unused]] int next_half) {
       constexpr bool FIRST = decltype(first)::value;
       constexpr bool SAME = decltype(same_item)::value;
       constexpr bool HALF = decltype(half_height_tile)::value;
@@ -1016,46 +1058,46 @@ __global__ __launch_bounds__(NTHREADS, TILE == 256 ? 1 : 2) void grouped_gemm_ke
         // a tile of half height: 8 products per K half, the same loads, three quarters of the fragment reads
         const uint8_t* qa = lds + ua * US;
         const uint8_t* qb = lds + ub * US;
-        dma_a(fa, 0);
+        dma_a(fa, kPart<0>);
         half_b(fb1[0], qb, 0, 1, 0);
         half_b(fb1[0], qb, 0, 1, 1);
         FP8GMM_SB(); FP8GMM_MF0(0, 1); FP8GMM_SB();
-        dma_a(fa, 1);
+        dma_a(fa, kPart<1>);
         half_b(fb1[1], qb, 1, 1, 0);
         half_b(fb1[1], qb, 1, 1, 1);
         FP8GMM_SB(); FP8GMM_MF0(0, 2); FP8GMM_SB();
-        dma_a(fa, 2);
+        dma_a(fa, kPart<2>);
         half_b(fb1[2], qb, 2, 1, 0);
         half_b(fb1[2], qb, 2, 1, 1);
         FP8GMM_SB(); FP8GMM_MF0(0, 3); FP8GMM_SB();
-        dma_a(fa, 3);
+        dma_a(fa, kPart<3>);
         half_b(fb1[3], qb, 3, 1, 0);
         half_b(fb1[3], qb, 3, 1, 1);
         FP8GMM_SB(); FP8GMM_MF0(1, 0); FP8GMM_SB();
-        dma_a(fa, 4);
+        dma_a(fa, kPart<4>);
         half_a(fa1[0], qa, 0, 1, 0, true);
         half_a(fa1[0], qa, 0, 1, 1, true);
         FP8GMM_SB(); FP8GMM_MF0(1, 1); FP8GMM_SB();
-        dma_a(fa, 5);
+        dma_a(fa, kPart<5>);
         half_a(fa1[1], qa, 1, 1, 0, true);
         half_a(fa1[1], qa, 1, 1, 1, true);
         FP8GMM_SB(); FP8GMM_MF0(1, 2); FP8GMM_SB();
-        dma_a(fa, 6);
-        dma_a(fa, 7);
+        dma_a(fa, kPart<6>);
+        dma_a(fa, kPart<7>);
         FP8GMM_SB(); FP8GMM_MF0(1, 3); FP8GMM_SB();
       } else if constexpr (TILE == 128) {
         const uint8_t* qa = lds + ua * US;
         const uint8_t* qb = lds + ub * US;
-        dma_a(fa, 0);
+        dma_a(fa, kPart<0>);
         read_frag_b(fb1[0], qb, 0, 1);
         FP8GMM_SB(); FP8GMM_MF0(0, 1); FP8GMM_SB();
-        dma_a(fa, 1);
+        dma_a(fa, kPart<1>);
         read_frag_b(fb1[1], qb, 1, 1);
         FP8GMM_SB(); FP8GMM_MF0(1, 0); FP8GMM_SB();
-        dma_a(fa, 2);
+        dma_a(fa, kPart<2>);
         read_frag_a(fa1[0], qa, 0, 1);
         FP8GMM_SB(); FP8GMM_MF0(1, 1); FP8GMM_SB();
-        dma_a(fa, 3);
+        dma_a(fa, kPart<3>);
         read_frag_a(fa1[1], qa, 1, 1);
       } else {
         // The fragment reads go out half a fragment at a time, after every MFMA.  A contraction-major operand takes 64
@@ -1064,42 +1106,42 @@ __global__ __launch_bounds__(NTHREADS, TILE == 256 ? 1 : 2) void grouped_gemm_ke
         // two MFMAs the second one can be held back (worth 0.5 % of a launch against that schedule).
         const uint8_t* qa = lds + ua * US;
         const uint8_t* qb = lds + ub * US;
-        dma_a(fa, 0);
+        dma_a(fa, kPart<0>);
         half_b(fb1[0], qb, 0, 1, 0);
         FP8GMM_SB(); FP8GMM_MF0(0, 1); FP8GMM_SB();
         half_b(fb1[0], qb, 0, 1, 1);
         half_b(fb1[1], qb, 1, 1, 0);
         FP8GMM_SB(); FP8GMM_MF0(0, 2); FP8GMM_SB();
-        dma_a(fa, 1);
+        dma_a(fa, kPart<1>);
         half_b(fb1[1], qb, 1, 1, 1);
         FP8GMM_SB(); FP8GMM_MF0(0, 3); FP8GMM_SB();
         half_b(fb1[2], qb, 2, 1, 0);
         half_b(fb1[2], qb, 2, 1, 1);
         FP8GMM_SB(); FP8GMM_MF0(1, 0); FP8GMM_SB();
-        dma_a(fa, 2);
+        dma_a(fa, kPart<2>);
         half_b(fb1[3], qb, 3, 1, 0);
         FP8GMM_SB(); FP8GMM_MF0(1, 1); FP8GMM_SB();
         half_b(fb1[3], qb, 3, 1, 1);
         FP8GMM_SB(); FP8GMM_MF0(1, 2); FP8GMM_SB();
-        dma_a(fa, 3);
+        dma_a(fa, kPart<3>);
         half_a(fa1[0], qa, 0, 1, 0);
         FP8GMM_SB(); FP8GMM_MF0(1, 3); FP8GMM_SB();
         half_a(fa1[0], qa, 0, 1, 1);
         FP8GMM_SB(); FP8GMM_MF0(2, 0); FP8GMM_SB();
-        dma_a(fa, 4);
+        dma_a(fa, kPart<4>);
         half_a(fa1[1], qa, 1, 1, 0);
         FP8GMM_SB(); FP8GMM_MF0(2, 1); FP8GMM_SB();
         half_a(fa1[1], qa, 1, 1, 1);
         FP8GMM_SB(); FP8GMM_MF0(2, 2); FP8GMM_SB();
-        dma_a(fa, 5);
+        dma_a(fa, kPart<5>);
         half_a(fa1[2], qa, 2, 1, 0);
         FP8GMM_SB(); FP8GMM_MF0(2, 3); FP8GMM_SB();
         half_a(fa1[2], qa, 2, 1, 1);
         FP8GMM_SB(); FP8GMM_MF0(3, 0); FP8GMM_SB();
-        dma_a(fa, 6);
+        dma_a(fa, kPart<6>);
         half_a(fa1[3], qa, 3, 1, 0);
         FP8GMM_SB(); FP8GMM_MF0(3, 1); FP8GMM_SB();
-        dma_a(fa, 7);
+        dma_a(fa, kPart<7>);
         half_a(fa1[3], qa, 3, 1, 1);
         FP8GMM_SB(); FP8GMM_MF0(3, 2); FP8GMM_MF0(3, 3); FP8GMM_SB();
       }
@@ -1119,38 +1161,38 @@ __global__ __launch_bounds__(NTHREADS, TILE == 256 ? 1 : 2) void grouped_gemm_ke
         // fragments, addressed as the tile of that step wants them (a tile of full height may follow)
         const uint8_t* qa = lds + na * US;
         const uint8_t* qb = lds + nb * US;
-        const bool nh = SAME ? true : read_half_next;
+        const int nh = SAME ? 1 : next_half;
         FP8GMM_SB(); FP8GMM_MF1(0, 0); FP8GMM_SB();
-        dma_b(ua, 0);
+        dma_b(ua, kPart<0>);
         half_b(fb0[0], qb, 0, 0, 0);
         half_b(fb0[0], qb, 0, 0, 1);
         FP8GMM_SB(); FP8GMM_MF1(0, 1); FP8GMM_SB();
-        dma_b(ua, 1);
+        dma_b(ua, kPart<1>);
         half_b(fb0[1], qb, 1, 0, 0);
         half_b(fb0[1], qb, 1, 0, 1);
         FP8GMM_SB(); FP8GMM_MF1(0, 2); FP8GMM_SB();
-        dma_b(ua, 2);
+        dma_b(ua, kPart<2>);
         half_b(fb0[2], qb, 2, 0, 0);
         half_b(fb0[2], qb, 2, 0, 1);
         FP8GMM_SB(); FP8GMM_MF1(0, 3); FP8GMM_SB();
-        dma_b(ua, 3);
+        dma_b(ua, kPart<3>);
         half_b(fb0[3], qb, 3, 0, 0);
         half_b(fb0[3], qb, 3, 0, 1);
         FP8GMM_SB(); FP8GMM_MF1(1, 0); FP8GMM_SB();
-        dma_b(ua, 4);
+        dma_b(ua, kPart<4>);
         half_a(fa0[0], qa, 0, 0, 0, nh);
         half_a(fa0[0], qa, 0, 0, 1, nh);
         FP8GMM_SB(); FP8GMM_MF1(1, 1); FP8GMM_SB();
-        dma_b(ua, 5);
+        dma_b(ua, kPart<5>);
         half_a(fa0[1], qa, 1, 0, 0, nh);
         half_a(fa0[1], qa, 1, 0, 1, nh);
         FP8GMM_SB(); FP8GMM_MF1(1, 2); FP8GMM_SB();
-        dma_b(ua, 6);
+        dma_b(ua, kPart<6>);
         if constexpr (!SAME) {
           half_a(fa0[2], qa, 2, 0, 0, nh);
           half_a(fa0[2], qa, 2, 0, 1, nh);
         }
-        dma_b(ua, 7);
+        dma_b(ua, kPart<7>);
         if constexpr (!SAME) {
           half_a(fa0[3], qa, 3, 0, 0, nh);
           half_a(fa0[3], qa, 3, 0, 1, nh);
@@ -1159,59 +1201,59 @@ __global__ __launch_bounds__(NTHREADS, TILE == 256 ? 1 : 2) void grouped_gemm_ke
         const uint8_t* qa = lds + na * US;
         const uint8_t* qb = lds + nb * US;
         FP8GMM_SB(); FP8GMM_MF1(0, 0); FP8GMM_SB();
-        dma_b(ua, 0);
+        dma_b(ua, kPart<0>);
         read_frag_b(fb0[0], qb, 0, 0);
         FP8GMM_SB(); FP8GMM_MF1(0, 1); FP8GMM_SB();
-        dma_b(ua, 1);
+        dma_b(ua, kPart<1>);
         read_frag_b(fb0[1], qb, 1, 0);
         FP8GMM_SB(); FP8GMM_MF1(1, 0); FP8GMM_SB();
-        dma_b(ua, 2);
+        dma_b(ua, kPart<2>);
         read_frag_a(fa0[0], qa, 0, 0);
         FP8GMM_SB(); FP8GMM_MF1(1, 1); FP8GMM_SB();
-        dma_b(ua, 3);
+        dma_b(ua, kPart<3>);
         read_frag_a(fa0[1], qa, 1, 0);
       } else {
         const uint8_t* qa = lds + na * US;
         const uint8_t* qb = lds + nb * US;
         // (after a step that may end its item, the next step's tile may be of half height)
-        const bool nh = decltype(same_item)::value ? false : read_half_next;
+        const int nh = SAME ? 0 : next_half;
         FP8GMM_SB(); FP8GMM_MF1(0, 0); FP8GMM_SB();
-        dma_b(ua, 0);
+        dma_b(ua, kPart<0>);
         half_b(fb0[0], qb, 0, 0, 0);
         FP8GMM_SB(); FP8GMM_MF1(0, 1); FP8GMM_SB();
         half_b(fb0[0], qb, 0, 0, 1);
         half_b(fb0[1], qb, 1, 0, 0);
         FP8GMM_SB(); FP8GMM_MF1(0, 2); FP8GMM_SB();
-        dma_b(ua, 1);
+        dma_b(ua, kPart<1>);
         half_b(fb0[1], qb, 1, 0, 1);
         FP8GMM_SB(); FP8GMM_MF1(0, 3); FP8GMM_SB();
         half_b(fb0[2], qb, 2, 0, 0);
         half_b(fb0[2], qb, 2, 0, 1);
         FP8GMM_SB(); FP8GMM_MF1(1, 0); FP8GMM_SB();
-        dma_b(ua, 2);
+        dma_b(ua, kPart<2>);
         half_b(fb0[3], qb, 3, 0, 0);
         FP8GMM_SB(); FP8GMM_MF1(1, 1); FP8GMM_SB();
         half_b(fb0[3], qb, 3, 0, 1);
         FP8GMM_SB(); FP8GMM_MF1(1, 2); FP8GMM_SB();
-        dma_b(ua, 3);
+        dma_b(ua, kPart<3>);
         half_a(fa0[0], qa, 0, 0, 0, nh);
         FP8GMM_SB(); FP8GMM_MF1(1, 3); FP8GMM_SB();
         half_a(fa0[0], qa, 0, 0, 1, nh);
         FP8GMM_SB(); FP8GMM_MF1(2, 0); FP8GMM_SB();
-        dma_b(ua, 4);
+        dma_b(ua, kPart<4>);
         half_a(fa0[1], qa, 1, 0, 0, nh);
         FP8GMM_SB(); FP8GMM_MF1(2, 1); FP8GMM_SB();
         half_a(fa0[1], qa, 1, 0, 1, nh);
         FP8GMM_SB(); FP8GMM_MF1(2, 2); FP8GMM_SB();
-        dma_b(ua, 5);
+        dma_b(ua, kPart<5>);
         half_a(fa0[2], qa, 2, 0, 0, nh);
         FP8GMM_SB(); FP8GMM_MF1(2, 3); FP8GMM_SB();
         half_a(fa0[2], qa, 2, 0, 1, nh);
         FP8GMM_SB(); FP8GMM_MF1(3, 0); FP8GMM_SB();
-        dma_b(ua, 6);
+        dma_b(ua, kPart<6>);
         half_a(fa0[3], qa, 3, 0, 0, nh);
         FP8GMM_SB(); FP8GMM_MF1(3, 1); FP8GMM_SB();
-        dma_b(ua, 7);
+        dma_b(ua, kPart<7>);
         half_a(fa0[3], qa, 3, 0, 1, nh);
       }
       // common to every sequence: the load cursor moves on (in the shadow of the step's last products)
@@ -1232,55 +1274,73 @@ __global__ __launch_bounds__(NTHREADS, TILE == 256 ? 1 : 2) void grouped_gemm_ke
     // next step lies in the same item.
     // The token fragments that a tile's LAST step reads belong to the next tile with K steps, and are addressed by
     // that tile's height.
-    const bool after_half = half_height(cp_next);
+    // (formed where it is wanted: at the top of the tile the next record is still on its way)
+    auto after_half = [&]() { return half_height(cp_next); };
     // One run of steps per height, one after the other, the run of the other height with no steps: as alternatives
     // behind a branch, the compiler carries the load cursor's scalar state (descriptors, LDS addresses) through the
     // join in vector registers, which the LDS-DMA statements cannot take.
     auto steps = [&](int nk, auto half_c) {
       int kt = 0;
       if (nk > 0) {
-        if (nk == 1) read_half_next = after_half;
-        k_step(std::false_type{}, std::true_type{}, half_c);
+        k_step(std::false_type{}, std::true_type{}, half_c, nk == 1 ? after_half() : (int)half_c());
+        fetch_factors();
         kt = 1;
       }
-      for (; kt + 3 < nk; ++kt) k_step(std::true_type{}, std::false_type{}, half_c);
-      for (; kt < nk; ++kt) {
-        if (kt == nk - 1) read_half_next = after_half;
-        k_step(std::false_type{}, std::false_type{}, half_c);
-      }
+      for (; kt + 3 < nk; ++kt) k_step(std::true_type{}, std::false_type{}, half_c, 0);
+      for (; kt < nk; ++kt) k_step(std::false_type{}, std::false_type{}, half_c, kt == nk - 1 ? after_half() : (int)half_c());
     };
-    if (g.nk == 0) static_for<MT * NT>([&](auto tc) { acc_tile_clear<16 * decltype(tc)::value>(); });
+    if (g.nk == 0) {
+      static_for<MT * NT>([&](auto tc) { acc_tile_clear<16 * decltype(tc)::value>(); });
+      fetch_factors();
+    }
     steps(cur_half ? 0 : g.nk, std::false_type{});
     if constexpr (TILE == 256) steps(cur_half ? g.nk : 0, std::true_type{});
     // ---- epilogue ----
-    uint8_t* const stage = lds + ((ua + 4) % RING) * US;  // free until the next step's token loads
+    fp8gmm_gemm_problem pr{};
+    pr.c = record->c;
+    pr.m = rows;
+    pr.n = record->n;
+    pr.ldc = record->ldc;
+    if constexpr (EPI != kPlain) {
+      pr.aux = record->aux;
+      pr.c_amax = record->c_amax;
+    }
+    // (from here on, and not earlier, the compiler may compute with the factors: that is where their reads are waited for)
+    asm volatile("" : "+s"(scale_a), "+s"(scale_b), "+s"(factor_c));
+    // (two roundings: the factors one by one)
+    const bool two = (epilogue & FP8GMM_EPI_TWO_ROUNDINGS) != 0;
+    const float scale_ab = two ? scale_a : scale_a * scale_b;
+    const float scale_c = two ? scale_b : factor_c;
+    uint8_t* const stage = lds + (ua == 0 ? RING - 1 : ua - 1) * US;  // free until the next step's token loads
     const bool more = cp_next.prob >= 0 && cp_next.nk > 0;  // the fragments in fa0 / fb0 open another tile
     const int mt = cur_half ? MT / 2 : MT;                  // 32-row blocks of this tile per wavefront
+    const int then_half = after_half();
+    const bool staged = staged_bf16_tile<TILE>(pr, m0, n0, out_kind, epilogue);
     if (g.slot >= 0) {
       // a piece of a tile that is shared along K: leave the accumulators for the fix-up kernel
       partial_store<TILE>(workspace + (size_t)g.slot * kPartialBytes);
       relaxed = 0;
       if (more) {
-        refetch_first_fragments(ua, after_half);
-        start_tile(after_half);
+        refetch_first_fragments(ua, then_half);
+        start_tile(then_half);
       }
-    } else if (more && staged_bf16_tile<TILE>(pr, m0, n0, out_kind, epilogue)) {
+    } else if (more && staged) {
       // the next tile's first products go out as the accumulators they overwrite are read out, in the shadow of
       // the epilogue's vector arithmetic
-      relaxed = tile_epilogue<TILE>(pr, m0, n0, out_kind, epilogue, stage, mt, !A_TR && !B_TR, !A_TR, scale_ab, scale_c,
-                                    [&fb0, &fa0, after_half](auto ic, auto jc) {
+      relaxed = tile_epilogue<TILE, EPI>(pr, m0, n0, out_kind, epilogue, true, stage, mt, !A_TR && !B_TR, !A_TR, scale_ab, scale_c,
+                                    [&fb0, &fa0, then_half](auto ic, auto jc) {
                                       constexpr int i = decltype(ic)::value, j = decltype(jc)::value;
-                                      if (i >= MT / 2 && after_half) return;
+                                      if (i >= MT / 2 && then_half) return;
                                       const i32x8 wf = fb0[j], tf = fa0[i];
                                       FP8GMM_MFMA_Z(i, j, wf, tf);
                                     });
       // a tile of half height released the lower blocks only
-      if (cur_half && !after_half) start_tile(false, true);
+      if (cur_half && !then_half) start_tile(false, true);
     } else {
-      relaxed = tile_epilogue<TILE>(pr, m0, n0, out_kind, epilogue, stage, mt, !A_TR && !B_TR, !A_TR, scale_ab, scale_c);
+      relaxed = tile_epilogue<TILE, EPI>(pr, m0, n0, out_kind, epilogue, staged, stage, mt, !A_TR && !B_TR, !A_TR, scale_ab, scale_c);
       if (more) {
-        refetch_first_fragments(ua, after_half);
-        start_tile(after_half);
+        refetch_first_fragments(ua, then_half);
+        start_tile(then_half);
       }
     }
   }
@@ -1310,14 +1370,15 @@ int prepare_variant(int dev) {
   static std::atomic<bool> attr_set[kMaxDevices];
   if (dev < 0 || dev >= kMaxDevices) return FP8GMM_ERR_NO_DEVICE;
   if (!attr_set[dev].load(std::memory_order_acquire)) {
-    const void* kernels[2] = {};
+    const void* kernels[2] = {};   // of one form: two kinds of epilogue
     int lds_bytes = 0;
     if constexpr (TILE == kTileDual) {
       kernels[0] = reinterpret_cast<const void*>(grouped_gemm_dual_kernel<A_FMT, B_FMT, A_TR, B_TR, false>);
       kernels[1] = reinterpret_cast<const void*>(grouped_gemm_dual_kernel<A_FMT, B_FMT, A_TR, B_TR, true>);
       lds_bytes = RING * BN * BK;
     } else {
-      kernels[0] = reinterpret_cast<const void*>(grouped_gemm_kernel<A_FMT, B_FMT, A_TR, B_TR, TILE>);
+      kernels[0] = reinterpret_cast<const void*>(grouped_gemm_kernel<A_FMT, B_FMT, A_TR, B_TR, TILE, kPlain>);
+      kernels[1] = reinterpret_cast<const void*>(grouped_gemm_kernel<A_FMT, B_FMT, A_TR, B_TR, TILE, kAny>);
       lds_bytes = RING * TILE * BK;
     }
     for (const void* kernel : kernels)
@@ -1346,8 +1407,14 @@ int launch_variant(const fp8gmm_gemm_problem* probs_dev, const fp8gmm_gemm_item*
       hipLaunchKernelGGL((grouped_gemm_dual_kernel<A_FMT, B_FMT, A_TR, B_TR, false>), dim3(grid), dim3(NTHREADS),
                          RING * BN * BK, stream, probs_dev, items_dev, merge_descs, merge_n);
   } else {
-    hipLaunchKernelGGL((grouped_gemm_kernel<A_FMT, B_FMT, A_TR, B_TR, TILE>), dim3(grid), dim3(NTHREADS),
-                       RING * TILE * BK, stream, probs_dev, items_dev, out_kind, epilogue, workspace, merge_descs, merge_n);
+    // The kernel that knows every kind of result keeps their constants and scalars in registers through the main loop, and
+    // is nine tenths epilogues; plain results, nearly all launches, have one of their own.
+    if (out_kind == FP8GMM_OUT_BF16 && !(epilogue & (FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU)))
+      hipLaunchKernelGGL((grouped_gemm_kernel<A_FMT, B_FMT, A_TR, B_TR, TILE, kPlain>), dim3(grid), dim3(NTHREADS),
+                         RING * TILE * BK, stream, probs_dev, items_dev, out_kind, epilogue, workspace, merge_descs, merge_n);
+    else
+      hipLaunchKernelGGL((grouped_gemm_kernel<A_FMT, B_FMT, A_TR, B_TR, TILE, kAny>), dim3(grid), dim3(NTHREADS),
+                         RING * TILE * BK, stream, probs_dev, items_dev, out_kind, epilogue, workspace, merge_descs, merge_n);
   }
   return hipGetLastError() == hipSuccess ? FP8GMM_OK : FP8GMM_ERR_LAUNCH;
 }

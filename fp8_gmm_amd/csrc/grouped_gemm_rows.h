@@ -133,15 +133,14 @@ __global__ __launch_bounds__(NTHREADS, 2) void grouped_gemm_rows_kernel(
   int ld_kt = 0, ld_nk = 0, ld_kmax = 0;
   i32x4 rsrc_a = {0, 0, 0, 0x00020000}, rsrc_b = {0, 0, 0, 0x00020000};
   uint32_t a_base = 0, b_base = 0, a_step = 0, b_step = 0;
-  auto load_setup = [&]() {
+  auto load_setup = [&]() {   // the record after this one is fetched last, as in grouped_gemm_kernel
     for (;;) {
-      const ItemLoad gl = ld_next_l;
-      const ItemTile gt = ld_next_t;
+      const ItemLoad& gl = ld_next_l;
+      const ItemTile& gt = ld_next_t;
       ld_live = gt.prob >= 0;
       if (!ld_live) break;
-      ld_next_l = item_load(r_ld + 1);   // every list ends with an end record
-      ld_next_t = item_tile(r_ld + 1);
-      if (gt.nk > 0) {
+      const bool take = gt.nk > 0;   // an item without K work needs no loads
+      if (take) {
         rsrc_a[0] = (int)(uint32_t)gl.a;
         rsrc_a[1] = (int)(uint32_t)(gl.a >> 32);
         rsrc_a[2] = (int)gl.a_bytes;
@@ -155,9 +154,12 @@ __global__ __launch_bounds__(NTHREADS, 2) void grouped_gemm_rows_kernel(
         ld_kmax = gt.k - dchunk * 16;
         ld_kt = gt.k_begin;
         ld_nk = gt.k_begin + gt.nk;
-        return;
       }
-      ++r_ld;   // an item without K work needs no loads
+      FP8GMM_RECORD_USED(gt);
+      ++r_ld;   // every list ends with an end record
+      ld_next_l = item_load(r_ld);
+      ld_next_t = item_tile(r_ld);
+      if (take) return;
     }
     // past the end of the stream: zero fill from empty descriptors, which keeps the vmcnt arithmetic uniform
     rsrc_a[2] = 0;
@@ -176,12 +178,9 @@ __global__ __launch_bounds__(NTHREADS, 2) void grouped_gemm_rows_kernel(
 #pragma unroll
     for (int j = 0; j < kPartsA; ++j) {
       const uint32_t v = k_ok ? a_base + k0 + j * a_step : 0xffffffffu;
-      FP8GMM_DMA(dst + NWAVES * j * 1024, v, rsrc_a);
+      FP8GMM_DMA(dst + NWAVES * j * 1024, 0, v, rsrc_a);
     }
-    if (ld_live && ++ld_kt == ld_nk) {
-      ++r_ld;
-      load_setup();
-    }
+    if (ld_live && ++ld_kt == ld_nk) load_setup();
   };
   auto read_frag = [&](const uint8_t* base, int hh) {
     const u32x4 lo = *reinterpret_cast<const u32x4*>(base + fc[hh][0]);
