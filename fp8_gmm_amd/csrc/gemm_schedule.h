@@ -55,6 +55,7 @@ struct Sched {
   int sk_wgs;                  // workgroups that take a piece of the region
   int64_t sk_c0, sk_cost;      // cost before the region, cost of the region (K = 128 steps)
   int64_t total_cost;          // cost of all tiles
+  bool halves;                 // the remainder [sk_begin, range_end) in tiles of half height, two per tile (sk_wgs is 0)
   bool gelu;                   // completing a shared tile includes the GELU epilogue
 };
 
@@ -129,6 +130,21 @@ FP8GMM_HD int dp_tile(const Sched& s, int j, int i) {
   return s.range_begin + s.wgs * i + (j + kRoundRotation * i) % s.wgs;
 }
 
+// ---- a last round of tiles of half height ----
+// A remainder of at most half a round leaves half of the workgroups without a tile while the others run a whole one.  Cut
+// into two items of half height (FP8GMM_ITEM_HALF_HEIGHT) it takes them kHalfStep / 100 of a step's time per K step and
+// kHalfTile / 100 steps for the result and the switch; no partial sums, no second launch.  Timed inside the kernel, 8 experts,
+// K = N = 4096, 8192 rows (2.25 rounds): whole tiles 43, 40 and, eight of them on 32 workgroups, 29 us; those as halves 20.
+// Halves between whole tiles take 0.62 of their time, but a last round of halves is a quarter of the traffic and a half of
+// the workgroups of a round, and its whole tiles would have run at 0.7: 75 is what separates the launches that gain from
+// those that are better off shared along K (K = 14336, 4.25 rounds: shared 710, halves 743).
+constexpr int kHalfStep = 75;
+constexpr int kHalfTile = 300;
+constexpr int kHalfMaxRounds = 12;    // with more full rounds than this a last round is not worth the look
+inline int64_t half_tile_x100(int64_t steps) { return steps * kHalfStep + kHalfTile; }
+// Workgroup j's item of the round behind `full` whole ones: which tile of the remainder, and which half of it.
+FP8GMM_HD int half_position(int wgs, int j, int full) { return (j + kRoundRotation * full) % wgs; }
+
 // One way to share a remainder: so many equal pieces, and the workspace slots that they leave.
 struct SkSplit {
   int pieces, slots;
@@ -140,7 +156,8 @@ struct SkRemainder {
   int64_t c0, cost;      // cost before it, its own
   int n_splits;          // 0: not worth a thought
   SkSplit split[kSkMaxPieces];
-  int64_t whole_x100, shared_x100[kSkMaxPieces];
+  int64_t whole_x100, shared_x100[kSkMaxPieces], half_x100;
+  bool timed, halves;    // the times above are there; the remainder is better off in tiles of half height (whole_x100 says so)
 };
 
 // A tile that k piece ends fall inside of is left in k + 1 slots; one that no end falls inside of needs none.
@@ -201,10 +218,13 @@ inline void sk_splits(const Sched& s, SkRemainder& r) {
 // Under one K the workgroups come to the remainder together; otherwise one that its whole tiles keep longer than the others
 // begins later, and whether it gets a tile, a piece or nothing of the remainder decides when the range is through.
 inline void sk_times(const Sched& s, SkRemainder& r) {
+  if (r.timed) return;
+  r.timed = true;
   const int W = s.wgs, full = (s.range_end - s.range_begin) / W;
   if (range_has_one_k(s)) {
-    const int64_t round = tile_cost(s, problem_of_tile(s, s.range_begin)) + kTileOverhead;
+    const int64_t steps = tile_cost(s, problem_of_tile(s, s.range_begin)), round = steps + kTileOverhead;
     r.whole_x100 = (full + (r.tiles > 0 ? 1 : 0)) * round * 100;
+    r.half_x100 = full * round * 100 + half_tile_x100(steps);
     for (int i = 0; i < r.n_splits; ++i)
       r.shared_x100[i] = (full * round + kTileOverhead) * 100 + r.cost * 100 / r.split[i].pieces;
     return;
@@ -233,6 +253,13 @@ inline void sk_times(const Sched& s, SkRemainder& r) {
   int64_t longest = 0;
   for (const int64_t l : load) longest = longest < l ? l : longest;
   r.whole_x100 = (longest < last ? last : longest) * 100;
+  r.half_x100 = longest * 100;
+  for (int j = 0; j < W; ++j) {
+    const int at = r.begin + half_position(W, j, full) / 2;
+    if (at >= s.range_end) continue;
+    const int64_t through = (j < workgroups ? load[j] * 100 : 0) + half_tile_x100(tile_cost(s, problem_of_tile(s, at)));
+    if (r.half_x100 < through) r.half_x100 = through;
+  }
   int64_t first = 0;   // the longest of the workgroups that get a piece
   for (int i = 0, j = 0; i < r.n_splits; ++i) {
     for (; j < r.split[i].pieces && j < workgroups; ++j) first = first < load[j] ? load[j] : first;
@@ -309,12 +336,13 @@ inline void sk_decide(const Sched (&all)[kNumXcd], SkRemainder (&rem)[kNumXcd], 
 // tile costs its K steps plus a fixed part (epilogue, tile switch) worth about kTileOverhead steps: balancing
 // K steps alone left the XCDs that hold the short-K problems 17 % more work than the others.
 inline void sched_init(Sched (&all)[kNumXcd], const fp8gmm_gemm_problem* probs, int nprob, int total_tiles, int wgs_per_xcd,
-                       bool sk_enable, bool gelu = false) {
+                       bool sk_enable, bool gelu = false, bool half_tail = false) {
   const int W = wgs_per_xcd;
   SkRemainder rem[kNumXcd];
   for (int x = 0; x < kNumXcd; ++x) {
     Sched& s = all[x];
     s.gelu = gelu;
+    s.halves = false;
     s.probs = probs;
     s.nprob = nprob;
     s.total_tiles = total_tiles;
@@ -332,19 +360,33 @@ inline void sched_init(Sched (&all)[kNumXcd], const fp8gmm_gemm_problem* probs, 
     SkRemainder& r = rem[x];
     r.n_splits = 0;
     r.whole_x100 = 0;
+    r.timed = r.halves = false;
     r.tiles = n_x % W;
     r.begin = s.range_end - r.tiles;
+    if (half_tail && r.tiles > 0 && 2 * r.tiles <= W && n_x / W <= kHalfMaxRounds) {
+      sk_times(s, r);
+      if (r.half_x100 < r.whole_x100) {
+        r.halves = true;
+        r.whole_x100 = r.half_x100;
+      }
+    }
     if (!sk_enable || !remainder_may_share(n_x, W)) continue;
     r.c0 = cost_before(s, r.begin);
     r.cost = cost_before(s, s.range_end) - r.c0;
     sk_splits(s, r);
   }
-  if (!sk_enable) return;
-  int pieces[kNumXcd];
-  sk_decide(all, rem, pieces);
+  int pieces[kNumXcd] = {};
+  if (sk_enable) sk_decide(all, rem, pieces);
   for (int x = 0; x < kNumXcd; ++x) {
-    if (pieces[x] == 0) continue;
     Sched& s = all[x];
+    if (pieces[x] == 0) {
+      if (rem[x].halves) {
+        s.halves = true;
+        s.dp_rounds = (s.range_end - s.range_begin) / W;
+        s.sk_begin = rem[x].begin;
+      }
+      continue;
+    }
     s.dp_rounds = (s.range_end - s.range_begin) / W;
     s.sk_begin = rem[x].begin;
     s.sk_wgs = pieces[x];

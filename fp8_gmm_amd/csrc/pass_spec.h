@@ -67,7 +67,7 @@ struct GemmRanges {
   struct Xcd {
     int32_t begin, end;      // tiles of the XCD's range
     int32_t dp_rounds;
-    int32_t sk_begin, sk_wgs, sk_c0, sk_cost;
+    int32_t sk_begin, sk_wgs, sk_c0, sk_cost;   // sk_wgs -1: the tiles from sk_begin on as two items of half height each
   } xcd[kNumXcd];
 };
 

@@ -191,13 +191,20 @@ __device__ void write_gemm(const PassTables& t, int g, int block, uint8_t* blob,
   const int own = index / ranges.grid;
 #pragma unroll 1
   for (int round = own;; ++round) {
-    int tile = -1, p = 0, k_begin = 0, nk = -1, slot = -1;
+    int tile = -1, p = 0, k_begin = 0, nk = -1, slot = -1, half = -1;
     if (!gm.large) {
       const int whole = xc.begin + whole_tile_of(gm.wgs, j, round);
       if (whole < xc.end) tile = whole;
     } else if (round < xc.dp_rounds) {   // only the last strided round can be partial, and then nothing is shared
       const int whole = xc.begin + gm.wgs * round + (j + kRoundRotation * round) % gm.wgs;
       if (whole < xc.sk_begin) tile = whole;
+    } else if (xc.sk_wgs < 0) {
+      // a last round of half tiles: two positions per tile; a tile of at most half height takes the first one
+      const int position = half_position(gm.wgs, j, round), pair = xc.sk_begin + position / 2;
+      if (round == xc.dp_rounds && pair < xc.end) {
+        tile = pair;
+        half = position % 2;
+      }
     } else if (j < xc.sk_wgs) {
       // the tiles under piece j of the shared remainder
       const int lo = gm.bound(xc, j), hi = gm.bound(xc, j + 1);
@@ -230,9 +237,11 @@ __device__ void write_gemm(const PassTables& t, int g, int block, uint8_t* blob,
     }
     int m0 = 0, n0 = 0;
     tile_origin(probs[p].m, probs[p].n, tile - begin[p], spec.tile_m, spec.tile_n, &m0, &n0);
-    const int flags = gm.large && slot < 0 && probs[p].m - m0 <= BM / 2 ? FP8GMM_ITEM_HALF_HEIGHT : 0;
+    if (half > 0) m0 += BM / 2;
+    if (m0 >= probs[p].m) break;
+    const int flags = gm.large && slot < 0 && (half >= 0 || probs[p].m - m0 <= BM / 2) ? FP8GMM_ITEM_HALF_HEIGHT : 0;
     if (round == own) {
-      o = gemm_item(probs[p], p, m0, n0, spec.tile_m, spec.tile_n, (spec.layout & FP8GMM_GEMM_A_KMAJOR) != 0,
+      o = gemm_item(probs[p], p, m0, n0, half >= 0 ? BM / 2 : spec.tile_m, spec.tile_n, (spec.layout & FP8GMM_GEMM_A_KMAJOR) != 0,
                     (spec.layout & FP8GMM_GEMM_B_KMAJOR) != 0, k_begin, nk, slot);
       o.flags = flags;
       if (nk > 0 || !gm.large) break;

@@ -300,11 +300,12 @@ static int plan_whole_tiles(const int TM, const int TN, const int kOverhead, fp8
 
 // Tail balancing can only pay when the launch has few rounds; it needs the whole grid even for few tiles.  Without it
 // the grid shrinks to the tiles there are.
-static bool share_tail(int stream_k, int total_tiles, int* grid) {
+// So does a last round of half tiles.
+static bool share_tail(int stream_k, int total_tiles, bool half_tail, int* grid) {
   using namespace fp8gmm;
   if (stream_k != 0 && (int64_t)total_tiles <= (int64_t)kSkMaxRounds * *grid && *grid > kNumXcd) return true;
   const int needed = ((total_tiles + kNumXcd - 1) / kNumXcd) * kNumXcd;
-  if (*grid > needed) *grid = needed;
+  if (*grid > needed && !half_tail) *grid = needed;
   return false;
 }
 
@@ -325,20 +326,21 @@ int fp8gmm_plan_grouped_gemm_launch(fp8gmm_gemm_problem* probs, int n, int layou
   const int layout_given = layout, grid_given = grid;
   // the epilogue flags only weigh the decision to share tiles along K (completing a tile costs more with them)
   const bool gelu = (layout & (FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU)) != 0;
-  layout &= ~(FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU);
+  const bool half_tail = (layout & FP8GMM_GEMM_HALF_TAIL) != 0;
+  layout &= ~(FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU | FP8GMM_GEMM_HALF_TAIL);
   int total_tiles = 0;
   const int rc = fp8gmm_plan_grouped_gemm_layout(probs, n, layout, &total_tiles);
   if (rc != FP8GMM_OK) return rc;
   plan->total_tiles = total_tiles;
   if (total_tiles == 0) return FP8GMM_OK;
-  const bool sk = share_tail(stream_k, total_tiles, &grid);
+  const bool sk = share_tail(stream_k, total_tiles, half_tail, &grid);
   const int wgs = grid / kNumXcd;
   const bool a_kmajor = (layout & FP8GMM_GEMM_A_KMAJOR) != 0, b_kmajor = (layout & FP8GMM_GEMM_B_KMAJOR) != 0;
 
   // pass 1: sizes.  The tiles that were shared along K first: the pieces of such a tile get consecutive
   // workspace slots, numbered from 0 over the launch, in K order.
   Sched sched[kNumXcd];
-  sched_init(sched, probs, n, total_tiles, wgs, sk, gelu);
+  sched_init(sched, probs, n, total_tiles, wgs, sk, gelu, half_tail);
   std::vector<int32_t> slot_map((size_t)kSlotsPerWg * grid, -1);
   std::vector<fp8gmm_gemm_fixup_desc> fix;
   int n_slots = 0;
@@ -450,6 +452,25 @@ int fp8gmm_plan_grouped_gemm_launch(fp8gmm_gemm_problem* probs, int n, int layou
       prob = it.prob;
       write_record(it, index);
     }
+    if (sx.halves) {   // behind full rounds only
+      const int position = half_position(wgs, j, sx.dp_rounds), tile = sx.sk_begin + position / 2;
+      if (tile < sx.range_end) {
+        const int p = problem_of_tile(sx, tile);
+        const fp8gmm_gemm_problem& pr = probs[p];
+        int m0 = 0, n0 = 0;
+        tile_origin(pr.m, pr.n, tile - pr.tile_begin, &m0, &n0);
+        m0 += position % 2 * (BM / 2);
+        if (m0 < pr.m) {
+          const size_t index = (size_t)r * grid + wg;
+          if (index < (size_t)max_items) {
+            fp8gmm_gemm_item o = gemm_item(pr, p, m0, n0, BM / 2, BN, a_kmajor, b_kmajor, 0, (pr.k + 127) / 128, -1);
+            o.flags = FP8GMM_ITEM_HALF_HEIGHT;
+            items[index] = o;
+          }
+          ++r;
+        }
+      }
+    }
     count[wg] = r;
     if (r > rounds) rounds = r;
   }
@@ -509,15 +530,17 @@ int plan_gemm_ranges(fp8gmm_gemm_problem* probs, int n, int layout, int grid, in
     const bool gelu = (layout & (FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU)) != 0;
     plan->tile = kGemmTileM;
     int total_tiles = 0;
-    const int rc = fp8gmm_plan_grouped_gemm_layout(probs, n, layout & ~(FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU), &total_tiles);
+    const bool half_tail = (layout & FP8GMM_GEMM_HALF_TAIL) != 0;
+    const int rc = fp8gmm_plan_grouped_gemm_layout(
+        probs, n, layout & ~(FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU | FP8GMM_GEMM_HALF_TAIL), &total_tiles);
     if (rc != FP8GMM_OK) return rc;
     plan->total_tiles = total_tiles;
     if (total_tiles == 0) return FP8GMM_OK;
-    const bool sk = share_tail(stream_k, total_tiles, &grid);
+    const bool sk = share_tail(stream_k, total_tiles, half_tail, &grid);
     const int wgs = grid / kNumXcd;
     plan->grid = grid;
     Sched sched[kNumXcd];
-    sched_init(sched, probs, n, total_tiles, wgs, sk, gelu);
+    sched_init(sched, probs, n, total_tiles, wgs, sk, gelu, half_tail);
     for (int x = 0; x < kNumXcd; ++x) {
       const Sched& s = sched[x];
       GemmRanges::Xcd& o = out->xcd[x];
@@ -525,11 +548,11 @@ int plan_gemm_ranges(fp8gmm_gemm_problem* probs, int n, int layout, int grid, in
       o.end = s.range_end;
       o.dp_rounds = s.dp_rounds;
       o.sk_begin = s.sk_begin;
-      o.sk_wgs = s.sk_wgs;
+      o.sk_wgs = s.halves ? -1 : s.sk_wgs;
       o.sk_c0 = (int32_t)s.sk_c0;
       o.sk_cost = (int32_t)s.sk_cost;
       out->total_cost = (int32_t)s.total_cost;
-      int rounds = s.dp_rounds;
+      int rounds = s.dp_rounds + (s.halves ? 1 : 0);
       for (int j = 0; j < s.sk_wgs; ++j) {
         // with a shared remainder every strided round is full: the pieces of workgroup j follow its dp_rounds tiles
         Cursor c;

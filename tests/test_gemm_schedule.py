@@ -468,3 +468,61 @@ def test_slot_cap_falls_back_to_whole_tiles():
     short, items_short, fix_short = _lib.plan_grouped_gemm_launch(table.copy(), 0, 256, free.n_slots - 1)
     assert (short.n_slots, short.n_fixups, len(fix_short)) == (0, 0, 0) and short.rounds == whole.rounds
     assert items_short.tobytes() == items_whole.tobytes()
+
+
+def half_tail_cases():
+    rng = np.random.default_rng(5)
+    yield [(8192, 4096, 4096)], 0                                 # 512 tiles: two whole rounds, nothing to cut
+    yield [(1100, 4096, 4096)] * 6 + [(100, 4096, 4096)] * 2, 0    # ragged last rows of tiles inside the remainder
+    yield [(256 * 9, 1024, 512)], 0                               # less than a round
+    yield [(300, 512, 0), (2304, 1024, 256)], 0                   # tiles without K work in front
+    wgrad = _lib.GEMM_A_KMAJOR | _lib.GEMM_B_KMAJOR
+    yield [(1408, 2048, int(k)) for k in rng.integers(0, 900, 9)], wgrad
+    yield [(640, 4096, 0), (640, 4096, 1700), (640, 4096, 40)], wgrad
+    for _ in range(12):
+        n = int(rng.integers(1, 9))
+        shapes = [(int(rng.integers(0, 3000)), 16 * int(rng.integers(1, 130)), 16 * int(rng.integers(0, 60))) for _ in range(n)]
+        yield shapes, int(rng.choice([0, _lib.GEMM_B_KMAJOR]))
+
+
+@pytest.mark.parametrize("grid", [256, 64])
+@pytest.mark.parametrize("stream_k", [False, True])
+def test_a_half_empty_last_round_in_tiles_of_half_height(grid, stream_k):
+    """With FP8GMM_GEMM_HALF_TAIL every 128-row half of every tile is still computed exactly once, by a whole tile, a half
+    or the pieces of a shared tile; a record of half height has the extents of its 128 rows; and no workgroup has a round
+    more than without."""
+    cut = 0
+    for shapes, layout in half_tail_cases():
+        t = np.zeros(len(shapes), dtype=_lib.GEMM_PROBLEM)
+        a_kmajor, b_kmajor = bool(layout & _lib.GEMM_A_KMAJOR), bool(layout & _lib.GEMM_B_KMAJOR)
+        t["a"], t["b"], t["c"] = 0x10000, 0x20000, 0x30000
+        for i, (m, n, k) in enumerate(shapes):
+            t[i]["m"], t[i]["n"], t[i]["k"] = m, n, k
+            t[i]["lda"], t[i]["ldb"], t[i]["ldc"] = m if a_kmajor else max(k, 16), n if b_kmajor else max(k, 16), n
+        base, before, _ = _lib.plan_grouped_gemm_launch(t.copy(), layout, grid, stream_k)
+        plan, items, fixups = _lib.plan_grouped_gemm_launch(t.copy(), layout | _lib.GEMM_HALF_TAIL, grid, stream_k)
+        assert plan.total_tiles == base.total_tiles and (plan.n_fixups > 0 or plan.rounds <= base.rounds)
+        done = {}
+        for r in items[items["prob"] >= 0]:
+            p, m0, n0, nk = int(r["prob"]), int(r["m0"]), int(r["n0"]), int(r["nk"])
+            m, n, k = shapes[p]
+            half = bool(r["flags"] & 1)
+            assert m0 < m and n0 < n and m0 % (128 if half else 256) == 0 and n0 % 256 == 0
+            assert half or r["slot"] >= 0 or m - m0 > 128
+            cut += m0 % 256 == 128
+            rows = min(m - m0, 256)
+            if half:
+                rows = min(rows, 128)
+                assert r["slot"] == -1
+            if k > 0:
+                if a_kmajor:
+                    assert r["a"] == 0x10000 + m0 and r["a_bytes"] == (k - 1) * m + (m - m0)
+                else:   # at most the item's rows
+                    assert r["a"] == 0x10000 + m0 * t[p]["lda"]
+                    assert r["a_bytes"] in ((rows - 1) * t[p]["lda"] + k, (min(m - m0, 256) - 1) * t[p]["lda"] + k if m - m0 <= 128 else 0)
+            for h in range(m0, min(m0 + (128 if half else 256), m), 128):
+                steps = done.setdefault((p, h, n0), np.zeros(max(1, -(-k // 128)), dtype=int))
+                steps[int(r["k_begin"]):int(r["k_begin"]) + max(nk, 1)] += 1
+        want = {(p, h, c) for p, (m, n, k) in enumerate(shapes) for h in range(0, m, 128) for c in range(0, n, 256)}
+        assert set(done) == want and all((s == 1).all() for s in done.values())
+    assert cut > 0

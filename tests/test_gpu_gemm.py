@@ -1079,3 +1079,52 @@ def test_dgelu_epilogue_on_random_operands(dev):
     live = ref_amax > 0
     assert torch.allclose(amax.cpu()[live], ref_amax[live], rtol=1e-3, atol=0)
     assert (amax.cpu()[~live] == 0).all()
+
+
+@pytest.mark.parametrize("out", ["bf16", "bf16-contraction-major", "two-roundings", "gelu-e4m3", "e5m2"])
+def test_half_tiles_of_a_last_round_give_the_same_bits(dev, monkeypatch, out):
+    """A half-empty last round as items of half height (FP8GMM_GEMM_HALF_TAIL) against whole tiles: less than a round, a round
+    and a bit, ragged last rows of tiles and narrow last columns among the cut tiles, contraction remainders, an element-wise
+    result pitch, empty contractions, a NaN row."""
+    import numpy as np
+
+    from fp8_gmm_amd import _lib
+
+    backend = _backend()
+    g = gen(91)
+    flag, cut = _lib.GEMM_HALF_TAIL, 0
+    for sizes, k, n in [([700, 0, 129, 128], 400, 1040), ([256] * 9, 272, 8192), ([900, 300, 2600], 528, 6928),
+                        ([1100, 1], 144, 520)]:
+        m, e = sum(sizes), len(sizes)
+        a = _q(randn_bf16((m, k), g, 4.0), E5M2 if out == "e5m2" else E4M3).to(dev)
+        b = _q(randn_bf16((e, n, k), g, 4.0), E4M3).to(dev)
+        a.view(torch.uint8)[m // 2, 3] = 0x7F
+        sa, sb = torch.rand(e, generator=g).to(dev), torch.rand(e, generator=g).to(dev)
+        results = []
+        for planned in (0, flag):
+            monkeypatch.setattr(_lib, "GEMM_HALF_TAIL", planned)
+            with backend.gemm_options(tile="256", stream_k=False):
+                if out == "bf16-contraction-major":   # one tall result per expert, contracted over k rows, none for the first
+                    ks = [0] + [k - 16 * i for i in range(e - 1)]
+                    am = [a.view(torch.uint8).flatten()[:kk * 912].view(a.dtype).view(kk, 912) for kk in ks]
+                    bm = [b[i].view(torch.uint8).flatten()[:kk * 400].view(b.dtype).view(kk, 400) for i, kk in enumerate(ks)]
+                    c = [torch.full((912, 400), 7.0, dtype=torch.bfloat16, device=dev) for _ in ks]
+                    backend.grouped_gemm(am, bm, c, sa, sb, transposed=True)
+                    results.append([x.view(torch.int16) for x in c])
+                elif out in ("bf16", "two-roundings"):
+                    c = backend.fp8_gmm(a, b, torch.tensor(sizes), sa, sb, cutlass=out == "two-roundings")
+                    results.append([c.view(torch.int16)])
+                else:
+                    pre = torch.zeros(m, n, dtype=torch.bfloat16, device=dev) if out == "gelu-e4m3" else None
+                    c = torch.zeros(m, n, dtype=torch.uint8, device=dev).view(E4M3 if out == "gelu-e4m3" else E5M2)
+                    amax = torch.zeros(e, device=dev)
+                    backend.fp8_gmm(a, b, torch.tensor(sizes), sa, sb, c, pre_gelu_out=pre, c_scales=sb, c_amaxes=amax)
+                    results.append([c.view(torch.uint8), amax] + ([pre.view(torch.int16)] if pre is not None else []))
+        for x, y in zip(*results):
+            assert torch.equal(x, y), (sizes, k, n)
+        table = np.zeros(e, dtype=_lib.GEMM_PROBLEM)
+        table["a"] = table["b"] = table["c"] = 0x10000
+        table["m"], table["n"], table["k"], table["lda"], table["ldb"], table["ldc"] = sizes, n, k, k, k, n
+        _, items, _ = _lib.plan_grouped_gemm_launch(table, flag, _lib.gemm_grid(_lib.init(0)), False)
+        cut += int((items["m0"][items["prob"] >= 0] % 256 == 128).sum())
+    assert cut > 50
