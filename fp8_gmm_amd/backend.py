@@ -804,7 +804,7 @@ def _launch_gemm(table, a_dtype, b_dtype, c_dtype, gelu, device, keep, b_kmajor=
     elif not epi and c_dtype == torch.bfloat16 and _dual_tiles(table, a_kmajor):
         plan, blob, off_items, off_fix = _lib.plan_grouped_gemm_blob(table, layout | _lib.GEMM_TILE_DUAL, grid, False)
     else:
-        plan, blob, off_items, off_fix = _lib.plan_grouped_gemm_blob(table, layout | epi | _lib.GEMM_HALF_TAIL, grid,
+        plan, blob, off_items, off_fix = _lib.plan_grouped_gemm_blob(table, layout | epi | _lib.GEMM_BALANCED, grid,
                                                                      options.stream_k)
     if plan.total_tiles == 0:
         return

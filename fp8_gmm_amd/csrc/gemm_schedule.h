@@ -43,6 +43,11 @@ constexpr int kSkPerSlot = 100;
 constexpr int kSkGeluPerTile = 150;
 constexpr int kPartialBytes = BM * BN * 4;  // one slot: the fp32 accumulators of one tile
 constexpr int kTileOverhead = 4;      // fixed cost of a tile (epilogue, switch) in K = 128 steps, measured
+// What a tile weighs besides its steps where the XCDs' ranges are cut (FP8GMM_GEMM_BALANCED; without it kTileOverhead).  Less
+// than what it costs its workgroup: a range of short contractions stores while another one reads.  17 weight gradients of
+// skewed splits inside a layer's step, 4 -> 3 / 2 / 1: 1.002, 0.988, 1.002 of the time (6 of 8960 x 832, 15230 rows 138 -> 127
+// us; the most that one loses is 2 %); 43 alone with operands from HBM: 0.994, 0.981, 0.985.
+constexpr int kTileWeight = 2;
 constexpr int kSlotsPerWg = 2;        // a piece that starts inside a tile, one that ends inside a tile
 
 struct Sched {
@@ -55,6 +60,7 @@ struct Sched {
   int sk_wgs;                  // workgroups that take a piece of the region
   int64_t sk_c0, sk_cost;      // cost before the region, cost of the region (K = 128 steps)
   int64_t total_cost;          // cost of all tiles
+  int tile_weight;             // of a tile besides its steps, where the ranges are cut
   bool halves;                 // the remainder [sk_begin, range_end) in tiles of half height, two per tile (sk_wgs is 0)
   bool gelu;                   // completing a shared tile includes the GELU epilogue
 };
@@ -78,7 +84,7 @@ FP8GMM_HD int64_t tile_cost(const Sched& s, int p) {
 }
 // Work before `tile` (0 <= tile <= total_tiles) when every tile counts its K steps plus `ov` steps of fixed
 // overhead; cost_begin is the plan's prefix sum of the K steps alone.  ov = 0 is the unit in which tiles are
-// cut along K; ov = kTileOverhead is the weight that balances the XCD ranges.
+// cut along K; ov = tile_weight is the weight that balances the XCD ranges.
 FP8GMM_HD int64_t work_before(const Sched& s, int tile, int ov) {
   const int p = problem_of_tile(s, tile);
   return (int64_t)s.probs[p].cost_begin + (int64_t)ov * s.probs[p].tile_begin +
@@ -107,8 +113,8 @@ FP8GMM_HD int first_tile_at_work(const Sched& s, int64_t c, int ov) {
 
 // first tile of XCD x's range (x = 8: the end of the last one)
 FP8GMM_HD int range_start(const Sched& s, int x) {
-  const int64_t total_work = s.total_cost + (int64_t)kTileOverhead * s.total_tiles;
-  return first_tile_at_work(s, (total_work * x + kNumXcd - 1) / kNumXcd, kTileOverhead);
+  const int64_t total_work = s.total_cost + (int64_t)s.tile_weight * s.total_tiles;
+  return first_tile_at_work(s, (total_work * x + kNumXcd - 1) / kNumXcd, s.tile_weight);
 }
 // Striding takes a range of n tiles full + 1 rounds, sharing the remainder full + rem / W: worth a thought when that saves
 // a twelfth of the launch by this count.  Measured, sharing returns about half of what the count promises (workgroups do
@@ -333,16 +339,17 @@ inline void sk_decide(const Sched (&all)[kNumXcd], SkRemainder (&rem)[kNumXcd], 
 // Workgroup i runs on XCD i % 8.  The tile list is cut into 8 contiguous ranges of equal WORK, one per XCD,
 // so that workgroups that share an L2 work on neighbouring tiles; the workgroups of an XCD stride through the
 // range, and share its remainder along K when that pays.  k differs per problem in the wgrad form, and a
-// tile costs its K steps plus a fixed part (epilogue, tile switch) worth about kTileOverhead steps: balancing
+// tile costs its K steps plus a fixed part (epilogue, tile switch): balancing
 // K steps alone left the XCDs that hold the short-K problems 17 % more work than the others.
 inline void sched_init(Sched (&all)[kNumXcd], const fp8gmm_gemm_problem* probs, int nprob, int total_tiles, int wgs_per_xcd,
-                       bool sk_enable, bool gelu = false, bool half_tail = false) {
+                       bool sk_enable, bool gelu = false, bool balanced = false) {
   const int W = wgs_per_xcd;
   SkRemainder rem[kNumXcd];
   for (int x = 0; x < kNumXcd; ++x) {
     Sched& s = all[x];
     s.gelu = gelu;
     s.halves = false;
+    s.tile_weight = balanced ? kTileWeight : kTileOverhead;
     s.probs = probs;
     s.nprob = nprob;
     s.total_tiles = total_tiles;
@@ -363,7 +370,7 @@ inline void sched_init(Sched (&all)[kNumXcd], const fp8gmm_gemm_problem* probs, 
     r.timed = r.halves = false;
     r.tiles = n_x % W;
     r.begin = s.range_end - r.tiles;
-    if (half_tail && r.tiles > 0 && 2 * r.tiles <= W && n_x / W <= kHalfMaxRounds) {
+    if (balanced && r.tiles > 0 && 2 * r.tiles <= W && n_x / W <= kHalfMaxRounds) {
       sk_times(s, r);
       if (r.half_x100 < r.whole_x100) {
         r.halves = true;

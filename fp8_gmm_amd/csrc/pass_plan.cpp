@@ -359,7 +359,7 @@ int write_pass(Pass& pass, void* blob, size_t blob_bytes, fp8gmm_pass_plan* out)
     // shared-tile records are few (at most one per workgroup): planned into a local array, appended afterwards
     static thread_local fp8gmm_gemm_fixup_desc fix[4096];
     const int rc = fp8gmm_plan_grouped_gemm_launch(
-        probs, e, l.gemm.layout | l.epi | (flag != 0 ? flag : FP8GMM_GEMM_HALF_TAIL), grid_of(flag, pass.grid),
+        probs, e, l.gemm.layout | l.epi | (flag != 0 ? flag : FP8GMM_GEMM_BALANCED), grid_of(flag, pass.grid),
         flag != 0 ? 0 : pass.stream_k, items, (int)room, fix, 4096, &rec->plan);
     if (rc != FP8GMM_OK && rc != FP8GMM_ERR_BUFFER_TOO_SMALL) return rc;
     if (rc == FP8GMM_ERR_BUFFER_TOO_SMALL) w.fits = false;
@@ -412,7 +412,7 @@ int lay_out_pass(Pass& pass, fp8gmm_pass_plan* out, PassTables* t) {
     fill_problems(pass, l.gemm, probs);
     const int flag = tile_flag(probs, e, pass, l);
     fp8gmm::GemmRanges* ranges = &t->ranges[t->n_gemms];
-    const int rc = fp8gmm::plan_gemm_ranges(probs, e, l.gemm.layout | l.epi | (flag != 0 ? flag : FP8GMM_GEMM_HALF_TAIL),
+    const int rc = fp8gmm::plan_gemm_ranges(probs, e, l.gemm.layout | l.epi | (flag != 0 ? flag : FP8GMM_GEMM_BALANCED),
                                             grid_of(flag, pass.grid),
                                             flag != 0 ? 0 : pass.stream_k, &rec->plan, ranges);
     if (rc != FP8GMM_OK) return rc;

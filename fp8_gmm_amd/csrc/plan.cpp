@@ -191,35 +191,39 @@ int fp8gmm_plan_grouped_gemm_layout(fp8gmm_gemm_problem* probs, int n, int layou
 // The same launch cut into 128 x 128 tiles (FP8GMM_GEMM_TILE_128), into 128 x 256 tiles for the kernel with two
 // sets of accumulators (FP8GMM_GEMM_TILE_DUAL), or into 64 x 128 tiles for few rows (FP8GMM_GEMM_TILE_ROWS): whole tiles only, the tile list in 8 contiguous ranges of equal
 // work, the workgroups of an XCD striding through their range.
-constexpr int kSmallTileOverhead = 3, kDualTileOverhead = 2, kRowsTileOverhead = 1;
+// What a tile weighs besides its steps when the XCDs' ranges are cut, in half steps: its epilogue and switch as far as its
+// workgroup's partner on the compute unit does not cover them; with two sets of accumulators, the slower steps that carry the
+// result.  Small tiles, 26 weight gradients of skewed splits inside a layer's step, 3 -> 2 / 1.5 / 1 / 0.5 steps a tile: 0.987,
+// 0.979, 0.987, 0.998 of the time in the mean (at 3 the XCDs with the short contractions were through after 87 us and those with
+// the long ones after 128; at 1.5: 64 of 1408 x 2048, 24576 rows 171 -> 156, 64 of 576 x 3536, 18873 297 -> 262; 35 of 320 x 992,
+// 31013 79 -> 85; with operands from HBM, launches alone, 0.968).  Row-sliced launches have one K and do not notice.
+constexpr int kSmallTileWeight = 3, kDualTileWeight = 4, kRowsTileWeight = 2;
 constexpr int kWholeTileForms = FP8GMM_GEMM_TILE_128 | FP8GMM_GEMM_TILE_DUAL | FP8GMM_GEMM_TILE_ROWS;
-// Tile and overhead of the form that `layout` asks for; false when it names none that exists with its other flags.
-static bool whole_tile_form(int layout, int* tm, int* tn, int* overhead) {
+// Tile and weight of the form that `layout` asks for; false when it names none that exists with its other flags.
+static bool whole_tile_form(int layout, int* tm, int* tn, int* weight) {
   switch (layout & kWholeTileForms) {
     case FP8GMM_GEMM_TILE_128:
       *tm = *tn = FP8GMM_GEMM_SMALL_TILE;
-      *overhead = kSmallTileOverhead;
+      *weight = kSmallTileWeight;
       return (layout & (FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU)) == 0;
     case FP8GMM_GEMM_TILE_DUAL:
       *tm = FP8GMM_GEMM_DUAL_TILE_M;
       *tn = fp8gmm::kGemmTileN;
-      *overhead = kDualTileOverhead;
+      *weight = kDualTileWeight;
       return (layout & (FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU)) == 0;
     case FP8GMM_GEMM_TILE_ROWS:
       *tm = FP8GMM_GEMM_ROWS_TILE_M;
       *tn = FP8GMM_GEMM_ROWS_TILE_N;
-      *overhead = kRowsTileOverhead;
+      *weight = kRowsTileWeight;
       return (layout & (FP8GMM_EPI_DGELU | FP8GMM_GEMM_A_KMAJOR | FP8GMM_GEMM_B_KMAJOR)) == 0;
   }
   return false;
 }
-// kOverhead: what a tile costs besides its steps, in K = 128 steps: epilogue and switch of a small tile on a
-// workgroup that shares its compute unit; with two sets of accumulators, the slower steps that carry the result.
 struct WholeTileCuts {
   std::vector<int64_t> tile_begin;        // per problem
   int cut[fp8gmm::kNumXcd + 1];           // XCD x takes the tiles [cut[x], cut[x + 1])
 };
-static int cut_whole_tiles(const int TM, const int TN, const int kOverhead, fp8gmm_gemm_problem* probs, int n, int layout,
+static int cut_whole_tiles(const int TM, const int TN, const int weight, fp8gmm_gemm_problem* probs, int n, int layout,
                            int grid, WholeTileCuts* out, fp8gmm_gemm_plan* plan) {
   using namespace fp8gmm;
   int unused = 0;
@@ -233,7 +237,7 @@ static int cut_whole_tiles(const int TM, const int TN, const int kOverhead, fp8g
     const int64_t tiles = (int64_t)((probs[p].m + TM - 1) / TM) * ((probs[p].n + TN - 1) / TN);
     const int64_t steps = (probs[p].k + 127) / 128;
     tile_begin[p + 1] = tile_begin[p] + tiles;
-    work_begin[p + 1] = work_begin[p] + tiles * ((steps > 0 ? steps : 1) + kOverhead);
+    work_begin[p + 1] = work_begin[p] + tiles * (2 * (steps > 0 ? steps : 1) + weight);
     if (tile_begin[p + 1] > INT32_MAX / 16) return FP8GMM_ERR_BAD_SHAPE;
   }
   const int total_tiles = (int)tile_begin[n];
@@ -268,11 +272,11 @@ static int cut_whole_tiles(const int TM, const int TN, const int kOverhead, fp8g
   return (int64_t)plan->rounds * grid > INT32_MAX / 64 ? FP8GMM_ERR_BAD_SHAPE : FP8GMM_OK;
 }
 
-static int plan_whole_tiles(const int TM, const int TN, const int kOverhead, fp8gmm_gemm_problem* probs, int n, int layout,
+static int plan_whole_tiles(const int TM, const int TN, const int weight, fp8gmm_gemm_problem* probs, int n, int layout,
                             int grid, fp8gmm_gemm_item* items, int max_items, fp8gmm_gemm_plan* plan) {
   using namespace fp8gmm;
   WholeTileCuts cuts;
-  const int rc = cut_whole_tiles(TM, TN, kOverhead, probs, n, layout, grid, &cuts, plan);
+  const int rc = cut_whole_tiles(TM, TN, weight, probs, n, layout, grid, &cuts, plan);
   if (rc != FP8GMM_OK || plan->total_tiles == 0) return rc;
   const bool a_kmajor = (layout & FP8GMM_GEMM_A_KMAJOR) != 0, b_kmajor = (layout & FP8GMM_GEMM_B_KMAJOR) != 0;
   const std::vector<int64_t>& tile_begin = cuts.tile_begin;
@@ -301,11 +305,11 @@ static int plan_whole_tiles(const int TM, const int TN, const int kOverhead, fp8
 // Tail balancing can only pay when the launch has few rounds; it needs the whole grid even for few tiles.  Without it
 // the grid shrinks to the tiles there are.
 // So does a last round of half tiles.
-static bool share_tail(int stream_k, int total_tiles, bool half_tail, int* grid) {
+static bool share_tail(int stream_k, int total_tiles, bool balanced, int* grid) {
   using namespace fp8gmm;
   if (stream_k != 0 && (int64_t)total_tiles <= (int64_t)kSkMaxRounds * *grid && *grid > kNumXcd) return true;
   const int needed = ((total_tiles + kNumXcd - 1) / kNumXcd) * kNumXcd;
-  if (*grid > needed && !half_tail) *grid = needed;
+  if (*grid > needed && !balanced) *grid = needed;
   return false;
 }
 
@@ -317,30 +321,30 @@ int fp8gmm_plan_grouped_gemm_launch(fp8gmm_gemm_problem* probs, int n, int layou
   *plan = fp8gmm_gemm_plan{};
   if (grid <= 0 || (grid % kNumXcd) != 0 || max_items < 0 || max_fixups < 0) return FP8GMM_ERR_BAD_ARGUMENT;
   if (layout & kWholeTileForms) {
-    int tm = 0, tn = 0, overhead = 0;
-    if (!whole_tile_form(layout, &tm, &tn, &overhead)) return FP8GMM_ERR_BAD_ARGUMENT;
-    return plan_whole_tiles(tm, tn, overhead, probs, n, layout & ~(kWholeTileForms | FP8GMM_EPI_GELU), grid, items, max_items,
+    int tm = 0, tn = 0, weight = 0;
+    if (!whole_tile_form(layout, &tm, &tn, &weight)) return FP8GMM_ERR_BAD_ARGUMENT;
+    return plan_whole_tiles(tm, tn, weight, probs, n, layout & ~(kWholeTileForms | FP8GMM_EPI_GELU), grid, items, max_items,
                             plan);
   }
   plan->tile = kGemmTileM;
   const int layout_given = layout, grid_given = grid;
   // the epilogue flags only weigh the decision to share tiles along K (completing a tile costs more with them)
   const bool gelu = (layout & (FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU)) != 0;
-  const bool half_tail = (layout & FP8GMM_GEMM_HALF_TAIL) != 0;
-  layout &= ~(FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU | FP8GMM_GEMM_HALF_TAIL);
+  const bool balanced = (layout & FP8GMM_GEMM_BALANCED) != 0;
+  layout &= ~(FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU | FP8GMM_GEMM_BALANCED);
   int total_tiles = 0;
   const int rc = fp8gmm_plan_grouped_gemm_layout(probs, n, layout, &total_tiles);
   if (rc != FP8GMM_OK) return rc;
   plan->total_tiles = total_tiles;
   if (total_tiles == 0) return FP8GMM_OK;
-  const bool sk = share_tail(stream_k, total_tiles, half_tail, &grid);
+  const bool sk = share_tail(stream_k, total_tiles, balanced, &grid);
   const int wgs = grid / kNumXcd;
   const bool a_kmajor = (layout & FP8GMM_GEMM_A_KMAJOR) != 0, b_kmajor = (layout & FP8GMM_GEMM_B_KMAJOR) != 0;
 
   // pass 1: sizes.  The tiles that were shared along K first: the pieces of such a tile get consecutive
   // workspace slots, numbered from 0 over the launch, in K order.
   Sched sched[kNumXcd];
-  sched_init(sched, probs, n, total_tiles, wgs, sk, gelu, half_tail);
+  sched_init(sched, probs, n, total_tiles, wgs, sk, gelu, balanced);
   std::vector<int32_t> slot_map((size_t)kSlotsPerWg * grid, -1);
   std::vector<fp8gmm_gemm_fixup_desc> fix;
   int n_slots = 0;
@@ -516,10 +520,10 @@ int plan_gemm_ranges(fp8gmm_gemm_problem* probs, int n, int layout, int grid, in
   *out = GemmRanges{};
   if (grid <= 0 || (grid % kNumXcd) != 0) return FP8GMM_ERR_BAD_ARGUMENT;
   if (layout & kWholeTileForms) {
-    int tm = 0, tn = 0, overhead = 0;
-    if (!whole_tile_form(layout, &tm, &tn, &overhead)) return FP8GMM_ERR_BAD_ARGUMENT;
+    int tm = 0, tn = 0, weight = 0;
+    if (!whole_tile_form(layout, &tm, &tn, &weight)) return FP8GMM_ERR_BAD_ARGUMENT;
     WholeTileCuts cuts;
-    const int rc = cut_whole_tiles(tm, tn, overhead, probs, n, layout & (FP8GMM_GEMM_A_KMAJOR | FP8GMM_GEMM_B_KMAJOR), grid,
+    const int rc = cut_whole_tiles(tm, tn, weight, probs, n, layout & (FP8GMM_GEMM_A_KMAJOR | FP8GMM_GEMM_B_KMAJOR), grid,
                                    &cuts, plan);
     if (rc != FP8GMM_OK || plan->total_tiles == 0) return rc;
     for (int x = 0; x < kNumXcd; ++x) {
@@ -530,17 +534,17 @@ int plan_gemm_ranges(fp8gmm_gemm_problem* probs, int n, int layout, int grid, in
     const bool gelu = (layout & (FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU)) != 0;
     plan->tile = kGemmTileM;
     int total_tiles = 0;
-    const bool half_tail = (layout & FP8GMM_GEMM_HALF_TAIL) != 0;
+    const bool balanced = (layout & FP8GMM_GEMM_BALANCED) != 0;
     const int rc = fp8gmm_plan_grouped_gemm_layout(
-        probs, n, layout & ~(FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU | FP8GMM_GEMM_HALF_TAIL), &total_tiles);
+        probs, n, layout & ~(FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU | FP8GMM_GEMM_BALANCED), &total_tiles);
     if (rc != FP8GMM_OK) return rc;
     plan->total_tiles = total_tiles;
     if (total_tiles == 0) return FP8GMM_OK;
-    const bool sk = share_tail(stream_k, total_tiles, half_tail, &grid);
+    const bool sk = share_tail(stream_k, total_tiles, balanced, &grid);
     const int wgs = grid / kNumXcd;
     plan->grid = grid;
     Sched sched[kNumXcd];
-    sched_init(sched, probs, n, total_tiles, wgs, sk, gelu, half_tail);
+    sched_init(sched, probs, n, total_tiles, wgs, sk, gelu, balanced);
     for (int x = 0; x < kNumXcd; ++x) {
       const Sched& s = sched[x];
       GemmRanges::Xcd& o = out->xcd[x];

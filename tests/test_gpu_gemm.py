@@ -1083,7 +1083,7 @@ def test_dgelu_epilogue_on_random_operands(dev):
 
 @pytest.mark.parametrize("out", ["bf16", "bf16-contraction-major", "two-roundings", "gelu-e4m3", "e5m2"])
 def test_half_tiles_of_a_last_round_give_the_same_bits(dev, monkeypatch, out):
-    """A half-empty last round as items of half height (FP8GMM_GEMM_HALF_TAIL) against whole tiles: less than a round, a round
+    """A half-empty last round as items of half height (FP8GMM_GEMM_BALANCED) against whole tiles: less than a round, a round
     and a bit, ragged last rows of tiles and narrow last columns among the cut tiles, contraction remainders, an element-wise
     result pitch, empty contractions, a NaN row."""
     import numpy as np
@@ -1092,7 +1092,7 @@ def test_half_tiles_of_a_last_round_give_the_same_bits(dev, monkeypatch, out):
 
     backend = _backend()
     g = gen(91)
-    flag, cut = _lib.GEMM_HALF_TAIL, 0
+    flag, cut = _lib.GEMM_BALANCED, 0
     for sizes, k, n in [([700, 0, 129, 128], 400, 1040), ([256] * 9, 272, 8192), ([900, 300, 2600], 528, 6928),
                         ([1100, 1], 144, 520)]:
         m, e = sum(sizes), len(sizes)
@@ -1102,7 +1102,7 @@ def test_half_tiles_of_a_last_round_give_the_same_bits(dev, monkeypatch, out):
         sa, sb = torch.rand(e, generator=g).to(dev), torch.rand(e, generator=g).to(dev)
         results = []
         for planned in (0, flag):
-            monkeypatch.setattr(_lib, "GEMM_HALF_TAIL", planned)
+            monkeypatch.setattr(_lib, "GEMM_BALANCED", planned)
             with backend.gemm_options(tile="256", stream_k=False):
                 if out == "bf16-contraction-major":   # one tall result per expert, contracted over k rows, none for the first
                     ks = [0] + [k - 16 * i for i in range(e - 1)]
