@@ -310,24 +310,19 @@ __device__ __forceinline__ int tile_epilogue(const fp8gmm_gemm_problem& pr, int 
           constexpr int i = u / kUnitsPerRow, jj = u % kUnitsPerRow;
           if (i >= mt) return;
           uint8_t* buf = mine + (kStageBytes >= 8192 ? (u & 1) * 4096 : 0);
-          u32x2 o[8];
           static_for<2>([&](auto jlc) {
             constexpr int jl = decltype(jlc)::value;
             const f32x16 t = acc_tile<16 * (NT * i + 2 * jj + jl)>();
             released(std::integral_constant<int, i>{}, std::integral_constant<int, 2 * jj + jl>{});
   #pragma unroll
-            for (int g = 0; g < 4; ++g)
-              o[4 * jl + g] = u32x2{scaled_bf16x2<decltype(two_c)::value>(t[4 * g + 0], t[4 * g + 1], s, cs),
-                                    scaled_bf16x2<decltype(two_c)::value>(t[4 * g + 2], t[4 * g + 3], s, cs)};
+            for (int g = 0; g < 4; ++g) {
+              const u32x2 o = {scaled_bf16x2<decltype(two_c)::value>(t[4 * g + 0], t[4 * g + 1], s, cs),
+                               scaled_bf16x2<decltype(two_c)::value>(t[4 * g + 2], t[4 * g + 3], s, cs)};
+              *reinterpret_cast<u32x2*>(buf + wr + (((4 * jl + g) ^ ((l32 >> 1) & 7)) << 4)) = o;
+            }
           });
-          // the previous unit's read-back was issued before this unit's conversion: store it now, and stage this one only then
-          // (the wait for the read-back is one for everything that LDS has been asked: with this unit's writes in front of
-          // it, it waited for them at every unit)
-          FP8GMM_SB();
+          // the previous unit's read-back was issued before this unit's conversion: store it now
           if (u > 0) store_unit((u - 1) / kUnitsPerRow, (u - 1) % kUnitsPerRow);
-          FP8GMM_SB();
-  #pragma unroll
-          for (int q = 0; q < 8; ++q) *reinterpret_cast<u32x2*>(buf + wr + ((q ^ ((l32 >> 1) & 7)) << 4)) = o[q];
           // only this wavefront touches `mine`, and its LDS operations complete in order
   #pragma unroll
           for (int it = 0; it < 4; ++it) {
