@@ -226,6 +226,8 @@ EXPORTS = (
     "fp8gmm_moe_scatter_backward",
     "fp8gmm_route_topk",
     "fp8gmm_route_topk_backward",
+    "fp8gmm_gating_workspace_bytes",
+    "fp8gmm_gating_backward",
     "fp8gmm_moe_gather",
     "fp8gmm_moe_scatter",
     "fp8gmm_moe_scatter_wgrad",
@@ -344,6 +346,10 @@ def load():
     L.fp8gmm_route_topk.argtypes = [vp, ci, ci, ci, ci, vp, vp, vp, vp]
     L.fp8gmm_route_topk_backward.restype = ci
     L.fp8gmm_route_topk_backward.argtypes = [vp, vp, vp, ci, ci, ci, vp, ci, vp]
+    L.fp8gmm_gating_workspace_bytes.restype = ctypes.c_size_t
+    L.fp8gmm_gating_workspace_bytes.argtypes = [ci, ci, ci]
+    L.fp8gmm_gating_backward.restype = ci
+    L.fp8gmm_gating_backward.argtypes = [vp, vp, vp, vp, vp, vp, ci, ci, ci, vp, vp]
     L.fp8gmm_moe_gather.restype = ci
     L.fp8gmm_moe_gather.argtypes = [vp, vp, vp, vp, ci, ci, ci, vp]
     L.fp8gmm_moe_scatter.restype = ci

@@ -52,7 +52,7 @@ class _RoutedModule(torch.nn.Module):
 
     def forward(self, input):
         input = input.view(-1, input.size(-1))
-        routing_logits = self.gating_network(input)
+        routing_logits, input = moe_ops.gating(self.gating_network, input)
         weights0, selected_experts = moe_ops.topk(routing_logits, self.top_k)
         expert_weights = weights0.flatten()
         top_experts = selected_experts.flatten()

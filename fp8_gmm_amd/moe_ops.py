@@ -88,6 +88,89 @@ def indices_and_bins(top_expert, sort_end_bit, n_experts):
     return indices, bin_ids, bins, tokens_per_expert
 
 
+MAX_GATING_EXPERTS = 128
+
+
+def _aligned(t):
+    """``t``, or a copy of it that is contiguous and starts on 16 bytes (what a saved-tensor or gradient hook returned
+    may be anything)."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone(memory_format=torch.contiguous_format)
+
+
+class _Gating(torch.autograd.Function):
+    """``(x weight^T, x)``: the logits, and x once more for what follows, so that its two gradients meet here and one
+    kernel adds them."""
+
+    @staticmethod
+    def forward(ctx, x, weight):
+        ctx.set_materialize_grads(False)
+        ctx.save_for_backward(x, weight)
+        return torch.nn.functional.linear(x, weight), x
+
+    @staticmethod
+    def backward(ctx, grad, grad_in):
+        if grad is None:
+            return grad_in, None
+        x, weight = ctx.saved_tensors
+        want_x, want_weight = ctx.needs_input_grad
+        if torch.is_grad_enabled():   # a graph of the backward pass is asked for
+            grad_x = grad_weight = None
+            if want_x:
+                grad_x = grad @ weight if grad_in is None else grad_in + grad @ weight
+            if want_weight:
+                grad_weight = grad.t() @ x
+            return grad_x, grad_weight
+        (tokens, experts), hidden, dev = grad.shape, x.shape[1], x.device
+        grad, x = _aligned(grad), _aligned(x)
+        weight = weight.contiguous()
+        grad_in = _aligned(grad_in) if grad_in is not None else None
+        L = _lib.load()
+        grad_x = torch.empty_like(x) if want_x else None
+        grad_weight = work = None
+        if want_weight:
+            grad_weight = torch.empty(experts, hidden, dtype=x.dtype, device=dev)
+            work = torch.empty(L.fp8gmm_gating_workspace_bytes(tokens, hidden, experts), dtype=torch.uint8, device=dev)
+        with torch.cuda.device(dev), _timed("gating_backward", lambda: 2 * tokens * hidden * (want_weight + 2 * want_x)):
+            rc = L.fp8gmm_gating_backward(grad.data_ptr(), x.data_ptr(), weight.data_ptr(),
+                                          grad_in.data_ptr() if grad_in is not None else None,
+                                          grad_x.data_ptr() if want_x else None,
+                                          grad_weight.data_ptr() if want_weight else None, tokens, hidden, experts,
+                                          work.data_ptr() if want_weight and work.numel() else None, _stream(dev))
+        _lib.check(rc)
+        return grad_x, grad_weight
+
+
+def _plain_linear(module):
+    """A ``torch.nn.Linear`` that is nothing but its product: no bias, hook, parametrisation or replaced forward."""
+    return (type(module) is torch.nn.Linear and module.bias is None and "forward" not in module.__dict__
+            and type(module._parameters.get("weight")) is torch.nn.Parameter
+            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks
+                     or module._backward_pre_hooks) and not torch.nn.modules.module._has_any_global_hook())
+
+
+def _gating_takes(x, weight):
+    """What fp8gmm_gating_backward computes; the general path is torch's linear and its gradients.  Inside these limits the
+    kernels are the faster ones throughout (csrc/gating.hip has both sides from 16 tokens and 1 expert to 16384 and 128);
+    the forward product stays torch's, whose bits decide the routing."""
+    tokens, hidden = x.shape
+    return (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.is_cuda and weight.device == x.device
+            and type(x) in (torch.Tensor, torch.nn.Parameter) and weight.dim() == 2 and weight.shape[1] == hidden
+            and 1 <= weight.shape[0] <= MAX_GATING_EXPERTS and 1 <= tokens <= 1 << 20 and 8 <= hidden <= 1 << 16
+            and hidden % 8 == 0 and x.is_contiguous() and weight.is_contiguous() and x.data_ptr() % 16 == 0)
+
+
+def gating(module, x):
+    """``(module(x), x)`` for a gating linear of a routed layer (fp8_gmm/example.py:47-50,84-86,112-113), to be followed by
+    a use of the returned ``x``: with gradients wanted for the rows, one backward pass on this package's kernels takes the
+    gradient of the logits and that of the returned rows together.  Where the module is more than a product, or the rows
+    are not what the kernels take, the module is called."""
+    if torch.is_grad_enabled() and x.requires_grad and _plain_linear(module) and not torch.is_autocast_enabled("cuda") \
+            and not torch.jit.is_tracing() and _gating_takes(x, module.weight):
+        return _Gating.apply(x, module.weight)
+    return module(x), x
+
+
 MAX_TOP_K = 8
 
 

@@ -601,6 +601,17 @@ int fp8gmm_route_topk(const void* scores, int scores_bf16, int tokens, int num_e
  * experts: the gradient of `weights` above with respect to `scores`, written as bf16 (grad_bf16 != 0) or fp32. */
 int fp8gmm_route_topk_backward(const float* probs, const int64_t* selected, const float* grad_weights, int tokens,
                                int num_experts, int top_k, void* grad_scores, int grad_bf16, void* stream);
+/*
+ * The backward pass of a bias-free gating linear, logits = x weight^T (the gating_network of fp8_gmm/example.py:38,76,109):
+ *   grad_weight = bf16(grad^T x),   grad_x = bf16(grad_in + grad weight),   products and sums in fp32, rounded once.
+ * grad: bf16 [tokens, experts]; x, grad_in, grad_x: bf16 [tokens, hidden]; weight, grad_weight: bf16 [experts, hidden];
+ * all contiguous and on 16 bytes, hidden a multiple of 8, at most 128 experts.  grad_in == NULL: nothing is added;
+ * grad_x or grad_weight == NULL: not computed.  workspace: fp8gmm_gating_workspace_bytes bytes on 16 bytes, for
+ * grad_weight alone.
+ */
+size_t fp8gmm_gating_workspace_bytes(int tokens, int hidden, int experts);
+int fp8gmm_gating_backward(const void* grad, const void* x, const void* weight, const void* grad_in, void* grad_x,
+                           void* grad_weight, int tokens, int hidden, int experts, void* workspace, void* stream);
 /* inverse[indices[i]] = i for a permutation `indices` of 0..n-1 (entries outside that range are skipped) */
 int fp8gmm_route_invert(const int32_t* indices, int n, int32_t* inverse, void* stream);
 /*

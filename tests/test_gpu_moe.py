@@ -310,3 +310,62 @@ def test_example_recipe_runs_every_kind_of_layer(dev, capsys):
     assert list(times) == list(example.KINDS) and all(t > 0 for t in times.values())
     lines = [line for line in capsys.readouterr().out.splitlines() if " run: " in line]
     assert len(lines) == 4 and lines[0].startswith("Bf16Module run: ") and lines[3].startswith("Fp8MlpModule run: ")
+
+
+@pytest.mark.parametrize("tokens,hidden,experts", [(1, 8, 1), (16, 64, 16), (17, 72, 5), (127, 136, 33), (128, 256, 32),
+                                                   (129, 264, 65), (1531, 1024, 16), (4097, 520, 128), (16385, 192, 8)])
+def test_gating_gradients_are_exact_on_whole_numbers(dev, tokens, hidden, experts):
+    """Edges of the token, column and expert tiles, one slice of tokens and many: sums of products of small whole numbers
+    are exact in fp32, so the one rounding to bf16 leaves nothing open.  Each gradient alone gives the same bits."""
+    ops = _ops()
+    gen = torch.Generator().manual_seed(tokens)
+    x, w, g, up = (torch.randint(-3, 4, shape, generator=gen).to(torch.bfloat16) for shape in
+                   [(tokens, hidden), (experts, hidden), (tokens, experts), (tokens, hidden)])
+    want_x = up.double() + g.double() @ w.double()
+    want_w = g.double().t() @ x.double()
+    alone_x = g.double() @ w.double()
+    linear = torch.nn.Linear(hidden, experts, bias=False, dtype=torch.bfloat16, device=dev)
+    linear.weight.data.copy_(w)
+    g, up = g.to(dev), up.to(dev)
+    for train, rows in ((True, True), (True, False), (False, True)):
+        xd = x.to(dev).requires_grad_()
+        linear.requires_grad_(train).zero_grad()
+        logits, again = ops.gating(linear, xd)
+        assert "Gating" in logits.grad_fn.name()
+        assert torch.equal(logits, torch.nn.functional.linear(xd, linear.weight)) and torch.equal(again, xd)
+        torch.autograd.backward((logits, again) if rows else (logits,), (g, up) if rows else (g,))
+        assert torch.equal(xd.grad.cpu(), (want_x if rows else alone_x).to(torch.bfloat16))
+        if train:
+            assert torch.equal(linear.weight.grad.cpu(), want_w.to(torch.bfloat16))
+
+
+def test_gating_calls_a_module_that_is_more_than_a_product(dev):
+    """Hooks, a bias, another class, rows the kernels do not take and rows without a gradient: the module is called, its
+    hooks with it; a graph of the backward pass can be asked for on either path."""
+    ops = _ops()
+    x = torch.randn(33, 64, device=dev).to(torch.bfloat16)
+
+    def linear(h=64, bias=False, dtype=torch.bfloat16):
+        return torch.nn.Linear(h, 6, bias=bias, dtype=dtype, device=dev)
+
+    seen = []
+    hooked = linear()
+    hooked.register_forward_hook(lambda *a: seen.append(1))
+    replaced = linear()
+    replaced.forward = lambda v: seen.append(2) or torch.nn.functional.linear(v, replaced.weight)
+    odd = torch.randn(33, 65, device=dev).to(torch.bfloat16)
+    wide = torch.randn(33, 128, device=dev).to(torch.bfloat16)
+    for module, rows in ((hooked, x), (replaced, x), (linear(bias=True), x), (torch.nn.Sequential(linear()), x),
+                         (linear(65), odd), (linear(), wide[:, :64]), (linear(dtype=torch.float32), x.float())):
+        rows = rows.detach().requires_grad_()
+        logits, again = ops.gating(module, rows)
+        assert again is rows and "Gating" not in logits.grad_fn.name()
+    assert seen == [1, 2]
+    logits, again = ops.gating(linear(), x)
+    assert again is x and "Gating" not in logits.grad_fn.name()
+    plain, xd = linear(), x.detach().requires_grad_()
+    logits, again = ops.gating(plain, xd)
+    first, = torch.autograd.grad((logits.float() ** 2).sum() + again.float().sum(), xd, create_graph=True)
+    second, = torch.autograd.grad(first.float().sum(), xd)
+    want = 2 * (plain.weight.float().t() @ plain.weight.float()).sum(0)     # the Hessian of |W x|^2 times ones
+    assert torch.allclose(second.float(), want.expand_as(second), rtol=2e-2, atol=2e-2 * want.abs().max().item())
