@@ -222,6 +222,7 @@ EXPORTS = (
     "fp8gmm_upload",
     "fp8gmm_route_workspace_bytes",
     "fp8gmm_route_sort",
+    "fp8gmm_route_sort_selected",
     "fp8gmm_route_invert",
     "fp8gmm_moe_scatter_backward",
     "fp8gmm_route_topk",
@@ -338,6 +339,8 @@ def load():
     L.fp8gmm_route_workspace_bytes.argtypes = [ci, ci]
     L.fp8gmm_route_sort.restype = ci
     L.fp8gmm_route_sort.argtypes = [vp, ci, ci, vp, vp, vp, vp, vp, vp, vp]
+    L.fp8gmm_route_sort_selected.restype = ci
+    L.fp8gmm_route_sort_selected.argtypes = [vp, ci, ci, vp, vp, vp, vp, vp, vp, vp]
     L.fp8gmm_route_invert.restype = ci
     L.fp8gmm_route_invert.argtypes = [vp, ci, vp, vp]
     L.fp8gmm_moe_scatter_backward.restype = ci

@@ -13,7 +13,8 @@
 //
 // Sorting is a counting sort in three small launches (ids are < 4096 and the list is at most a few hundred
 // thousand entries): per-chunk histograms, a scan that turns them into start offsets, and a stable placement in
-// which a single-wavefront workgroup walks its chunk in order.  The row movers are HBM-bound: one wavefront per
+// which a single-wavefront workgroup walks its chunk in order; a short list takes the three steps in one workgroup of
+// one launch.  The row movers are HBM-bound: one wavefront per
 // row, 16 bytes per lane per access.
 #include "device_utils.h"
 
@@ -23,15 +24,19 @@ namespace {
 constexpr int kRouteChunk = 512;        // list entries per workgroup of the counting sort
 constexpr int kRouteSteps = kRouteChunk / 64;
 constexpr int kRouteMaxExperts = 4096;  // size of the per-workgroup expert table in LDS (16 KB)
+constexpr int kRouteSmallWaves = 16;      // a list of at most so many chunks ..
+constexpr int kRouteSmallExperts = 512;   // .. over so many experts is sorted by one workgroup (32 KB of tables)
 constexpr int kRowWaves = 4;            // wavefronts (= rows in flight) per workgroup of the row movers
 
+// `int64_t` ids are taken by their low 32 bits, as a conversion to int32 before the call would leave them
 __device__ __forceinline__ int clamp_expert(int e, int num_experts) {
   return e < 0 ? 0 : (e >= num_experts ? num_experts - 1 : e);
 }
 
 // counts[b][e] = entries of chunk b that go to expert e
-__global__ __launch_bounds__(64) void route_count_kernel(const int32_t* __restrict__ expert_of, int n,
-                                                         int num_experts, int32_t* __restrict__ counts) {
+template <typename Id>
+__global__ __launch_bounds__(64) void route_count_kernel(const Id* __restrict__ expert_of, int n, int num_experts,
+                                                         int32_t* __restrict__ counts) {
   __shared__ int32_t table[kRouteMaxExperts];
   const int lane = threadIdx.x;
   for (int e = lane; e < num_experts; e += 64) table[e] = 0;
@@ -41,7 +46,7 @@ __global__ __launch_bounds__(64) void route_count_kernel(const int32_t* __restri
 #pragma unroll
   for (int r = 0; r < kRouteSteps; ++r) {
     const int64_t i = base + r * 64 + lane;
-    ids[r] = i < n ? expert_of[i] : -1;
+    ids[r] = i < n ? (int32_t)expert_of[i] : -1;
   }
 #pragma unroll
   for (int r = 0; r < kRouteSteps; ++r)
@@ -118,11 +123,23 @@ __global__ __launch_bounds__(256) void route_scan_kernel(int32_t* __restrict__ c
   for (int64_t i = tid; i < cells; i += 256) counts[i] += total[i % num_experts];
 }
 
+// The lanes that hold the same expert as this one, found bit by bit of the expert id: one ballot per bit,
+// ceil(log2(num_experts)) of them, whatever the number of distinct experts in the wavefront.
+__device__ __forceinline__ uint64_t same_expert(int e, bool valid, int bits) {
+  uint64_t same = __ballot(valid);
+  for (int k = 0; k < bits; ++k) {
+    const bool set = (e >> k) & 1;
+    const uint64_t has = __ballot(valid && set);
+    same &= set ? has : ~has;
+  }
+  return same;
+}
+
 // Stable placement: the single wavefront of a workgroup walks its chunk 64 entries at a time, in order; within
 // a group of 64 an entry's rank among the entries of the same expert is the number of lower lanes that hold
-// that expert.  The lanes that hold the same expert are found bit by bit of the expert id: one ballot per bit,
-// ceil(log2(num_experts)) of them, whatever the number of distinct experts in the group.
-__global__ __launch_bounds__(64) void route_place_kernel(const int32_t* __restrict__ expert_of, int n,
+// that expert.
+template <typename Id>
+__global__ __launch_bounds__(64) void route_place_kernel(const Id* __restrict__ expert_of, int n,
                                                          int num_experts, const int32_t* __restrict__ offsets,
                                                          int32_t* __restrict__ bin_ids,
                                                          int32_t* __restrict__ indices,
@@ -139,19 +156,14 @@ __global__ __launch_bounds__(64) void route_place_kernel(const int32_t* __restri
 #pragma unroll
   for (int r = 0; r < kRouteSteps; ++r) {
     const int64_t i = base + r * 64 + lane;
-    ids[r] = i < n ? expert_of[i] : 0;
+    ids[r] = i < n ? (int32_t)expert_of[i] : 0;
   }
 #pragma unroll
   for (int r = 0; r < kRouteSteps; ++r) {
     const int64_t i = base + r * 64 + lane;
     const bool valid = i < n;
     const int e = valid ? clamp_expert(ids[r], num_experts) : 0;
-    uint64_t same = __ballot(valid);
-    for (int k = 0; k < bits; ++k) {
-      const bool set = (e >> k) & 1;
-      const uint64_t has = __ballot(valid && set);
-      same &= set ? has : ~has;
-    }
+    const uint64_t same = same_expert(e, valid, bits);
     // for a valid lane `same` now marks the valid lanes with its expert
     const int pos = valid ? next[e] + __popcll(same & below) : 0;
     __syncthreads();
@@ -160,6 +172,92 @@ __global__ __launch_bounds__(64) void route_place_kernel(const int32_t* __restri
     if (valid) {
       if (bin_ids != nullptr) bin_ids[pos] = e;
       if (indices != nullptr) indices[pos] = (int32_t)i;
+      if (inverse != nullptr) inverse[i] = pos;
+    }
+  }
+}
+
+// The whole sort of a short list in one launch of one workgroup: its wavefronts are the chunks, their tables stay in LDS.
+// Bound by the latency of a launch and of the LDS steps.  Entries x experts, one launch against three, back to back:
+// 512 x 4 5.4 us (9.6), 3062 x 16 8.3 (12.7), 3062 x 128 10.6 (29.2), 8192 x 4 11.5 (10.5), 8192 x 16 11.9 (12.8),
+// 8192 x 128 14.6 (30.2), 8192 x 512 18.5 (28.0): the lines are where one workgroup has no more entries to a lane.
+// Where the host is the limit, two launches less count for more than these.
+template <typename Id>
+__global__ __launch_bounds__(kRouteSmallWaves * 64) void route_small_kernel(
+    const Id* __restrict__ expert_of, int n, int num_experts, int32_t* __restrict__ bin_ids,
+    int32_t* __restrict__ indices, int32_t* __restrict__ inverse, int32_t* __restrict__ tokens_per_expert,
+    int32_t* __restrict__ bins) {
+  __shared__ int32_t table[kRouteSmallWaves][kRouteSmallExperts];
+  __shared__ int32_t end[kRouteSmallExperts];
+  const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  // chunks of whole groups of 64, shared out evenly
+  const int steps = (n + kRouteSmallWaves * 64 - 1) / (kRouteSmallWaves * 64);  // at most kRouteSteps
+  const int base = wave * steps * 64;
+  int32_t ids[kRouteSteps];  // all loads of the chunk in flight at once
+#pragma unroll
+  for (int r = 0; r < kRouteSteps; ++r) {
+    const int i = base + r * 64 + lane;
+    ids[r] = r < steps && i < n ? clamp_expert((int32_t)expert_of[i], num_experts) : -1;
+  }
+  for (int e = lane; e < num_experts; e += 64) table[wave][e] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kRouteSteps; ++r)
+    if (ids[r] >= 0) atomicAdd(&table[wave][ids[r]], 1);
+  __syncthreads();
+  // a thread per expert: its chunks' counts become starts within the expert, then the first wavefront's scan over the
+  // experts gives where each expert ends
+  if (tid < num_experts) {
+    int32_t run = 0;
+#pragma unroll
+    for (int w = 0; w < kRouteSmallWaves; ++w) {
+      const int32_t c = table[w][tid];
+      table[w][tid] = run;
+      run += c;
+    }
+    end[tid] = run;
+    if (tokens_per_expert != nullptr) tokens_per_expert[tid] = run;
+  }
+  __syncthreads();
+  if (wave == 0) {
+    int32_t run = 0;
+    for (int e0 = 0; e0 < num_experts; e0 += 64) {
+      const int e = e0 + lane;
+      int32_t incl = e < num_experts ? end[e] : 0;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const int32_t below = __shfl_up(incl, d, 64);
+        if (lane >= d) incl += below;
+      }
+      if (e < num_experts) {
+        end[e] = run + incl;
+        if (bins != nullptr) bins[e] = run + incl;
+      }
+      run += __shfl(incl, 63, 64);
+    }
+  }
+  __syncthreads();
+  if (tid < num_experts) {
+    const int32_t start = tid > 0 ? end[tid - 1] : 0;
+#pragma unroll
+    for (int w = 0; w < kRouteSmallWaves; ++w) table[w][tid] += start;
+  }
+  __syncthreads();
+  const uint64_t below = (1ull << lane) - 1ull;
+  int bits = 0;
+  while ((1 << bits) < num_experts) ++bits;
+#pragma unroll
+  for (int r = 0; r < kRouteSteps; ++r) {
+    const int e = ids[r];
+    const uint64_t same = same_expert(e, e >= 0, bits);
+    const int pos = e >= 0 ? table[wave][e] + __popcll(same & below) : 0;
+    __syncthreads();
+    if (e >= 0 && (same & below) == 0) table[wave][e] += __popcll(same);  // the lowest lane of every expert's group
+    __syncthreads();
+    if (e >= 0) {
+      const int i = base + r * 64 + lane;
+      if (bin_ids != nullptr) bin_ids[pos] = e;
+      if (indices != nullptr) indices[pos] = i;
       if (inverse != nullptr) inverse[i] = pos;
     }
   }
@@ -488,25 +586,56 @@ size_t fp8gmm_route_workspace_bytes(int n, int num_experts) {
   return chunks * (size_t)num_experts * sizeof(int32_t);
 }
 
-int fp8gmm_route_sort(const int32_t* expert_of, int n, int num_experts, int32_t* bin_ids, int32_t* indices,
-                      int32_t* inverse, int32_t* tokens_per_expert, int32_t* bins, void* workspace, void* stream) {
-  using namespace fp8gmm;
+}  // extern "C"
+
+namespace fp8gmm {
+namespace {
+
+template <typename Id>
+int route_sort(const Id* expert_of, int n, int num_experts, int32_t* bin_ids, int32_t* indices, int32_t* inverse,
+               int32_t* tokens_per_expert, int32_t* bins, void* workspace, void* stream) {
   if (n < 0 || num_experts < 1 || num_experts > kRouteMaxExperts) return FP8GMM_ERR_BAD_ARGUMENT;
   if (workspace == nullptr && n > 0) return FP8GMM_ERR_NULL_POINTER;
   if (n > 0 && expert_of == nullptr) return FP8GMM_ERR_NULL_POINTER;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  const bool totals = tokens_per_expert != nullptr || bins != nullptr;
+  const bool places = bin_ids != nullptr || indices != nullptr || inverse != nullptr;
+  if (n <= kRouteSmallWaves * kRouteChunk && num_experts <= kRouteSmallExperts) {
+    if (totals || (n > 0 && places))
+      hipLaunchKernelGGL(route_small_kernel<Id>, dim3(1), dim3(kRouteSmallWaves * 64), 0, s, expert_of, n, num_experts,
+                         bin_ids, indices, inverse, tokens_per_expert, bins);
+    return hipGetLastError() == hipSuccess ? FP8GMM_OK : FP8GMM_ERR_LAUNCH;
+  }
   const int chunks = (n + kRouteChunk - 1) / kRouteChunk;
   int32_t* counts = static_cast<int32_t*>(workspace);
   if (chunks > 0)
-    hipLaunchKernelGGL(route_count_kernel, dim3(chunks), dim3(64), 0, s, expert_of, n, num_experts, counts);
+    hipLaunchKernelGGL(route_count_kernel<Id>, dim3(chunks), dim3(64), 0, s, expert_of, n, num_experts, counts);
   // with an empty list the scan still writes the (all-zero) totals and bins
-  if (chunks > 0 || tokens_per_expert != nullptr || bins != nullptr)
+  if (chunks > 0 || totals)
     hipLaunchKernelGGL(route_scan_kernel, dim3(1), dim3(256), 0, s, counts, chunks, num_experts, tokens_per_expert,
                        bins);
-  if (chunks > 0 && (bin_ids != nullptr || indices != nullptr || inverse != nullptr))
-    hipLaunchKernelGGL(route_place_kernel, dim3(chunks), dim3(64), 0, s, expert_of, n, num_experts, counts, bin_ids,
+  if (chunks > 0 && places)
+    hipLaunchKernelGGL(route_place_kernel<Id>, dim3(chunks), dim3(64), 0, s, expert_of, n, num_experts, counts, bin_ids,
                        indices, inverse);
   return hipGetLastError() == hipSuccess ? FP8GMM_OK : FP8GMM_ERR_LAUNCH;
+}
+
+}  // namespace
+}  // namespace fp8gmm
+
+extern "C" {
+
+int fp8gmm_route_sort(const int32_t* expert_of, int n, int num_experts, int32_t* bin_ids, int32_t* indices,
+                      int32_t* inverse, int32_t* tokens_per_expert, int32_t* bins, void* workspace, void* stream) {
+  return fp8gmm::route_sort(expert_of, n, num_experts, bin_ids, indices, inverse, tokens_per_expert, bins, workspace,
+                            stream);
+}
+
+int fp8gmm_route_sort_selected(const int64_t* selected, int n, int num_experts, int32_t* bin_ids, int32_t* indices,
+                               int32_t* inverse, int32_t* tokens_per_expert, int32_t* bins, void* workspace,
+                               void* stream) {
+  return fp8gmm::route_sort(selected, n, num_experts, bin_ids, indices, inverse, tokens_per_expert, bins, workspace,
+                            stream);
 }
 
 int fp8gmm_route_invert(const int32_t* indices, int n, int32_t* inverse, void* stream) {

@@ -33,7 +33,7 @@ class _RoutedModule(torch.nn.Module):
     def start_experts(self):
         """Enqueue what the experts' pass can do before the host knows the split (nothing, by default)."""
 
-    def compute(self, x, tokens_per_expert, indices, bin_ids, expert_weights, bins, top_k):
+    def compute(self, x, tokens_per_expert, indices, bin_ids, expert_weights, bins, top_k, inverse=None):
         x = x.view(-1, x.size(-1))
         # The host needs the split to plan the expert launches.  Its copy is enqueued ahead of the gather and of the
         # experts' weight casts, which need nothing from the host: the GPU has that work to do while the host waits
@@ -43,12 +43,12 @@ class _RoutedModule(torch.nn.Module):
             self._counts_ready = torch.cuda.Event()
         self._counts_host.copy_(tokens_per_expert, non_blocking=True)
         self._counts_ready.record()
-        x = moe_ops.gather(x, indices, bin_ids, bins, top_k)
+        x = moe_ops.gather(x, indices, bin_ids, bins, top_k, inverse)
         self.start_experts()
         self._counts_ready.synchronize()
         batch_sizes = self._counts_host.to(torch.long, copy=True)   # the page-locked buffer is reused by the next step
         out = self.experts(x, batch_sizes)
-        return moe_ops.scatter(out, indices, bin_ids, expert_weights, bins, top_k)
+        return moe_ops.scatter(out, indices, bin_ids, expert_weights, bins, top_k, inverse)
 
     def forward(self, input):
         input = input.view(-1, input.size(-1))
@@ -57,9 +57,11 @@ class _RoutedModule(torch.nn.Module):
         expert_weights = weights0.flatten()
         top_experts = selected_experts.flatten()
         with torch.no_grad():
-            indices, bin_ids, bins, tokens_per_expert = moe_ops.indices_and_bins(
-                top_experts, self.sort_end_bit, self.n_experts)
-        return self.compute(input, tokens_per_expert, indices, bin_ids, expert_weights, bins, self.top_k)
+            indices, bin_ids, bins, tokens_per_expert, inverse = moe_ops.indices_bins_and_inverse(
+                top_experts, self.n_experts)
+        # another compute, of a subclass or set on the module, is called as ever, without the inverse
+        more = (inverse,) if getattr(self.compute, "__func__", None) is _RoutedModule.compute else ()
+        return self.compute(input, tokens_per_expert, indices, bin_ids, expert_weights, bins, self.top_k, *more)
 
 
 class Fp8LinearModule(_RoutedModule):

@@ -31,13 +31,13 @@ def _check_ids(x):
         _fail("fp8_gmm_amd: expert ids must be a contiguous 1-D int32 tensor")
 
 
-def route(top_expert, num_experts, want_sort=True, want_inverse=False, want_counts=True):
-    """One pass over the expert ids: ``(bin_ids, indices, inverse, tokens_per_expert, bins)``, None where not asked for."""
-    _check_ids(top_expert)
+def _check_experts(num_experts):
     if not 1 <= num_experts <= MAX_EXPERTS:
         _fail(f"fp8_gmm_amd: between 1 and {MAX_EXPERTS} experts are supported, got {num_experts}")
+
+
+def _route(sort_ids, top_expert, num_experts, want_sort, want_inverse, want_counts):
     n, dev = top_expert.numel(), top_expert.device
-    L = _lib.load()
 
     def new(count):
         return torch.empty(count, dtype=torch.int32, device=dev)
@@ -47,16 +47,23 @@ def route(top_expert, num_experts, want_sort=True, want_inverse=False, want_coun
     inverse = new(n) if want_inverse else None
     counts = new(num_experts) if want_counts else None
     bins = new(num_experts) if want_counts else None
-    work = torch.empty(L.fp8gmm_route_workspace_bytes(n, num_experts), dtype=torch.uint8, device=dev)
+    work = torch.empty(_lib.load().fp8gmm_route_workspace_bytes(n, num_experts), dtype=torch.uint8, device=dev)
 
     def ptr(t):
         return t.data_ptr() if t is not None and t.numel() else None
 
     with torch.cuda.device(dev):
-        rc = L.fp8gmm_route_sort(ptr(top_expert), n, num_experts, ptr(bin_ids), ptr(indices), ptr(inverse),
-                                 ptr(counts), ptr(bins), ptr(work), _stream(dev))
+        rc = sort_ids(ptr(top_expert), n, num_experts, ptr(bin_ids), ptr(indices), ptr(inverse), ptr(counts), ptr(bins),
+                      ptr(work), _stream(dev))
     _lib.check(rc)
     return bin_ids, indices, inverse, counts, bins
+
+
+def route(top_expert, num_experts, want_sort=True, want_inverse=False, want_counts=True):
+    """One pass over the expert ids: ``(bin_ids, indices, inverse, tokens_per_expert, bins)``, None where not asked for."""
+    _check_ids(top_expert)
+    _check_experts(num_experts)
+    return _route(_lib.load().fp8gmm_route_sort, top_expert, num_experts, want_sort, want_inverse, want_counts)
 
 
 def sort(x, end_bit=None):
@@ -83,9 +90,21 @@ def indices_and_bins(top_expert, sort_end_bit, n_experts):
     """``(indices, bin_ids, bins, tokens_per_expert)`` as the example's helper of the same name returns them
     (fp8_gmm/example.py:26-32), from one library call instead of three operators."""
     del sort_end_bit  # the counting sort needs the expert count, not a bit count
-    top_expert = top_expert.int().contiguous()
-    bin_ids, indices, _, tokens_per_expert, bins = route(top_expert, n_experts)
+    indices, bin_ids, bins, tokens_per_expert, _ = indices_bins_and_inverse(top_expert, n_experts, False)
     return indices, bin_ids, bins, tokens_per_expert
+
+
+def indices_bins_and_inverse(top_expert, n_experts, want_inverse=True):
+    """The four of ``indices_and_bins`` and the inverse of ``indices``, for ``gather`` and ``scatter``."""
+    if top_expert.dtype == torch.int64 and top_expert.is_cuda and top_expert.dim() == 1:
+        # the router's choices as they are, without a conversion in front
+        _check_experts(n_experts)
+        bin_ids, indices, inverse, tokens_per_expert, bins = _route(
+            _lib.load().fp8gmm_route_sort_selected, top_expert.contiguous(), n_experts, True, want_inverse, True)
+    else:
+        bin_ids, indices, inverse, tokens_per_expert, bins = route(top_expert.int().contiguous(), n_experts,
+                                                                   want_inverse=want_inverse)
+    return indices, bin_ids, bins, tokens_per_expert, inverse
 
 
 MAX_GATING_EXPERTS = 128
@@ -267,23 +286,24 @@ def _scatter_rows(x, inverse, weights, top_k):
 
 class _Gather(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x, indices, top_k):
-        ctx.save_for_backward(indices)
+    def forward(ctx, x, indices, top_k, inverse):
+        ctx.save_for_backward(indices if inverse is None else None, inverse)
         ctx.top_k = top_k
         return _gather_rows(x, indices, None, top_k)
 
     @staticmethod
     def backward(ctx, grad):
-        (indices,) = ctx.saved_tensors
-        return _scatter_rows(grad.contiguous(), _invert(indices), None, ctx.top_k), None, None
+        indices, inverse = ctx.saved_tensors
+        inverse = _invert(indices) if inverse is None else inverse
+        return _scatter_rows(grad.contiguous(), inverse, None, ctx.top_k), None, None, None
 
 
 class _Scatter(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x, indices, weights, top_k):
+    def forward(ctx, x, indices, weights, top_k, inverse):
         ctx.save_for_backward(x if weights is not None and ctx.needs_input_grad[2] else None, indices, weights)
         ctx.top_k = top_k
-        return _scatter_rows(x, _invert(indices), weights, top_k)
+        return _scatter_rows(x, _invert(indices) if inverse is None else inverse, weights, top_k)
 
     @staticmethod
     def backward(ctx, grad):
@@ -299,7 +319,7 @@ class _Scatter(torch.autograd.Function):
                                                              weights.data_ptr(), grad_x.data_ptr(), grad_w.data_ptr(),
                                                              rows, hidden, ctx.top_k, _stream(grad.device))
             _lib.check(rc)
-            return grad_x, None, grad_w, None
+            return grad_x, None, grad_w, None, None
         grad_x = _gather_rows(grad, indices, weights, ctx.top_k) if ctx.needs_input_grad[0] else None
         grad_w = None
         if weights is not None and ctx.needs_input_grad[2]:
@@ -309,31 +329,36 @@ class _Scatter(torch.autograd.Function):
                                                           grad_w.data_ptr(), x.shape[0], x.shape[1], ctx.top_k,
                                                           _stream(grad.device))
             _lib.check(rc)
-        return grad_x, None, grad_w, None
+        return grad_x, None, grad_w, None, None
 
 
-def gather(x, indices, bin_ids, bins, top_k):
+def gather(x, indices, bin_ids, bins, top_k, inverse=None):
     """Rows of ``x[tokens, hidden]`` into expert order: ``out[i] = x[indices[i] // top_k]``, ``[tokens * top_k,
     hidden]`` (``megablocks.ops.gather``; ``bin_ids`` and ``bins`` are accepted for that signature and unused).
-    Differentiable in ``x``."""
+    ``inverse``: that of ``indices``, where the caller has it.  Differentiable in ``x``."""
     del bin_ids, bins
     _check_rows(x, "gather input")
     _check_indices(indices, x.shape[0] * top_k)
-    return _Gather.apply(x.contiguous(), indices, int(top_k))
+    if inverse is not None:
+        _check_indices(inverse, x.shape[0] * top_k)
+    return _Gather.apply(x.contiguous(), indices, int(top_k), inverse)
 
 
-def scatter(x, indices, bin_ids, weights, bins, top_k):
+def scatter(x, indices, bin_ids, weights, bins, top_k, inverse=None):
     """Rows in expert order back to token order, weighted: ``out[t] = sum_k weights[t * top_k + k] * x[pos(t, k)]``
     with ``pos`` the inverse of ``indices``; ``weights`` ``[tokens * top_k]`` in (token, choice) order, or None for
-    a plain sum (``megablocks.ops.scatter``).  Differentiable in ``x`` and ``weights``."""
+    a plain sum (``megablocks.ops.scatter``).  ``inverse``: that of ``indices``, where the caller has it.
+    Differentiable in ``x`` and ``weights``."""
     del bin_ids, bins
     _check_rows(x, "scatter input")
     top_k = int(top_k)
     if x.shape[0] % top_k:
         _fail("fp8_gmm_amd: scatter needs tokens * top_k rows")
     _check_indices(indices, x.shape[0])
+    if inverse is not None:
+        _check_indices(inverse, x.shape[0])
     if weights is not None:
         if weights.numel() != x.shape[0]:
             _fail(f"fp8_gmm_amd: expected {x.shape[0]} scatter weights, got {weights.numel()}")
         weights = weights.reshape(-1).float().contiguous()  # differentiable; a no-op for the example's fp32 weights
-    return _Scatter.apply(x.contiguous(), indices, weights, top_k)
+    return _Scatter.apply(x.contiguous(), indices, weights, top_k, inverse)

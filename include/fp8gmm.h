@@ -588,6 +588,10 @@ int fp8gmm_upload(void* dst_dev, const void* src_host, size_t bytes, void* strea
 size_t fp8gmm_route_workspace_bytes(int n, int num_experts);
 int fp8gmm_route_sort(const int32_t* expert_of, int n, int num_experts, int32_t* bin_ids, int32_t* indices,
                       int32_t* inverse, int32_t* tokens_per_expert, int32_t* bins, void* workspace, void* stream);
+/* The same on the ids as fp8gmm_route_topk writes them (`selected`, the low 32 bits of each). */
+int fp8gmm_route_sort_selected(const int64_t* selected, int n, int num_experts, int32_t* bin_ids, int32_t* indices,
+                               int32_t* inverse, int32_t* tokens_per_expert, int32_t* bins, void* workspace,
+                               void* stream);
 /*
  * The router's choice, replacing `topk` of fp8_gmm/example.py:15-23 (softmax over the experts in fp32, then
  * torch.topk; without its moe_renorm option): probs[t, :] = softmax(scores[t, :]) and, for k < top_k (at most 8),

@@ -54,6 +54,24 @@ def test_sort_histogram_and_bins(dev, n, e, kind):
     assert inverse.cpu().tolist() == orc.invert(want_indices).tolist()
 
 
+@pytest.mark.parametrize("n,e", [(1, 512), (1024, 512), (1025, 300), (3062, 16), (8192, 128), (8193, 128), (8192, 513)])
+def test_short_lists_and_the_routers_own_ids(dev, n, e):
+    """Both sides of the limits of the one-launch sort; int64 ids, some out of range, give what their int32 conversion gives."""
+    ops = _ops()
+    ids = _ids(n, e, 7 + n, "zipf")
+    ids[::97] = -5
+    ids[1::89] = e + 3
+    want_indices, want_bin_ids, want_bins, want_counts = orc.indices_and_bins(ids.clip(0, e - 1), e)
+    for x in (torch.tensor(ids, device=dev), torch.tensor(ids, dtype=torch.int32, device=dev)):
+        indices, bin_ids, bins, counts, inverse = ops.indices_bins_and_inverse(x, e)
+        assert indices.cpu().tolist() == want_indices.tolist()
+        assert bin_ids.cpu().tolist() == want_bin_ids.tolist()
+        assert counts.cpu().tolist() == want_counts.tolist()
+        assert bins.cpu().tolist() == want_bins.tolist()
+        assert inverse.cpu().tolist() == orc.invert(want_indices).tolist()
+        assert all(torch.equal(a, b) for a, b in zip(ops.indices_and_bins(x, 1, e), (indices, bin_ids, bins, counts)))
+
+
 def test_out_of_range_ids_are_clamped(dev):
     ops = _ops()
     x = torch.tensor([5, -3, 2, 9, 0], dtype=torch.int32, device=dev)
