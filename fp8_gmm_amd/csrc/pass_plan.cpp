@@ -385,10 +385,11 @@ int lay_out_pass(Pass& pass, fp8gmm_pass_plan* out, PassTables* t) {
   t->experts = e;
   t->n_casts = t->n_gemms = 0;
   int64_t rows = 0;
+  t->row_begin[0] = 0;
   for (int i = 0; i < e; ++i) {
     rows += pass.group_sizes[i];
     if (pass.group_sizes[i] > INT32_MAX / 2 || rows > FP8GMM_PASS_MAX_ROWS) return FP8GMM_ERR_BAD_SHAPE;
-    t->rows[i] = (int32_t)pass.group_sizes[i];
+    t->row_begin[i + 1] = (int32_t)rows;
   }
   static thread_local std::vector<fp8gmm_gemm_problem> scratch;
   scratch.resize((size_t)e + 1);

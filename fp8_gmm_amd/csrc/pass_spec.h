@@ -84,7 +84,7 @@ struct PassTables {
   CastSpec cast[kPassMaxCasts];
   GemmSpec gemm[kPassMaxGemms];
   GemmRanges ranges[kPassMaxGemms];
-  int32_t rows[kPassMaxExperts];
+  int32_t row_begin[kPassMaxExperts + 1];               // rows in front of every expert, of all of them behind the last
 };
 static_assert(sizeof(PassTables) <= FP8GMM_PASS_TABLES_BYTES, "the opaque buffer of the C ABI");
 

@@ -26,48 +26,86 @@ constexpr int kThreads = 256;
 constexpr int kExperts = kPassMaxExperts;
 static_assert(kPassRecordsPerBlock == kThreads, "a lane per record");
 
-// exclusive prefix sums of v[0 .. n) in place, their total in v[n]; all threads of the workgroup
-__device__ void exclusive_scan(int* v, int n, int* wave_sums) {
-  const int lane = threadIdx.x % kWaveSize, wave = threadIdx.x / kWaveSize;
-  int carry = 0;
-  for (int base = 0; base < n; base += kThreads) {
-    const int i = base + (int)threadIdx.x;
-    const int own = i < n ? v[i] : 0;
-    int sum = own;   // inclusive over the wavefront
-    for (int d = 1; d < kWaveSize; d <<= 1) {
-      const int up = __shfl_up(sum, d);
-      if (lane >= d) sum += up;
-    }
-    if (lane == kWaveSize - 1) wave_sums[wave] = sum;
-    __syncthreads();
-    int before = carry;
-    for (int w = 0; w < wave; ++w) before += wave_sums[w];
-    for (int w = 0; w < kThreads / kWaveSize; ++w) carry += wave_sums[w];
-    if (i < n) v[i] = before + sum - own;
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) v[n] = carry;
-  __syncthreads();
+// Inclusive sums over a wavefront, all of whose lanes are here: four shifts inside rows of 16 lanes, then the last lane of
+// rows 0 and 2 to the row behind and that of the lower half to the upper one.  Data-parallel primitives: a shuffle through
+// LDS is ten times as far away, and six of them follow each other.
+__device__ __forceinline__ int wave_inclusive(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr:1, 2, 4, 8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31
+  return v;
 }
 
-__device__ void write_cast(const PassTables& t, const CastSpec& spec, uint8_t* blob, const int* row_begin, int* scan,
-                           int* wave_sums) {
+constexpr int kScans = 3;   // lists that are summed side by side
+struct Scan {
+  int v[kScans];
+};
+
+// Exclusive prefix sums of `kScans` lists at once: `value(i)` are the entries i of [0, n), n >= 1; `take(i, sums)` gets the
+// sums in front of entry i, in the thread that gave its values; the totals are returned.  All threads of the workgroup; what
+// `value` and `take` have stored is visible to all of them behind it.
+template <typename Value, typename Take>
+__device__ __forceinline__ Scan exclusive_scan(int n, int (*wave_sums)[kThreads / kWaveSize], Value value, Take take) {
+  const int lane = threadIdx.x % kWaveSize, wave = threadIdx.x / kWaveSize;
+  Scan carry = {};
+#pragma unroll 1
+  for (int base = 0; base < n; base += kThreads) {
+    const int i = base + (int)threadIdx.x;
+    Scan own = {}, sum;
+    if (i < n) own = value(i);
+#pragma unroll
+    for (int q = 0; q < kScans; ++q) {
+      sum.v[q] = wave_inclusive(own.v[q]);
+      if (lane == kWaveSize - 1) wave_sums[q][wave] = sum.v[q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kScans; ++q) {
+      sum.v[q] += carry.v[q] - own.v[q];
+#pragma unroll
+      for (int w = 0; w < kThreads / kWaveSize; ++w) {
+        const int of = wave_sums[q][w];
+        sum.v[q] += w < wave ? of : 0;
+        carry.v[q] += of;
+      }
+    }
+    if (i < n) take(i, sum);
+    __syncthreads();
+  }
+  return carry;
+}
+
+// `sums`: room for the sums of every run
+__device__ void write_cast(const PassTables& t, const CastSpec& spec, uint8_t* blob, const int* row_begin,
+                           int* const (&sums)[kScans], int (*wave_sums)[kThreads / kWaveSize]) {
+  static_assert(sizeof(spec.run) / sizeof(spec.run[0]) == kScans, "the runs of a cast side by side");
   fp8gmm_tensor_desc* out = reinterpret_cast<fp8gmm_tensor_desc*>(blob + spec.table_offset);
+  const Scan total = exclusive_scan(
+      t.experts, wave_sums,
+      [&](int i) {
+        Scan own = {};
+#pragma unroll
+        for (int s = 0; s < kScans; ++s)
+          if (s < spec.n_runs) own.v[s] = cast_blocks(cast_desc(spec.run[s], i, row_begin[i], row_begin[i + 1] - row_begin[i]));
+        return own;
+      },
+      [&](int i, const Scan& before) {
+#pragma unroll
+        for (int s = 0; s < kScans; ++s) sums[s][i] = before.v[s];
+      });
   int block = 0;
-  for (int s = 0; s < spec.n_runs; ++s) {
-    for (int i = threadIdx.x; i < t.experts; i += kThreads) {
-      const int rows = row_begin[i + 1] - row_begin[i];
-      scan[i] = cast_blocks(cast_desc(spec.run[s], i, row_begin[i], rows));
-    }
-    __syncthreads();
-    exclusive_scan(scan, t.experts, wave_sums);
-    for (int i = threadIdx.x; i < t.experts; i += kThreads) {
-      fp8gmm_tensor_desc d = cast_desc(spec.run[s], i, row_begin[i], row_begin[i + 1] - row_begin[i]);
-      d.block_begin = block + scan[i];
-      out[s * t.experts + i] = d;
-    }
-    block += scan[t.experts];
-    __syncthreads();
+#pragma unroll
+  for (int s = 0; s < kScans; ++s) {
+    if (s < spec.n_runs)
+      for (int i = threadIdx.x; i < t.experts; i += kThreads) {
+        fp8gmm_tensor_desc d = cast_desc(spec.run[s], i, row_begin[i], row_begin[i + 1] - row_begin[i]);
+        d.block_begin = block + sums[s][i];
+        out[s * t.experts + i] = d;
+      }
+    block += total.v[s];
   }
 }
 
@@ -123,48 +161,46 @@ struct Gemm {   // one GEMM's view inside a workgroup; the arrays are in LDS
 };
 
 __device__ void write_gemm(const PassTables& t, int g, int block, uint8_t* blob, const int* row_begin,
-                           fp8gmm_gemm_problem* probs, int* begin, int* cost, int* slots, int* wave_sums) {
+                           fp8gmm_gemm_problem* probs, int* begin, int* cost, int* slots,
+                           int (*wave_sums)[kThreads / kWaveSize]) {
   const GemmSpec& spec = t.gemm[g];
   const GemmRanges& ranges = t.ranges[g];
   const int n = t.experts;
   const Gemm gm{spec, ranges, probs, begin, cost, n, ranges.grid / kNumXcd, spec.tile_m == BM && spec.tile_n == BN};
-  // problems, the tiles and K steps in front of each (in 256 x 256 tiles: what the problem table records)
-  for (int i = threadIdx.x; i < n; i += kThreads) {
-    probs[i] = gemm_problem(spec, i, row_begin[i], row_begin[i + 1] - row_begin[i]);
-    const int tiles = ((probs[i].m + BM - 1) / BM) * ((probs[i].n + BN - 1) / BN);
-    begin[i] = tiles;
-    cost[i] = tiles * gm.steps_of(i);
-  }
-  __syncthreads();
-  exclusive_scan(begin, n, wave_sums);
-  exclusive_scan(cost, n, wave_sums);
-  for (int i = threadIdx.x; i < n; i += kThreads) {
-    probs[i].tile_begin = begin[i];
-    probs[i].cost_begin = cost[i];
-  }
-  __syncthreads();
+  // problems, the tiles and K steps in front of each (in 256 x 256 tiles: what the problem table records), and the tiles of
+  // the launch's own size
+  exclusive_scan(
+      n, wave_sums,
+      [&](int i) {
+        const fp8gmm_gemm_problem p = gemm_problem(spec, i, row_begin[i], row_begin[i + 1] - row_begin[i]);
+        probs[i] = p;
+        const int tiles = ((p.m + BM - 1) / BM) * ((p.n + BN - 1) / BN), steps = (p.k + 127) / 128;
+        const int own = ((p.m + spec.tile_m - 1) / spec.tile_m) * ((p.n + spec.tile_n - 1) / spec.tile_n);
+        return Scan{{tiles, tiles * (steps > 0 ? steps : 1), own}};
+      },
+      [&](int i, const Scan& before) {
+        probs[i].tile_begin = before.v[0];
+        probs[i].cost_begin = cost[i] = before.v[1];
+        begin[i] = before.v[2];
+      });
   if (block == 0) {
-    uint32_t* dst = reinterpret_cast<uint32_t*>(blob + spec.table_offset);
-    const uint32_t* src = reinterpret_cast<const uint32_t*>(probs);
+    static_assert(sizeof(fp8gmm_gemm_problem) % 16 == 0, "copied in words of 16 bytes");
+    u32x4* dst = reinterpret_cast<u32x4*>(blob + spec.table_offset);
+    const u32x4* src = reinterpret_cast<const u32x4*>(probs);
 #pragma unroll 1
-    for (int i = threadIdx.x; i < n * (int)(sizeof(fp8gmm_gemm_problem) / 4); i += kThreads) dst[i] = src[i];
+    for (int i = threadIdx.x; i < n * (int)(sizeof(fp8gmm_gemm_problem) / 16); i += kThreads) dst[i] = src[i];
   }
   if (ranges.total_tiles == 0) return;
-  if (!gm.large) {   // the launch's own tile counts
-    for (int i = threadIdx.x; i < n; i += kThreads)
-      begin[i] = ((probs[i].m + spec.tile_m - 1) / spec.tile_m) * ((probs[i].n + spec.tile_n - 1) / spec.tile_n);
-    __syncthreads();
-    exclusive_scan(begin, n, wave_sums);
-  }
   // Tiles shared along K: their workspace slots, numbered in the order (XCD, piece boundary); slots[i] becomes the first
   // slot of the tile that boundary i = (XCD, j) completes and, 16 bits up, the number of that tile.
   if (ranges.n_fixups > 0) {
-    for (int i = threadIdx.x; i < ranges.grid; i += kThreads) {
-      int p = 0, pieces = 0;
-      slots[i] = gm.completed_by(i / gm.wgs, i % gm.wgs, &p, &pieces) >= 0 ? pieces + (1 << 16) : 0;
-    }
-    __syncthreads();
-    exclusive_scan(slots, ranges.grid, wave_sums);
+    exclusive_scan(
+        ranges.grid, wave_sums,
+        [&](int i) {
+          int p = 0, pieces = 0;
+          return Scan{{gm.completed_by(i / gm.wgs, i % gm.wgs, &p, &pieces) >= 0 ? pieces + (1 << 16) : 0}};
+        },
+        [&](int i, const Scan& before) { slots[i] = before.v[0]; });
     if (block == 0) {
       fp8gmm_gemm_fixup_desc* fix = reinterpret_cast<fp8gmm_gemm_fixup_desc*>(blob + spec.fixups_offset);
 #pragma unroll 1
@@ -266,10 +302,11 @@ __global__ __launch_bounds__(kThreads) void pass_tables_kernel(const PassTables 
     run_scaling_update(updates, (int)blockIdx.x - update_block);
     return;
   }
-  __shared__ fp8gmm_gemm_problem probs[kExperts];
-  __shared__ int row_begin[kExperts + 1], begin[kExperts + 1], cost[kExperts + 1];
-  __shared__ int slots[FP8GMM_PASS_MAX_GRID + 1];
-  __shared__ int wave_sums[kThreads / kWaveSize];
+  __shared__ __attribute__((aligned(16))) fp8gmm_gemm_problem probs[kExperts];
+  __shared__ int begin[kExperts], cost[kExperts];
+  __shared__ int slots[FP8GMM_PASS_MAX_GRID];
+  static_assert(FP8GMM_PASS_MAX_GRID >= kExperts, "the third run of a cast");
+  __shared__ int wave_sums[kScans][kThreads / kWaveSize];
   static_assert(sizeof(PassTables) <= kThreads * 16, "four words per lane");
   __shared__ __attribute__((aligned(16))) uint32_t copy[kThreads * 4];
   const PassTables& t = *reinterpret_cast<const PassTables*>(copy);
@@ -290,16 +327,13 @@ __global__ __launch_bounds__(kThreads) void pass_tables_kernel(const PassTables 
     for (int i = threadIdx.x; i < copy_n; i += kThreads) copy_dst[i] = copy_src[i];
     return;
   }
-  for (int i = threadIdx.x; i < t.experts; i += kThreads) row_begin[i] = t.rows[i];
-  __syncthreads();
-  exclusive_scan(row_begin, t.experts, wave_sums);
   if (block < t.n_casts) {
-    write_cast(t, t.cast[block], blob, row_begin, begin, wave_sums);
+    write_cast(t, t.cast[block], blob, t.row_begin, {begin, cost, slots}, wave_sums);
     return;
   }
   int g = 0;
   while (g + 1 < t.n_gemms && block >= t.first_block[t.n_casts + g + 1]) ++g;
-  write_gemm(t, g, block - t.first_block[t.n_casts + g], blob, row_begin, probs, begin, cost, slots, wave_sums);
+  write_gemm(t, g, block - t.first_block[t.n_casts + g], blob, t.row_begin, probs, begin, cost, slots, wave_sums);
 }
 
 }  // namespace
