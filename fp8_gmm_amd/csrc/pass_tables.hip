@@ -14,6 +14,10 @@
 // copied to LDS with one load per lane at the start, not line by line as the code meets it) and its own instructions
 // (fetched line by line: one copy of every computation, 32-bit arithmetic - 64-bit divisions inlined from the host's
 // functions made it 34 KB and 12 - 16 us).
+// Then come steps that wait for each other: the prefix sums.  One round of them, several lists side by side and without LDS
+// inside a wavefront, against up to four rounds of shuffles, us a launch under a kernel trace: 8 experts 9.0 -> 6.0, 64 experts
+// 10.9 -> 7.3, 128 experts 10.0 -> 7.5, with tiles shared along K 14.7 -> 12.0 (the rest is numbering their slots); with the
+// update of 1280 columns on the side 13.2 -> 11.3, which is that update's time.
 #include "device_utils.h"
 #include "internal.h"
 #include "pass_spec.h"
