@@ -162,8 +162,9 @@ struct SkRemainder {
   int64_t c0, cost;      // cost before it, its own
   int n_splits;          // 0: not worth a thought
   SkSplit split[kSkMaxPieces];
+  // of `sk_times`, which wants the splits; where halves are through first, whole_x100 is their time from then on
   int64_t whole_x100, shared_x100[kSkMaxPieces], half_x100;
-  bool timed, halves;    // the times above are there; the remainder is better off in tiles of half height (whole_x100 says so)
+  bool timed, halves;
 };
 
 // A tile that k piece ends fall inside of is left in k + 1 slots; one that no end falls inside of needs none.
@@ -344,7 +345,7 @@ inline void sk_decide(const Sched (&all)[kNumXcd], SkRemainder (&rem)[kNumXcd], 
 inline void sched_init(Sched (&all)[kNumXcd], const fp8gmm_gemm_problem* probs, int nprob, int total_tiles, int wgs_per_xcd,
                        bool sk_enable, bool gelu = false, bool balanced = false) {
   const int W = wgs_per_xcd;
-  SkRemainder rem[kNumXcd];
+  SkRemainder rem[kNumXcd] = {};
   for (int x = 0; x < kNumXcd; ++x) {
     Sched& s = all[x];
     s.gelu = gelu;
@@ -365,11 +366,13 @@ inline void sched_init(Sched (&all)[kNumXcd], const fp8gmm_gemm_problem* probs, 
     s.sk_c0 = 0;
     s.sk_cost = 0;
     SkRemainder& r = rem[x];
-    r.n_splits = 0;
-    r.whole_x100 = 0;
-    r.timed = r.halves = false;
     r.tiles = n_x % W;
     r.begin = s.range_end - r.tiles;
+    if (sk_enable && remainder_may_share(n_x, W)) {
+      r.c0 = cost_before(s, r.begin);
+      r.cost = cost_before(s, s.range_end) - r.c0;
+      sk_splits(s, r);
+    }
     if (balanced && r.tiles > 0 && 2 * r.tiles <= W && n_x / W <= kHalfMaxRounds) {
       sk_times(s, r);
       if (r.half_x100 < r.whole_x100) {
@@ -377,10 +380,6 @@ inline void sched_init(Sched (&all)[kNumXcd], const fp8gmm_gemm_problem* probs, 
         r.whole_x100 = r.half_x100;
       }
     }
-    if (!sk_enable || !remainder_may_share(n_x, W)) continue;
-    r.c0 = cost_before(s, r.begin);
-    r.cost = cost_before(s, s.range_end) - r.c0;
-    sk_splits(s, r);
   }
   int pieces[kNumXcd] = {};
   if (sk_enable) sk_decide(all, rem, pieces);

@@ -228,15 +228,17 @@ def test_pieces_end_where_tiles_end_unless_whole_tiles_are_faster():
 
 # The rule for sharing, with everything counted from its definition: K = 128 steps of time, in hundredths.
 LAUNCH, PER_SLOT, GELU_PER_TILE = 400, 100, 150
+HALF_STEP, HALF_TILE, HALF_ROUNDS = 75, 300, 12   # of FP8GMM_GEMM_BALANCED, which also cuts the ranges at 2 steps a tile
 
 
-def shared_pieces(costs, wgs, gelu):
+def shared_pieces(costs, wgs, gelu, balanced=False):
     """costs: K steps of the tiles, in order.  Slots and shared tiles of a launch, if an XCD takes the number of pieces with
     which its last workgroup is through first, at the price of the XCDs that share, and the launch shares where its last XCD
-    is through sooner for it."""
+    is through sooner for it.  `balanced`: against a remainder that is cut into tiles of half height where that is faster than
+    whole ones; with the number of tiles that are cut so behind the two."""
     n = len(costs)
     before = np.concatenate([[0], np.cumsum(costs)])
-    work = before + 4 * np.arange(n + 1)
+    work = before + (2 if balanced else 4) * np.arange(n + 1)
     cut = [int(np.searchsorted(work, -(-int(work[-1]) * x // 8))) for x in range(9)]
     ranges = []   # per XCD: (time with whole tiles, [(time but for the slots, slots, tiles cut, tiles)])
     for x in range(8):
@@ -248,7 +250,12 @@ def shared_pieces(costs, wgs, gelu):
         for i in range(full):   # workgroup j's place in round i is j + 5 i
             load += own[i * wgs + (np.arange(wgs) + 5 * i) % wgs] + 4
         last = [int(load[j] + own[full * wgs + p]) + 4 for j in range(wgs) for p in [(j + 5 * full) % wgs] if p < rem]
-        whole, ways = max([int(load.max())] + last) * 100, []
+        whole, ways, halved = max([int(load.max())] + last) * 100, [], 0
+        if balanced and 0 < 2 * rem <= wgs and full <= HALF_ROUNDS:   # workgroup j's place names a tile and one of its halves
+            through = [int(load[j]) * 100 + HALF_STEP * int(own[full * wgs + p // 2]) + HALF_TILE
+                       for j in range(wgs) for p in [(j + 5 * full) % wgs] if p // 2 < rem]
+            if max([int(load.max()) * 100] + through) < whole:
+                whole, halved = max([int(load.max()) * 100] + through), rem
         ends = np.concatenate([[0], np.cumsum(own[full * wgs:])])
         cost, most = int(ends[-1]), min(wgs, int(ends[-1]) // 4, 8 * rem)
         if rem and full <= 24 and (wgs - rem) * 12 >= wgs * (full + 1):
@@ -257,18 +264,22 @@ def shared_pieces(costs, wgs, gelu):
                           if ends[t] != cost * j // pieces]
                 through = max(int(load.max()) * 100, (int(load[:pieces].max()) + 4) * 100 + cost * 100 // pieces)
                 ways.append((through, len(inside) + len(set(inside)), len(set(inside)), rem))
-        ranges.append((whole, ways))
+        ranges.append((whole, ways, halved))
+
+    def outcome(kept):   # per range: what it shares, None for nothing
+        cut = (sum(halved for k, (_, _, halved) in zip(kept, ranges) if not k),) if balanced else ()
+        return (sum(k[1] for k in kept if k), sum(k[2] for k in kept if k)) + cut
 
     def decide(sharing):
         chosen = []   # per range: (when it is through, slots, tiles), None for whole tiles
-        for whole, ways in ranges:
+        for whole, ways, _ in ranges:
             takes = [t + LAUNCH + (slots * PER_SLOT + (rem * GELU_PER_TILE if gelu else 0)) * sharing // 8
                      for t, slots, _, rem in ways]
             best = takes.index(min(takes)) if takes else 0
             chosen.append((takes[best],) + ways[best][1:3] if takes and takes[best] < whole else None)
         return chosen, sum(c is not None for c in chosen)
 
-    sharing = sum(bool(ways) for _, ways in ranges)
+    sharing = sum(bool(ways) for _, ways, _ in ranges)
     chosen, count = decide(sharing)
     if 0 < count < sharing:
         sharing = count
@@ -277,12 +288,11 @@ def shared_pieces(costs, wgs, gelu):
             sharing += 1
             chosen, count = decide(sharing)
     if count == 0:
-        return 0, 0
-    last = max(c[0] if c else whole + LAUNCH for c, (whole, _) in zip(chosen, ranges))
-    if last >= max(whole for whole, _ in ranges):
-        return 0, 0
-    kept = [c for c, (whole, _) in zip(chosen, ranges) if c and whole + LAUNCH > last]
-    return sum(c[1] for c in kept), sum(c[2] for c in kept)
+        return outcome(chosen)
+    last = max(c[0] if c else whole + LAUNCH for c, (whole, _, _) in zip(chosen, ranges))
+    if last >= max(whole for whole, _, _ in ranges):
+        return outcome([None] * len(ranges))
+    return outcome([c if c and whole + LAUNCH > last else None for c, (whole, _, _) in zip(chosen, ranges)])
 
 
 def test_sharing_is_priced_by_the_slots_and_the_xcds_that_there_are():
@@ -525,3 +535,68 @@ def test_a_half_empty_last_round_in_tiles_of_half_height(grid, stream_k):
         want = {(p, h, c) for p, (m, n, k) in enumerate(shapes) for h in range(0, m, 128) for c in range(0, n, 256)}
         assert set(done) == want and all((s == 1).all() for s in done.values())
     assert cut > 0
+
+
+def cut_tiles(items):
+    """Tiles that run as two items of half height (those without a row in the upper half have one item and do not count)."""
+    recs = items[items["prob"] >= 0]
+    return int((recs["m0"] % 256 == 128).sum())
+
+
+def test_halves_are_compared_with_whole_tiles_and_sharing_with_the_better():
+    """What a flagged launch does with its remainders, against the rule counted from its definition: whole tiles, halves,
+    shared tiles, and XCDs of one launch that differ."""
+    rng = np.random.default_rng(12)
+    seen = {"whole": 0, "halves": 0, "shared": 0, "both": 0}
+    for case in range(400):
+        e = int(rng.choice([1, 2, 4, 8, 16, 64]))
+        tiles = int(rng.integers(1, 2 + 1200 // e))
+        if case % 2:   # one contraction
+            k = np.full(e, 16 * int(rng.integers(8, 900)))
+        else:
+            k = rng.multinomial(int(rng.choice([4000, 12000, 40000])), rng.dirichlet(np.full(e, float(rng.choice([0.5, 1, 20])))))
+            k = (k + 15) // 16 * 16
+        gelu = case % 3 == 0
+        table, total = make_table([(256 * tiles, 256, int(v)) for v in k])
+        plan, items, fixups = _lib.plan_grouped_gemm_launch(table, (_lib.EPI_GELU if gelu else 0) | _lib.GEMM_BALANCED, 256, True)
+        costs = np.repeat([max(1, -(-int(v) // 128)) for v in k], tiles)
+        got = (plan.n_slots, len(fixups), cut_tiles(items))
+        assert got == shared_pieces(costs, 32, gelu, balanced=True), (case, e, tiles, k.tolist())
+        seen["both" if got[1] and got[2] else "shared" if got[1] else "halves" if got[2] else "whole"] += 1
+    assert min(seen.values()) > 10, seen
+
+
+def test_a_plan_depends_on_its_table_alone():
+    """Planned first thing on a new thread, again on that thread behind launches of other kinds, and here: the same bytes.
+    Eight experts, 2.25 rounds: halves for 32 steps, 4.25 rounds of 112: shared."""
+    import threading
+
+    grid = 256
+    lists = [[(1024, 4608, 4096)] * 8, [(4352, 4096, 14336)] * 4, [(256, 256, 4096)], [(1100, 4096, 4096)] * 8, [(251, 200, 3584)],
+             [(m, 4096, 14336) for m in MLP], [(4096, 768, (m + 127) // 128 * 128) for m in MLP]]
+    tables = [make_table(shapes)[0] for shapes in lists]
+
+    def planned(table, layout=_lib.GEMM_BALANCED):
+        plan, items, fixups = _lib.plan_grouped_gemm_launch(table.copy(), layout, grid, True)
+        return items.tobytes(), fixups.tobytes(), (plan.n_slots, len(fixups), cut_tiles(items))
+
+    first = []
+
+    def on_a_new_thread(table):
+        def work():
+            got = [planned(table)]
+            for other in tables:
+                for layout in (_lib.GEMM_BALANCED, 0, _lib.GEMM_BALANCED | _lib.EPI_GELU):
+                    planned(other, layout)
+                    got.append(planned(table))
+            assert all(g == got[0] for g in got)
+            first.append(got[0])
+        thread = threading.Thread(target=work)
+        thread.start()
+        thread.join()
+
+    for i, table in enumerate(tables):
+        on_a_new_thread(table)
+        assert len(first) == i + 1, "the thread's plans differ"
+        assert planned(table) == first[i]
+    assert first[0][2] == (0, 0, 64) and first[1][2] == (256, 64, 0)

@@ -1128,3 +1128,34 @@ def test_half_tiles_of_a_last_round_give_the_same_bits(dev, monkeypatch, out):
         _, items, _ = _lib.plan_grouped_gemm_launch(table, flag, _lib.gemm_grid(_lib.init(0)), False)
         cut += int((items["m0"][items["prob"] >= 0] % 256 == 128).sum())
     assert cut > 50
+
+
+@pytest.mark.parametrize("m,n,ks", [(368, 416, [208, 1280, 2512]), (416, 432, [528, 2064, 0]), (752, 368, [592, 2528])])
+def test_halves_next_to_shared_tiles_in_one_launch_are_exact(dev, monkeypatch, m, n, ks):
+    """Contractions of several lengths, contraction-major operands: the remainders of some XCDs run in tiles of half height,
+    those of others are shared along K.  Operands from {0, +-0.25 .. +-2}: every sum is exact, whoever adds what."""
+    from fp8_gmm_amd import _lib
+
+    backend = _backend()
+    plans, plan_blob = [], _lib.plan_grouped_gemm_blob
+
+    def watched(table, layout, grid, stream_k):
+        got = plan_blob(table, layout, grid, stream_k)
+        plan, blob, off_items, off_fix = got
+        items = blob[off_items: off_fix].view(_lib.GEMM_ITEM)
+        plans.append((plan.n_fixups, int((items["m0"][items["prob"] >= 0] % 256 == 128).sum())))
+        return got
+
+    monkeypatch.setattr(_lib, "plan_grouped_gemm_blob", watched)
+    g = gen(m + n)
+    vals = torch.tensor([0.0, 0.5, -0.5, 1.0, -1.0, 2.0, -2.0, 0.25])
+    a, b = ([_q(vals[torch.randint(0, 8, (k, width), generator=g)].to(torch.bfloat16), E4M3).to(dev) for k in ks]
+            for width in (m, n))
+    one = torch.ones(len(ks), device=dev)
+    c = [torch.full((m, n), 7.0, dtype=torch.bfloat16, device=dev) for _ in ks]
+    with backend.gemm_options(tile="256", stream_k=True):
+        backend.grouped_gemm(a, b, c, one, one, transposed=True)
+    assert len(plans) == 1 and min(plans[0]) > 0, plans
+    for i in range(len(ks)):
+        want = (a[i].float().t().contiguous() @ b[i].float()).to(torch.bfloat16)
+        assert torch.equal(c[i].view(torch.int16), want.view(torch.int16)), f"expert {i}"
