@@ -54,32 +54,36 @@ def test_power_of_two_operands_are_exact(dev, a_dtype, m, n, k):
     assert torch.equal(dc.cpu().view(torch.int16), c.view(torch.int16))
 
 
+def launched_plans(monkeypatch):
+    """A list that every grouped GEMM planned from here on adds itself to: (plan, shared-tile records, tiles that run as two
+    items of half height)."""
+    from fp8_gmm_amd import _lib
+
+    plans, plan_blob = [], _lib.plan_grouped_gemm_blob
+
+    def watched(*args):
+        plan, blob, off_items, off_fix = got = plan_blob(*args)
+        items = blob[off_items: off_fix].view(_lib.GEMM_ITEM)
+        cut = int((items["m0"][items["prob"] >= 0] % 256 == 128).sum()) if (plan.tile, plan.tile_m) == (256, 0) else 0
+        plans.append((plan, blob[off_fix:].view(_lib.GEMM_FIXUP), cut))
+        return got
+
+    monkeypatch.setattr(_lib, "plan_grouped_gemm_blob", watched)
+    return plans
+
+
 @pytest.mark.parametrize("a_dtype", [E4M3, E5M2])
 @pytest.mark.parametrize("sizes,n,k", [([256], 256, 4096), ([700], 520, 4112), ([300, 0, 513, 90], 512, 7168)])
 def test_tiles_shared_along_k_are_exact(dev, a_dtype, sizes, n, k, monkeypatch):
     """Few tiles and a long K: the launch cuts tiles along K, leaves fp32 partial sums in its workspace and
     completes them in the fix-up pass.  With operands from {0, +-0.25 .. +-2} every partial sum is exact, so
     the result must still equal the exactly rounded oracle result bit for bit: a piece that is dropped,
-    added twice or taken from the wrong slot cannot pass.  The plan proves that this launch really does cut
+    added twice or taken from the wrong slot cannot pass.  The plans launched prove that they really do cut
     tiles (the 256 x 256 tile is forced: left to itself the backend gives a launch this small the 128 x 128 tile,
     which is never shared)."""
-    import numpy as np
-
-    from fp8_gmm_amd import _lib
-
     backend = _backend()
     monkeypatch.setattr(backend.options, "tile", "256")
-    table = np.zeros(len(sizes), dtype=_lib.GEMM_PROBLEM)
-    for i, m in enumerate(sizes):
-        table[i]["a"], table[i]["b"], table[i]["c"] = 0x1000, 0x1000, 0x1000
-        table[i]["m"], table[i]["n"], table[i]["k"] = m, n, k
-        table[i]["lda"] = table[i]["ldb"] = k
-        table[i]["ldc"] = n
-    grid = _lib.gemm_grid(torch.cuda.get_device_properties(dev).multi_processor_count)
-    plan, items, fixups = _lib.plan_grouped_gemm_launch(table, 0, grid, True)
-    assert plan.n_fixups > 0 and (items["slot"] >= 0).sum() == plan.n_slots >= 2, \
-        "this shape was meant to exercise the shared-tile path"
-
+    plans = launched_plans(monkeypatch)
     g = gen(7 + n + k)
     vals = torch.tensor([0.0, 0.5, -0.5, 1.0, -1.0, 2.0, -2.0, 0.25])
     m_total, e = sum(sizes), len(sizes)
@@ -114,35 +118,30 @@ def test_tiles_shared_along_k_are_exact(dev, a_dtype, sizes, n, k, monkeypatch):
             if m:
                 assert torch.allclose(am[i].cpu(), gelu[row:row + m].abs().max(), rtol=1e-3)
             row += m
+    assert len(plans) == (2 if a_dtype == E4M3 else 1)
+    for plan, fixups, _ in plans:
+        assert len(fixups) > 0 and fixups["n_pieces"].sum() == plan.n_slots >= 2, \
+            "this shape was meant to exercise the shared-tile path"
 
 
 @pytest.mark.parametrize("pieces", [3, 4, 5, 7, 8])
 def test_shared_tiles_of_every_number_of_pieces_are_exact(dev, pieces, monkeypatch):
-    """One tile, cut into as many pieces as its K = 128 steps allow (four each): the fix-up launch reads the first piece
-    and the following ones three at a time, with one, two or three of them in the last turn.  Exact sums, as above; the
-    tile's last row and columns are missing."""
-    from fp8_gmm_amd import _lib
-
+    """One tile, cut into as many pieces as its K = 128 steps allow (four each, and three more steps, with which three pieces
+    are through before two tiles of half height): the fix-up launch reads the first piece and the following ones three at a
+    time, with one, two or three of them in the last turn.  Exact sums, as above; the tile's last row and columns are
+    missing."""
     backend = _backend()
     monkeypatch.setattr(backend.options, "tile", "256")
-    m, n, k = 251, 200, 512 * pieces
-    import numpy as np
-
-    table = np.zeros(1, dtype=_lib.GEMM_PROBLEM)
-    table[0]["a"] = table[0]["b"] = table[0]["c"] = 0x1000
-    table[0]["m"], table[0]["n"], table[0]["k"] = m, n, k
-    table[0]["lda"] = table[0]["ldb"] = k
-    table[0]["ldc"] = n
-    grid = _lib.gemm_grid(torch.cuda.get_device_properties(dev).multi_processor_count)
-    plan, _, fixups = _lib.plan_grouped_gemm_launch(table, 0, grid, True)
-    assert len(fixups) == 1 and fixups[0]["n_pieces"] == pieces
-
+    m, n, k = 251, 200, 512 * pieces + 384
+    plans = launched_plans(monkeypatch)
     g = gen(pieces)
     vals = torch.tensor([0.0, 0.5, -0.5, 1.0, -1.0, 2.0, -2.0, 0.25])
     a = _q(vals[torch.randint(0, 8, (m, k), generator=g)].to(torch.bfloat16), E4M3)
     b = _q(vals[torch.randint(0, 8, (1, n, k), generator=g)].to(torch.bfloat16), E4M3)
     one = torch.ones(1, device=dev)
     got = backend.fp8_gmm(a.to(dev), b.to(dev), torch.tensor([m]), one, one)
+    (_, fixups, _), = plans
+    assert len(fixups) == 1 and fixups[0]["n_pieces"] == pieces
     want = (a.float() @ b[0].float().t()).to(torch.bfloat16)
     assert torch.equal(got.cpu().view(torch.int16), want.view(torch.int16))
 
@@ -351,6 +350,7 @@ def test_shared_tiles_on_concurrent_streams(dev, monkeypatch):
         ops.append((a, b))
         wants.append((a.float() @ b[0].float().t()).to(torch.bfloat16))
     one = torch.ones(1, device=dev)
+    plans = launched_plans(monkeypatch)
     torch.cuda.synchronize()
     for rep in range(3):
         outs = []
@@ -360,6 +360,7 @@ def test_shared_tiles_on_concurrent_streams(dev, monkeypatch):
         torch.cuda.synchronize()
         for i, (c, want) in enumerate(zip(outs, wants)):
             assert torch.equal(c.view(torch.int16), want.view(torch.int16)), f"stream {i}, repetition {rep}"
+    assert len(plans) == 3 * len(streams) and all(plan.n_slots >= 2 for plan, _, _ in plans)
 
 
 def test_batched_uploads_runs_the_queued_launches_in_order(dev):
@@ -418,11 +419,12 @@ def test_batched_uploads_runs_the_queued_launches_in_order(dev):
 
 @pytest.mark.parametrize("tile", ["256", "128", "dual", "auto"])
 @pytest.mark.parametrize("b_transposed", [False, True])
-def test_two_roundings_in_the_epilogue_equal_the_separate_scaling(dev, tile, b_transposed):
+def test_two_roundings_in_the_epilogue_equal_the_separate_scaling(dev, monkeypatch, tile, b_transposed):
     """``cutlass=True`` rounds the product to bf16, multiplies by both factors and rounds again inside the GEMM: the same
     bits as an unscaled launch followed by ``multi_scale_mul``, in every tile form, on edge tiles, on pitches that only
     take element stores, on tiles shared along K, with NaN and saturated products, and for experts without rows."""
     backend = _backend()
+    plans = launched_plans(monkeypatch)
     g = gen(4711)
     for sizes, k, n in [([137, 0, 259, 60], 256, 272), ([1], 16, 16), ([513, 40], 2048, 144 if b_transposed else 150),
                         ([300, 2, 700], 4096, 1024)]:
@@ -437,6 +439,7 @@ def test_two_roundings_in_the_epilogue_equal_the_separate_scaling(dev, tile, b_t
             backend.multi_scale_mul(list(torch.split(want, sizes)), sa, sb)
             got = backend.fp8_gmm(a, b, torch.tensor(sizes), sa, sb, cutlass=True, b_transposed=b_transposed)
         assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (sizes, k, n)
+    assert tile != "256" or (any(plan.n_slots > 0 for plan, _, _ in plans) and any(cut > 0 for _, _, cut in plans))
 
 
 @pytest.mark.parametrize("out", ["bf16", "two-roundings", "gelu-e4m3", "e5m2"])
@@ -1045,9 +1048,11 @@ def test_dgelu_epilogue_is_exact_on_exact_operands(dev, out_dtype, sizes, n, k, 
     got.view(torch.uint8).fill_(0x55)
     amax = torch.zeros(e, device=dev)
     bd = b.to(dev).transpose(1, 2).contiguous() if b_kn else b.to(dev)
+    plans = launched_plans(monkeypatch)
     backend.fp8_gmm(a.to(dev), bd, torch.tensor(sizes), _scalars(sa, dev), _scalars(sb, dev), got, out_dtype, None,
                     _scalars(cs, dev), list(amax.unbind(0)), True, False, b_transposed=b_kn, dgelu_pre=pre.to(dev))
     torch.cuda.synchronize()
+    assert k != 4096 or plans[0][0].n_fixups == 1
     assert_bytes_equal(got.cpu(), want, "fused dgelu fp8 bytes")
     assert_scalar_bits_equal(amax.cpu(), torch.cat(want_amax), "fused dgelu amax")
     assert torch.cat(want_amax).max() > 0
@@ -1134,19 +1139,8 @@ def test_half_tiles_of_a_last_round_give_the_same_bits(dev, monkeypatch, out):
 def test_halves_next_to_shared_tiles_in_one_launch_are_exact(dev, monkeypatch, m, n, ks):
     """Contractions of several lengths, contraction-major operands: the remainders of some XCDs run in tiles of half height,
     those of others are shared along K.  Operands from {0, +-0.25 .. +-2}: every sum is exact, whoever adds what."""
-    from fp8_gmm_amd import _lib
-
     backend = _backend()
-    plans, plan_blob = [], _lib.plan_grouped_gemm_blob
-
-    def watched(table, layout, grid, stream_k):
-        got = plan_blob(table, layout, grid, stream_k)
-        plan, blob, off_items, off_fix = got
-        items = blob[off_items: off_fix].view(_lib.GEMM_ITEM)
-        plans.append((plan.n_fixups, int((items["m0"][items["prob"] >= 0] % 256 == 128).sum())))
-        return got
-
-    monkeypatch.setattr(_lib, "plan_grouped_gemm_blob", watched)
+    plans = launched_plans(monkeypatch)
     g = gen(m + n)
     vals = torch.tensor([0.0, 0.5, -0.5, 1.0, -1.0, 2.0, -2.0, 0.25])
     a, b = ([_q(vals[torch.randint(0, 8, (k, width), generator=g)].to(torch.bfloat16), E4M3).to(dev) for k in ks]
@@ -1155,7 +1149,8 @@ def test_halves_next_to_shared_tiles_in_one_launch_are_exact(dev, monkeypatch, m
     c = [torch.full((m, n), 7.0, dtype=torch.bfloat16, device=dev) for _ in ks]
     with backend.gemm_options(tile="256", stream_k=True):
         backend.grouped_gemm(a, b, c, one, one, transposed=True)
-    assert len(plans) == 1 and min(plans[0]) > 0, plans
+    (plan, _, cut), = plans
+    assert plan.n_fixups > 0 and cut > 0
     for i in range(len(ks)):
         want = (a[i].float().t().contiguous() @ b[i].float()).to(torch.bfloat16)
         assert torch.equal(c[i].view(torch.int16), want.view(torch.int16)), f"expert {i}"
