@@ -7,14 +7,22 @@
 // Both are bound by the rows of x and of its gradient, which pass once; the products are v_mfma_f32_16x16x32_bf16 and
 // hide behind the loads.  A row of a fragment may be any expert and a column any token or column of x, as long as
 // both operands agree, so the assignment below is the one that makes a lane's accumulators consecutive in memory.
-// Measured, microseconds, operands from HBM, against a library product (and torch's addition behind the second one):
-//   tokens, hidden, experts     grad_W              grad_x + grad_in
-//   16384, 4096, 16             33   (library 61)   65   (109)       134 MB read; 134 MB read, 134 MB written
-//   16384, 4096, 40             49   (107)          74   (112)
-//   16384, 4096, 128            82   (141)          80   (104)
-//   16384, 4096, 100 and 65     84, 89 (111, 121)   127, 144 (117)   both together less than the library's as well
-//   4096, 1024, 64              16   (28)           8    (23)
-//   1531, 1024, 16              7    (19)           4.4  (23)        the library's figures are its host path
+// Measured, microseconds, operands from HBM, against the library's products and torch's addition behind the one of x
+// (some 22 of which per product are its host path, where it is the longer one):
+//   tokens, hidden, experts   grad_x + grad_in        with grad_W as well
+//   16384, 4096, 16           65    (library 108)     99    (185)        134 MB read, 134 MB written; 134 MB more read
+//   16384, 4096, 64           78    (95)              130   (227)
+//   16384, 4096, 72, 104      79    (111, 116)        165   (242, 249)
+//   16384, 4096, 66, 100      119, 131 (112, 116)     201, 211 (243, 249)
+//   16384, 4096, 65, 127      143, 152 (115, 125)     228, 238 (254, 270)
+//   4096, 4096, 64, 72, 100   24, 30, 40 (32, 37, 37) 44, 65, 76 (61, 65, 66)
+//   8192, 4096, 65, 100       81, 70 (65, 65)         134, 120 (137, 135)
+//   4096, 2048, 65, 100       30, 24 (28, 29)         57, 52 (64, 59)
+//   4096, 8192, 64, 72, 100   39, 45, 67 (55, 63, 65) 68, 96, 117 (84, 92, 95)
+//   1024, 16384, 63, 104      33, 28 (36, 36)         52, 64 (53, 52)
+//   16384, 1024, 63, 65       33, 50 (38, 39)         54, 86 (181, 172)
+//   1531, 1024, 16, 65        5, 12 (22)              11, 25 (42)
+//   64, 4096, 16, 127         4, 7 (22)               7, 16 (42)
 #include <algorithm>
 
 #include "device_utils.h"

@@ -168,15 +168,26 @@ def _plain_linear(module):
                      or module._backward_pre_hooks) and not torch.nn.modules.module._has_any_global_hook())
 
 
+def _gating_is_faster(tokens, hidden, experts, trained):
+    """Whether fp8gmm_gating_backward is ahead of the library's products and torch's addition (csrc/gating.hip has both sides).
+    Up to 64 experts it is.  Beyond, a row of gradients whose bytes are no multiple of 16 is loaded in pieces of 2 or 4, which
+    the input gradient alone does not make up for; the weight gradient's time goes with the columns too, the library's with
+    the tokens only.  Short batches wait for the library's launches."""
+    if experts <= 64 or tokens * hidden <= 1 << 21:
+        return True
+    whole = experts % 8 == 0
+    return hidden <= (4096 if whole or tokens >= 8192 else 2048) if trained else whole
+
+
 def _gating_takes(x, weight):
-    """What fp8gmm_gating_backward computes; the general path is torch's linear and its gradients.  Inside these limits the
-    kernels are the faster ones throughout (csrc/gating.hip has both sides from 16 tokens and 1 expert to 16384 and 128);
-    the forward product stays torch's, whose bits decide the routing."""
+    """What fp8gmm_gating_backward computes, where it is faster; the general path is torch's linear and its gradients.  The
+    forward product stays torch's, whose bits decide the routing."""
     tokens, hidden = x.shape
     return (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.is_cuda and weight.device == x.device
             and type(x) in (torch.Tensor, torch.nn.Parameter) and weight.dim() == 2 and weight.shape[1] == hidden
             and 1 <= weight.shape[0] <= MAX_GATING_EXPERTS and 1 <= tokens <= 1 << 20 and 8 <= hidden <= 1 << 16
-            and hidden % 8 == 0 and x.is_contiguous() and weight.is_contiguous() and x.data_ptr() % 16 == 0)
+            and hidden % 8 == 0 and x.is_contiguous() and weight.is_contiguous() and x.data_ptr() % 16 == 0
+            and _gating_is_faster(tokens, hidden, weight.shape[0], weight.requires_grad))
 
 
 def gating(module, x):

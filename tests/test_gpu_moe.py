@@ -387,3 +387,18 @@ def test_gating_calls_a_module_that_is_more_than_a_product(dev):
     second, = torch.autograd.grad(first.float().sum(), xd)
     want = 2 * (plain.weight.float().t() @ plain.weight.float()).sum(0)     # the Hessian of |W x|^2 times ones
     assert torch.allclose(second.float(), want.expand_as(second), rtol=2e-2, atol=2e-2 * want.abs().max().item())
+
+
+@pytest.mark.parametrize("tokens,hidden,experts,trained,kernels", [
+    (1 << 16, 64, 64, False, True), (1 << 15, 72, 63, True, True),                        # up to 64 experts
+    (1 << 15, 64, 65, False, True), ((1 << 15) + 1, 64, 65, False, False),                # up to 2^21 values of x
+    ((1 << 15) + 1, 64, 72, False, True), ((1 << 15) + 1, 64, 65, True, True),            # whole 16 bytes of gradients a token
+    (1025, 2048, 100, True, True), (1025, 2056, 100, True, False), (1025, 2056, 104, True, True),
+    (1025, 4104, 104, True, False), (8191, 4096, 127, True, False), (8192, 4096, 127, True, True),
+    (8192, 4104, 127, True, False), (8192, 4104, 128, False, True)])
+def test_gating_runs_on_the_kernels_where_they_are_faster(dev, tokens, hidden, experts, trained, kernels):
+    """Many experts: the general path where the library's products are ahead (both sides in csrc/gating.hip)."""
+    linear = torch.nn.Linear(hidden, experts, bias=False, dtype=torch.bfloat16, device=dev).requires_grad_(trained)
+    x = torch.zeros(tokens, hidden, dtype=torch.bfloat16, device=dev, requires_grad=True)
+    logits, again = _ops().gating(linear, x)
+    assert ("Gating" in logits.grad_fn.name()) == kernels == (again is not x)
