@@ -124,7 +124,9 @@ class _Gating(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight):
         ctx.set_materialize_grads(False)
-        ctx.save_for_backward(x, weight)
+        # what torch's linear would keep: with a frozen weight the caller may change the rows in place afterwards
+        ctx.save_for_backward(x if ctx.needs_input_grad[1] else None, weight if ctx.needs_input_grad[0] else None)
+        ctx.hidden = x.shape[1]
         return torch.nn.functional.linear(x, weight), x
 
     @staticmethod
@@ -140,18 +142,20 @@ class _Gating(torch.autograd.Function):
             if want_weight:
                 grad_weight = grad.t() @ x
             return grad_x, grad_weight
-        (tokens, experts), hidden, dev = grad.shape, x.shape[1], x.device
-        grad, x = _aligned(grad), _aligned(x)
-        weight = weight.contiguous()
+        (tokens, experts), hidden, dev = grad.shape, ctx.hidden, grad.device
+        grad = _aligned(grad)
+        x = _aligned(x) if want_weight else None
+        weight = weight.contiguous() if want_x else None
         grad_in = _aligned(grad_in) if grad_in is not None else None
         L = _lib.load()
-        grad_x = torch.empty_like(x) if want_x else None
+        grad_x = torch.empty(tokens, hidden, dtype=grad.dtype, device=dev) if want_x else None
         grad_weight = work = None
         if want_weight:
-            grad_weight = torch.empty(experts, hidden, dtype=x.dtype, device=dev)
+            grad_weight = torch.empty(experts, hidden, dtype=grad.dtype, device=dev)
             work = torch.empty(L.fp8gmm_gating_workspace_bytes(tokens, hidden, experts), dtype=torch.uint8, device=dev)
         with torch.cuda.device(dev), _timed("gating_backward", lambda: 2 * tokens * hidden * (want_weight + 2 * want_x)):
-            rc = L.fp8gmm_gating_backward(grad.data_ptr(), x.data_ptr(), weight.data_ptr(),
+            rc = L.fp8gmm_gating_backward(grad.data_ptr(), x.data_ptr() if want_weight else None,
+                                          weight.data_ptr() if want_x else None,
                                           grad_in.data_ptr() if grad_in is not None else None,
                                           grad_x.data_ptr() if want_x else None,
                                           grad_weight.data_ptr() if want_weight else None, tokens, hidden, experts,

@@ -402,3 +402,23 @@ def test_gating_runs_on_the_kernels_where_they_are_faster(dev, tokens, hidden, e
     x = torch.zeros(tokens, hidden, dtype=torch.bfloat16, device=dev, requires_grad=True)
     logits, again = _ops().gating(linear, x)
     assert ("Gating" in logits.grad_fn.name()) == kernels == (again is not x)
+
+
+@pytest.mark.parametrize("layer", ["linear", "mlp"])
+def test_rows_may_be_changed_in_place_behind_a_layer_whose_gate_is_frozen(dev, layer):
+    """``x += layer(x)``: with a frozen gating weight nothing of the pass needs the rows as they were."""
+    from fp8_gmm_amd.moe import Fp8LinearModule, Fp8MlpModule
+
+    torch.manual_seed(5)
+    module = (Fp8MlpModule if layer == "mlp" else Fp8LinearModule)(64, 96, 4, 2, device=dev)
+    module.gating_network.requires_grad_(False)
+    rows = torch.randn(70, 64, device=dev).to(torch.bfloat16)
+    grads = []
+    for in_place in (False, True):
+        leaf = rows.clone().requires_grad_()
+        x = leaf * 1
+        out = module(x)
+        y = x.add_(out) if in_place else x + out
+        y.backward(torch.ones_like(y))
+        grads.append(leaf.grad)
+    assert torch.isfinite(grads[0].float()).all() and torch.equal(grads[0], grads[1])
