@@ -409,12 +409,12 @@ def test_rows_may_be_changed_in_place_behind_a_layer_whose_gate_is_frozen(dev, l
     """``x += layer(x)``: with a frozen gating weight nothing of the pass needs the rows as they were."""
     from fp8_gmm_amd.moe import Fp8LinearModule, Fp8MlpModule
 
-    torch.manual_seed(5)
-    module = (Fp8MlpModule if layer == "mlp" else Fp8LinearModule)(64, 96, 4, 2, device=dev)
-    module.gating_network.requires_grad_(False)
-    rows = torch.randn(70, 64, device=dev).to(torch.bfloat16)
+    rows = torch.randn(70, 64, generator=torch.Generator().manual_seed(4)).to(torch.bfloat16).to(dev)
     grads = []
     for in_place in (False, True):
+        torch.manual_seed(5)   # a module each: a pass changes its scaling state
+        module = (Fp8MlpModule if layer == "mlp" else Fp8LinearModule)(64, 96, 4, 2, device=dev)
+        module.gating_network.requires_grad_(False)
         leaf = rows.clone().requires_grad_()
         x = leaf * 1
         out = module(x)
