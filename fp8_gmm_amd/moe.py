@@ -52,15 +52,17 @@ class _RoutedModule(torch.nn.Module):
 
     def forward(self, input):
         input = input.view(-1, input.size(-1))
-        routing_logits, input = moe_ops.gating(self.gating_network, input)
+        # Another compute, of a subclass or set on the module, is called as ever: on the rows themselves, which it may change in
+        # place where nothing else needs them, and without the inverse.
+        own = getattr(self.compute, "__func__", None) is _RoutedModule.compute
+        routing_logits, input = moe_ops.gating(self.gating_network, input) if own else (self.gating_network(input), input)
         weights0, selected_experts = moe_ops.topk(routing_logits, self.top_k)
         expert_weights = weights0.flatten()
         top_experts = selected_experts.flatten()
         with torch.no_grad():
             indices, bin_ids, bins, tokens_per_expert, inverse = moe_ops.indices_bins_and_inverse(
                 top_experts, self.n_experts)
-        # another compute, of a subclass or set on the module, is called as ever, without the inverse
-        more = (inverse,) if getattr(self.compute, "__func__", None) is _RoutedModule.compute else ()
+        more = (inverse,) if own else ()
         return self.compute(input, tokens_per_expert, indices, bin_ids, expert_weights, bins, self.top_k, *more)
 
 

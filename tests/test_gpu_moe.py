@@ -422,3 +422,27 @@ def test_rows_may_be_changed_in_place_behind_a_layer_whose_gate_is_frozen(dev, l
         y.backward(torch.ones_like(y))
         grads.append(leaf.grad)
     assert torch.isfinite(grads[0].float()).all() and torch.equal(grads[0], grads[1])
+
+
+def test_a_compute_of_ones_own_may_change_the_rows_in_place(dev):
+    """With a frozen gate nothing else needs the rows as they were, and a subclass gets the rows themselves."""
+    from fp8_gmm_amd.moe import Fp8MlpModule
+
+    class Doubled(Fp8MlpModule):
+        in_place = False
+
+        def compute(self, x, *rest):
+            return super().compute(x.mul_(2) if self.in_place else x * 2, *rest)
+
+    rows = torch.randn(70, 64, generator=torch.Generator().manual_seed(4)).to(torch.bfloat16).to(dev)
+    results = []
+    for in_place in (False, True):
+        torch.manual_seed(5)
+        module = Doubled(64, 96, 4, 2, device=dev)
+        module.in_place = in_place
+        module.gating_network.requires_grad_(False)
+        leaf = rows.clone().requires_grad_()
+        y = module(leaf * 1)
+        y.backward(torch.ones_like(y))
+        results.append((y, leaf.grad))
+    assert all(torch.equal(a, b) for a, b in zip(*results))
