@@ -135,14 +135,19 @@ class _Gating(torch.autograd.Function):
             return grad_in, None
         x, weight = ctx.saved_tensors
         want_x, want_weight = ctx.needs_input_grad
-        if torch.is_grad_enabled():   # a graph of the backward pass is asked for
+        (tokens, experts), hidden, dev = grad.shape, ctx.hidden, grad.device
+
+        def as_saved(t, rows):
+            return t.dtype == torch.bfloat16 and t.device == dev and t.shape == (rows, hidden)
+
+        # a graph of the backward pass is asked for, or a saved-tensor hook returned what the kernels do not read: torch's products
+        if torch.is_grad_enabled() or want_weight and not as_saved(x, tokens) or want_x and not as_saved(weight, experts):
             grad_x = grad_weight = None
             if want_x:
                 grad_x = grad @ weight if grad_in is None else grad_in + grad @ weight
             if want_weight:
                 grad_weight = grad.t() @ x
             return grad_x, grad_weight
-        (tokens, experts), hidden, dev = grad.shape, ctx.hidden, grad.device
         grad = _aligned(grad)
         x = _aligned(x) if want_weight else None
         weight = weight.contiguous() if want_x else None

@@ -446,3 +446,30 @@ def test_a_compute_of_ones_own_may_change_the_rows_in_place(dev):
         y.backward(torch.ones_like(y))
         results.append((y, leaf.grad))
     assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+def test_gating_gradients_check_what_saved_tensor_hooks_return(dev):
+    """Such a hook may hand the backward pass another type, device or shape: what torch's linear makes of it, an error, and no
+    kernel on memory that is not what it reads.  (Gradient hooks that change these are refused by autograd.)"""
+    ops = _ops()
+    gen = torch.Generator().manual_seed(9)
+    x, w, g = (torch.randint(-3, 4, shape, generator=gen).to(torch.bfloat16).to(dev) for shape in [(40, 64), (6, 64), (40, 6)])
+    linear = torch.nn.Linear(64, 6, bias=False, dtype=torch.bfloat16, device=dev)
+    linear.weight.data.copy_(w)
+
+    def passes(kernels, unpack):
+        linear.zero_grad()
+        xd = x.clone().requires_grad_()
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+            logits = ops.gating(linear, xd)[0] if kernels else linear(xd)
+        assert ("Gating" in logits.grad_fn.name()) == kernels
+        logits.backward(g)
+        return xd.grad, linear.weight.grad
+
+    want = passes(False, lambda t: t)
+    for same in (lambda t: t, lambda t: t.cpu().to(dev), lambda t: t.t().contiguous().t()):
+        assert all(torch.equal(a, b) for a, b in zip(passes(True, same), want))
+    for other in (lambda t: t.float(), lambda t: t.cpu(), lambda t: t[:, :32], lambda t: t[:3]):
+        for kernels in (False, True):
+            with pytest.raises(RuntimeError):
+                passes(kernels, other)
