@@ -25,7 +25,7 @@ GEMM_A_KMAJOR = 4
 GEMM_TILE_128 = 0x100   # planning flag: 128 x 128 tiles, two workgroups per compute unit
 GEMM_TILE_DUAL = 0x200  # planning flag: 128 x 256 tiles for the kernel form with two sets of accumulators
 GEMM_TILE_ROWS = 0x400
-GEMM_BALANCED = 0x800   # planning flag: 256 x 256 tiles, ranges by what tiles take an XCD, half-empty last rounds in half tiles
+GEMM_BALANCED = 0x800   # planning flag: 256 x 256 tiles, a half-empty last round runs in tiles of half height
 GEMM_ROWS_TILE_M = 64
 
 OP_QUANTIZE = 0

@@ -43,11 +43,6 @@ constexpr int kSkPerSlot = 100;
 constexpr int kSkGeluPerTile = 150;
 constexpr int kPartialBytes = BM * BN * 4;  // one slot: the fp32 accumulators of one tile
 constexpr int kTileOverhead = 4;      // fixed cost of a tile (epilogue, switch) in K = 128 steps, measured
-// What a tile weighs besides its steps where the XCDs' ranges are cut (FP8GMM_GEMM_BALANCED; without it kTileOverhead).  Less
-// than what it costs its workgroup: a range of short contractions stores while another one reads.  17 weight gradients of
-// skewed splits inside a layer's step, 4 -> 3 / 2 / 1: 1.002, 0.988, 1.002 of the time (6 of 8960 x 832, 15230 rows 138 -> 127
-// us; the most that one loses is 2 %); 43 alone with operands from HBM: 0.994, 0.981, 0.985.
-constexpr int kTileWeight = 2;
 constexpr int kSlotsPerWg = 2;        // a piece that starts inside a tile, one that ends inside a tile
 
 struct Sched {
@@ -60,7 +55,6 @@ struct Sched {
   int sk_wgs;                  // workgroups that take a piece of the region
   int64_t sk_c0, sk_cost;      // cost before the region, cost of the region (K = 128 steps)
   int64_t total_cost;          // cost of all tiles
-  int tile_weight;             // of a tile besides its steps, where the ranges are cut
   bool halves;                 // the remainder [sk_begin, range_end) in tiles of half height, two per tile (sk_wgs is 0)
   bool gelu;                   // completing a shared tile includes the GELU epilogue
 };
@@ -84,7 +78,7 @@ FP8GMM_HD int64_t tile_cost(const Sched& s, int p) {
 }
 // Work before `tile` (0 <= tile <= total_tiles) when every tile counts its K steps plus `ov` steps of fixed
 // overhead; cost_begin is the plan's prefix sum of the K steps alone.  ov = 0 is the unit in which tiles are
-// cut along K; ov = tile_weight is the weight that balances the XCD ranges.
+// cut along K; ov = kTileOverhead is the weight that balances the XCD ranges.
 FP8GMM_HD int64_t work_before(const Sched& s, int tile, int ov) {
   const int p = problem_of_tile(s, tile);
   return (int64_t)s.probs[p].cost_begin + (int64_t)ov * s.probs[p].tile_begin +
@@ -113,8 +107,8 @@ FP8GMM_HD int first_tile_at_work(const Sched& s, int64_t c, int ov) {
 
 // first tile of XCD x's range (x = 8: the end of the last one)
 FP8GMM_HD int range_start(const Sched& s, int x) {
-  const int64_t total_work = s.total_cost + (int64_t)s.tile_weight * s.total_tiles;
-  return first_tile_at_work(s, (total_work * x + kNumXcd - 1) / kNumXcd, s.tile_weight);
+  const int64_t total_work = s.total_cost + (int64_t)kTileOverhead * s.total_tiles;
+  return first_tile_at_work(s, (total_work * x + kNumXcd - 1) / kNumXcd, kTileOverhead);
 }
 // Striding takes a range of n tiles full + 1 rounds, sharing the remainder full + rem / W: worth a thought when that saves
 // a twelfth of the launch by this count.  Measured, sharing returns about half of what the count promises (workgroups do
@@ -139,15 +133,28 @@ FP8GMM_HD int dp_tile(const Sched& s, int j, int i) {
 // ---- a last round of tiles of half height ----
 // A remainder of at most half a round leaves half of the workgroups without a tile while the others run a whole one.  Cut
 // into two items of half height (FP8GMM_ITEM_HALF_HEIGHT) it takes them kHalfStep / 100 of a step's time per K step and
-// kHalfTile / 100 steps for the result and the switch; no partial sums, no second launch.  Timed inside the kernel, 8 experts,
-// K = N = 4096, 8192 rows (2.25 rounds): whole tiles 43, 40 and, eight of them on 32 workgroups, 29 us; those as halves 20.
-// Halves between whole tiles take 0.62 of their time, but a last round of halves is a quarter of the traffic and a half of
-// the workgroups of a round, and its whole tiles would have run at 0.7: 75 is what separates the launches that gain from
-// those that are better off shared along K (K = 14336, 4.25 rounds: shared 710, halves 743).
-constexpr int kHalfStep = 75;
+// kHalfTile / 100 steps for the result and the switch; no partial sums, no second launch.  Measured on launches of one
+// contraction that the tile rules leave to this tile, halves against whole tiles: less than a round, 0.65 - 0.8 of the time
+// with up to 4 tiles on 32 workgroups, 0.75 - 0.95 with up to 16; a round and a bit 0.88 - 0.95, two 0.95, more 0.97 - 1.
+// A range that may share is asked first, against whole tiles: what it then shares took 0.92 of the time that it took in halves
+// (K = 14336, 4.25 rounds: 735 us against 761, whole tiles 771; remainders that are most of the launch 0.6 - 0.9), and halves
+// are for what sharing does not pay for (K = 4096, 2.25 rounds: 136 us, whole tiles and shared 144).
+// With the GELU an item stores three bytes per value: beyond kHalfGeluTiles / 16 of a round, halves of short contractions lose
+// (12 tiles of 4 - 12 steps 1.03 - 1.15, 16 of 3 steps 1.23 of the time of whole ones), and from kHalfGeluSteps on they gain
+// 2 - 12 %.  With the GELU's derivative, which reads the pre-activation, they take 0.55 - 0.98, with one launch of 15 losing.
+// Against the plans without halves: 150 launches, three quarters of them with the GELU, 0.933 of the time in the mean, the worst
+// 1.03; 120 with the derivative 0.77 (1.05); 150 weight gradients of skewed splits 0.989 (1.025).
+constexpr int kHalfStep = 95;
 constexpr int kHalfTile = 300;
 constexpr int kHalfMaxRounds = 12;    // with more full rounds than this a last round is not worth the look
+constexpr int kHalfGeluTiles = 5;
+constexpr int kHalfGeluSteps = 32;
 inline int64_t half_tile_x100(int64_t steps) { return steps * kHalfStep + kHalfTile; }
+FP8GMM_HD bool remainder_may_halve(int n_tiles, int W, int64_t steps, int epilogue) {
+  const int rem = n_tiles % W;
+  return rem != 0 && 2 * rem <= W && n_tiles / W <= kHalfMaxRounds &&
+         (!(epilogue & FP8GMM_EPI_GELU) || 16 * rem <= kHalfGeluTiles * W || steps >= kHalfGeluSteps);
+}
 // Workgroup j's item of the round behind `full` whole ones: which tile of the remainder, and which half of it.
 FP8GMM_HD int half_position(int wgs, int j, int full) { return (j + kRoundRotation * full) % wgs; }
 
@@ -162,9 +169,9 @@ struct SkRemainder {
   int64_t c0, cost;      // cost before it, its own
   int n_splits;          // 0: not worth a thought
   SkSplit split[kSkMaxPieces];
-  // of `sk_times`, which wants the splits; where halves are through first, whole_x100 is their time from then on
-  int64_t whole_x100, shared_x100[kSkMaxPieces], half_x100;
-  bool timed, halves;
+  int64_t whole_x100, shared_x100[kSkMaxPieces], half_x100;   // of `sk_times`, which wants the splits
+  bool timed;
+  bool halves;           // if it is not shared, it runs in tiles of half height
 };
 
 // A tile that k piece ends fall inside of is left in k + 1 slots; one that no end falls inside of needs none.
@@ -329,7 +336,8 @@ inline void sk_decide(const Sched (&all)[kNumXcd], SkRemainder (&rem)[kNumXcd], 
   for (int x = 0; x < kNumXcd; ++x) {
     if (all[x].range_begin == all[x].range_end) continue;
     if (rem[x].n_splits == 0) sk_times(all[x], rem[x]);
-    const int64_t own = pieces[x] > 0 ? through[x] : rem[x].whole_x100 + kSkFixupLaunch * 100;
+    const int64_t alone = rem[x].halves ? rem[x].half_x100 : rem[x].whole_x100;
+    const int64_t own = pieces[x] > 0 ? through[x] : alone + kSkFixupLaunch * 100;
     whole = whole < rem[x].whole_x100 ? rem[x].whole_x100 : whole;
     last = last < own ? own : last;
   }
@@ -343,14 +351,13 @@ inline void sk_decide(const Sched (&all)[kNumXcd], SkRemainder (&rem)[kNumXcd], 
 // tile costs its K steps plus a fixed part (epilogue, tile switch): balancing
 // K steps alone left the XCDs that hold the short-K problems 17 % more work than the others.
 inline void sched_init(Sched (&all)[kNumXcd], const fp8gmm_gemm_problem* probs, int nprob, int total_tiles, int wgs_per_xcd,
-                       bool sk_enable, bool gelu = false, bool balanced = false) {
+                       bool sk_enable, int epilogue = 0, bool balanced = false) {
   const int W = wgs_per_xcd;
   SkRemainder rem[kNumXcd] = {};
   for (int x = 0; x < kNumXcd; ++x) {
     Sched& s = all[x];
-    s.gelu = gelu;
+    s.gelu = (epilogue & (FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU)) != 0;
     s.halves = false;
-    s.tile_weight = balanced ? kTileWeight : kTileOverhead;
     s.probs = probs;
     s.nprob = nprob;
     s.total_tiles = total_tiles;
@@ -373,12 +380,9 @@ inline void sched_init(Sched (&all)[kNumXcd], const fp8gmm_gemm_problem* probs, 
       r.cost = cost_before(s, s.range_end) - r.c0;
       sk_splits(s, r);
     }
-    if (balanced && r.tiles > 0 && 2 * r.tiles <= W && n_x / W <= kHalfMaxRounds) {
+    if (balanced && r.tiles > 0 && remainder_may_halve(n_x, W, tile_cost(s, problem_of_tile(s, r.begin)), epilogue)) {
       sk_times(s, r);
-      if (r.half_x100 < r.whole_x100) {
-        r.halves = true;
-        r.whole_x100 = r.half_x100;
-      }
+      r.halves = r.half_x100 < r.whole_x100;
     }
   }
   int pieces[kNumXcd] = {};

@@ -302,9 +302,8 @@ static int plan_whole_tiles(const int TM, const int TN, const int weight, fp8gmm
   return FP8GMM_OK;
 }
 
-// Tail balancing can only pay when the launch has few rounds; it needs the whole grid even for few tiles.  Without it
-// the grid shrinks to the tiles there are.
-// So does a last round of half tiles.
+// Sharing tiles can only pay when the launch has few rounds; it needs the whole grid even for few tiles, and so does a last
+// round of half tiles.  Otherwise the grid shrinks to the tiles there are.
 static bool share_tail(int stream_k, int total_tiles, bool balanced, int* grid) {
   using namespace fp8gmm;
   if (stream_k != 0 && (int64_t)total_tiles <= (int64_t)kSkMaxRounds * *grid && *grid > kNumXcd) return true;
@@ -328,8 +327,8 @@ int fp8gmm_plan_grouped_gemm_launch(fp8gmm_gemm_problem* probs, int n, int layou
   }
   plan->tile = kGemmTileM;
   const int layout_given = layout, grid_given = grid;
-  // the epilogue flags only weigh the decision to share tiles along K (completing a tile costs more with them)
-  const bool gelu = (layout & (FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU)) != 0;
+  // the epilogue flags only weigh the decisions on the last round (completing a shared tile costs more with them)
+  const int epilogue = layout & (FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU);
   const bool balanced = (layout & FP8GMM_GEMM_BALANCED) != 0;
   layout &= ~(FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU | FP8GMM_GEMM_BALANCED);
   int total_tiles = 0;
@@ -344,7 +343,7 @@ int fp8gmm_plan_grouped_gemm_launch(fp8gmm_gemm_problem* probs, int n, int layou
   // pass 1: sizes.  The tiles that were shared along K first: the pieces of such a tile get consecutive
   // workspace slots, numbered from 0 over the launch, in K order.
   Sched sched[kNumXcd];
-  sched_init(sched, probs, n, total_tiles, wgs, sk, gelu, balanced);
+  sched_init(sched, probs, n, total_tiles, wgs, sk, epilogue, balanced);
   std::vector<int32_t> slot_map((size_t)kSlotsPerWg * grid, -1);
   std::vector<fp8gmm_gemm_fixup_desc> fix;
   int n_slots = 0;
@@ -531,7 +530,7 @@ int plan_gemm_ranges(fp8gmm_gemm_problem* probs, int n, int layout, int grid, in
       out->xcd[x].end = cuts.cut[x + 1];
     }
   } else {
-    const bool gelu = (layout & (FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU)) != 0;
+    const int epilogue = layout & (FP8GMM_EPI_GELU | FP8GMM_EPI_DGELU);
     plan->tile = kGemmTileM;
     int total_tiles = 0;
     const bool balanced = (layout & FP8GMM_GEMM_BALANCED) != 0;
@@ -544,7 +543,7 @@ int plan_gemm_ranges(fp8gmm_gemm_problem* probs, int n, int layout, int grid, in
     const int wgs = grid / kNumXcd;
     plan->grid = grid;
     Sched sched[kNumXcd];
-    sched_init(sched, probs, n, total_tiles, wgs, sk, gelu, balanced);
+    sched_init(sched, probs, n, total_tiles, wgs, sk, epilogue, balanced);
     for (int x = 0; x < kNumXcd; ++x) {
       const Sched& s = sched[x];
       GemmRanges::Xcd& o = out->xcd[x];

@@ -188,10 +188,10 @@ typedef struct fp8gmm_gemm_problem {
  * FP8GMM_EPI_DGELU excepted; never shares tiles along K (stream_k is ignored).  No counterpart in the reference. */
 #define FP8GMM_GEMM_TILE_ROWS 0x400
 
-/* Planning flag (`layout` of fp8gmm_plan_grouped_gemm_launch only, 256 x 256 tiles): the XCDs' ranges are cut by what tiles of
- * several contractions take them, and where the last round of a range would occupy at most half of its workgroups, each of its
- * tiles may become two items of half height (FP8GMM_ITEM_HALF_HEIGHT: rows m0 .. m0 + 127 each) on two workgroups.  Same
- * products in the same order: whole tiles get the same bits.  No counterpart in the reference. */
+/* Planning flag (`layout` of fp8gmm_plan_grouped_gemm_launch only, 256 x 256 tiles): where the last round of an XCD's range would
+ * occupy at most half of its workgroups and is not shared along K, each of its tiles may become two items of half height
+ * (FP8GMM_ITEM_HALF_HEIGHT: rows m0 .. m0 + 127 each) on two workgroups.  Same products in the same order: the same bits.  No
+ * counterpart in the reference. */
 #define FP8GMM_GEMM_BALANCED 0x800
 #define FP8GMM_GEMM_ROWS_TILE_M 64
 #define FP8GMM_GEMM_ROWS_TILE_N 128

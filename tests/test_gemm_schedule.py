@@ -228,17 +228,17 @@ def test_pieces_end_where_tiles_end_unless_whole_tiles_are_faster():
 
 # The rule for sharing, with everything counted from its definition: K = 128 steps of time, in hundredths.
 LAUNCH, PER_SLOT, GELU_PER_TILE = 400, 100, 150
-HALF_STEP, HALF_TILE, HALF_ROUNDS = 75, 300, 12   # of FP8GMM_GEMM_BALANCED, which also cuts the ranges at 2 steps a tile
+HALF_STEP, HALF_TILE, HALF_ROUNDS, HALF_GELU = 95, 300, 12, (5, 32)   # of FP8GMM_GEMM_BALANCED
 
 
 def shared_pieces(costs, wgs, gelu, balanced=False):
     """costs: K steps of the tiles, in order.  Slots and shared tiles of a launch, if an XCD takes the number of pieces with
     which its last workgroup is through first, at the price of the XCDs that share, and the launch shares where its last XCD
-    is through sooner for it.  `balanced`: against a remainder that is cut into tiles of half height where that is faster than
-    whole ones; with the number of tiles that are cut so behind the two."""
+    is through sooner for it.  `balanced`: a remainder that is not shared is cut into tiles of half height where that is
+    faster than whole ones; with the number of tiles that are cut so behind the two."""
     n = len(costs)
     before = np.concatenate([[0], np.cumsum(costs)])
-    work = before + (2 if balanced else 4) * np.arange(n + 1)
+    work = before + 4 * np.arange(n + 1)
     cut = [int(np.searchsorted(work, -(-int(work[-1]) * x // 8))) for x in range(9)]
     ranges = []   # per XCD: (time with whole tiles, [(time but for the slots, slots, tiles cut, tiles)])
     for x in range(8):
@@ -250,12 +250,13 @@ def shared_pieces(costs, wgs, gelu, balanced=False):
         for i in range(full):   # workgroup j's place in round i is j + 5 i
             load += own[i * wgs + (np.arange(wgs) + 5 * i) % wgs] + 4
         last = [int(load[j] + own[full * wgs + p]) + 4 for j in range(wgs) for p in [(j + 5 * full) % wgs] if p < rem]
-        whole, ways, halved = max([int(load.max())] + last) * 100, [], 0
-        if balanced and 0 < 2 * rem <= wgs and full <= HALF_ROUNDS:   # workgroup j's place names a tile and one of its halves
-            through = [int(load[j]) * 100 + HALF_STEP * int(own[full * wgs + p // 2]) + HALF_TILE
-                       for j in range(wgs) for p in [(j + 5 * full) % wgs] if p // 2 < rem]
-            if max([int(load.max()) * 100] + through) < whole:
-                whole, halved = max([int(load.max()) * 100] + through), rem
+        whole, ways, alone, halved = max([int(load.max())] + last) * 100, [], None, 0
+        if balanced and 0 < 2 * rem <= wgs and full <= HALF_ROUNDS \
+                and (not gelu or 16 * rem <= HALF_GELU[0] * wgs or own[full * wgs] >= HALF_GELU[1]):
+            # workgroup j's place names a tile and one of its halves
+            alone = max([int(load.max()) * 100] + [int(load[j]) * 100 + HALF_STEP * int(own[full * wgs + p // 2]) + HALF_TILE
+                                                   for j in range(wgs) for p in [(j + 5 * full) % wgs] if p // 2 < rem])
+            halved = rem if alone < whole else 0
         ends = np.concatenate([[0], np.cumsum(own[full * wgs:])])
         cost, most = int(ends[-1]), min(wgs, int(ends[-1]) // 4, 8 * rem)
         if rem and full <= 24 and (wgs - rem) * 12 >= wgs * (full + 1):
@@ -264,22 +265,22 @@ def shared_pieces(costs, wgs, gelu, balanced=False):
                           if ends[t] != cost * j // pieces]
                 through = max(int(load.max()) * 100, (int(load[:pieces].max()) + 4) * 100 + cost * 100 // pieces)
                 ways.append((through, len(inside) + len(set(inside)), len(set(inside)), rem))
-        ranges.append((whole, ways, halved))
+        ranges.append((whole, ways, alone if halved else whole, halved))
 
     def outcome(kept):   # per range: what it shares, None for nothing
-        cut = (sum(halved for k, (_, _, halved) in zip(kept, ranges) if not k),) if balanced else ()
+        cut = (sum(halved for k, (*_, halved) in zip(kept, ranges) if not k),) if balanced else ()
         return (sum(k[1] for k in kept if k), sum(k[2] for k in kept if k)) + cut
 
     def decide(sharing):
         chosen = []   # per range: (when it is through, slots, tiles), None for whole tiles
-        for whole, ways, _ in ranges:
+        for whole, ways, *_ in ranges:
             takes = [t + LAUNCH + (slots * PER_SLOT + (rem * GELU_PER_TILE if gelu else 0)) * sharing // 8
                      for t, slots, _, rem in ways]
             best = takes.index(min(takes)) if takes else 0
             chosen.append((takes[best],) + ways[best][1:3] if takes and takes[best] < whole else None)
         return chosen, sum(c is not None for c in chosen)
 
-    sharing = sum(bool(ways) for _, ways, _ in ranges)
+    sharing = sum(bool(ways) for _, ways, *_ in ranges)
     chosen, count = decide(sharing)
     if 0 < count < sharing:
         sharing = count
@@ -289,10 +290,10 @@ def shared_pieces(costs, wgs, gelu, balanced=False):
             chosen, count = decide(sharing)
     if count == 0:
         return outcome(chosen)
-    last = max(c[0] if c else whole + LAUNCH for c, (whole, _, _) in zip(chosen, ranges))
-    if last >= max(whole for whole, _, _ in ranges):
+    last = max(c[0] if c else alone + LAUNCH for c, (_, _, alone, _) in zip(chosen, ranges))
+    if last >= max(whole for whole, *_ in ranges):
         return outcome([None] * len(ranges))
-    return outcome([c if c and whole + LAUNCH > last else None for c, (whole, _, _) in zip(chosen, ranges)])
+    return outcome([c if c and whole + LAUNCH > last else None for c, (whole, *_) in zip(chosen, ranges)])
 
 
 def test_sharing_is_priced_by_the_slots_and_the_xcds_that_there_are():
@@ -543,7 +544,7 @@ def cut_tiles(items):
     return int((recs["m0"] % 256 == 128).sum())
 
 
-def test_halves_are_compared_with_whole_tiles_and_sharing_with_the_better():
+def test_what_is_not_shared_runs_in_halves_where_they_are_faster():
     """What a flagged launch does with its remainders, against the rule counted from its definition: whole tiles, halves,
     shared tiles, and XCDs of one launch that differ."""
     rng = np.random.default_rng(12)
@@ -568,7 +569,7 @@ def test_halves_are_compared_with_whole_tiles_and_sharing_with_the_better():
 
 def test_a_plan_depends_on_its_table_alone():
     """Planned first thing on a new thread, again on that thread behind launches of other kinds, and here: the same bytes.
-    Eight experts, 2.25 rounds: halves for 32 steps, 4.25 rounds of 112: shared."""
+    Eight experts of 32 steps, 2.25 rounds: halves; four of 112, 4.25 rounds: shared."""
     import threading
 
     grid = 256
