@@ -730,7 +730,7 @@ __global__ __launch_bounds__(NTHREADS, TILE == 256 ? 1 : 2) void grouped_gemm_ke
   int fat_off[MT];
 #pragma unroll
   for (int i = 0; i < MT; ++i) fat_off[i] = tr_row + (((wave_m * (WM / 16) + 2 * i + tr_g) ^ tr_swz) << 4);
-  // Tiles of half height (FP8GMM_ITEM_HALF_HEIGHT: at most 128 valid rows): the wavefronts stand two by two on
+  // Items of half height (FP8GMM_ITEM_HALF_HEIGHT: at most 128 rows of a tile): the wavefronts stand two by two on
   // rows wave_m * 64 + 32 i, i < 2, and issue half the products.  Row-major tokens: the fragment addresses move
   // down by wave_m * 64 rows, a uniform amount that goes into the unit's base address (half_rows_back).
   // Contraction-major: the 16-byte chunk of fragment i is chunk wave_m * 4 + 2 i + tr_g (fat_half).

@@ -196,7 +196,9 @@ int fp8gmm_plan_grouped_gemm_layout(fp8gmm_gemm_problem* probs, int n, int layou
 // result.  Small tiles, 26 weight gradients of skewed splits inside a layer's step, 3 -> 2 / 1.5 / 1 / 0.5 steps a tile: 0.987,
 // 0.979, 0.987, 0.998 of the time in the mean (at 3 the XCDs with the short contractions were through after 87 us and those with
 // the long ones after 128; at 1.5: 64 of 1408 x 2048, 24576 rows 171 -> 156, 64 of 576 x 3536, 18873 297 -> 262; 35 of 320 x 992,
-// 31013 79 -> 85; with operands from HBM, launches alone, 0.968).  Row-sliced launches have one K and do not notice.
+// 31013 79 -> 85).  Of 400 drawn launches alone, operands from HBM, 3 -> 1.5: 0.9955 in the mean, 93 more than 3 % faster and 51
+// slower; steps of 14 drawn layers, three splits each, within the spread of their runs.  Row-sliced launches have one K and do not
+// notice.
 constexpr int kSmallTileWeight = 3, kDualTileWeight = 4, kRowsTileWeight = 2;
 constexpr int kWholeTileForms = FP8GMM_GEMM_TILE_128 | FP8GMM_GEMM_TILE_DUAL | FP8GMM_GEMM_TILE_ROWS;
 // Tile and weight of the form that `layout` asks for; false when it names none that exists with its other flags.

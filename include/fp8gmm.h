@@ -221,9 +221,10 @@ typedef struct fp8gmm_gemm_item {
   int32_t slot;        /* -1: whole tile, the epilogue runs; else the workspace slot that receives the partial sums */
   int32_t flags;       /* FP8GMM_ITEM_* */
 } fp8gmm_gemm_item;    /* 64 bytes */
-/* The tile holds at most 128 valid rows (the last row of tiles of a ragged problem): the kernel runs it at half
+/* The item is at most 128 rows of its tile: the last row of tiles of a ragged problem where it has no more, or one of the two
+ * halves of a tile that FP8GMM_GEMM_BALANCED cuts (m0 is then the half's first row).  The kernel runs it at half
  * height - its wavefronts stand on rows 64 w + 32 i, i < 2, and issue half the products; same loads, same bits.
- * Whole 256 x 256 tiles only (never a piece of a tile shared along K).  In a record without K steps (nk == 0) the
+ * 256 x 256 tiles only, and all of their contraction (never a piece of a tile shared along K).  In a record without K steps (nk == 0) the
  * bit one position up repeats this flag of the workgroup's next record that has K steps: the kernel's load stream
  * skips records without K steps, and what it fetches at the end of a tile is laid out for the tile that follows. */
 #define FP8GMM_ITEM_HALF_HEIGHT 1
@@ -648,7 +649,8 @@ int fp8gmm_moe_scatter_backward(const void* x, const void* grad_out, const int32
 /*
  * The work items that workgroup `wg` of a grouped-GEMM launch with `grid` workgroups (a multiple of 8)
  * processes, in order, for the HOST table `probs` (after fp8gmm_plan_grouped_gemm).  stream_k != 0:
- * as in a launch that shares the tail tiles of each XCD's range along K.  Writes up to max_items records
+ * as in a launch that shares the tail tiles of each XCD's range along K, planned without FP8GMM_GEMM_BALANCED (what that
+ * adds is in the records of fp8gmm_plan_grouped_gemm_launch only).  Writes up to max_items records
  * of 7 int32 - tile, problem, m0, n0, k_begin, nk, slot (k_begin / nk in steps of 128 bytes of K; slot = -1
  * when the item is a whole tile, else its position 2 * workgroup or 2 * workgroup + 1 in the launch's uncompacted
  * slot numbering; fp8gmm_plan_grouped_gemm_launch renumbers the slots in use from 0) - and returns the

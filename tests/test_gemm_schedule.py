@@ -10,6 +10,9 @@ What must hold for ANY problem list, grid and tail-balancing choice (the kernel 
   * the tiles of a problem map one-to-one onto the 256 x 256 blocks of its output, and 32 consecutive tiles of
     a large problem form a compact block (at most 12 distinct row / column blocks), not a strip.
 The expectations are stated from these properties, not recomputed with the scheduler's formulas.
+
+The introspection calls show the schedule of a launch planned without FP8GMM_GEMM_BALANCED.  The launches of the modules and of
+the operand-level calls set it: what it adds is checked on the work lists themselves, further down.
 """
 import numpy as np
 import pytest
@@ -490,7 +493,11 @@ def half_tail_cases():
     wgrad = _lib.GEMM_A_KMAJOR | _lib.GEMM_B_KMAJOR
     yield [(1408, 2048, int(k)) for k in rng.integers(0, 900, 9)], wgrad
     yield [(640, 4096, 0), (640, 4096, 1700), (640, 4096, 40)], wgrad
-    for _ in range(12):
+    yield [(m, 4096, 14336) for m in MLP], 0                       # shared along K
+    yield [(4096, 1408, (m + 127) // 128 * 128) for m in MLP], wgrad
+    for ks in ([208, 1280, 2512], [1440, 0, 0, 0]):                # some XCDs share, others cut
+        yield [(368, 416, k) for k in ks], wgrad
+    for _ in range(30):
         n = int(rng.integers(1, 9))
         shapes = [(int(rng.integers(0, 3000)), 16 * int(rng.integers(1, 130)), 16 * int(rng.integers(0, 60))) for _ in range(n)]
         yield shapes, int(rng.choice([0, _lib.GEMM_B_KMAJOR]))
@@ -500,8 +507,9 @@ def half_tail_cases():
 @pytest.mark.parametrize("stream_k", [False, True])
 def test_a_half_empty_last_round_in_tiles_of_half_height(grid, stream_k):
     """With FP8GMM_GEMM_BALANCED every 128-row half of every tile is still computed exactly once, by a whole tile, a half
-    or the pieces of a shared tile; and a record of half height has the extents of its 128 rows."""
-    cut = 0
+    or the pieces of a shared tile, whose slots follow each other in K order and are completed by one record; a record of half
+    height has the extents of its 128 rows; lists end, and are no longer than without the flag where nothing is cut."""
+    cut = shared = 0
     for shapes, layout in half_tail_cases():
         t = np.zeros(len(shapes), dtype=_lib.GEMM_PROBLEM)
         a_kmajor, b_kmajor = bool(layout & _lib.GEMM_A_KMAJOR), bool(layout & _lib.GEMM_B_KMAJOR)
@@ -511,8 +519,12 @@ def test_a_half_empty_last_round_in_tiles_of_half_height(grid, stream_k):
             t[i]["lda"], t[i]["ldb"], t[i]["ldc"] = m if a_kmajor else max(k, 16), n if b_kmajor else max(k, 16), n
         base, before, _ = _lib.plan_grouped_gemm_launch(t.copy(), layout, grid, stream_k)
         plan, items, fixups = _lib.plan_grouped_gemm_launch(t.copy(), layout | _lib.GEMM_BALANCED, grid, stream_k)
-        assert plan.total_tiles == base.total_tiles
-        done = {}
+        assert plan.total_tiles == base.total_tiles and len(items) == plan.rounds * plan.grid
+        lists = items["prob"].reshape(plan.rounds, plan.grid) >= 0
+        assert not lists[-1].any() and (lists[1:] <= lists[:-1]).all()   # no record behind an end
+        if not cut_tiles(items):
+            assert (plan.n_slots, plan.n_fixups) == (base.n_slots, base.n_fixups) and plan.rounds <= base.rounds
+        done, pieces = {}, {}
         for r in items[items["prob"] >= 0]:
             p, m0, n0, nk = int(r["prob"]), int(r["m0"]), int(r["n0"]), int(r["nk"])
             m, n, k = shapes[p]
@@ -520,6 +532,9 @@ def test_a_half_empty_last_round_in_tiles_of_half_height(grid, stream_k):
             assert m0 < m and n0 < n and m0 % (128 if half else 256) == 0 and n0 % 256 == 0
             assert half or r["slot"] >= 0 or m - m0 > 128
             cut += m0 % 256 == 128
+            if r["slot"] >= 0:
+                assert nk < -(-k // 128)
+                pieces.setdefault((p, m0, n0), []).append((int(r["k_begin"]), int(r["slot"])))
             rows = min(m - m0, 256)
             if half:
                 rows = min(rows, 128)
@@ -535,7 +550,13 @@ def test_a_half_empty_last_round_in_tiles_of_half_height(grid, stream_k):
                 steps[int(r["k_begin"]):int(r["k_begin"]) + max(nk, 1)] += 1
         want = {(p, h, c) for p, (m, n, k) in enumerate(shapes) for h in range(0, m, 128) for c in range(0, n, 256)}
         assert set(done) == want and all((s == 1).all() for s in done.values())
-    assert cut > 0
+        assert sorted(s for tile in pieces.values() for _, s in tile) == list(range(plan.n_slots))
+        assert plan.n_fixups == len(fixups) == len(pieces)
+        for f in fixups:
+            slots = [s for _, s in sorted(pieces.pop((int(f["prob"]), int(f["m0"]), int(f["n0"]))))]
+            assert slots == list(range(int(f["first_slot"]), int(f["first_slot"] + f["n_pieces"])))
+        shared += len(fixups)
+    assert cut > 0 and (shared > 0) == stream_k
 
 
 def cut_tiles(items):
