@@ -74,6 +74,12 @@ __device__ __forceinline__ uint32_t cvt4_fp8(float v0, float v1, float v2, float
   return w;
 }
 
+// The same for values that are no NaN.
+template <int FMT>
+__device__ __forceinline__ uint32_t cvt4_fp8_numbers(float v0, float v1, float v2, float v3) {
+  return cvt_pk_fp8_sat<FMT, true>(v2, v3, cvt_pk_fp8_sat<FMT, false>(v0, v1, 0u));
+}
+
 template <int FMT>
 __device__ __forceinline__ uint8_t cvt1_fp8(float v) {
   return (uint8_t)(cvt4_fp8<FMT>(v, 0.f, 0.f, 0.f) & 0xffu);
@@ -135,6 +141,18 @@ __device__ __forceinline__ void buf_store8(u32x2 v, __amdgpu_buffer_rsrc_t r, ui
 __device__ __forceinline__ float amax_step(float acc, float x) {
   const float ax = fabsf(x);
   return (ax > acc) ? ax : acc;
+}
+
+// max(acc, |a|, |b|) that is a NaN from the first NaN on, in one instruction for two values.  The casts take their tiles this
+// way, without a look at the single value, and take the tile again, value by value (amax_step, cvt4_fp8), where the maximum
+// tells of a NaN: 4 instructions a value where the looks made it 7, and a branch for every four.
+__device__ __forceinline__ float amax_or_nan(float acc, float a, float b) {
+  asm("v_maximum3_f32 %0, %0, |%1|, |%2|" : "+v"(acc) : "v"(a), "v"(b));
+  return acc;
+}
+// A scale that makes no NaN of a number: neither zero, nor infinite, nor a NaN.
+__device__ __forceinline__ bool keeps_numbers(float scale) {
+  return (__float_as_uint(scale) & 0x7fffffffu) - 1u < 0x7f800000u - 1u;
 }
 
 // Wave-wide max of non-negative floats; every lane gets the result.

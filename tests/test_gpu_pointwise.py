@@ -531,3 +531,39 @@ def test_transposed_copies_of_either_store_form(dev, shapes, op):
         assert torch.equal(outs[i].view(torch.uint8), want[i].view(torch.uint8)) and torch.equal(amax[i], want_amax[i]), i
         t = touts[i].view(torch.uint8)
         assert torch.equal(t[:, :rows], want[i].view(torch.uint8).t()) and not t[:, rows:].any(), i
+
+
+@pytest.mark.parametrize("dtype", FP8_DTYPES)
+@pytest.mark.parametrize("numel", [8, 2048, 16384, 16391, 40003])
+def test_a_single_nan_anywhere_and_scales_that_are_no_numbers(dev, dtype, numel):
+    """The casts take a tile without a look at its values and once more where its maximum tells of a NaN: one NaN (quiet, or
+    signalling) at either end of a piece, a step, a block or the tail, infinities and denormals beside it, and scales that make
+    a NaN of a number, against the oracle, byte for byte; the maximum leaves NaNs out."""
+    backend = _backend()
+    g = gen(numel)
+    x0 = randn_bf16((numel,), g)
+    x0[::7] = float("inf")
+    x0[1::11] = 1e-39
+    places = sorted({p for p in (0, 7, 8, 2047, 2048, 16383, 16384, numel - 1, numel // 2) if p < numel})
+    ins, scales = [], []
+    for p in places:
+        for bits in (0x7FC0, 0x7F81, -1):   # quiet, signalling, negative
+            x = x0.clone()
+            x.view(torch.int16)[p] = bits
+            ins.append(x)
+            scales.append(torch.tensor([3.7]))
+    for s in (0.0, -0.0, float("inf"), float("nan"), -float("inf"), 1e-42, 3e38):
+        ins.append(x0.clone())
+        scales.append(torch.tensor([s]))
+    pre = [randn_bf16((numel,), g) for _ in ins]
+    for cast, more in ((ref.multi_quantize, ()), (ref.multi_cast_dgelu, (pre,))):
+        n = len(ins)
+        outs, amaxes = [torch.empty(numel, dtype=dtype) for _ in range(n)], [torch.zeros(1) for _ in range(n)]
+        cast(ins, *more, outs, scales, amaxes)
+        d_outs, d_amaxes = [torch.empty(numel, dtype=dtype, device=dev) for _ in range(n)], _to_dev([torch.zeros(1)] * n, dev)
+        getattr(backend, cast.__name__)(_to_dev(ins, dev), *[_to_dev(m, dev) for m in more], d_outs, _to_dev(scales, dev),
+                                        d_amaxes)
+        torch.cuda.synchronize()
+        for i in range(n):
+            assert_bytes_equal(d_outs[i], outs[i], f"{cast.__name__} {i}")
+            assert_scalar_bits_equal(d_amaxes[i], amaxes[i], f"amax of {cast.__name__} {i}")
