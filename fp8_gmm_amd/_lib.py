@@ -34,6 +34,7 @@ OP_PAD_TRANSPOSE = 2
 OP_PAD_CAST_TRANSPOSE = 3
 OP_PAD_CAST_TRANSPOSE_DGELU = 4
 OP_CAST_DGELU = 5
+OP_ROUTED_CAST, OP_ROUTED_GRADIENT = 6, 7   # of routed passes
 
 # struct fp8gmm_tensor_desc (128 bytes)
 TENSOR_DESC = np.dtype(
@@ -117,6 +118,13 @@ class GemmPlan(ctypes.Structure):
                 ("tile_m", ctypes.c_int32), ("reserved", ctypes.c_int32)]
 
 
+class RoutedRows(ctypes.Structure):
+    """struct fp8gmm_routed_rows: rows of a pass that come from, or go back to, tokens"""
+
+    _fields_ = [("inverse", ctypes.c_void_p), ("weights", ctypes.c_void_p), ("y", ctypes.c_void_p),
+                ("grad_weights", ctypes.c_void_p), ("top_k", ctypes.c_int32), ("reserved", ctypes.c_int32)]
+
+
 class LinearPass(ctypes.Structure):
     """struct fp8gmm_linear_pass: one pass of a grouped linear layer, as the pass planner takes it"""
 
@@ -180,6 +188,7 @@ PASS_CAST = 1
 PASS_GEMM = 2
 LINEAR_FORWARD, LINEAR_BACKWARD, MLP_FORWARD, MLP_BACKWARD = range(4)
 PASS_MAX_EXPERTS = 384
+ROUTED_MAX_TOP_K = 8
 PASS_MAX_ROWS = 0x7FFFFFFF
 PASS_MAX_GRID = 512
 PassTables = ctypes.c_uint64 * (4032 // 8)   # FP8GMM_PASS_TABLES_BYTES, opaque
@@ -202,6 +211,8 @@ EXPORTS = (
     "fp8gmm_lay_out_pass",
     "fp8gmm_build_pass",
     "fp8gmm_run_planned",
+    "fp8gmm_lay_out_routed_pass",
+    "fp8gmm_run_routed",
     "fp8gmm_host_alloc",
     "fp8gmm_host_free",
     "fp8gmm_delayed_scaling_updates",
@@ -321,6 +332,11 @@ def load():
     L.fp8gmm_build_pass.argtypes = [vp, vp, ctypes.POINTER(ScalingUpdate), ci, vp, vp, ci, vp]
     L.fp8gmm_run_planned.restype = ci
     L.fp8gmm_run_planned.argtypes = [vp, ctypes.POINTER(PassLaunch), vp, ctypes.c_size_t, vp]
+    L.fp8gmm_lay_out_routed_pass.restype = ci
+    L.fp8gmm_lay_out_routed_pass.argtypes = [ci, vp, ctypes.POINTER(RoutedRows), ctypes.POINTER(PassPlan), vp]
+    L.fp8gmm_run_routed.restype = ci
+    L.fp8gmm_run_routed.argtypes = [vp, ctypes.POINTER(PassLaunch), ctypes.POINTER(RoutedRows), ctypes.c_int64, vp,
+                                    ctypes.c_size_t, vp]
     L.fp8gmm_sizeof_linear_pass.restype = ctypes.c_size_t
     L.fp8gmm_sizeof_linear_pass.argtypes = []
     L.fp8gmm_sizeof_pass_plan.restype = ctypes.c_size_t

@@ -90,19 +90,20 @@ std::atomic<bool> kernel_timing{false};
 
 // Builds the tables of a pass and enqueues its launches on the current stream.
 void run_pass(int which, const void* desc, const at::Device& device, const Setup* update, Due* due, const Tensor& snapshot_of,
-              const Tensor& snapshot) {
+              const Tensor& snapshot, const fp8gmm_routed_rows* routed = nullptr, int64_t rows = 0) {
   const bool backward = which == FP8GMM_LINEAR_BACKWARD || which == FP8GMM_MLP_BACKWARD;
   if (backward && kernel_timing.load(std::memory_order_relaxed)) {
     // the same launches one by one, each between two events (a module does not come here for such a forward pass)
     const size_t bytes = which == FP8GMM_LINEAR_BACKWARD ? sizeof(fp8gmm_linear_pass) : sizeof(fp8gmm_mlp_pass);
     py::gil_scoped_acquire gil;
     py::module_::import("fp8_gmm_amd.backend")
-        .attr("run_described_pass")(which, (int)device.index(), py::bytes(static_cast<const char*>(desc), bytes));
+        .attr("run_described_pass")(which, (int)device.index(), py::bytes(static_cast<const char*>(desc), bytes),
+                                    py::bytes(reinterpret_cast<const char*>(routed), routed != nullptr ? sizeof(*routed) : 0));
     return;
   }
   fp8gmm_pass_plan plan;
   alignas(16) unsigned char tables[FP8GMM_PASS_TABLES_BYTES];
-  check(fp8gmm_lay_out_pass(which, desc, &plan, tables));
+  check(fp8gmm_lay_out_routed_pass(which, desc, routed, &plan, tables));
   const auto bytes = at::TensorOptions().dtype(at::kByte).device(device);
   const Tensor blob = at::empty({plan.blob_bytes}, bytes);
   void* const stream = current_stream(device);
@@ -136,15 +137,119 @@ void run_pass(int which, const void* desc, const at::Device& device, const Setup
   Tensor workspace;
   if (slots > 0) workspace = at::empty({(int64_t)slots * FP8GMM_GEMM_SLOT_BYTES}, bytes);
   for (int i = 0; i < plan.n_launches; ++i)
-    check(fp8gmm_run_planned(blob.data_ptr(), &plan.launch[i], ptr<void>(workspace),
-                             (size_t)slots * FP8GMM_GEMM_SLOT_BYTES, stream));
+    check(fp8gmm_run_routed(blob.data_ptr(), &plan.launch[i], routed, rows, ptr<void>(workspace),
+                            (size_t)slots * FP8GMM_GEMM_SLOT_BYTES, stream));
 }
 
+// Rows of a pass that come from tokens, go back to tokens, or both: what gather and scatter of a routed layer around the
+// module would do (fp8gmm_routed_rows).
+struct Route {
+  Tensor indices, inverse;   // int32, a permutation of the rows and its inverse, as the sort wrote them
+  Tensor weights;            // fp32, of the rows in (token, choice) order: those of scatter
+  int64_t top_k = 1;
+  bool gathers = false, scatters = false;
+};
+
+// `rows`: of the pass.
+void check_route(const Route& r, int64_t rows, const Tensor& x) {
+  auto list = [&](const Tensor& t, at::ScalarType type) {
+    return t.defined() && t.scalar_type() == type && t.dim() == 1 && t.is_contiguous() && t.numel() == rows &&
+           t.device() == x.device();
+  };
+  TORCH_CHECK(r.top_k >= 1 && r.top_k <= FP8GMM_ROUTED_MAX_TOP_K && rows % r.top_k == 0 && rows <= INT32_MAX,
+              "fp8_gmm_amd: rows are not top_k of every token");
+  TORCH_CHECK(list(r.indices, at::kInt) && list(r.inverse, at::kInt), "fp8_gmm_amd: expected ", rows, " int32 indices");
+  TORCH_CHECK(!r.scatters || list(r.weights, at::kFloat), "fp8_gmm_amd: expected ", rows, " fp32 scatter weights");
+}
+
+// What a row mover takes: contiguous, on 16 bytes.
+Tensor aligned(const Tensor& t) {
+  const Tensor c = t.contiguous();
+  return reinterpret_cast<uintptr_t>(c.data_ptr()) % 16 == 0 ? c : c.clone(at::MemoryFormat::Contiguous);
+}
+
+// out[t] = sum of the rows of token t, weighted where `weights` is defined
+Tensor scatter_rows(const Tensor& rows, const Tensor& inverse, const Tensor& weights, int64_t top_k) {
+  const Tensor out = at::empty({rows.size(0) / top_k, rows.size(1)}, rows.options());
+  check(fp8gmm_moe_scatter(ptr<const void>(rows), ptr<const int32_t>(inverse), ptr<const float>(weights), ptr<void>(out),
+                           (int)out.size(0), (int)out.size(1), (int)top_k, current_stream(rows.device())));
+  return out;
+}
+
+// The part of a route that a backward pass needs.
+struct SavedRoute {
+  bool gathers = false, scatters = false, want_weights = false;
+  int64_t top_k = 1, rows = 0;
+  SavedVariable indices, inverse, weights, y;
+  void save(const Route& r, const Tensor& rows_out, bool dgrad, bool want) {
+    gathers = r.gathers;
+    scatters = r.scatters;
+    want_weights = want;
+    top_k = r.top_k;
+    rows = r.indices.numel();
+    if (scatters) {
+      weights = SavedVariable(r.weights, false);
+      if (want) {
+        indices = SavedVariable(r.indices, false);
+        y = SavedVariable(rows_out, false);
+      }
+    }
+    if (scatters || (gathers && dgrad)) inverse = SavedVariable(r.inverse, false);
+  }
+  void reset() {
+    for (SavedVariable* v : {&indices, &inverse, &weights, &y}) v->reset_data();
+  }
+  // The kernels follow addresses, and a saved-tensor hook may return anything.
+  Tensor list(SavedVariable& v, at::ScalarType type, const at::Device& device) const {
+    const Tensor t = v.unpack();
+    TORCH_CHECK(t.scalar_type() == type && t.numel() == rows && t.is_contiguous() && t.device() == device,
+                "fp8_gmm_amd: a saved-tensor hook returned another tensor than was saved");
+    return t;
+  }
+};
+
+// The gradient of a pass's result as its launches read it: rows, or tokens with what scatter's gradient wants besides.
+struct RoutedGradient {
+  Tensor dy, inverse, weights, y, grad_weights;
+  fp8gmm_routed_rows rows{};
+  RoutedGradient(SavedRoute& r, const Tensor& grad, bool want_weights) : dy(grad) {
+    if (!r.scatters) return;
+    dy = aligned(grad);
+    TORCH_CHECK(dy.size(0) * r.top_k == r.rows, "fp8_gmm_amd: a gradient of another size than the result");
+    inverse = r.list(r.inverse, at::kInt, dy.device());
+    weights = r.list(r.weights, at::kFloat, dy.device());
+    if (want_weights) {
+      y = r.y.unpack();
+      TORCH_CHECK(y.scalar_type() == at::kBFloat16 && y.dim() == 2 && y.size(0) == r.rows && y.size(1) == dy.size(1) &&
+                      y.device() == dy.device(),
+                  "fp8_gmm_amd: a saved-tensor hook returned another tensor than was saved");
+      y = aligned(y);
+      grad_weights = at::empty({r.rows}, weights.options());
+    }
+    rows.inverse = ptr<const int32_t>(inverse);
+    rows.weights = ptr<const float>(weights);
+    rows.y = ptr<const void>(y);
+    rows.grad_weights = ptr<float>(grad_weights);
+    rows.top_k = (int32_t)r.top_k;
+  }
+  const fp8gmm_routed_rows* routed(const SavedRoute& r) const { return r.scatters ? &rows : nullptr; }
+  int64_t size(const SavedRoute& r) const { return r.scatters ? r.rows : dy.size(0); }
+  // grad_weights alone: nothing upstream of the rows wants a gradient
+  void weights_only(SavedRoute& r) const {
+    const Tensor indices = r.list(r.indices, at::kInt, dy.device());
+    check(fp8gmm_moe_scatter_wgrad(ptr<const void>(y), ptr<const void>(dy), ptr<const int32_t>(indices), rows.grad_weights, (int)r.rows,
+                                   (int)dy.size(1), (int)r.top_k, current_stream(dy.device())));
+  }
+};
+
 // The kernels follow addresses: what they read has to be there.  `w` [experts, out, x's columns].
-void check_shapes(const std::vector<int64_t>& sizes, const Tensor& x, const Tensor& w, const Setup& s, int gemms) {
+void check_shapes(const std::vector<int64_t>& sizes, const Tensor& x, const Tensor& w, const Setup& s, int gemms,
+                  const Route* route) {
   int64_t rows = 0;
   for (const int64_t n : sizes) rows += n;
-  TORCH_CHECK(rows == x.size(0), "group_sizes must sum to the number of input rows");
+  TORCH_CHECK(rows == x.size(0) * (route != nullptr && route->gathers ? route->top_k : 1),
+              "group_sizes must sum to the number of input rows");
+  if (route != nullptr) check_route(*route, rows, x);
   TORCH_CHECK((int64_t)sizes.size() <= w.size(0), "fp8_gmm_amd: group_sizes has ", sizes.size(), " entries for ", w.size(0),
               " weights");
   TORCH_CHECK(x.size(1) == w.size(2), "fp8_gmm_amd: the input has ", x.size(1), " columns, the weights expect ", w.size(2));
@@ -191,60 +296,82 @@ struct GroupedLinearBackward : public Node {
   int64_t in = 0, out = 0;
   SavedVariable x_fp8, w_fp8;
   Tensor scale_inv;   // the forward factors as they were
+  SavedRoute route;
 
   std::string name() const override { return "GroupedLinearBackward"; }
   void release_variables() override {
     const std::lock_guard<std::mutex> lock(mutex_);   // backward passes of several threads may meet in one graph
     x_fp8.reset_data();
     w_fp8.reset_data();
+    route.reset();
   }
   variable_list apply(variable_list&& grads) override {
     const std::lock_guard<std::mutex> lock(mutex_);
     at::AutoGradMode no_grad(false);
-    variable_list result(2);
+    variable_list result(route.scatters ? 3 : 2);
     const bool dgrad = task_should_compute_output(0), wgrad = task_should_compute_output(1);
-    const Tensor dy = gradient_of_result(*this, grads);
-    const c10::OptionalDeviceGuard guard(dy.device());
+    const bool rgrad = route.want_weights && task_should_compute_output(2);
+    const Tensor grad = gradient_of_result(*this, grads);
+    const c10::OptionalDeviceGuard guard(grad.device());
+    const RoutedGradient from(route, grad, rgrad);
+    const Tensor& dy = from.dy;
+    if (rgrad) result[2] = from.grad_weights;
+    if (!dgrad && !wgrad && route.scatters) {
+      if (rgrad) from.weights_only(route);
+      return result;
+    }
+    const int64_t rows = from.size(route);
     const Tensor x = wgrad ? x_fp8.unpack() : Tensor(), w = dgrad ? w_fp8.unpack() : Tensor();
-    const Tensor dy_fp8 = at::empty(dy.sizes(), dy.options().dtype(setup.bwd_type()));
-    if (dgrad) result[0] = at::empty({dy.size(0), in}, dy.options());
+    const Tensor dy_fp8 = at::empty({rows, out}, dy.options().dtype(setup.bwd_type()));
+    Tensor dx;
+    if (dgrad) dx = at::empty({rows, in}, dy.options());
     if (wgrad) result[1] = at::empty({(int64_t)sizes.size(), out, in}, dy.options());
-    fp8gmm_linear_pass d = linear_desc(setup, sizes, dy.size(0), in, out);
+    fp8gmm_linear_pass d = linear_desc(setup, sizes, rows, in, out);
     d.dgrad = dgrad;
     d.wgrad = wgrad;
     d.dy = ptr<void>(dy);
     d.dy_fp8 = ptr<void>(dy_fp8);
     d.x_fp8 = ptr<void>(x);
     d.w_fp8 = ptr<void>(w);
-    d.dx = ptr<void>(result[0]);
+    d.dx = ptr<void>(dx);
     d.dw = ptr<void>(result[1]);
     d.fwd_scale_inv = ptr<float>(scale_inv);
     d.bwd_scale = ptr<float>(setup.bwd_scale);
     d.bwd_scale_inv = ptr<float>(setup.bwd_scale_inv);
     d.bwd_amax = ptr<float>(setup.bwd_amax);
-    run_pass(FP8GMM_LINEAR_BACKWARD, &d, dy.device(), nullptr, nullptr, Tensor(), Tensor());
+    run_pass(FP8GMM_LINEAR_BACKWARD, &d, dy.device(), nullptr, nullptr, Tensor(), Tensor(), from.routed(route), rows);
+    if (dgrad) result[0] = route.gathers ? scatter_rows(dx, route.list(route.inverse, at::kInt, dx.device()), Tensor(), route.top_k) : dx;
     return result;
   }
 };
 
 Tensor linear_step(const Tensor& x, const Tensor& w, const py::object& group_sizes, const std::optional<Tensor>& cached,
-                   bool cast_weights, const Setup& setup, Due& due) {
+                   bool cast_weights, const Setup& setup, Due& due, const Route* route) {
   return with_python_errors([&, sizes = sizes_of(group_sizes)]() mutable {
     py::gil_scoped_release no_gil;
-    check_shapes(sizes, x, w, setup, 1);
+    check_shapes(sizes, x, w, setup, 1, route);
     check_no_tangent({x, w});
+    const bool gathers = route != nullptr && route->gathers, scatters = route != nullptr && route->scatters;
+    if (scatters) check_no_tangent({route->weights});
     const c10::OptionalDeviceGuard guard(x.device());
     const bool grad = at::GradMode::is_enabled();
     const bool dgrad = grad && x.requires_grad(), wgrad = grad && w.requires_grad();
-    Tensor y, x_fp8, w_fp8, scale_inv;
+    const bool rgrad = grad && scatters && route->weights.requires_grad();
+    const int64_t tokens = gathers ? x.size(0) * route->top_k : x.size(0);   // rows of the pass
+    Tensor y, rows_out, x_fp8, w_fp8, scale_inv;
     {
       at::AutoGradMode no_grad(false);
       const auto fp8 = x.options().dtype(setup.fwd_type());
-      x_fp8 = at::empty(x.sizes(), fp8);
+      x_fp8 = at::empty({tokens, x.size(1)}, fp8);
       w_fp8 = cached.has_value() ? *cached : at::empty(w.sizes(), fp8);
-      y = at::empty({x.size(0), w.size(1)}, x.options());
+      y = at::empty({tokens, w.size(1)}, x.options());
       if (dgrad || wgrad) scale_inv = at::empty_like(setup.fwd_scale_inv);
-      fp8gmm_linear_pass d = linear_desc(setup, sizes, x.size(0), w.size(2), w.size(1));
+      fp8gmm_linear_pass d = linear_desc(setup, sizes, tokens, w.size(2), w.size(1));
+      fp8gmm_routed_rows routed{};
+      if (gathers) {
+        routed.inverse = ptr<const int32_t>(route->inverse);
+        routed.top_k = (int32_t)route->top_k;
+      }
       d.cast_weights = cast_weights;
       d.x = ptr<void>(x);
       d.x_fp8 = ptr<void>(x_fp8);
@@ -255,11 +382,17 @@ Tensor linear_step(const Tensor& x, const Tensor& w, const py::object& group_siz
       d.fwd_scale_inv = ptr<float>(setup.fwd_scale_inv);
       d.fwd_amax = ptr<float>(setup.fwd_amax);
       run_pass(FP8GMM_LINEAR_FORWARD, &d, x.device(), &setup, &due, scale_inv.defined() ? setup.fwd_scale_inv : Tensor(),
-               scale_inv);
+               scale_inv, gathers ? &routed : nullptr, tokens);
+      if (scatters) {
+        rows_out = y;
+        y = scatter_rows(rows_out, route->inverse, route->weights, route->top_k);
+      }
     }
-    if (dgrad || wgrad) {
+    if (dgrad || wgrad || rgrad) {
       auto node = std::shared_ptr<GroupedLinearBackward>(new GroupedLinearBackward(), torch::autograd::deleteNode);
-      node->set_next_edges(torch::autograd::collect_next_edges(x, w));
+      if (scatters) node->set_next_edges(torch::autograd::collect_next_edges(x, w, route->weights));
+      else node->set_next_edges(torch::autograd::collect_next_edges(x, w));
+      if (route != nullptr) node->route.save(*route, rows_out, dgrad, rgrad);
       node->setup = setup;
       node->sizes = std::move(sizes);
       node->in = w.size(2);
@@ -296,26 +429,37 @@ struct GroupedMlpBackward : public Node {
   int64_t hidden = 0, ffn = 0;
   SavedVariable x_fp8, w1_fp8, w2_fp8, pre, act_fp8;
   Tensor scale_inv;
+  SavedRoute route;
 
   std::string name() const override { return "GroupedMlpBackward"; }
   void release_variables() override {
     const std::lock_guard<std::mutex> lock(mutex_);   // backward passes of several threads may meet in one graph
     for (SavedVariable* v : {&x_fp8, &w1_fp8, &w2_fp8, &pre, &act_fp8}) v->reset_data();
+    route.reset();
   }
   variable_list apply(variable_list&& grads) override {
     const std::lock_guard<std::mutex> lock(mutex_);
     at::AutoGradMode no_grad(false);
-    variable_list result(3);
+    variable_list result(route.scatters ? 4 : 3);
     const bool want_x = dgrad && task_should_compute_output(0);
     const bool want_w = wgrad && (task_should_compute_output(1) || task_should_compute_output(2));
-    const Tensor dy = gradient_of_result(*this, grads);
-    const c10::OptionalDeviceGuard guard(dy.device());
-    const int64_t tokens = dy.size(0), e = (int64_t)sizes.size();
+    const bool rgrad = route.want_weights && task_should_compute_output(3);
+    const Tensor grad = gradient_of_result(*this, grads);
+    const c10::OptionalDeviceGuard guard(grad.device());
+    const RoutedGradient from(route, grad, rgrad);
+    const Tensor& dy = from.dy;
+    if (rgrad) result[3] = from.grad_weights;
+    if (!want_x && !want_w && route.scatters) {
+      if (rgrad) from.weights_only(route);
+      return result;
+    }
+    const int64_t tokens = from.size(route), e = (int64_t)sizes.size();
     const auto bf16 = dy.options(), fp8 = dy.options().dtype(setup.bwd_type());
     const Tensor p = pre.unpack(), w2 = w2_fp8.unpack(), w1 = want_x ? w1_fp8.unpack() : Tensor();
     const Tensor x = want_w ? x_fp8.unpack() : Tensor(), act = want_w ? act_fp8.unpack() : Tensor();
-    const Tensor dy_fp8 = at::empty(dy.sizes(), fp8), dact = at::empty({tokens, ffn}, bf16), dpre = at::empty({tokens, ffn}, fp8);
-    if (want_x) result[0] = at::empty(dy.sizes(), bf16);
+    const Tensor dy_fp8 = at::empty({tokens, hidden}, fp8), dact = at::empty({tokens, ffn}, bf16), dpre = at::empty({tokens, ffn}, fp8);
+    Tensor dx;
+    if (want_x) dx = at::empty({tokens, hidden}, bf16);
     if (want_w) {
       result[1] = at::empty({e, ffn, hidden}, bf16);
       result[2] = at::empty({e, hidden, ffn}, bf16);
@@ -332,43 +476,52 @@ struct GroupedMlpBackward : public Node {
     d.dy_fp8 = ptr<void>(dy_fp8);
     d.dact = ptr<void>(dact);
     d.dpre_fp8 = ptr<void>(dpre);
-    d.dx = ptr<void>(result[0]);
+    d.dx = ptr<void>(dx);
     d.dw1 = ptr<void>(result[1]);
     d.dw2 = ptr<void>(result[2]);
     d.fwd_scale_inv = ptr<float>(scale_inv);
     d.bwd_scale = ptr<float>(setup.bwd_scale);
     d.bwd_scale_inv = ptr<float>(setup.bwd_scale_inv);
     d.bwd_amax = ptr<float>(setup.bwd_amax);
-    run_pass(FP8GMM_MLP_BACKWARD, &d, dy.device(), nullptr, nullptr, Tensor(), Tensor());
+    run_pass(FP8GMM_MLP_BACKWARD, &d, dy.device(), nullptr, nullptr, Tensor(), Tensor(), from.routed(route), tokens);
+    if (want_x) result[0] = route.gathers ? scatter_rows(dx, route.list(route.inverse, at::kInt, dx.device()), Tensor(), route.top_k) : dx;
     return result;
   }
 };
 
 Tensor mlp_step(const Tensor& x, const Tensor& w1, const Tensor& w2, const py::object& group_sizes,
                 const std::optional<Tensor>& cached1, const std::optional<Tensor>& cached2, bool cast_weights,
-                const Setup& setup, Due& due) {
+                const Setup& setup, Due& due, const Route* route) {
   return with_python_errors([&, sizes = sizes_of(group_sizes)]() mutable {
     py::gil_scoped_release no_gil;
-    check_shapes(sizes, x, w1, setup, 2);
+    check_shapes(sizes, x, w1, setup, 2, route);
     TORCH_CHECK(w2.size(0) == w1.size(0) && w2.size(1) == w1.size(2) && w2.size(2) == w1.size(1),
                 "fp8_gmm_amd: fc2's weights do not follow fc1's");
     check_no_tangent({x, w1, w2});
+    const bool gathers = route != nullptr && route->gathers, scatters = route != nullptr && route->scatters;
+    if (scatters) check_no_tangent({route->weights});
     const c10::OptionalDeviceGuard guard(x.device());
     const bool grad = at::GradMode::is_enabled();
     const bool dgrad = grad && x.requires_grad(), wgrad = grad && w1.requires_grad();
-    const int64_t tokens = x.size(0), hidden = x.size(1), ffn = w1.size(1);
-    Tensor y, x_fp8, w1_fp8, w2_fp8, pre, act_fp8, scale_inv;
+    const bool rgrad = grad && scatters && route->weights.requires_grad();
+    const int64_t tokens = gathers ? x.size(0) * route->top_k : x.size(0), hidden = x.size(1), ffn = w1.size(1);   // rows of the pass
+    Tensor y, rows_out, x_fp8, w1_fp8, w2_fp8, pre, act_fp8, scale_inv;
     {
       at::AutoGradMode no_grad(false);
       const auto fp8 = x.options().dtype(setup.fwd_type());
-      x_fp8 = at::empty(x.sizes(), fp8);
+      x_fp8 = at::empty({tokens, hidden}, fp8);
       w1_fp8 = cached1.has_value() ? *cached1 : at::empty(w1.sizes(), fp8);
       w2_fp8 = cached2.has_value() ? *cached2 : at::empty(w2.sizes(), fp8);
       pre = at::empty({tokens, ffn}, x.options());
       act_fp8 = at::empty({tokens, ffn}, fp8);
-      y = at::empty(x.sizes(), x.options());
+      y = at::empty({tokens, hidden}, x.options());
       if (dgrad || wgrad) scale_inv = at::empty_like(setup.fwd_scale_inv);
       fp8gmm_mlp_pass d = mlp_desc(setup, sizes, tokens, hidden, ffn);
+      fp8gmm_routed_rows routed{};
+      if (gathers) {
+        routed.inverse = ptr<const int32_t>(route->inverse);
+        routed.top_k = (int32_t)route->top_k;
+      }
       d.cast_weights = cast_weights;
       d.x = ptr<void>(x);
       d.x_fp8 = ptr<void>(x_fp8);
@@ -383,19 +536,27 @@ Tensor mlp_step(const Tensor& x, const Tensor& w1, const Tensor& w2, const py::o
       d.fwd_scale_inv = ptr<float>(setup.fwd_scale_inv);
       d.fwd_amax = ptr<float>(setup.fwd_amax);
       run_pass(FP8GMM_MLP_FORWARD, &d, x.device(), &setup, &due, scale_inv.defined() ? setup.fwd_scale_inv : Tensor(),
-               scale_inv);
+               scale_inv, gathers ? &routed : nullptr, tokens);
+      if (scatters) {
+        rows_out = y;
+        y = scatter_rows(rows_out, route->inverse, route->weights, route->top_k);
+      }
     }
-    if (dgrad || wgrad) {
+    if (dgrad || wgrad || rgrad) {
       auto node = std::shared_ptr<GroupedMlpBackward>(new GroupedMlpBackward(), torch::autograd::deleteNode);
-      node->set_next_edges(torch::autograd::collect_next_edges(x, w1, w2));
+      if (scatters) node->set_next_edges(torch::autograd::collect_next_edges(x, w1, w2, route->weights));
+      else node->set_next_edges(torch::autograd::collect_next_edges(x, w1, w2));
+      if (route != nullptr) node->route.save(*route, rows_out, dgrad, rgrad);
       node->setup = setup;
       node->sizes = std::move(sizes);
       node->dgrad = dgrad;
       node->wgrad = wgrad;
       node->hidden = hidden;
       node->ffn = ffn;
-      node->pre = SavedVariable(pre, false);
-      node->w2_fp8 = SavedVariable(w2_fp8, false);
+      if (dgrad || wgrad) {
+        node->pre = SavedVariable(pre, false);
+        node->w2_fp8 = SavedVariable(w2_fp8, false);
+      }
       if (dgrad) node->w1_fp8 = SavedVariable(w1_fp8, false);
       if (wgrad) {
         node->x_fp8 = SavedVariable(x_fp8, false);
@@ -481,8 +642,15 @@ PYBIND11_MODULE(_host, m) {
         return Due{true, fwd_max, bwd_max, margin, most_recent, keep_weights};
       }))
       .def_readonly("due", &Due::due);
-  m.def("linear_step", &linear_step);
-  m.def("mlp_step", &mlp_step);
+  py::class_<Route>(m, "Route")
+      .def(py::init([](const Tensor& indices, const Tensor& inverse, const std::optional<Tensor>& weights, int64_t top_k,
+                       bool gathers, bool scatters) {
+        return Route{indices, inverse, weights.value_or(Tensor()), top_k, gathers, scatters};
+      }));
+  m.def("linear_step", &linear_step, py::arg("x"), py::arg("w"), py::arg("group_sizes"), py::arg("cached"), py::arg("cast_weights"),
+        py::arg("setup"), py::arg("due"), py::arg("route") = nullptr);
+  m.def("mlp_step", &mlp_step, py::arg("x"), py::arg("w1"), py::arg("w2"), py::arg("group_sizes"), py::arg("cached1"),
+        py::arg("cached2"), py::arg("cast_weights"), py::arg("setup"), py::arg("due"), py::arg("route") = nullptr);
   m.def("cast_weights", &cast_weights);
   m.def("set_kernel_timing", [](bool on) { kernel_timing.store(on, std::memory_order_relaxed); });
 }

@@ -20,6 +20,11 @@ int launch_gemm_merging(const fp8gmm_gemm_problem* probs_dev, int n, const fp8gm
                         int out_kind, int epilogue, void* workspace, size_t workspace_bytes,
                         const fp8gmm_tensor_desc* merge_descs, int merge_n, void* stream);
 
+// The casts of routed rows (FP8GMM_OP_ROUTED_*, fp8gmm_routed_rows), `rows` of them in all; without `merge` the merge of the
+// experts' maxima is left to the GEMM launch that follows, as above.
+int launch_routed_cast(fp8gmm_tensor_desc* descs_dev, int n, int op, int out_fmt, const fp8gmm_routed_rows& routed, int64_t rows,
+                       bool merge, void* stream);
+
 struct GemmRanges;
 struct PassTables;
 

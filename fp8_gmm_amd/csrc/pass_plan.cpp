@@ -59,6 +59,14 @@ struct Pass {
     c.out_fmt = out_fmt;
     return c;
   }
+  // The rows of the pass: slices of `in` [rows, cols], or what `routed` says of tokens.
+  CastSpec& add_rows_cast(int fmt, const fp8gmm_routed_rows* routed, int routed_op, const void* in, void* out, int64_t cols,
+                          const float* scale, float* amax, int stride) {
+    CastSpec& c = add_cast(routed != nullptr ? routed_op : FP8GMM_OP_QUANTIZE, fmt);
+    slices(c, in, nullptr, out, cols, scale, amax, stride);
+    c.run[0].routed = routed != nullptr;
+    return c;
+  }
   // slices of a token-major tensor [tokens, cols]
   static void slices(CastSpec& c, const void* in, const void* in2, void* out, int64_t cols, const float* scale, float* amax,
                      int stride) {
@@ -249,7 +257,7 @@ int describe_cast(const Pass& pass, const Pass::Launch& l, fp8gmm_pass_launch* r
     for (int i = 0; i < pass.experts; ++i) {
       const int64_t numel = l.cast.run[r].cols > 0 ? pass.group_sizes[i] * l.cast.run[r].cols : l.cast.run[r].numel;
       if (numel >= ((int64_t)1 << 31)) return FP8GMM_ERR_BAD_SHAPE;
-      blocks += (numel + fp8gmm::kPwBlockElems - 1) / fp8gmm::kPwBlockElems;
+      blocks += (numel + fp8gmm::kPwBlockElems - 1) / fp8gmm::kPwBlockElems;   // routed rows: whether there are any
       work += numel * per_element;
     }
   if (blocks > INT32_MAX / 2) return FP8GMM_ERR_BAD_SHAPE;
@@ -457,6 +465,18 @@ bool rows_missing(const Desc* s, std::initializer_list<const void*> tensors) {
     if (t == nullptr) return true;
   return false;
 }
+// What the kernels of routed rows follow: `tensors` are the token-major tensors of the pass that they read or write.
+int check_routed(const fp8gmm_routed_rows* r, int64_t tokens, bool backward, std::initializer_list<const void*> tensors) {
+  if (r == nullptr) return FP8GMM_OK;
+  if (r->top_k < 1 || r->top_k > FP8GMM_ROUTED_MAX_TOP_K || tokens % r->top_k != 0 || tokens > INT32_MAX)
+    return FP8GMM_ERR_BAD_ARGUMENT;
+  if (tokens == 0) return FP8GMM_OK;
+  if (r->inverse == nullptr || (backward && r->weights == nullptr)) return FP8GMM_ERR_NULL_POINTER;
+  if (backward && r->grad_weights != nullptr && r->y == nullptr) return FP8GMM_ERR_NULL_POINTER;
+  uintptr_t low = backward ? reinterpret_cast<uintptr_t>(r->y) : 0;
+  for (const void* t : tensors) low |= reinterpret_cast<uintptr_t>(t);
+  return (low & 15) == 0 ? FP8GMM_OK : FP8GMM_ERR_ALIGNMENT;
+}
 bool tile_policy_ok(int p) { return p == 0 || p == 128 || p == 256 || p == FP8GMM_GEMM_TILE_DUAL || p == FP8GMM_GEMM_TILE_ROWS; }
 
 void begin_pass(Pass& p, int experts, const int64_t* sizes, int grid, int stream_k, int tile_policy) {
@@ -480,7 +500,7 @@ int check_common(const fp8gmm_linear_pass* s) {
   return FP8GMM_OK;
 }
 
-int linear_forward(const fp8gmm_linear_pass* s, Pass& p) {
+int linear_forward(const fp8gmm_linear_pass* s, const fp8gmm_routed_rows* routed, Pass& p) {
   const int rc = check_common(s);
   if (rc != FP8GMM_OK) return rc;
   if (rows_missing(s, {s->x, s->x_fp8, s->y}) || s->w_fp8 == nullptr || s->fwd_scale == nullptr ||
@@ -488,18 +508,23 @@ int linear_forward(const fp8gmm_linear_pass* s, Pass& p) {
     return FP8GMM_ERR_NULL_POINTER;
   const int K = s->in_features, N = s->out_features;
   if ((int64_t)N * K >= ((int64_t)1 << 31)) return FP8GMM_ERR_BAD_SHAPE;
+  const int routed_rc = check_routed(routed, s->tokens, false, {s->x, s->x_fp8});
+  if (routed_rc != FP8GMM_OK) return routed_rc;
   begin_pass(p, s->experts, s->group_sizes, s->grid, s->stream_k, s->tile_policy);
-  // cast: the experts' activation slices, then (unless cached copies are reused) their weights
-  CastSpec& cast = p.add_cast(FP8GMM_OP_QUANTIZE, s->fwd_fmt);
-  Pass::slices(cast, s->x, nullptr, s->x_fp8, K, s->fwd_scale, s->fwd_amax, 3);
-  if (s->cast_weights) Pass::stack(cast, s->w, s->w_fp8, (int64_t)N * K, s->fwd_scale + 1, s->fwd_amax + 1);
+  // cast: the experts' activation slices, then (unless cached copies are reused) their weights; routed rows have a launch of
+  // their own, right in front of the GEMM that reads them
+  if (routed != nullptr && s->cast_weights)
+    Pass::stack(p.add_cast(FP8GMM_OP_QUANTIZE, s->fwd_fmt), s->w, s->w_fp8, (int64_t)N * K, s->fwd_scale + 1, s->fwd_amax + 1);
+  CastSpec& cast = p.add_rows_cast(s->fwd_fmt, routed, FP8GMM_OP_ROUTED_CAST, s->x, s->x_fp8, K, s->fwd_scale, s->fwd_amax, 3);
+  if (routed == nullptr && s->cast_weights)
+    Pass::stack(cast, s->w, s->w_fp8, (int64_t)N * K, s->fwd_scale + 1, s->fwd_amax + 1);
   // y[rows of expert i] = x_fp8[rows] . w_fp8[i]^T
   p.row_gemm(s->x_fp8, s->w_fp8, s->y, 2, nullptr, N, K, false, s->fwd_fmt, s->fwd_fmt, s->fwd_scale_inv, 3,
              s->fwd_scale_inv + 1).two_roundings = s->two_roundings != 0;
   return FP8GMM_OK;
 }
 
-int linear_backward(const fp8gmm_linear_pass* s, Pass& p) {
+int linear_backward(const fp8gmm_linear_pass* s, const fp8gmm_routed_rows* routed, Pass& p) {
   const int rc = check_common(s);
   if (rc != FP8GMM_OK) return rc;
   if (rows_missing(s, {s->dy, s->dy_fp8}) || s->bwd_scale == nullptr || s->bwd_scale_inv == nullptr ||
@@ -509,9 +534,10 @@ int linear_backward(const fp8gmm_linear_pass* s, Pass& p) {
       (s->wgrad && (s->dw == nullptr || rows_missing(s, {s->x_fp8}))))
     return FP8GMM_ERR_NULL_POINTER;
   const int K = s->in_features, N = s->out_features;
+  const int routed_rc = check_routed(routed, s->tokens, true, {s->dy, s->dy_fp8});
+  if (routed_rc != FP8GMM_OK) return routed_rc;
   begin_pass(p, s->experts, s->group_sizes, s->grid, s->stream_k, s->tile_policy);
-  CastSpec& cast = p.add_cast(FP8GMM_OP_QUANTIZE, s->bwd_fmt);
-  Pass::slices(cast, s->dy, nullptr, s->dy_fp8, N, s->bwd_scale, s->bwd_amax, 2);
+  p.add_rows_cast(s->bwd_fmt, routed, FP8GMM_OP_ROUTED_GRADIENT, s->dy, s->dy_fp8, N, s->bwd_scale, s->bwd_amax, 2);
   // dw[i] = dy_fp8[rows]^T . x_fp8[rows]: both read in place, contraction over the expert's rows.  Ahead of the data
   // gradient: its operands are the tensors the casts have just written, and a launch that reads them later, behind
   // the data gradient's pass over all the weights, finds less of them in the memory-side cache (config 3: 139 -> 126 us)
@@ -540,7 +566,7 @@ int check_mlp(const fp8gmm_mlp_pass* s) {
   return FP8GMM_OK;
 }
 
-int mlp_forward(const fp8gmm_mlp_pass* s, Pass& p) {
+int mlp_forward(const fp8gmm_mlp_pass* s, const fp8gmm_routed_rows* routed, Pass& p) {
   const int rc = check_mlp(s);
   if (rc != FP8GMM_OK) return rc;
   if (rows_missing(s, {s->x, s->x_fp8, s->pre, s->act_fp8, s->y}) || s->w1_fp8 == nullptr || s->w2_fp8 == nullptr ||
@@ -549,15 +575,19 @@ int mlp_forward(const fp8gmm_mlp_pass* s, Pass& p) {
     return FP8GMM_ERR_NULL_POINTER;
   const int H = s->hidden, F = s->ffn;
   const int64_t g2 = 3 * (int64_t)s->experts;   // first forward slot of the fc2 GEMMs
+  const int routed_rc = check_routed(routed, s->tokens, false, {s->x, s->x_fp8});
+  if (routed_rc != FP8GMM_OK) return routed_rc;
   begin_pass(p, s->experts, s->group_sizes, s->grid, s->stream_k, s->tile_policy);
   // cast.  fc2's weights first and the input last: the launch walks its table in order, and what it wrote last is
   // what the memory-side cache still holds when fc1's GEMM starts reading
-  CastSpec& cast = p.add_cast(FP8GMM_OP_QUANTIZE, s->fwd_fmt);
   if (s->cast_weights) {
+    CastSpec& cast = p.add_cast(FP8GMM_OP_QUANTIZE, s->fwd_fmt);
     Pass::stack(cast, s->w2, s->w2_fp8, (int64_t)H * F, s->fwd_scale + g2 + 1, s->fwd_amax + g2 + 1);
     Pass::stack(cast, s->w1, s->w1_fp8, (int64_t)H * F, s->fwd_scale + 1, s->fwd_amax + 1);
+    if (routed == nullptr) Pass::slices(cast, s->x, nullptr, s->x_fp8, H, s->fwd_scale, s->fwd_amax, 3);
   }
-  Pass::slices(cast, s->x, nullptr, s->x_fp8, H, s->fwd_scale, s->fwd_amax, 3);
+  if (routed != nullptr || !s->cast_weights)
+    p.add_rows_cast(s->fwd_fmt, routed, FP8GMM_OP_ROUTED_CAST, s->x, s->x_fp8, H, s->fwd_scale, s->fwd_amax, 3);
   // fc1 with the GELU in its epilogue: pre (bf16) and act_fp8 = fp8(gelu(pre) * scale of fc2's input)
   Pass::Launch& fc1 = p.row_gemm(s->x_fp8, s->w1_fp8, s->act_fp8, 1, s->pre, F, H, false, s->fwd_fmt, s->fwd_fmt,
                                  s->fwd_scale_inv, 3, s->fwd_scale_inv + 1);
@@ -570,7 +600,7 @@ int mlp_forward(const fp8gmm_mlp_pass* s, Pass& p) {
   return FP8GMM_OK;
 }
 
-int mlp_backward(const fp8gmm_mlp_pass* s, Pass& p) {
+int mlp_backward(const fp8gmm_mlp_pass* s, const fp8gmm_routed_rows* routed, Pass& p) {
   const int rc = check_mlp(s);
   if (rc != FP8GMM_OK) return rc;
   if (rows_missing(s, {s->dy, s->dy_fp8, s->pre, s->dact, s->dpre_fp8}) || s->w2_fp8 == nullptr ||
@@ -581,11 +611,12 @@ int mlp_backward(const fp8gmm_mlp_pass* s, Pass& p) {
     return FP8GMM_ERR_NULL_POINTER;
   const int H = s->hidden, F = s->ffn;
   const int64_t f2 = 3 * (int64_t)s->experts, b2 = 2 * (int64_t)s->experts;   // first slots of the fc2 GEMMs
+  const int routed_rc = check_routed(routed, s->tokens, true, {s->dy, s->dy_fp8});
+  if (routed_rc != FP8GMM_OK) return routed_rc;
   begin_pass(p, s->experts, s->group_sizes, s->grid, s->stream_k, s->tile_policy);
   // cast of the gradient.  It takes the first group of backward slots although it belongs to fc2, and the
   // gradient of pre the second (fp8_gmm/grouped_mlp.py:183-184,278-279): the groups follow the order of the pass
-  CastSpec& cast = p.add_cast(FP8GMM_OP_QUANTIZE, s->bwd_fmt);
-  Pass::slices(cast, s->dy, nullptr, s->dy_fp8, H, s->bwd_scale, s->bwd_amax, 2);
+  p.add_rows_cast(s->bwd_fmt, routed, FP8GMM_OP_ROUTED_GRADIENT, s->dy, s->dy_fp8, H, s->bwd_scale, s->bwd_amax, 2);
   // dw2[i] (H x F) = dy_fp8[rows_i]^T . act_fp8[rows_i]
   if (s->wgrad)
     p.weight_gradient(s->dy_fp8, s->act_fp8, s->dw2, H, F, s->bwd_fmt, s->fwd_fmt, s->bwd_scale_inv, s->fwd_scale_inv + f2);
@@ -606,10 +637,10 @@ int mlp_backward(const fp8gmm_mlp_pass* s, Pass& p) {
 }
 
 template <class Desc>
-int plan_pass(int (*describe)(const Desc*, Pass&), const Desc* desc, void* blob, size_t blob_bytes, fp8gmm_pass_plan* out) {
+int plan_pass(int (*describe)(const Desc*, const fp8gmm_routed_rows*, Pass&), const Desc* desc, void* blob, size_t blob_bytes, fp8gmm_pass_plan* out) {
   if (out == nullptr) return FP8GMM_ERR_NULL_POINTER;
   Pass pass;
-  const int rc = describe(desc, pass);
+  const int rc = describe(desc, nullptr, pass);
   if (rc != FP8GMM_OK) return rc;
   memset(out, 0, sizeof(*out));
   return write_pass(pass, blob, blob_bytes, out);
@@ -632,20 +663,25 @@ int fp8gmm_plan_mlp_backward(const fp8gmm_mlp_pass* s, void* blob, size_t blob_b
   return plan_pass(mlp_backward, s, blob, blob_bytes, out);
 }
 
-int fp8gmm_lay_out_pass(int which, const void* desc, fp8gmm_pass_plan* out, void* tables) {
+int fp8gmm_lay_out_routed_pass(int which, const void* desc, const fp8gmm_routed_rows* routed, fp8gmm_pass_plan* out,
+                               void* tables) {
   if (out == nullptr || desc == nullptr || tables == nullptr) return FP8GMM_ERR_NULL_POINTER;
   Pass pass;
   int rc = FP8GMM_ERR_BAD_ARGUMENT;
   switch (which) {
-    case FP8GMM_LINEAR_FORWARD: rc = linear_forward(static_cast<const fp8gmm_linear_pass*>(desc), pass); break;
-    case FP8GMM_LINEAR_BACKWARD: rc = linear_backward(static_cast<const fp8gmm_linear_pass*>(desc), pass); break;
-    case FP8GMM_MLP_FORWARD: rc = mlp_forward(static_cast<const fp8gmm_mlp_pass*>(desc), pass); break;
-    case FP8GMM_MLP_BACKWARD: rc = mlp_backward(static_cast<const fp8gmm_mlp_pass*>(desc), pass); break;
+    case FP8GMM_LINEAR_FORWARD: rc = linear_forward(static_cast<const fp8gmm_linear_pass*>(desc), routed, pass); break;
+    case FP8GMM_LINEAR_BACKWARD: rc = linear_backward(static_cast<const fp8gmm_linear_pass*>(desc), routed, pass); break;
+    case FP8GMM_MLP_FORWARD: rc = mlp_forward(static_cast<const fp8gmm_mlp_pass*>(desc), routed, pass); break;
+    case FP8GMM_MLP_BACKWARD: rc = mlp_backward(static_cast<const fp8gmm_mlp_pass*>(desc), routed, pass); break;
     default: break;
   }
   if (rc != FP8GMM_OK) return rc;
   memset(out, 0, sizeof(*out));
   return lay_out_pass(pass, out, static_cast<PassTables*>(tables));
+}
+
+int fp8gmm_lay_out_pass(int which, const void* desc, fp8gmm_pass_plan* out, void* tables) {
+  return fp8gmm_lay_out_routed_pass(which, desc, nullptr, out, tables);
 }
 
 int fp8gmm_build_pass(const void* tables, void* blob_dev, const fp8gmm_scaling_update* updates, int n_updates,
@@ -659,6 +695,11 @@ int fp8gmm_build_pass(const void* tables, void* blob_dev, const fp8gmm_scaling_u
 
 int fp8gmm_run_planned(const void* blob_dev, const fp8gmm_pass_launch* rec, void* workspace, size_t workspace_bytes,
                        void* stream) {
+  return fp8gmm_run_routed(blob_dev, rec, nullptr, 0, workspace, workspace_bytes, stream);
+}
+
+int fp8gmm_run_routed(const void* blob_dev, const fp8gmm_pass_launch* rec, const fp8gmm_routed_rows* routed, int64_t rows,
+                      void* workspace, size_t workspace_bytes, void* stream) {
   if (rec == nullptr) return FP8GMM_ERR_NULL_POINTER;
   if (rec->kind == FP8GMM_PASS_NOTHING) return FP8GMM_OK;
   if (blob_dev == nullptr) return FP8GMM_ERR_NULL_POINTER;
@@ -674,6 +715,10 @@ int fp8gmm_run_planned(const void* blob_dev, const fp8gmm_pass_launch* rec, void
         if (rec->merge_n != 0)
           return fp8gmm::launch_cast_unmerged(descs, rec->n, rec->total_blocks, rec->out_fmt, true, stream);
         return fp8gmm_multi_cast_dgelu(descs, rec->n, rec->total_blocks, rec->out_fmt, stream);
+      case FP8GMM_OP_ROUTED_CAST:
+      case FP8GMM_OP_ROUTED_GRADIENT:
+        if (routed == nullptr) return FP8GMM_ERR_NULL_POINTER;
+        return fp8gmm::launch_routed_cast(descs, rec->n, rec->op, rec->out_fmt, *routed, rows, rec->merge_n == 0, stream);
       default: return FP8GMM_ERR_BAD_ARGUMENT;
     }
   }

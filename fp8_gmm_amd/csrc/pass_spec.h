@@ -23,7 +23,7 @@ struct CastRun {
   int64_t cols;
   int64_t numel;
   int32_t slot_stride;
-  int32_t reserved;
+  int32_t routed;         // FP8GMM_OP_ROUTED_*: `in` are tokens, an expert's rows begin with rows_padded
 };
 
 struct CastSpec {
@@ -98,13 +98,21 @@ FP8GMM_HD void* offset_ptr(void* base, int64_t bytes) {
 // descriptor of expert i of a run (block_begin is the caller's)
 FP8GMM_HD fp8gmm_tensor_desc cast_desc(const CastRun& s, int i, int64_t row_begin, int64_t rows) {
   fp8gmm_tensor_desc d{};
+  d.scale = s.scale + (int64_t)i * s.slot_stride;
+  d.amax = s.amax + (int64_t)i * s.slot_stride;
+  if (s.routed) {
+    d.in = s.in;
+    d.out = offset_ptr(s.out, row_begin * s.cols);
+    d.rows = (int32_t)rows;
+    d.cols = (int32_t)s.cols;
+    d.rows_padded = (int32_t)row_begin;
+    return d;
+  }
   const int64_t numel = s.cols > 0 ? rows * s.cols : s.numel;
   const int64_t first = s.cols > 0 ? row_begin * s.cols : (int64_t)i * s.numel;
   d.in = offset_ptr(s.in, first * 2);
   d.in2 = offset_ptr(s.in2, first * 2);
   d.out = offset_ptr(s.out, first);
-  d.scale = s.scale + (int64_t)i * s.slot_stride;
-  d.amax = s.amax + (int64_t)i * s.slot_stride;
   d.rows = numel > 0;
   d.cols = (int32_t)numel;
   return d;

@@ -16,7 +16,11 @@
 // which a single-wavefront workgroup walks its chunk in order; a short list takes the three steps in one workgroup of
 // one launch.  The row movers are HBM-bound: one wavefront per
 // row, 16 bytes per lane per access.
+#include <type_traits>
+
 #include "device_utils.h"
+#include "internal.h"
+#include "pass_spec.h"
 
 namespace fp8gmm {
 namespace {
@@ -471,6 +475,146 @@ __global__ __launch_bounds__(kRowWaves * 64) void moe_scatter_backward_kernel(co
   if (lane == 0 && ok) grad_w[idx] = acc;
 }
 
+// The cast of routed rows (fp8gmm_routed_rows).  A wavefront takes choices side by side, (token, choice) after (token, choice):
+// the token's row, which it keeps for the token's other choices, is cast into the rows of the expert that the choice is for,
+// with that expert's scale.  GRADIENT: the row is weighted and rounded to bf16 first, and its product with the row of `y` at the
+// same place is the gradient of the weight.
+// Which expert a place belongs to follows from the descriptors (rows_padded: the first of its rows); a lane looks that up for
+// one choice, for all of a wavefront's at once.  Maxima meet in LDS and go to the descriptors once per workgroup.
+// Bound: HBM.  Against a launch that moves the rows and one that casts them, 16384 tokens of 4096 columns, two choices each of
+// 16 experts: 155 -> 64 us (268 MB; forward), 197 -> 98 (537 MB; gradient); the layer's step 5439 -> 5223 (with the casts of
+// `amax_or_nan`).  3062 rows of 1024: 12 -> 10 and 13 -> 14, a launch less each.
+constexpr int kRoutedWaves = 8;
+constexpr int kRoutedLoads = 8, kRoutedChunk = kRoutedLoads * 64 * 8;   // 16-byte loads of a row under way per lane
+template <int FMT, bool GRADIENT>
+__global__ __launch_bounds__(kRoutedWaves * 64) void routed_cast_kernel(fp8gmm_tensor_desc* __restrict__ descs, int n,
+                                                                        const fp8gmm_routed_rows routed, int rows,
+                                                                        int per_wave) {
+  __shared__ int begin[kPassMaxExperts];
+  __shared__ float scales[kPassMaxExperts];
+  __shared__ uint32_t maxima[kPassMaxExperts];   // of values that are not negative: their bits are in their order
+  const int lane = threadIdx.x % 64, top_k = routed.top_k;
+  const int first = (blockIdx.x * kRoutedWaves + __builtin_amdgcn_readfirstlane(threadIdx.x / 64)) * per_wave;
+  const int count = rows - first < per_wave ? rows - first : per_wave;   // may be negative
+  // lane i: choice first + i
+  int place = 0, expert = 0;
+  float weight = 1.f;
+  if (lane < count) {
+    place = routed.inverse[first + lane];
+    if constexpr (GRADIENT) weight = routed.weights[first + lane];
+  }
+  for (int e = threadIdx.x; e < n; e += kRoutedWaves * 64) {
+    begin[e] = descs[e].rows_padded;
+    scales[e] = descs[e].scale != nullptr ? *descs[e].scale : 1.f;
+    maxima[e] = 0;
+  }
+  const int hidden = descs[0].cols;
+  const uint16_t* const in = static_cast<const uint16_t*>(descs[0].in);
+  uint8_t* const out = static_cast<uint8_t*>(descs[0].out);   // of the first expert: all rows
+  u32x4 v[kRoutedLoads];   // of a token's row, all of it as long as it is not longer: asked for ahead of what it waits for
+  auto fetch = [&](u32x4 (&to)[kRoutedLoads], const __amdgpu_buffer_rsrc_t& from, int c0) {
+#pragma unroll
+    for (int u = 0; u < kRoutedLoads; ++u)
+      if (c0 + u * 64 * 8 < hidden) to[u] = buf_load16_stream(from, (uint32_t)(c0 + (u * 64 + lane) * 8) * 2u);
+  };
+  auto row_of_token = [&](int t) { return make_rsrc(in + (size_t)t * hidden, (uint32_t)hidden * 2u); };
+  int t = first / top_k, k = first - t * top_k;
+  if (count > 0) fetch(v, row_of_token(t), 0);
+  __syncthreads();
+  int hi = n - 1;
+  while (expert < hi) {   // the last expert whose rows begin at or in front of the place: those without rows lie in front
+    const int mid = (expert + hi + 1) >> 1;
+    if (begin[mid] <= place) expert = mid; else hi = mid - 1;
+  }
+  const float scale = scales[expert];
+  const bool dot = GRADIENT && routed.grad_weights != nullptr;
+#pragma unroll 1
+  for (int own = 0; own < count; ++own) {
+    const int row = __builtin_amdgcn_readlane(place, own);
+    const float sc = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(scale), own));
+    const float w = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(weight), own));
+    const bool ok = (uint32_t)row < (uint32_t)rows;   // no place: nothing is read or stored
+    const bool kept = own > 0 && k > 0;                // the token's row, where it is not longer than a chunk
+    const __amdgpu_buffer_rsrc_t rs = row_of_token(t);
+    const __amdgpu_buffer_rsrc_t rd = make_rsrc(out + (ok ? (size_t)row * hidden : 0), ok ? (uint32_t)hidden : 0u);
+    const __amdgpu_buffer_rsrc_t ry = make_rsrc(static_cast<const uint16_t*>(routed.y) + (dot && ok ? (size_t)row * hidden : 0),
+                                                dot && ok ? (uint32_t)hidden * 2u : 0u);
+    float acc = 0.f, mx = 0.f;
+#pragma unroll 1
+    for (int c0 = 0; c0 < hidden; c0 += kRoutedChunk) {
+      u32x4 vy[GRADIENT ? kRoutedLoads : 1];
+      if (c0 > 0 || (kept && hidden > kRoutedChunk)) fetch(v, rs, c0);
+      if constexpr (GRADIENT) {
+        fetch(vy, ry, c0);
+#pragma unroll
+        for (int u = 0; u < kRoutedLoads; ++u) {
+          if (c0 + u * 64 * 8 >= hidden) break;
+          const uint32_t p[4] = {v[u].x, v[u].y, v[u].z, v[u].w}, py[4] = {vy[u].x, vy[u].y, vy[u].z, vy[u].w};
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            acc = __builtin_fmaf(bf16_lo_to_f32(py[q]), bf16_lo_to_f32(p[q]), acc);
+            acc = __builtin_fmaf(bf16_hi_to_f32(py[q]), bf16_hi_to_f32(p[q]), acc);
+          }
+        }
+      }
+      float most = 0.f;   // of this chunk
+      auto take = [&](auto numbers) {
+#pragma unroll
+        for (int u = 0; u < kRoutedLoads; ++u) {
+          if (c0 + u * 64 * 8 >= hidden) break;
+          uint32_t p[4] = {v[u].x, v[u].y, v[u].z, v[u].w}, o[2];
+          if constexpr (GRADIENT)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) p[q] = scale_bf16x2(p[q], w);
+#pragma unroll
+          for (int q = 0; q < 2; ++q) {
+            const float x0 = bf16_lo_to_f32(p[2 * q]), x1 = bf16_hi_to_f32(p[2 * q]);
+            const float x2 = bf16_lo_to_f32(p[2 * q + 1]), x3 = bf16_hi_to_f32(p[2 * q + 1]);
+            if constexpr (decltype(numbers)::value) {
+              most = amax_or_nan(amax_or_nan(most, x0, x1), x2, x3);
+              o[q] = cvt4_fp8_numbers<FMT>(x0 * sc, x1 * sc, x2 * sc, x3 * sc);
+            } else {
+              most = amax_step(amax_step(most, x0), x1);
+              most = amax_step(amax_step(most, x2), x3);
+              o[q] = cvt4_fp8<FMT>(x0 * sc, x1 * sc, x2 * sc, x3 * sc);
+            }
+          }
+          buf_store8(u32x2{o[0], o[1]}, rd, (uint32_t)(c0 + (u * 64 + lane) * 8));
+          __builtin_amdgcn_sched_barrier(0);   // pieces side by side would take more registers
+        }
+      };
+      take(std::true_type{});
+      if (__builtin_expect(!keeps_numbers(sc) || most != most, 0)) {
+        most = 0.f;
+        fetch(v, rs, c0);
+        take(std::false_type{});
+      }
+      mx = fmaxf(mx, most);
+    }
+    if (++k == top_k) {
+      k = 0;
+      ++t;
+      if (own + 1 < count) fetch(v, row_of_token(t), 0);
+    }
+    mx = wave_max(mx);
+    if (lane == 0) atomicMax(&maxima[__builtin_amdgcn_readlane(expert, own)], __float_as_uint(mx));
+    if constexpr (GRADIENT) {
+      if (dot) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+        if (lane == 0) routed.grad_weights[first + own] = acc;
+      }
+    }
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < n; e += kRoutedWaves * 64) {
+    // amax only grows, so a value already at or above this one (even a stale one) makes the atomic redundant
+    float* const slot = reinterpret_cast<float*>(&descs[e].amax_partial);
+    const float m = __uint_as_float(maxima[e]);
+    if (m > 0.f && descs[e].amax != nullptr && !(__builtin_nontemporal_load(slot) >= m)) atomic_max_nonneg(slot, m);
+  }
+}
+
 constexpr int kTopKMax = 8;  // choices per token that the selection keeps in registers
 
 template <bool BF16>
@@ -576,6 +720,36 @@ bool rows_vectorisable(const void* a, const void* b, int hidden) {
 }
 
 }  // namespace
+
+int launch_routed_cast(fp8gmm_tensor_desc* descs_dev, int n, int op, int out_fmt, const fp8gmm_routed_rows& routed, int64_t rows,
+                       bool merge, void* stream) {
+  if (n < 0 || n > kPassMaxExperts || rows < 0 || rows > INT32_MAX - 65536) return FP8GMM_ERR_BAD_ARGUMENT;
+  if (out_fmt != FP8GMM_E4M3 && out_fmt != FP8GMM_E5M2) return FP8GMM_ERR_BAD_FORMAT;
+  if (n == 0 || rows == 0) return FP8GMM_OK;
+  const bool gradient = op == FP8GMM_OP_ROUTED_GRADIENT;
+  if (descs_dev == nullptr || routed.inverse == nullptr || (gradient && routed.weights == nullptr) ||
+      (gradient && routed.grad_weights != nullptr && routed.y == nullptr))
+    return FP8GMM_ERR_NULL_POINTER;
+  if (routed.top_k < 1 || routed.top_k > FP8GMM_ROUTED_MAX_TOP_K || rows % routed.top_k != 0) return FP8GMM_ERR_BAD_ARGUMENT;
+  // One choice a wavefront while that leaves fewer than a thousand workgroups, then whole tokens: a token's row is read once,
+  // and an expert's maximum looked at by fewer workgroups.
+  int per_wave = (int)(rows / (kRoutedWaves * 1024)) / routed.top_k * routed.top_k;
+  per_wave = per_wave < 1 ? 1 : per_wave > 64 / routed.top_k * routed.top_k ? 64 / routed.top_k * routed.top_k : per_wave;
+  const int per_block = kRoutedWaves * per_wave;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const dim3 grid((unsigned)((rows + per_block - 1) / per_block)), block(kRoutedWaves * 64);
+  if (gradient && out_fmt == FP8GMM_E4M3)
+    hipLaunchKernelGGL((routed_cast_kernel<FP8GMM_E4M3, true>), grid, block, 0, s, descs_dev, n, routed, (int)rows, per_wave);
+  else if (gradient)
+    hipLaunchKernelGGL((routed_cast_kernel<FP8GMM_E5M2, true>), grid, block, 0, s, descs_dev, n, routed, (int)rows, per_wave);
+  else if (out_fmt == FP8GMM_E4M3)
+    hipLaunchKernelGGL((routed_cast_kernel<FP8GMM_E4M3, false>), grid, block, 0, s, descs_dev, n, routed, (int)rows, per_wave);
+  else
+    hipLaunchKernelGGL((routed_cast_kernel<FP8GMM_E5M2, false>), grid, block, 0, s, descs_dev, n, routed, (int)rows, per_wave);
+  if (merge) hipLaunchKernelGGL(amax_merge_kernel, dim3((n + 255) / 256), dim3(256), 0, s, descs_dev, n);
+  return hipGetLastError() == hipSuccess ? FP8GMM_OK : FP8GMM_ERR_LAUNCH;
+}
+
 }  // namespace fp8gmm
 
 extern "C" {

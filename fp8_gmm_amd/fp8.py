@@ -306,6 +306,16 @@ class Fp8GroupedModuleBase(torch.nn.Module):
                 return False
         return float(meta["recipe"].margin) == int(meta["recipe"].margin)
 
+    def _takes_route(self, cls, input, *weights):
+        """Whether a call of this module may be replaced by a pass that fetches its rows from tokens or hands them back as
+        tokens (``_routed``): the class's own forward, with nothing hooked to it, on the native host path.  To be asked behind
+        ``cast_weights_ahead``, which prepares the scaling state."""
+        return (type(self).forward is cls.forward and "forward" not in self.__dict__ and "recipe" in self.fp8_meta
+                and not (self._forward_hooks or self._forward_pre_hooks or self._backward_hooks or self._backward_pre_hooks)
+                and not torch.nn.modules.module._has_any_global_hook()
+                and all(type(w) is torch.nn.Parameter for w in weights)
+                and type(input) in (torch.Tensor, torch.nn.Parameter) and self._native(input, *weights))
+
     def _native_setup(self, device):
         """The module's scaling state and the launch policy in force, as the native host path takes them."""
         from . import _lib, backend
@@ -330,13 +340,14 @@ class Fp8GroupedModuleBase(torch.nn.Module):
         r = meta["recipe"]
         return Due(meta["fp8_max_fwd"], meta["fp8_max_bwd"], int(r.margin), r.amax_compute_algo != "max", due[0])
 
-    def _native_pass(self, step, input, weights, group_sizes, caches, refresh, setup, due):
+    def _native_pass(self, step, input, weights, group_sizes, caches, refresh, setup, due, route=None):
         """A pass of the native host path, ``step``, behind the scaling update that ``_prepare`` found due, with the fp8
-        weights of ``caches`` (None: temporaries).  A refused pass leaves the scaling state as the other paths do: updated."""
+        weights of ``caches`` (None: temporaries).  ``route``: where its rows come from and go to.  A refused pass leaves the
+        scaling state as the other paths do: updated."""
         native_due = self._native_due(due)
         try:
             held = [None] * len(weights) if caches is None else [c.take(w, setup, refresh) for c, w in zip(caches, weights)]
-            out = step(input, *weights, group_sizes, *held, refresh, setup, native_due)
+            out = step(input, *weights, group_sizes, *held, refresh, setup, native_due, route)
         except BaseException:
             if native_due.due:
                 self._run_update(due)

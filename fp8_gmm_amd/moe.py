@@ -13,6 +13,12 @@ import torch
 from . import moe_ops
 from .grouped_linear import GroupedLinear
 from .grouped_mlp import GroupedMlp
+from .native import Route
+
+
+def _own(module, cls):
+    """Whether what a routed layer calls its experts with is the class's own."""
+    return type(module).experts is cls.experts and "experts" not in module.__dict__
 
 
 class _RoutedModule(torch.nn.Module):
@@ -33,8 +39,19 @@ class _RoutedModule(torch.nn.Module):
     def start_experts(self):
         """Enqueue what the experts' pass can do before the host knows the split (nothing, by default)."""
 
+    def experts_on_routed_rows(self, x, batch_sizes, indices, inverse, weights, top_k):
+        """``scatter(experts(gather(x)))`` in passes that fetch the rows and hand them back themselves; None where the experts
+        are called as they are."""
+        return None
+
     def compute(self, x, tokens_per_expert, indices, bin_ids, expert_weights, bins, top_k, inverse=None):
+        return self._compute(x, tokens_per_expert, indices, bin_ids, expert_weights, bins, top_k, inverse, False)
+
+    def _compute(self, x, tokens_per_expert, indices, bin_ids, expert_weights, bins, top_k, inverse, sorted_here):
         x = x.view(-1, x.size(-1))
+        # Rows that the experts' own casts can fetch are not gathered: the mover would write bf16 rows that the cast reads.  Of
+        # lists that are surely a permutation and its inverse.
+        routed = sorted_here and moe_ops.routed_rows_fit(x, indices, inverse, expert_weights, top_k)
         # The host needs the split to plan the expert launches.  Its copy is enqueued ahead of the gather and of the
         # experts' weight casts, which need nothing from the host: the GPU has that work to do while the host waits
         # for the counts and plans the launches.
@@ -43,10 +60,16 @@ class _RoutedModule(torch.nn.Module):
             self._counts_ready = torch.cuda.Event()
         self._counts_host.copy_(tokens_per_expert, non_blocking=True)
         self._counts_ready.record()
-        x = moe_ops.gather(x, indices, bin_ids, bins, top_k, inverse)
+        if not routed:
+            x = moe_ops.gather(x, indices, bin_ids, bins, top_k, inverse)
         self.start_experts()
         self._counts_ready.synchronize()
         batch_sizes = self._counts_host.to(torch.long, copy=True)   # the page-locked buffer is reused by the next step
+        if routed:
+            out = self.experts_on_routed_rows(x, batch_sizes, indices, inverse, expert_weights, top_k)
+            if out is not None:
+                return out
+            x = moe_ops.gather(x, indices, bin_ids, bins, top_k, inverse)
         out = self.experts(x, batch_sizes)
         return moe_ops.scatter(out, indices, bin_ids, expert_weights, bins, top_k, inverse)
 
@@ -62,8 +85,9 @@ class _RoutedModule(torch.nn.Module):
         with torch.no_grad():
             indices, bin_ids, bins, tokens_per_expert, inverse = moe_ops.indices_bins_and_inverse(
                 top_experts, self.n_experts)
-        more = (inverse,) if own else ()
-        return self.compute(input, tokens_per_expert, indices, bin_ids, expert_weights, bins, self.top_k, *more)
+        if own:
+            return self._compute(input, tokens_per_expert, indices, bin_ids, expert_weights, bins, self.top_k, inverse, True)
+        return self.compute(input, tokens_per_expert, indices, bin_ids, expert_weights, bins, self.top_k)
 
 
 class Fp8LinearModule(_RoutedModule):
@@ -82,6 +106,16 @@ class Fp8LinearModule(_RoutedModule):
     def experts(self, x, batch_sizes):
         return self.grouped_linear2(self.act(self.grouped_linear1(x, batch_sizes)), batch_sizes)
 
+    def experts_on_routed_rows(self, x, batch_sizes, indices, inverse, weights, top_k):
+        first, second = self.grouped_linear1, self.grouped_linear2
+        if not _own(self, Fp8LinearModule) or type(first) is not GroupedLinear or type(second) is not GroupedLinear \
+                or not first._takes_routed_rows(x):
+            return None
+        rows = self.act(first._routed(x, batch_sizes, Route(indices, inverse, None, top_k, True, False)))
+        if second._takes_routed_rows(rows):
+            return second._routed(rows, batch_sizes, Route(indices, inverse, weights, top_k, False, True))
+        return moe_ops.scatter(second(rows, batch_sizes), indices, None, weights, None, top_k, inverse)
+
 
 class Fp8MlpModule(_RoutedModule):
     """One ``GroupedMlp`` (tanh-GELU fused into the first GEMM) as the experts (fp8_gmm/example.py:106-130)."""
@@ -95,3 +129,9 @@ class Fp8MlpModule(_RoutedModule):
 
     def experts(self, x, batch_sizes):
         return self.grouped_mlp(x, batch_sizes)
+
+    def experts_on_routed_rows(self, x, batch_sizes, indices, inverse, weights, top_k):
+        mlp = self.grouped_mlp
+        if not _own(self, Fp8MlpModule) or type(mlp) is not GroupedMlp or not mlp._takes_routed_rows(x):
+            return None
+        return mlp._routed(x, batch_sizes, Route(indices, inverse, weights, top_k, True, True))

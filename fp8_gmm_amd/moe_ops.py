@@ -352,6 +352,25 @@ class _Scatter(torch.autograd.Function):
         return grad_x, None, grad_w, None, None
 
 
+def routed_rows_fit(x, indices, inverse, weights, top_k):
+    """Whether the experts' casts can fetch and weigh the rows themselves (fp8gmm_routed_rows) in place of ``gather`` and
+    ``scatter`` around them: tensors as those two make them, nothing that looks at the launches or at the autograd functions
+    one by one."""
+    from .backend import kernel_timing
+
+    def plain(t, dtype, dim):
+        return type(t) is torch.Tensor and t.dtype == dtype and t.dim() == dim and t.is_contiguous() and t.device == x.device
+
+    rows = x.shape[0] * top_k if x.dim() == 2 else -1
+    return (x.is_cuda and type(x) in (torch.Tensor, torch.nn.Parameter) and x.dtype == torch.bfloat16 and x.dim() == 2
+            and x.is_contiguous() and x.data_ptr() % 16 == 0 and x.shape[1] % 16 == 0
+            and plain(indices, torch.int32, 1) and plain(inverse, torch.int32, 1) and plain(weights, torch.float32, 1)
+            and indices.numel() == inverse.numel() == weights.numel() == rows and 1 <= top_k <= _lib.ROUTED_MAX_TOP_K
+            and kernel_timing._active is None
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and torch._C._autograd._top_saved_tensors_default_hooks(True) is None)
+
+
 def gather(x, indices, bin_ids, bins, top_k, inverse=None):
     """Rows of ``x[tokens, hidden]`` into expert order: ``out[i] = x[indices[i] // top_k]``, ``[tokens * top_k,
     hidden]`` (``megablocks.ops.gather``; ``bin_ids`` and ``bins`` are accepted for that signature and unused).

@@ -101,6 +101,9 @@ typedef struct fp8gmm_tensor_desc {
 #define FP8GMM_OP_PAD_CAST_TRANSPOSE 3
 #define FP8GMM_OP_PAD_CAST_TRANSPOSE_DGELU 4
 #define FP8GMM_OP_CAST_DGELU 5
+/* launches of routed passes only (fp8gmm_lay_out_routed_pass) */
+#define FP8GMM_OP_ROUTED_CAST 6
+#define FP8GMM_OP_ROUTED_GRADIENT 7
 
 /*
  * One GEMM of a grouped launch:  c[m, n] = epilogue( a[m, k] . b[n, k]^T ).
@@ -547,6 +550,31 @@ int fp8gmm_delayed_scaling_updates(const fp8gmm_scaling_update* updates, int n, 
 int fp8gmm_lay_out_pass(int which, const void* pass, fp8gmm_pass_plan* out, void* tables);
 int fp8gmm_build_pass(const void* tables, void* blob_dev, const fp8gmm_scaling_update* updates, int n_updates,
                       const float* copy_src, float* copy_dst, int copy_n, void* stream);
+
+/*
+ * A pass whose rows come from, or go back to, tokens: what gather and scatter of a routed layer (fp8_gmm/example.py:52,59,
+ * 88,94,115,119) would write and the cast read again is formed inside the cast, which is a launch of its own
+ * (FP8GMM_OP_ROUTED_*).  `tokens` of the pass counts its rows.
+ * With `inverse` a permutation of the rows, choice k of token t being row inverse[t * top_k + k] of the pass:
+ *   forward : x is bf16 [tokens / top_k, columns]; the row is x[t]   (fp8gmm_moe_gather)
+ *   backward: dy is bf16 [tokens / top_k, columns]; the row is bf16(weights[t * top_k + k] * dy[t]), and
+ *             grad_weights[t * top_k + k] = < the row of y, dy[t] > unless grad_weights is NULL   (fp8gmm_moe_scatter_backward)
+ * The same bits as those calls in front of the cast.  All of it device memory; x, dy, y and the fp8 rows on 16 bytes.  Laid out
+ * as by fp8gmm_lay_out_pass; every launch of such a pass is run by fp8gmm_run_routed with the same `routed` and the pass's
+ * number of rows (fp8gmm_run_planned refuses the cast).
+ */
+#define FP8GMM_ROUTED_MAX_TOP_K 8
+typedef struct fp8gmm_routed_rows {
+  const int32_t* inverse;            /* [tokens] */
+  const float* weights;              /* backward: fp32 [tokens] */
+  const void* y;                     /* backward, with grad_weights: bf16 [tokens, columns], the rows that were scattered */
+  float* grad_weights;               /* backward: fp32 [tokens], or NULL */
+  int32_t top_k, reserved;
+} fp8gmm_routed_rows;                /* 40 bytes */
+int fp8gmm_lay_out_routed_pass(int which, const void* pass, const fp8gmm_routed_rows* routed, fp8gmm_pass_plan* out,
+                               void* tables);
+int fp8gmm_run_routed(const void* blob_dev, const fp8gmm_pass_launch* launch, const fp8gmm_routed_rows* routed, int64_t rows,
+                      void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * Page-locked host memory that the device can read (for fp8gmm_upload's source), allocated also while a stream is

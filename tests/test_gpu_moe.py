@@ -473,3 +473,106 @@ def test_gating_gradients_check_what_saved_tensor_hooks_return(dev):
         for kernels in (False, True):
             with pytest.raises(RuntimeError):
                 passes(kernels, other)
+
+
+def _layer_results(layer, state, x, dy, frozen, steps=2):
+    """Outputs, gradients and scaling state of a routed layer over some steps."""
+    from fp8_gmm_amd import DelayedScaling, fp8_autocast
+
+    layer.load_state_dict(state)
+    for name, p in layer.named_parameters():
+        p.requires_grad_(not any(f in name for f in frozen))
+        p.grad = None
+    results = []
+    for step in range(steps):
+        xs = (x * (1 + step)).detach().requires_grad_("x" not in frozen)
+        with fp8_autocast(fp8_recipe=DelayedScaling(amax_history_len=4)):
+            out = layer(xs)
+        results.append(out.detach().clone())
+        if out.requires_grad:
+            out.backward(dy)
+            results += [t.grad.clone() for t in [xs] + list(layer.parameters()) if t.grad is not None]
+            for p in layer.parameters():
+                p.grad = None
+    for m in layer.modules():
+        if "scaling_fwd" in getattr(m, "fp8_meta", {}):
+            results += [t.clone() for d in ("scaling_fwd", "scaling_bwd") for t in m.fp8_meta[d].state().values()]
+    return results
+
+
+@pytest.mark.parametrize("kind,tokens,hidden,inner,experts,top_k,frozen", [
+    ("mlp", 300, 256, 512, 8, 2, ()), ("mlp", 37, 2064, 48, 5, 3, ()), ("mlp", 1, 16, 16, 4, 1, ()),
+    ("mlp", 65, 4112, 160, 100, 2, ("gating", "x")), ("mlp", 64, 256, 256, 4, 2, ("grouped",)),
+    ("mlp", 64, 256, 256, 4, 2, ("grouped", "x")), ("mlp", 64, 256, 256, 4, 2, ("grouped", "x", "gating")),
+    ("linear", 301, 1024, 528, 16, 2, ()), ("linear", 5, 48, 2064, 3, 3, ("gating",)), ("linear", 0, 64, 64, 4, 2, ()),
+    ("linear", 130, 256, 128, 8, 2, ("grouped_linear1", "x")), ("cutlass", 77, 272, 528, 6, 2, ()),
+    ("mlp", 9000, 256, 64, 16, 2, ()), ("mlp", 3000, 64, 64, 300, 8, ()), ("linear", 40, 256, 64, 4, 2, ("nan",))])
+def test_routed_rows_give_the_bits_of_gather_and_scatter(dev, monkeypatch, kind, tokens, hidden, inner, experts, top_k, frozen):
+    """A layer whose experts' casts fetch and weigh their rows themselves against the same layer between moe_ops.gather and
+    moe_ops.scatter: outputs, every gradient and the scaling state, bit for bit."""
+    ops = _ops()
+    from fp8_gmm_amd.moe import Fp8LinearModule, Fp8MlpModule
+
+    torch.manual_seed(tokens + hidden)
+    layer = Fp8MlpModule(hidden, inner, experts, top_k) if kind == "mlp" else \
+        Fp8LinearModule(hidden, inner, experts, top_k, cutlass=kind == "cutlass")
+    twin = Fp8MlpModule(hidden, inner, experts, top_k) if kind == "mlp" else \
+        Fp8LinearModule(hidden, inner, experts, top_k, cutlass=kind == "cutlass")
+    state = layer.state_dict()
+    x = torch.randn(tokens, hidden, device=dev).to(torch.bfloat16)
+    dy = (torch.randn(tokens, hidden, device=dev) * 1e-2).to(torch.bfloat16)
+    if "nan" in frozen:
+        frozen = ()
+        x[3, 5], x[7, 200], dy[4, 255], dy[9, 0] = float("nan"), float("inf"), float("nan"), -float("inf")
+    calls = []
+    for name in ("gather", "scatter"):
+        monkeypatch.setattr(ops, name, lambda *a, _f=getattr(ops, name), _n=name, **k: (calls.append(_n), _f(*a, **k))[1])
+    got = _layer_results(layer, state, x, dy, frozen)
+    assert not calls
+    monkeypatch.setattr(ops, "routed_rows_fit", lambda *a: False)
+    want = _layer_results(twin, state, x, dy, frozen)
+    assert calls and len(got) == len(want)
+    for a, b in zip(got, want):
+        assert a.dtype == b.dtype and a.shape == b.shape
+        assert torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))
+
+
+def test_routed_rows_are_left_to_gather_where_something_looks_on(dev, monkeypatch):
+    """A hook on the experts, a replaced `experts`, saved-tensor hooks and an open block of kernel timing see what they saw."""
+    ops = _ops()
+    from fp8_gmm_amd import backend
+    from fp8_gmm_amd.moe import Fp8LinearModule, Fp8MlpModule
+
+    calls = []
+    gather = ops.gather
+    monkeypatch.setattr(ops, "gather", lambda *a, **k: (calls.append("gather"), gather(*a, **k))[1])
+    x = torch.randn(64, 256, device=dev).to(torch.bfloat16).requires_grad_()
+
+    def gathers(layer):
+        calls.clear()
+        layer(x).sum().backward()
+        return bool(calls)
+
+    layer = Fp8MlpModule(256, 128, 4, 2)
+    assert not gathers(layer)
+    seen = []
+    handle = layer.grouped_mlp.register_forward_hook(lambda m, i, o: seen.append(i[0].shape))
+    assert gathers(layer) and seen == [torch.Size([128, 256])]
+    handle.remove()
+    assert not gathers(layer)
+    layer.experts = lambda rows, sizes: layer.grouped_mlp(rows, sizes)
+    assert gathers(layer)
+    del layer.experts
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t.to(dev)):
+        assert gathers(layer)
+    with backend.kernel_timing():
+        assert gathers(layer)
+    two = Fp8LinearModule(256, 128, 4, 2)
+    two.grouped_linear2.register_forward_hook(lambda m, i, o: seen.append(o.shape))
+    assert not gathers(two) and seen[-1] == torch.Size([128, 256])   # the first layer fetches, the second is called
+
+    class Rows(Fp8MlpModule):
+        def experts(self, rows, sizes):
+            return super().experts(rows * 1, sizes)
+
+    assert gathers(Rows(256, 128, 4, 2))
