@@ -18,6 +18,8 @@
 
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/Event.h>
+#include <c10/core/impl/VirtualGuardImpl.h>
 #include <c10/hip/HIPStream.h>
 
 #include <atomic>
@@ -613,6 +615,180 @@ void cast_weights(const std::vector<Tensor>& weights, const std::vector<Tensor>&
   }
 }
 
+// ---- routing around the experts -----------------------------------------------------------------------------------
+// What moe_ops._Gating, _TopK and the sort do, without the interpreter: a short batch waits for its host, and a routed layer's
+// forward and backward pass through those took 250 of 600 us.
+
+// (x weight^T, x): the logits, and x once more for what follows, so that its two gradients meet here and one kernel adds them.
+struct GatingBackward : public Node {
+  int64_t hidden = 0;
+  SavedVariable x, weight;   // what torch's linear would keep: with a frozen weight the rows may be changed in place afterwards
+
+  std::string name() const override { return "GatingBackward"; }
+  void release_variables() override {
+    const std::lock_guard<std::mutex> lock(mutex_);
+    x.reset_data();
+    weight.reset_data();
+  }
+  variable_list apply(variable_list&& grads) override {
+    const std::lock_guard<std::mutex> lock(mutex_);
+    variable_list result(2);
+    const Tensor &grad = grads[0], &grad_in = grads[1];
+    if (!grad.defined()) {
+      result[0] = grad_in;
+      return result;
+    }
+    const c10::OptionalDeviceGuard guard(grad.device());
+    const bool want_x = task_should_compute_output(0), want_weight = task_should_compute_output(1);
+    const int64_t tokens = grad.size(0), experts = grad.size(1);
+    const Tensor rows = want_weight ? x.unpack() : Tensor(), w = want_x ? weight.unpack() : Tensor();
+    auto as_saved = [&](const Tensor& t, int64_t n) {
+      return t.scalar_type() == at::kBFloat16 && t.device() == grad.device() && t.dim() == 2 && t.size(0) == n && t.size(1) == hidden;
+    };
+    // a graph of the backward pass is asked for, or a saved-tensor hook returned what the kernels do not read: torch's products
+    if (at::GradMode::is_enabled() || (want_weight && !as_saved(rows, tokens)) || (want_x && !as_saved(w, experts))) {
+      if (want_x) result[0] = grad_in.defined() ? grad_in + grad.mm(w) : grad.mm(w);
+      if (want_weight) result[1] = grad.t().mm(rows);
+      return result;
+    }
+    if (kernel_timing.load(std::memory_order_relaxed)) {
+      py::gil_scoped_acquire gil;
+      auto or_none = [](const Tensor& t) { return t.defined() ? py::cast(t) : py::none(); };
+      const auto both = py::module_::import("fp8_gmm_amd.moe_ops")
+                            .attr("_gating_gradients")(grad, or_none(rows), or_none(w), or_none(grad_in))
+                            .cast<std::pair<std::optional<Tensor>, std::optional<Tensor>>>();
+      if (want_x) result[0] = *both.first;
+      if (want_weight) result[1] = *both.second;
+      return result;
+    }
+    const Tensor g = aligned(grad), in = grad_in.defined() ? aligned(grad_in) : Tensor();
+    const Tensor xs = want_weight ? aligned(rows) : Tensor(), ws = want_x ? w.contiguous() : Tensor();
+    if (want_x) result[0] = at::empty({tokens, hidden}, g.options());
+    Tensor work;
+    if (want_weight) {
+      result[1] = at::empty({experts, hidden}, g.options());
+      work = at::empty({(int64_t)fp8gmm_gating_workspace_bytes((int)tokens, (int)hidden, (int)experts)}, g.options().dtype(at::kByte));
+    }
+    check(fp8gmm_gating_backward(ptr<void>(g), ptr<void>(xs), ptr<void>(ws), ptr<void>(in), ptr<void>(result[0]),
+                                 ptr<void>(result[1]), (int)tokens, (int)hidden, (int)experts, ptr<void>(work),
+                                 current_stream(g.device())));
+    return result;
+  }
+};
+
+std::pair<Tensor, Tensor> gating(const Tensor& x, const Tensor& weight) {
+  py::gil_scoped_release no_gil;
+  TORCH_CHECK(x.dim() == 2 && weight.dim() == 2 && x.size(1) == weight.size(1) && x.scalar_type() == at::kBFloat16 &&
+                  weight.scalar_type() == at::kBFloat16 && x.is_contiguous() && weight.is_contiguous(),
+              "fp8_gmm_amd: rows and gate that do not fit together");
+  check_no_tangent({x, weight});
+  Tensor logits, rows;
+  {
+    at::AutoGradMode no_grad(false);
+    logits = at::linear(x, weight);
+    rows = x.detach();
+  }
+  auto node = std::shared_ptr<GatingBackward>(new GatingBackward(), torch::autograd::deleteNode);
+  node->set_next_edges(torch::autograd::collect_next_edges(x, weight));
+  node->hidden = x.size(1);
+  if (weight.requires_grad()) node->x = SavedVariable(x, false);
+  if (x.requires_grad()) node->weight = SavedVariable(weight, false);
+  torch::autograd::set_history(logits, node);
+  torch::autograd::set_history(rows, node);
+  return {logits, rows};
+}
+
+// The chain from the weights of the chosen experts back to the scores.
+struct RouteTopKBackward : public Node {
+  SavedVariable probs, selected;
+  int64_t tokens = 0, experts = 0, top_k = 0;
+  at::ScalarType type = at::kBFloat16;
+
+  std::string name() const override { return "RouteTopKBackward"; }
+  void release_variables() override {
+    const std::lock_guard<std::mutex> lock(mutex_);
+    probs.reset_data();
+    selected.reset_data();
+  }
+  variable_list apply(variable_list&& grads) override {
+    const std::lock_guard<std::mutex> lock(mutex_);
+    at::AutoGradMode no_grad(false);
+    const Tensor grad = gradient_of_result(*this, grads), p = probs.unpack(), s = selected.unpack();
+    TORCH_CHECK(p.scalar_type() == at::kFloat && p.numel() == tokens * experts && p.is_contiguous() && p.device() == grad.device() &&
+                    s.scalar_type() == at::kLong && s.numel() == tokens * top_k && s.is_contiguous() && s.device() == grad.device(),
+                "fp8_gmm_amd: a saved-tensor hook returned another tensor than was saved");
+    const c10::OptionalDeviceGuard guard(grad.device());
+    const Tensor result = at::empty({tokens, experts}, grad.options().dtype(type));
+    check(fp8gmm_route_topk_backward(ptr<float>(p), ptr<int64_t>(s), ptr<float>(grad), (int)tokens, (int)experts, (int)top_k,
+                                     ptr<void>(result), type == at::kBFloat16, current_stream(grad.device())));
+    return {result};
+  }
+};
+
+// Rows per expert on their way to the host.
+struct Counts {
+  Tensor host;   // page-locked
+  c10::Event event;
+  std::vector<int64_t> wait() {
+    event.synchronize();
+    const int32_t* p = host.const_data_ptr<int32_t>();
+    return std::vector<int64_t>(p, p + host.numel());
+  }
+};
+
+// The router's choice, the sort of its (token, choice) pairs by expert and the copy of the experts' row counts to the host:
+// (weights fp32 [tokens * top_k], indices, bin_ids, bins, tokens_per_expert, inverse, Counts).
+py::tuple route(const Tensor& scores, int64_t top_k) {
+  Tensor weights, indices, bin_ids, bins, counts, inverse;
+  std::unique_ptr<Counts> copy;
+  {
+    py::gil_scoped_release no_gil;
+    TORCH_CHECK(scores.is_cuda() && scores.dim() == 2 && scores.is_contiguous() &&
+                    (scores.scalar_type() == at::kBFloat16 || scores.scalar_type() == at::kFloat) &&
+                    scores.size(0) * top_k <= INT32_MAX,
+                "fp8_gmm_amd: scores that the routing kernels do not take");
+    check_no_tangent({scores});
+    const c10::OptionalDeviceGuard guard(scores.device());
+    const int64_t tokens = scores.size(0), experts = scores.size(1), rows = tokens * top_k;
+    const bool grad = at::GradMode::is_enabled() && scores.requires_grad();
+    void* const stream = current_stream(scores.device());
+    Tensor probs, selected;
+    {
+      at::AutoGradMode no_grad(false);
+      const auto ints = scores.options().dtype(at::kInt);
+      probs = at::empty({tokens, experts}, scores.options().dtype(at::kFloat));
+      weights = at::empty({rows}, probs.options());
+      selected = at::empty({tokens, top_k}, scores.options().dtype(at::kLong));
+      check(fp8gmm_route_topk(ptr<void>(scores), scores.scalar_type() == at::kBFloat16, (int)tokens, (int)experts, (int)top_k,
+                              ptr<float>(probs), ptr<float>(weights), ptr<int64_t>(selected), stream));
+      indices = at::empty({rows}, ints);
+      bin_ids = at::empty({rows}, ints);
+      inverse = at::empty({rows}, ints);
+      counts = at::empty({experts}, ints);
+      bins = at::empty({experts}, ints);
+      const Tensor work = at::empty({(int64_t)fp8gmm_route_workspace_bytes((int)rows, (int)experts)}, ints.dtype(at::kByte));
+      check(fp8gmm_route_sort_selected(ptr<int64_t>(selected), (int)rows, (int)experts, ptr<int32_t>(bin_ids), ptr<int32_t>(indices),
+                                       ptr<int32_t>(inverse), ptr<int32_t>(counts), ptr<int32_t>(bins), ptr<void>(work), stream));
+      copy.reset(new Counts{at::empty({experts}, at::TensorOptions().dtype(at::kInt).pinned_memory(true)),
+                            c10::Event(scores.device().type())});
+      copy->host.copy_(counts, /*non_blocking=*/true);
+      copy->event.record(c10::impl::VirtualGuardImpl(scores.device().type()).getStream(scores.device()));
+    }
+    if (grad) {
+      auto node = std::shared_ptr<RouteTopKBackward>(new RouteTopKBackward(), torch::autograd::deleteNode);
+      node->set_next_edges(torch::autograd::collect_next_edges(scores));
+      node->probs = SavedVariable(probs, false);
+      node->selected = SavedVariable(selected, false);
+      node->tokens = tokens;
+      node->experts = experts;
+      node->top_k = top_k;
+      node->type = scores.scalar_type();
+      torch::autograd::set_history(weights, node);
+    }
+  }
+  return py::make_tuple(weights, indices, bin_ids, bins, counts, inverse, std::move(copy));
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_host, m) {
@@ -652,5 +828,8 @@ PYBIND11_MODULE(_host, m) {
   m.def("mlp_step", &mlp_step, py::arg("x"), py::arg("w1"), py::arg("w2"), py::arg("group_sizes"), py::arg("cached1"),
         py::arg("cached2"), py::arg("cast_weights"), py::arg("setup"), py::arg("due"), py::arg("route") = nullptr);
   m.def("cast_weights", &cast_weights);
+  py::class_<Counts>(m, "Counts").def("wait", &Counts::wait, py::call_guard<py::gil_scoped_release>());
+  m.def("gating", &gating);
+  m.def("route", &route);
   m.def("set_kernel_timing", [](bool on) { kernel_timing.store(on, std::memory_order_relaxed); });
 }

@@ -13,7 +13,7 @@ import torch
 from . import moe_ops
 from .grouped_linear import GroupedLinear
 from .grouped_mlp import GroupedMlp
-from .native import Route
+from .native import Route, route
 
 
 def _own(module, cls):
@@ -47,7 +47,7 @@ class _RoutedModule(torch.nn.Module):
     def compute(self, x, tokens_per_expert, indices, bin_ids, expert_weights, bins, top_k, inverse=None):
         return self._compute(x, tokens_per_expert, indices, bin_ids, expert_weights, bins, top_k, inverse, False)
 
-    def _compute(self, x, tokens_per_expert, indices, bin_ids, expert_weights, bins, top_k, inverse, sorted_here):
+    def _compute(self, x, tokens_per_expert, indices, bin_ids, expert_weights, bins, top_k, inverse, sorted_here, counts=None):
         x = x.view(-1, x.size(-1))
         # Rows that the experts' own casts can fetch are not gathered: the mover would write bf16 rows that the cast reads.  Of
         # lists that are surely a permutation and its inverse.
@@ -55,16 +55,20 @@ class _RoutedModule(torch.nn.Module):
         # The host needs the split to plan the expert launches.  Its copy is enqueued ahead of the gather and of the
         # experts' weight casts, which need nothing from the host: the GPU has that work to do while the host waits
         # for the counts and plans the launches.
-        if self._counts_host is None or self._counts_host.numel() != tokens_per_expert.numel():
-            self._counts_host = torch.empty(tokens_per_expert.shape, dtype=tokens_per_expert.dtype, pin_memory=True)
-            self._counts_ready = torch.cuda.Event()
-        self._counts_host.copy_(tokens_per_expert, non_blocking=True)
-        self._counts_ready.record()
+        if counts is None:
+            if self._counts_host is None or self._counts_host.numel() != tokens_per_expert.numel():
+                self._counts_host = torch.empty(tokens_per_expert.shape, dtype=tokens_per_expert.dtype, pin_memory=True)
+                self._counts_ready = torch.cuda.Event()
+            self._counts_host.copy_(tokens_per_expert, non_blocking=True)
+            self._counts_ready.record()
         if not routed:
             x = moe_ops.gather(x, indices, bin_ids, bins, top_k, inverse)
         self.start_experts()
-        self._counts_ready.synchronize()
-        batch_sizes = self._counts_host.to(torch.long, copy=True)   # the page-locked buffer is reused by the next step
+        if counts is not None:   # on their way since the sort
+            batch_sizes = torch.tensor(counts.wait(), dtype=torch.long)
+        else:
+            self._counts_ready.synchronize()
+            batch_sizes = self._counts_host.to(torch.long, copy=True)   # the page-locked buffer is reused by the next step
         if routed:
             out = self.experts_on_routed_rows(x, batch_sizes, indices, inverse, expert_weights, top_k)
             if out is not None:
@@ -79,6 +83,9 @@ class _RoutedModule(torch.nn.Module):
         # place where nothing else needs them, and without the inverse.
         own = getattr(self.compute, "__func__", None) is _RoutedModule.compute
         routing_logits, input = moe_ops.gating(self.gating_network, input) if own else (self.gating_network(input), input)
+        if own and moe_ops.router_fits(routing_logits, self.top_k, self.n_experts):
+            expert_weights, indices, bin_ids, bins, tokens_per_expert, inverse, counts = route(routing_logits, self.top_k)
+            return self._compute(input, tokens_per_expert, indices, bin_ids, expert_weights, bins, self.top_k, inverse, True, counts)
         weights0, selected_experts = moe_ops.topk(routing_logits, self.top_k)
         expert_weights = weights0.flatten()
         top_experts = selected_experts.flatten()

@@ -18,7 +18,7 @@ are clamped into the range instead of being undefined.
 """
 import torch
 
-from . import _lib
+from . import _lib, native
 from .backend import _fail, _stream, _timed
 
 MAX_EXPERTS = 4096  # size of the on-chip expert table of the sort kernels
@@ -148,25 +148,42 @@ class _Gating(torch.autograd.Function):
             if want_weight:
                 grad_weight = grad.t() @ x
             return grad_x, grad_weight
-        grad = _aligned(grad)
-        x = _aligned(x) if want_weight else None
-        weight = weight.contiguous() if want_x else None
-        grad_in = _aligned(grad_in) if grad_in is not None else None
-        L = _lib.load()
-        grad_x = torch.empty(tokens, hidden, dtype=grad.dtype, device=dev) if want_x else None
-        grad_weight = work = None
-        if want_weight:
-            grad_weight = torch.empty(experts, hidden, dtype=grad.dtype, device=dev)
-            work = torch.empty(L.fp8gmm_gating_workspace_bytes(tokens, hidden, experts), dtype=torch.uint8, device=dev)
-        with torch.cuda.device(dev), _timed("gating_backward", lambda: 2 * tokens * hidden * (want_weight + 2 * want_x)):
-            rc = L.fp8gmm_gating_backward(grad.data_ptr(), x.data_ptr() if want_weight else None,
-                                          weight.data_ptr() if want_x else None,
-                                          grad_in.data_ptr() if grad_in is not None else None,
-                                          grad_x.data_ptr() if want_x else None,
-                                          grad_weight.data_ptr() if want_weight else None, tokens, hidden, experts,
-                                          work.data_ptr() if want_weight and work.numel() else None, _stream(dev))
-        _lib.check(rc)
-        return grad_x, grad_weight
+        return _gating_gradients(grad, x if want_weight else None, weight if want_x else None, grad_in)
+
+
+def _gating_gradients(grad, x, weight, grad_in):
+    """``(grad_x, grad_weight)``: the first where the weight is given, the second where the rows are."""
+    want_x, want_weight = weight is not None, x is not None
+    (tokens, experts), dev = grad.shape, grad.device
+    hidden = (x if want_weight else weight).shape[1]
+    grad = _aligned(grad)
+    x = _aligned(x) if want_weight else None
+    weight = weight.contiguous() if want_x else None
+    grad_in = _aligned(grad_in) if grad_in is not None else None
+    L = _lib.load()
+    grad_x = torch.empty(tokens, hidden, dtype=grad.dtype, device=dev) if want_x else None
+    grad_weight = work = None
+    if want_weight:
+        grad_weight = torch.empty(experts, hidden, dtype=grad.dtype, device=dev)
+        work = torch.empty(L.fp8gmm_gating_workspace_bytes(tokens, hidden, experts), dtype=torch.uint8, device=dev)
+    with torch.cuda.device(dev), _timed("gating_backward", lambda: 2 * tokens * hidden * (want_weight + 2 * want_x)):
+        rc = L.fp8gmm_gating_backward(grad.data_ptr(), x.data_ptr() if want_weight else None,
+                                      weight.data_ptr() if want_x else None,
+                                      grad_in.data_ptr() if grad_in is not None else None,
+                                      grad_x.data_ptr() if want_x else None,
+                                      grad_weight.data_ptr() if want_weight else None, tokens, hidden, experts,
+                                      work.data_ptr() if want_weight and work.numel() else None, _stream(dev))
+    _lib.check(rc)
+    return grad_x, grad_weight
+
+
+def _unwatched():
+    """Nothing that looks at the launches or at the autograd functions one by one: the native host path has nodes of its own."""
+    from .backend import kernel_timing
+
+    return (kernel_timing._active is None and torch._C._functorch.peek_interpreter_stack() is None
+            and torch._C._autograd._top_saved_tensors_default_hooks(True) is None and not torch.jit.is_tracing()
+            and not torch.compiler.is_compiling())
 
 
 def _plain_linear(module):
@@ -206,7 +223,7 @@ def gating(module, x):
     are not what the kernels take, the module is called."""
     if torch.is_grad_enabled() and x.requires_grad and _plain_linear(module) and not torch.is_autocast_enabled("cuda") \
             and not torch.jit.is_tracing() and _gating_takes(x, module.weight):
-        return _Gating.apply(x, module.weight)
+        return native.gating(x, module.weight) if _unwatched() else _Gating.apply(x, module.weight)
     return module(x), x
 
 
@@ -354,10 +371,7 @@ class _Scatter(torch.autograd.Function):
 
 def routed_rows_fit(x, indices, inverse, weights, top_k):
     """Whether the experts' casts can fetch and weigh the rows themselves (fp8gmm_routed_rows) in place of ``gather`` and
-    ``scatter`` around them: tensors as those two make them, nothing that looks at the launches or at the autograd functions
-    one by one."""
-    from .backend import kernel_timing
-
+    ``scatter`` around them: tensors as those two make them, nobody looking on."""
     def plain(t, dtype, dim):
         return type(t) is torch.Tensor and t.dtype == dtype and t.dim() == dim and t.is_contiguous() and t.device == x.device
 
@@ -366,9 +380,14 @@ def routed_rows_fit(x, indices, inverse, weights, top_k):
             and x.is_contiguous() and x.data_ptr() % 16 == 0 and x.shape[1] % 16 == 0
             and plain(indices, torch.int32, 1) and plain(inverse, torch.int32, 1) and plain(weights, torch.float32, 1)
             and indices.numel() == inverse.numel() == weights.numel() == rows and 1 <= top_k <= _lib.ROUTED_MAX_TOP_K
-            and kernel_timing._active is None
-            and torch._C._functorch.peek_interpreter_stack() is None
-            and torch._C._autograd._top_saved_tensors_default_hooks(True) is None)
+            and _unwatched())
+
+
+def router_fits(scores, top_k, experts):
+    """Whether ``native.route`` takes ``topk``, ``indices_bins_and_inverse`` and the copy of the counts in one call."""
+    return (type(scores) is torch.Tensor and scores.is_cuda and scores.dim() == 2 and scores.is_contiguous()
+            and scores.dtype in (torch.bfloat16, torch.float32) and scores.shape[1] == experts <= MAX_EXPERTS
+            and 1 <= top_k <= min(MAX_TOP_K, experts) and _unwatched())
 
 
 def gather(x, indices, bin_ids, bins, top_k, inverse=None):

@@ -576,3 +576,68 @@ def test_routed_rows_are_left_to_gather_where_something_looks_on(dev, monkeypatc
             return super().experts(rows * 1, sizes)
 
     assert gathers(Rows(256, 128, 4, 2))
+
+
+@pytest.mark.parametrize("tokens,experts,top_k,dtype", [(1, 1, 1, torch.float32), (1531, 16, 2, torch.bfloat16),
+                                                         (5000, 128, 8, torch.bfloat16), (33, 600, 3, torch.float32),
+                                                         (0, 4, 2, torch.bfloat16)])
+def test_native_routing_gives_the_bits_of_the_functions(dev, tokens, experts, top_k, dtype):
+    """native.route against topk, the sort and the counts one by one; the gradient of its weights against topk's."""
+    ops = _ops()
+    from fp8_gmm_amd import native
+
+    g = torch.Generator().manual_seed(tokens + experts)
+    scores = torch.randn(tokens, experts, generator=g).to(dtype).to(dev)
+    a, b = scores.clone().requires_grad_(), scores.clone().requires_grad_()
+    assert ops.router_fits(a, top_k, experts) is (type(a) is torch.Tensor)
+    weights, indices, bin_ids, bins, counts, inverse, posted = native.route(a, top_k)
+    want_weights, selected = ops.topk(b, top_k)
+    want = ops.indices_bins_and_inverse(selected.flatten(), experts)
+    for x, y in zip((indices, bin_ids, bins, counts, inverse), want):
+        assert x.dtype == y.dtype and torch.equal(x, y)
+    assert posted.wait() == counts.cpu().tolist()
+    assert torch.equal(weights, want_weights.flatten()) and weights.requires_grad
+    grad = torch.randn(tokens * top_k, generator=g).to(dev)
+    weights.backward(grad)
+    want_weights.flatten().backward(grad)
+    assert torch.equal(a.grad, b.grad) and a.grad.dtype == dtype
+    with torch.no_grad():
+        assert not native.route(a, top_k)[0].requires_grad
+
+
+def test_native_gating_differentiates_twice_and_is_timed(dev):
+    """A graph of the gating gradients is torch's own; a block of kernel timing that opens behind the forward pass sees the
+    backward launches, with the same bits."""
+    ops = _ops()
+    from fp8_gmm_amd import backend
+    from fp8_gmm_amd.moe import Fp8MlpModule
+
+    gate = torch.nn.Linear(256, 8, bias=False).to(torch.bfloat16).to(dev)
+    x = torch.randn(64, 256, device=dev).to(torch.bfloat16).requires_grad_()
+    logits, rows = ops.gating(gate, x)
+    assert logits.grad_fn.name() == rows.grad_fn.name() == "GatingBackward"
+    assert torch.equal(rows, x) and torch.equal(logits, torch.nn.functional.linear(x, gate.weight))
+    up = torch.randn(64, 8, device=dev).to(torch.bfloat16).requires_grad_()
+    (gx,) = torch.autograd.grad(logits, x, up, create_graph=True)
+    gw, gup = torch.autograd.grad(gx, (gate.weight, up), torch.ones_like(gx))
+    assert torch.equal(gx, up.detach() @ gate.weight)
+    assert torch.equal(gw, up.detach().t() @ torch.ones_like(gx)) and torch.equal(gup, torch.ones_like(gx) @ gate.weight.t())
+    logits, rows = ops.gating(gate, x)   # the rows' gradient alone
+    assert torch.equal(torch.autograd.grad(rows, x, torch.ones_like(x))[0], torch.ones_like(x))
+
+    layer = Fp8MlpModule(256, 128, 4, 2)
+    twin = Fp8MlpModule(256, 128, 4, 2)
+    twin.load_state_dict(layer.state_dict())
+    dy = torch.randn(64, 256, device=dev).to(torch.bfloat16)
+    grads = []
+    for module, timed in ((layer, False), (twin, True)):
+        x.grad = None
+        out = module(x)
+        if timed:
+            with backend.kernel_timing() as timing:
+                out.backward(dy)
+            assert {"routed_gradient", "grouped_gemm", "gating_backward"} <= set(timing.summary())
+        else:
+            out.backward(dy)
+        grads.append([x.grad.clone()] + [p.grad.clone() for p in module.parameters()])
+    assert all(torch.equal(a, b) for a, b in zip(*grads))
