@@ -1016,6 +1016,48 @@ def test_weight_gradient_with_a_transposed_gradient_copy_gives_the_same_bits(dev
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("stream_k", [False, True], ids=["whole", "shared"])
+@pytest.mark.parametrize("c_scale", [64.0, 0.0, float("inf"), float("nan")])
+def test_gelu_epilogue_of_ragged_tiles_with_nan_and_scales_that_are_no_numbers(dev, c_scale, stream_k):
+    """The staged form of the fused GELU leaves out the 32-row blocks that hold no row of the problem and looks for a NaN
+    once per block; the per-element form (a row pitch that is not a multiple of 16) does neither.  Experts whose last
+    tile ends around every block's edge, with a row or a column of NaN: same bytes, same amax, and nothing written behind
+    the rows."""
+    backend = _backend()
+    g = gen(977)
+    sizes = [1, 31, 32, 33, 97, 128, 129, 160, 161, 255, 256, 257, 0, 300]
+    m, e, k, n, extra = sum(sizes), len(sizes), 1024 if stream_k else 128, 272, 8
+    a = _q(randn_bf16((m, k), g), E4M3)
+    b = _q(randn_bf16((e, n, k), g), E4M3)
+    row = 0
+    for i, rows in enumerate(sizes):
+        if rows and i % 3 == 0:
+            a.view(torch.uint8)[row + rows - 1, 7] = 0x7F     # a row of NaN, in the last block with rows
+        elif rows and i % 3 == 1:
+            b.view(torch.uint8)[i, (37 * i) % n, 7] = 0x7F    # a column of NaN, also in what lies behind the rows
+        row += rows
+    b_wide = torch.zeros(e, n + extra, k, dtype=torch.uint8).view(E4M3)
+    b_wide.view(torch.uint8)[:, :n] = b.view(torch.uint8)
+    ones, scales = torch.ones(e, device=dev), torch.full((e,), c_scale, device=dev)
+
+    def run(weights, cols):
+        c = torch.full((m + 300, cols), 0x55, dtype=torch.uint8, device=dev).view(E4M3)
+        pre = torch.full((m + 300, cols), 7.0, dtype=torch.bfloat16, device=dev)
+        amax = torch.zeros(3 * e, device=dev)
+        with backend.gemm_options(tile="256", stream_k=stream_k):
+            backend.fp8_gmm(a.to(dev), weights.to(dev), torch.tensor(sizes), ones, ones, c[:m], E4M3, pre[:m], scales,
+                            [amax[3 * i:3 * i + 1] for i in range(e)], False, False)
+        assert (c.view(torch.uint8)[m:] == 0x55).all() and (pre[m:] == 7).all()
+        return c[:m, :n].view(torch.uint8).cpu(), pre[:m, :n].contiguous().view(torch.int16).cpu(), amax.cpu()
+
+    got, want = run(b, n), run(b_wide, n + extra)
+    assert_bytes_equal(got[0], want[0], "fp8 gelu output")
+    assert_bytes_equal(got[1], want[1], "pre-gelu output")
+    assert_scalar_bits_equal(got[2], want[2], "amax")
+    assert torch.isfinite(got[2]).all() and (got[0] == 0x7F).any()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("out_dtype", [E5M2, E4M3], ids=["e5m2", "e4m3"])
 @pytest.mark.parametrize("sizes,n,k,b_kn", [
     ([300, 0, 513, 90], 512, 256, True),     # whole tiles in n, ragged rows: the staged form, rows past m
