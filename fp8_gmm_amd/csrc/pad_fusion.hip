@@ -276,12 +276,22 @@ __global__ __launch_bounds__(kPtThreads) void multi_pad_kernel(fp8gmm_tensor_des
     block_amax_merge<kPtThreads / kWaveSize>(mx, d.amax != nullptr ? &descs[t].amax_partial : nullptr, stage);
 }
 
+// Large launches of the cast claim this much more LDS than the 16 KB of the tile, so that three workgroups share a compute unit
+// (3 x 52 KB of 160) where the registers would let four: bound by HBM, they gain nothing from more loads in flight, and fewer
+// tiles at a time keep fewer rows of the two outputs open.  Kernel alone, four against three workgroups: 8 tensors of up to
+// 8191 rows of 4096 (one draw) 149.6 / 142.6 us, 9568 tiles of 2048 columns 116.7 / 113.8, 8960 of 8192 109.5 / 106.3, 7680 of
+// 4000 110.0 / 105.5, 6300 of 6400 76.4 / 74.1, 17584 of 14336 210.0 / 204.0; two are as slow as four.  Below 6144 tiles a launch
+// is too short (3456 tiles 38.0 / 40.5), and with the dGELU it needs the wavefronts for its arithmetic (5504 tiles 92 / 97).
+constexpr int kApartTiles = 2 * kStreamTiles;
+constexpr size_t kApartLds = 36000;
+
 template <int OP>
 int launch_fmt(fp8gmm_tensor_desc* descs_dev, int n, int total_blocks, int out_fmt, hipStream_t s) {
+  const size_t apart = OP == OP_CAST && total_blocks >= kApartTiles ? kApartLds : 0;
   if (out_fmt == FP8GMM_E4M3)
-    hipLaunchKernelGGL((multi_pad_kernel<OP, FP8GMM_E4M3>), dim3(total_blocks), dim3(kPtThreads), 0, s, descs_dev, n);
+    hipLaunchKernelGGL((multi_pad_kernel<OP, FP8GMM_E4M3>), dim3(total_blocks), dim3(kPtThreads), apart, s, descs_dev, n);
   else
-    hipLaunchKernelGGL((multi_pad_kernel<OP, FP8GMM_E5M2>), dim3(total_blocks), dim3(kPtThreads), 0, s, descs_dev, n);
+    hipLaunchKernelGGL((multi_pad_kernel<OP, FP8GMM_E5M2>), dim3(total_blocks), dim3(kPtThreads), apart, s, descs_dev, n);
   if (OP != OP_TRANSPOSE) hipLaunchKernelGGL(amax_merge_kernel, dim3((n + 255) / 256), dim3(256), 0, s, descs_dev, n);
   return hipGetLastError() == hipSuccess ? FP8GMM_OK : FP8GMM_ERR_LAUNCH;
 }
