@@ -182,24 +182,29 @@ Tensor scatter_rows(const Tensor& rows, const Tensor& inverse, const Tensor& wei
 struct SavedRoute {
   bool gathers = false, scatters = false, want_weights = false;
   int64_t top_k = 1, rows = 0;
-  SavedVariable indices, inverse, weights, y;
+  struct Kept {
+    SavedVariable indices, inverse, weights, y;
+  };
+  std::unique_ptr<Kept> kept;   // of a routed pass only
   void save(const Route& r, const Tensor& rows_out, bool dgrad, bool want) {
     gathers = r.gathers;
     scatters = r.scatters;
     want_weights = want;
     top_k = r.top_k;
     rows = r.indices.numel();
+    kept = std::make_unique<Kept>();
     if (scatters) {
-      weights = SavedVariable(r.weights, false);
+      kept->weights = SavedVariable(r.weights, false);
       if (want) {
-        indices = SavedVariable(r.indices, false);
-        y = SavedVariable(rows_out, false);
+        kept->indices = SavedVariable(r.indices, false);
+        kept->y = SavedVariable(rows_out, false);
       }
     }
-    if (scatters || (gathers && dgrad)) inverse = SavedVariable(r.inverse, false);
+    if (scatters || (gathers && dgrad)) kept->inverse = SavedVariable(r.inverse, false);
   }
   void reset() {
-    for (SavedVariable* v : {&indices, &inverse, &weights, &y}) v->reset_data();
+    if (kept == nullptr) return;
+    for (SavedVariable* v : {&kept->indices, &kept->inverse, &kept->weights, &kept->y}) v->reset_data();
   }
   // The kernels follow addresses, and a saved-tensor hook may return anything.
   Tensor list(SavedVariable& v, at::ScalarType type, const at::Device& device) const {
@@ -218,10 +223,10 @@ struct RoutedGradient {
     if (!r.scatters) return;
     dy = aligned(grad);
     TORCH_CHECK(dy.size(0) * r.top_k == r.rows, "fp8_gmm_amd: a gradient of another size than the result");
-    inverse = r.list(r.inverse, at::kInt, dy.device());
-    weights = r.list(r.weights, at::kFloat, dy.device());
+    inverse = r.list(r.kept->inverse, at::kInt, dy.device());
+    weights = r.list(r.kept->weights, at::kFloat, dy.device());
     if (want_weights) {
-      y = r.y.unpack();
+      y = r.kept->y.unpack();
       TORCH_CHECK(y.scalar_type() == at::kBFloat16 && y.dim() == 2 && y.size(0) == r.rows && y.size(1) == dy.size(1) &&
                       y.device() == dy.device(),
                   "fp8_gmm_amd: a saved-tensor hook returned another tensor than was saved");
@@ -238,7 +243,7 @@ struct RoutedGradient {
   int64_t size(const SavedRoute& r) const { return r.scatters ? r.rows : dy.size(0); }
   // grad_weights alone: nothing upstream of the rows wants a gradient
   void weights_only(SavedRoute& r) const {
-    const Tensor indices = r.list(r.indices, at::kInt, dy.device());
+    const Tensor indices = r.list(r.kept->indices, at::kInt, dy.device());
     check(fp8gmm_moe_scatter_wgrad(ptr<const void>(y), ptr<const void>(dy), ptr<const int32_t>(indices), rows.grad_weights, (int)r.rows,
                                    (int)dy.size(1), (int)r.top_k, current_stream(dy.device())));
   }
@@ -342,7 +347,7 @@ struct GroupedLinearBackward : public Node {
     d.bwd_scale_inv = ptr<float>(setup.bwd_scale_inv);
     d.bwd_amax = ptr<float>(setup.bwd_amax);
     run_pass(FP8GMM_LINEAR_BACKWARD, &d, dy.device(), nullptr, nullptr, Tensor(), Tensor(), from.routed(route), rows);
-    if (dgrad) result[0] = route.gathers ? scatter_rows(dx, route.list(route.inverse, at::kInt, dx.device()), Tensor(), route.top_k) : dx;
+    if (dgrad) result[0] = route.gathers ? scatter_rows(dx, route.list(route.kept->inverse, at::kInt, dx.device()), Tensor(), route.top_k) : dx;
     return result;
   }
 };
@@ -486,7 +491,7 @@ struct GroupedMlpBackward : public Node {
     d.bwd_scale_inv = ptr<float>(setup.bwd_scale_inv);
     d.bwd_amax = ptr<float>(setup.bwd_amax);
     run_pass(FP8GMM_MLP_BACKWARD, &d, dy.device(), nullptr, nullptr, Tensor(), Tensor(), from.routed(route), tokens);
-    if (want_x) result[0] = route.gathers ? scatter_rows(dx, route.list(route.inverse, at::kInt, dx.device()), Tensor(), route.top_k) : dx;
+    if (want_x) result[0] = route.gathers ? scatter_rows(dx, route.list(route.kept->inverse, at::kInt, dx.device()), Tensor(), route.top_k) : dx;
     return result;
   }
 };

@@ -340,6 +340,15 @@ class Fp8GroupedModuleBase(torch.nn.Module):
         r = meta["recipe"]
         return Due(meta["fp8_max_fwd"], meta["fp8_max_bwd"], int(r.margin), r.amax_compute_algo != "max", due[0])
 
+    def _routed_pass(self, step, input, weights, group_sizes, num_gemms, route, two_roundings=False):
+        """The native pass of ``forward`` without ``is_first_microbatch`` on the rows of ``route``."""
+        refuse_tracing()
+        ahead = self._take_ahead(None)
+        due = self._prepare(input.device, None, num_gemms) if ahead is None else None
+        setup = self._native_setup(input.device)
+        setup.two_roundings = two_roundings
+        return self._native_pass(step, input, weights, group_sizes, ahead, ahead is None, setup, due, route)
+
     def _native_pass(self, step, input, weights, group_sizes, caches, refresh, setup, due, route=None):
         """A pass of the native host path, ``step``, behind the scaling update that ``_prepare`` found due, with the fp8
         weights of ``caches`` (None: temporaries).  ``route``: where its rows come from and go to.  A refused pass leaves the

@@ -364,17 +364,6 @@ class GroupedLinear(Fp8GroupedModuleBase):
         return self._cast_ahead([(self.weight_tensor, Fp8TensorType.kWeightGroup1)])
 
     def forward(self, input, group_sizes, is_first_microbatch=None):
-        return self._pass(input, group_sizes, is_first_microbatch, None)
-
-    def _takes_routed_rows(self, input):
-        return self._takes_route(GroupedLinear, input, self.weight_tensor)
-
-    def _routed(self, input, group_sizes, route):
-        """``forward`` on the rows of ``route`` (``native.Route``), where ``_takes_routed_rows``: one pass instead of
-        ``moe_ops.gather``, forward and ``moe_ops.scatter``, the same bits."""
-        return self._pass(input, group_sizes, None, route)
-
-    def _pass(self, input, group_sizes, is_first_microbatch, route):
         refuse_tracing()
         ahead = self._take_ahead(is_first_microbatch)
         due = None
@@ -390,7 +379,7 @@ class GroupedLinear(Fp8GroupedModuleBase):
         if self._native(input, weight):
             setup = self._native_setup(input.device)
             setup.two_roundings = bool(self.cutlass)
-            return self._native_pass(linear_step, input, (weight,), group_sizes, caches, refresh, setup, due, route)
+            return self._native_pass(linear_step, input, (weight,), group_sizes, caches, refresh, setup, due)
         self._run_update(due)
         grad = torch.is_grad_enabled()
         args = (input, weight, group_sizes, self.fp8_meta, grad, self.cutlass)
@@ -399,3 +388,11 @@ class GroupedLinear(Fp8GroupedModuleBase):
         if grad:
             return _GroupedLinear.apply(*args)
         return _GroupedLinear.forward(None, *args)
+
+    def _takes_routed_rows(self, input):
+        return self._takes_route(GroupedLinear, input, self.weight_tensor)
+
+    def _routed(self, input, group_sizes, route):
+        """``forward`` on the rows of ``route`` (``native.Route``), where ``_takes_routed_rows``: one pass instead of
+        ``moe_ops.gather``, forward and ``moe_ops.scatter``, the same bits."""
+        return self._routed_pass(linear_step, input, (self.weight_tensor,), group_sizes, self.num_groups, route, bool(self.cutlass))

@@ -448,18 +448,6 @@ class GroupedMlp(Fp8GroupedModuleBase):
         return self._cast_ahead([(self.fc1_weight, _T.kWeightGroup1), (self.fc2_weight, _T.kWeightGroup2)])
 
     def forward(self, input, group_sizes, has_tp=False, tp_group=None, is_first_microbatch=None):
-        return self._pass(input, group_sizes, has_tp, tp_group, is_first_microbatch, None)
-
-    def _takes_routed_rows(self, input):
-        return not self.fp8_meta["fused_dgelu"] and "capture" not in self.fp8_meta \
-            and self._takes_route(GroupedMlp, input, self.fc1_weight, self.fc2_weight)
-
-    def _routed(self, input, group_sizes, route):
-        """``forward`` on the rows of ``route`` (``native.Route``), where ``_takes_routed_rows``: one pass instead of
-        ``moe_ops.gather``, forward and ``moe_ops.scatter``, the same bits."""
-        return self._pass(input, group_sizes, False, None, None, route)
-
-    def _pass(self, input, group_sizes, has_tp, tp_group, is_first_microbatch, route):
         refuse_tracing()
         ahead = self._take_ahead(is_first_microbatch)
         due = None
@@ -474,7 +462,7 @@ class GroupedMlp(Fp8GroupedModuleBase):
         w1, w2 = self.fc1_weight, self.fc2_weight
         if not has_tp and not self.fp8_meta["fused_dgelu"] and "capture" not in self.fp8_meta and self._native(input, w1, w2):
             setup = self._native_setup(input.device)
-            return self._native_pass(mlp_step, input, (w1, w2), group_sizes, caches, refresh, setup, due, route)
+            return self._native_pass(mlp_step, input, (w1, w2), group_sizes, caches, refresh, setup, due)
         self._run_update(due)
         grad = torch.is_grad_enabled()
         args = (input, w1, w2, group_sizes, self.fp8_meta, grad, has_tp, tp_group)
@@ -483,3 +471,12 @@ class GroupedMlp(Fp8GroupedModuleBase):
         if grad:
             return _GroupedMlp.apply(*args)
         return _GroupedMlp.forward(None, *args)
+
+    def _takes_routed_rows(self, input):
+        return not self.fp8_meta["fused_dgelu"] and "capture" not in self.fp8_meta \
+            and self._takes_route(GroupedMlp, input, self.fc1_weight, self.fc2_weight)
+
+    def _routed(self, input, group_sizes, route):
+        """``forward`` on the rows of ``route`` (``native.Route``), where ``_takes_routed_rows``: one pass instead of
+        ``moe_ops.gather``, forward and ``moe_ops.scatter``, the same bits."""
+        return self._routed_pass(mlp_step, input, (self.fc1_weight, self.fc2_weight), group_sizes, 2 * self.num_groups, route)
