@@ -244,9 +244,10 @@ __device__ __forceinline__ bool staged_bf16_tile(const fp8gmm_gemm_problem& pr, 
          (interior || (cv & 7) == 0);
 }
 // 32-row blocks of a wavefront's sub-tile, which begins with row `first` of the tile and has `most` of them, that hold some of
-// the tile's `rows` rows: the last tile of an expert often holds a few.  The epilogues with arithmetic leave the others out (a
-// GELU tile takes 12 - 14 us, all of it vector instructions).  The plain form does not: it takes 4 us, and with the skip in
-// its straight line the weight gradients, which have no such rows, lost 5 % (16 experts of 256 rows, 4096 x 6400: 202 -> 214 us).
+// the tile's `rows` rows: the last tile of an expert often holds a few.  The GELU form leaves the others out (a tile takes
+// 12 - 14 us, all of it vector instructions).  The plain form does not: it takes 4 us, and with the skip in its straight line the
+// weight gradients, which have no such rows, lost 5 % (16 experts of 256 rows, 4096 x 6400: 202 -> 214 us); nor does the form
+// with the derivative, whose reads one block ahead the compiler then waits for at once.
 __device__ __forceinline__ int row_blocks(int rows, int first, int most) {
   const int n = (rows - first + 31) >> 5;
   return n < 0 ? 0 : n < most ? n : most;
@@ -489,9 +490,9 @@ __device__ __forceinline__ int tile_epilogue(const fp8gmm_gemm_problem& pr, int 
       fetch(0, pre[0]);
       static_for<MT>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
-        if (i >= blocks) return;
+        if (i >= mt) return;
         if constexpr (i + 1 < MT) {
-          if (i + 1 < blocks) fetch(i + 1, pre[(i + 1) & 1]);
+          if (i + 1 < mt) fetch(i + 1, pre[(i + 1) & 1]);
         }
         uint32_t f8[NT][4];
         static_for<NT>([&](auto jc) {
