@@ -39,10 +39,13 @@ class _RoutedModule(torch.nn.Module):
     def start_experts(self):
         """Enqueue what the experts' pass can do before the host knows the split (nothing, by default)."""
 
+    def takes_routed_rows(self, x):
+        """Whether ``experts_on_routed_rows`` takes the place of gather, ``experts`` and scatter; asked behind ``start_experts``."""
+        return False
+
     def experts_on_routed_rows(self, x, batch_sizes, indices, inverse, weights, top_k):
-        """``scatter(experts(gather(x)))`` in passes that fetch the rows and hand them back themselves; None where the experts
-        are called as they are."""
-        return None
+        """``scatter(experts(gather(x)))`` in passes that fetch the rows and hand them back themselves."""
+        raise NotImplementedError
 
     def compute(self, x, tokens_per_expert, indices, bin_ids, expert_weights, bins, top_k, inverse=None):
         return self._compute(x, tokens_per_expert, indices, bin_ids, expert_weights, bins, top_k, inverse, False)
@@ -64,16 +67,16 @@ class _RoutedModule(torch.nn.Module):
         if not routed:
             x = moe_ops.gather(x, indices, bin_ids, bins, top_k, inverse)
         self.start_experts()
+        if routed and not self.takes_routed_rows(x):
+            routed = False
+            x = moe_ops.gather(x, indices, bin_ids, bins, top_k, inverse)   # ahead of the wait as well
         if counts is not None:   # on their way since the sort
             batch_sizes = torch.tensor(counts.wait(), dtype=torch.long)
         else:
             self._counts_ready.synchronize()
             batch_sizes = self._counts_host.to(torch.long, copy=True)   # the page-locked buffer is reused by the next step
         if routed:
-            out = self.experts_on_routed_rows(x, batch_sizes, indices, inverse, expert_weights, top_k)
-            if out is not None:
-                return out
-            x = moe_ops.gather(x, indices, bin_ids, bins, top_k, inverse)
+            return self.experts_on_routed_rows(x, batch_sizes, indices, inverse, expert_weights, top_k)
         out = self.experts(x, batch_sizes)
         return moe_ops.scatter(out, indices, bin_ids, expert_weights, bins, top_k, inverse)
 
@@ -113,11 +116,13 @@ class Fp8LinearModule(_RoutedModule):
     def experts(self, x, batch_sizes):
         return self.grouped_linear2(self.act(self.grouped_linear1(x, batch_sizes)), batch_sizes)
 
+    def takes_routed_rows(self, x):
+        first, second = self.grouped_linear1, self.grouped_linear2
+        return (_own(self, Fp8LinearModule) and type(first) is GroupedLinear and type(second) is GroupedLinear
+                and first._takes_routed_rows(x))
+
     def experts_on_routed_rows(self, x, batch_sizes, indices, inverse, weights, top_k):
         first, second = self.grouped_linear1, self.grouped_linear2
-        if not _own(self, Fp8LinearModule) or type(first) is not GroupedLinear or type(second) is not GroupedLinear \
-                or not first._takes_routed_rows(x):
-            return None
         rows = self.act(first._routed(x, batch_sizes, Route(indices, inverse, None, top_k, True, False)))
         if second._takes_routed_rows(rows):
             return second._routed(rows, batch_sizes, Route(indices, inverse, weights, top_k, False, True))
@@ -137,8 +142,8 @@ class Fp8MlpModule(_RoutedModule):
     def experts(self, x, batch_sizes):
         return self.grouped_mlp(x, batch_sizes)
 
+    def takes_routed_rows(self, x):
+        return _own(self, Fp8MlpModule) and type(self.grouped_mlp) is GroupedMlp and self.grouped_mlp._takes_routed_rows(x)
+
     def experts_on_routed_rows(self, x, batch_sizes, indices, inverse, weights, top_k):
-        mlp = self.grouped_mlp
-        if not _own(self, Fp8MlpModule) or type(mlp) is not GroupedMlp or not mlp._takes_routed_rows(x):
-            return None
-        return mlp._routed(x, batch_sizes, Route(indices, inverse, weights, top_k, True, True))
+        return self.grouped_mlp._routed(x, batch_sizes, Route(indices, inverse, weights, top_k, True, True))

@@ -578,6 +578,36 @@ def test_routed_rows_are_left_to_gather_where_something_looks_on(dev, monkeypatc
     assert gathers(Rows(256, 128, 4, 2))
 
 
+def test_gathered_rows_are_gathered_ahead_of_the_wait_for_the_counts(dev, monkeypatch):
+    """Where a layer's experts do not fetch their rows themselves, the GPU has the gather to do while the host waits."""
+    from fp8_gmm_amd import moe
+
+    ops, order, native = _ops(), [], moe.route
+    gather = ops.gather
+
+    class Waits:
+        def __init__(self, counts):
+            self.counts = counts
+
+        def wait(self):
+            order.append("wait")
+            return self.counts.wait()
+
+    def route(scores, top_k):
+        *lists, counts = native(scores, top_k)
+        return (*lists, Waits(counts))
+
+    monkeypatch.setattr(ops, "gather", lambda *a, **k: (order.append("gather"), gather(*a, **k))[1])
+    monkeypatch.setattr(moe, "route", route)
+    x = torch.randn(64, 256, device=dev).to(torch.bfloat16)
+    layer = moe.Fp8MlpModule(256, 128, 4, 2)
+    want = layer(x)
+    assert order == ["wait"]
+    layer.grouped_mlp.register_forward_hook(lambda *a: None)
+    got = layer(x)
+    assert order == ["wait", "gather", "wait"] and got.shape == want.shape
+
+
 @pytest.mark.parametrize("tokens,experts,top_k,dtype", [(1, 1, 1, torch.float32), (1531, 16, 2, torch.bfloat16),
                                                          (5000, 128, 8, torch.bfloat16), (33, 600, 3, torch.float32),
                                                          (0, 4, 2, torch.bfloat16)])
