@@ -19,7 +19,7 @@ are clamped into the range instead of being undefined.
 import torch
 
 from . import _lib, native
-from .backend import _fail, _stream, _timed
+from .backend import _fail, _stream, _timed, kernel_timing
 
 MAX_EXPERTS = 4096  # size of the on-chip expert table of the sort kernels
 
@@ -179,8 +179,6 @@ def _gating_gradients(grad, x, weight, grad_in):
 
 def _unwatched():
     """Nothing that looks at the launches or at the autograd functions one by one: the native host path has nodes of its own."""
-    from .backend import kernel_timing
-
     return (kernel_timing._active is None and torch._C._functorch.peek_interpreter_stack() is None
             and torch._C._autograd._top_saved_tensors_default_hooks(True) is None and not torch.jit.is_tracing()
             and not torch.compiler.is_compiling())
@@ -375,12 +373,13 @@ def routed_rows_fit(x, indices, inverse, weights, top_k):
     def plain(t, dtype, dim):
         return type(t) is torch.Tensor and t.dtype == dtype and t.dim() == dim and t.is_contiguous() and t.device == x.device
 
+    if not _unwatched():
+        return False
     rows = x.shape[0] * top_k if x.dim() == 2 else -1
     return (x.is_cuda and type(x) in (torch.Tensor, torch.nn.Parameter) and x.dtype == torch.bfloat16 and x.dim() == 2
             and x.is_contiguous() and x.data_ptr() % 16 == 0 and x.shape[1] % 16 == 0
             and plain(indices, torch.int32, 1) and plain(inverse, torch.int32, 1) and plain(weights, torch.float32, 1)
-            and indices.numel() == inverse.numel() == weights.numel() == rows and 1 <= top_k <= _lib.ROUTED_MAX_TOP_K
-            and _unwatched())
+            and indices.numel() == inverse.numel() == weights.numel() == rows and 1 <= top_k <= _lib.ROUTED_MAX_TOP_K)
 
 
 def router_fits(scores, top_k, experts):
