@@ -197,19 +197,29 @@ __global__ __launch_bounds__(kScalingThreads) void delayed_scaling_updates_kerne
 }  // namespace fp8gmm
 
 namespace {
+// Very large plain casts claim this much LDS per workgroup, so that five share a compute unit (of 160 KB) where the registers
+// would let eight: bound by HBM, they have more loads in flight than it takes, and fewer workgroups at a time keep fewer of its rows
+// open.  Eight against five, kernel alone: the forward cast of an MLP's step, 8 experts of 4096 x 14336, 16384 rows 511 / 491 us
+// (61 thousand workgroups), both weight stacks of 16 experts of 4096 x 6400 399 / 391 (51 thousand); tensors of 49 - 66
+// thousand 417 / 411, 426 / 413, 484 / 477, 537 / 525, 550 / 544.  Smaller launches gain as little as they lose inside a step
+// (33 thousand 247 / 248, 14 thousand 115 / 115); the dGELU form needs the wavefronts for its arithmetic (200 / 204).
+constexpr int kApartBlocks = 40000;
+constexpr size_t kApartLds = 32000;
+
 template <bool DGELU>
 int launch_quantize(fp8gmm_tensor_desc* descs_dev, int n, int total_blocks, int out_fmt, void* stream, bool merge = true) {
   if (n < 0 || total_blocks < 0) return FP8GMM_ERR_BAD_ARGUMENT;
   if (out_fmt != FP8GMM_E4M3 && out_fmt != FP8GMM_E5M2) return FP8GMM_ERR_BAD_FORMAT;
   if (n == 0 || total_blocks == 0) return FP8GMM_OK;
   if (descs_dev == nullptr) return FP8GMM_ERR_NULL_POINTER;
+  const size_t apart = !DGELU && total_blocks >= kApartBlocks ? kApartLds : 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (out_fmt == FP8GMM_E4M3)
     hipLaunchKernelGGL((fp8gmm::multi_quantize_kernel<FP8GMM_E4M3, DGELU>), dim3(total_blocks),
-                       dim3(fp8gmm::kPwThreads), 0, s, descs_dev, n);
+                       dim3(fp8gmm::kPwThreads), apart, s, descs_dev, n);
   else
     hipLaunchKernelGGL((fp8gmm::multi_quantize_kernel<FP8GMM_E5M2, DGELU>), dim3(total_blocks),
-                       dim3(fp8gmm::kPwThreads), 0, s, descs_dev, n);
+                       dim3(fp8gmm::kPwThreads), apart, s, descs_dev, n);
   if (merge) hipLaunchKernelGGL(fp8gmm::amax_merge_kernel, dim3((n + 255) / 256), dim3(256), 0, s, descs_dev, n);
   return hipGetLastError() == hipSuccess ? FP8GMM_OK : FP8GMM_ERR_LAUNCH;
 }
