@@ -140,6 +140,15 @@ class _timed:
         return False
 
 
+def _timed_launch(rec):
+    """The bracket of a launch of a planned pass; ``rec``: its record, or the record's bytes (the native host path)."""
+    if isinstance(rec, bytes):
+        rec = _lib.PassLaunch.from_buffer_copy(rec)
+    gemm = rec.kind == _lib.PASS_GEMM
+    return _timed("grouped_gemm" if gemm else _OP_NAMES[rec.op], lambda: rec.work, lambda: rec.bytes,
+                  (lambda: gemm_form(rec.a_fmt, rec.epilogue, rec.plan)) if gemm else None)
+
+
 _OP_NAMES = {
     _lib.OP_QUANTIZE: "multi_quantize",
     _lib.OP_SCALE_MUL: "multi_scale_mul",
@@ -1000,10 +1009,10 @@ def warm_up(device=None):
 # ------------------------------------------------------------------------------------------------
 # a whole pass of a grouped linear layer, planned by one library call
 # ------------------------------------------------------------------------------------------------
-def _run_pass(device, which, desc, fields, snapshot, host_planned, routed=None):
+def _run_pass(device, which, desc, fields, snapshot, host_planned):
     """Fill the pass description `desc` from `fields`, have its tables built and enqueue its launches.  The tables are
     written by a kernel of the library from a description of the pass (fp8gmm_build_pass), which also takes the
-    `snapshot` (source, destination) of fp32 values; `routed`: a pass of routed rows; a pass of more experts or rows than the kernel takes is planned on
+    `snapshot` (source, destination) of fp32 values; a pass of more experts or rows than the kernel takes is planned on
     the host (`host_planned`: planning function, bound on its bytes) and uploaded."""
     L = _lib.load()
     flush_uploads()   # launches queued before this pass come first
@@ -1017,15 +1026,13 @@ def _run_pass(device, which, desc, fields, snapshot, host_planned, routed=None):
             value = value.ctypes.data
         setattr(desc, name, value)
     index = device.index if device.index is not None else torch.cuda.current_device()
-    if not desc.grid:   # else described with its launch policy (run_described_pass)
-        desc.grid = _lib.gemm_grid(_lib.init(index))
-        desc.stream_k = int(bool(options.stream_k))
-        desc.tile_policy = TILE_POLICIES[options.tile]
-    grid = desc.grid
+    grid = desc.grid = _lib.gemm_grid(_lib.init(index))
+    desc.stream_k = int(bool(options.stream_k))
+    desc.tile_policy = TILE_POLICIES[options.tile]
     plan = _lib.PassPlan()
     if desc.experts <= _lib.PASS_MAX_EXPERTS and desc.tokens <= _lib.PASS_MAX_ROWS and 2 * grid <= _lib.PASS_MAX_GRID:
         tables = _lib.PassTables()
-        _lib.check(L.fp8gmm_lay_out_routed_pass(which, ctypes.byref(desc), routed, ctypes.byref(plan), tables))
+        _lib.check(L.fp8gmm_lay_out_pass(which, ctypes.byref(desc), ctypes.byref(plan), tables))
         with _on_device(device):
             blob = torch.empty(plan.blob_bytes, dtype=torch.uint8, device=device)
             src, dst = snapshot if snapshot is not None else (None, None)
@@ -1047,19 +1054,10 @@ def _run_pass(device, which, desc, fields, snapshot, host_planned, routed=None):
             gemm = rec.kind == _lib.PASS_GEMM
             ws = _gemm_workspace(device, rec.plan.n_slots) if gemm else None
             ws_ptr, ws_bytes = (ws.data_ptr(), ws.numel()) if ws is not None else (None, 0)
-            with _timed("grouped_gemm" if gemm else _OP_NAMES[rec.op], lambda: rec.work, lambda: rec.bytes,
-                        (lambda: gemm_form(rec.a_fmt, rec.epilogue, rec.plan)) if gemm else None):
-                rc = L.fp8gmm_run_routed(base, ctypes.byref(rec), routed, desc.tokens, ws_ptr, ws_bytes, stream)
+            with _timed_launch(rec):
+                rc = L.fp8gmm_run_planned(base, ctypes.byref(rec), ws_ptr, ws_bytes, stream)
             _lib.check(rc)
     return plan
-
-
-def run_described_pass(which, device_index, desc, routed=b""):
-    """A backward pass as the native host path describes it (the bytes of its C structures), launch by launch: where
-    ``kernel_timing`` wants every launch bracketed with events.  The launch policy is the description's."""
-    desc = (_lib.LinearPass if which == _lib.LINEAR_BACKWARD else _lib.MlpPass).from_buffer_copy(desc)
-    rows = ctypes.byref(_lib.RoutedRows.from_buffer_copy(routed)) if routed else None
-    _run_pass(torch.device("cuda", device_index), which, desc, {}, None, None, rows)
 
 
 def _plan_on_host(device, desc, plan, plan_fn, bound_fn, grid):

@@ -90,19 +90,26 @@ struct Due {
 // Whether a block of backend.kernel_timing is open (set_kernel_timing).
 std::atomic<bool> kernel_timing{false};
 
+// Enqueues what `launch` does; inside a block of kernel_timing between two events, under what `block` makes of the module
+// `backend`: a bracket of that block.  On the current device and stream, as the launch.
+template <class Block, class Launch>
+void timed(Block&& block, Launch&& launch) {
+  if (!kernel_timing.load(std::memory_order_relaxed)) return launch();
+  py::gil_scoped_acquire gil;
+  const py::object bracket = block(py::module_::import("fp8_gmm_amd.backend"));
+  bracket.attr("__enter__")();
+  launch();
+  bracket.attr("__exit__")(py::none(), py::none(), py::none());
+}
+// ... that moves `bytes` bytes under a name of its own.
+template <class Launch>
+void timed(const char* name, int64_t bytes, Launch&& launch) {
+  timed([&](const py::module_& backend) { return backend.attr("_timed")(name, py::cpp_function([bytes] { return bytes; })); }, launch);
+}
+
 // Builds the tables of a pass and enqueues its launches on the current stream.
 void run_pass(int which, const void* desc, const at::Device& device, const Setup* update, Due* due, const Tensor& snapshot_of,
               const Tensor& snapshot, const fp8gmm_routed_rows* routed = nullptr, int64_t rows = 0) {
-  const bool backward = which == FP8GMM_LINEAR_BACKWARD || which == FP8GMM_MLP_BACKWARD;
-  if (backward && kernel_timing.load(std::memory_order_relaxed)) {
-    // the same launches one by one, each between two events (a module does not come here for such a forward pass)
-    const size_t bytes = which == FP8GMM_LINEAR_BACKWARD ? sizeof(fp8gmm_linear_pass) : sizeof(fp8gmm_mlp_pass);
-    py::gil_scoped_acquire gil;
-    py::module_::import("fp8_gmm_amd.backend")
-        .attr("run_described_pass")(which, (int)device.index(), py::bytes(static_cast<const char*>(desc), bytes),
-                                    py::bytes(reinterpret_cast<const char*>(routed), routed != nullptr ? sizeof(*routed) : 0));
-    return;
-  }
   fp8gmm_pass_plan plan;
   alignas(16) unsigned char tables[FP8GMM_PASS_TABLES_BYTES];
   check(fp8gmm_lay_out_routed_pass(which, desc, routed, &plan, tables));
@@ -138,9 +145,17 @@ void run_pass(int which, const void* desc, const at::Device& device, const Setup
   // partial sums of tiles shared along K: from the caching allocator, which hands memory out again in stream order
   Tensor workspace;
   if (slots > 0) workspace = at::empty({(int64_t)slots * FP8GMM_GEMM_SLOT_BYTES}, bytes);
-  for (int i = 0; i < plan.n_launches; ++i)
-    check(fp8gmm_run_routed(blob.data_ptr(), &plan.launch[i], routed, rows, ptr<void>(workspace),
-                            (size_t)slots * FP8GMM_GEMM_SLOT_BYTES, stream));
+  for (int i = 0; i < plan.n_launches; ++i) {
+    const fp8gmm_pass_launch& l = plan.launch[i];
+    if (l.kind == FP8GMM_PASS_NOTHING) continue;
+    timed([&](const py::module_& backend) {
+            return backend.attr("_timed_launch")(py::bytes(reinterpret_cast<const char*>(&l), sizeof(l)));
+          },
+          [&] {
+            check(fp8gmm_run_routed(blob.data_ptr(), &l, routed, rows, ptr<void>(workspace), (size_t)slots * FP8GMM_GEMM_SLOT_BYTES,
+                                    stream));
+          });
+  }
 }
 
 // Rows of a pass that come from tokens, go back to tokens, or both: what gather and scatter of a routed layer around the
@@ -173,8 +188,10 @@ Tensor aligned(const Tensor& t) {
 // out[t] = sum of the rows of token t, weighted where `weights` is defined
 Tensor scatter_rows(const Tensor& rows, const Tensor& inverse, const Tensor& weights, int64_t top_k) {
   const Tensor out = at::empty({rows.size(0) / top_k, rows.size(1)}, rows.options());
-  check(fp8gmm_moe_scatter(ptr<const void>(rows), ptr<const int32_t>(inverse), ptr<const float>(weights), ptr<void>(out),
-                           (int)out.size(0), (int)out.size(1), (int)top_k, current_stream(rows.device())));
+  timed("moe_scatter", 2 * (rows.numel() + out.numel()), [&] {
+    check(fp8gmm_moe_scatter(ptr<const void>(rows), ptr<const int32_t>(inverse), ptr<const float>(weights), ptr<void>(out),
+                             (int)out.size(0), (int)out.size(1), (int)top_k, current_stream(rows.device())));
+  });
   return out;
 }
 
@@ -656,16 +673,6 @@ struct GatingBackward : public Node {
       if (want_weight) result[1] = grad.t().mm(rows);
       return result;
     }
-    if (kernel_timing.load(std::memory_order_relaxed)) {
-      py::gil_scoped_acquire gil;
-      auto or_none = [](const Tensor& t) { return t.defined() ? py::cast(t) : py::none(); };
-      const auto both = py::module_::import("fp8_gmm_amd.moe_ops")
-                            .attr("_gating_gradients")(grad, or_none(rows), or_none(w), or_none(grad_in))
-                            .cast<std::pair<std::optional<Tensor>, std::optional<Tensor>>>();
-      if (want_x) result[0] = *both.first;
-      if (want_weight) result[1] = *both.second;
-      return result;
-    }
     const Tensor g = aligned(grad), in = grad_in.defined() ? aligned(grad_in) : Tensor();
     const Tensor xs = want_weight ? aligned(rows) : Tensor(), ws = want_x ? w.contiguous() : Tensor();
     if (want_x) result[0] = at::empty({tokens, hidden}, g.options());
@@ -674,9 +681,11 @@ struct GatingBackward : public Node {
       result[1] = at::empty({experts, hidden}, g.options());
       work = at::empty({(int64_t)fp8gmm_gating_workspace_bytes((int)tokens, (int)hidden, (int)experts)}, g.options().dtype(at::kByte));
     }
-    check(fp8gmm_gating_backward(ptr<void>(g), ptr<void>(xs), ptr<void>(ws), ptr<void>(in), ptr<void>(result[0]),
-                                 ptr<void>(result[1]), (int)tokens, (int)hidden, (int)experts, ptr<void>(work),
-                                 current_stream(g.device())));
+    timed("gating_backward", 2 * tokens * hidden * (want_weight + 2 * want_x), [&] {
+      check(fp8gmm_gating_backward(ptr<void>(g), ptr<void>(xs), ptr<void>(ws), ptr<void>(in), ptr<void>(result[0]),
+                                   ptr<void>(result[1]), (int)tokens, (int)hidden, (int)experts, ptr<void>(work),
+                                   current_stream(g.device())));
+    });
     return result;
   }
 };

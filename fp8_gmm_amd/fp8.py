@@ -287,7 +287,7 @@ class Fp8GroupedModuleBase(torch.nn.Module):
 
     def _native(self, input, *weights):
         """Whether a pass on these tensors can take the native host path: the default layout and options, planned
-        passes, nothing that looks at the launches one by one."""
+        passes, no launches queued in front of it."""
         from . import _lib, backend
 
         return (input.is_cuda and input.dtype == torch.bfloat16 and input.dim() == 2 and input.is_contiguous()
@@ -297,7 +297,7 @@ class Fp8GroupedModuleBase(torch.nn.Module):
     def _native_weights(self, _lib, backend, device, weights):
         """What ``_native`` asks of everything but the input (``_lib``, ``backend``: the caller has imported them)."""
         meta = self.fp8_meta
-        if not (meta["planned_passes"] and not meta["reference_layout"] and backend.kernel_timing._active is None
+        if not (meta["planned_passes"] and not meta["reference_layout"]
                 and self.num_groups <= _lib.PASS_MAX_EXPERTS and getattr(backend._pending, "items", None) is None):
             return False
         for w in weights:

@@ -19,7 +19,7 @@ are clamped into the range instead of being undefined.
 import torch
 
 from . import _lib, native
-from .backend import _fail, _stream, _timed, kernel_timing
+from .backend import _fail, _stream, _timed
 
 MAX_EXPERTS = 4096  # size of the on-chip expert table of the sort kernels
 
@@ -178,8 +178,8 @@ def _gating_gradients(grad, x, weight, grad_in):
 
 
 def _unwatched():
-    """Nothing that looks at the launches or at the autograd functions one by one: the native host path has nodes of its own."""
-    return (kernel_timing._active is None and torch._C._functorch.peek_interpreter_stack() is None
+    """Nothing that looks at the autograd functions one by one: the native host path has nodes of its own."""
+    return (torch._C._functorch.peek_interpreter_stack() is None
             and torch._C._autograd._top_saved_tensors_default_hooks(True) is None and not torch.jit.is_tracing()
             and not torch.compiler.is_compiling())
 

@@ -2,6 +2,8 @@
 and the routed example layers end to end.  Integer results and copied rows are compared bit for bit; scatter's
 bf16 output too (the kernel and the oracle follow the same fp32 sequence); only the per-row dot products of
 scatter's weight gradient, whose summation order differs, get a tolerance (1e-5 relative to the row norms)."""
+import contextlib
+
 import numpy as np
 import pytest
 import torch
@@ -538,9 +540,8 @@ def test_routed_rows_give_the_bits_of_gather_and_scatter(dev, monkeypatch, kind,
 
 
 def test_routed_rows_are_left_to_gather_where_something_looks_on(dev, monkeypatch):
-    """A hook on the experts, a replaced `experts`, saved-tensor hooks and an open block of kernel timing see what they saw."""
+    """A hook on the experts, a replaced `experts` and saved-tensor hooks see what they saw."""
     ops = _ops()
-    from fp8_gmm_amd import backend
     from fp8_gmm_amd.moe import Fp8LinearModule, Fp8MlpModule
 
     calls = []
@@ -565,8 +566,6 @@ def test_routed_rows_are_left_to_gather_where_something_looks_on(dev, monkeypatc
     del layer.experts
     with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t.to(dev)):
         assert gathers(layer)
-    with backend.kernel_timing():
-        assert gathers(layer)
     two = Fp8LinearModule(256, 128, 4, 2)
     two.grouped_linear2.register_forward_hook(lambda m, i, o: seen.append(o.shape))
     assert not gathers(two) and seen[-1] == torch.Size([128, 256])   # the first layer fetches, the second is called
@@ -576,6 +575,45 @@ def test_routed_rows_are_left_to_gather_where_something_looks_on(dev, monkeypatc
             return super().experts(rows * 1, sizes)
 
     assert gathers(Rows(256, 128, 4, 2))
+
+
+@pytest.mark.parametrize("kind,launches", [
+    ("mlp", {"multi_quantize": 1, "routed_cast": 1, "routed_gradient": 1, "multi_cast_dgelu": 1, "grouped_gemm": 6,
+             "moe_scatter": 2, "gating_backward": 1}),
+    ("linear", {"multi_quantize": 4, "routed_cast": 1, "routed_gradient": 1, "grouped_gemm": 6, "moe_scatter": 2,
+                "gating_backward": 1})])
+def test_kernel_timing_of_a_routed_layer_is_that_of_its_launches(dev, monkeypatch, kind, launches):
+    """A block of kernel timing around a routed layer's step records the launches that the step makes without it: no gather,
+    the casts that fetch their rows, the same bits."""
+    ops = _ops()
+    from fp8_gmm_amd import DelayedScaling, backend, fp8_autocast
+    from fp8_gmm_amd.moe import Fp8LinearModule, Fp8MlpModule
+
+    make = lambda: (Fp8MlpModule if kind == "mlp" else Fp8LinearModule)(256, 128, 4, 2)
+    state = make().state_dict()
+    x0 = torch.randn(64, 256, device=dev).to(torch.bfloat16)
+    dy = torch.randn(64, 256, device=dev).to(torch.bfloat16)
+    gathers, gather = [], ops.gather
+    monkeypatch.setattr(ops, "gather", lambda *a, **k: (gathers.append(1), gather(*a, **k))[1])
+
+    def steps(timed):
+        layer, results = make(), []
+        layer.load_state_dict(state)
+        for _ in range(3):   # the second and third begin with a scaling update
+            x = x0.clone().requires_grad_()
+            layer.zero_grad()
+            with fp8_autocast(fp8_recipe=DelayedScaling(amax_history_len=4)):
+                with backend.kernel_timing() if timed else contextlib.nullcontext() as timing:
+                    out = layer(x)
+                    out.backward(dy)
+            results += [out.detach(), x.grad] + [p.grad.clone() for p in layer.parameters()]
+            if timed:
+                assert {name: rec["launches"] for name, rec in timing.summary().items()} == launches
+        return results
+
+    for a, b in zip(steps(False), steps(True)):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+    assert not gathers
 
 
 def test_gathered_rows_are_gathered_ahead_of_the_wait_for_the_counts(dev, monkeypatch):
