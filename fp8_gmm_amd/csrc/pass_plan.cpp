@@ -677,7 +677,16 @@ int fp8gmm_lay_out_routed_pass(int which, const void* desc, const fp8gmm_routed_
   }
   if (rc != FP8GMM_OK) return rc;
   memset(out, 0, sizeof(*out));
-  return lay_out_pass(pass, out, static_cast<PassTables*>(tables));
+  rc = lay_out_pass(pass, out, static_cast<PassTables*>(tables));
+  if (rc != FP8GMM_OK || routed == nullptr) return rc;
+  for (int i = 0; i < out->n_launches; ++i) {
+    fp8gmm_pass_launch& l = out->launch[i];
+    if (l.op != FP8GMM_OP_ROUTED_CAST && l.op != FP8GMM_OP_ROUTED_GRADIENT) continue;
+    // described as a cast of its rows: 2 B read + 1 B written per element.  A token is read once, a row of y once.
+    const bool reads_y = l.op == FP8GMM_OP_ROUTED_GRADIENT && routed->grad_weights != nullptr;
+    l.work = l.bytes = l.work / 3 * (1 + 2.0 / routed->top_k + (reads_y ? 2 : 0));
+  }
+  return FP8GMM_OK;
 }
 
 int fp8gmm_lay_out_pass(int which, const void* desc, fp8gmm_pass_plan* out, void* tables) {

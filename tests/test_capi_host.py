@@ -459,3 +459,28 @@ def test_passes_without_rows_need_no_row_tensors():
         assert rc([0, 0], row_tensors + (always,)) == -1
         for name in row_tensors:
             assert rc([0, 3], (name,)) == -1, (which, name)
+
+
+def _routed(**over):
+    fields = dict(inverse=1 << 40, weights=2 << 40, y=3 << 40, grad_weights=4 << 40, top_k=2)
+    fields.update(over)
+    return _lib.RoutedRows(**fields)
+
+
+def test_routed_casts_count_the_bytes_that_they_move():
+    """The bytes of a cast that fetches its rows: every token and every row of ``y`` read once, every fp8 row written once."""
+    lib = _lib.load()
+    plan, tables = _lib.PassPlan(), _lib.PassTables()
+    sizes, h, f = [4, 0, 8], 64, 96
+    for which, describe, cols, gradient in ((_lib.LINEAR_FORWARD, _linear_pass, h, False), (_lib.LINEAR_BACKWARD, _linear_pass, f, True),
+                                            (_lib.MLP_FORWARD, _mlp_pass, h, False), (_lib.MLP_BACKWARD, _mlp_pass, h, True)):
+        for top_k, y in ((1, True), (2, True), (4, True), (2, False)):
+            d = describe(sizes, h, f)
+            routed = _routed(top_k=top_k) if y else _routed(top_k=top_k, y=0, grad_weights=0)
+            assert lib.fp8gmm_lay_out_routed_pass(which, ctypes.byref(d[0]), ctypes.byref(routed), ctypes.byref(plan), tables) == 0
+            casts = [plan.launch[i] for i in range(plan.n_launches) if plan.launch[i].op in (_lib.OP_ROUTED_CAST, _lib.OP_ROUTED_GRADIENT)]
+            want = 12 // top_k * cols * 2 + 12 * cols * (3 if gradient and y else 1)
+            assert [(c.work, c.bytes) for c in casts] == [(want, want)], (which, top_k, y)
+        d = describe([0, 0], h, f)
+        assert lib.fp8gmm_lay_out_routed_pass(which, ctypes.byref(d[0]), ctypes.byref(_routed()), ctypes.byref(plan), tables) == 0
+        assert all(plan.launch[i].work == 0 for i in range(plan.n_launches) if plan.launch[i].op >= _lib.OP_ROUTED_CAST)
