@@ -533,7 +533,7 @@ __global__ __launch_bounds__(kRoutedWaves * 64) void routed_cast_kernel(fp8gmm_t
     const int row = __builtin_amdgcn_readlane(place, own);
     const float sc = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(scale), own));
     const float w = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(weight), own));
-    const bool ok = (uint32_t)row < (uint32_t)rows;   // no place: nothing is read or stored
+    const bool ok = (uint32_t)row < (uint32_t)rows;   // no place: no row is written, no maximum raised, no gradient but 0
     const bool kept = own > 0 && k > 0;                // the token's row, where it is not longer than a chunk
     const __amdgpu_buffer_rsrc_t rs = row_of_token(t);
     const __amdgpu_buffer_rsrc_t rd = make_rsrc(out + (ok ? (size_t)row * hidden : 0), ok ? (uint32_t)hidden : 0u);
@@ -597,12 +597,12 @@ __global__ __launch_bounds__(kRoutedWaves * 64) void routed_cast_kernel(fp8gmm_t
       if (own + 1 < count) fetch(v, row_of_token(t), 0);
     }
     mx = wave_max(mx);
-    if (lane == 0) atomicMax(&maxima[__builtin_amdgcn_readlane(expert, own)], __float_as_uint(mx));
+    if (lane == 0 && ok) atomicMax(&maxima[__builtin_amdgcn_readlane(expert, own)], __float_as_uint(mx));
     if constexpr (GRADIENT) {
       if (dot) {
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
-        if (lane == 0) routed.grad_weights[first + own] = acc;
+        if (lane == 0) routed.grad_weights[first + own] = ok ? acc : 0.f;
       }
     }
   }

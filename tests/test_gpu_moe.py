@@ -539,6 +539,32 @@ def test_routed_rows_give_the_bits_of_gather_and_scatter(dev, monkeypatch, kind,
         assert torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))
 
 
+def test_choices_without_a_place_leave_nothing_behind(dev):
+    """An entry of ``inverse`` that is no row of the pass: the choice is left out, as the row movers leave it out, of the experts'
+    maxima too, and its weight has a gradient of zero."""
+    from fp8_gmm_amd import GroupedLinear, native
+
+    x, dy = torch.randn(8, 64, device=dev).to(torch.bfloat16), torch.randn(8, 32, device=dev).to(torch.bfloat16)
+    places = [1, 0, -1, 2, 3, 8, 6, 7]     # of the tokens' choices; the rows 4 and 5 are nobody's
+    x[2, 5], x[5, 7] = 1000.0, 2000.0
+    dy[2, 3], dy[5, 9] = float("inf"), 500.0
+    inverse = torch.tensor(places, dtype=torch.int32, device=dev)
+    weights = torch.full((8,), 0.5, device=dev, requires_grad=True)
+    layer = GroupedLinear(64, 32, 3, torch.bfloat16, device=dev)
+    layer.cast_weights_ahead()
+    xi = x.clone().requires_grad_()
+    out = layer._routed(xi, torch.tensor([3, 0, 5]), native.Route(inverse.clone(), inverse, weights, 1, True, True))
+    out.backward(dy)
+    experts = [[t for t, p in enumerate(places) if lo <= p < hi] for lo, hi in ((0, 3), (3, 8))]
+    fwd, bwd = layer.fp8_meta["scaling_fwd"].amax_history[0], layer.fp8_meta["scaling_bwd"].amax_history[0]
+    for slot, tokens in zip((0, 2), experts):
+        assert fwd[3 * slot].item() == x[tokens].abs().max().item()
+        assert bwd[2 * slot].item() == (dy[tokens] * 0.5).abs().max().item()
+    assert fwd[3].item() == 0 and bwd[2].item() == 0
+    assert weights.grad[2] == 0 and weights.grad[5] == 0
+    assert not out[[2, 5]].any() and not xi.grad[[2, 5]].any()
+
+
 def test_routed_rows_are_left_to_gather_where_something_looks_on(dev, monkeypatch):
     """A hook on the experts, a replaced `experts` and saved-tensor hooks see what they saw."""
     ops = _ops()
