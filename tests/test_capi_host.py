@@ -484,3 +484,55 @@ def test_routed_casts_count_the_bytes_that_they_move():
         d = describe([0, 0], h, f)
         assert lib.fp8gmm_lay_out_routed_pass(which, ctypes.byref(d[0]), ctypes.byref(_routed()), ctypes.byref(plan), tables) == 0
         assert all(plan.launch[i].work == 0 for i in range(plan.n_launches) if plan.launch[i].op >= _lib.OP_ROUTED_CAST)
+
+
+def test_routed_passes_are_laid_out_and_refused():
+    """What the kernels of routed rows follow is checked on the host: addresses, alignment, choices per token.  The launches: the
+    weights' cast in front merges its own maxima, the rows' cast leaves that to the GEMM that follows."""
+    lib = _lib.load()
+    plan, tables = _lib.PassPlan(), _lib.PassTables()
+    sizes, h, f = [4, 0, 8], 64, 96
+    passes = ((_lib.LINEAR_FORWARD, _linear_pass, "x", "x_fp8"), (_lib.LINEAR_BACKWARD, _linear_pass, "dy", "dy_fp8"),
+              (_lib.MLP_FORWARD, _mlp_pass, "x", "x_fp8"), (_lib.MLP_BACKWARD, _mlp_pass, "dy", "dy_fp8"))
+
+    def lay_out(which, describe, routed, sizes=sizes, **over):
+        d = describe(sizes, h, f, **over)
+        return lib.fp8gmm_lay_out_routed_pass(which, ctypes.byref(d[0]), ctypes.byref(routed) if routed else None, ctypes.byref(plan),
+                                              tables)
+
+    cast, gemm, dgelu = (_lib.PASS_CAST, _lib.OP_QUANTIZE), (_lib.PASS_GEMM, 0), (_lib.PASS_CAST, _lib.OP_CAST_DGELU)
+    rows, grads = (_lib.PASS_CAST, _lib.OP_ROUTED_CAST), (_lib.PASS_CAST, _lib.OP_ROUTED_GRADIENT)
+    for (which, describe, _, _), launches in zip(passes, ([cast, rows, gemm], [grads, gemm, gemm], [cast, rows, gemm, gemm],
+                                                          [grads, gemm, gemm, dgelu, gemm, gemm])):
+        assert lay_out(which, describe, _routed()) == 0
+        got = [plan.launch[i] for i in range(plan.n_launches)]
+        assert [(l.kind, l.op) for l in got] == launches
+        for i, l in enumerate(got):
+            if l.kind == _lib.PASS_CAST:
+                last = got[i + 1].kind == _lib.PASS_GEMM
+                assert l.merge_n == (l.n if last else 0)
+                assert not last or (got[i + 1].merge_n, got[i + 1].merge_offset) == (l.n, l.table_offset)
+            if l.op >= _lib.OP_ROUTED_CAST:
+                assert l.n == len(sizes)
+                # not without its route, whatever the route's rows are (nothing is launched)
+                assert lib.fp8gmm_run_planned(1 << 40, ctypes.byref(l), None, 0, None) == -1
+                assert lib.fp8gmm_run_routed(1 << 40, ctypes.byref(l), None, 12, None, 0, None) == -1
+                for bad, count, status in ((dict(inverse=0), 12, -1), (dict(top_k=0), 12, -6), (dict(top_k=9), 12, -6),
+                                           (dict(top_k=5), 12, -6), (dict(), -1, -6), (dict(), 1 << 31, -6), (dict(), 0, 0)):
+                    routed = _routed(**bad)
+                    assert lib.fp8gmm_run_routed(1 << 40, ctypes.byref(l), ctypes.byref(routed), count, None, 0, None) == status
+    for which, describe, source, target in passes:
+        backward = source == "dy"
+        for bad, status in ((dict(top_k=0), -6), (dict(top_k=-1), -6), (dict(top_k=9), -6), (dict(top_k=5), -6), (dict(inverse=0), -1),
+                            (dict(weights=0), -1 if backward else 0), (dict(y=0), -1 if backward else 0),
+                            (dict(y=0, grad_weights=0), 0), (dict(y=(3 << 40) + 8), -4 if backward else 0)):
+            assert lay_out(which, describe, _routed(**bad)) == status, (which, bad)
+        for name in (source, target):
+            assert lay_out(which, describe, _routed(), **{name: (5 << 40) + 8}) == -4
+            assert lay_out(which, describe, _routed(), **{name: 0}) == -1
+        assert lay_out(which, describe, _routed(inverse=0, weights=0), sizes=[0, 0]) == 0   # no rows: nothing is read
+        assert lay_out(which, describe, _routed(), tokens=13) == -2
+        assert lay_out(which, describe, None) == 0 and not any(plan.launch[i].op >= _lib.OP_ROUTED_CAST for i in range(plan.n_launches))
+    assert lib.fp8gmm_lay_out_routed_pass(0, None, ctypes.byref(_routed()), ctypes.byref(plan), tables) == -1
+    d = _linear_pass(sizes, h, f)
+    assert lib.fp8gmm_lay_out_routed_pass(9, ctypes.byref(d[0]), ctypes.byref(_routed()), ctypes.byref(plan), tables) == -6

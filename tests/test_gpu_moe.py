@@ -508,7 +508,12 @@ def _layer_results(layer, state, x, dy, frozen, steps=2):
     ("mlp", 64, 256, 256, 4, 2, ("grouped", "x")), ("mlp", 64, 256, 256, 4, 2, ("grouped", "x", "gating")),
     ("linear", 301, 1024, 528, 16, 2, ()), ("linear", 5, 48, 2064, 3, 3, ("gating",)), ("linear", 0, 64, 64, 4, 2, ()),
     ("linear", 130, 256, 128, 8, 2, ("grouped_linear1", "x")), ("cutlass", 77, 272, 528, 6, 2, ()),
-    ("mlp", 9000, 256, 64, 16, 2, ()), ("mlp", 3000, 64, 64, 300, 8, ()), ("linear", 40, 256, 64, 4, 2, ("nan",))])
+    ("mlp", 9000, 256, 64, 16, 2, ()), ("mlp", 3000, 64, 64, 300, 8, ()), ("linear", 40, 256, 64, 4, 2, ("nan",)),
+    # a wavefront that goes on to a second token (from 16384 rows of one choice, 32768 of two), the last ones with fewer; rows of
+    # two pieces, fetched again for the token's second choice (from 16384 rows); NaN in tokens that are not a wavefront's first
+    ("mlp", 16411, 64, 48, 16, 2, ()), ("linear", 16411, 64, 48, 5, 1, ()), ("mlp", 8203, 4112, 16, 6, 2, ()),
+    ("linear", 8203, 4112, 16, 6, 2, ("nan",)), ("mlp", 16411, 64, 48, 16, 2, ("nan",)), ("mlp", 16411, 4112, 16, 6, 2, ("nan",)),
+    ("linear", 12301, 96, 32, 7, 4, ("nan",)), ("mlp", 40, 8224, 32, 3, 2, ("nan",))])
 def test_routed_rows_give_the_bits_of_gather_and_scatter(dev, monkeypatch, kind, tokens, hidden, inner, experts, top_k, frozen):
     """A layer whose experts' casts fetch and weigh their rows themselves against the same layer between moe_ops.gather and
     moe_ops.scatter: outputs, every gradient and the scaling state, bit for bit."""
@@ -525,7 +530,9 @@ def test_routed_rows_give_the_bits_of_gather_and_scatter(dev, monkeypatch, kind,
     dy = (torch.randn(tokens, hidden, device=dev) * 1e-2).to(torch.bfloat16)
     if "nan" in frozen:
         frozen = ()
-        x[3, 5], x[7, 200], dy[4, 255], dy[9, 0] = float("nan"), float("inf"), float("nan"), -float("inf")
+        x[3, 5], x[7, -56], dy[4, -1], dy[9, 0] = float("nan"), float("inf"), float("nan"), -float("inf")
+        if tokens > 8000:
+            x[-1, -1], x[5001, 9], dy[-2, -1], dy[6003, 17] = float("nan"), float("inf"), float("nan"), float("inf")
     calls = []
     for name in ("gather", "scatter"):
         monkeypatch.setattr(ops, name, lambda *a, _f=getattr(ops, name), _n=name, **k: (calls.append(_n), _f(*a, **k))[1])
@@ -601,6 +608,30 @@ def test_routed_rows_are_left_to_gather_where_something_looks_on(dev, monkeypatc
             return super().experts(rows * 1, sizes)
 
     assert gathers(Rows(256, 128, 4, 2))
+
+
+@pytest.mark.parametrize("kind", ["mlp", "linear"])
+def test_routed_passes_cast_the_weights_themselves_where_nobody_did(dev, monkeypatch, kind):
+    """A layer that starts nothing ahead of its counts: the routed pass casts the experts' weights as well, behind the scaling
+    update that is due, with the bits of gather and scatter."""
+    ops = _ops()
+    from fp8_gmm_amd.moe import Fp8LinearModule, Fp8MlpModule
+
+    class Late((Fp8MlpModule if kind == "mlp" else Fp8LinearModule)):
+        def start_experts(self):
+            pass
+
+    x, dy = torch.randn(77, 64, device=dev).to(torch.bfloat16), torch.randn(77, 64, device=dev).to(torch.bfloat16)
+    layer, twin, calls, gather = Late(64, 48, 5, 2), Late(64, 48, 5, 2), [], ops.gather
+    state = layer.state_dict()
+    monkeypatch.setattr(ops, "gather", lambda *a, **k: (calls.append(1), gather(*a, **k))[1])
+    got = _layer_results(layer, state, x, dy, (), steps=4)
+    assert len(calls) == 1   # of the first step, which has no scaling state yet
+    monkeypatch.setattr(ops, "routed_rows_fit", lambda *a: False)
+    want = _layer_results(twin, state, x, dy, (), steps=4)
+    assert len(calls) == 5 and len(got) == len(want)
+    for a, b in zip(got, want):
+        assert torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))
 
 
 @pytest.mark.parametrize("kind,launches", [
