@@ -482,8 +482,10 @@ __global__ __launch_bounds__(kRowWaves * 64) void moe_scatter_backward_kernel(co
 // Which expert a place belongs to follows from the descriptors (rows_padded: the first of its rows); a lane looks that up for
 // one choice, for all of a wavefront's at once.  Maxima meet in LDS and go to the descriptors once per workgroup.
 // Bound: HBM.  Against a launch that moves the rows and one that casts them, 16384 tokens of 4096 columns, two choices each of
-// 16 experts: 155 -> 64 us (268 MB; forward), 197 -> 98 (537 MB; gradient); the layer's step 5439 -> 5223 (with the casts of
-// `amax_or_nan`).  3062 rows of 1024: 12 -> 10 and 13 -> 14, a launch less each.
+// 16 experts: 145 -> 45 us (268 MB; forward), 193 -> 93 (537 MB; gradient).  3000 rows of 1024: 10 -> 4.7 and 10.5 -> 6.0.
+// Rows of more than one piece are fetched again for every choice: 32768 rows of 8192 columns 342 -> 130 and 443 -> 235, 131072 of
+// 6144 1050 -> 488 and 1365 -> 813.  Of narrow rows few lanes work: 131072 of 64 columns 41 -> 32 and 57 -> 64, of 256 56 -> 34 and
+// 78 -> 72; few wide ones wait for their pieces one by one: 64 of 14336 8.9 -> 8.0 and 10.1 -> 13.1.
 constexpr int kRoutedWaves = 8;
 constexpr int kRoutedLoads = 8, kRoutedChunk = kRoutedLoads * 64 * 8;   // 16-byte loads of a row under way per lane
 template <int FMT, bool GRADIENT>
@@ -731,9 +733,12 @@ int launch_routed_cast(fp8gmm_tensor_desc* descs_dev, int n, int op, int out_fmt
       (gradient && routed.grad_weights != nullptr && routed.y == nullptr))
     return FP8GMM_ERR_NULL_POINTER;
   if (routed.top_k < 1 || routed.top_k > FP8GMM_ROUTED_MAX_TOP_K || rows % routed.top_k != 0) return FP8GMM_ERR_BAD_ARGUMENT;
-  // One choice a wavefront while that leaves fewer than a thousand workgroups, then whole tokens: a token's row is read once,
-  // and an expert's maximum looked at by fewer workgroups.
-  int per_wave = (int)(rows / (kRoutedWaves * 1024)) / routed.top_k * routed.top_k;
+  // One choice a wavefront up to 1024 workgroups, then as many as keep to those, and whole tokens once that is one: a token's row
+  // is read once then, and an expert's maximum looked at by no more workgroups.  (One choice up to 1024 * top_k workgroups instead:
+  // 34000 rows of 512 columns, eight choices each of 384 experts, 24.4 / 16.0 us forward and 41 / 31 the gradient; the launches
+  // that it replaces took 39 there for the gradient.)
+  int per_wave = (int)(rows / (kRoutedWaves * 1024));
+  if (per_wave >= routed.top_k) per_wave -= per_wave % routed.top_k;
   per_wave = per_wave < 1 ? 1 : per_wave > 64 / routed.top_k * routed.top_k ? 64 / routed.top_k * routed.top_k : per_wave;
   const int per_block = kRoutedWaves * per_wave;
   hipStream_t s = static_cast<hipStream_t>(stream);

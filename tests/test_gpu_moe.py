@@ -513,7 +513,9 @@ def _layer_results(layer, state, x, dy, frozen, steps=2):
     # two pieces, fetched again for the token's second choice (from 16384 rows); NaN in tokens that are not a wavefront's first
     ("mlp", 16411, 64, 48, 16, 2, ()), ("linear", 16411, 64, 48, 5, 1, ()), ("mlp", 8203, 4112, 16, 6, 2, ()),
     ("linear", 8203, 4112, 16, 6, 2, ("nan",)), ("mlp", 16411, 64, 48, 16, 2, ("nan",)), ("mlp", 16411, 4112, 16, 6, 2, ("nan",)),
-    ("linear", 12301, 96, 32, 7, 4, ("nan",)), ("mlp", 40, 8224, 32, 3, 2, ("nan",))])
+    ("linear", 12301, 96, 32, 7, 4, ("nan",)), ("mlp", 40, 8224, 32, 3, 2, ("nan",)),
+    # wavefronts that begin and end inside a token (from 16384 rows of three choices or more)
+    ("mlp", 5501, 64, 48, 7, 3, ("nan",)), ("linear", 5501, 4112, 16, 7, 3, ("nan",)), ("mlp", 5301, 96, 32, 20, 8, ("nan",))])
 def test_routed_rows_give_the_bits_of_gather_and_scatter(dev, monkeypatch, kind, tokens, hidden, inner, experts, top_k, frozen):
     """A layer whose experts' casts fetch and weigh their rows themselves against the same layer between moe_ops.gather and
     moe_ops.scatter: outputs, every gradient and the scaling state, bit for bit."""
