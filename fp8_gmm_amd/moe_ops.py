@@ -367,6 +367,15 @@ class _Scatter(torch.autograd.Function):
         return grad_x, None, grad_w, None, None
 
 
+def _gathering_is_faster(tokens, hidden, top_k):
+    """Whether many narrow rows had better be gathered: of fewer than 256 columns the casts that fetch them keep few lanes busy
+    (131072 rows of 128 columns: the gradient's 69 us where the launches that it replaces take 64, the forward one 33 and 45), and the gather
+    is what the GPU has to do while the host waits for the counts.  A layer's step, fetched / gathered: 131072 rows of 64 columns 663 /
+    624 us with one choice, 568 / 541 with two, 489 / 456 with eight; of 128 659 / 626, 580 / 557 and 502 / 473; of 256 752 / 743, 640 /
+    636 and 546 / 548; 65536 rows of 128 435 / 416 with one, but 384 / 407 and 357 / 413; 32768 324 / 403: the host has less to do."""
+    return hidden < 256 and (tokens >= 1 << 16 or tokens * top_k > 1 << 16)
+
+
 def routed_rows_fit(x, indices, inverse, weights, top_k):
     """Whether the experts' casts can fetch and weigh the rows themselves (fp8gmm_routed_rows) in place of ``gather`` and
     ``scatter`` around them: tensors as those two make them, nobody looking on."""
@@ -379,7 +388,8 @@ def routed_rows_fit(x, indices, inverse, weights, top_k):
     return (x.is_cuda and type(x) in (torch.Tensor, torch.nn.Parameter) and x.dtype == torch.bfloat16 and x.dim() == 2
             and x.is_contiguous() and x.data_ptr() % 16 == 0 and x.shape[1] % 16 == 0
             and plain(indices, torch.int32, 1) and plain(inverse, torch.int32, 1) and plain(weights, torch.float32, 1)
-            and indices.numel() == inverse.numel() == weights.numel() == rows and 1 <= top_k <= _lib.ROUTED_MAX_TOP_K)
+            and indices.numel() == inverse.numel() == weights.numel() == rows and 1 <= top_k <= _lib.ROUTED_MAX_TOP_K
+            and not _gathering_is_faster(x.shape[0], x.shape[1], top_k))
 
 
 def router_fits(scores, top_k, experts):

@@ -612,6 +612,22 @@ def test_routed_rows_are_left_to_gather_where_something_looks_on(dev, monkeypatc
     assert gathers(Rows(256, 128, 4, 2))
 
 
+@pytest.mark.parametrize("tokens,hidden,top_k,fetched", [
+    (65535, 240, 1, True), (65536, 240, 1, False), (65536, 256, 1, True), (32768, 64, 2, True), (32769, 64, 2, False),
+    (32769, 256, 2, True), (8192, 16, 8, True), (8193, 16, 8, False)])
+def test_many_narrow_rows_are_gathered(dev, monkeypatch, tokens, hidden, top_k, fetched):
+    """Rows of few columns in large numbers, which the casts fetch slower than they are gathered, on either side of the line."""
+    ops = _ops()
+    from fp8_gmm_amd.moe import Fp8MlpModule
+
+    calls, gather = [], ops.gather
+    monkeypatch.setattr(ops, "gather", lambda *a, **k: (calls.append(1), gather(*a, **k))[1])
+    x = torch.randn(tokens, hidden, device=dev).to(torch.bfloat16).requires_grad_()
+    layer = Fp8MlpModule(hidden, 16, 16, top_k)
+    layer(x).sum().backward()
+    assert bool(calls) is not fetched and torch.isfinite(x.grad).all()
+
+
 @pytest.mark.parametrize("kind", ["mlp", "linear"])
 def test_routed_passes_cast_the_weights_themselves_where_nobody_did(dev, monkeypatch, kind):
     """A layer that starts nothing ahead of its counts: the routed pass casts the experts' weights as well, behind the scaling
