@@ -18,8 +18,9 @@ namespace fp8gmm {
 namespace {
 
 // NaNs are looked for once per lane, behind its 64 values (amax_or_nan), and the values taken one by one only where there is
-// one: training steps of 128 experts (65536 rows, 2048 -> 768 -> 2048) 1221 -> 1210 us (cast + dGELU 58 -> 54, forward cast 249
-// -> 245), of 16 experts (4096 rows, 4096 -> 6400 -> 4096) 1083 -> 1077, against a look at every value and a branch for every four.
+// one: in the step of 128 experts (65536 rows, 2048 -> 768 -> 2048) cast + dGELU 58 -> 54 us, forward cast 249 -> 245, against a look
+// at every value and a branch for every four.  A step gains no more than its runs differ by (1209 -> 1199; 16 experts of 4096 x 6400,
+// 4096 rows: 1053, 1054).
 // DGELU: the value cast is x = in * dgelu(in2) (in = gradient of the GELU output, in2 = pre-GELU activation),
 // the same product, in the same order, as the transposing kernel forms.
 template <int FMT, bool DGELU>
@@ -197,9 +198,10 @@ __global__ __launch_bounds__(kScalingThreads) void delayed_scaling_updates_kerne
 }  // namespace fp8gmm
 
 namespace {
-// Very large plain casts claim this much LDS per workgroup, so that five share a compute unit (of 160 KB) where the registers
-// would let eight: bound by HBM, they have more loads in flight than it takes, and fewer workgroups at a time keep fewer of its rows
-// open.  Eight against five, kernel alone: the forward cast of an MLP's step, 8 experts of 4096 x 14336, 16384 rows 511 / 491 us
+// Very large plain casts claim this much LDS per workgroup, so that four share a compute unit where the registers would let eight
+// (with the 16 bytes of `stage` 26 of its 128 granules of 1280 bytes; at 31744 bytes, which leave five, nothing is gained: 522 / 509 us
+// for the first of these): bound by HBM, they have more loads in flight than it takes, and fewer workgroups at a time keep fewer of its
+// rows open.  Eight against four, kernel alone: the forward cast of an MLP's step, 8 experts of 4096 x 14336, 16384 rows 511 / 491 us
 // (61 thousand workgroups), both weight stacks of 16 experts of 4096 x 6400 399 / 391 (51 thousand); tensors of 49 - 66
 // thousand 417 / 411, 426 / 413, 484 / 477, 537 / 525, 550 / 544.  Smaller launches gain as little as they lose inside a step
 // (33 thousand 247 / 248, 14 thousand 115 / 115); the dGELU form needs the wavefronts for its arithmetic (200 / 204).

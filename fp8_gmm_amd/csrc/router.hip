@@ -482,10 +482,11 @@ __global__ __launch_bounds__(kRowWaves * 64) void moe_scatter_backward_kernel(co
 // Which expert a place belongs to follows from the descriptors (rows_padded: the first of its rows); a lane looks that up for
 // one choice, for all of a wavefront's at once.  Maxima meet in LDS and go to the descriptors once per workgroup.
 // Bound: HBM.  Against a launch that moves the rows and one that casts them, 16384 tokens of 4096 columns, two choices each of
-// 16 experts: 145 -> 45 us (268 MB; forward), 193 -> 93 (537 MB; gradient).  3000 rows of 1024: 10 -> 4.7 and 10.5 -> 6.0.
-// Rows of more than one piece are fetched again for every choice: 32768 rows of 8192 columns 342 -> 130 and 443 -> 235, 131072 of
-// 6144 1050 -> 488 and 1365 -> 813.  Of narrow rows few lanes work: 131072 of 64 columns 41 -> 32 and 57 -> 64, of 256 56 -> 34 and
-// 78 -> 72; few wide ones wait for their pieces one by one: 64 of 14336 8.9 -> 8.0 and 10.1 -> 13.1.
+// 16 experts, inside a layer's step: 155 -> 65 us (268 MB; forward), 197 -> 103 (537 MB; gradient).  Both again and again on the same
+// buffers: 145 -> 45 and 193 -> 93; 3000 rows of 1024 columns 10 -> 4.7 and 10.5 -> 6.0.  Rows of more than one piece are fetched again for
+// every choice: 32768 rows of 8192 columns 342 -> 130 and 443 -> 235, 131072 of 6144 1050 -> 488 and 1365 -> 813.  Of narrow rows few lanes
+// work (131072 of 64 columns 41 -> 32 and 57 -> 64, of 256 56 -> 34 and 78 -> 72: moe_ops gathers many of less than 256); few wide
+// ones wait for their pieces one by one (64 of 14336 8.9 -> 8.0 and 10.1 -> 13.1).
 constexpr int kRoutedWaves = 8;
 constexpr int kRoutedLoads = 8, kRoutedChunk = kRoutedLoads * 64 * 8;   // 16-byte loads of a row under way per lane
 template <int FMT, bool GRADIENT>

@@ -559,7 +559,8 @@ int fp8gmm_build_pass(const void* tables, void* blob_dev, const fp8gmm_scaling_u
  *   forward : x is bf16 [tokens / top_k, columns]; the row is x[t]   (fp8gmm_moe_gather)
  *   backward: dy is bf16 [tokens / top_k, columns]; the row is bf16(weights[t * top_k + k] * dy[t]), and
  *             grad_weights[t * top_k + k] = < the row of y, dy[t] > unless grad_weights is NULL   (fp8gmm_moe_scatter_backward)
- * The same bits as those calls in front of the cast.  All of it device memory; x, dy, y and the fp8 rows on 16 bytes.  Laid out
+ * The same bits as those calls in front of the cast; a choice whose entry is no row of the pass is left out: no row, no maximum, a
+ * gradient of 0 for its weight.  All of it device memory; x, dy, y and the fp8 rows on 16 bytes.  Laid out
  * as by fp8gmm_lay_out_pass; every launch of such a pass is run by fp8gmm_run_routed with the same `routed` and the pass's
  * number of rows (fp8gmm_run_planned refuses the cast).
  */
